@@ -316,16 +316,16 @@ int dl_prob_layer_eval_ws_nodes(const float *x, const int32_t *idx32, const floa
  * and learnable_mapping_cuda.forward/.backward for argmax selection
  * (learnable_mapping_cuda_kernel.cu:22-81,236-257; learnable_layer.py:216-236).
  *   x [B,I], W [M,I], m [B,M];   S = softmax(W / tau) along I, never materialised.
- * precision: 0 = fp32 operands on the fp32 matrix cores (reference numerics),
+ * precision: 0 = fp32 operands (reference numerics; each the exact sum of three bf16 planes on the matrix cores),
  *            1 = bf16 operands, fp32 accumulation (tolerance documented with the tests).
  * stats (dl_soft_map_saved_bytes bytes) is written by the forward and read by the backward.
  *   gx = gm * S,   gW = S * (G - r) / tau with G = gm^T x and r[o] = sum_b gm[b,o] m[b,o].
  * ------------------------------------------------------------------------ */
-/* size of `stats`: what the forward keeps for the backward (row maximum and 1/sum; with
- * precision 1 also the bf16 softmax numerators, M*I*2 bytes) */
+/* size of `stats`: what the forward keeps for the backward (row maximum, 1/sum, the packed x and the softmax
+ * numerators as bf16 planes: M*I*2 bytes with precision 1, M*I*6 with precision 0, rounded up to whole tiles) */
 size_t dl_soft_map_saved_bytes(int B, int I, int M, int precision);
-/* scratch of either direction (one size for both): the backward's r [M] and partial gx products and,
- * with precision 1, the bf16 copies of x and gm.  The forward only needs it with precision 1. */
+/* scratch of either direction (one size for both): partial products of small shapes, the backward's partial r and
+ * packed x and gm.  With precision 0 the forward runs without it (ws = NULL), then without splitting the reduction. */
 size_t dl_soft_map_workspace_bytes(int B, int I, int M, int precision);
 int dl_soft_map_fwd(const float *x, const float *W, float tau, float *m, float *stats,
                     void *ws, size_t ws_bytes, int B, int I, int M, int precision, void *stream);

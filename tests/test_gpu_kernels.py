@@ -579,6 +579,39 @@ def test_soft_mapping_bf16_operands(shape, tau):
     assert np.abs(Wt.grad.cpu().numpy() - gW).max() <= 1e-2 * np.abs(gW).max()
 
 
+@pytest.mark.parametrize("precision", [0, 1])
+@pytest.mark.parametrize("shape", [
+    (1, 1, 1), (64, 31, 127), (128, 128, 256),   # one tile and its edges; rows of W that are no multiple of 8
+    (129, 129, 257), (256, 1030, 300),           # 256-row tiles begin; every dimension one past a tile; widths of no 16-byte rows
+    (257, 2050, 70), (300, 4100, 1050),          # row statistics with 512 and 1024 threads per block; ragged batches
+    (40, 8200, 33),                              # rows too wide for the registers: read three times
+    (70, 200, 70000),                            # gW in tiles of 256 rows of W; the last of them ragged
+])
+def test_soft_mapping_tile_edges(shape, precision):
+    """Every padded edge of the matrix products against float64, in the 2-norm.  fp32 operands: a softmax entry carries
+    |w - max| / tau * 2^-23 from its exponent (here below 5 * 2^-23) and two roundings, a sum of n products sqrt(n) * 2^-24
+    for n <= 70000: below 1e-5 together.  bf16 operands: three factors rounded to 2^-9 each, 1e-2.  gW = S (G - r) / tau is a
+    difference: its error is that of its two terms (with one input it is exactly zero, and they are not)."""
+    ops = _ops()
+    B, I, M = shape
+    g = torch.Generator("cuda").manual_seed(B + I + M)
+    x = torch.rand(B, I, device="cuda", generator=g)
+    W = torch.randn(M, I, device="cuda", generator=g) * 0.5
+    gm = torch.randn(B, M, device="cuda", generator=g)
+    xt, Wt = x.clone().requires_grad_(), W.clone().requires_grad_()
+    m = ops.SoftMapFunction.apply(xt, Wt, 1.0, precision)
+    m.backward(gm)
+    xd, Wd = x.double().requires_grad_(), W.double().requires_grad_()
+    md = xd @ torch.softmax(Wd, dim=-1).t()
+    md.backward(gm.double())
+    limit = 1e-5 if precision == 0 else 1e-2
+    S, G, r = torch.softmax(Wd.detach(), dim=-1), gm.double().t() @ x.double(), (gm.double() * md.detach()).sum(0)
+    terms = (S * G).norm() + (S * r[:, None]).norm()
+    for got, want, size in ((m.detach(), md.detach(), md.norm()), (xt.grad, xd.grad, xd.grad.norm()), (Wt.grad, Wd.grad, terms)):
+        assert torch.isfinite(got).all()
+        assert float((got.double() - want).norm()) <= limit * float(size)
+
+
 def test_soft_and_hard_mapping_against_reference_vectors(golden):
     ops = _ops()
     g = golden
