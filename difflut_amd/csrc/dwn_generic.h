@@ -3,6 +3,7 @@
 // alpha_n / beta_n (nullable, device [N]): every node's own alpha and beta instead of the scalars.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <stdint.h>
 
 int dwn_generic_forward(const float *x, const int *idx32, const float *luts, float *y, int B, int I, int N, int k, int O,
                         hipStream_t s);
@@ -15,3 +16,5 @@ size_t dwn_generic_smooth_bytes(int N, int k, int O);
 // Eval forward for any input values; returns at once when *skip_if_set (device, nullable) is non-zero.
 int dwn_generic_eval(const float *x, const int *idx32, const float *luts, float *y, int B, int I, int N, int k, int O,
                      const int *skip_if_set, hipStream_t s);
+// the address bytes [B/64][N][64] of a k = 7 or 8 layer from x alone
+int dwn_generic_addresses(const float *x, const int *idx32, uint8_t *addrT, int B, int I, int N, int k, hipStream_t s);

@@ -192,6 +192,21 @@ int dwn_generic_forward(const float *x, const int *idx32, const float *luts, flo
     return dl_launch_status();
 }
 
+// addresses of every (node, row) as the lookup forward of k = 7 and 8 saves them, [tile][node][64], rows past B zero
+__global__ __launch_bounds__(256) void dwn_generic_addr(const float *__restrict__ x, const int *__restrict__ idx32,
+                                                         uint8_t *__restrict__ addrT, long long total, int B, int I, int N, int K) {
+    const long long e = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (e >= total) return;
+    const long long tn = e >> 6;
+    const long long b = tn / N * 64 + (e & 63);
+    addrT[e] = b < B ? (uint8_t)dwn_addr_generic(x + (size_t)b * I, idx32 + (size_t)(tn % N) * K, K) : (uint8_t)0;
+}
+int dwn_generic_addresses(const float *x, const int *idx32, uint8_t *addrT, int B, int I, int N, int k, hipStream_t s) {
+    const long long total = (long long)((B + 63) / 64) * N * 64;
+    dwn_generic_addr<<<dl_ceil_div(total, 256), 256, 0, s>>>(x, idx32, addrT, total, B, I, N, k);
+    return dl_launch_status();
+}
+
 size_t dwn_generic_smooth_bytes(int N, int k, int O) { return ((size_t)N * O << k) * sizeof(float); }
 
 int dwn_generic_backward(const float *x, const int *idx32, const int *inv_ptr, const int *inv_pos, const float *luts,

@@ -21,7 +21,10 @@
 //                           gx[b,i] = sum gyT[c][b] * D[c][j][a'(b)]  - a gather in fixed order; its launch
 //                           also carries the blocks that add the histogram partials in chunk order (no
 //                           floating-point atomics anywhere)
-// k > 6 goes to the one-thread-per-element kernels of dwn_generic.hip.
+// k = 7 and 8 take the same layout with tables over 2 and 4 registers.  (The one-thread-per-element kernels they went
+// through before spent 726 us of 894 on two random 4-byte table reads per row and connection: 1024 rows, 4096 -> 2048
+// nodes of 8 inputs.  Here a connection of 64 rows costs two coalesced loads of its coefficient row and two lane reads:
+// 29 us, all five kernels 85 us.)  k > 8 goes to the kernels of dwn_generic.hip, where a row would take 4 registers or more.
 #include "dl_common.h"
 #include <algorithm>
 #include <mutex>
@@ -36,6 +39,18 @@ __device__ __forceinline__ unsigned dwn_shift_in(unsigned addr, u64 mask) {
     u64 carry_out;
     asm("v_addc_co_u32_e64 %0, %1, %2, %2, %3" : "=v"(out), "=s"(carry_out) : "v"(addr), "s"(mask));
     return out;
+}
+
+// entry `a` of a table kept 64 entries to a register, one per lane
+template <int NR>
+__device__ __forceinline__ float dwn_table_read(const float (&entry)[NR], unsigned a) {
+    float v = dl_lane_read(entry[0], (int)a);  // (the lane number wraps at 64)
+#pragma unroll
+    for (int r = 1; r < NR; ++r) {
+        const float u = dl_lane_read(entry[r], (int)a);
+        v = (a >> 6) == (unsigned)r ? u : v;
+    }
+    return v;
 }
 
 // ---------------------------------------------------------------------------------
@@ -147,6 +162,7 @@ __global__ __launch_bounds__(64 * DWN_FW) void dwn_lookup_fwd(const u64 *__restr
     const __amdgpu_buffer_rsrc_t rs_addr =
         __builtin_amdgcn_make_buffer_rsrc((void *)(addrT + (size_t)t * N * 64), 0, N * 64, 0x00020000);
     const int lane4s = (lane & (L - 1)) * 4;
+    constexpr int NR = L > 64 ? L / 64 : 1;  // registers of a table
     const int cend = min(DWN_TC, NO - c0);
     const int wbeg = wave * DWN_WC;
     // slot s = (column within my 16) * K + j  ->  lane s % 64 of register s / 64
@@ -165,12 +181,14 @@ __global__ __launch_bounds__(64 * DWN_FW) void dwn_lookup_fwd(const u64 *__restr
 #pragma unroll
         for (int g = 0; g < DWN_WC; g += DWN_CG) {
             u64 w[DWN_CG][K];
-            float entry[DWN_CG];
+            float entry[DWN_CG][NR];
 #pragma unroll
             for (int q = 0; q < DWN_CG; ++q) {
                 const int c = FULL ? c0 + wbeg + g + q : min(c0 + wbeg + g + q, NO - 1);
                 // table row of column c, one entry per lane; the row offset travels in an SGPR
-                entry[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs_luts, lane4s, c * (L * 4), 0));
+#pragma unroll
+                for (int r = 0; r < NR; ++r)
+                    entry[q][r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs_luts, lane4s & 255, c * (L * 4) + r * 256, 0));
 #pragma unroll
                 for (int j = 0; j < K; ++j) {
                     constexpr int dummy = 0;
@@ -188,7 +206,7 @@ __global__ __launch_bounds__(64 * DWN_FW) void dwn_lookup_fwd(const u64 *__restr
                 unsigned addr = 0;
 #pragma unroll
                 for (int j = K - 1; j >= 0; --j) addr = dwn_shift_in(addr, w[q][j]);
-                const float v = dl_lane_read(entry[q], (int)addr);
+                const float v = dwn_table_read<NR>(entry[q], addr);
                 if (FULL || cc < cend) {
                     tile[cc][lane] = EVAL ? (v >= 0.5f ? 1.0f : 0.0f) : v;
                     if (CHAIN && planes_out) {  // the next layer's view of this column: bit r = (y[64t+r][c] >= 0.5)
@@ -430,6 +448,58 @@ __device__ __forceinline__ void dwn_table_block(const DwnTables &tb, int block) 
     else dwn_efd_table_block(tb, block);
 }
 
+// The D form of tables with 128 or 256 entries, one block per table, the table in LDS as doubles.  EFD with |beta| <= 1/2:
+// smoothed along every input once; the difference across bit j is then (1 - beta) times the D-form value.  Other betas:
+// smoothed along all inputs but j, for every j.  Stabilised node: the 2^(k-1)-term sums.
+__global__ __launch_bounds__(256) void dwn_wide_tables(DwnTables tb) {
+    __shared__ double tab[256], tmp[256];
+    __shared__ double rec[16];
+    const int c = blockIdx.x, K = tb.K, L = 1 << K, Lh = L >> 1, a = threadIdx.x;
+    const double alpha = tb.alpha_n ? (double)tb.alpha_n[c / tb.O] : (double)tb.alpha;
+    const double beta = tb.beta_n ? (double)tb.beta_n[c / tb.O] : (double)tb.beta;
+    float *__restrict__ D = tb.D + (size_t)c * K * Lh;
+    if (a < L) tab[a] = (double)tb.luts[(size_t)c * L + a];
+    if (a < 16) rec[a] = 1.0 / (double)(a + 1);
+    __syncthreads();
+    auto smooth = [&](double *t, int skip) {  // t <- t smoothed along every input but `skip`; called by the whole block
+        for (int m = 0; m < K; ++m) {
+            if (m == skip) continue;
+            double lo = 0.0, hi = 0.0;
+            const bool mine = a < L && !((a >> m) & 1);
+            if (mine) { lo = t[a]; hi = t[a | (1 << m)]; }
+            __syncthreads();
+            if (mine) { t[a] = lo + beta * hi; t[a | (1 << m)] = hi + beta * lo; }
+            __syncthreads();
+        }
+    };
+    auto squeeze = [](int v, int j) { return (v & ((1 << j) - 1)) | ((v >> (j + 1)) << j); };
+    if (tb.scale) {
+        const double sc = (double)tb.scale[c / tb.O];
+        for (int o = a; o < K * Lh; o += 256) {
+            const int j = o / Lh, ap = o - j * Lh, low = (1 << j) - 1;
+            double acc = 0.0;
+            for (int kp = 0; kp < Lh; ++kp) {
+                const int at = (kp & low) | ((kp & ~low) << 1);
+                acc += (tab[at | (1 << j)] - tab[at]) * rec[__popc(ap ^ kp)];
+            }
+            D[o] = (float)(sc * acc);
+        }
+    } else if (beta >= -0.5 && beta <= 0.5) {
+        smooth(tab, -1);
+        if (a < L)
+            for (int j = 0; j < K; ++j)
+                if (!((a >> j) & 1)) D[j * Lh + squeeze(a, j)] = (float)(alpha / (1.0 - beta) * (tab[a | (1 << j)] - tab[a]));
+    } else {
+        for (int j = 0; j < K; ++j) {
+            if (a < L) tmp[a] = tab[a];
+            __syncthreads();
+            smooth(tmp, j);
+            if (a < L && !((a >> j) & 1)) D[j * Lh + squeeze(a, j)] = (float)(alpha * (tmp[a | (1 << j)] - tmp[a]));
+            __syncthreads();
+        }
+    }
+}
+
 // gluts[c][a] *= scale[c / O]: the stabilised node scales its table gradient as well
 __global__ __launch_bounds__(256) void dwn_scale_tables(float *__restrict__ gluts, const float *__restrict__ scale,
                                                          long long total, int L, int O) {
@@ -493,33 +563,38 @@ __device__ __forceinline__ bool dwn_quad_merge(unsigned a, float v, int hr, floa
 // column tile the block's bins are the result.  With several, every block stores its bins as a partial
 // ([chunk][column][bin]) and dwn_reduce_partials adds them in chunk order afterwards, so the sums do not depend on the
 // order the blocks ran in (no floating-point atomics).  scale (nullable): the stabilised node's per-node factor.
-__device__ __forceinline__ void dwn_hist_flush(const float (*hist)[65], int c0, int cend, int L, long long NOL, int chunks,
+__device__ __forceinline__ void dwn_hist_flush(const float *hist, int ld, int c0, int cend, int L, long long NOL, int chunks,
                                                float *__restrict__ partial, float *__restrict__ gluts,
                                                const float *__restrict__ scale, int O) {
     if (chunks == 1) {
         for (int e = threadIdx.x; e < cend * L; e += 256)
-            gluts[(size_t)c0 * L + e] = hist[e / L][e % L] * (scale ? scale[(c0 + e / L) / O] : 1.0f);
+            gluts[(size_t)c0 * L + e] = hist[e / L * ld + e % L] * (scale ? scale[(c0 + e / L) / O] : 1.0f);
         return;
     }
     float *mine = partial + (size_t)blockIdx.y * NOL + (size_t)c0 * L;
-    for (int e = threadIdx.x; e < cend * L; e += 256) mine[e] = hist[e / L][e % L];
+    for (int e = threadIdx.x; e < cend * L; e += 256) mine[e] = hist[e / L * ld + e % L];
 }
 
-template <bool WRITE_T>
+// WIDE: tables of more than 64 entries, whose bins are dynamic LDS (64 columns of L + 1 floats; 66 KB at k = 8, so one
+// block per CU and dwn_hist_grid asks for as many)
+template <bool WRITE_T, bool WIDE = false>
 __global__ __launch_bounds__(256) void dwn_bwd_transpose_hist(const float *__restrict__ gy, const uint8_t *__restrict__ addrT,
                                                                float *__restrict__ gyT, float *__restrict__ gluts,
                                                                int B, int NO, int O, int L, int BP, int BT,
                                                                int tiles_per_chunk, float *__restrict__ partial,
                                                                const float *__restrict__ scale, int chunks, DwnTables tb) {
     __shared__ float tile[64][DWN_HC + 1];       // [row][column]
-    __shared__ float hist[DWN_HC][65];           // [column][bin]
+    __shared__ float hist_s[WIDE ? 1 : DWN_HC * 65];  // [column][bin]
+    extern __shared__ float hist_d[];
+    float *const hist = WIDE ? hist_d : hist_s;
+    const int ld = WIDE ? L + 1 : 65;
     __shared__ __align__(16) uint8_t atile[DWN_HC][64 + 4];  // [column][row] addresses
     if ((int)blockIdx.y >= chunks) return dwn_table_block(tb, ((int)blockIdx.y - chunks) * gridDim.x + blockIdx.x);
     const int c0 = blockIdx.x * DWN_HC;
     const int lane = threadIdx.x & 63;
     const int wave = dl_uniform(threadIdx.x >> 6);
     const int cend = min(DWN_HC, NO - c0);
-    for (int e = threadIdx.x; e < DWN_HC * 65; e += 256) (&hist[0][0])[e] = 0.0f;
+    for (int e = threadIdx.x; e < DWN_HC * ld; e += 256) hist[e] = 0.0f;
     const int t_begin = blockIdx.y * tiles_per_chunk;
     const int t_end = min(BT, t_begin + tiles_per_chunk);
     const bool vec4 = (NO % 4 == 0) && cend == DWN_HC;
@@ -579,13 +654,13 @@ __global__ __launch_bounds__(256) void dwn_bwd_transpose_hist(const float *__res
                 const float v = tile[r0 + hr][hc];  // rows past B carry 0
                 const unsigned a = atile[hc][r0 + hr];
                 float sum;
-                if (dwn_quad_merge(a, v, hr, sum)) dwn_bin_add(&hist[hc][a], sum);
+                if (dwn_quad_merge(a, v, hr, sum)) dwn_bin_add(&hist[hc * ld + a], sum);
             }
         }
     }
     __syncthreads();
     // scale (nullable): the stabilised node multiplies a node's table gradient by its gradient_scale
-    dwn_hist_flush(hist, c0, cend, L, (long long)NO * L, chunks, partial, gluts, scale, O);
+    dwn_hist_flush(hist, ld, c0, cend, L, (long long)NO * L, chunks, partial, gluts, scale, O);
 }
 
 // hist_tiled: the histogram alone, for gy that arrives tile-major ([B/64][N*O][64]).  Nothing has to be
@@ -656,7 +731,7 @@ __global__ __launch_bounds__(256) void dwn_bwd_hist_tiled(const float *__restric
         }
     }
     __syncthreads();
-    dwn_hist_flush(hist, c0, cend, L, (long long)NO * L, chunks, partial, gluts, nullptr, O);
+    dwn_hist_flush(&hist[0][0], 65, c0, cend, L, (long long)NO * L, chunks, partial, gluts, nullptr, O);
 }
 
 // ---------------------------------------------------------------------------------
@@ -695,11 +770,12 @@ __global__ __launch_bounds__(256) void dwn_bwd_gx(const float *__restrict__ gyT,
     for (int r = 0; r < WI; ++r) tile[wbeg + r][lane] = 0.0f;  // inputs nobody reads keep 0
     const int ebeg = __builtin_amdgcn_readlane(myptr, 0);
     const int eend = __builtin_amdgcn_readlane(myptr, WI);
+    constexpr int NR = !SFORM && Lh > 64 ? Lh / 64 : 1;  // registers of a coefficient row
     struct Group {
         int rj[DWN_EG], ri[DWN_EG];
         bool live[DWN_EG];
         unsigned a[DWN_EG];
-        float g[DWN_EG], coef[DWN_EG];
+        float g[DWN_EG], coef[DWN_EG][NR];
     };
     float acc = 0.0f;  // running sum of the input `cur`
     int cur = -1;
@@ -767,9 +843,11 @@ __global__ __launch_bounds__(256) void dwn_bwd_gx(const float *__restrict__ gyT,
                 if (O1) {
                     G.g[q] = gy_t[(size_t)rn * 64];
                     if (SFORM)
-                        G.coef[q] = D[(size_t)rn * (2 * Lh) + (lane & (2 * Lh - 1))];
+                        G.coef[q][0] = D[(size_t)rn * (2 * Lh) + (lane & (2 * Lh - 1))];
                     else
-                        G.coef[q] = D[((size_t)rn * K + G.rj[q]) * Lh + (lane & (Lh - 1))];
+#pragma unroll
+                        for (int r2 = 0; r2 < NR; ++r2)
+                            G.coef[q][r2] = D[((size_t)rn * K + G.rj[q]) * Lh + (lane & (Lh - 1)) + r2 * 64];
                 } else {
                     G.g[q] = __int_as_float(rn);  // node number; outputs are walked in evaluate()
                 }
@@ -783,11 +861,11 @@ __global__ __launch_bounds__(256) void dwn_bwd_gx(const float *__restrict__ gyT,
                 const unsigned ap = (G.a[q] & ((1u << j_) - 1u)) | ((G.a[q] >> (j_ + 1)) << j_);
                 float term;
                 if (O1 && SFORM) {
-                    const float hi = dl_lane_read(G.coef[q], (int)(G.a[q] | (1u << j_)));
-                    const float lo = dl_lane_read(G.coef[q], (int)(G.a[q] & ~(1u << j_)));
+                    const float hi = dl_lane_read(G.coef[q][0], (int)(G.a[q] | (1u << j_)));
+                    const float lo = dl_lane_read(G.coef[q][0], (int)(G.a[q] & ~(1u << j_)));
                     term = G.g[q] * (hi - lo);
                 } else if (O1) {
-                    term = G.g[q] * dl_lane_read(G.coef[q], (int)ap);
+                    term = G.g[q] * dwn_table_read<NR>(G.coef[q], ap);
                 } else {
                     const int rn = __float_as_int(G.g[q]);
                     term = 0.0f;
@@ -798,8 +876,10 @@ __global__ __launch_bounds__(256) void dwn_bwd_gx(const float *__restrict__ gyT,
                             term += gy_t[c * 64] * (dl_lane_read(coef, (int)(G.a[q] | (1u << j_))) -
                                                     dl_lane_read(coef, (int)(G.a[q] & ~(1u << j_))));
                         } else {
-                            const float coef = D[(c * K + j_) * Lh + (lane & (Lh - 1))];
-                            term += gy_t[c * 64] * dl_lane_read(coef, (int)ap);
+                            float coef[NR];
+#pragma unroll
+                            for (int r2 = 0; r2 < NR; ++r2) coef[r2] = D[(c * K + j_) * Lh + (lane & (Lh - 1)) + r2 * 64];
+                            term += gy_t[c * 64] * dwn_table_read<NR>(coef, ap);
                         }
                     }
                 }
@@ -1222,9 +1302,11 @@ static inline size_t dwn_gyT_bytes(int B, int N, int O) {
 }
 // grid of the histogram kernels: column tiles x chunks of batch tiles.  Enough blocks to fill 256 CUs several times
 // over; four blocks fit a CU (LDS), so at most about 1024 of them - all resident at once, no second, mostly empty round.
-static inline void dwn_hist_grid(long long NO, int BT, int &col_tiles, int &chunks, int &tpc) {
+// Wide tables' bins leave room for two blocks (k = 7) or one (k = 8), and a partial set of theirs is 2 or 4 times as long.
+static inline void dwn_hist_grid(long long NO, int k, int BT, int &col_tiles, int &chunks, int &tpc) {
     col_tiles = dl_ceil_div(NO, DWN_HC);
-    chunks = col_tiles >= 1024 ? 1 : 1024 / col_tiles;
+    const int blocks = k <= DL_MAX_FAST_K ? 1024 : (k == 7 ? 512 : 256);
+    chunks = col_tiles >= blocks ? 1 : blocks / col_tiles;
     if (chunks > BT) chunks = BT;
     tpc = dl_ceil_div(BT, chunks);
     chunks = dl_ceil_div(BT, tpc);
@@ -1238,11 +1320,12 @@ static inline void dwn_hist_grid(long long NO, int BT, int &col_tiles, int &chun
 #define DWN_ROW_CHUNK_BYTES 172e6  // gy tile-major + saved addresses of a chunk (the headline's 4096 rows: 168 MB)
 static inline int dwn_walk_rows(int BT, int I, int N, int k, int O, int gx_tiled);
 static inline int dwn_row_chunks(int BT, int I, int N, int k, int O) {
-    (void)I, (void)k;
+    (void)I;
     int tiles = (int)(DWN_ROW_CHUNK_BYTES / ((double)N * O * 320));
     if (tiles < 32) tiles = 32;  // (the walking gather wants 32 tiles)
     if (2 * BT < 3 * tiles) return 1;
-    if (dl_ceil_div((long long)N * O, DWN_HC) > 512) return 1;  // (a chunk's histogram must leave partial sets)
+    // (a chunk's histogram must leave partial sets)
+    if (dl_ceil_div((long long)N * O, DWN_HC) > (k <= DL_MAX_FAST_K ? 512 : (k == 7 ? 256 : 128))) return 1;
     return (BT + tiles / 2) / tiles;
 }
 // the tiles of chunk c of n: as even as they come (BT / n each, the first BT % n one more), so that no chunk is tiny
@@ -1255,12 +1338,12 @@ static inline size_t dwn_partial_bytes(int B, int I, int N, int k, int O) {
     if (n > 1) {
         size_t sets = 0;
         for (int c = 0; c < n; ++c) {
-            dwn_hist_grid((long long)N * O, dwn_row_chunk_tiles(BT, n, c), col_tiles, chunks, tpc);
+            dwn_hist_grid((long long)N * O, k, dwn_row_chunk_tiles(BT, n, c), col_tiles, chunks, tpc);
             sets += chunks;
         }
         return dl_align256(sets * N * O * sizeof(float) << k);
     }
-    dwn_hist_grid((long long)N * O, BT, col_tiles, chunks, tpc);
+    dwn_hist_grid((long long)N * O, k, BT, col_tiles, chunks, tpc);
     return chunks > 1 ? dl_align256((size_t)chunks * N * O * sizeof(float) << k) : 0;
 }
 
@@ -1284,17 +1367,23 @@ static inline bool dwn_fast(int N, int k, int O) {
     return k <= DL_MAX_FAST_K && N < (1 << 23) && (long long)N * O * ((long long)4 << k) < 0x7fffffffLL;
 }
 
+// the same for tables of 128 and 256 entries: single layers only, and only with the caller's saved and workspace arrays
+static inline bool dwn_wide(int N, int k, int O) {
+    return (k == 7 || k == 8) && N < (1 << 23) && (long long)N * O * ((long long)4 << k) < 0x7fffffffLL;
+}
+static inline bool dwn_lanes(int N, int k, int O) { return dwn_fast(N, k, O) || dwn_wide(N, k, O); }
+
 extern "C" size_t dl_dwn_saved_bytes(int B, int I, int N, int k, int O) {
     (void)I;
-    if (!dwn_fast(N, k, O)) return 256;  // nothing is kept; a token allocation keeps callers simple
+    if (!dwn_lanes(N, k, O)) return 256;  // nothing is kept; a token allocation keeps callers simple
     return dl_align256((size_t)N * dwn_bt(B) * 64);
 }
 extern "C" size_t dl_dwn_fwd_workspace_bytes(int B, int I, int N, int k, int O) {
-    return dwn_fast(N, k, O) ? dwn_planes_bytes(B, I) : 256;
+    return dwn_lanes(N, k, O) ? dwn_planes_bytes(B, I) : 256;
 }
 extern "C" size_t dl_dwn_bwd_workspace_bytes(int B, int I, int N, int k, int O) {
-    return dwn_fast(N, k, O) ? dwn_table_bytes(N, k, O) + dwn_gyT_bytes(B, N, O) + dwn_partial_bytes(B, I, N, k, O)
-                             : dl_align256(dwn_generic_smooth_bytes(N, k, O));  // k > 6: the smoothed tables
+    return dwn_lanes(N, k, O) ? dwn_table_bytes(N, k, O) + dwn_gyT_bytes(B, N, O) + dwn_partial_bytes(B, I, N, k, O)
+                              : dl_align256(dwn_generic_smooth_bytes(N, k, O));  // k > 8: the smoothed tables
 }
 
 template <int K>
@@ -1336,7 +1425,15 @@ static void dwn_launch_lookup(const u64 *planes, const int *idx32, const float *
 #undef DWN_LOOKUP
 }
 
-// forward of the k <= 6 path: x -> bit-planes (scratch) -> y and the saved addresses
+template <int K>
+static void dwn_launch_lookup_wide(const u64 *planes, const int *idx32, const float *luts, float *y, uint8_t *addrT, int B,
+                                   int I, int N, int O, hipStream_t s) {
+    const int BT = dwn_bt(B), grid = dl_xcd_grid(dl_ceil_div((long long)N * O, DWN_TC), BT);
+    if (O == 1) DL_TIMED("dwn_lookup_fwd", s, (dwn_lookup_fwd<K, true><<<grid, 64 * DWN_FW, 0, s>>>(planes, idx32, luts, y, addrT, nullptr, B, I, N, O, BT)));
+    else DL_TIMED("dwn_lookup_fwd", s, (dwn_lookup_fwd<K, false><<<grid, 64 * DWN_FW, 0, s>>>(planes, idx32, luts, y, addrT, nullptr, B, I, N, O, BT)));
+}
+
+// forward of the k <= 8 path: x -> bit-planes (scratch) -> y and the saved addresses
 static int dwn_forward_fast(const float *x, const int32_t *idx32, const float *luts, float *y, void *saved, u64 *planes,
                             int B, int I, int N, int k, int O, hipStream_t s) {
     const int BT = dwn_bt(B);
@@ -1351,9 +1448,18 @@ static int dwn_forward_fast(const float *x, const int32_t *idx32, const float *l
         case 3: dwn_launch_lookup<3>(planes, idx32, luts, y, addrT, nullptr, B, I, N, O, s); break;
         case 4: dwn_launch_lookup<4>(planes, idx32, luts, y, addrT, nullptr, B, I, N, O, s); break;
         case 5: dwn_launch_lookup<5>(planes, idx32, luts, y, addrT, nullptr, B, I, N, O, s); break;
+        case 7: dwn_launch_lookup_wide<7>(planes, idx32, luts, y, addrT, B, I, N, O, s); break;
+        case 8: dwn_launch_lookup_wide<8>(planes, idx32, luts, y, addrT, B, I, N, O, s); break;
         default: dwn_launch_lookup<6>(planes, idx32, luts, y, addrT, nullptr, B, I, N, O, s); break;
     }
     return dl_launch_status();
+}
+
+// Any other forward.  What a backward of k = 7 or 8 would read from `saved` is written whenever the caller brings it.
+static int dwn_forward_generic(const float *x, const int32_t *idx32, const float *luts, float *y, void *saved, int B, int I, int N,
+                               int k, int O, hipStream_t s) {
+    const int rc = dwn_generic_forward(x, idx32, luts, y, B, I, N, k, O, s);
+    return rc || !saved || !dwn_wide(N, k, O) ? rc : dwn_generic_addresses(x, idx32, (uint8_t *)saved, B, I, N, k, s);
 }
 
 extern "C" int dl_dwn_layer_fwd(const float *x, const int32_t *idx32, const float *luts, float *y, void *saved,
@@ -1362,7 +1468,11 @@ extern "C" int dl_dwn_layer_fwd(const float *x, const int32_t *idx32, const floa
     int rc = dwn_check(B, I, N, k, O);
     if (rc) return rc;
     hipStream_t s = (hipStream_t)stream;
-    if (!dwn_fast(N, k, O)) return dwn_generic_forward(x, idx32, luts, y, B, I, N, k, O, s);
+    if (!dwn_fast(N, k, O)) {
+        if (dwn_wide(N, k, O) && saved && ws && ws_bytes >= dl_dwn_fwd_workspace_bytes(B, I, N, k, O))
+            return dwn_forward_fast(x, idx32, luts, y, saved, (u64 *)ws, B, I, N, k, O, s);
+        return dwn_forward_generic(x, idx32, luts, y, saved, B, I, N, k, O, s);
+    }
     if (!saved || !ws) return DL_ERR_NULL;
     if (ws_bytes < dl_dwn_fwd_workspace_bytes(B, I, N, k, O)) return DL_ERR_WORKSPACE;
     return dwn_forward_fast(x, idx32, luts, y, saved, (u64 *)ws, B, I, N, k, O, s);
@@ -1400,7 +1510,8 @@ extern "C" int dl_dwn_layer_fwd_static(const float *x, const int32_t *idx32, con
     int rc = dwn_check(B, I, N, k, O);
     if (rc) return rc;
     hipStream_t s = (hipStream_t)stream;
-    if (!dwn_fast(N, k, O)) return dwn_generic_forward(x, idx32, luts, y, B, I, N, k, O, s);  // uses no scratch
+    if (!dwn_fast(N, k, O) && !(dwn_wide(N, k, O) && saved && dwn_planes_bytes(B, I) <= (size_t)DL_DWN_STATIC_SCRATCH_BYTES))
+        return dwn_forward_generic(x, idx32, luts, y, saved, B, I, N, k, O, s);  // uses no scratch
     if (!saved) return DL_ERR_NULL;
     if (dwn_planes_bytes(B, I) > (size_t)DL_DWN_STATIC_SCRATCH_BYTES) return DL_ERR_SCRATCH;
     void *planes = nullptr;
@@ -1442,7 +1553,18 @@ static void dwn_launch_gx(const float *gyT, const uint8_t *addrT, const float *D
 #undef DWN_GX
 }
 
-// backward of the k <= 6 path; gy row-major [B, N*O] or (gy_tiled) tile-major [B/64][N*O][64];
+template <int K>
+static void dwn_launch_gx_wide(const float *gyT, const uint8_t *addrT, const float *D, const int *inv_ptr, const int *inv_pos,
+                               float *gx, int B, int I, int N, int O, const DwnReduce &red, hipStream_t s) {
+    const int BT = dwn_bt(B), rb = dwn_reduce_blocks(red);
+#define DWN_GX(O1_, WI_)                                                                                                 do {                                                                                                                     const int grid = dl_xcd_grid(dl_ceil_div(I, 4 * WI_), BT);                                                           DL_TIMED("dwn_bwd_gx", s, (dwn_bwd_gx<K, O1_, false, WI_><<<grid + rb, 256, 0, s>>>(                                                               gyT, addrT, D, inv_ptr, inv_pos, gx, B, I, N, O, BT, 0, grid, red)));              } while (0)
+    if (O == 1 && (long long)N * K >= 6LL * I) DWN_GX(true, DWN_WI_SMALL);  // the rule of dwn_launch_gx
+    else if (O == 1) DWN_GX(true, DWN_WI);
+    else DWN_GX(false, DWN_WI);
+#undef DWN_GX
+}
+
+// backward of the k <= 8 path (k > 6: row-major, no head, nothing fused); gy row-major [B, N*O] or (gy_tiled) tile-major [B/64][N*O][64];
 // gx row-major [B, I] or (gx_tiled) tile-major [B/64][I][64]
 // scale == null: EFD weights alpha * beta^h; otherwise the stabilised weights scale[n] / (h + 1),
 // which also multiply the table gradient
@@ -1552,7 +1674,7 @@ static int dwn_backward_fast(const void *saved, const int32_t *inv_ptr, const in
         if (n > 1) {  // in chunks of rows, each through this function again
             int total = 0, sets = 0;
             for (int c = 0; c < n; ++c) {
-                dwn_hist_grid(NO, dwn_row_chunk_tiles(BT, n, c), col_tiles, chunks, tpc);
+                dwn_hist_grid(NO, k, dwn_row_chunk_tiles(BT, n, c), col_tiles, chunks, tpc);
                 total += chunks;
             }
             for (int c = 0; c < n; ++c) {
@@ -1563,28 +1685,34 @@ static int dwn_backward_fast(const void *saved, const int32_t *inv_ptr, const in
                                                     alpha, beta, scale, gx + (size_t)t0 * 64 * I, 0, gluts, ws, rows, I, N, k, O, s,
                                                     nullptr, alpha_n, beta_n, nullptr, &r);
                 if (rcode) return rcode;
-                dwn_hist_grid(NO, tiles, col_tiles, chunks, tpc);
+                dwn_hist_grid(NO, k, tiles, col_tiles, chunks, tpc);
                 sets += chunks;
             }
             return DL_OK;
         }
     }
     if (rc) partial = rc->partial_base + (size_t)rc->set_offset * NO * L;
-    dwn_hist_grid(NO, BT, col_tiles, chunks, tpc);
-    const bool sform = !scale && beta >= -0.5f && beta <= 0.5f;
+    dwn_hist_grid(NO, k, BT, col_tiles, chunks, tpc);
+    const bool wide = k > DL_MAX_FAST_K;
+    const bool sform = !wide && !scale && beta >= -0.5f && beta <= 0.5f;
     // The coefficient tables of the gather depend on the tables only, so their blocks ride in the histogram's launch
     // (extra rows of its grid, dispatched last: they fill the tail in which the histogram blocks drain); the
     // fixed-order sum of the histogram partials rides in the gather's launch the same way.
     // the walking gather of a layer too wide for one XCD's resident blocks packs two D-form rows into a register; for
     // |beta| <= 1/2 its table then holds the differences of the S form (the bits the other gathers compute from it)
-    const int walk_rows = gx ? dwn_walk_rows(BT, I, N, k, O, gx_tiled) : 0;
+    const int walk_rows = gx && !wide ? dwn_walk_rows(BT, I, N, k, O, gx_tiled) : 0;
     const bool walk_pack = walk_rows == 6 || (walk_rows == 3 && dl_ceil_div(I, 4 * DWN_WI) > DWN_RESIDENT);
     const bool gather = gx || prev;  // (prev without gx: the input gradient is summed for the bins in front, not stored)
     const int fused_wi = prev && (gx_tiled || !gx) && O == 1 && sform ? dwn_fused_wi(I, N, k) : 0;
     const bool fused_pack = fused_wi && dwn_fused_pack(I, N, k);
     DwnTables tb = {gather && (!rc || rc->first) ? luts : nullptr, D, scale, alpha_n, beta_n, alpha, beta, (int)NO, k, O,
                     sform ? (walk_pack || fused_pack ? 2 : 1) : 0};
+    if (wide && tb.luts) {
+        DL_TIMED("dwn_wide_tables", s, (dwn_wide_tables<<<(unsigned)NO, 256, 0, s>>>(tb)));
+        tb.luts = nullptr;
+    }
     const dim3 hgrid(col_tiles, chunks + dl_ceil_div(dwn_table_blocks(tb), col_tiles));
+    const size_t wide_bins = (size_t)DWN_HC * (L + 1) * sizeof(float);
     if (!gluts) {
         // the table gradient of this layer is already there (the gather of the layer behind filled its bins): only the
         // coefficient tables remain to be built.  gy is tile-major in that case.
@@ -1596,7 +1724,18 @@ static int dwn_backward_fast(const void *saved, const int32_t *inv_ptr, const in
     else if (gy_tiled)
         DL_TIMED("dwn_bwd_hist_tiled", s,
                  (dwn_bwd_hist_tiled<false><<<hgrid, 256, 0, s>>>(gy, addrT, gluts, (int)NO, O, L, BT, tpc, partial, chunks, tb)));
-    else if (gather)
+    else if (wide) {
+        const void *fn = gather ? reinterpret_cast<const void *>(&dwn_bwd_transpose_hist<true, true>)
+                                : reinterpret_cast<const void *>(&dwn_bwd_transpose_hist<false, true>);
+        const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)wide_bins);
+        if (e != hipSuccess) return (int)e;
+        if (gather)
+            DL_TIMED("dwn_bwd_transpose_hist", s, (dwn_bwd_transpose_hist<true, true><<<hgrid, 256, wide_bins, s>>>(
+                                                      gy, addrT, gyT, gluts, B, (int)NO, O, L, BP, BT, tpc, partial, scale, chunks, tb)));
+        else
+            DL_TIMED("dwn_bwd_transpose_hist", s, (dwn_bwd_transpose_hist<false, true><<<hgrid, 256, wide_bins, s>>>(
+                                                      gy, addrT, gyT, gluts, B, (int)NO, O, L, BP, BT, tpc, partial, scale, chunks, tb)));
+    } else if (gather)
         DL_TIMED("dwn_bwd_transpose_hist", s, (dwn_bwd_transpose_hist<true><<<hgrid, 256, 0, s>>>(
                                                   gy, addrT, gyT, gluts, B, (int)NO, O, L, BP, BT, tpc, partial, scale, chunks, tb)));
     else
@@ -1700,6 +1839,8 @@ static int dwn_backward_fast(const void *saved, const int32_t *inv_ptr, const in
             case 3: dwn_launch_gx<3>(src, addrT, D, inv_ptr, inv_pos, gx, B, I, N, O, sform, gx_tiled, red, s); break;
             case 4: dwn_launch_gx<4>(src, addrT, D, inv_ptr, inv_pos, gx, B, I, N, O, sform, gx_tiled, red, s); break;
             case 5: dwn_launch_gx<5>(src, addrT, D, inv_ptr, inv_pos, gx, B, I, N, O, sform, gx_tiled, red, s); break;
+            case 7: dwn_launch_gx_wide<7>(src, addrT, D, inv_ptr, inv_pos, gx, B, I, N, O, red, s); break;
+            case 8: dwn_launch_gx_wide<8>(src, addrT, D, inv_ptr, inv_pos, gx, B, I, N, O, red, s); break;
             default: dwn_launch_gx<6>(src, addrT, D, inv_ptr, inv_pos, gx, B, I, N, O, sform, gx_tiled, red, s); break;
         }
     }
@@ -1718,7 +1859,7 @@ extern "C" int dl_dwn_layer_bwd(const float *x, const void *saved, const int32_t
     int rc = dwn_check(B, I, N, k, O);
     if (rc) return rc;
     hipStream_t s = (hipStream_t)stream;
-    if (!dwn_fast(N, k, O)) {
+    if (!dwn_fast(N, k, O) && !(dwn_wide(N, k, O) && saved && ws && ws_bytes >= dl_dwn_bwd_workspace_bytes(B, I, N, k, O))) {
         if (!x) return DL_ERR_NULL;
         return dwn_generic_backward(x, idx32, inv_ptr, inv_pos, luts, gy, alpha, beta, nullptr, gx, gluts, B, I, N, k, O, s,
                                     nullptr, nullptr, fabsf(beta), ws, ws_bytes);
@@ -1739,7 +1880,7 @@ extern "C" int dl_dwn_layer_bwd_nodes(const float *x, const void *saved, const i
     int rc = dwn_check(B, I, N, k, O);
     if (rc) return rc;
     hipStream_t s = (hipStream_t)stream;
-    if (!dwn_fast(N, k, O)) {
+    if (!dwn_fast(N, k, O) && !(dwn_wide(N, k, O) && saved && ws && ws_bytes >= dl_dwn_bwd_workspace_bytes(B, I, N, k, O))) {
         if (!x) return DL_ERR_NULL;
         return dwn_generic_backward(x, idx32, inv_ptr, inv_pos, luts, gy, 0.0f, 0.0f, nullptr, gx, gluts, B, I, N, k, O, s,
                                     alpha_n, beta_n, beta_abs_max, ws, ws_bytes);
@@ -1760,7 +1901,7 @@ extern "C" int dl_dwn_stable_layer_bwd(const float *x, const void *saved, const 
     int rc = dwn_check(B, I, N, k, O);
     if (rc) return rc;
     hipStream_t s = (hipStream_t)stream;
-    if (!dwn_fast(N, k, O)) {
+    if (!dwn_fast(N, k, O) && !(dwn_wide(N, k, O) && saved && ws && ws_bytes >= dl_dwn_bwd_workspace_bytes(B, I, N, k, O))) {
         if (!x) return DL_ERR_NULL;
         return dwn_generic_backward(x, idx32, inv_ptr, inv_pos, luts, gy, 0.0f, 0.0f, gradient_scale, gx, gluts, B, I, N, k,
                                     O, s);

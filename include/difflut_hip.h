@@ -84,7 +84,7 @@ int dl_gather_bwd(const float *gm, const int32_t *inv_ptr, const int32_t *inv_po
  *   y     [B,N*O]
  * Training forward: addr = sum_j [x[b,idx[n,j]] >= 0.5] << j;  y[b,n,d] = luts[n,d,addr].
  * `saved` (dl_dwn_saved_bytes) receives what the backward needs instead of x:
- * for k <= DL_MAX_FAST_K the address of every (node, row), node-major.
+ * for k <= 8 the address of every (node, row), node-major.
  * `ws` (dl_dwn_fwd_workspace_bytes) is scratch that may be reused after the call.
  * ------------------------------------------------------------------------ */
 size_t dl_dwn_saved_bytes(int B, int I, int N, int k, int O);
@@ -99,7 +99,7 @@ int dl_dwn_layer_fwd(const float *x, const int32_t *idx32, const float *luts, fl
  * dl_dwn_layer_fwd puts into `ws` go to a device array owned by the library instead
  * (DL_DWN_STATIC_SCRATCH_BYTES on every GPU the library runs on, held until the process ends).  The call
  * allocates and frees nothing.  Limit: ceil(B/64) * I * 8 <= DL_DWN_STATIC_SCRATCH_BYTES when
- * k <= DL_MAX_FAST_K (e.g. B = 4096 with I = 16384), otherwise DL_ERR_SCRATCH; larger k uses no scratch.
+ * k <= DL_MAX_FAST_K (e.g. B = 4096 with I = 16384), otherwise DL_ERR_SCRATCH; larger k does without it.
  * All calls on one GPU share that GPU's array: calls that overlap on one GPU (two streams, two threads)
  * race on it and must be serialised by the caller.  Nothing in it has to survive between calls.
  * The first call on each device also looks up the device address of the array (hipGetSymbolAddress, which may
@@ -113,10 +113,11 @@ int dl_dwn_layer_fwd_static(const float *x, const int32_t *idx32, const float *l
  *                 sum_kappa s(kappa_j) luts[n,d,kappa] beta^popc((addr ^ kappa) & ~(1<<j))
  *   gluts[n,d,e] = sum_b [addr(b,n) = e] gy[b,n,d]
  * gx may be null (input does not need a gradient); gx and gluts are overwritten.
- * x is only read when k > DL_MAX_FAST_K (then `saved` is unused) and may be null otherwise.  For k > DL_MAX_FAST_K the
- * workspace is optional (ws may be null): with dl_dwn_bwd_workspace_bytes of it, |beta| <= 1/2 and k <= 12 the input
- * gradient is taken from tables smoothed once per call (two loads per row and connection); without, from the 2^k-term
- * sum of the formula per row and connection.  The table gradient of that path is summed with atomics. */
+ * k <= DL_MAX_FAST_K: x is not read and may be null.  k = 7, 8: with `saved` as the forward wrote it (every forward given a
+ * `saved` does) and dl_dwn_bwd_workspace_bytes of workspace the same kernels run and x is not read; without either, and for
+ * k > 8, x is read and `saved` is not.  Then the workspace is optional (ws may be null): with it, |beta| <= 1/2 and
+ * k <= 12 the input gradient is taken from tables smoothed once per call (two loads per row and connection); without, from
+ * the 2^k-term sum of the formula per row and connection.  The table gradient of that path is summed with atomics. */
 int dl_dwn_layer_bwd(const float *x, const void *saved, const int32_t *idx32,
                      const int32_t *inv_ptr, const int32_t *inv_pos,
                      const float *luts, const float *gy, float alpha, float beta,

@@ -338,6 +338,47 @@ def test_dwn_backward_more_than_six_inputs(shape, beta):
     np.testing.assert_allclose(lt.grad.cpu().numpy(), gl, rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("k", [7, 8])
+@pytest.mark.parametrize("B,I,N,O", [(64, 128, 64, 1),    # whole tiles
+                                     (65, 131, 65, 2),    # one past a batch tile and a column tile
+                                     (1000, 48, 140, 1),  # lists of about 20 entries per input; several chunks of tiles
+                                     (130, 700, 129, 1)])
+def test_dwn_tables_of_more_than_one_register(B, I, N, O, k):
+    """k = 7 and 8: EFD with small and large |beta| (two ways to build the coefficient rows) and the gradient-stabilised
+    node, against the oracle; and the forward without a workspace leaves the same addresses.  Coefficients are built in double
+    and rounded once: rtol 1e-5 with a floor of 1e-6 of the largest gradient."""
+    ops = _ops()
+    from difflut_amd import _native as nat
+    x, idx, luts, gy = make_case(B + I + N + k, B, I, N, k, O)
+    plan = ops.MappingPlan(dev(idx, torch.int32), I)
+    want = orc.dwn_layer_forward(x, idx, luts)
+    for beta in (1.0 / 3.0, 0.9):
+        xt = dev(x).requires_grad_(); lt = dev(luts).requires_grad_()
+        y = ops.DWNLayerFunction.apply(xt, lt, plan, 0.3, beta)
+        assert np.array_equal(y.detach().cpu().numpy().reshape(B, N, O), want)
+        y.backward(dev(gy.reshape(B, -1)))
+        gx, gl = orc.dwn_layer_backward(x, idx, luts, gy, np.float32(0.3), np.float32(beta))
+        np.testing.assert_allclose(xt.grad.cpu().numpy(), gx, rtol=1e-5, atol=1e-6 * float(np.abs(gx).max()))
+        np.testing.assert_allclose(lt.grad.cpu().numpy(), gl, rtol=1e-5, atol=1e-5)
+    scale = np.linspace(0.5, 1.5, N).astype(np.float32)
+    xt = dev(x).requires_grad_(); lt = dev(luts).requires_grad_()
+    ops.DWNStableLayerFunction.apply(xt, ops.table_sigmoid(lt), dev(scale), plan).backward(dev(gy.reshape(B, -1)))
+    gx, gl = orc.stable_layer_backward(x, idx, luts, gy, scale)  # luts as the raw tables
+    np.testing.assert_allclose(xt.grad.cpu().numpy(), gx, rtol=1e-5, atol=1e-6 * float(np.abs(gx).max()))
+    np.testing.assert_allclose(lt.grad.cpu().numpy(), gl, rtol=1e-5, atol=1e-5)
+    lib, dims = nat.lib(), (B, I, N, k, O)
+    xd, ld, bt = dev(x), dev(luts), (B + 63) // 64
+    saved = torch.empty(2, lib.dl_dwn_saved_bytes(*dims), dtype=torch.uint8, device="cuda")
+    ws = torch.empty(lib.dl_dwn_fwd_workspace_bytes(*dims), dtype=torch.uint8, device="cuda")
+    y = torch.empty(B, N * O, device="cuda")
+    for q, w in enumerate((ws, None)):
+        nat.check(lib.dl_dwn_layer_fwd(nat.ptr(xd), nat.ptr(plan.idx32), nat.ptr(ld), nat.ptr(y), nat.ptr(saved[q]), nat.ptr(w),
+                                       0 if w is None else w.numel(), *dims, nat.stream()))
+        assert np.array_equal(y.cpu().numpy().reshape(B, N, O), want)
+    got = saved[:, :bt * N * 64].view(2, bt, N, 64).permute(0, 1, 3, 2).reshape(2, bt * 64, N)[:, :B]
+    assert torch.equal(got[0], got[1])
+
+
 def test_dwn_no_input_grad_and_unused_inputs():
     ops = _ops()
     B, I, N, k, O = 40, 50, 3, 2, 1  # 44 of the 50 inputs feed no node: their gradient must be 0
