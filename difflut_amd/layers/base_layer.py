@@ -71,6 +71,15 @@ class BankedParameter(nn.Parameter):
         return (nn.Parameter, (self.data.clone(), self.requires_grad))
 
 
+def _node_getter(nodes):
+    """row -> node without ModuleList.__getitem__, whose index arithmetic costs more than the checks below (they run on
+    every call of a layer).  Looks the node up anew each time, so a replaced node is seen."""
+    if not isinstance(nodes, nn.ModuleList):
+        return nodes.__getitem__
+    modules, keys = nodes._modules, [str(row) for row in range(len(nodes))]
+    return lambda row: modules[keys[row]]
+
+
 class ParameterBank:
     """The parameter `name` of N nodes as one leaf tensor [N, *shape]."""
 
@@ -78,6 +87,7 @@ class ParameterBank:
         self.nodes, self.name = nodes, name
         self.flat = None
         self._stale = False  # set when another bank takes over one of my nodes, or a node's parameter is reassigned
+        self._count = self._row_bytes = 0
         self.tie()
 
     def tie(self, keep_grad=None):
@@ -94,17 +104,22 @@ class ParameterBank:
         view = flat.detach()
         for row, node in enumerate(self.nodes):
             node._parameters[self.name] = BankedParameter(view[row], self, row)
+        self._count = len(params)
+        self._row_bytes = flat[0].numel() * flat.element_size()
+        self._node = _node_getter(self.nodes)
         self._stale = False
 
+    def __getstate__(self):
+        return {k: v for k, v in self.__dict__.items() if k != "_node"}  # tie() makes it again
+
     def tied(self):
-        if self._stale:
+        if self._stale or len(self.nodes) != self._count:
             return False
-        first = self.nodes[0]._parameters[self.name]
-        last = self.nodes[-1]._parameters[self.name]
-        step = self.flat[0].numel() * self.flat.element_size()
+        first = self._node(0)._parameters[self.name]
+        last = self._node(self._count - 1)._parameters[self.name]
         base = self.flat.data_ptr()
         return (isinstance(first, BankedParameter) and first._bank is self and first.device == self.flat.device
-                and first.data_ptr() == base and last.data_ptr() == base + step * (len(self.nodes) - 1))
+                and first.data_ptr() == base and last.data_ptr() == base + self._row_bytes * (self._count - 1))
 
     def tensor(self):
         if not self.tied():
@@ -140,10 +155,14 @@ class ScalarBank:
             view._scalar_bank = self
             node._buffers[self.name] = view
             self._views.append(view)
+        self._node = _node_getter(self.nodes)
         self._stale, self._key = False, None
 
+    def __getstate__(self):
+        return {k: v for k, v in self.__dict__.items() if k != "_node"}  # tie() makes it again
+
     def _is_view(self, row):
-        return self.nodes[row]._buffers[self.name] is self._views[row]
+        return self._node(row)._buffers[self.name] is self._views[row]
 
     def tied(self):
         """Every node's buffer is still the view handed out by tie().  All nodes are checked on small layers; on large
@@ -152,11 +171,18 @@ class ScalarBank:
         if self._stale or not self._views or self._views[0].device != self.flat.device:
             return False
         n = len(self.nodes)
+        if n != len(self._views):
+            return False
         if n <= 4 * self._PROBES:
-            return all(self._is_view(row) for row in range(n))
-        rows = [0, n - 1] + [(self._probe + i) % n for i in range(self._PROBES)]
-        self._probe = (self._probe + self._PROBES) % n
-        return all(self._is_view(row) for row in rows)
+            rows = range(n)
+        else:
+            rows = [0, n - 1] + [(self._probe + i) % n for i in range(self._PROBES)]
+            self._probe = (self._probe + self._PROBES) % n
+        node, name, views = self._node, self.name, self._views
+        for row in rows:
+            if node(row)._buffers[name] is not views[row]:
+                return False
+        return True
 
     def tensor(self):
         """The float32 device array [N] for the kernels (the bank itself when it is float32)."""
@@ -170,7 +196,16 @@ class ScalarBank:
         self._key = None
 
     def abs_max(self):
-        flat = self.tensor()
+        self.tensor()
+        return self._known_abs_max()
+
+    def tensor_and_abs_max(self):
+        """Both from one check of the nodes."""
+        values = self.tensor()
+        return values, self._known_abs_max()
+
+    def _known_abs_max(self):
+        flat = self.flat
         key = (self.flat._version, self.flat.data_ptr())
         if key != self._key:
             self._abs_max = float(flat.detach().abs().max())
@@ -323,7 +358,7 @@ class BaseLUTLayer(ABC, LUTLayerMixin, nn.Module):
         """(alpha [N], beta [N], max |beta|) of a DWN layer for the kernels: the nodes' own values as float32 device
         arrays (every call reads the nodes' current values, dwn_node.py:450) and the host value that selects the form
         of the coefficient table."""
-        return self._scalars["alpha"].tensor(), self._scalars["beta"].tensor(), self._scalars["beta"].abs_max()
+        return (self._scalars["alpha"].tensor(), *self._scalars["beta"].tensor_and_abs_max())
 
     def temperatures(self):
         """The nodes' temperatures [N] as a float32 device array (probabilistic_node.py:277-282 reads each node's)."""

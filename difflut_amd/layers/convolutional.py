@@ -148,7 +148,7 @@ class ConvolutionalLayer(LUTLayerMixin, nn.Module):
         the nodes of all its sub-layers): DWN (alpha [nodes], beta [nodes], max |beta|), probabilistic temperature [nodes]."""
         banks = self._level_scalar_banks[level]
         if self._kind == "dwn":
-            return banks["alpha"].tensor(), banks["beta"].tensor(), banks["beta"].abs_max()
+            return (banks["alpha"].tensor(), *banks["beta"].tensor_and_abs_max())
         return banks["temperature"].tensor()
 
     def invalidate_scalars(self):

@@ -17,7 +17,7 @@ FAST_K = 6
 
 
 def _f32(t):
-    return t.contiguous().float()
+    return t if t.dtype is torch.float32 and t.is_contiguous() else t.contiguous().float()
 
 
 def _bytes(n, device):
