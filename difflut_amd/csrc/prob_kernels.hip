@@ -16,16 +16,15 @@ typedef float prob_f4 __attribute__((ext_vector_type(4)));
 // k <= 6 path.  As for the DWN nodes, a wavefront's 64 lanes are 64 batch rows and everything
 // that belongs to a node is wave-uniform: its input indices are scalar byte offsets, its sigmoid
 // table is read through scalar loads.  Tensors that cross the [batch, feature] boundary are
-// re-tiled once: xT [B/64][I][64], gyT [B/64][N*O][64], gmT [B/64][N*O*k][64], so the row of an
+// re-tiled once: xT [B/64][I][64], gmT [B/64][N*O*k][64], so the row of an
 // input (or a column's gradient) for a batch tile is 256 contiguous bytes, whatever the mapping.
 //   sig_table   : sig[c][a] = sigmoid(raw[n,a,d] / T), c = n*O + d                (tiny)
-//   to_tiles    : [B][C] -> [B/64][C][64], rows past B are zero        (x; gy only for k > 5, see bwd_t)
+//   to_tiles    : [B][C] -> [B/64][C][64], rows past B are zero
 //   fwd_t       : per (column, batch tile): fold the table along x_0, x_1, ... ; y leaves through
 //                 an LDS transpose as whole rows
-//   bwd_t       : one wavefront per column over a chunk of batch tiles.  The fold is run forward
-//                 keeping the differences of every level, then backward: that gives dy/dx_j for
-//                 all j and, at the bottom, p_a = dy/dtable_a (the product weights) in about
-//                 5 * 2^k operations.  Table-gradient partials stay in registers over the chunk,
+//   bwd_t       : one wavefront per column over a chunk of batch tiles.  The product weights factor into those of
+//                 the lower and of the upper inputs; that gives dy/dx_j for all j and the table gradient in about
+//                 3 * 2^k operations.  Table-gradient partials stay in registers over the chunk,
 //                 are summed across lanes once and written per chunk; gm_j goes to gmT.
 //   reduce      : fixed-order sum of the chunk partials, times sigmoid'(w/T)/T
 //   gather_t    : gx[b,i] = sum over the CSR entries (n,j) of input i (and d) of gmT: a wavefront
@@ -184,26 +183,86 @@ __global__ __launch_bounds__(64 * PROB_FW) void prob_fwd_t(const float *__restri
     }
 }
 
-// one wavefront per (column, chunk of batch tiles); W wavefronts per block.
+// 1 / d to about half a unit of the last place: the hardware reciprocal and one Newton step
+__device__ __forceinline__ float prob_rcp(float d) {
+    const float r = __builtin_amdgcn_rcpf(d);
+    return fmaf(r, fmaf(-d, r, 1.0f), r);
+}
+// u[a] = product over the inputs j of (x_j if bit j of a is set, else 1 - x_j)
+template <int KH>
+__device__ __forceinline__ void prob_products(const float *x, const float *om, float (&u)[1 << KH]) {
+    u[0] = 1.0f;
+#pragma unroll
+    for (int j = 0; j < KH; ++j)
+#pragma unroll
+        for (int a = (1 << j) - 1; a >= 0; --a) {
+            u[a | (1 << j)] = u[a] * x[j];
+            u[a] = u[a] * om[j];
+        }
+}
+// dx[j] = d/dx_j of the multilinear interpolation of v at x
+template <int KH>
+__device__ __forceinline__ void prob_fold_gradient(const float (&v0)[1 << KH], const float *x, const float *om, float *dx) {
+    constexpr int L = 1 << KH;
+    float diff[L - 1];  // level j occupies [L - (L >> j), L - (L >> (j + 1)))
+    float v[L];
+#pragma unroll
+    for (int a = 0; a < L; ++a) v[a] = v0[a];
+    int base = 0;
+#pragma unroll
+    for (int j = 0; j < KH; ++j) {
+#pragma unroll
+        for (int a = 0; a < (L >> (j + 1)); ++a) {
+            diff[base + a] = v[2 * a + 1] - v[2 * a];
+            v[a] = fmaf(x[j], diff[base + a], v[2 * a]);
+        }
+        base += L >> (j + 1);
+    }
+    // bar_KH[0] = 1; dx_j = sum_a bar_{j+1}[a] d_j[a]; bar_j[2a] = bar_{j+1}[a] (1 - x_j), bar_j[2a+1] = bar_{j+1}[a] x_j
+    float bar[L];
+    bar[0] = 1.0f;
+#pragma unroll
+    for (int j = KH - 1; j >= 0; --j) {
+        const int cnt = L >> (j + 1);
+        base -= cnt;
+        float sum = 0.0f;
+#pragma unroll
+        for (int a = 0; a < cnt; ++a) sum = fmaf(bar[a], diff[base + a], sum);
+        dx[j] = sum;
+        if (j > 0) {
+#pragma unroll
+            for (int a = cnt - 1; a >= 0; --a) {
+                const float w = bar[a];
+                bar[2 * a + 1] = w * x[j];
+                bar[2 * a] = w * om[j];
+            }
+        }
+    }
+}
+
+// one wavefront per (column, chunk of batch tiles); sixteen wavefronts, i.e. sixteen columns, per block.
 // HYB (hybrid node): the table is used as given and the input gradient carries the factor
 // q / (q + 1e-8), q = x_j (1 - x_j), of that node's backward.
-// W = 4: gy arrives tile-major (gyT [B/64][N*O][64], written by prob_to_tiles).  W = 16 (k <= 5, where 16 wavefronts
-// of this kernel fit a CU's registers): gy is the row-major gradient itself; the block's 16 columns are 64 contiguous
-// bytes of a row, the 64 x 16 piece of a batch tile is fetched one value per thread a tile ahead and turned through
-// the LDS (two buffers, one barrier per tile), so the re-tiling pass and its launch are not needed.
-template <int K, bool HYB, int W = 4>
-__global__ __launch_bounds__(64 * W) void prob_bwd_t(const float *__restrict__ xT, const float *__restrict__ gyT,
-                                                     const int *__restrict__ idx32, const float *__restrict__ sig,
-                                                     float *__restrict__ gmT, float *__restrict__ gpart, int I, int N,
-                                                     int O, int BT, int tiles_per_chunk, int want_gm, int B = 0) {
-    constexpr int L = 1 << K;
-    constexpr bool GYROW = W == 16;
-    __shared__ float gturn[GYROW ? 2 : 1][GYROW ? W : 1][GYROW ? 65 : 1];  // [buffer][column][row]
+// The weight of table entry a is a product over the inputs, so it factors into one over the lower KL and one over the upper
+// KU inputs, p[lo, hi] = u[lo] w[hi]: with V[lo] = sum_hi T[lo, hi] w[hi] and Z[hi] = sum_lo T[lo, hi] u[lo] the gradients
+// of the lower inputs are those of the interpolation of the 2^KL values V, of the upper ones those of Z, and the table
+// gradient is g u[lo] w[hi].  Three times 2^k multiply-adds and little else (k = 6: about 280 instructions per column
+// and 64 rows where the fold of the whole table and its reverse took 440), and of arrays of 2^k only the table gradient
+// stays in registers: sixteen wavefronts of it fit a CU at every k, where the fold left room for eight at k = 6.
+// gy is the row-major gradient itself: the block's 16 columns are 64 contiguous bytes of a row, the 64 x 16 piece of a
+// batch tile is fetched one value per thread a tile ahead and turned through the LDS (two buffers, one barrier per tile).
+template <int K, bool HYB>
+__global__ __launch_bounds__(1024) void prob_bwd_t(const float *__restrict__ xT, const float *__restrict__ gy,
+                                                   const int *__restrict__ idx32, const float *__restrict__ sig,
+                                                   float *__restrict__ gmT, float *__restrict__ gpart, int I, int N,
+                                                   int O, int BT, int tiles_per_chunk, int want_gm, int B) {
+    constexpr int L = 1 << K, W = 16;
+    constexpr int KL = K / 2, KU = K - KL, LL = 1 << KL, LU = 1 << KU;
+    __shared__ float gturn[2][W][65];  // [buffer][column][row]
     const int NO = N * O;
     const int lane = threadIdx.x & 63;
     const int c_raw = blockIdx.x * W + dl_uniform(threadIdx.x >> 6);
-    if (!GYROW && c_raw >= NO) return;
-    const bool live = c_raw < NO;        // GYROW: wavefronts past the last column still serve the barriers
+    const bool live = c_raw < NO;        // wavefronts past the last column still serve the barriers
     const int c = live ? c_raw : NO - 1;
     const int chunk = blockIdx.y;
     const int n = c / O;
@@ -218,78 +277,63 @@ __global__ __launch_bounds__(64 * W) void prob_bwd_t(const float *__restrict__ x
     for (int a = 0; a < L; ++a) acc[a] = 0.0f;
     const int t0 = chunk * tiles_per_chunk, t1 = min(BT, t0 + tiles_per_chunk);
     float nxs[K], ng = 0.0f;  // operands of the next batch tile, requested one tile ahead
-    const int trow = threadIdx.x >> 4, tcol = threadIdx.x & 15;  // GYROW: my value of the 64 x 16 piece
+    const int trow = threadIdx.x >> 4, tcol = threadIdx.x & 15;  // my value of the 64 x 16 piece
     auto request = [&](int t) {
         const __amdgpu_buffer_rsrc_t rs_x = __builtin_amdgcn_make_buffer_rsrc((void *)(xT + (size_t)t * I * 64), 0, I * 256, PROB_RSRC);
 #pragma unroll
         for (int j = 0; j < K; ++j) nxs[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs_x, lane4, off[j], 0));
-        if (GYROW) {
-            const int b = t * 64 + trow, cc = blockIdx.x * W + tcol;
-            ng = (b < B && cc < NO) ? gyT[(size_t)b * NO + cc] : 0.0f;
-        } else {
-            ng = gyT[((size_t)t * NO + c) * 64 + lane];
-        }
+        const int b = t * 64 + trow, cc = blockIdx.x * W + tcol;
+        ng = (b < B && cc < NO) ? gy[(size_t)b * NO + cc] : 0.0f;
     };
     if (t0 < t1) request(t0);
     for (int t = t0; t < t1; ++t) {
-        float xs[K];
+        float xs[K], om[K];
 #pragma unroll
-        for (int j = 0; j < K; ++j) xs[j] = nxs[j];
-        float g = ng;
-        if (GYROW) {
-            const int buf = (t - t0) & 1;
-            gturn[buf][tcol][trow] = ng;
-            __syncthreads();  // the other buffer is rewritten only after the next barrier: its readers are done by then
-            g = gturn[buf][threadIdx.x >> 6][lane];
-        }
+        for (int j = 0; j < K; ++j) { xs[j] = nxs[j]; om[j] = 1.0f - nxs[j]; }
+        const int buf = (t - t0) & 1;
+        gturn[buf][tcol][trow] = ng;
+        __syncthreads();  // the other buffer is rewritten only after the next barrier: its readers are done by then
+        const float g = gturn[buf][threadIdx.x >> 6][lane];
         if (t + 1 < t1) request(t + 1);
-        // forward fold, keeping the differences d_j[a] = lvl_j[2a+1] - lvl_j[2a] of every level
-        float diff[L > 1 ? L - 1 : 1];  // level j occupies [L - (L >> j), L - (L >> (j+1)))
-        float v[L / 2 > 0 ? L / 2 : 1];
+        float u[LL], w[LU], dx[K];
+        prob_products<KL>(xs, om, u);
+        prob_products<KU>(xs + KL, om + KL, w);
+        if (want_gm) {
+            if constexpr (KL > 0) {
+                float V[LL];
 #pragma unroll
-        for (int a = 0; a < L / 2; ++a) {
-            diff[a] = tab[2 * a + 1] - tab[2 * a];
-            v[a] = fmaf(xs[0], diff[a], tab[2 * a]);
-        }
-        int base = L / 2;
+                for (int lo = 0; lo < LL; ++lo) {
+                    V[lo] = tab[lo] * w[0];
 #pragma unroll
-        for (int j = 1; j < K; ++j) {
-#pragma unroll
-            for (int a = 0; a < (L >> (j + 1)); ++a) {
-                diff[base + a] = v[2 * a + 1] - v[2 * a];
-                v[a] = fmaf(xs[j], diff[base + a], v[2 * a]);
+                    for (int hi = 1; hi < LU; ++hi) V[lo] = fmaf(tab[lo | (hi << KL)], w[hi], V[lo]);
+                }
+                prob_fold_gradient<KL>(V, xs, om, dx);
             }
-            base += L >> (j + 1);
-        }
-        // backward: bar_K[0] = 1; dx_j = sum_a bar_{j+1}[a] d_j[a]; bar_j[2a] = bar_{j+1}[a] (1 - x_j), bar_j[2a+1] = bar_{j+1}[a] x_j
-        float bar[L];
-        bar[0] = 1.0f;
-        float dx[K];
+            float Z[LU];
 #pragma unroll
-        for (int j = K - 1; j >= 0; --j) {
-            base -= L >> (j + 1);
-            const int cnt = L >> (j + 1);
-            float sum = 0.0f;
+            for (int hi = 0; hi < LU; ++hi) {
+                Z[hi] = tab[hi << KL] * u[0];
 #pragma unroll
-            for (int a = 0; a < cnt; ++a) sum = fmaf(bar[a], diff[base + a], sum);
-            const float om = 1.0f - xs[j];
+                for (int lo = 1; lo < LL; ++lo) Z[hi] = fmaf(tab[lo | (hi << KL)], u[lo], Z[hi]);
+            }
+            prob_fold_gradient<KU>(Z, xs + KL, om + KL, dx + KL);
             if (HYB) {
-                const float q = xs[j] * om;
-                sum = sum * q / (q + PROB_HYBRID_EPS);
-            }
-            dx[j] = sum;
 #pragma unroll
-            for (int a = cnt - 1; a >= 0; --a) {
-                const float w = bar[a];
-                bar[2 * a + 1] = w * xs[j];
-                bar[2 * a] = w * om;
+                for (int j = 0; j < K; ++j) {
+                    const float q = xs[j] * om[j];
+                    dx[j] *= q * prob_rcp(q + PROB_HYBRID_EPS);
+                }
+            }
+            if (live) {
+#pragma unroll
+                for (int j = 0; j < K; ++j) gmT[(((size_t)t * NO + c) * K + j) * 64 + lane] = g * dx[j];
             }
         }
 #pragma unroll
-        for (int a = 0; a < L; ++a) acc[a] = fmaf(g, bar[a], acc[a]);
-        if (want_gm && live) {
+        for (int lo = 0; lo < LL; ++lo) {
+            const float gu = g * u[lo];
 #pragma unroll
-            for (int j = 0; j < K; ++j) gmT[(((size_t)t * NO + c) * K + j) * 64 + lane] = g * dx[j];
+            for (int hi = 0; hi < LU; ++hi) acc[lo | (hi << KL)] = fmaf(gu, w[hi], acc[lo | (hi << KL)]);
         }
     }
     // Sum the 64 per-row partials of every table entry with L - 1 + (6 - K) exchanges instead of 6 L:
@@ -580,13 +624,22 @@ static inline bool prob_fast(int I, int N, int k, int O) {
 // temperature.clamp(min=1e-6); with a per-node array the kernels take every node's own value
 static inline ProbTemp prob_temp(float t, const float *t_n) { return ProbTemp{1.0f / (t > 1e-6f ? t : 1e-6f), t_n}; }
 static inline int prob_bt(int B) { return (B + 63) / 64; }
-// batch tiles per wavefront of prob_bwd_t: enough (column, chunk) wavefronts to fill the chip
-static inline int prob_tiles_per_chunk(int B, int N, int O) {
-    const int BT = prob_bt(B);
-    int chunks = dl_ceil_div(4096, (long long)N * O);
-    if (chunks > BT) chunks = BT;
-    if (chunks < 1) chunks = 1;
-    return dl_ceil_div(BT, chunks);
+// Batch tiles per wavefront of prob_bwd_t.  Its blocks (16 columns x one chunk of tiles) share 256 CUs: the fullest CU has
+// ceil(blocks / 256) of them, and a block spends about 2 (k <= 4), 4 or 6 (k = 6) tiles' time on its table and its sums over
+// the lanes.  2000 x 3001 -> 5003 hybrid nodes of 4 inputs (313 blocks a chunk): one chunk 82 us, four 64; where one chunk
+// is 256 blocks, more of them lose (1024 x 4096 -> 4096 nodes: k = 4 27.7 -> 27.3 us, k = 5 32.4 -> 34.7).
+static inline int prob_tiles_per_chunk(int B, int N, int k, int O) {
+    const int BT = prob_bt(B), own = k >= 6 ? 6 : (k == 5 ? 4 : 2);
+    const long long blocks = dl_ceil_div((long long)N * O, 16);
+    int best = BT;
+    double best_cost = 0.0;
+    for (int c = 1; c <= BT && c <= 16; ++c) {
+        const int tpc = dl_ceil_div(BT, c);
+        const long long all = blocks * dl_ceil_div(BT, tpc);
+        const double cost = (all > 256 ? (double)dl_ceil_div(all, 256) : 1.1) * (tpc + own);
+        if (c == 1 || cost < best_cost) { best = tpc; best_cost = cost; }
+    }
+    return best;
 }
 static inline size_t prob_sig_bytes(int N, int k, int O) { return dl_align256((size_t)N * O * ((size_t)1 << k) * sizeof(float)); }
 static inline size_t prob_xT_bytes(int B, int I) { return dl_align256((size_t)prob_bt(B) * I * 64 * sizeof(float)); }
@@ -599,9 +652,8 @@ extern "C" size_t dl_prob_saved_bytes(int B, int I, int N, int k, int O) {
 extern "C" size_t dl_prob_bwd_workspace_bytes(int B, int I, int N, int k, int O) {
     if (B <= 0 || I <= 0 || N <= 0 || k <= 0 || O <= 0 || !prob_fast(I, N, k, O)) return 256;
     const size_t BT = prob_bt(B);
-    const int chunks = dl_ceil_div(prob_bt(B), prob_tiles_per_chunk(B, N, O));
-    return prob_sig_bytes(N, k, O) + prob_xT_bytes(B, I) + dl_align256(BT * N * O * 64 * sizeof(float)) +
-           dl_align256(BT * N * O * k * 64 * sizeof(float)) + dl_align256((size_t)chunks * N * O * ((size_t)1 << k) * sizeof(float));
+    const int chunks = dl_ceil_div(prob_bt(B), prob_tiles_per_chunk(B, N, k, O));
+    return prob_sig_bytes(N, k, O) + prob_xT_bytes(B, I) + dl_align256(BT * N * O * k * 64 * sizeof(float)) + dl_align256((size_t)chunks * N * O * ((size_t)1 << k) * sizeof(float));
 }
 
 #define PROB_DISPATCH(K, CALL) \
@@ -668,12 +720,11 @@ static int prob_backward(const float *x, const void *saved, const int32_t *idx32
     if (!ws) return DL_ERR_NULL;
     if (ws_bytes < dl_prob_bwd_workspace_bytes(B, I, N, k, O)) return DL_ERR_WORKSPACE;
     const int BT = prob_bt(B), L = 1 << k, NO = N * O;
-    const int tpc = prob_tiles_per_chunk(B, N, O);
+    const int tpc = prob_tiles_per_chunk(B, N, k, O);
     const int chunks = dl_ceil_div(BT, tpc);
     char *w = (char *)ws;
     float *sig = (float *)w; w += prob_sig_bytes(N, k, O);
     float *xT = (float *)w; w += prob_xT_bytes(B, I);
-    float *gyT = (float *)w; w += dl_align256((size_t)BT * NO * 64 * sizeof(float));
     float *gmT = (float *)w; w += dl_align256((size_t)BT * NO * k * 64 * sizeof(float));
     float *gpart = (float *)w;
     if (saved) {  // what the forward of the same x, raw_w and temperature left
@@ -683,25 +734,12 @@ static int prob_backward(const float *x, const void *saved, const int32_t *idx32
         DL_TIMED("prob_sig_table", s, (prob_sig_table<<<dl_ceil_div(WT, 256), 256, 0, s>>>(raw_w, inv_t, sig, N, L, O)));
         DL_TIMED("prob_to_tiles_x", s, (prob_to_tiles<<<dim3(dl_ceil_div(I, 64), BT), 256, 0, s>>>(x, xT, B, I)));
     }
-    if (k <= 5) {  // 16 wavefronts per block take gy as it is (see prob_bwd_t)
 #define CALL(KK)                                                                                                       \
     DL_TIMED("prob_bwd_t", s,                                                                                          \
-             (prob_bwd_t<KK, false, 16><<<dim3(dl_ceil_div(NO, 16), chunks), 1024, 0, s>>>(xT, gy, idx32, sig, gmT, gpart, I, N, \
-                                                                                        O, BT, tpc, gx != nullptr, B)))
-        switch (k) {
-            case 1: CALL(1); break; case 2: CALL(2); break; case 3: CALL(3); break; case 4: CALL(4); break;
-            default: CALL(5); break;
-        }
+             (prob_bwd_t<KK, false><<<dim3(dl_ceil_div(NO, 16), chunks), 1024, 0, s>>>(xT, gy, idx32, sig, gmT, gpart, I, N, \
+                                                                                    O, BT, tpc, gx != nullptr, B)))
+    PROB_DISPATCH(k, CALL)
 #undef CALL
-    } else {
-        DL_TIMED("prob_to_tiles_gy", s, (prob_to_tiles<<<dim3(dl_ceil_div(NO, 64), BT), 256, 0, s>>>(gy, gyT, B, NO)));
-#define CALL(KK)                                                                                                    \
-    DL_TIMED("prob_bwd_t", s,                                                                                       \
-             (prob_bwd_t<KK, false><<<dim3(dl_ceil_div(NO, 4), chunks), 256, 0, s>>>(xT, gyT, idx32, sig, gmT, gpart, I, N, O, \
-                                                                                  BT, tpc, gx != nullptr)))
-        PROB_DISPATCH(k, CALL)
-#undef CALL
-    }
     const ProbReduce R = {gpart, sig, inv_t, graw, N, L, O, chunks};
     prob_launch_gather_and_reduce(gmT, inv_ptr, inv_pos, gx, B, I, N, k, O, BT, R, WT, s);
     return dl_launch_status();
@@ -748,19 +786,17 @@ extern "C" int dl_hybrid_layer_bwd(const float *x, const int32_t *idx32, const i
     if (!ws) return DL_ERR_NULL;
     if (ws_bytes < dl_hybrid_bwd_workspace_bytes(B, I, N, k, O)) return DL_ERR_WORKSPACE;
     const int BT = prob_bt(B), L = 1 << k, NO = N * O;
-    const int tpc = prob_tiles_per_chunk(B, N, O);
+    const int tpc = prob_tiles_per_chunk(B, N, k, O);
     const int chunks = dl_ceil_div(BT, tpc);
     char *w = (char *)ws;
     float *xT = (float *)w; w += prob_xT_bytes(B, I);
-    float *gyT = (float *)w; w += dl_align256((size_t)BT * NO * 64 * sizeof(float));
     float *gmT = (float *)w; w += dl_align256((size_t)BT * NO * k * 64 * sizeof(float));
     float *gpart = (float *)w;
     DL_TIMED("prob_to_tiles_x", s, (prob_to_tiles<<<dim3(dl_ceil_div(I, 64), BT), 256, 0, s>>>(x, xT, B, I)));
-    DL_TIMED("prob_to_tiles_gy", s, (prob_to_tiles<<<dim3(dl_ceil_div(NO, 64), BT), 256, 0, s>>>(gy, gyT, B, NO)));
 #define CALL(KK)                                                                                                          \
     DL_TIMED("hybrid_bwd_t", s,                                                                                           \
-             (prob_bwd_t<KK, true><<<dim3(dl_ceil_div(NO, 4), chunks), 256, 0, s>>>(xT, gyT, idx32, luts, gmT, gpart, I, N, O, \
-                                                                                 BT, tpc, gx != nullptr)))
+             (prob_bwd_t<KK, true><<<dim3(dl_ceil_div(NO, 16), chunks), 1024, 0, s>>>(xT, gy, idx32, luts, gmT, gpart, I, N, O, \
+                                                                                   BT, tpc, gx != nullptr, B)))
     PROB_DISPATCH(k, CALL)
 #undef CALL
     const ProbReduce R = {gpart, nullptr, ProbTemp{1.0f, nullptr}, gluts, N, L, O, chunks};

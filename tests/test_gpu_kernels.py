@@ -555,6 +555,31 @@ def test_prob_layer_forward_backward(shape, T):
     np.testing.assert_allclose(wt.grad.cpu().numpy(), gw, rtol=1e-5, atol=2e-6)
 
 
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("B,N,O,T", [(64, 16, 1, 1.0),     # one block of sixteen columns, one batch tile
+                                     (321, 17, 1, 0.5),    # a column and a row past that; several chunks of tiles
+                                     (1025, 250, 2, 1.0),  # more blocks than fit one per chunk
+                                     (130, 4100, 1, 1.0)]) # one chunk
+def test_prob_backward_factored_weights(B, N, O, T, k):
+    """The product weights factor into those of the lower k / 2 and of the upper inputs, sixteen columns to a block.  The
+    gradient of an input with 2^k terms of size |gy| <= 4 rounds to a few 1e-7 of that: rtol 1e-5, floor 5e-6; table
+    gradients sum up to 1025 rows: floor 1e-5."""
+    ops = _ops()
+    I = 37 + N // 3
+    rng = np.random.default_rng(B + N + k)
+    x = rng.uniform(0, 1, (B, I)).astype(np.float32)
+    x[:, 0] = (x[:, 0] > 0.5)  # exact zeros and ones among the inputs
+    idx = orc.random_mapping(I, N, k, seed=4).numpy().astype(np.int64)
+    raw = rng.uniform(-1, 1, (N, 1 << k, O)).astype(np.float32)
+    gy = rng.uniform(-4, 4, (B, N, O)).astype(np.float32)
+    plan = ops.MappingPlan(dev(idx, torch.int32), I)
+    xt = dev(x).requires_grad_(); wt = dev(raw).requires_grad_()
+    ops.ProbLayerFunction.apply(xt, wt, plan, T).backward(dev(gy.reshape(B, -1)))
+    gx, gw = orc.prob_layer_backward(x, idx, raw, gy, T)
+    np.testing.assert_allclose(xt.grad.cpu().numpy(), gx, rtol=1e-5, atol=5e-6)
+    np.testing.assert_allclose(wt.grad.cpu().numpy(), gw, rtol=1e-5, atol=1e-5)
+
+
 @pytest.mark.parametrize("tag", ["k4o2", "k6o1"])
 def test_prob_node_against_reference_vectors(golden, tag):
     from difflut_amd.nodes.probabilistic_node import probabilistic_forward
