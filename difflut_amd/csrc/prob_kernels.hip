@@ -764,7 +764,9 @@ extern "C" int dl_prob_layer_bwd_nodes(const float *x, const void *saved, const 
 // Hybrid nodes: the forward is the DWN lookup; the backward is the probabilistic one on the table as given.
 extern "C" size_t dl_hybrid_bwd_workspace_bytes(int B, int I, int N, int k, int O) {
     if (B <= 0 || I <= 0 || N <= 0 || k <= 0 || O <= 0 || !prob_fast(I, N, k, O)) return 256;
-    return dl_prob_bwd_workspace_bytes(B, I, N, k, O) - prob_sig_bytes(N, k, O);
+    // (one more [B, N O] array than the kernels use: the size never shrinks below what callers have been told before)
+    return dl_prob_bwd_workspace_bytes(B, I, N, k, O) - prob_sig_bytes(N, k, O) +
+           dl_align256((size_t)prob_bt(B) * N * O * 64 * sizeof(float));
 }
 
 extern "C" int dl_hybrid_layer_bwd(const float *x, const int32_t *idx32, const int32_t *inv_ptr, const int32_t *inv_pos,
