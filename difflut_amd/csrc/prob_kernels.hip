@@ -649,11 +649,13 @@ extern "C" size_t dl_prob_saved_bytes(int B, int I, int N, int k, int O) {
     if (B <= 0 || I <= 0 || N <= 0 || k <= 0 || O <= 0 || !prob_fast(I, N, k, O)) return 256;
     return prob_sig_bytes(N, k, O) + prob_xT_bytes(B, I);
 }
+// (with room for one more [B, N O] array than the kernels use: the size does not shrink below what callers sized by before)
 extern "C" size_t dl_prob_bwd_workspace_bytes(int B, int I, int N, int k, int O) {
     if (B <= 0 || I <= 0 || N <= 0 || k <= 0 || O <= 0 || !prob_fast(I, N, k, O)) return 256;
     const size_t BT = prob_bt(B);
     const int chunks = dl_ceil_div(prob_bt(B), prob_tiles_per_chunk(B, N, k, O));
-    return prob_sig_bytes(N, k, O) + prob_xT_bytes(B, I) + dl_align256(BT * N * O * k * 64 * sizeof(float)) + dl_align256((size_t)chunks * N * O * ((size_t)1 << k) * sizeof(float));
+    return prob_sig_bytes(N, k, O) + prob_xT_bytes(B, I) + dl_align256(BT * N * O * 64 * sizeof(float)) +
+           dl_align256(BT * N * O * k * 64 * sizeof(float)) + dl_align256((size_t)chunks * N * O * ((size_t)1 << k) * sizeof(float));
 }
 
 #define PROB_DISPATCH(K, CALL) \
@@ -764,9 +766,7 @@ extern "C" int dl_prob_layer_bwd_nodes(const float *x, const void *saved, const 
 // Hybrid nodes: the forward is the DWN lookup; the backward is the probabilistic one on the table as given.
 extern "C" size_t dl_hybrid_bwd_workspace_bytes(int B, int I, int N, int k, int O) {
     if (B <= 0 || I <= 0 || N <= 0 || k <= 0 || O <= 0 || !prob_fast(I, N, k, O)) return 256;
-    // (one more [B, N O] array than the kernels use: the size never shrinks below what callers have been told before)
-    return dl_prob_bwd_workspace_bytes(B, I, N, k, O) - prob_sig_bytes(N, k, O) +
-           dl_align256((size_t)prob_bt(B) * N * O * 64 * sizeof(float));
+    return dl_prob_bwd_workspace_bytes(B, I, N, k, O) - prob_sig_bytes(N, k, O);
 }
 
 extern "C" int dl_hybrid_layer_bwd(const float *x, const int32_t *idx32, const int32_t *inv_ptr, const int32_t *inv_pos,
