@@ -24,6 +24,16 @@ def _bytes(n, device):
     return torch.empty(max(int(n), 256), dtype=torch.uint8, device=device)
 
 
+def _per_node(values, N, device):
+    """A number or tensor of per-node values as the float32 device array [N] the kernels read; what a layer's bank hands
+    over is that already (five torch calls less per array)."""
+    if (torch.is_tensor(values) and values.dtype is torch.float32 and values.dim() == 1 and values.shape[0] == N
+            and values.device == device and not values.requires_grad and values.is_contiguous()):
+        return values
+    values = torch.as_tensor(values, dtype=torch.float32, device=device).detach()
+    return values.reshape(-1).expand(N).contiguous()
+
+
 class MappingPlan:
     """Device-side form of an index table idx [N,k] over I inputs.
 
@@ -157,8 +167,7 @@ class DWNLayerFunction(torch.autograd.Function):
         nat.check(lib.dl_dwn_layer_fwd(nat.ptr(x), nat.ptr(plan.idx32), nat.ptr(luts), nat.ptr(y), nat.ptr(saved),
                                        nat.ptr(ws), ws.numel(), *dims, nat.stream()))
         if torch.is_tensor(alpha) or torch.is_tensor(beta):
-            alpha = torch.as_tensor(alpha, dtype=torch.float32, device=x.device).expand(N).contiguous()
-            beta = torch.as_tensor(beta, dtype=torch.float32, device=x.device).expand(N).contiguous()
+            alpha, beta = _per_node(alpha, N, x.device), _per_node(beta, N, x.device)
             if beta_abs_max is None:
                 beta_abs_max = float(beta.abs().max())
             ctx.ab = (alpha, beta, float(beta_abs_max))
@@ -307,8 +316,7 @@ class DWNStackFunction(torch.autograd.Function):
             groups, tau = ctx.head if headed else (1, 1.0)
             if len(ctx.scalars[l]) == 3:  # every node's own alpha and beta
                 alpha_n, beta_n, beta_max = ctx.scalars[l]
-                alpha_n = _f32(alpha_n.detach()).reshape(-1).expand(N).contiguous()
-                beta_n = _f32(beta_n.detach()).reshape(-1).expand(N).contiguous()
+                alpha_n, beta_n = _per_node(alpha_n, N, device), _per_node(beta_n, N, device)
                 # the gather of this layer can fill the table gradient of the layer in front as it goes: that layer's
                 # own pass over its [B, N] output gradient is then left out
                 k_prev = ctx.dims_all[l - 1][3] if l > 0 else 0
@@ -519,7 +527,7 @@ def _node_temperatures(temperature, N, device):
     """None for one temperature (a number), else the nodes' own values as a float32 device array [N]."""
     if not torch.is_tensor(temperature):
         return None
-    return temperature.detach().to(device=device, dtype=torch.float32).reshape(-1).expand(N).contiguous()
+    return _per_node(temperature, N, device)
 
 
 class ProbLayerFunction(torch.autograd.Function):
