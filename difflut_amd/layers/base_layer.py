@@ -73,11 +73,12 @@ class BankedParameter(nn.Parameter):
 
 def _node_getter(nodes):
     """row -> node without ModuleList.__getitem__, whose index arithmetic costs more than the checks below (they run on
-    every call of a layer).  Looks the node up anew each time, so a replaced node is seen."""
+    every call of a layer).  Looks the node up anew each time, in the list's present dict (deleting an entry gives it a
+    new one), so a replaced node is seen."""
     if not isinstance(nodes, nn.ModuleList):
         return nodes.__getitem__
-    modules, keys = nodes._modules, [str(row) for row in range(len(nodes))]
-    return lambda row: modules[keys[row]]
+    keys = [str(row) for row in range(len(nodes))]
+    return lambda row: nodes._modules[keys[row]]
 
 
 class ParameterBank:

@@ -316,6 +316,20 @@ def test_bank_notices_nodes_taken_over_or_replaced():
     assert torch.equal(bank.tensor()[6], torch.zeros(1, 8))
 
 
+def test_banks_notice_a_deleted_and_an_appended_node():
+    """Deleting an entry of a ModuleList gives the list a new dict; a node appended afterwards restores the count, so
+    only the nodes themselves tell."""
+    layer, other = _small_dwn_layer(), _small_dwn_layer()
+    last = layer.nodes[11].luts.detach().clone()
+    del layer.nodes[0]
+    layer.nodes.append(other.nodes[5])
+    layer.nodes[11].alpha.fill_(0.125)
+    assert not layer._banks["luts"].tied() and not layer._scalars["alpha"].tied()
+    flat = layer._banks["luts"].tensor()
+    assert torch.equal(flat[10], last) and torch.equal(flat[11], layer.nodes[11].luts)
+    assert float(layer.efd_scalars()[0][11]) == 0.125
+
+
 def test_scalar_buffers_are_banked_and_differences_are_seen():
     layer = _small_dwn_layer()
     alpha, beta = layer._scalars["alpha"], layer._scalars["beta"]
