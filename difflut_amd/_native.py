@@ -53,6 +53,11 @@ SIGNATURES = {
     "dl_table_sigmoid_bwd": (_I, [_P, _P, _P, ctypes.c_longlong, _P]),
     "dl_hybrid_bwd_workspace_bytes": (_Z, [_I] * 5),
     "dl_hybrid_layer_bwd": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _Z, _I, _I, _I, _I, _I, _P]),
+    "dl_hybrid_saved_bytes": (_Z, [_I] * 5),
+    "dl_hybrid_fwd_workspace_bytes": (_Z, [_I] * 5),
+    "dl_hybrid_bwd_saved_workspace_bytes": (_Z, [_I] * 5),
+    "dl_hybrid_layer_fwd": (_I, [_P, _P, _P, _P, _P, _Z, _P, _Z, _I, _I, _I, _I, _I, _P]),
+    "dl_hybrid_layer_bwd_saved": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _Z, _I, _I, _I, _I, _I, _P]),
     "dl_prob_saved_bytes": (_Z, [_I] * 5),
     "dl_prob_bwd_workspace_bytes": (_Z, [_I] * 5),
     "dl_prob_layer_fwd": (_I, [_P, _P, _P, _F, _P, _P, _Z, _I, _I, _I, _I, _I, _P]),

@@ -53,10 +53,16 @@ __global__ __launch_bounds__(256) void prob_sig_table(const float *__restrict__ 
 // grid (ceil(C / 64), B/64 rounded up), 256 threads.  With `sig` set the launch carries extra rows of blocks
 // (blockIdx.y >= tiles) that build the sigmoid table in the same launch: the two jobs are independent and each is
 // too short to fill the machine on its own.
+// PLANES (the hybrid node's forward): the bit-planes a DWN lookup reads leave in the same pass, one ballot per column of the
+// tile in the LDS (word (t, c), bit r = src[64 t + r][c] >= 0.5, 0 past the batch).  HBM bound; x used to be read once by the
+// lookup's own packing pass and again by the backward's re-tiling.  Hybrid layer 4096 x 16384 -> 8192 nodes of six inputs,
+// forward + backward: 718 -> 683 us.
+template <bool PLANES = false>
 __global__ __launch_bounds__(256) void prob_to_tiles(const float *__restrict__ src, float *__restrict__ dst, int B, int C,
                                                       int tiles = 1 << 30, const float *__restrict__ raw = nullptr,
                                                       ProbTemp T = {1.0f, nullptr}, float *__restrict__ sig = nullptr,
-                                                      int N = 0, int L = 1, int O = 1) {
+                                                      int N = 0, int L = 1, int O = 1,
+                                                      unsigned long long *__restrict__ planes = nullptr) {
     __shared__ float tile[64][65];  // [column][row]
     if ((int)blockIdx.y >= tiles) {
         const long long e = ((long long)(blockIdx.y - tiles) * gridDim.x + blockIdx.x) * 256 + threadIdx.x;
@@ -87,6 +93,16 @@ __global__ __launch_bounds__(256) void prob_to_tiles(const float *__restrict__ s
         }
     }
     __syncthreads();
+    if (PLANES) {
+        const int lane = threadIdx.x & 63, cw = (threadIdx.x >> 6) * 16;
+        unsigned long long mine = 0;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) {
+            const unsigned long long mask = __ballot(tile[cw + q][lane] >= 0.5f);
+            mine = lane == q ? mask : mine;
+        }
+        if (lane < 16 && c0 + cw + lane < C) planes[(size_t)t * C + c0 + cw + lane] = mine;
+    }
 #pragma unroll
     for (int pass = 0; pass < 4; ++pass) {
         const int e = pass * 256 + threadIdx.x;
@@ -682,7 +698,7 @@ static int prob_forward(const float *x, const int32_t *idx32, const float *raw_w
     {   // x re-tiled and the sigmoid table built in one launch
         const int gx_ = dl_ceil_div(I, 64);
         const int extra = dl_ceil_div(dl_ceil_div((long long)N * L * O, 256), gx_);
-        DL_TIMED("prob_to_tiles_x+sig_table", s, (prob_to_tiles<<<dim3(gx_, BT + extra), 256, 0, s>>>(
+        DL_TIMED("prob_to_tiles_x+sig_table", s, (prob_to_tiles<false><<<dim3(gx_, BT + extra), 256, 0, s>>>(
                                                      x, xT, B, I, BT, raw_w, inv_t, sig, N, L, O)));
     }
     const int grid = dl_xcd_grid(dl_ceil_div((long long)N * O, PROB_TC), BT);
@@ -734,7 +750,7 @@ static int prob_backward(const float *x, const void *saved, const int32_t *idx32
         xT = (float *)((char *)saved + prob_sig_bytes(N, k, O));
     } else {
         DL_TIMED("prob_sig_table", s, (prob_sig_table<<<dl_ceil_div(WT, 256), 256, 0, s>>>(raw_w, inv_t, sig, N, L, O)));
-        DL_TIMED("prob_to_tiles_x", s, (prob_to_tiles<<<dim3(dl_ceil_div(I, 64), BT), 256, 0, s>>>(x, xT, B, I)));
+        DL_TIMED("prob_to_tiles_x", s, (prob_to_tiles<false><<<dim3(dl_ceil_div(I, 64), BT), 256, 0, s>>>(x, xT, B, I)));
     }
 #define CALL(KK)                                                                                                       \
     DL_TIMED("prob_bwd_t", s,                                                                                          \
@@ -769,9 +785,50 @@ extern "C" size_t dl_hybrid_bwd_workspace_bytes(int B, int I, int N, int k, int 
     return dl_prob_bwd_workspace_bytes(B, I, N, k, O) - prob_sig_bytes(N, k, O);
 }
 
-extern "C" int dl_hybrid_layer_bwd(const float *x, const int32_t *idx32, const int32_t *inv_ptr, const int32_t *inv_pos,
-                                   const float *luts, const float *gy, float *gx, float *gluts, void *ws, size_t ws_bytes,
-                                   int B, int I, int N, int k, int O, void *stream) {
+// The forward leaves x re-tiled for the backward where both take the tiled path.
+static inline bool hybrid_tiled(int B, int I, int N, int k, int O) {
+    return prob_check(B, I, N, k, O) == DL_OK && prob_fast(I, N, k, O);
+}
+extern "C" size_t dl_dwn_saved_bytes(int B, int I, int N, int k, int O);
+extern "C" size_t dl_dwn_fwd_workspace_bytes(int B, int I, int N, int k, int O);
+extern "C" size_t dl_dwn_planes_bytes(int B, int C);
+extern "C" int dl_dwn_layer_fwd(const float *x, const int32_t *idx32, const float *luts, float *y, void *saved, void *ws,
+                                size_t ws_bytes, int B, int I, int N, int k, int O, void *stream);
+extern "C" int dl_dwn_layer_fwd_planes(const void *planes_in, const int32_t *idx32, const float *luts, float *y,
+                                       void *planes_out, void *saved, int B, int I, int N, int k, int O, void *stream);
+extern "C" size_t dl_hybrid_saved_bytes(int B, int I, int N, int k, int O) {
+    return hybrid_tiled(B, I, N, k, O) ? prob_xT_bytes(B, I) : 256;
+}
+// the lookup's addresses, which nothing reads afterwards, and its planes or workspace
+extern "C" size_t dl_hybrid_fwd_workspace_bytes(int B, int I, int N, int k, int O) {
+    if (B <= 0 || I <= 0 || N <= 0 || k <= 0 || O <= 0) return 256;
+    const size_t planes = dl_align256(dl_dwn_planes_bytes(B, I)), own = dl_align256(dl_dwn_fwd_workspace_bytes(B, I, N, k, O));
+    return dl_align256(dl_dwn_saved_bytes(B, I, N, k, O)) + (planes > own ? planes : own);
+}
+extern "C" int dl_hybrid_layer_fwd(const float *x, const int32_t *idx32, const float *luts, float *y, void *saved,
+                                   size_t saved_bytes, void *ws, size_t ws_bytes, int B, int I, int N, int k, int O,
+                                   void *stream) {
+    if (!x || !idx32 || !luts || !y || !saved || !ws) return DL_ERR_NULL;
+    if (B <= 0 || I <= 0 || N <= 0 || k <= 0 || O <= 0) return DL_ERR_SHAPE;
+    if (saved_bytes < dl_hybrid_saved_bytes(B, I, N, k, O) || ws_bytes < dl_hybrid_fwd_workspace_bytes(B, I, N, k, O))
+        return DL_ERR_WORKSPACE;
+    hipStream_t s = (hipStream_t)stream;
+    const size_t addr_bytes = dl_align256(dl_dwn_saved_bytes(B, I, N, k, O));
+    char *rest = (char *)ws + addr_bytes;
+    if (hybrid_tiled(B, I, N, k, O)) {
+        const int BT = prob_bt(B);
+        DL_TIMED("hybrid_tiles+planes", s,
+                 (prob_to_tiles<true><<<dim3(dl_ceil_div(I, 64), BT), 256, 0, s>>>(
+                     x, (float *)saved, B, I, 1 << 30, nullptr, ProbTemp{1.0f, nullptr}, nullptr, 0, 1, 1, (unsigned long long *)rest)));
+        const int rc = dl_dwn_layer_fwd_planes(rest, idx32, luts, y, nullptr, ws, B, I, N, k, O, stream);
+        if (rc != DL_ERR_UNSUPPORTED) return rc;
+    }
+    return dl_dwn_layer_fwd(x, idx32, luts, y, ws, rest, ws_bytes - addr_bytes, B, I, N, k, O, stream);
+}
+
+static int hybrid_backward(const float *x, const void *saved, const int32_t *idx32, const int32_t *inv_ptr,
+                           const int32_t *inv_pos, const float *luts, const float *gy, float *gx, float *gluts, void *ws,
+                           size_t ws_bytes, size_t ws_needed, int B, int I, int N, int k, int O, void *stream) {
     if (!x || !idx32 || !luts || !gy || !gluts) return DL_ERR_NULL;
     if (gx && (!inv_ptr || !inv_pos)) return DL_ERR_NULL;
     int rc = prob_check(B, I, N, k, O);
@@ -786,15 +843,19 @@ extern "C" int dl_hybrid_layer_bwd(const float *x, const int32_t *idx32, const i
         return dl_launch_status();
     }
     if (!ws) return DL_ERR_NULL;
-    if (ws_bytes < dl_hybrid_bwd_workspace_bytes(B, I, N, k, O)) return DL_ERR_WORKSPACE;
+    if (ws_bytes < ws_needed) return DL_ERR_WORKSPACE;
     const int BT = prob_bt(B), L = 1 << k, NO = N * O;
     const int tpc = prob_tiles_per_chunk(B, N, k, O);
     const int chunks = dl_ceil_div(BT, tpc);
     char *w = (char *)ws;
-    float *xT = (float *)w; w += prob_xT_bytes(B, I);
+    const float *xT = (const float *)saved;  // what the forward of the same x left
+    if (!saved) {
+        float *own = (float *)w; w += prob_xT_bytes(B, I);
+        DL_TIMED("prob_to_tiles_x", s, (prob_to_tiles<false><<<dim3(dl_ceil_div(I, 64), BT), 256, 0, s>>>(x, own, B, I)));
+        xT = own;
+    }
     float *gmT = (float *)w; w += dl_align256((size_t)BT * NO * k * 64 * sizeof(float));
     float *gpart = (float *)w;
-    DL_TIMED("prob_to_tiles_x", s, (prob_to_tiles<<<dim3(dl_ceil_div(I, 64), BT), 256, 0, s>>>(x, xT, B, I)));
 #define CALL(KK)                                                                                                          \
     DL_TIMED("hybrid_bwd_t", s,                                                                                           \
              (prob_bwd_t<KK, true><<<dim3(dl_ceil_div(NO, 16), chunks), 1024, 0, s>>>(xT, gy, idx32, luts, gmT, gpart, I, N, O, \
@@ -804,6 +865,26 @@ extern "C" int dl_hybrid_layer_bwd(const float *x, const int32_t *idx32, const i
     const ProbReduce R = {gpart, nullptr, ProbTemp{1.0f, nullptr}, gluts, N, L, O, chunks};
     prob_launch_gather_and_reduce(gmT, inv_ptr, inv_pos, gx, B, I, N, k, O, BT, R, WT, s);
     return dl_launch_status();
+}
+
+extern "C" int dl_hybrid_layer_bwd(const float *x, const int32_t *idx32, const int32_t *inv_ptr, const int32_t *inv_pos,
+                                   const float *luts, const float *gy, float *gx, float *gluts, void *ws, size_t ws_bytes,
+                                   int B, int I, int N, int k, int O, void *stream) {
+    return hybrid_backward(x, nullptr, idx32, inv_ptr, inv_pos, luts, gy, gx, gluts, ws, ws_bytes,
+                           dl_hybrid_bwd_workspace_bytes(B, I, N, k, O), B, I, N, k, O, stream);
+}
+extern "C" size_t dl_hybrid_bwd_saved_workspace_bytes(int B, int I, int N, int k, int O) {
+    if (!hybrid_tiled(B, I, N, k, O)) return 256;
+    const size_t BT = prob_bt(B);
+    const int chunks = dl_ceil_div(prob_bt(B), prob_tiles_per_chunk(B, N, k, O));
+    return dl_align256(BT * N * O * k * 64 * sizeof(float)) + dl_align256((size_t)chunks * N * O * ((size_t)1 << k) * sizeof(float));
+}
+extern "C" int dl_hybrid_layer_bwd_saved(const float *x, const void *saved, const int32_t *idx32, const int32_t *inv_ptr,
+                                         const int32_t *inv_pos, const float *luts, const float *gy, float *gx, float *gluts,
+                                         void *ws, size_t ws_bytes, int B, int I, int N, int k, int O, void *stream) {
+    if (!saved) return DL_ERR_NULL;
+    return hybrid_backward(x, saved, idx32, inv_ptr, inv_pos, luts, gy, gx, gluts, ws, ws_bytes,
+                           dl_hybrid_bwd_saved_workspace_bytes(B, I, N, k, O), B, I, N, k, O, stream);
 }
 
 // Eval forward with a workspace: the binarised sigmoid table of every node is the table of a DWN layer, so the

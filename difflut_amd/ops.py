@@ -442,16 +442,21 @@ class TableSigmoidFunction(torch.autograd.Function):
         return graw
 
 
-def _dwn_lookup(x, luts, plan):
-    """Training forward shared by the DWN-type nodes: (y, saved, dims)."""
+def _lookup_dims(x, luts, plan):
     B, I = x.shape
     N, O, L = luts.shape
     k = plan.k
     if (N, 1 << k, I) != (plan.N, L, plan.I):
         raise RuntimeError(f"shape mismatch: x {tuple(x.shape)}, luts {tuple(luts.shape)}, mapping [{plan.N},{k}] "
                            f"over {plan.I} inputs")
+    return B, I, N, k, O
+
+
+def _dwn_lookup(x, luts, plan):
+    """Training forward shared by the DWN-type nodes: (y, saved, dims)."""
+    dims = _lookup_dims(x, luts, plan)
+    B, _, N, _, O = dims
     lib = nat.lib()
-    dims = (B, I, N, k, O)
     y = torch.empty((B, N * O), dtype=torch.float32, device=x.device)
     saved = _bytes(lib.dl_dwn_saved_bytes(*dims), x.device)
     ws = _bytes(lib.dl_dwn_fwd_workspace_bytes(*dims), x.device)
@@ -495,31 +500,49 @@ class DWNStableLayerFunction(torch.autograd.Function):
 
 
 class HybridLayerFunction(torch.autograd.Function):
-    """Thresholded lookup forward, probabilistic backward on the real-valued inputs (hybrid_node.py:33-204)."""
+    """Thresholded lookup forward, probabilistic backward on the real-valued inputs (hybrid_node.py:33-204).  Where a
+    backward will follow (`keep_tiles`), the forward re-tiles x for it in the pass that thresholds it."""
 
     @staticmethod
-    def forward(ctx, x, luts, plan):
+    def forward(ctx, x, luts, plan, keep_tiles=True):
         nat.require_device(x, luts)
         x, luts = _f32(x), _f32(luts)
-        y, _, dims = _dwn_lookup(x, luts, plan)
-        ctx.save_for_backward(x, luts)
+        tiles = None
+        if keep_tiles and plan.k <= FAST_K:
+            dims = _lookup_dims(x, luts, plan)
+            B, _, N, _, O = dims
+            lib = nat.lib()
+            y = torch.empty((B, N * O), dtype=torch.float32, device=x.device)
+            tiles = _bytes(lib.dl_hybrid_saved_bytes(*dims), x.device)
+            ws = _bytes(lib.dl_hybrid_fwd_workspace_bytes(*dims), x.device)
+            nat.check(lib.dl_hybrid_layer_fwd(nat.ptr(x), nat.ptr(plan.idx32), nat.ptr(luts), nat.ptr(y), nat.ptr(tiles),
+                                              tiles.numel(), nat.ptr(ws), ws.numel(), *dims, nat.stream()))
+        else:
+            y, _, dims = _dwn_lookup(x, luts, plan)
+        ctx.save_for_backward(x, luts, tiles)
         ctx.plan, ctx.dims = plan, dims
         return y
 
     @staticmethod
     def backward(ctx, gy):
-        x, luts = ctx.saved_tensors
+        x, luts, tiles = ctx.saved_tensors
         B, I, N, k, O = ctx.dims
         plan = ctx.plan
         gy = _f32(gy)
         lib = nat.lib()
         gx = torch.empty((B, I), dtype=torch.float32, device=gy.device) if ctx.needs_input_grad[0] else None
         gl = torch.empty_like(luts)
-        ws = _bytes(lib.dl_hybrid_bwd_workspace_bytes(*ctx.dims), gy.device)
-        nat.check(lib.dl_hybrid_layer_bwd(nat.ptr(x), nat.ptr(plan.idx32), nat.ptr(plan.inv_ptr), nat.ptr(plan.inv_pos),
-                                          nat.ptr(luts), nat.ptr(gy), nat.ptr(gx), nat.ptr(gl), nat.ptr(ws), ws.numel(),
-                                          *ctx.dims, nat.stream()))
-        return gx, gl, None
+        if tiles is None:
+            ws = _bytes(lib.dl_hybrid_bwd_workspace_bytes(*ctx.dims), gy.device)
+            nat.check(lib.dl_hybrid_layer_bwd(nat.ptr(x), nat.ptr(plan.idx32), nat.ptr(plan.inv_ptr), nat.ptr(plan.inv_pos),
+                                              nat.ptr(luts), nat.ptr(gy), nat.ptr(gx), nat.ptr(gl), nat.ptr(ws), ws.numel(),
+                                              *ctx.dims, nat.stream()))
+        else:
+            ws = _bytes(lib.dl_hybrid_bwd_saved_workspace_bytes(*ctx.dims), gy.device)
+            nat.check(lib.dl_hybrid_layer_bwd_saved(nat.ptr(x), nat.ptr(tiles), nat.ptr(plan.idx32), nat.ptr(plan.inv_ptr),
+                                                    nat.ptr(plan.inv_pos), nat.ptr(luts), nat.ptr(gy), nat.ptr(gx),
+                                                    nat.ptr(gl), nat.ptr(ws), ws.numel(), *ctx.dims, nat.stream()))
+        return gx, gl, None, None
 
 
 # ----------------------------------------------------------------------------- Probabilistic
@@ -753,7 +776,10 @@ def dwn_stable_layer(x, luts, scale, plan):
 
 
 def hybrid_layer(x, luts, plan):
-    return HybridLayerFunction.apply(x, luts, plan) if x.is_cuda else cpu_ops.hybrid_layer(x, luts, plan)
+    if not x.is_cuda:
+        return cpu_ops.hybrid_layer(x, luts, plan)
+    keep = torch.is_grad_enabled() and (x.requires_grad or luts.requires_grad)  # a backward may follow
+    return HybridLayerFunction.apply(x, luts, plan, keep)
 
 
 def table_sigmoid(raw):

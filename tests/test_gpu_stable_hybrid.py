@@ -99,6 +99,31 @@ def test_stable_no_input_grad_and_scalar_scale():
         ops.DWNStableLayerFunction.apply(dev(x), dev(orc.table_sigmoid(raw)), torch.ones(N + 1, device=DEV), plan)
 
 
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1, 1), (64, 64, 16, 6, 1), (65, 63, 70, 6, 1), (130, 1000, 300, 4, 2),
+                                   (63, 4101, 129, 5, 1), (200, 128, 40, 3, 1)])
+@pytest.mark.parametrize("aligned", [True, False])
+def test_hybrid_forward_that_keeps_the_tiles_is_the_one_that_does_not(shape, aligned):
+    """The pass that re-tiles x and takes its bit-planes against the separate passes: the same sums in the same order, so
+    the same bits; thresholds at 0.5, NaN and infinities included."""
+    B, I, N, k, O = shape
+    ops = _ops()
+    g = torch.Generator().manual_seed(sum(shape))
+    buf = torch.rand(B * I + 1, generator=g)
+    buf[::7], buf[3::31], buf[5::41] = 0.5, float("nan"), float("inf")
+    x = buf.to(DEV)[0 if aligned else 1:][:B * I].view(B, I)
+    idx = torch.randint(0, I, (N, k), generator=g, dtype=torch.int32)
+    plan = ops.MappingPlan(idx.to(DEV), I)
+    luts, gy = torch.rand(N, O, 1 << k, generator=g).to(DEV), torch.randn(B, N * O, generator=g).to(DEV)
+    results = []
+    for keep in (True, False):
+        xt, lt = x.detach().requires_grad_(), luts.clone().requires_grad_()
+        y = ops.HybridLayerFunction.apply(xt, lt, plan, keep)
+        y.backward(gy)
+        results.append([t.detach().cpu().view(torch.int32) for t in (y, xt.grad, lt.grad)])
+    for kept, apart in zip(*results):
+        assert torch.equal(kept, apart)
+
+
 @pytest.mark.parametrize("shape", SHAPES)
 def test_hybrid_layer_forward_backward(shape):
     B, I, N, k, O = shape
