@@ -741,10 +741,13 @@ __global__ __launch_bounds__(256) void dwn_bwd_hist_tiled(const float *__restric
 // per step with wave-uniform addressing: the 8 x 3 vector loads of a step are requested together,
 // then evaluated.  The entries of one input are consecutive, so its sum is
 // kept in a register and written to the LDS tile once, in CSR order (reproducible sums).
+// OC = outputs per node whose gradients and coefficient rows are requested with the step (1 or 2); 0: any number, walked one
+// after the other while the entry is evaluated, one load at a time.  Two outputs per node, walked -> requested: 1000 rows,
+// 3137 -> 2999 nodes of five inputs 58.6 -> 30.0 us; 4096 rows, 8192 -> 4096 nodes of six 212 -> 128 us.
 #define DWN_WI 16        // inputs per wavefront (slab of 64 inputs per block)
 #define DWN_WI_SMALL 4   // for layers with long CSR lists per input: slabs of 16 inputs
 #define DWN_EG 8
-template <int K, bool O1, bool SFORM, int WI = DWN_WI>
+template <int K, int OC, bool SFORM, int WI = DWN_WI>
 __global__ __launch_bounds__(256) void dwn_bwd_gx(const float *__restrict__ gyT, const uint8_t *__restrict__ addrT,
                                                    const float *__restrict__ D, const int *__restrict__ inv_ptr,
                                                    const int *__restrict__ inv_pos, float *__restrict__ gx,
@@ -770,12 +773,13 @@ __global__ __launch_bounds__(256) void dwn_bwd_gx(const float *__restrict__ gyT,
     for (int r = 0; r < WI; ++r) tile[wbeg + r][lane] = 0.0f;  // inputs nobody reads keep 0
     const int ebeg = __builtin_amdgcn_readlane(myptr, 0);
     const int eend = __builtin_amdgcn_readlane(myptr, WI);
+    constexpr int ND = OC > 0 ? OC : 1;
     constexpr int NR = !SFORM && Lh > 64 ? Lh / 64 : 1;  // registers of a coefficient row
     struct Group {
         int rj[DWN_EG], ri[DWN_EG];
         bool live[DWN_EG];
         unsigned a[DWN_EG];
-        float g[DWN_EG], coef[DWN_EG][NR];
+        float g[DWN_EG][ND], coef[DWN_EG][ND][NR];
     };
     float acc = 0.0f;  // running sum of the input `cur`
     int cur = -1;
@@ -785,11 +789,11 @@ __global__ __launch_bounds__(256) void dwn_bwd_gx(const float *__restrict__ gyT,
     // so there is no bookkeeping per entry.  Same order of additions as the general loop below.
     constexpr int FAN = 3;
     bool uniform3 = false;
-    if (WI == 16 && O1 && SFORM) {
+    if (WI == 16 && OC == 1 && SFORM) {
         const int len = __shfl_down(myptr, 1) - myptr;  // lanes 0..15: entries of my input
         uniform3 = __ballot(lane >= WI || len == FAN) == ~0ull;
     }
-    if (WI == 16 && O1 && SFORM && uniform3) {
+    if (WI == 16 && OC == 1 && SFORM && uniform3) {
         const int p = lane < WI * FAN ? inv_pos[ebeg + lane] : 0;
         const int n = p / K;
         const int rec = (n << 3) | (p - n * K);
@@ -840,16 +844,20 @@ __global__ __launch_bounds__(256) void dwn_bwd_gx(const float *__restrict__ gyT,
                 G.rj[q] = (rr >> 5) & 7;
                 G.ri[q] = rr & 31;
                 G.a[q] = addr_t[(size_t)rn * 64];
-                if (O1) {
-                    G.g[q] = gy_t[(size_t)rn * 64];
-                    if (SFORM)
-                        G.coef[q][0] = D[(size_t)rn * (2 * Lh) + (lane & (2 * Lh - 1))];
-                    else
+                if (OC > 0) {
 #pragma unroll
-                        for (int r2 = 0; r2 < NR; ++r2)
-                            G.coef[q][r2] = D[((size_t)rn * K + G.rj[q]) * Lh + (lane & (Lh - 1)) + r2 * 64];
+                    for (int d = 0; d < ND; ++d) {
+                        const size_t c = (size_t)rn * ND + d;
+                        G.g[q][d] = gy_t[c * 64];
+                        if (SFORM)
+                            G.coef[q][d][0] = D[c * (2 * Lh) + (lane & (2 * Lh - 1))];
+                        else
+#pragma unroll
+                            for (int r2 = 0; r2 < NR; ++r2)
+                                G.coef[q][d][r2] = D[(c * K + G.rj[q]) * Lh + (lane & (Lh - 1)) + r2 * 64];
+                    }
                 } else {
-                    G.g[q] = __int_as_float(rn);  // node number; outputs are walked in evaluate()
+                    G.g[q][0] = __int_as_float(rn);  // node number; outputs are walked in evaluate()
                 }
             }
         };
@@ -860,14 +868,21 @@ __global__ __launch_bounds__(256) void dwn_bwd_gx(const float *__restrict__ gyT,
                 const int j_ = G.rj[q];
                 const unsigned ap = (G.a[q] & ((1u << j_) - 1u)) | ((G.a[q] >> (j_ + 1)) << j_);
                 float term;
-                if (O1 && SFORM) {
-                    const float hi = dl_lane_read(G.coef[q][0], (int)(G.a[q] | (1u << j_)));
-                    const float lo = dl_lane_read(G.coef[q][0], (int)(G.a[q] & ~(1u << j_)));
-                    term = G.g[q] * (hi - lo);
-                } else if (O1) {
-                    term = G.g[q] * dwn_table_read<NR>(G.coef[q], ap);
+                if (OC > 0) {
+                    term = 0.0f;
+#pragma unroll
+                    for (int d = 0; d < ND; ++d) {
+                        float coef;
+                        if (SFORM)
+                            coef = dl_lane_read(G.coef[q][d][0], (int)(G.a[q] | (1u << j_))) -
+                                   dl_lane_read(G.coef[q][d][0], (int)(G.a[q] & ~(1u << j_)));
+                        else
+                            coef = dwn_table_read<NR>(G.coef[q][d], ap);
+                        if (OC == 1) term = G.g[q][d] * coef;
+                        else term += G.g[q][d] * coef;
+                    }
                 } else {
-                    const int rn = __float_as_int(G.g[q]);
+                    const int rn = __float_as_int(G.g[q][0]);
                     term = 0.0f;
                     for (int d = 0; d < O; ++d) {
                         const size_t c = (size_t)rn * O + d;
@@ -1533,23 +1548,25 @@ static void dwn_launch_gx(const float *gyT, const uint8_t *addrT, const float *D
     // 179 us); 31 - 4 (368 vs 442 us); 69 with tile-major output - 1 (249 vs 265 vs 375 us).
     if (O == 1 && sform && out_tiled && (long long)N * K >= 32LL * I) {
         const int grid_s = dl_xcd_grid(dl_ceil_div(I, 4), BT);
-        DL_TIMED("dwn_bwd_gx", s, (dwn_bwd_gx<K, true, true, 1><<<grid_s + rb, 256, 0, s>>>(gyT, addrT, D, inv_ptr, inv_pos, gx, B,
+        DL_TIMED("dwn_bwd_gx", s, (dwn_bwd_gx<K, 1, true, 1><<<grid_s + rb, 256, 0, s>>>(gyT, addrT, D, inv_ptr, inv_pos, gx, B,
                                                                                           I, N, O, BT, out_tiled, grid_s, red)));
         return;
     }
     if (O == 1 && sform && (long long)N * K >= 6LL * I) {
         const int grid_s = dl_xcd_grid(dl_ceil_div(I, 4 * DWN_WI_SMALL), BT);
-        DL_TIMED("dwn_bwd_gx", s, (dwn_bwd_gx<K, true, true, DWN_WI_SMALL><<<grid_s + rb, 256, 0, s>>>(
+        DL_TIMED("dwn_bwd_gx", s, (dwn_bwd_gx<K, 1, true, DWN_WI_SMALL><<<grid_s + rb, 256, 0, s>>>(
                                       gyT, addrT, D, inv_ptr, inv_pos, gx, B, I, N, O, BT, out_tiled, grid_s, red)));
         return;
     }
     const int grid = dl_xcd_grid(dl_ceil_div(I, 4 * DWN_WI), BT);
 #define DWN_GX(O1_, S_) \
     DL_TIMED("dwn_bwd_gx", s, (dwn_bwd_gx<K, O1_, S_><<<grid + rb, 256, 0, s>>>(gyT, addrT, D, inv_ptr, inv_pos, gx, B, I, N, O, BT, out_tiled, grid, red)))
-    if (O == 1 && sform) DWN_GX(true, true);
-    else if (O == 1) DWN_GX(true, false);
-    else if (sform) DWN_GX(false, true);
-    else DWN_GX(false, false);
+    if (O == 1 && sform) DWN_GX(1, true);
+    else if (O == 1) DWN_GX(1, false);
+    else if (O == 2 && sform) DWN_GX(2, true);
+    else if (O == 2) DWN_GX(2, false);
+    else if (sform) DWN_GX(0, true);
+    else DWN_GX(0, false);
 #undef DWN_GX
 }
 
@@ -1557,10 +1574,16 @@ template <int K>
 static void dwn_launch_gx_wide(const float *gyT, const uint8_t *addrT, const float *D, const int *inv_ptr, const int *inv_pos,
                                float *gx, int B, int I, int N, int O, const DwnReduce &red, hipStream_t s) {
     const int BT = dwn_bt(B), rb = dwn_reduce_blocks(red);
-#define DWN_GX(O1_, WI_)                                                                                                 do {                                                                                                                     const int grid = dl_xcd_grid(dl_ceil_div(I, 4 * WI_), BT);                                                           DL_TIMED("dwn_bwd_gx", s, (dwn_bwd_gx<K, O1_, false, WI_><<<grid + rb, 256, 0, s>>>(                                                               gyT, addrT, D, inv_ptr, inv_pos, gx, B, I, N, O, BT, 0, grid, red)));              } while (0)
-    if (O == 1 && (long long)N * K >= 6LL * I) DWN_GX(true, DWN_WI_SMALL);  // the rule of dwn_launch_gx
-    else if (O == 1) DWN_GX(true, DWN_WI);
-    else DWN_GX(false, DWN_WI);
+#define DWN_GX(O1_, WI_)                                                                                        \
+    do {                                                                                                        \
+        const int grid = dl_xcd_grid(dl_ceil_div(I, 4 * WI_), BT);                                              \
+        DL_TIMED("dwn_bwd_gx", s, (dwn_bwd_gx<K, O1_, false, WI_><<<grid + rb, 256, 0, s>>>(                    \
+                                      gyT, addrT, D, inv_ptr, inv_pos, gx, B, I, N, O, BT, 0, grid, red)));     \
+    } while (0)
+    if (O == 1 && (long long)N * K >= 6LL * I) DWN_GX(1, DWN_WI_SMALL);  // the rule of dwn_launch_gx
+    else if (O == 1) DWN_GX(1, DWN_WI);
+    else if (O == 2) DWN_GX(2, DWN_WI);
+    else DWN_GX(0, DWN_WI);
 #undef DWN_GX
 }
 

@@ -70,6 +70,27 @@ def test_dwn_layer_forward_backward(shape):
     np.testing.assert_allclose(lt.grad.cpu().numpy(), gl, rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1, 2), (64, 17, 40, 6, 2), (65, 130, 61, 5, 2), (130, 9, 33, 3, 2), (66, 64, 30, 8, 2),
+                                   (66, 64, 30, 7, 2), (70, 33, 20, 4, 3)])
+@pytest.mark.parametrize("beta", [1.0 / 3.0, 0.75])  # both forms of the coefficient table
+def test_dwn_backward_several_outputs_per_node(shape, beta):
+    """Two outputs per node are requested with a step's entries, three and more are walked: both forms, lists shorter and
+    longer than a step of eight."""
+    B, I, N, k, O = shape
+    ops = _ops()
+    x, idx, luts, gy = make_case(sum(shape) + 5, *shape)
+    plan = ops.MappingPlan(dev(idx, torch.int32), I)
+    xt, lt = dev(x).requires_grad_(), dev(luts).requires_grad_()
+    alpha = 0.5 * 0.75 ** (k - 1)
+    ops.DWNLayerFunction.apply(xt, lt, plan, alpha, beta).backward(dev(gy.reshape(B, N * O)))
+    gx, gl = orc.dwn_layer_backward(x, idx, luts, gy, np.float32(alpha), np.float32(beta))
+    # a term is alpha |gy| |D| with |D| <= 2 (1 + beta)^(k-1) |lut|, at most 11.3 |gy| here (k = 8, beta = 0.75), and a sum has
+    # O N k / I of them: 64 roundings of 6e-8 of terms of that size, as an absolute floor
+    size = alpha * 2.0 * (1.0 + beta) ** (k - 1)
+    np.testing.assert_allclose(xt.grad.cpu().numpy(), gx, rtol=1e-5, atol=max(2e-6, 64 * 6e-8 * size))
+    np.testing.assert_allclose(lt.grad.cpu().numpy(), gl, rtol=1e-5, atol=1e-5)
+
+
 @pytest.mark.parametrize("shape", [(33000, 50, 300, 6, 1), (40000, 7, 40, 2, 1)])
 def test_dwn_backward_few_inputs_many_rows(shape):
     """Few inputs read by many nodes over many rows (the shape of the first level of a convolutional layer:
