@@ -52,18 +52,32 @@ __device__ __forceinline__ unsigned softmap_pk_bf16(float lo, float hi) {
 __device__ __forceinline__ float softmap_lo(unsigned p) { return __uint_as_float(p << 16); }
 __device__ __forceinline__ float softmap_hi(unsigned p) { return __uint_as_float(p & 0xffff0000u); }
 
-// Plane `p` of eight values as a unit; v is replaced by what is left for the planes below.
-__device__ __forceinline__ uint4 softmap_unit(float *v) {
+// The next plane of eight values as a unit; v is replaced by what is left for the planes below.  Finite values of `cut` and
+// above (0: none) are cut to 8 bits instead of rounded: float32's largest values would round to an infinity, and what the
+// first cut left would round up to a sum of planes that is one.  The planes still add up to the value.
+__device__ __forceinline__ uint4 softmap_unit(float *v, float cut = 0.0f) {
     unsigned w[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const float a = v[2 * j], b = v[2 * j + 1];
         w[j] = softmap_pk_bf16(a, b);
+        if (cut > 0.0f) {
+            if (fabsf(a) >= cut && __builtin_isfinite(a)) w[j] = (w[j] & 0xffff0000u) | (__float_as_uint(a) >> 16);
+            if (fabsf(b) >= cut && __builtin_isfinite(b)) w[j] = (w[j] & 0xffffu) | (__float_as_uint(b) & 0xffff0000u);
+        }
         const float ra = a - softmap_lo(w[j]), rb = b - softmap_hi(w[j]);
         v[2 * j] = __builtin_isfinite(softmap_lo(w[j])) ? ra : 0.0f;
         v[2 * j + 1] = __builtin_isfinite(softmap_hi(w[j])) ? rb : 0.0f;
     }
     return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+// Where plane p of an operand of NP planes is cut: 2^127 and above first (one plane rounds, as any conversion to bf16 does),
+// then what that leaves from 2^119 on; less than that cannot carry the first plane, at most 2^128 - 2^120, over the top.
+// E is at most 1.
+template <int NP>
+__device__ __forceinline__ constexpr float softmap_cut(int p) {
+    return NP == 1 || p > 1 ? 0.0f : p == 0 ? 0x1p127f : 0x1p119f;
 }
 
 // ---------------------------------------------------------------------------------
@@ -201,7 +215,7 @@ __global__ __launch_bounds__(256) void softmap_pack(const float *__restrict__ sr
             if (8 * rb < Rp) {
                 char *d = rows8 + ((size_t)rb * Cp + col) * SM_UNIT;
 #pragma unroll
-                for (int p = 0; p < NP; ++p) *reinterpret_cast<uint4 *>(d + p * rows_plane) = softmap_unit(v + 8 * h);
+                for (int p = 0; p < NP; ++p) *reinterpret_cast<uint4 *>(d + p * rows_plane) = softmap_unit(v + 8 * h, softmap_cut<NP>(p));
             }
         }
     }
@@ -215,7 +229,7 @@ __global__ __launch_bounds__(256) void softmap_pack(const float *__restrict__ sr
                 for (int j = 0; j < 8; ++j) w[j] = tile[c][cb * 8 + j];
                 char *d = cols8 + ((size_t)(blockIdx.x * 8 + cb) * Rp + row) * SM_UNIT;
 #pragma unroll
-                for (int p = 0; p < NP; ++p) *reinterpret_cast<uint4 *>(d + p * cols_plane) = softmap_unit(w);
+                for (int p = 0; p < NP; ++p) *reinterpret_cast<uint4 *>(d + p * cols_plane) = softmap_unit(w, softmap_cut<NP>(p));
             }
         }
     }

@@ -167,6 +167,8 @@ class DWNLayerFunction(torch.autograd.Function):
         nat.check(lib.dl_dwn_layer_fwd(nat.ptr(x), nat.ptr(plan.idx32), nat.ptr(luts), nat.ptr(y), nat.ptr(saved),
                                        nat.ptr(ws), ws.numel(), *dims, nat.stream()))
         if torch.is_tensor(alpha) or torch.is_tensor(beta):
+            if any(torch.is_tensor(v) and v.dim() > 1 for v in (alpha, beta)):
+                raise RuntimeError("alpha and beta of a layer are numbers or tensors [N]")
             alpha, beta = _per_node(alpha, N, x.device), _per_node(beta, N, x.device)
             if beta_abs_max is None:
                 beta_abs_max = float(beta.abs().max())

@@ -699,6 +699,23 @@ def test_soft_mapping_tile_edges(shape, precision):
         assert float((got.double() - want).norm()) <= limit * float(size)
 
 
+@pytest.mark.parametrize("value", [float(np.finfo(np.float32).min), 3.3999999e38, 3.38e38])
+def test_soft_mapping_of_values_beyond_bf16(value):
+    """Finite float32 values up to the largest stay finite through the bf16 planes (3.39e38 and above would round to an
+    infinity, and the lowest value's two upper planes could add up to one).  Each output is one dominant product, or a sum
+    of terms of one sign: 1e-5 of it, as above."""
+    ops = _ops()
+    g = torch.Generator("cuda").manual_seed(5)
+    x = torch.rand(70, 200, device="cuda", generator=g)
+    x[::3, 17] = value
+    W = torch.randn(130, 200, device="cuda", generator=g) * 0.5
+    W[::2, 17] = 4.0  # the largest of its row: the value itself is summed
+    m = ops.SoftMapFunction.apply(x, W, 1.0, 0)
+    want = x.double() @ torch.softmax(W.double(), dim=-1).t()
+    assert torch.isfinite(m).all()
+    assert float(((m.double() - want).abs() / want.abs()).max()) <= 1e-5
+
+
 def test_soft_and_hard_mapping_against_reference_vectors(golden):
     ops = _ops()
     g = golden
