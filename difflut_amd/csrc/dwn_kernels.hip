@@ -946,6 +946,75 @@ __global__ __launch_bounds__(256) void dwn_bwd_gx(const float *__restrict__ gyT,
 }
 
 // ---------------------------------------------------------------------------------
+// bwd_gx_long: the same sums, tile-major, for inputs with long CSR lists (the patch columns of a convolution, 69 entries each).
+// A wavefront keeps one input and takes DWN_LT batch tiles at once: an entry is decoded and its coefficient row loaded once
+// for all of them, and the address and gradient rows of four entries x four tiles are in flight together.  Bound by those
+// rows, 320 bytes per entry and tile from the L2.  First level of convolutional trees (100 columns, 1152 nodes, 147456
+// rows): the layer's training step 1107 -> 960 us.  A lane past the end of the list loads entry 0's rows and adds nothing: a branch
+// around it would keep the compiler from requesting the step's loads together.
+#define DWN_LT 4  // batch tiles per wavefront
+#define DWN_LE 4  // entries per step
+template <int K>
+__global__ __launch_bounds__(256) void dwn_bwd_gx_long(const float *__restrict__ gyT, const uint8_t *__restrict__ addrT,
+                                                        const float *__restrict__ D, const int *__restrict__ inv_ptr,
+                                                        const int *__restrict__ inv_pos, float *__restrict__ gx, int I,
+                                                        int N, int BT, int gather_blocks, DwnReduce red) {
+    if ((int)blockIdx.x >= gather_blocks) return dwn_reduce_block(red, (int)blockIdx.x - gather_blocks);
+    constexpr int L = 1 << K;
+    int slab, group;
+    if (!dl_xcd_map((I + 3) / 4, (BT + DWN_LT - 1) / DWN_LT, slab, group)) return;
+    const int lane = threadIdx.x & 63;
+    const int i = slab * 4 + dl_uniform(threadIdx.x >> 6);
+    if (i >= I) return;
+    const int t0 = group * DWN_LT;
+    const uint8_t *addr_t[DWN_LT];
+    const float *gy_t[DWN_LT];
+    float acc[DWN_LT];
+#pragma unroll
+    for (int u = 0; u < DWN_LT; ++u) {
+        const size_t first = (size_t)min(t0 + u, BT - 1) * N * 64;  // tiles past the last repeat it and are not stored
+        addr_t[u] = addrT + first;
+        gy_t[u] = gyT + first;
+        acc[u] = 0.0f;
+    }
+    const int ebeg = dl_uniform(inv_ptr[i]), eend = dl_uniform(inv_ptr[i + 1]);
+    for (int base = ebeg; base < eend; base += 64) {
+        const int p = base + lane < eend ? inv_pos[base + lane] : 0;
+        const int n = p / K;
+        const int rec = (n << 3) | (p - n * K);
+        const int cnt = min(64, eend - base);
+        for (int s0 = 0; s0 < cnt; s0 += DWN_LE) {
+            int rj[DWN_LE];
+            unsigned a[DWN_LE][DWN_LT];
+            float g[DWN_LE][DWN_LT], coef[DWN_LE];
+#pragma unroll
+            for (int q = 0; q < DWN_LE; ++q) {  // s0 + q <= 63: s0 is a multiple of DWN_LE
+                const int r = __builtin_amdgcn_readlane(rec, s0 + q);
+                const int rn = r >> 3;
+                rj[q] = r & 7;
+#pragma unroll
+                for (int u = 0; u < DWN_LT; ++u) {
+                    a[q][u] = addr_t[u][(size_t)rn * 64 + lane];
+                    g[q][u] = gy_t[u][(size_t)rn * 64 + lane];
+                }
+                coef[q] = D[(size_t)rn * L + (lane & (L - 1))];
+            }
+#pragma unroll
+            for (int q = 0; q < DWN_LE; ++q)
+#pragma unroll
+                for (int u = 0; u < DWN_LT; ++u) {
+                    const float term = g[q][u] * (dl_lane_read(coef[q], (int)(a[q][u] | (1u << rj[q]))) -
+                                                  dl_lane_read(coef[q], (int)(a[q][u] & ~(1u << rj[q]))));
+                    acc[u] = s0 + q < cnt ? acc[u] + term : acc[u];
+                }
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < DWN_LT; ++u)
+        if (t0 + u < BT) __builtin_nontemporal_store(acc[u], &gx[((size_t)(t0 + u) * I + i) * 64 + lane]);
+}
+
+// ---------------------------------------------------------------------------------
 // bwd_gx_walk: the input gradient by blocks that keep their slab of 64 inputs and walk batch tiles, in two roles.
 // HIST (chained layers): written tile-major, with the table-gradient histogram of the layer IN FRONT folded in.  In a
 // chain the input gradient of layer l + 1 is the output gradient of layer l: column i of it, together with the addresses
@@ -1546,6 +1615,16 @@ static void dwn_launch_gx(const float *gyT, const uint8_t *addrT, const float *D
     // mapping) want fewer inputs per wavefront: more, shorter and evenly filled blocks.  Measured at B = 4096, k = 6:
     // lists of 3 - 16 inputs per wavefront is best (169 vs 221 us); 7.7 - 4 inputs (67 vs 73 us); 15 - 4 (134 vs
     // 179 us); 31 - 4 (368 vs 442 us); 69 with tile-major output - 1 (249 vs 265 vs 375 us).
+    // There four batch tiles per wavefront (dwn_bwd_gx_long) once the blocks fill the card; below 2048 they do not. By rows
+    // (100 columns, 1152 nodes), one tile / four, us, with a form of it that gained half as much: 147456 rows 587 / 525, 36864
+    // 152 / 147, 18432 (1800 blocks) 81.5 / 83.5, 9216 46 / 50, 4608 27 / 40.
+    if (O == 1 && sform && out_tiled && (long long)N * K >= 32LL * I &&
+        (long long)dl_ceil_div(I, 4) * dl_ceil_div(BT, DWN_LT) >= 2048) {
+        const int grid_l = dl_xcd_grid(dl_ceil_div(I, 4), dl_ceil_div(BT, DWN_LT));
+        DL_TIMED("dwn_bwd_gx", s, (dwn_bwd_gx_long<K><<<grid_l + rb, 256, 0, s>>>(gyT, addrT, D, inv_ptr, inv_pos, gx, I, N, BT,
+                                                                                   grid_l, red)));
+        return;
+    }
     if (O == 1 && sform && out_tiled && (long long)N * K >= 32LL * I) {
         const int grid_s = dl_xcd_grid(dl_ceil_div(I, 4), BT);
         DL_TIMED("dwn_bwd_gx", s, (dwn_bwd_gx<K, 1, true, 1><<<grid_s + rb, 256, 0, s>>>(gyT, addrT, D, inv_ptr, inv_pos, gx, B,

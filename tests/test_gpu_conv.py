@@ -201,6 +201,26 @@ def test_grouped_connections_cover_every_channel(seed):
     assert y.shape == (2, 16, 6, 6) and torch.isfinite(y).all()
 
 
+def test_conv_gather_of_four_batch_tiles_equals_that_of_one():
+    """29 images of 28 x 28 are 261 batch tiles of patches and 125 columns, 66 x 32 blocks of the gather that takes four tiles
+    per wavefront: the last group has one tile, the last block one column.  15 + 14 images stay with one tile:
+    same terms in the same order, so the same bits."""
+    torch.manual_seed(21)
+    layer = _build("dwn", 2, 5, 32, 5, 1, 0, 32).train()
+    assert layer.bank_parameters()[0].shape[0] == 1152
+    x = (torch.rand(29, 5, 28, 28, device=DEV) < 0.5).float()
+    gy = torch.randn(29, 32, 24, 24, device=DEV)
+
+    def gradient(rows):
+        part = x[rows].clone().requires_grad_()
+        layer(part).backward(gy[rows])
+        return part.grad
+
+    whole = gradient(slice(0, 29))
+    assert whole.abs().max() > 0
+    assert torch.equal(whole, torch.cat([gradient(slice(0, 15)), gradient(slice(15, 29))]))
+
+
 def test_conv_bank_parameters_train_in_place():
     """An optimizer over bank_parameters() (one tensor per depth level) updates the per-node parameters the
     state dict shows."""
