@@ -950,7 +950,7 @@ __global__ __launch_bounds__(256) void dwn_bwd_gx(const float *__restrict__ gyT,
 // A wavefront keeps one input and takes DWN_LT batch tiles at once: an entry is decoded and its coefficient row loaded once
 // for all of them, and the address and gradient rows of four entries x four tiles are in flight together.  Bound by those
 // rows, 320 bytes per entry and tile from the L2.  First level of convolutional trees (100 columns, 1152 nodes, 147456
-// rows): the layer's training step 1107 -> 960 us.  A lane past the end of the list loads entry 0's rows and adds nothing: a branch
+// rows): 608 -> 463 us a launch, the layer's training step 1107 -> 960.  A lane past the end of the list loads entry 0's rows and adds nothing: a branch
 // around it would keep the compiler from requesting the step's loads together.
 #define DWN_LT 4  // batch tiles per wavefront
 #define DWN_LE 4  // entries per step
@@ -1615,9 +1615,9 @@ static void dwn_launch_gx(const float *gyT, const uint8_t *addrT, const float *D
     // mapping) want fewer inputs per wavefront: more, shorter and evenly filled blocks.  Measured at B = 4096, k = 6:
     // lists of 3 - 16 inputs per wavefront is best (169 vs 221 us); 7.7 - 4 inputs (67 vs 73 us); 15 - 4 (134 vs
     // 179 us); 31 - 4 (368 vs 442 us); 69 with tile-major output - 1 (249 vs 265 vs 375 us).
-    // There four batch tiles per wavefront (dwn_bwd_gx_long) once the blocks fill the card; below 2048 they do not. By rows
-    // (100 columns, 1152 nodes), one tile / four, us, with a form of it that gained half as much: 147456 rows 587 / 525, 36864
-    // 152 / 147, 18432 (1800 blocks) 81.5 / 83.5, 9216 46 / 50, 4608 27 / 40.
+    // There four batch tiles per wavefront (dwn_bwd_gx_long) once there are blocks enough. By rows (100
+    // columns, 1152 nodes), one tile / four, us: 147456 rows 608 / 463, 36864 157 / 127, 23040 (2250 blocks) 103 / 88.  The gain
+    // shrinks towards the line; a slower form of the kernel lost below it (18432 rows 81.5 / 83.5, 9216 46 / 50, 4608 27 / 40).
     if (O == 1 && sform && out_tiled && (long long)N * K >= 32LL * I &&
         (long long)dl_ceil_div(I, 4) * dl_ceil_div(BT, DWN_LT) >= 2048) {
         const int grid_l = dl_xcd_grid(dl_ceil_div(I, 4), dl_ceil_div(BT, DWN_LT));
