@@ -3,11 +3,11 @@
 //
 //   forward   m[b,o]  = rs[o] * sum_i x[b,i] E[o,i]          E = exp((W - max)/tau), rs = 1 / row sum
 //   backward  gx[b,i] = sum_o gs[b,o] E[o,i]                  gs = gm * rs
-//             gW[o,i] = E[o,i] (G[o,i] - rs[o] r[o]) / tau    G = gs^T x, r[o] = sum_b gm[b,o] m[b,o]
-//             (r is the row sum of (gm^T x) * S written through the saved forward output, so the M x I
+//             gW[o,i] = rs[o] E[o,i] (G[o,i] - r[o]) / tau    G = gm^T x, r[o] = sum_b gm[b,o] m[b,o]
+//             (r is the row sum of G * S written through the saved forward output, so the M x I
 //              matrix G never needs a second pass)
 //
-// Operands.  precision 1 rounds x, E and gs to bf16 once (nearest even).  precision 0 keeps fp32 values: every operand
+// Operands.  precision 1 rounds x, E, gs (for gx) and gm (for gW) to bf16 once (nearest even).  precision 0 keeps fp32 values: every operand
 // is the EXACT sum of three bf16 planes (8 + 8 + 8 significant bits, each the rounding of what the planes above left), and
 // a product is the six plane products hi*hi, hi*mid, mid*hi, mid*mid, hi*lo, lo*hi.  The three products left out are
 // below 2^-26 of |a*b| (|mid| <= 2^-9 |a|, |lo| <= 2^-18 |a|), less than the 2^-24 by which one fp32 multiply-add rounds,
@@ -172,8 +172,8 @@ __global__ __launch_bounds__(T) void softmap_rowstats(const float *__restrict__ 
 }
 
 // ---------------------------------------------------------------------------------
-// src [R][C] fp32 -> units along the rows [Rp/8][Cp] and / or along the columns [Cp/8][Rp], NP planes each, scaled per
-// column where `colscale` is given, padding zero.  With `other`: dots[chunk][c] = sum of src * other over the 64 rows of
+// src [R][C] fp32 -> units along the rows [Rp/8][Cp] and / or along the columns [Cp/8][Rp], NP planes each, the latter scaled
+// per column where `colscale` is given, padding zero.  With `other`: dots[chunk][c] = sum of src * other over the 64 rows of
 // the chunk (unscaled; the reader adds the chunks in order).  Block = 64 columns x 64 rows: a thread has sixteen rows of a
 // column, so units along the rows leave straight from registers; those along the columns go through the LDS (row
 // stride 65 words, no conflicts).
@@ -202,10 +202,7 @@ __global__ __launch_bounds__(256) void softmap_pack(const float *__restrict__ sr
         part[g][c] = dot;
     }
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        v[i] *= f;
-        tile[g * 16 + i][c] = v[i];
-    }
+    for (int i = 0; i < 16; ++i) tile[g * 16 + i][c] = v[i] * f;
     __syncthreads();
     if (other && g == 0) dots[(size_t)blockIdx.y * Cp + col] = ((part[0][c] + part[1][c]) + part[2][c]) + part[3][c];
     if (rows8) {
@@ -303,7 +300,7 @@ __device__ __forceinline__ void softmap_stage_barrier() {
 // products, the latter what the matrix cores hold under power; gW adds 602 MB of stores and 301 (602) MB of reads.
 // MODE 0: forward   rows=b cols=o red=i   A = x    B = E (turned)   out = C rs[o]
 // MODE 1: gx        rows=b cols=i red=o   A = gs   B = E
-// MODE 2: gW        rows=o cols=i red=b   A = gs   B = x            out = E (C - rs r) / tau
+// MODE 2: gW        rows=o cols=i red=b   A = gm   B = x            out = rs E (C - r) / tau
 // Block = 256 threads = 2 x 2 wavefronts, tile 64 FA x 128, a wavefront FA x 2 MFMA tiles of 32 x 32.  FA = 4 (256 rows):
 // per MFMA a block pulls 24 KB per 32 reduction steps (NP = 1), 48 bytes per clock and CU at the matrix peak where
 // 128 x 128 tiles need 64, all that an L2 channel delivers.  Two blocks share a CU (accumulators 128 registers, 72 KB of LDS
@@ -443,20 +440,21 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
                 }
         }
     } else {
-        // rs r of the tile's rows (the partial r added in order) and, for E rebuilt from W, their maxima
+        // of the tile's rows: r (its parts added in order), for E rebuilt from W the maximum, and rs / tau
         float *rr = reinterpret_cast<float *>(lds);
         softmap_stage_barrier<0>();
         if (tid < TR) {
             float t = 0.0f;
             for (int q = 0; q < g.parts; ++q) t += g.dots[(size_t)q * g.dot_ld + r0 + tid];
-            rr[tid] = t * g.rs[r0 + tid];
+            rr[tid] = t;
             rr[TR + tid] = g.mx[r0 + tid];
+            rr[2 * TR + tid] = g.rs[r0 + tid] * g.inv_tau;
         }
         __syncthreads();
         // 32 rows x 64 columns at a time go through the wavefront's own corner of the LDS, so that a lane owns four consecutive
         // columns of a row: 16-byte stores in runs of 256 bytes
         constexpr int TS = 68;  // floats per staged row: 64 + 4 keeps 16-byte alignment
-        float *stg = rr + 2 * TR + wave * (32 * TS);
+        float *stg = rr + 3 * TR + wave * (32 * TS);
         const int rrow = lane >> 4, c4 = (lane & 15) * 4, col4 = c0 + wn + c4;
         const bool vec = C % 4 == 0 && g.vec_out;
 #pragma unroll
@@ -479,8 +477,9 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
                     float o[4] = {acc[i][j][4 * q] - rv.x, acc[i][j][4 * q + 1] - rv.y, acc[i][j][4 * q + 2] - rv.z,
                                   acc[i][j][4 * q + 3] - rv.w};
                     if (NP == 1) {
-                        o[0] *= softmap_lo(e[j][q].x) * g.inv_tau; o[1] *= softmap_hi(e[j][q].x) * g.inv_tau;
-                        o[2] *= softmap_lo(e[j][q].y) * g.inv_tau; o[3] *= softmap_hi(e[j][q].y) * g.inv_tau;
+                        const float4 fv = *reinterpret_cast<const float4 *>(rr + 2 * TR + lr0 + 8 * q + 4 * kh);
+                        o[0] *= softmap_lo(e[j][q].x) * fv.x; o[1] *= softmap_hi(e[j][q].x) * fv.y;
+                        o[2] *= softmap_lo(e[j][q].y) * fv.z; o[3] *= softmap_hi(e[j][q].y) * fv.w;
                     }
 #pragma unroll
                     for (int n = 0; n < 4; ++n) stg[(8 * q + 4 * kh + n) * TS + j * 32 + l32] = o[n];
@@ -496,9 +495,9 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
                     if (row < R && col4 < C) {
                         if (NP == 3) {
                             const float4 w = *reinterpret_cast<const float4 *>(g.W + at);
-                            const float mx = rr[TR + lr0 + lr];
-                            o.x *= softmap_e(w.x, mx, g.scale) * g.inv_tau; o.y *= softmap_e(w.y, mx, g.scale) * g.inv_tau;
-                            o.z *= softmap_e(w.z, mx, g.scale) * g.inv_tau; o.w *= softmap_e(w.w, mx, g.scale) * g.inv_tau;
+                            const float mx = rr[TR + lr0 + lr], f = rr[2 * TR + lr0 + lr];
+                            o.x *= softmap_e(w.x, mx, g.scale) * f; o.y *= softmap_e(w.y, mx, g.scale) * f;
+                            o.z *= softmap_e(w.z, mx, g.scale) * f; o.w *= softmap_e(w.w, mx, g.scale) * f;
                         }
                         __builtin_nontemporal_store(__builtin_bit_cast(floatx4, o), reinterpret_cast<floatx4 *>(g.out + at));
                     }
@@ -507,7 +506,7 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
 #pragma unroll
                     for (int n = 0; n < 4; ++n)
                         if (row < R && col4 + n < C)
-                            g.out[at + n] = NP == 3 ? os[n] * (softmap_e(g.W[at + n], rr[TR + lr0 + lr], g.scale) * g.inv_tau) : os[n];
+                            g.out[at + n] = NP == 3 ? os[n] * (softmap_e(g.W[at + n], rr[TR + lr0 + lr], g.scale) * rr[2 * TR + lr0 + lr]) : os[n];
                 }
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -587,7 +586,7 @@ extern "C" size_t dl_soft_map_saved_bytes(int B, int I, int M, int precision) {
     return 2 * softmap_vec_bytes(h) + h.np * (h.x_plane + h.e_plane);
 }
 
-// workspace: partial products of the forward or of gx, partial r, x and gs in units along the batch, gs along the rows of W
+// workspace: partial products of the forward or of gx, partial r, x and gm in units along the batch, gs along the rows of W
 static inline size_t softmap_part_bytes(const SoftmapShape &h) {
     const size_t fwd = h.fwd_chunks > 1 ? (size_t)h.fwd_chunks * h.B * h.M : 0, gx = h.gx_chunks > 1 ? (size_t)h.gx_chunks * h.B * h.I : 0;
     return dl_align256((fwd > gx ? fwd : gx) * sizeof(float));
@@ -687,7 +686,7 @@ extern "C" int dl_soft_map_bwd(const float *x, const float *W, float tau, const 
     float *part = (float *)w; w += softmap_part_bytes(h);
     float *dots = (float *)w; w += softmap_dots_bytes(h);
     char *xb = w; w += h.np * h.x_plane;     // x  [Bp/8][Ip]
-    char *gb = w; w += h.np * h.g_plane;     // gs [Bp/8][Mp]
+    char *gb = w; w += h.np * h.g_plane;     // gm [Bp/8][Mp]
     char *go = w;                            // gs [Mp/8][Bp]
     softmap_pack_launch(h.np, x, nullptr, nullptr, nullptr, xb, h.x_plane, nullptr, 0, B, I, h.Bp, h.Ip, s);
     softmap_pack_launch(h.np, gm, rs, m, dots, gb, h.g_plane, go, h.g_plane, B, M, h.Bp, h.Mp, s);

@@ -699,6 +699,27 @@ def test_soft_mapping_tile_edges(shape, precision):
         assert float((got.double() - want).norm()) <= limit * float(size)
 
 
+def test_soft_mapping_bf16_gradient_of_w_takes_gm_itself():
+    """With bf16 operands gW's products are of gm and x rounded once each; 1 / row sum comes in fp32 afterwards.  The same
+    arithmetic in float64 leaves fp32 roundings, and an exponential that falls on the other side of a bf16 rounding boundary
+    (one in 2^15 entries by 2^-8, in the 2-norm 2e-5): 1e-4.  Rounding gm / row sum instead differs by 5e-3."""
+    ops = _ops()
+    B, I, M, tau = 200, 300, 70, 0.7
+    g = torch.Generator("cuda").manual_seed(9)
+    x = torch.rand(B, I, device="cuda", generator=g)
+    W = torch.randn(M, I, device="cuda", generator=g)
+    gm = torch.randn(B, M, device="cuda", generator=g)
+    xt, Wt = x.clone().requires_grad_(), W.clone().requires_grad_()
+    m = ops.SoftMapFunction.apply(xt, Wt, tau, 1)
+    m.backward(gm)
+    E = torch.exp((W - W.max(dim=1, keepdim=True).values) / tau).bfloat16().double()
+    S = E / E.sum(dim=1, keepdim=True)
+    G = gm.bfloat16().double().t() @ x.bfloat16().double()
+    r = (gm.double() * m.detach().double()).sum(0)
+    want = S * (G - r[:, None]) / tau
+    assert float((Wt.grad.double() - want).norm()) <= 1e-4 * float(want.norm())
+
+
 @pytest.mark.parametrize("value", [float(np.finfo(np.float32).min), 3.3999999e38, 3.38e38])
 def test_soft_mapping_of_values_beyond_bf16(value):
     """Finite float32 values up to the largest stay finite through the bf16 planes (3.39e38 and above would round to an
