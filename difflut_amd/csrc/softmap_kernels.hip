@@ -7,14 +7,16 @@
 //             (r is the row sum of G * S written through the saved forward output, so the M x I
 //              matrix G never needs a second pass)
 //
-// Operands.  precision 1 rounds x, E, gs (for gx) and gm (for gW) to bf16 once (nearest even).  precision 0 keeps fp32 values: every operand
-// is the EXACT sum of three bf16 planes (8 + 8 + 8 significant bits, each the rounding of what the planes above left), and
-// a product is the six plane products hi*hi, hi*mid, mid*hi, mid*mid, hi*lo, lo*hi.  The three products left out are
+// Operands.  precision 1 rounds x, E, gs (for gx) and gm (for gW) to bf16 once (nearest even).  precision 0 keeps fp32 values:
+// every operand, times 2^24, is the EXACT sum of three bf16 planes (8 + 8 + 8 significant bits, each the rounding of what
+// the planes above left; the factor keeps the lowest plane of every fp32 value, denormal ones included, a normal number).
+// A product is the six plane products hi*hi, hi*mid, mid*hi, mid*mid, hi*lo, lo*hi.  The three products left out are
 // below 2^-26 of |a*b| (|mid| <= 2^-9 |a|, |lo| <= 2^-18 |a|), less than the 2^-24 by which one fp32 multiply-add rounds,
-// and bf16 products are exact in fp32, so the result is an fp32 product sum: at 512 x 3136 x 6000 gx and gW stand
-// 1.3e-6 and 1.5e-6 from float64 (2-norm), where v_mfma_f32_32x32x2_f32 gave 2.1e-6 and 2.6e-6.  Six bf16 products at
-// 2.5 PFLOP/s are 417 TFLOP/s of fp32 work against 157 on the fp32 matrix cores.  (An infinity keeps its sign in the high
-// plane and has zeros below it: outputs it reaches are infinite or NaN.)
+// and bf16 products are exact in fp32, so the result is an fp32 product sum, times 2^48.  Six bf16 products at
+// 2.5 PFLOP/s are 417 TFLOP/s of fp32 work against 157 on the fp32 matrix cores.
+// Where a sum of an operand's size could overflow with that factor, or as the sum before rs, while the result does not, and
+// for infinities and NaN, which planes do not carry, the product is computed with fp32 multiply-adds instead
+// (softmap_plain): the pack pass notes the largest magnitude (softmap_note_large).
 //
 // Layout.  An MFMA lane wants 8 consecutive reduction steps of one row: a "unit" of 16 bytes.  Every operand is stored
 // as [reduction / 8][rows] units, rows padded to whole tiles with zeros, by the pass that has it in registers anyway
@@ -52,32 +54,34 @@ __device__ __forceinline__ unsigned softmap_pk_bf16(float lo, float hi) {
 __device__ __forceinline__ float softmap_lo(unsigned p) { return __uint_as_float(p << 16); }
 __device__ __forceinline__ float softmap_hi(unsigned p) { return __uint_as_float(p & 0xffff0000u); }
 
-// The next plane of eight values as a unit; v is replaced by what is left for the planes below.  Finite values of `cut` and
-// above (0: none) are cut to 8 bits instead of rounded: float32's largest values would round to an infinity, and what the
-// first cut left would round up to a sum of planes that is one.  The planes still add up to the value.
-__device__ __forceinline__ uint4 softmap_unit(float *v, float cut = 0.0f) {
+#define SM_SCALE 0x1p24f    // of an operand that is cut into planes
+#define SM_UNSCALE 0x1p-48f // of a product of two
+#define SM_LARGE 0x1p16f    // values below need no look at whether a product of theirs could overflow
+#define SM_BOUND 0x1p78f    // times 2^48, and 1 % for the planes' rounding: below 2^127
+
+// The next plane of eight values as a unit; v is replaced by what is left for the planes below.
+__device__ __forceinline__ uint4 softmap_unit(float *v) {
     unsigned w[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const float a = v[2 * j], b = v[2 * j + 1];
-        w[j] = softmap_pk_bf16(a, b);
-        if (cut > 0.0f) {
-            if (fabsf(a) >= cut && __builtin_isfinite(a)) w[j] = (w[j] & 0xffff0000u) | (__float_as_uint(a) >> 16);
-            if (fabsf(b) >= cut && __builtin_isfinite(b)) w[j] = (w[j] & 0xffffu) | (__float_as_uint(b) & 0xffff0000u);
-        }
-        const float ra = a - softmap_lo(w[j]), rb = b - softmap_hi(w[j]);
-        v[2 * j] = __builtin_isfinite(softmap_lo(w[j])) ? ra : 0.0f;
-        v[2 * j + 1] = __builtin_isfinite(softmap_hi(w[j])) ? rb : 0.0f;
+        w[j] = softmap_pk_bf16(v[2 * j], v[2 * j + 1]);
+        v[2 * j] -= softmap_lo(w[j]);
+        v[2 * j + 1] -= softmap_hi(w[j]);
     }
     return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-// Where plane p of an operand of NP planes is cut: 2^127 and above first (one plane rounds, as any conversion to bf16 does),
-// then what that leaves from 2^119 on; less than that cannot carry the first plane, at most 2^128 - 2^120, over the top.
-// E is at most 1.
-template <int NP>
-__device__ __forceinline__ constexpr float softmap_cut(int p) {
-    return NP == 1 || p > 1 ? 0.0f : p == 0 ? 0x1p127f : 0x1p119f;
+// Largest magnitude of an operand, as bits (a NaN is larger than all); stays 0 while every value is below SM_LARGE, which is
+// why the word is hardly ever written.  `big`: the bits of this thread's largest.
+__device__ __forceinline__ void softmap_note_large(unsigned *largest, unsigned big) {
+    if (__ballot(big >= __float_as_uint(SM_LARGE)) == 0) return;
+    for (int off = 32; off > 0; off >>= 1) big = max(big, (unsigned)__shfl_xor((int)big, off));
+    if ((threadIdx.x & 63) == 0 && big > __hip_atomic_load(largest, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(largest, big);
+}
+__device__ __forceinline__ float softmap_largest(const unsigned *largest) {
+    const unsigned big = *largest;
+    return __uint_as_float(max(big, __float_as_uint(SM_LARGE)));
 }
 
 // ---------------------------------------------------------------------------------
@@ -89,7 +93,7 @@ __device__ __forceinline__ constexpr float softmap_cut(int p) {
 template <int NP, int T, int NQ>
 __global__ __launch_bounds__(T) void softmap_rowstats(const float *__restrict__ W, float scale, float *__restrict__ mxs,
                                                       float *__restrict__ rss, char *__restrict__ E, size_t plane, int M,
-                                                      int I, int Ip) {
+                                                      int I, int Ip, unsigned *__restrict__ largest) {
     constexpr int WV = T / 64;
     __shared__ float red[2][8][WV];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -132,6 +136,10 @@ __global__ __launch_bounds__(T) void softmap_rowstats(const float *__restrict__ 
     };
     auto store = [&](int i, float *e) {
         if (i < Ip) {
+            if (NP > 1) {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) e[j] *= SM_SCALE;
+            }
 #pragma unroll
             for (int p = 0; p < NP; ++p)
                 *reinterpret_cast<uint4 *>(reinterpret_cast<char *>(out + i) + p * plane) = softmap_unit(e);
@@ -168,20 +176,24 @@ __global__ __launch_bounds__(T) void softmap_rowstats(const float *__restrict__ 
         for (int q = 1; q < WV; ++q) mj = fmaxf(mj, red[0][tid][q]);
         mxs[o0 + tid] = o0 + tid < M ? mj : 0.0f;
         rss[o0 + tid] = o0 + tid < M ? 1.0f / t : 0.0f;
+        if (largest && blockIdx.x == 0 && tid == 0) *largest = 0;  // of x, which is packed after this
     }
 }
 
 // ---------------------------------------------------------------------------------
 // src [R][C] fp32 -> units along the rows [Rp/8][Cp] and / or along the columns [Cp/8][Rp], NP planes each, the latter scaled
-// per column where `colscale` is given, padding zero.  With `other`: dots[chunk][c] = sum of src * other over the 64 rows of
-// the chunk (unscaled; the reader adds the chunks in order).  Block = 64 columns x 64 rows: a thread has sixteen rows of a
-// column, so units along the rows leave straight from registers; those along the columns go through the LDS (row
-// stride 65 words, no conflicts).
+// per column where `colscale` is given, padding zero; three planes are those of 2^24 times the value.  With `other`:
+// dots[chunk][c] = sum of src * other over the 64 rows of the chunk (unscaled; the reader adds the chunks in order).
+// Block = 64 columns x 64 rows: a thread has sixteen rows of a column, so units along the rows leave straight from registers;
+// those along the columns go through the LDS (row stride 65 words, no conflicts).  `largest` (three planes; nullable): see
+// softmap_note_large; `clear` (nullable): such a word that a later launch fills.
 template <int NP>
 __global__ __launch_bounds__(256) void softmap_pack(const float *__restrict__ src, const float *__restrict__ colscale,
                                                     const float *__restrict__ other, float *__restrict__ dots,
                                                     char *__restrict__ rows8, size_t rows_plane, char *__restrict__ cols8,
-                                                    size_t cols_plane, int R, int C, int Rp, int Cp) {
+                                                    size_t cols_plane, int R, int C, int Rp, int Cp, unsigned *__restrict__ largest,
+                                                    unsigned *__restrict__ clear) {
+    if (clear && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *clear = 0;
     __shared__ float tile[64][65];
     __shared__ float part[4][64];
     const int c = threadIdx.x & 63, g = threadIdx.x >> 6;
@@ -201,6 +213,15 @@ __global__ __launch_bounds__(256) void softmap_pack(const float *__restrict__ sr
         }
         part[g][c] = dot;
     }
+    if (NP > 1) {
+        unsigned big = 0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            big = max(big, __float_as_uint(v[i]) & 0x7fffffffu);
+            v[i] *= SM_SCALE;
+        }
+        if (largest) softmap_note_large(largest, big);
+    }
 #pragma unroll
     for (int i = 0; i < 16; ++i) tile[g * 16 + i][c] = v[i] * f;
     __syncthreads();
@@ -212,7 +233,7 @@ __global__ __launch_bounds__(256) void softmap_pack(const float *__restrict__ sr
             if (8 * rb < Rp) {
                 char *d = rows8 + ((size_t)rb * Cp + col) * SM_UNIT;
 #pragma unroll
-                for (int p = 0; p < NP; ++p) *reinterpret_cast<uint4 *>(d + p * rows_plane) = softmap_unit(v + 8 * h, softmap_cut<NP>(p));
+                for (int p = 0; p < NP; ++p) *reinterpret_cast<uint4 *>(d + p * rows_plane) = softmap_unit(v + 8 * h);
             }
         }
     }
@@ -226,7 +247,7 @@ __global__ __launch_bounds__(256) void softmap_pack(const float *__restrict__ sr
                 for (int j = 0; j < 8; ++j) w[j] = tile[c][cb * 8 + j];
                 char *d = cols8 + ((size_t)(blockIdx.x * 8 + cb) * Rp + row) * SM_UNIT;
 #pragma unroll
-                for (int p = 0; p < NP; ++p) *reinterpret_cast<uint4 *>(d + p * cols_plane) = softmap_unit(w, softmap_cut<NP>(p));
+                for (int p = 0; p < NP; ++p) *reinterpret_cast<uint4 *>(d + p * cols_plane) = softmap_unit(w);
             }
         }
     }
@@ -430,7 +451,7 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const int col = c0 + wn + j * 32 + l32;
-            const float f = MODE == 0 ? g.rs[col] : 1.0f;
+            const float f = (NP == 3 ? SM_UNSCALE : 1.0f) * (MODE == 0 ? g.rs[col] : 1.0f);
 #pragma unroll
             for (int i = 0; i < FA; ++i)
 #pragma unroll
@@ -474,8 +495,9 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const float4 rv = *reinterpret_cast<const float4 *>(rr + lr0 + 8 * q + 4 * kh);
-                    float o[4] = {acc[i][j][4 * q] - rv.x, acc[i][j][4 * q + 1] - rv.y, acc[i][j][4 * q + 2] - rv.z,
-                                  acc[i][j][4 * q + 3] - rv.w};
+                    constexpr float f = NP == 3 ? SM_UNSCALE : 1.0f;
+                    float o[4] = {acc[i][j][4 * q] * f - rv.x, acc[i][j][4 * q + 1] * f - rv.y,
+                                  acc[i][j][4 * q + 2] * f - rv.z, acc[i][j][4 * q + 3] * f - rv.w};
                     if (NP == 1) {
                         const float4 fv = *reinterpret_cast<const float4 *>(rr + 2 * TR + lr0 + 8 * q + 4 * kh);
                         o[0] *= softmap_lo(e[j][q].x) * fv.x; o[1] *= softmap_hi(e[j][q].x) * fv.y;
@@ -524,6 +546,155 @@ static void softmap_launch(const SoftmapArgs &g, hipStream_t s) {
                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
     softmap_mfma<MODE, NP, FA><<<dl_xcd_grid(g.inner_count, g.outer_count), 256, lds_bytes, s>>>(g);
 }
+
+// ---------------------------------------------------------------------------------
+// The products of precision 0 on the fp32 matrix cores (v_mfma_f32_32x32x2_f32), for operands that the planes do not carry.
+// Launched behind every product; where the largest magnitudes allow the planes, which is all but always, a block reads them
+// and ends (6 us of launch).  Else: 128 x 128 outputs per block and step, 2 x 2 wavefronts of 2 x 2 MFMA tiles, 16 reduction
+// steps through the LDS with the next 16 on their way; every 128 steps the sums go into a second set of registers, so that
+// long reductions round less.  512 x 3136 x 48000 with one infinite input: forward 2.34 ms, gW 2.37 (1.26 and 1.31 when the fp32
+// matrix cores carried every call; such a call is an exception now).
+struct SoftmapPlain {
+    const float *x, *W, *gm, *mx, *rs, *dots;
+    float *m, *gx, *gW;
+    const unsigned *x_largest, *gm_largest;
+    int B, I, M, parts, dot_ld;
+    float scale, inv_tau;
+};
+#define SM_PT 128  // edge of a tile
+#define SM_PLD 132 // its row in the LDS
+template <int MODE>
+__device__ void softmap_plain_tile(const SoftmapPlain &p, float (&As)[16][SM_PLD], float (&Bs)[16][SM_PLD], int r0, int c0) {
+    const int R = MODE == 2 ? p.M : p.B, C = MODE == 0 ? p.M : p.I, K = MODE == 0 ? p.I : MODE == 1 ? p.M : p.B;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, kh = lane >> 5, l32 = lane & 31;
+    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+    auto softmax = [&](int o, int i) -> float {
+        return softmap_e(p.W[(size_t)o * p.I + i], p.mx[o], p.scale) * p.rs[o];
+    };
+    // (rows and columns past the end repeat the last and are not stored)
+    auto a_at = [&](int row, int k) -> float {
+        row = min(row, R - 1);
+        // the forward's halved: a sum of weights that round to more than one must not overflow on the way
+        return MODE == 0 ? 0.5f * p.x[(size_t)row * p.I + k] : MODE == 1 ? p.gm[(size_t)row * p.M + k] : p.gm[(size_t)k * p.M + row];
+    };
+    auto b_at = [&](int col, int k) -> float {
+        col = min(col, C - 1);
+        return MODE == 0 ? softmax(col, k) : MODE == 1 ? softmax(k, col) : p.x[(size_t)k * p.I + col];
+    };
+    // neighbouring threads along what is contiguous in memory: the reduction, or rows / columns
+    constexpr bool A_ALONG_K = MODE != 2, B_ALONG_K = MODE == 0;
+    float na[8], nb[8];
+    auto fetch_as = [&](int k0, auto whole) {
+        int t = tid;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            // addresses are made anew, and for two elements at a time: all of them do not fit the registers
+            if (q % 2 == 0) asm volatile("" : "+v"(t)::"memory");
+            const int e = q * 256 + t;
+            const int ka = k0 + (A_ALONG_K ? e & 15 : e >> 7), kb = k0 + (B_ALONG_K ? e & 15 : e >> 7);
+            const int ra = r0 + (A_ALONG_K ? e >> 4 : e & 127), cb = c0 + (B_ALONG_K ? e >> 4 : e & 127);
+            na[q] = decltype(whole)::value || ka < K ? a_at(ra, ka) : 0.0f;
+            nb[q] = decltype(whole)::value || kb < K ? b_at(cb, kb) : 0.0f;
+        }
+    };
+    auto fetch = [&](int k0) {
+        if (k0 + 16 <= K) fetch_as(k0, std::true_type{});
+        else fetch_as(k0, std::false_type{});
+    };
+    floatx16 acc[2][2], sum[2][2];
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[t >> 1][t & 1][v] = sum[t >> 1][t & 1][v] = 0.0f;
+    fetch(0);
+    for (int k0 = 0; k0 < K; k0 += 16) {
+        __syncthreads();
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int e = q * 256 + tid;
+            if (A_ALONG_K) As[e & 15][e >> 4] = na[q];
+            else As[e >> 7][e & 127] = na[q];
+            if (B_ALONG_K) Bs[e & 15][e >> 4] = nb[q];
+            else Bs[e >> 7][e & 127] = nb[q];
+        }
+        __syncthreads();
+        if (k0 + 16 < K) fetch(k0 + 16);
+#pragma unroll
+        for (int kk = 0; kk < 8; ++kk) {
+            const int k = 2 * kk + kh;
+            const float a0 = As[k][wm + l32], a1 = As[k][wm + 32 + l32], b0 = Bs[k][wn + l32], b1 = Bs[k][wn + 32 + l32];
+            acc[0][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b0, acc[0][0], 0, 0, 0);
+            acc[0][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b1, acc[0][1], 0, 0, 0);
+            acc[1][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b0, acc[1][0], 0, 0, 0);
+            acc[1][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b1, acc[1][1], 0, 0, 0);
+        }
+        if ((k0 & 127) == 112 || k0 + 16 >= K) {
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    sum[t >> 1][t & 1][v] += acc[t >> 1][t & 1][v];
+                    acc[t >> 1][t & 1][v] = 0.0f;
+                }
+        }
+    }
+    if (MODE == 2) {  // of the tile's rows: r, the maximum and rs / tau
+        __syncthreads();
+        if (tid < SM_PT) {
+            const int row = min(r0 + tid, R - 1);
+            float r = 0.0f;
+            for (int q = 0; q < p.parts; ++q) r += p.dots[(size_t)q * p.dot_ld + row];
+            As[0][tid] = r;
+            As[1][tid] = p.mx[row];
+            As[2][tid] = p.rs[row] * p.inv_tau;
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const int lr = wm + i * 32 + 8 * (v >> 2) + 4 * kh + (v & 3), row = r0 + lr;
+            if (row >= R) continue;
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int col = c0 + wn + j * 32 + l32;
+                if (col >= C) continue;
+                float o = sum[i][j][v];
+                if (MODE == 0) {  // a mean of finite values is no larger than they are
+                    const bool finite = __builtin_isfinite(o);
+                    o *= 2.0f;
+                    if (finite) o = fminf(fmaxf(o, -3.402823466e38f), 3.402823466e38f);
+                    p.m[(size_t)row * C + col] = o;
+                } else if (MODE == 1) {
+                    p.gx[(size_t)row * C + col] = o;
+                } else {
+                    const size_t at = (size_t)row * C + col;
+                    p.gW[at] = (o - As[0][lr]) * (softmap_e(p.W[at], As[1][lr], p.scale) * As[2][lr]);
+                }
+            }
+        }
+}
+template <bool BWD>
+__global__ __launch_bounds__(256, 2) void softmap_plain(SoftmapPlain p) {
+    __shared__ float As[16][SM_PLD], Bs[16][SM_PLD];
+    const float x = softmap_largest(p.x_largest), gm = BWD ? softmap_largest(p.gm_largest) : 0.0f;
+    const int bt = (p.B + SM_PT - 1) / SM_PT, it = (p.I + SM_PT - 1) / SM_PT, mt = (p.M + SM_PT - 1) / SM_PT;
+    // the largest sums the planes' accumulators could see, without the factor (a NaN compares false)
+    if (!BWD) {
+        if (x * (float)p.I < SM_BOUND) return;
+        for (long long t = blockIdx.x; t < (long long)bt * mt; t += gridDim.x)
+            softmap_plain_tile<0>(p, As, Bs, (int)(t % bt) * SM_PT, (int)(t / bt) * SM_PT);
+        return;
+    }
+    if (!(gm * (float)p.M < SM_BOUND))
+        for (long long t = blockIdx.x; t < (long long)bt * it; t += gridDim.x)
+            softmap_plain_tile<1>(p, As, Bs, (int)(t / it) * SM_PT, (int)(t % it) * SM_PT);
+    if (!(gm * (float)p.B * x < SM_BOUND))
+        for (long long t = blockIdx.x; t < (long long)mt * it; t += gridDim.x)
+            softmap_plain_tile<2>(p, As, Bs, (int)(t / it) * SM_PT, (int)(t % it) * SM_PT);
+}
+#define SM_PLAIN_BLOCKS 512  // two per CU
 
 // ---------------------------------------------------------------------------------
 static int softmap_check(int B, int I, int M, int precision) {
@@ -578,15 +749,17 @@ static SoftmapShape softmap_shape(int B, int I, int M, int precision) {
     return h;
 }
 
-// `stats`, kept for the backward: max [Mp], 1/sum [Mp], x in units along the inputs (the forward's operand) and E
+// `stats`, kept for the backward: max [Mp], 1/sum [Mp], x in units along the inputs (the forward's operand), E, and with
+// fp32 operands the largest magnitude of x
 static inline size_t softmap_vec_bytes(const SoftmapShape &h) { return dl_align256((size_t)h.Mp * sizeof(float)); }
 extern "C" size_t dl_soft_map_saved_bytes(int B, int I, int M, int precision) {
     if (B <= 0 || I <= 0 || M <= 0) return 256;
     const SoftmapShape h = softmap_shape(B, I, M, precision);
-    return 2 * softmap_vec_bytes(h) + h.np * (h.x_plane + h.e_plane);
+    return 2 * softmap_vec_bytes(h) + h.np * (h.x_plane + h.e_plane) + (h.np > 1 ? 256 : 0);
 }
 
-// workspace: partial products of the forward or of gx, partial r, x and gm in units along the batch, gs along the rows of W
+// workspace: partial products of the forward or of gx, partial r, x and gm in units along the batch, gs along the rows of W, the
+// largest magnitude of gm
 static inline size_t softmap_part_bytes(const SoftmapShape &h) {
     const size_t fwd = h.fwd_chunks > 1 ? (size_t)h.fwd_chunks * h.B * h.M : 0, gx = h.gx_chunks > 1 ? (size_t)h.gx_chunks * h.B * h.I : 0;
     return dl_align256((fwd > gx ? fwd : gx) * sizeof(float));
@@ -601,10 +774,11 @@ extern "C" size_t dl_soft_map_workspace_bytes(int B, int I, int M, int precision
 }
 
 template <int NP>
-static void softmap_stats_launch(const SoftmapShape &h, const float *W, float scale, float *mx, float *rs, char *E, hipStream_t s) {
+static void softmap_stats_launch(const SoftmapShape &h, const float *W, float scale, float *mx, float *rs, char *E,
+                                 unsigned *largest, hipStream_t s) {
     const int grid = h.Mp / 8;
 #define SM_STATS(T, NQ) \
-    DL_TIMED("softmap_rowstats", s, (softmap_rowstats<NP, T, NQ><<<grid, T, 0, s>>>(W, scale, mx, rs, E, h.e_plane, h.M, h.I, h.Ip)))
+    DL_TIMED("softmap_rowstats", s, (softmap_rowstats<NP, T, NQ><<<grid, T, 0, s>>>(W, scale, mx, rs, E, h.e_plane, h.M, h.I, h.Ip, largest)))
     if (h.Ip <= 256 * 4) SM_STATS(256, 4);
     else if (h.Ip <= 256 * 8) SM_STATS(256, 8);
     else if (h.Ip <= 512 * 8) SM_STATS(512, 8);
@@ -613,12 +787,13 @@ static void softmap_stats_launch(const SoftmapShape &h, const float *W, float sc
 #undef SM_STATS
 }
 static void softmap_pack_launch(int np, const float *src, const float *colscale, const float *other, float *dots, char *rows8,
-                                size_t rows_plane, char *cols8, size_t cols_plane, int R, int C, int Rp, int Cp, hipStream_t s) {
+                                size_t rows_plane, char *cols8, size_t cols_plane, int R, int C, int Rp, int Cp, unsigned *largest,
+                                unsigned *clear, hipStream_t s) {
     const dim3 grid(Cp / 64, dl_ceil_div(Rp, 64));
     if (np == 1)
-        DL_TIMED("softmap_pack", s, (softmap_pack<1><<<grid, 256, 0, s>>>(src, colscale, other, dots, rows8, rows_plane, cols8, cols_plane, R, C, Rp, Cp)));
+        DL_TIMED("softmap_pack", s, (softmap_pack<1><<<grid, 256, 0, s>>>(src, colscale, other, dots, rows8, rows_plane, cols8, cols_plane, R, C, Rp, Cp, largest, clear)));
     else
-        DL_TIMED("softmap_pack", s, (softmap_pack<3><<<grid, 256, 0, s>>>(src, colscale, other, dots, rows8, rows_plane, cols8, cols_plane, R, C, Rp, Cp)));
+        DL_TIMED("softmap_pack", s, (softmap_pack<3><<<grid, 256, 0, s>>>(src, colscale, other, dots, rows8, rows_plane, cols8, cols_plane, R, C, Rp, Cp, largest, clear)));
 }
 static void softmap_reduce(const float *part, float *out, long long total, int chunks, hipStream_t s) {
     if (total % 4 == 0 && ((uintptr_t)out & 15) == 0)
@@ -639,6 +814,8 @@ static void softmap_product(const char *name, const SoftmapShape &h, int fa, con
     }
 }
 
+static inline int softmap_plain_grid(long long tiles) { return tiles < SM_PLAIN_BLOCKS ? (int)tiles : SM_PLAIN_BLOCKS; }
+
 extern "C" int dl_soft_map_fwd(const float *x, const float *W, float tau, float *m, float *stats, void *ws,
                                size_t ws_bytes, int B, int I, int M, int precision, void *stream) {
     if (!x || !W || !m || !stats) return DL_ERR_NULL;
@@ -653,9 +830,10 @@ extern "C" int dl_soft_map_fwd(const float *x, const float *W, float tau, float 
     char *p = (char *)stats;
     float *mx = (float *)p, *rs = (float *)(p + softmap_vec_bytes(h));
     char *x8 = p + 2 * softmap_vec_bytes(h), *E = x8 + h.np * h.x_plane;
-    if (h.np == 1) softmap_stats_launch<1>(h, W, SM_LOG2E / tau, mx, rs, E, s);
-    else softmap_stats_launch<3>(h, W, SM_LOG2E / tau, mx, rs, E, s);
-    softmap_pack_launch(h.np, x, nullptr, nullptr, nullptr, nullptr, 0, x8, h.x_plane, B, I, h.Bp, h.Ip, s);
+    unsigned *x_largest = h.np > 1 ? (unsigned *)(E + h.np * h.e_plane) : nullptr;
+    if (h.np == 1) softmap_stats_launch<1>(h, W, SM_LOG2E / tau, mx, rs, E, x_largest, s);
+    else softmap_stats_launch<3>(h, W, SM_LOG2E / tau, mx, rs, E, x_largest, s);
+    softmap_pack_launch(h.np, x, nullptr, nullptr, nullptr, nullptr, 0, x8, h.x_plane, B, I, h.Bp, h.Ip, x_largest, nullptr, s);
     SoftmapArgs g{};
     g.A = x8; g.a_plane = h.x_plane; g.lda = h.Bp;
     g.Bm = E; g.b_plane = h.e_plane; g.ldb = h.Ip;
@@ -666,6 +844,13 @@ extern "C" int dl_soft_map_fwd(const float *x, const float *W, float tau, float 
     g.rs = rs;
     softmap_product<0>("softmap_fwd", h, h.fa, g, s);
     if (h.fwd_chunks > 1) softmap_reduce((const float *)ws, m, (long long)B * M, h.fwd_chunks, s);
+    if (h.np > 1) {
+        SoftmapPlain q{};
+        q.x = x; q.W = W; q.mx = mx; q.rs = rs; q.m = m; q.x_largest = x_largest;
+        q.B = B; q.I = I; q.M = M; q.scale = SM_LOG2E / tau;
+        const int grid = softmap_plain_grid((long long)dl_ceil_div(B, SM_PT) * dl_ceil_div(M, SM_PT));
+        DL_TIMED("softmap_plain", s, (softmap_plain<false><<<grid, 256, 0, s>>>(q)));
+    }
     return dl_launch_status();
 }
 
@@ -682,14 +867,16 @@ extern "C" int dl_soft_map_bwd(const float *x, const float *W, float tau, const 
     const char *p = (const char *)stats;
     const float *mx = (const float *)p, *rs = (const float *)(p + softmap_vec_bytes(h));
     const char *E = p + 2 * softmap_vec_bytes(h) + h.np * h.x_plane;
+    const unsigned *x_largest = h.np > 1 ? (const unsigned *)(E + h.np * h.e_plane) : nullptr;
     char *w = (char *)ws;
     float *part = (float *)w; w += softmap_part_bytes(h);
     float *dots = (float *)w; w += softmap_dots_bytes(h);
     char *xb = w; w += h.np * h.x_plane;     // x  [Bp/8][Ip]
     char *gb = w; w += h.np * h.g_plane;     // gm [Bp/8][Mp]
-    char *go = w;                            // gs [Mp/8][Bp]
-    softmap_pack_launch(h.np, x, nullptr, nullptr, nullptr, xb, h.x_plane, nullptr, 0, B, I, h.Bp, h.Ip, s);
-    softmap_pack_launch(h.np, gm, rs, m, dots, gb, h.g_plane, go, h.g_plane, B, M, h.Bp, h.Mp, s);
+    char *go = w; w += h.np * h.g_plane;     // gs [Mp/8][Bp]
+    unsigned *gm_largest = h.np > 1 ? (unsigned *)w : nullptr;
+    softmap_pack_launch(h.np, x, nullptr, nullptr, nullptr, xb, h.x_plane, nullptr, 0, B, I, h.Bp, h.Ip, nullptr, gm_largest, s);
+    softmap_pack_launch(h.np, gm, rs, m, dots, gb, h.g_plane, go, h.g_plane, B, M, h.Bp, h.Mp, gm_largest, nullptr, s);
     SoftmapArgs g{};
     g.A = go; g.a_plane = h.g_plane; g.lda = h.Bp;
     g.Bm = E; g.b_plane = h.e_plane; g.ldb = h.Ip;
@@ -712,5 +899,13 @@ extern "C" int dl_soft_map_bwd(const float *x, const float *W, float tau, const 
     q.mx = mx; q.W = W; q.E = E; q.lde = h.Ip; q.scale = SM_LOG2E / tau; q.inv_tau = 1.0f / tau;
     q.vec_out = (((uintptr_t)W | (uintptr_t)gW) & 15) == 0;
     softmap_product<2>("softmap_gw", h, fa, q, s);
+    if (h.np > 1) {
+        SoftmapPlain u{};
+        u.x = x; u.W = W; u.gm = gm; u.mx = mx; u.rs = rs; u.dots = dots; u.gx = gx; u.gW = gW;
+        u.x_largest = x_largest; u.gm_largest = gm_largest;
+        u.B = B; u.I = I; u.M = M; u.parts = q.parts; u.dot_ld = q.dot_ld; u.scale = q.scale; u.inv_tau = q.inv_tau;
+        const int grid = softmap_plain_grid((long long)(M > B ? dl_ceil_div(M, SM_PT) : dl_ceil_div(B, SM_PT)) * dl_ceil_div(I, SM_PT));
+        DL_TIMED("softmap_plain", s, (softmap_plain<true><<<grid, 256, 0, s>>>(u)));
+    }
     return dl_launch_status();
 }

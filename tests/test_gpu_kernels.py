@@ -737,6 +737,64 @@ def test_soft_mapping_of_values_beyond_bf16(value):
     assert float(((m.double() - want).abs() / want.abs()).max()) <= 1e-5
 
 
+LOWEST = float(np.finfo(np.float32).min)
+
+
+@pytest.mark.parametrize("case", ["two_lowest", "all_lowest", "largest", "infinite", "nan", "huge", "tiny", "denormal"])
+@pytest.mark.parametrize("side", ["x", "gm"])
+@pytest.mark.parametrize("shape", [(70, 200, 130), (130, 300, 17), (200, 3000, 2000)])
+def test_soft_mapping_fp32_range(shape, side, case):
+    """fp32 operands of any magnitude give what fp32 sums give: against float64, infinities and NaN in the same places, finite
+    results within 1e-5 in the 2-norm (as test_soft_mapping_tile_edges derives it).
+    Magnitudes are mixed with ordinary values in two rows, or are those of the whole operand (huge, tiny, denormal)."""
+    ops = _ops()
+    B, I, M = shape
+    g = torch.Generator("cuda").manual_seed(B + len(case))
+    x = torch.rand(B, I, device="cuda", generator=g) + 0.1
+    W = torch.randn(M, I, device="cuda", generator=g) * 0.5
+    W[:3] = 0.0  # equal weights
+    gm = torch.rand(B, M, device="cuda", generator=g) + 0.1
+    v, other = (x, gm) if side == "x" else (gm, x)
+    if case in ("two_lowest", "all_lowest", "largest"):
+        other *= 1e-3  # products of the two stay within float32
+    if case == "two_lowest":
+        v[3, 5] = v[3, 11] = v[40, 2] = v[40, 9] = LOWEST
+    elif case == "all_lowest":
+        v[3], v[40] = LOWEST, LOWEST
+    elif case == "largest":
+        v[3, 5], v[40, 2] = -LOWEST, LOWEST
+    elif case == "infinite":
+        v[3, 5], v[40, 2], v[41, 1] = float("inf"), float("-inf"), float("inf")
+    elif case == "nan":
+        v[3, 5] = float("nan")
+    else:
+        v *= {"huge": 1e30, "tiny": 1e-33, "denormal": 1e-38}[case]
+    xt, Wt = x.clone().requires_grad_(), W.clone().requires_grad_()
+    m = ops.SoftMapFunction.apply(xt, Wt, 1.0, 0)
+    m.backward(gm)
+    xd, Wd = x.double().requires_grad_(), W.double().requires_grad_()
+    S = torch.softmax(Wd, dim=-1)
+    md = xd @ S.t()
+    md.backward(gm.double())
+    Sd, G, r = S.detach(), gm.double().t() @ x.double(), (gm.double() * md.detach()).sum(0)
+    # gW = S (G - r) is a difference: its error is that of its terms, and where G and r are infinite alike it is NaN
+    terms = Sd * (G.abs() + r.abs()[:, None])
+    for got, want, size in ((m.detach(), md.detach(), x.double().abs() @ Sd.t()), (xt.grad, xd.grad, gm.double().abs() @ Sd),
+                            (Wt.grad, Wd.grad, terms)):
+        got = got.double()
+        assert torch.equal(torch.isnan(got), torch.isnan(want))
+        assert torch.equal(torch.isinf(got), torch.isinf(want)) and torch.equal(got[torch.isinf(want)], want[torch.isinf(want)])
+        finite = torch.isfinite(want)
+        scale = float(size[finite].norm()) if finite.any() else 0.0
+        err = float((got[finite] - want[finite]).norm())
+        assert err <= 1e-5 * scale + 1e-43 * finite.sum().sqrt(), (err, scale)
+    # the forward is a mean: no larger than the values it is of, whatever the rounding of the weights
+    if side == "x" and case in ("two_lowest", "all_lowest", "largest"):
+        assert torch.isfinite(m).all()
+        rel = (m.detach().double() - md.detach()).abs() / md.detach().abs()
+        assert float(rel.max()) <= 1e-5
+
+
 def test_soft_and_hard_mapping_against_reference_vectors(golden):
     ops = _ops()
     g = golden
