@@ -39,6 +39,7 @@ typedef short shortx8 __attribute__((ext_vector_type(8)));
 
 #define SM_LOG2E 1.4426950408889634f
 #define SM_TC 128  // columns of an output tile
+#define SM_GX_STAGE 16 // reduction steps of a stage with three planes
 #define SM_UNIT 16 // bytes of a unit
 
 // exp((w - mx)/tau), with scale = log2(e)/tau: one subtract, one multiply, the hardware exp2.
@@ -186,12 +187,13 @@ __global__ __launch_bounds__(T) void softmap_rowstats(const float *__restrict__ 
 // dots[chunk][c] = sum of src * other over the 64 rows of the chunk (unscaled; the reader adds the chunks in order).
 // Block = 64 columns x 64 rows: a thread has sixteen rows of a column, so units along the rows leave straight from registers;
 // those along the columns go through the LDS (row stride 65 words, no conflicts).  `largest` (three planes; nullable): see
-// softmap_note_large; `clear` (nullable): such a word that a later launch fills.
+// softmap_note_large; `clear` (nullable): such a word that a later launch fills.  `alternate` (three planes): factor of every
+// second group of SM_GX_STAGE columns in the units along the columns.
 template <int NP>
 __global__ __launch_bounds__(256) void softmap_pack(const float *__restrict__ src, const float *__restrict__ colscale,
                                                     const float *__restrict__ other, float *__restrict__ dots,
                                                     char *__restrict__ rows8, size_t rows_plane, char *__restrict__ cols8,
-                                                    size_t cols_plane, int R, int C, int Rp, int Cp, unsigned *__restrict__ largest,
+                                                    size_t cols_plane, int R, int C, int Rp, int Cp, float alternate, unsigned *__restrict__ largest,
                                                     unsigned *__restrict__ clear) {
     if (clear && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *clear = 0;
     __shared__ float tile[64][65];
@@ -199,7 +201,8 @@ __global__ __launch_bounds__(256) void softmap_pack(const float *__restrict__ sr
     const int c = threadIdx.x & 63, g = threadIdx.x >> 6;
     const int col = blockIdx.x * 64 + c, r0 = blockIdx.y * 64;
     float v[16], dot = 0.0f;
-    const float f = colscale && col < C ? colscale[col] : 1.0f;
+    float f = colscale && col < C ? colscale[col] : 1.0f;
+    if (NP > 1 && (col / SM_GX_STAGE) % 2 != 0) f *= alternate;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
         const int r = r0 + g * 16 + i;
@@ -253,34 +256,30 @@ __global__ __launch_bounds__(256) void softmap_pack(const float *__restrict__ sr
     }
 }
 
-// out[e] = sum over chunks of part[chunk][e], fixed order; VEC = 4 when total is a multiple of 4
+// out[e] = sum over chunks of part[chunk][e], fixed order; VEC = 4 when total is a multiple of 4.  Summed in double, so that the
+// result is rounded once however many chunks there are (bound by the reads: no slower).
 template <int VEC>
 __global__ __launch_bounds__(256) void softmap_reduce_chunks(const float *__restrict__ part, float *__restrict__ out,
                                                               long long total, int chunks) {
     const long long e = ((long long)blockIdx.x * 256 + threadIdx.x) * VEC;
     if (e >= total) return;
     if (VEC == 4) {
-        float4 acc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        double acc[4] = {0.0, 0.0, 0.0, 0.0};
+        auto add = [&](const float4 &p) { acc[0] += p.x; acc[1] += p.y; acc[2] += p.z; acc[3] += p.w; };
         int c = 0;
         for (; c + 4 <= chunks; c += 4) {  // four independent loads in flight, added in chunk order
             const float4 p0 = *reinterpret_cast<const float4 *>(part + (size_t)c * total + e);
             const float4 p1 = *reinterpret_cast<const float4 *>(part + (size_t)(c + 1) * total + e);
             const float4 p2 = *reinterpret_cast<const float4 *>(part + (size_t)(c + 2) * total + e);
             const float4 p3 = *reinterpret_cast<const float4 *>(part + (size_t)(c + 3) * total + e);
-            acc.x += p0.x; acc.y += p0.y; acc.z += p0.z; acc.w += p0.w;
-            acc.x += p1.x; acc.y += p1.y; acc.z += p1.z; acc.w += p1.w;
-            acc.x += p2.x; acc.y += p2.y; acc.z += p2.z; acc.w += p2.w;
-            acc.x += p3.x; acc.y += p3.y; acc.z += p3.z; acc.w += p3.w;
+            add(p0); add(p1); add(p2); add(p3);
         }
-        for (; c < chunks; ++c) {
-            const float4 p = *reinterpret_cast<const float4 *>(part + (size_t)c * total + e);
-            acc.x += p.x; acc.y += p.y; acc.z += p.z; acc.w += p.w;
-        }
-        *reinterpret_cast<float4 *>(out + e) = acc;
+        for (; c < chunks; ++c) add(*reinterpret_cast<const float4 *>(part + (size_t)c * total + e));
+        *reinterpret_cast<float4 *>(out + e) = make_float4((float)acc[0], (float)acc[1], (float)acc[2], (float)acc[3]);
     } else {
-        float acc = 0.0f;
+        double acc = 0.0;
         for (int c = 0; c < chunks; ++c) acc += part[(size_t)c * total + e];
-        out[e] = acc;
+        out[e] = (float)acc;
     }
 }
 
@@ -315,9 +314,15 @@ __device__ __forceinline__ void softmap_stage_barrier() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
+// gx with three planes sums the six products of a stage by themselves and adds them to the running sum in one rounding, because
+// its reduction is the long one; and as the matrix cores round sums of bf16 products towards minus infinity, which would add up
+// over thousands of stages, every second stage comes with the sign of gs turned (SM_GX_STAGE) and is subtracted.  Against
+// float64 (2-norm), 512 x 3136 x 48000: 1.15e-6 with one running sum for everything, 0.50e-6 by stages, 0.32e-6 with turned
+// signs as well; on the fp32 matrix cores 0.62e-6.  It costs 675 -> 725 us there.
+//
 // One product kernel, three operand modes.  At 512 x 3136 x 48000 (1.54e11 flop a product; before: 128 x 128 tiles staged
-// through registers) forward / gx / gW take 182 / 160 / 298 us with bf16 operands (before 236 / 453 / 365) and 673 / 668 /
-// 812 us with three planes (before, on the fp32 matrix cores, 1318 / 1494 / 1347): 0.85-0.96 and 1.37 PFLOP/s of bf16
+// through registers) forward / gx / gW take 182 / 160 / 298 us with bf16 operands (before 236 / 453 / 365) and 660 / 725 /
+// 840 us with three planes (before, on the fp32 matrix cores, 1318 / 1494 / 1347): 0.85-0.96 and 1.27-1.40 PFLOP/s of bf16
 // products, the latter what the matrix cores hold under power; gW adds 602 MB of stores and 301 (602) MB of reads.
 // MODE 0: forward   rows=b cols=o red=i   A = x    B = E (turned)   out = C rs[o]
 // MODE 1: gx        rows=b cols=i red=o   A = gs   B = E
@@ -329,9 +334,10 @@ __device__ __forceinline__ void softmap_stage_barrier() {
 template <int MODE, int NP, int FA>
 __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
     constexpr int TR = 64 * FA, TC = SM_TC;
-    constexpr int KC = NP == 1 ? 32 : 16, KB = KC / 8;
+    constexpr int KC = NP == 1 ? 32 : SM_GX_STAGE, KB = KC / 8;
     constexpr int NBUF = NP == 3 && FA == 4 ? 2 : 3, AHEAD = NBUF - 1;
     constexpr int A_BYTES = NP * TR * KC * 2, STAGE = NP * (TR + TC) * KC * 2;
+    constexpr bool BY_STAGE = NP == 3 && MODE == 1;
     constexpr int NA = NP * KB * (TR / 64) / 4, NB = NP * KB * (TC / 64) / 4;  // loads per wavefront and stage
     static_assert(NP * KB * (TR / 64) % 4 == 0 && NP * KB * (TC / 64) % 4 == 0, "whole loads per wavefront");
     extern __shared__ __align__(16) char lds[];
@@ -395,7 +401,7 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
     } else {
         b_rd = A_BYTES + (kh * TC + wn + l32) * SM_UNIT;
     }
-    auto compute = [&](int buf) __attribute__((always_inline)) {
+    auto compute = [&](int buf, float sign) __attribute__((always_inline)) {
         const unsigned base = buf * STAGE;
 #pragma unroll
         for (int kk = 0; kk < KC / 16; ++kk) {
@@ -420,13 +426,33 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
             }
             // small products first
             constexpr int PA[6] = {0, 2, 1, 0, 1, 0}, PB[6] = {2, 0, 1, 1, 0, 0};
+            if (BY_STAGE) {
 #pragma unroll
-            for (int t = NP == 3 ? 0 : 5; t < 6; ++t)
-#pragma unroll
-                for (int i = 0; i < FA; ++i)
+                for (int i = 0; i < FA; ++i) {
+                    floatx16 step[2];
 #pragma unroll
                     for (int j = 0; j < 2; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[PA[t]][i], b[PB[t]][j], acc[i][j], 0, 0, 0);
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) step[j][v] = 0.0f;
+#pragma unroll
+                    for (int t = 0; t < 6; ++t)
+#pragma unroll
+                        for (int j = 0; j < 2; ++j)
+                            step[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[PA[t] % NP][i], b[PB[t] % NP][j], step[j], 0, 0, 0);
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) acc[i][j][v] = fmaf(sign, step[j][v], acc[i][j][v]);
+                }
+            } else {
+#pragma unroll
+                for (int t = NP == 3 ? 0 : 5; t < 6; ++t)
+#pragma unroll
+                    for (int i = 0; i < FA; ++i)
+#pragma unroll
+                        for (int j = 0; j < 2; ++j)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[PA[t]][i], b[PB[t]][j], acc[i][j], 0, 0, 0);
+            }
         }
     };
 
@@ -438,7 +464,7 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
         if (s + AHEAD <= nst) softmap_stage_barrier<(NA + NB) * (AHEAD - 1)>();
         else softmap_stage_barrier<0>();
         if (s + AHEAD < nst) issue(s + AHEAD, nbuf);
-        compute(buf);
+        compute(buf, (s_begin + s) % 2 ? -1.0f : 1.0f);
         buf = buf + 1 == NBUF ? 0 : buf + 1;
         nbuf = nbuf + 1 == NBUF ? 0 : nbuf + 1;
     }
@@ -787,13 +813,13 @@ static void softmap_stats_launch(const SoftmapShape &h, const float *W, float sc
 #undef SM_STATS
 }
 static void softmap_pack_launch(int np, const float *src, const float *colscale, const float *other, float *dots, char *rows8,
-                                size_t rows_plane, char *cols8, size_t cols_plane, int R, int C, int Rp, int Cp, unsigned *largest,
-                                unsigned *clear, hipStream_t s) {
+                                size_t rows_plane, char *cols8, size_t cols_plane, int R, int C, int Rp, int Cp, float alternate,
+                                unsigned *largest, unsigned *clear, hipStream_t s) {
     const dim3 grid(Cp / 64, dl_ceil_div(Rp, 64));
     if (np == 1)
-        DL_TIMED("softmap_pack", s, (softmap_pack<1><<<grid, 256, 0, s>>>(src, colscale, other, dots, rows8, rows_plane, cols8, cols_plane, R, C, Rp, Cp, largest, clear)));
+        DL_TIMED("softmap_pack", s, (softmap_pack<1><<<grid, 256, 0, s>>>(src, colscale, other, dots, rows8, rows_plane, cols8, cols_plane, R, C, Rp, Cp, alternate, largest, clear)));
     else
-        DL_TIMED("softmap_pack", s, (softmap_pack<3><<<grid, 256, 0, s>>>(src, colscale, other, dots, rows8, rows_plane, cols8, cols_plane, R, C, Rp, Cp, largest, clear)));
+        DL_TIMED("softmap_pack", s, (softmap_pack<3><<<grid, 256, 0, s>>>(src, colscale, other, dots, rows8, rows_plane, cols8, cols_plane, R, C, Rp, Cp, alternate, largest, clear)));
 }
 static void softmap_reduce(const float *part, float *out, long long total, int chunks, hipStream_t s) {
     if (total % 4 == 0 && ((uintptr_t)out & 15) == 0)
@@ -833,7 +859,7 @@ extern "C" int dl_soft_map_fwd(const float *x, const float *W, float tau, float 
     unsigned *x_largest = h.np > 1 ? (unsigned *)(E + h.np * h.e_plane) : nullptr;
     if (h.np == 1) softmap_stats_launch<1>(h, W, SM_LOG2E / tau, mx, rs, E, x_largest, s);
     else softmap_stats_launch<3>(h, W, SM_LOG2E / tau, mx, rs, E, x_largest, s);
-    softmap_pack_launch(h.np, x, nullptr, nullptr, nullptr, nullptr, 0, x8, h.x_plane, B, I, h.Bp, h.Ip, x_largest, nullptr, s);
+    softmap_pack_launch(h.np, x, nullptr, nullptr, nullptr, nullptr, 0, x8, h.x_plane, B, I, h.Bp, h.Ip, 1.0f, x_largest, nullptr, s);
     SoftmapArgs g{};
     g.A = x8; g.a_plane = h.x_plane; g.lda = h.Bp;
     g.Bm = E; g.b_plane = h.e_plane; g.ldb = h.Ip;
@@ -875,8 +901,8 @@ extern "C" int dl_soft_map_bwd(const float *x, const float *W, float tau, const 
     char *gb = w; w += h.np * h.g_plane;     // gm [Bp/8][Mp]
     char *go = w; w += h.np * h.g_plane;     // gs [Mp/8][Bp]
     unsigned *gm_largest = h.np > 1 ? (unsigned *)w : nullptr;
-    softmap_pack_launch(h.np, x, nullptr, nullptr, nullptr, xb, h.x_plane, nullptr, 0, B, I, h.Bp, h.Ip, nullptr, gm_largest, s);
-    softmap_pack_launch(h.np, gm, rs, m, dots, gb, h.g_plane, go, h.g_plane, B, M, h.Bp, h.Mp, gm_largest, nullptr, s);
+    softmap_pack_launch(h.np, x, nullptr, nullptr, nullptr, xb, h.x_plane, nullptr, 0, B, I, h.Bp, h.Ip, 1.0f, nullptr, gm_largest, s);
+    softmap_pack_launch(h.np, gm, rs, m, dots, gb, h.g_plane, go, h.g_plane, B, M, h.Bp, h.Mp, -1.0f, gm_largest, nullptr, s);
     SoftmapArgs g{};
     g.A = go; g.a_plane = h.g_plane; g.lda = h.Bp;
     g.Bm = E; g.b_plane = h.e_plane; g.ldb = h.Ip;

@@ -737,6 +737,21 @@ def test_soft_mapping_of_values_beyond_bf16(value):
     assert float(((m.double() - want).abs() / want.abs()).max()) <= 1e-5
 
 
+def test_soft_mapping_fp32_input_gradient_does_not_drift():
+    """The long reduction of gx (24000 selections) stays an fp32 sum.  Independent roundings of 2^-25 (rms): of S two and its
+    exponent's (|w - max| about 2), 1.2e-7 together; of the running sum one per 16 products, 75 in a chunk, sqrt(75 / 2) of them
+    in the 2-norm, 1.8e-7: 2.2e-7, limit 3e-7.  One running sum for all plane products, rounded downwards, has 6.2e-7."""
+    ops = _ops()
+    B, I, M = 64, 3136, 24000
+    g = torch.Generator("cuda").manual_seed(3)
+    x = torch.rand(B, I, device="cuda", generator=g).requires_grad_()
+    W = torch.randn(M, I, device="cuda", generator=g) * 0.5
+    gm = torch.randn(B, M, device="cuda", generator=g)
+    ops.SoftMapFunction.apply(x, W.requires_grad_(), 1.0, 0).backward(gm)
+    want = gm.double() @ torch.softmax(W.detach().double(), dim=-1)
+    assert float((x.grad.double() - want).norm()) <= 3e-7 * float(want.norm())
+
+
 LOWEST = float(np.finfo(np.float32).min)
 
 
