@@ -195,11 +195,13 @@ __global__ __launch_bounds__(256) void softmap_pack(const float *__restrict__ sr
                                                     char *__restrict__ rows8, size_t rows_plane, char *__restrict__ cols8,
                                                     size_t cols_plane, int R, int C, int Rp, int Cp, float alternate, unsigned *__restrict__ largest,
                                                     unsigned *__restrict__ clear) {
-    if (clear && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) *clear = 0;
+    // (a grid of one dimension: the second holds 65535 blocks, 4.19 million rows)
+    const int cb64 = Cp / 64, bx = blockIdx.x % cb64, by = blockIdx.x / cb64;
+    if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0;
     __shared__ float tile[64][65];
     __shared__ float part[4][64];
     const int c = threadIdx.x & 63, g = threadIdx.x >> 6;
-    const int col = blockIdx.x * 64 + c, r0 = blockIdx.y * 64;
+    const int col = bx * 64 + c, r0 = by * 64;
     float v[16], dot = 0.0f;
     float f = colscale && col < C ? colscale[col] : 1.0f;
     if (NP > 1 && (col / SM_GX_STAGE) % 2 != 0) f *= alternate;
@@ -228,7 +230,7 @@ __global__ __launch_bounds__(256) void softmap_pack(const float *__restrict__ sr
 #pragma unroll
     for (int i = 0; i < 16; ++i) tile[g * 16 + i][c] = v[i] * f;
     __syncthreads();
-    if (other && g == 0) dots[(size_t)blockIdx.y * Cp + col] = ((part[0][c] + part[1][c]) + part[2][c]) + part[3][c];
+    if (other && g == 0) dots[(size_t)by * Cp + col] = ((part[0][c] + part[1][c]) + part[2][c]) + part[3][c];
     if (rows8) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -248,7 +250,7 @@ __global__ __launch_bounds__(256) void softmap_pack(const float *__restrict__ sr
                 float w[8];
 #pragma unroll
                 for (int j = 0; j < 8; ++j) w[j] = tile[c][cb * 8 + j];
-                char *d = cols8 + ((size_t)(blockIdx.x * 8 + cb) * Rp + row) * SM_UNIT;
+                char *d = cols8 + ((size_t)(bx * 8 + cb) * Rp + row) * SM_UNIT;
 #pragma unroll
                 for (int p = 0; p < NP; ++p) *reinterpret_cast<uint4 *>(d + p * cols_plane) = softmap_unit(w);
             }
@@ -815,7 +817,7 @@ static void softmap_stats_launch(const SoftmapShape &h, const float *W, float sc
 static void softmap_pack_launch(int np, const float *src, const float *colscale, const float *other, float *dots, char *rows8,
                                 size_t rows_plane, char *cols8, size_t cols_plane, int R, int C, int Rp, int Cp, float alternate,
                                 unsigned *largest, unsigned *clear, hipStream_t s) {
-    const dim3 grid(Cp / 64, dl_ceil_div(Rp, 64));
+    const int grid = Cp / 64 * dl_ceil_div(Rp, 64);
     if (np == 1)
         DL_TIMED("softmap_pack", s, (softmap_pack<1><<<grid, 256, 0, s>>>(src, colscale, other, dots, rows8, rows_plane, cols8, cols_plane, R, C, Rp, Cp, alternate, largest, clear)));
     else

@@ -810,6 +810,23 @@ def test_soft_mapping_fp32_range(shape, side, case):
         assert float(rel.max()) <= 1e-5
 
 
+@pytest.mark.parametrize("precision", [0, 1])
+def test_soft_mapping_of_more_rows_than_a_grid_dimension(precision):
+    """4.19 million rows are 65536 blocks of 64 rows; limits as in test_soft_mapping_tile_edges."""
+    ops = _ops()
+    B, I, M = 4_194_400, 3, 2
+    g = torch.Generator("cuda").manual_seed(1)
+    x = torch.rand(B, I, device="cuda", generator=g).requires_grad_()
+    W = torch.randn(M, I, device="cuda", generator=g)
+    gm = torch.randn(B, M, device="cuda", generator=g)
+    m = ops.SoftMapFunction.apply(x, W, 1.0, precision)
+    m.backward(gm)
+    S = torch.softmax(W.double(), dim=-1)
+    limit = 1e-5 if precision == 0 else 1e-2
+    for got, want in ((m.detach(), x.detach().double() @ S.t()), (x.grad, gm.double() @ S)):
+        assert float((got.double() - want).abs().max()) <= limit * float(want.abs().max())
+
+
 def test_soft_and_hard_mapping_against_reference_vectors(golden):
     ops = _ops()
     g = golden
