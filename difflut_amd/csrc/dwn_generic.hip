@@ -13,15 +13,17 @@ __device__ __forceinline__ unsigned dwn_addr_generic(const float *xrow, const in
 
 __global__ __launch_bounds__(256) void dwn_generic_fwd(const float *__restrict__ x, const int *__restrict__ idx32,
                                                         const float *__restrict__ luts, float *__restrict__ y,
-                                                        int B, int I, int N, int K, int O) {
+                                                        int B, int I, int N, int K, int O, uint8_t *__restrict__ addrT,
+                                                        int rows) {
     const long long gid = (long long)blockIdx.x * 256 + threadIdx.x;
     const long long NO = (long long)N * O;
-    if (gid >= (long long)B * NO) return;
+    if (gid >= (long long)rows * NO) return;
     const int b = (int)(gid / NO);
     const long long c = gid % NO;
     const int n = (int)(c / O);
-    const unsigned a = dwn_addr_generic(x + (size_t)b * I, idx32 + (size_t)n * K, K);
-    y[gid] = luts[(c << K) + a];
+    const unsigned a = b < B ? dwn_addr_generic(x + (size_t)b * I, idx32 + (size_t)n * K, K) : 0;
+    if (b < B) y[gid] = luts[(c << K) + a];
+    if (addrT && c % O == 0) addrT[((size_t)(b >> 6) * N + n) * 64 + (b & 63)] = (uint8_t)a;
 }
 
 __global__ __launch_bounds__(256) void dwn_generic_bwd_gx(const float *__restrict__ x, const int *__restrict__ idx32,
@@ -153,11 +155,17 @@ __global__ __launch_bounds__(256) void dwn_generic_zero(float *p, long long n) {
 #define DWN_GENERIC_LDS_FLOATS 32768
 __global__ __launch_bounds__(1024) void dwn_generic_fwd_lds(const float *__restrict__ x, const int *__restrict__ idx32,
                                                              const float *__restrict__ luts, float *__restrict__ y, int B,
-                                                             int I, long long NO, int K, int O) {
+                                                             int I, long long NO, int K, int O, uint8_t *__restrict__ addrT,
+                                                             int rows) {
     extern __shared__ float dwn_generic_row[];
     float *row = dwn_generic_row;
     const bool vec = (I & 3) == 0 && (((uintptr_t)x) & 15) == 0;
-    for (int b = blockIdx.x; b < B; b += gridDim.x) {
+    for (int b = blockIdx.x; b < rows; b += gridDim.x) {
+        uint8_t *addr = addrT ? addrT + (size_t)(b >> 6) * (NO / O) * 64 + (b & 63) : nullptr;
+        if (b >= B) {  // (only with addresses)
+            for (long long n = threadIdx.x; n < NO / O; n += 1024) addr[n * 64] = 0;
+            continue;
+        }
         const float *xrow = x + (size_t)b * I;
         __syncthreads();  // the readers of the row before are done
         if (vec) {
@@ -170,13 +178,18 @@ __global__ __launch_bounds__(1024) void dwn_generic_fwd_lds(const float *__restr
         for (long long c = threadIdx.x; c < NO; c += 1024) {
             const unsigned a = dwn_addr_generic(row, idx32 + (size_t)(c / O) * K, K);
             __builtin_nontemporal_store(luts[(c << K) + a], y + (size_t)b * NO + c);
+            if (addr && c % O == 0) addr[c / O * 64] = (uint8_t)a;
         }
     }
 }
 
+// addrT (nullable; k = 7 and 8): the address of every (node, row) as the lookup forward saves it, [tile][node][64], rows past
+// B zero.  Its bytes leave with the rows of y: 1024 rows, 4096 -> 2048 nodes of 8 inputs 44 us, 37 without addresses (a pass of
+// its own over x: 105).
 int dwn_generic_forward(const float *x, const int *idx32, const float *luts, float *y, int B, int I, int N, int k, int O,
-                        hipStream_t s) {
+                        hipStream_t s, uint8_t *addrT) {
     const long long NO = (long long)N * O;
+    const int rows = addrT ? (B + 63) / 64 * 64 : B;
     if (I <= DWN_GENERIC_LDS_FLOATS && NO >= 1024) {
         const size_t lds = (size_t)I * sizeof(float);
         if (lds > 64 * 1024) {
@@ -185,25 +198,10 @@ int dwn_generic_forward(const float *x, const int *idx32, const float *luts, flo
             if (e != hipSuccess) return (int)e;
         }
         const int per_cu = lds + 1024 <= 80 * 1024 ? 2 : 1;
-        dwn_generic_fwd_lds<<<B < 256 * per_cu ? B : 256 * per_cu, 1024, lds, s>>>(x, idx32, luts, y, B, I, NO, k, O);
+        dwn_generic_fwd_lds<<<rows < 256 * per_cu ? rows : 256 * per_cu, 1024, lds, s>>>(x, idx32, luts, y, B, I, NO, k, O, addrT, rows);
         return dl_launch_status();
     }
-    dwn_generic_fwd<<<dl_ceil_div((long long)B * N * O, 256), 256, 0, s>>>(x, idx32, luts, y, B, I, N, k, O);
-    return dl_launch_status();
-}
-
-// addresses of every (node, row) as the lookup forward of k = 7 and 8 saves them, [tile][node][64], rows past B zero
-__global__ __launch_bounds__(256) void dwn_generic_addr(const float *__restrict__ x, const int *__restrict__ idx32,
-                                                         uint8_t *__restrict__ addrT, long long total, int B, int I, int N, int K) {
-    const long long e = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (e >= total) return;
-    const long long tn = e >> 6;
-    const long long b = tn / N * 64 + (e & 63);
-    addrT[e] = b < B ? (uint8_t)dwn_addr_generic(x + (size_t)b * I, idx32 + (size_t)(tn % N) * K, K) : (uint8_t)0;
-}
-int dwn_generic_addresses(const float *x, const int *idx32, uint8_t *addrT, int B, int I, int N, int k, hipStream_t s) {
-    const long long total = (long long)((B + 63) / 64) * N * 64;
-    dwn_generic_addr<<<dl_ceil_div(total, 256), 256, 0, s>>>(x, idx32, addrT, total, B, I, N, k);
+    dwn_generic_fwd<<<dl_ceil_div((long long)rows * N * O, 256), 256, 0, s>>>(x, idx32, luts, y, B, I, N, k, O, addrT, rows);
     return dl_launch_status();
 }
 

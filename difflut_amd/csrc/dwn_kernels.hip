@@ -1542,8 +1542,7 @@ static int dwn_forward_fast(const float *x, const int32_t *idx32, const float *l
 // Any other forward.  What a backward of k = 7 or 8 would read from `saved` is written whenever the caller brings it.
 static int dwn_forward_generic(const float *x, const int32_t *idx32, const float *luts, float *y, void *saved, int B, int I, int N,
                                int k, int O, hipStream_t s) {
-    const int rc = dwn_generic_forward(x, idx32, luts, y, B, I, N, k, O, s);
-    return rc || !saved || !dwn_wide(N, k, O) ? rc : dwn_generic_addresses(x, idx32, (uint8_t *)saved, B, I, N, k, s);
+    return dwn_generic_forward(x, idx32, luts, y, B, I, N, k, O, s, dwn_wide(N, k, O) ? (uint8_t *)saved : nullptr);
 }
 
 extern "C" int dl_dwn_layer_fwd(const float *x, const int32_t *idx32, const float *luts, float *y, void *saved,
@@ -1594,8 +1593,9 @@ extern "C" int dl_dwn_layer_fwd_static(const float *x, const int32_t *idx32, con
     int rc = dwn_check(B, I, N, k, O);
     if (rc) return rc;
     hipStream_t s = (hipStream_t)stream;
-    if (!dwn_fast(N, k, O) && !(dwn_wide(N, k, O) && saved && dwn_planes_bytes(B, I) <= (size_t)DL_DWN_STATIC_SCRATCH_BYTES))
-        return dwn_forward_generic(x, idx32, luts, y, saved, B, I, N, k, O, s);  // uses no scratch
+    // k > 6 keeps off the shared array, as the header promises: such calls may overlap (1024 rows, 4096 -> 2048 nodes of 8
+    // inputs: 44 us, 18 with planes in the shared array)
+    if (!dwn_fast(N, k, O)) return dwn_forward_generic(x, idx32, luts, y, saved, B, I, N, k, O, s);
     if (!saved) return DL_ERR_NULL;
     if (dwn_planes_bytes(B, I) > (size_t)DL_DWN_STATIC_SCRATCH_BYTES) return DL_ERR_SCRATCH;
     void *planes = nullptr;

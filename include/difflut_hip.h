@@ -99,9 +99,10 @@ int dl_dwn_layer_fwd(const float *x, const int32_t *idx32, const float *luts, fl
  * dl_dwn_layer_fwd puts into `ws` go to a device array owned by the library instead
  * (DL_DWN_STATIC_SCRATCH_BYTES on every GPU the library runs on, held until the process ends).  The call
  * allocates and frees nothing.  Limit: ceil(B/64) * I * 8 <= DL_DWN_STATIC_SCRATCH_BYTES when
- * k <= DL_MAX_FAST_K (e.g. B = 4096 with I = 16384), otherwise DL_ERR_SCRATCH; larger k does without it.
+ * k <= DL_MAX_FAST_K (e.g. B = 4096 with I = 16384), otherwise DL_ERR_SCRATCH; larger k uses no scratch.
  * All calls on one GPU share that GPU's array: calls that overlap on one GPU (two streams, two threads)
- * race on it and must be serialised by the caller.  Nothing in it has to survive between calls.
+ * race on it and must be serialised by the caller (k > DL_MAX_FAST_K: they may overlap).  Nothing in it has to survive
+ * between calls.
  * The first call on each device also looks up the device address of the array (hipGetSymbolAddress, which may
  * load the code object): make that call before any stream capture begins; every later call on the device only
  * enqueues kernels and can be captured. */

@@ -64,6 +64,34 @@ def test_static_scratch_forward_at_its_limit_and_beyond():
     assert rc == -6 and b"scratch" in lib.dl_error_string(rc)
 
 
+@pytest.mark.parametrize("k", [7, 8])
+def test_static_forward_of_wide_nodes_keeps_off_the_shared_array(k):
+    """Calls with k > 6 may overlap on one GPU: nothing is packed into the library's array (whose only writer is the pack
+    kernel), and the addresses for the backward are there all the same."""
+    from difflut_amd import _native as nat
+    lib = nat.lib()
+    nat.profile_read()
+    nat.profile_enable(True)
+    try:
+        _run_both(lib, nat, 31, 130, 64, 30, k, 1)
+        names = [name for name, _ in nat.profile_read()]
+    finally:
+        nat.profile_enable(False)
+    # the call with a workspace packs its own planes; the other one does not
+    assert names.count("dwn_pack_planes") == 1
+    dims = (130, 64, 30, k, 1)
+    x = torch.rand(130, 64, device=DEV)
+    idx = orc.random_mapping(64, 30, k, seed=5).to(torch.int32).to(DEV).contiguous()
+    luts = torch.rand(30, 1, 1 << k, device=DEV)
+    y = torch.empty(130, 30, device=DEV)
+    saved = torch.zeros(lib.dl_dwn_saved_bytes(*dims), dtype=torch.uint8, device=DEV)
+    nat.check(lib.dl_dwn_layer_fwd_static(x.data_ptr(), idx.data_ptr(), luts.data_ptr(), y.data_ptr(), saved.data_ptr(), *dims,
+                                          nat.stream()))
+    addr = sum(((x[:, idx[:, j].long()] >= 0.5).long() << j) for j in range(k))
+    got = saved[: 3 * 30 * 64].view(3, 30, 64).permute(0, 2, 1).reshape(192, 30)[:130].long()
+    assert torch.equal(got, addr)
+
+
 def test_static_scratch_forward_allocates_nothing_and_can_be_captured():
     """After the first call on the device (which looks up the array's address) a call neither changes the device's
     free memory nor needs anything a stream capture forbids: the same call replayed from a HIP graph, with eager
