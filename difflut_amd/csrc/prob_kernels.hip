@@ -256,7 +256,7 @@ __device__ __forceinline__ void prob_fold_gradient(const float (&v0)[1 << KH], c
     }
 }
 
-// one wavefront per (column, chunk of batch tiles); sixteen wavefronts, i.e. sixteen columns, per block.
+// one wavefront per (column, chunk of batch tiles); W wavefronts, i.e. sixteen columns (or four), per block.
 // HYB (hybrid node): the table is used as given and the input gradient carries the factor
 // q / (q + 1e-8), q = x_j (1 - x_j), of that node's backward.
 // The weight of table entry a is a product over the inputs, so it factors into one over the lower KL and one over the upper
@@ -267,12 +267,14 @@ __device__ __forceinline__ void prob_fold_gradient(const float (&v0)[1 << KH], c
 // stays in registers: sixteen wavefronts of it fit a CU at every k, where the fold left room for eight at k = 6.
 // gy is the row-major gradient itself: the block's 16 columns are 64 contiguous bytes of a row, the 64 x 16 piece of a
 // batch tile is fetched one value per thread a tile ahead and turned through the LDS (two buffers, one barrier per tile).
-template <int K, bool HYB>
-__global__ __launch_bounds__(1024) void prob_bwd_t(const float *__restrict__ xT, const float *__restrict__ gy,
+// W = 4 (at most 12 columns): blocks of four columns, so that at most three wavefronts of a block have none, and four
+// blocks on a CU.  65536 rows x 8 columns, k = 6: 84 us in blocks of sixteen and at most 16 chunks, 14.5 in blocks of four.
+template <int K, bool HYB, int W = 16>
+__global__ __launch_bounds__(64 * W) void prob_bwd_t(const float *__restrict__ xT, const float *__restrict__ gy,
                                                    const int *__restrict__ idx32, const float *__restrict__ sig,
                                                    float *__restrict__ gmT, float *__restrict__ gpart, int I, int N,
                                                    int O, int BT, int tiles_per_chunk, int want_gm, int B) {
-    constexpr int L = 1 << K, W = 16;
+    constexpr int L = 1 << K;
     constexpr int KL = K / 2, KU = K - KL, LL = 1 << KL, LU = 1 << KU;
     __shared__ float gturn[2][W][65];  // [buffer][column][row]
     const int NO = N * O;
@@ -293,7 +295,7 @@ __global__ __launch_bounds__(1024) void prob_bwd_t(const float *__restrict__ xT,
     for (int a = 0; a < L; ++a) acc[a] = 0.0f;
     const int t0 = chunk * tiles_per_chunk, t1 = min(BT, t0 + tiles_per_chunk);
     float nxs[K], ng = 0.0f;  // operands of the next batch tile, requested one tile ahead
-    const int trow = threadIdx.x >> 4, tcol = threadIdx.x & 15;  // my value of the 64 x 16 piece
+    const int trow = threadIdx.x / W, tcol = threadIdx.x % W;  // my value of the 64 x W piece
     auto request = [&](int t) {
         const __amdgpu_buffer_rsrc_t rs_x = __builtin_amdgcn_make_buffer_rsrc((void *)(xT + (size_t)t * I * 64), 0, I * 256, PROB_RSRC);
 #pragma unroll
@@ -395,7 +397,15 @@ __device__ __forceinline__ void prob_reduce_element(const ProbReduce &R, long lo
     const long long total = (long long)N * L * O;
     if (e >= total) return;
     float acc = 0.0f;
-    for (int ch = 0; ch < chunks; ++ch) acc += gpart[(size_t)ch * total + e];
+    int ch = 0;
+    for (; ch + 8 <= chunks; ch += 8) {  // eight loads in flight, added in chunk order (one at a time: 0.2 us a chunk)
+        float part[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) part[q] = gpart[(size_t)(ch + q) * total + e];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) acc += part[q];
+    }
+    for (; ch < chunks; ++ch) acc += gpart[(size_t)ch * total + e];
     if (!sig) {
         graw[e] = acc;
         return;
@@ -640,21 +650,30 @@ static inline bool prob_fast(int I, int N, int k, int O) {
 // temperature.clamp(min=1e-6); with a per-node array the kernels take every node's own value
 static inline ProbTemp prob_temp(float t, const float *t_n) { return ProbTemp{1.0f / (t > 1e-6f ? t : 1e-6f), t_n}; }
 static inline int prob_bt(int B) { return (B + 63) / 64; }
-// Batch tiles per wavefront of prob_bwd_t.  Its blocks (16 columns x one chunk of tiles) share 256 CUs: the fullest CU has
-// ceil(blocks / 256) of them, and a block spends about 2 (k <= 4), 4 or 6 (k = 6) tiles' time on its table and its sums over
-// the lanes.  2000 x 3001 -> 5003 hybrid nodes of 4 inputs (313 blocks a chunk): one chunk 82 us, four 64; where one chunk
-// is 256 blocks, more of them lose (1024 x 4096 -> 4096 nodes: k = 4 27.7 -> 27.3 us, k = 5 32.4 -> 34.7).
+static inline int prob_block_columns(long long NO) { return NO <= 12 ? 4 : 16; }
+// Batch tiles per wavefront of prob_bwd_t.  Its blocks (16 or 4 columns x one chunk of tiles) share 256 CUs of 16 wavefronts:
+// the fullest CU has so many rounds of them, a block spends about 2 (k <= 4), 4 or 6 (k = 6) tiles' time on its table and
+// its sums over the lanes, and the sum over the chunks costs a twentieth of a tile's time each.  2000 x 3001 -> 5003 hybrid
+// nodes of 4 inputs (313 blocks a chunk): one chunk 82 us, four 64; 1024 x 4096 -> 4096 nodes, where one chunk is 256 blocks,
+// keep it (k = 5: 31.7 against 34.7 in more).  Few columns over many rows, with at most 16 chunks / as here, kernel and
+// gather with the sum, us: 147456 rows x 32 columns, k = 6 243 + 42 / 52 + 46, k = 4 144 + 27 / 37 + 29; 65536 rows x 1 column, k = 6
+// 67 + 7 / 11 + 11, x 64 columns, k = 4 57 + 17 / 26 + 17.
 static inline int prob_tiles_per_chunk(int B, int N, int k, int O) {
     const int BT = prob_bt(B), own = k >= 6 ? 6 : (k == 5 ? 4 : 2);
-    const long long blocks = dl_ceil_div((long long)N * O, 16);
+    const int W = prob_block_columns((long long)N * O), resident = 256 * 16 / W;
+    const long long blocks = dl_ceil_div((long long)N * O, W);
     int best = BT;
     double best_cost = 0.0;
-    for (int c = 1; c <= BT && c <= 16; ++c) {
-        const int tpc = dl_ceil_div(BT, c);
-        const long long all = blocks * dl_ceil_div(BT, tpc);
-        const double cost = (all > 256 ? (double)dl_ceil_div(all, 256) : 1.1) * (tpc + own);
-        if (c == 1 || cost < best_cost) { best = tpc; best_cost = cost; }
-    }
+    auto consider = [&](long long c) {
+        if (c < 1 || c > BT) return;
+        const int tpc = dl_ceil_div(BT, c), chunks = dl_ceil_div(BT, tpc);
+        const long long all = blocks * chunks;
+        const double cost = (all > resident ? (double)dl_ceil_div(all, resident) : 1.1) * (tpc + own) + 0.05 * chunks;
+        if (best_cost == 0.0 || cost < best_cost) { best = tpc; best_cost = cost; }
+    };
+    for (int c = 1; c <= 16; ++c) consider(c);
+    for (int c = 20; c <= BT; c += c / 4) consider(c);
+    for (int rounds = 1; rounds <= 4; ++rounds) consider(rounds * resident / blocks);  // no CU idle in the last round
     return best;
 }
 static inline size_t prob_sig_bytes(int N, int k, int O) { return dl_align256((size_t)N * O * ((size_t)1 << k) * sizeof(float)); }
@@ -719,6 +738,22 @@ extern "C" int dl_prob_layer_fwd_nodes(const float *x, const int32_t *idx32, con
     return prob_forward(x, idx32, raw_w, prob_temp(1.0f, temperature_n), y, saved, saved_bytes, B, I, N, k, O, stream);
 }
 
+template <bool HYB>
+static void prob_launch_bwd(const char *name, const float *xT, const float *gy, const int32_t *idx32, const float *table,
+                            float *gmT, float *gpart, int B, int I, int N, int k, int O, int tpc, bool want_gm, hipStream_t s) {
+    const int BT = prob_bt(B), NO = N * O, W = prob_block_columns(NO);
+    const dim3 grid(dl_ceil_div(NO, W), dl_ceil_div(BT, tpc));
+#define CALL(KK)                                                                                                                  \
+    do {                                                                                                                          \
+        if (W == 4) DL_TIMED(name, s, (prob_bwd_t<KK, HYB, 4><<<grid, 256, 0, s>>>(xT, gy, idx32, table, gmT, gpart, I, N, O, BT, \
+                                                                                   tpc, want_gm, B)));                            \
+        else DL_TIMED(name, s, (prob_bwd_t<KK, HYB><<<grid, 1024, 0, s>>>(xT, gy, idx32, table, gmT, gpart, I, N, O, BT, tpc,     \
+                                                                          want_gm, B)));                                          \
+    } while (0)
+    PROB_DISPATCH(k, CALL)
+#undef CALL
+}
+
 static int prob_backward(const float *x, const void *saved, const int32_t *idx32, const int32_t *inv_ptr,
                          const int32_t *inv_pos, const float *raw_w, ProbTemp inv_t, const float *gy, float *gx, float *graw,
                          void *ws, size_t ws_bytes, int B, int I, int N, int k, int O, void *stream) {
@@ -752,12 +787,7 @@ static int prob_backward(const float *x, const void *saved, const int32_t *idx32
         DL_TIMED("prob_sig_table", s, (prob_sig_table<<<dl_ceil_div(WT, 256), 256, 0, s>>>(raw_w, inv_t, sig, N, L, O)));
         DL_TIMED("prob_to_tiles_x", s, (prob_to_tiles<false><<<dim3(dl_ceil_div(I, 64), BT), 256, 0, s>>>(x, xT, B, I)));
     }
-#define CALL(KK)                                                                                                       \
-    DL_TIMED("prob_bwd_t", s,                                                                                          \
-             (prob_bwd_t<KK, false><<<dim3(dl_ceil_div(NO, 16), chunks), 1024, 0, s>>>(xT, gy, idx32, sig, gmT, gpart, I, N, \
-                                                                                    O, BT, tpc, gx != nullptr, B)))
-    PROB_DISPATCH(k, CALL)
-#undef CALL
+    prob_launch_bwd<false>("prob_bwd_t", xT, gy, idx32, sig, gmT, gpart, B, I, N, k, O, tpc, gx != nullptr, s);
     const ProbReduce R = {gpart, sig, inv_t, graw, N, L, O, chunks};
     prob_launch_gather_and_reduce(gmT, inv_ptr, inv_pos, gx, B, I, N, k, O, BT, R, WT, s);
     return dl_launch_status();
@@ -856,12 +886,7 @@ static int hybrid_backward(const float *x, const void *saved, const int32_t *idx
     }
     float *gmT = (float *)w; w += dl_align256((size_t)BT * NO * k * 64 * sizeof(float));
     float *gpart = (float *)w;
-#define CALL(KK)                                                                                                          \
-    DL_TIMED("hybrid_bwd_t", s,                                                                                           \
-             (prob_bwd_t<KK, true><<<dim3(dl_ceil_div(NO, 16), chunks), 1024, 0, s>>>(xT, gy, idx32, luts, gmT, gpart, I, N, O, \
-                                                                                   BT, tpc, gx != nullptr, B)))
-    PROB_DISPATCH(k, CALL)
-#undef CALL
+    prob_launch_bwd<true>("hybrid_bwd_t", xT, gy, idx32, luts, gmT, gpart, B, I, N, k, O, tpc, gx != nullptr, s);
     const ProbReduce R = {gpart, nullptr, ProbTemp{1.0f, nullptr}, gluts, N, L, O, chunks};
     prob_launch_gather_and_reduce(gmT, inv_ptr, inv_pos, gx, B, I, N, k, O, BT, R, WT, s);
     return dl_launch_status();

@@ -601,6 +601,37 @@ def test_prob_backward_factored_weights(B, N, O, T, k):
     np.testing.assert_allclose(wt.grad.cpu().numpy(), gw, rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("k", [1, 4, 6])
+@pytest.mark.parametrize("hybrid", [False, True])
+@pytest.mark.parametrize("B,N,O", [(63, 1, 1), (5000, 1, 1),    # one column
+                                   (700, 3, 2), (700, 6, 2),   # blocks of four columns, the last half empty; their largest
+                                   (700, 13, 1),               # one column more: blocks of sixteen
+                                   (4160, 32, 1), (4161, 5, 1)])  # many chunks, a tile each and with a last one
+def test_prob_backward_of_few_columns(B, N, O, hybrid, k):
+    """Few columns over many rows: blocks of four columns, chunks down to one batch tile.  Floors as in
+    test_prob_backward_factored_weights; table gradients sum up to 5000 rows of size 4, about sqrt(5000) * 4 * 6e-8: floor 2e-5."""
+    ops = _ops()
+    I = 11
+    rng = np.random.default_rng(B + N + k)
+    x = rng.uniform(0, 1, (B, I)).astype(np.float32)
+    idx = orc.random_mapping(I, N, k, seed=4).numpy().astype(np.int64)
+    gy = rng.uniform(-4, 4, (B, N, O)).astype(np.float32)
+    plan = ops.MappingPlan(dev(idx, torch.int32), I)
+    xt = dev(x).requires_grad_()
+    if hybrid:
+        raw = rng.uniform(-1, 1, (N, O, 1 << k)).astype(np.float32)
+        wt = dev(raw).requires_grad_()
+        ops.hybrid_layer(xt, ops.table_sigmoid(wt), plan).backward(dev(gy.reshape(B, -1)))
+        gx, gw = orc.hybrid_layer_backward(x, idx, raw, gy)
+    else:
+        raw = rng.uniform(-1, 1, (N, 1 << k, O)).astype(np.float32)
+        wt = dev(raw).requires_grad_()
+        ops.ProbLayerFunction.apply(xt, wt, plan, 1.0).backward(dev(gy.reshape(B, -1)))
+        gx, gw = orc.prob_layer_backward(x, idx, raw, gy, 1.0)
+    np.testing.assert_allclose(xt.grad.cpu().numpy(), gx, rtol=1e-5, atol=5e-6)
+    np.testing.assert_allclose(wt.grad.cpu().numpy(), gw, rtol=1e-5, atol=2e-5)
+
+
 @pytest.mark.parametrize("tag", ["k4o2", "k6o1"])
 def test_prob_node_against_reference_vectors(golden, tag):
     from difflut_amd.nodes.probabilistic_node import probabilistic_forward

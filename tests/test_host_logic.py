@@ -267,6 +267,24 @@ def test_argument_checks_of_the_later_entry_points_need_no_gpu():
     assert lib.dl_hybrid_bwd_workspace_bytes(*dims) >= 4096 * (16384 + 8192 + 6 * 8192) * 4
 
 
+@pytest.mark.parametrize("B,N,k", [(147456, 32, 6), (147456, 32, 4), (65536, 1, 6), (65536, 64, 4), (65536, 8, 6)])
+def test_narrow_layers_are_cut_into_chunks_that_fill_the_card(B, N, k):
+    """The probabilistic backward of few columns over many rows: what its workspace holds of partial table gradients says into
+    how many chunks of rows it is cut; with one wavefront per column and chunk, 4096 would fill 256 CUs.  At least a fifth of
+    that (fewer chunks are a shorter sum over them)."""
+    from difflut_amd import _native as nat
+    lib = nat.lib()
+
+    def up(v):
+        return (v + 255) // 256 * 256
+
+    I, tiles = 40, (B + 63) // 64
+    hybrid = lib.dl_hybrid_bwd_saved_workspace_bytes(B, I, N, k, 1)  # dL/d(mapped inputs) and the partial sums
+    chunks = (hybrid - up(tiles * N * k * 64 * 4)) // (N * 4 << k)
+    assert chunks <= tiles
+    assert N * chunks >= min(N * tiles, 4096) // 5 or chunks >= 64
+
+
 # ------------------------------------------------------------------------------ parameter and scalar banks
 def _small_dwn_layer(n=12, k=3, inputs=20):
     from difflut_amd.layers import RandomLayer
