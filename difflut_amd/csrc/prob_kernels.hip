@@ -18,8 +18,8 @@ typedef float prob_f4 __attribute__((ext_vector_type(4)));
 // table is read through scalar loads.  Tensors that cross the [batch, feature] boundary are
 // re-tiled once: xT [B/64][I][64], gmT [B/64][N*O*k][64], so the row of an
 // input (or a column's gradient) for a batch tile is 256 contiguous bytes, whatever the mapping.
-//   sig_table   : sig[c][a] = sigmoid(raw[n,a,d] / T), c = n*O + d                (tiny)
-//   to_tiles    : [B][C] -> [B/64][C][64], rows past B are zero
+//   to_tiles    : [B][C] -> [B/64][C][64], rows past B are zero; carries the tables (tiny): sig[c][a] =
+//                 sigmoid(raw[n,a,d] / T), c = n*O + d, and cen, the same less a value of the column's own
 //   fwd_t       : per (column, batch tile): fold the table along x_0, x_1, ... ; y leaves through
 //                 an LDS transpose as whole rows
 //   bwd_t       : one wavefront per column over a chunk of batch tiles.  The product weights factor into those of
@@ -50,31 +50,43 @@ __global__ __launch_bounds__(256) void prob_sig_table(const float *__restrict__ 
     sig[e] = dl_sigmoid(raw[((size_t)n * L + a) * O + d] * prob_inv_t_of(T, n));
 }
 
-// grid (ceil(C / 64), B/64 rounded up), 256 threads.  With `sig` set the launch carries extra rows of blocks
-// (blockIdx.y >= tiles) that build the sigmoid table in the same launch: the two jobs are independent and each is
-// too short to fill the machine on its own.
+// Tables for the backward, element e of [column][2^k]: sig (nullable) the sigmoid table, cen the same less a value of the
+// column's own, which no gradient of the inputs depends on: sums of it round by what the table varies, not by what it is.
+struct ProbTables {
+    const float *raw, *luts;  // probabilistic: weights [N][L][O], hybrid: the table as given, [N O][L]
+    ProbTemp T;
+    float *sig, *cen;
+    int N, L, O;
+};
+__device__ __forceinline__ void prob_table_element(const ProbTables &q, long long e) {
+    if (e >= (long long)q.N * q.L * q.O) return;
+    const int a = (int)(e % q.L);
+    const long long c = e / q.L;
+    const int n = (int)(c / q.O), d = (int)(c % q.O);
+    const float inv = q.luts ? 1.0f : prob_inv_t_of(q.T, n);
+    auto value = [&](int at) -> float {
+        return q.luts ? q.luts[c * q.L + at] : dl_sigmoid(q.raw[((size_t)n * q.L + at) * q.O + d] * inv);
+    };
+    const float v = value(a);
+    if (q.sig) q.sig[e] = v;
+    q.cen[e] = v - (q.L > 2 ? 0.5f * (value(0) + value(q.L - 1)) : value(0));  // (k = 1: the one difference itself)
+}
+
+// ceil(C / 64) * tiles blocks of 256 threads, and behind them those that build the tables of `q` (prob_table_blocks): the
+// two jobs are independent and each is too short to fill the machine on its own.
 // PLANES (the hybrid node's forward): the bit-planes a DWN lookup reads leave in the same pass, one ballot per column of the
 // tile in the LDS (word (t, c), bit r = src[64 t + r][c] >= 0.5, 0 past the batch).  HBM bound; x used to be read once by the
 // lookup's own packing pass and again by the backward's re-tiling.  Hybrid layer 4096 x 16384 -> 8192 nodes of six inputs,
 // forward + backward: 718 -> 683 us.
 template <bool PLANES = false>
 __global__ __launch_bounds__(256) void prob_to_tiles(const float *__restrict__ src, float *__restrict__ dst, int B, int C,
-                                                      int tiles = 1 << 30, const float *__restrict__ raw = nullptr,
-                                                      ProbTemp T = {1.0f, nullptr}, float *__restrict__ sig = nullptr,
-                                                      int N = 0, int L = 1, int O = 1,
-                                                      unsigned long long *__restrict__ planes = nullptr) {
+                                                      int tiles, ProbTables q, unsigned long long *__restrict__ planes = nullptr) {
     __shared__ float tile[64][65];  // [column][row]
-    if ((int)blockIdx.y >= tiles) {
-        const long long e = ((long long)(blockIdx.y - tiles) * gridDim.x + blockIdx.x) * 256 + threadIdx.x;
-        if (e < (long long)N * L * O) {
-            const int a = (int)(e % L);
-            const long long c = e / L;
-            const int n = (int)(c / O), d = (int)(c % O);
-            sig[e] = dl_sigmoid(raw[((size_t)n * L + a) * O + d] * prob_inv_t_of(T, n));
-        }
+    const int cols = (C + 63) / 64, t = blockIdx.x / cols, c0 = (int)(blockIdx.x % cols) * 64;
+    if (t >= tiles) {
+        prob_table_element(q, ((long long)blockIdx.x - (long long)cols * tiles) * 256 + threadIdx.x);
         return;
     }
-    const int t = blockIdx.y, c0 = blockIdx.x * 64;
     if ((C & 3) == 0 && c0 + 64 <= C && (((uintptr_t)src) & 15) == 0) {
 #pragma unroll
         for (int pass = 0; pass < 4; ++pass) {
@@ -110,6 +122,14 @@ __global__ __launch_bounds__(256) void prob_to_tiles(const float *__restrict__ s
         const prob_f4 v = {tile[c][r], tile[c][r + 1], tile[c][r + 2], tile[c][r + 3]};
         if (c0 + c < C) *reinterpret_cast<prob_f4 *>(dst + ((size_t)t * C + c0 + c) * 64 + r) = v;
     }
+}
+
+static inline int prob_table_blocks(const ProbTables &q) { return dl_ceil_div((long long)q.N * q.L * q.O, 256); }
+template <bool PLANES = false>
+static void prob_launch_to_tiles(const char *name, const float *x, float *xT, int B, int I, const ProbTables &q, hipStream_t s,
+                                 unsigned long long *planes = nullptr) {
+    const int BT = (B + 63) / 64, grid = dl_ceil_div(I, 64) * BT + prob_table_blocks(q);
+    DL_TIMED(name, s, (prob_to_tiles<PLANES><<<grid, 256, 0, s>>>(x, xT, B, I, BT, q, planes)));
 }
 
 // table of one column as wave-uniform values
@@ -265,13 +285,16 @@ __device__ __forceinline__ void prob_fold_gradient(const float (&v0)[1 << KH], c
 // gradient is g u[lo] w[hi].  Three times 2^k multiply-adds and little else (k = 6: about 280 instructions per column
 // and 64 rows where the fold of the whole table and its reverse took 440), and of arrays of 2^k only the table gradient
 // stays in registers: sixteen wavefronts of it fit a CU at every k, where the fold left room for eight at k = 6.
+// The sums V and Z are of the table less a value of the column's own (cen): they are taken differences of, and with the
+// table itself, whose values are about 0.5, gx stood 3.0e-7 from float64 (2-norm; uniform x, k = 6; hybrid 2.2e-7) where the fold
+// gave 2.3e-7 (1.7e-7); with cen 1.6e-7 (1.4e-7).
 // gy is the row-major gradient itself: the block's 16 columns are 64 contiguous bytes of a row, the 64 x 16 piece of a
 // batch tile is fetched one value per thread a tile ahead and turned through the LDS (two buffers, one barrier per tile).
 // W = 4 (at most 12 columns): blocks of four columns, so that at most three wavefronts of a block have none, and four
 // blocks on a CU.  65536 rows x 8 columns, k = 6: 84 us in blocks of sixteen and at most 16 chunks, 14.5 in blocks of four.
 template <int K, bool HYB, int W = 16>
 __global__ __launch_bounds__(64 * W) void prob_bwd_t(const float *__restrict__ xT, const float *__restrict__ gy,
-                                                   const int *__restrict__ idx32, const float *__restrict__ sig,
+                                                   const int *__restrict__ idx32, const float *__restrict__ cen,
                                                    float *__restrict__ gmT, float *__restrict__ gpart, int I, int N,
                                                    int O, int BT, int tiles_per_chunk, int want_gm, int B) {
     constexpr int L = 1 << K;
@@ -289,7 +312,7 @@ __global__ __launch_bounds__(64 * W) void prob_bwd_t(const float *__restrict__ x
 #pragma unroll
     for (int j = 0; j < K; ++j) off[j] = idx32[(size_t)n * K + j] * 256;
     float tab[L];
-    prob_load_table<K>(sig, c, tab);
+    prob_load_table<K>(cen, c, tab);
     float acc[L];
 #pragma unroll
     for (int a = 0; a < L; ++a) acc[a] = 0.0f;
@@ -679,10 +702,10 @@ static inline int prob_tiles_per_chunk(int B, int N, int k, int O) {
 static inline size_t prob_sig_bytes(int N, int k, int O) { return dl_align256((size_t)N * O * ((size_t)1 << k) * sizeof(float)); }
 static inline size_t prob_xT_bytes(int B, int I) { return dl_align256((size_t)prob_bt(B) * I * 64 * sizeof(float)); }
 
-// what the forward leaves for the backward: the sigmoid table and the re-tiled input
+// what the forward leaves for the backward: the sigmoid table, the re-tiled input and the table less a value per column
 extern "C" size_t dl_prob_saved_bytes(int B, int I, int N, int k, int O) {
     if (B <= 0 || I <= 0 || N <= 0 || k <= 0 || O <= 0 || !prob_fast(I, N, k, O)) return 256;
-    return prob_sig_bytes(N, k, O) + prob_xT_bytes(B, I);
+    return 2 * prob_sig_bytes(N, k, O) + prob_xT_bytes(B, I);
 }
 // (with room for one more [B, N O] array than the kernels use: the size does not shrink below what callers sized by before)
 extern "C" size_t dl_prob_bwd_workspace_bytes(int B, int I, int N, int k, int O) {
@@ -714,12 +737,9 @@ static int prob_forward(const float *x, const int32_t *idx32, const float *raw_w
     const int BT = prob_bt(B), L = 1 << k;
     float *sig = (float *)saved;
     float *xT = (float *)((char *)saved + prob_sig_bytes(N, k, O));
-    {   // x re-tiled and the sigmoid table built in one launch
-        const int gx_ = dl_ceil_div(I, 64);
-        const int extra = dl_ceil_div(dl_ceil_div((long long)N * L * O, 256), gx_);
-        DL_TIMED("prob_to_tiles_x+sig_table", s, (prob_to_tiles<false><<<dim3(gx_, BT + extra), 256, 0, s>>>(
-                                                     x, xT, B, I, BT, raw_w, inv_t, sig, N, L, O)));
-    }
+    // x re-tiled and the tables built in one launch
+    prob_launch_to_tiles("prob_to_tiles_x+sig_table", x, xT, B, I,
+                         ProbTables{raw_w, nullptr, inv_t, sig, (float *)((char *)xT + prob_xT_bytes(B, I)), N, L, O}, s);
     const int grid = dl_xcd_grid(dl_ceil_div((long long)N * O, PROB_TC), BT);
 #define CALL(KK) DL_TIMED("prob_fwd_t", s, (prob_fwd_t<KK><<<grid, 64 * PROB_FW, 0, s>>>(xT, idx32, sig, y, B, I, N, O, BT)))
     PROB_DISPATCH(k, CALL)
@@ -778,16 +798,17 @@ static int prob_backward(const float *x, const void *saved, const int32_t *idx32
     char *w = (char *)ws;
     float *sig = (float *)w; w += prob_sig_bytes(N, k, O);
     float *xT = (float *)w; w += prob_xT_bytes(B, I);
+    float *cen = (float *)w; w += prob_sig_bytes(N, k, O);
     float *gmT = (float *)w; w += dl_align256((size_t)BT * NO * k * 64 * sizeof(float));
     float *gpart = (float *)w;
     if (saved) {  // what the forward of the same x, raw_w and temperature left
         sig = (float *)saved;
         xT = (float *)((char *)saved + prob_sig_bytes(N, k, O));
+        cen = (float *)((char *)xT + prob_xT_bytes(B, I));
     } else {
-        DL_TIMED("prob_sig_table", s, (prob_sig_table<<<dl_ceil_div(WT, 256), 256, 0, s>>>(raw_w, inv_t, sig, N, L, O)));
-        DL_TIMED("prob_to_tiles_x", s, (prob_to_tiles<false><<<dim3(dl_ceil_div(I, 64), BT), 256, 0, s>>>(x, xT, B, I)));
+        prob_launch_to_tiles("prob_to_tiles_x+sig_table", x, xT, B, I, ProbTables{raw_w, nullptr, inv_t, sig, cen, N, L, O}, s);
     }
-    prob_launch_bwd<false>("prob_bwd_t", xT, gy, idx32, sig, gmT, gpart, B, I, N, k, O, tpc, gx != nullptr, s);
+    prob_launch_bwd<false>("prob_bwd_t", xT, gy, idx32, cen, gmT, gpart, B, I, N, k, O, tpc, gx != nullptr, s);
     const ProbReduce R = {gpart, sig, inv_t, graw, N, L, O, chunks};
     prob_launch_gather_and_reduce(gmT, inv_ptr, inv_pos, gx, B, I, N, k, O, BT, R, WT, s);
     return dl_launch_status();
@@ -827,7 +848,7 @@ extern "C" int dl_dwn_layer_fwd(const float *x, const int32_t *idx32, const floa
 extern "C" int dl_dwn_layer_fwd_planes(const void *planes_in, const int32_t *idx32, const float *luts, float *y,
                                        void *planes_out, void *saved, int B, int I, int N, int k, int O, void *stream);
 extern "C" size_t dl_hybrid_saved_bytes(int B, int I, int N, int k, int O) {
-    return hybrid_tiled(B, I, N, k, O) ? prob_xT_bytes(B, I) : 256;
+    return hybrid_tiled(B, I, N, k, O) ? prob_xT_bytes(B, I) + prob_sig_bytes(N, k, O) : 256;
 }
 // the lookup's addresses, which nothing reads afterwards, and its planes or workspace
 extern "C" size_t dl_hybrid_fwd_workspace_bytes(int B, int I, int N, int k, int O) {
@@ -846,10 +867,8 @@ extern "C" int dl_hybrid_layer_fwd(const float *x, const int32_t *idx32, const f
     const size_t addr_bytes = dl_align256(dl_dwn_saved_bytes(B, I, N, k, O));
     char *rest = (char *)ws + addr_bytes;
     if (hybrid_tiled(B, I, N, k, O)) {
-        const int BT = prob_bt(B);
-        DL_TIMED("hybrid_tiles+planes", s,
-                 (prob_to_tiles<true><<<dim3(dl_ceil_div(I, 64), BT), 256, 0, s>>>(
-                     x, (float *)saved, B, I, 1 << 30, nullptr, ProbTemp{1.0f, nullptr}, nullptr, 0, 1, 1, (unsigned long long *)rest)));
+        const ProbTables q{nullptr, luts, ProbTemp{1.0f, nullptr}, nullptr, (float *)((char *)saved + prob_xT_bytes(B, I)), N, 1 << k, O};
+        prob_launch_to_tiles<true>("hybrid_tiles+planes", x, (float *)saved, B, I, q, s, (unsigned long long *)rest);
         const int rc = dl_dwn_layer_fwd_planes(rest, idx32, luts, y, nullptr, ws, B, I, N, k, O, stream);
         if (rc != DL_ERR_UNSUPPORTED) return rc;
     }
@@ -878,15 +897,17 @@ static int hybrid_backward(const float *x, const void *saved, const int32_t *idx
     const int tpc = prob_tiles_per_chunk(B, N, k, O);
     const int chunks = dl_ceil_div(BT, tpc);
     char *w = (char *)ws;
-    const float *xT = (const float *)saved;  // what the forward of the same x left
+    const float *xT = (const float *)saved;  // what the forward of the same x and luts left
     if (!saved) {
-        float *own = (float *)w; w += prob_xT_bytes(B, I);
-        DL_TIMED("prob_to_tiles_x", s, (prob_to_tiles<false><<<dim3(dl_ceil_div(I, 64), BT), 256, 0, s>>>(x, own, B, I)));
+        float *own = (float *)w; w += prob_xT_bytes(B, I) + prob_sig_bytes(N, k, O);
+        prob_launch_to_tiles("prob_to_tiles_x", x, own, B, I,
+                             ProbTables{nullptr, luts, ProbTemp{1.0f, nullptr}, nullptr, (float *)((char *)own + prob_xT_bytes(B, I)), N, L, O}, s);
         xT = own;
     }
+    const float *cen = (const float *)((const char *)xT + prob_xT_bytes(B, I));
     float *gmT = (float *)w; w += dl_align256((size_t)BT * NO * k * 64 * sizeof(float));
     float *gpart = (float *)w;
-    prob_launch_bwd<true>("hybrid_bwd_t", xT, gy, idx32, luts, gmT, gpart, B, I, N, k, O, tpc, gx != nullptr, s);
+    prob_launch_bwd<true>("hybrid_bwd_t", xT, gy, idx32, cen, gmT, gpart, B, I, N, k, O, tpc, gx != nullptr, s);
     const ProbReduce R = {gpart, nullptr, ProbTemp{1.0f, nullptr}, gluts, N, L, O, chunks};
     prob_launch_gather_and_reduce(gmT, inv_ptr, inv_pos, gx, B, I, N, k, O, BT, R, WT, s);
     return dl_launch_status();

@@ -601,6 +601,37 @@ def test_prob_backward_factored_weights(B, N, O, T, k):
     np.testing.assert_allclose(wt.grad.cpu().numpy(), gw, rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("hybrid", [False, True])
+def test_prob_input_gradient_rounds_by_what_the_table_varies(hybrid):
+    """k = 6, uniform x, tables sigmoid(N(0, 1)): values of 0.5 +- 0.2.  Against float64 in the 2-norm: each weight is a product
+    of three factors (3 roundings of 2^-25 rms, 9e-8), sums of eight terms of 0.2 are taken differences of (1e-7), the output
+    is a product and a sum (4e-8): 1.4e-7, limit 2.1e-7.  Sums of the table itself, of 0.5, give 3.0e-7 (hybrid 2.2e-7)."""
+    ops = _ops()
+    B, I, N, k = 1000, 400, 300, 6
+    g = torch.Generator("cuda").manual_seed(k)
+    idx = torch.stack([torch.randperm(I, device="cuda", generator=g)[:k] for _ in range(N)])
+    plan = ops.MappingPlan(idx, I)
+    x = torch.rand(B, I, device="cuda", generator=g)
+    gy = torch.randn(B, N, device="cuda", generator=g)
+    raw = torch.randn(N, 1 << k, device="cuda", generator=g)
+    xt = x.clone().requires_grad_()
+    table = ops.table_sigmoid(raw) if hybrid else raw
+    if hybrid:
+        ops.hybrid_layer(xt, table.view(N, 1, 1 << k).clone().requires_grad_(), plan).backward(gy)
+    else:
+        ops.ProbLayerFunction.apply(xt, raw.view(N, 1 << k, 1).clone().requires_grad_(), plan, 1.0).backward(gy)
+    cols = [x.double()[:, idx[:, j]].requires_grad_() for j in range(k)]
+    v = (table if hybrid else torch.sigmoid(raw.double())).double().expand(B, N, 1 << k)
+    for c in cols:
+        v = v[..., 0::2] * (1 - c.unsqueeze(-1)) + v[..., 1::2] * c.unsqueeze(-1)
+    v.squeeze(-1).backward(gy.double())
+    want = torch.zeros(B, I, dtype=torch.float64, device="cuda")
+    for j, c in enumerate(cols):
+        q = c.detach() * (1 - c.detach())
+        want.index_add_(1, idx[:, j], c.grad * q / (q + 1e-8) if hybrid else c.grad)
+    assert float((xt.grad.double() - want).norm()) <= 2.1e-7 * float(want.norm())
+
+
 @pytest.mark.parametrize("k", [1, 4, 6])
 @pytest.mark.parametrize("hybrid", [False, True])
 @pytest.mark.parametrize("B,N,O", [(63, 1, 1), (5000, 1, 1),    # one column
