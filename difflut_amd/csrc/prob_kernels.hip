@@ -219,11 +219,6 @@ __global__ __launch_bounds__(64 * PROB_FW) void prob_fwd_t(const float *__restri
     }
 }
 
-// 1 / d to about half a unit of the last place: the hardware reciprocal and one Newton step
-__device__ __forceinline__ float prob_rcp(float d) {
-    const float r = __builtin_amdgcn_rcpf(d);
-    return fmaf(r, fmaf(-d, r, 1.0f), r);
-}
 // u[a] = product over the inputs j of (x_j if bit j of a is set, else 1 - x_j)
 template <int KH>
 __device__ __forceinline__ void prob_products(const float *x, const float *om, float (&u)[1 << KH]) {
@@ -362,7 +357,7 @@ __global__ __launch_bounds__(64 * W) void prob_bwd_t(const float *__restrict__ x
 #pragma unroll
                 for (int j = 0; j < K; ++j) {
                     const float q = xs[j] * om[j];
-                    dx[j] *= q * prob_rcp(q + PROB_HYBRID_EPS);
+                    dx[j] = dx[j] * q / (q + PROB_HYBRID_EPS);
                 }
             }
             if (live) {

@@ -124,6 +124,23 @@ def test_hybrid_forward_that_keeps_the_tiles_is_the_one_that_does_not(shape, ali
         assert torch.equal(kept, apart)
 
 
+def test_hybrid_gradient_factor_over_the_range_of_x():
+    """One input per node: the input gradient is gy (T1 - T0) q / (q + 1e-8), q = x (1 - x), exactly rounded operations (the
+    sum, the product with q, the quotient and the product with gy: 4 * 2^-24), for x at which q is tiny, ordinary or near float32's largest, and 0 at 0 and 1."""
+    ops = _ops()
+    x = torch.tensor([0.0, 1.0, 1e-30, 1e-12, 1e-9, 1e-8, 3e-8, 1e-4, 0.3, 0.5, 0.999, 1 - 2.0 ** -24, 1.0 + 2.0 ** -23, -1e-9,
+                      -3e-7, -2.5, 17.0, 1e6, -1e10, 1e15, 1.2e19, -1.3e19], device=DEV)
+    B = x.numel()
+    plan = ops.MappingPlan(torch.zeros(1, 1, dtype=torch.int32, device=DEV), 1)
+    table = torch.tensor([[[0.25, 0.75]]], device=DEV)
+    gy = torch.linspace(0.5, 1.5, B, device=DEV)
+    xt = x.view(B, 1).clone().requires_grad_()
+    ops.hybrid_layer(xt, table.clone().requires_grad_(), plan).backward(gy.view(B, 1))
+    q = (x * (1.0 - x)).double()  # as fp32 rounds it
+    want = gy.double() * 0.5 * q / (q + float(np.float32(1e-8)))
+    np.testing.assert_allclose(xt.grad.view(-1).double().cpu().numpy(), want.cpu().numpy(), rtol=4 * 2.0 ** -24, atol=0)
+
+
 @pytest.mark.parametrize("shape", SHAPES)
 def test_hybrid_layer_forward_backward(shape):
     B, I, N, k, O = shape
