@@ -84,6 +84,8 @@ def _node_getter(nodes):
 class ParameterBank:
     """The parameter `name` of N nodes as one leaf tensor [N, *shape]."""
 
+    _node = None  # of a bank that was copied, until it is asked (its nodes may not be whole yet when it is restored)
+
     def __init__(self, nodes, name):
         self.nodes, self.name = nodes, name
         self.flat = None
@@ -111,11 +113,13 @@ class ParameterBank:
         self._stale = False
 
     def __getstate__(self):
-        return {k: v for k, v in self.__dict__.items() if k != "_node"}  # tie() makes it again
+        return {k: v for k, v in self.__dict__.items() if k != "_node"}  # tied() and tie() make it again
 
     def tied(self):
         if self._stale or len(self.nodes) != self._count:
             return False
+        if self._node is None:
+            self._node = _node_getter(self.nodes)
         first = self._node(0)._parameters[self.name]
         last = self._node(self._count - 1)._parameters[self.name]
         base = self.flat.data_ptr()
@@ -136,6 +140,7 @@ class ScalarBank:
     `abs_max()` (the largest magnitude, which selects the form of the EFD coefficient table): read back when the
     bank's version counter changes or after `invalidate()`."""
 
+    _node = None  # as for the ParameterBank
     _PROBES = 16  # nodes checked per call beyond the first and the last when the layer is large
 
     def __init__(self, nodes, name):
@@ -160,10 +165,7 @@ class ScalarBank:
         self._stale, self._key = False, None
 
     def __getstate__(self):
-        return {k: v for k, v in self.__dict__.items() if k != "_node"}  # tie() makes it again
-
-    def _is_view(self, row):
-        return self._node(row)._buffers[self.name] is self._views[row]
+        return {k: v for k, v in self.__dict__.items() if k != "_node"}  # tied() and tie() make it again
 
     def tied(self):
         """Every node's buffer is still the view handed out by tie().  All nodes are checked on small layers; on large
@@ -179,6 +181,8 @@ class ScalarBank:
         else:
             rows = [0, n - 1] + [(self._probe + i) % n for i in range(self._PROBES)]
             self._probe = (self._probe + self._PROBES) % n
+        if self._node is None:
+            self._node = _node_getter(self.nodes)
         node, name, views = self._node, self.name, self._views
         for row in rows:
             if node(row)._buffers[name] is not views[row]:

@@ -348,6 +348,22 @@ def test_banks_notice_a_deleted_and_an_appended_node():
     assert float(layer.efd_scalars()[0][11]) == 0.125
 
 
+@pytest.mark.parametrize("how", ["copy", "deepcopy", "pickle"])
+def test_a_copied_bank_answers_by_itself(how):
+    """A bank that is copied without its layer (in a user's own object, or while a layer is being put together again) can be
+    asked before it is tied: a deep copy's nodes hold plain parameters, a shallow one's belong to the original."""
+    import copy
+    import pickle
+    layer = _small_dwn_layer()
+    twin = {"copy": copy.copy, "deepcopy": copy.deepcopy, "pickle": lambda b: pickle.loads(pickle.dumps(b))}[how]
+    for bank in (layer._banks["luts"], layer._scalars["alpha"]):
+        values = bank.flat.detach().clone()
+        other = twin(bank)
+        other.tied()
+        assert torch.equal(other.tensor().detach(), values)
+        assert other.tied()
+
+
 def test_scalar_buffers_are_banked_and_differences_are_seen():
     layer = _small_dwn_layer()
     alpha, beta = layer._scalars["alpha"], layer._scalars["beta"]
