@@ -873,7 +873,8 @@ extern "C" int dl_hybrid_layer_fwd(const float *x, const int32_t *idx32, const f
 static int hybrid_backward(const float *x, const void *saved, const int32_t *idx32, const int32_t *inv_ptr,
                            const int32_t *inv_pos, const float *luts, const float *gy, float *gx, float *gluts, void *ws,
                            size_t ws_bytes, size_t ws_needed, int B, int I, int N, int k, int O, void *stream) {
-    if (!x || !idx32 || !luts || !gy || !gluts) return DL_ERR_NULL;
+    if (!idx32 || !luts || !gy || !gluts) return DL_ERR_NULL;
+    if (!x && !(saved && hybrid_tiled(B, I, N, k, O))) return DL_ERR_NULL;
     if (gx && (!inv_ptr || !inv_pos)) return DL_ERR_NULL;
     int rc = prob_check(B, I, N, k, O);
     if (rc) return rc;

@@ -521,7 +521,8 @@ class HybridLayerFunction(torch.autograd.Function):
                                               tiles.numel(), nat.ptr(ws), ws.numel(), *dims, nat.stream()))
         else:
             y, _, dims = _dwn_lookup(x, luts, plan)
-        ctx.save_for_backward(x, luts, tiles)
+        # the backward reads x itself only where it was not re-tiled
+        ctx.save_for_backward(None if tiles is not None and tiles.numel() > 256 else x, luts, tiles)
         ctx.plan, ctx.dims = plan, dims
         return y
 

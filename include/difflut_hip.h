@@ -264,9 +264,10 @@ int dl_hybrid_layer_bwd(const float *x, const int32_t *idx32,
                         const float *luts, const float *gy, float *gx, float *gluts,
                         void *ws, size_t ws_bytes,
                         int B, int I, int N, int k, int O, void *stream);
-/* The same pair for a forward that a backward will follow: the forward leaves x re-tiled in `saved` (dl_hybrid_saved_bytes:
- * [ceil(B/64)][I][64] fp32) in the pass that takes the lookup's bit-planes, the backward of the same x reads it there.  y as
- * dl_dwn_layer_fwd writes it.  x is read by the backward only where the tiled path does not apply (k > DL_MAX_FAST_K). */
+/* The same pair for a forward that a backward will follow: the forward leaves x re-tiled and the tables less a value per
+ * column in `saved` (dl_hybrid_saved_bytes: [ceil(B/64)][I][64] and [N*O][2^k] fp32) in the pass that takes the lookup's bit-planes, the backward of the same x reads it there.  y as
+ * dl_dwn_layer_fwd writes it.  x is read by the backward only where the tiled path does not apply (dl_hybrid_saved_bytes reports 256) and may be
+ * null otherwise. */
 size_t dl_hybrid_saved_bytes(int B, int I, int N, int k, int O);
 size_t dl_hybrid_fwd_workspace_bytes(int B, int I, int N, int k, int O);
 size_t dl_hybrid_bwd_saved_workspace_bytes(int B, int I, int N, int k, int O);

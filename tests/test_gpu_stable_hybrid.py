@@ -141,6 +141,23 @@ def test_hybrid_gradient_factor_over_the_range_of_x():
     np.testing.assert_allclose(xt.grad.view(-1).double().cpu().numpy(), want.cpu().numpy(), rtol=4 * 2.0 ** -24, atol=0)
 
 
+def test_hybrid_forward_keeps_one_copy_of_x():
+    """Between forward and backward a hybrid layer holds y, x re-tiled and the tables' copy, not x itself as well."""
+    ops = _ops()
+    B, I, N, k = 256, 4096, 64, 6
+    g = torch.Generator(DEV).manual_seed(1)
+    plan = ops.MappingPlan(torch.randint(0, I, (N, k), device=DEV, generator=g), I)
+    table = torch.rand(N, 1, 1 << k, device=DEV, generator=g).requires_grad_()
+    leaf = torch.rand(B, I, device=DEV, generator=g).requires_grad_()
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    y = ops.hybrid_layer(leaf * 1.0, table, plan)  # an input that nobody else holds
+    held = torch.cuda.memory_allocated() - before
+    assert held < 4 * (1.25 * B * I + B * N) + 4 * 2 * N * 64
+    y.sum().backward()
+    assert torch.isfinite(leaf.grad).all()
+
+
 @pytest.mark.parametrize("shape", SHAPES)
 def test_hybrid_layer_forward_backward(shape):
     B, I, N, k, O = shape
