@@ -34,6 +34,12 @@ def _per_node(values, N, device):
     return values.reshape(-1).expand(N).contiguous()
 
 
+def _backward_reads_x(N, k, O):
+    """Whether the DWN backward needs x: not where the forward leaves the address of every node and row (k <= 6 and, within
+    the bounds of the library's dwn_wide, 7 and 8)."""
+    return k > 8 or (k > FAST_K and not (N < 1 << 23 and N * O * (4 << k) < 0x7fffffff))
+
+
 class MappingPlan:
     """Device-side form of an index table idx [N,k] over I inputs.
 
@@ -175,7 +181,7 @@ class DWNLayerFunction(torch.autograd.Function):
             ctx.ab = (alpha, beta, float(beta_abs_max))
         else:
             ctx.ab = (float(alpha), float(beta))
-        ctx.save_for_backward(luts, saved, x if k > FAST_K else None)
+        ctx.save_for_backward(luts, saved, x if _backward_reads_x(N, k, O) else None)
         ctx.plan, ctx.dims = plan, dims
         return y
 
@@ -480,7 +486,7 @@ class DWNStableLayerFunction(torch.autograd.Function):
         if scale.numel() != luts.shape[0]:
             raise RuntimeError(f"gradient_scale has {scale.numel()} entries for {luts.shape[0]} nodes")
         y, saved, dims = _dwn_lookup(x, luts, plan)
-        ctx.save_for_backward(luts, saved, scale, x if plan.k > FAST_K else None)
+        ctx.save_for_backward(luts, saved, scale, x if _backward_reads_x(*dims[2:]) else None)
         ctx.plan, ctx.dims = plan, dims
         return y
 

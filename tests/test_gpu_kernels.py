@@ -400,6 +400,27 @@ def test_dwn_tables_of_more_than_one_register(B, I, N, O, k):
     assert torch.equal(got[0], got[1])
 
 
+@pytest.mark.parametrize("k", [6, 7, 8])
+@pytest.mark.parametrize("stable", [False, True])
+def test_dwn_forward_keeps_addresses_instead_of_x(k, stable):
+    """Between forward and backward a layer whose backward reads the saved addresses does not hold x."""
+    ops = _ops()
+    B, I, N = 256, 4096, 32
+    g = torch.Generator("cuda").manual_seed(k)
+    plan = ops.MappingPlan(torch.randint(0, I, (N, k), device="cuda", generator=g), I)
+    luts = torch.rand(N, 1, 1 << k, device="cuda", generator=g).requires_grad_()
+    leaf = torch.rand(B, I, device="cuda", generator=g).requires_grad_()
+    scale = torch.ones(N, device="cuda")
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    x = leaf * 1.0
+    y = ops.dwn_stable_layer(x, luts, scale, plan) if stable else ops.DWNLayerFunction.apply(x, luts, plan, 0.3, 1.0 / 3.0)
+    del x
+    assert torch.cuda.memory_allocated() - before < 2 * B * I
+    y.sum().backward()
+    assert torch.isfinite(leaf.grad).all() and leaf.grad.abs().max() > 0
+
+
 def test_dwn_no_input_grad_and_unused_inputs():
     ops = _ops()
     B, I, N, k, O = 40, 50, 3, 2, 1  # 44 of the 50 inputs feed no node: their gradient must be 0
