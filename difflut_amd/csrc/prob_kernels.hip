@@ -702,13 +702,22 @@ extern "C" size_t dl_prob_saved_bytes(int B, int I, int N, int k, int O) {
     if (B <= 0 || I <= 0 || N <= 0 || k <= 0 || O <= 0 || !prob_fast(I, N, k, O)) return 256;
     return 2 * prob_sig_bytes(N, k, O) + prob_xT_bytes(B, I);
 }
-// (with room for one more [B, N O] array than the kernels use: the size does not shrink below what callers sized by before)
-extern "C" size_t dl_prob_bwd_workspace_bytes(int B, int I, int N, int k, int O) {
-    if (B <= 0 || I <= 0 || N <= 0 || k <= 0 || O <= 0 || !prob_fast(I, N, k, O)) return 256;
+// dL/d(mapped inputs) and the partial table gradients
+static inline size_t prob_gm_bytes(int B, int N, int k, int O) {
     const size_t BT = prob_bt(B);
     const int chunks = dl_ceil_div(prob_bt(B), prob_tiles_per_chunk(B, N, k, O));
-    return prob_sig_bytes(N, k, O) + prob_xT_bytes(B, I) + dl_align256(BT * N * O * 64 * sizeof(float)) +
-           dl_align256(BT * N * O * k * 64 * sizeof(float)) + dl_align256((size_t)chunks * N * O * ((size_t)1 << k) * sizeof(float));
+    return dl_align256(BT * N * O * k * 64 * sizeof(float)) + dl_align256((size_t)chunks * N * O * ((size_t)1 << k) * sizeof(float));
+}
+// of a backward that is handed what the forward left
+extern "C" size_t dl_prob_bwd_saved_workspace_bytes(int B, int I, int N, int k, int O) {
+    if (B <= 0 || I <= 0 || N <= 0 || k <= 0 || O <= 0 || !prob_fast(I, N, k, O)) return 256;
+    return prob_gm_bytes(B, N, k, O);
+}
+// of one that makes it itself, with room for a whole [B, N O] array in the place of the table less a value per column
+extern "C" size_t dl_prob_bwd_workspace_bytes(int B, int I, int N, int k, int O) {
+    if (B <= 0 || I <= 0 || N <= 0 || k <= 0 || O <= 0 || !prob_fast(I, N, k, O)) return 256;
+    return prob_sig_bytes(N, k, O) + prob_xT_bytes(B, I) + dl_align256((size_t)prob_bt(B) * N * O * 64 * sizeof(float)) +
+           prob_gm_bytes(B, N, k, O);
 }
 
 #define PROB_DISPATCH(K, CALL) \
@@ -786,23 +795,18 @@ static int prob_backward(const float *x, const void *saved, const int32_t *idx32
         return dl_launch_status();
     }
     if (!ws) return DL_ERR_NULL;
-    if (ws_bytes < dl_prob_bwd_workspace_bytes(B, I, N, k, O)) return DL_ERR_WORKSPACE;
+    if (ws_bytes < (saved ? prob_gm_bytes(B, N, k, O) : dl_prob_bwd_workspace_bytes(B, I, N, k, O))) return DL_ERR_WORKSPACE;
     const int BT = prob_bt(B), L = 1 << k, NO = N * O;
     const int tpc = prob_tiles_per_chunk(B, N, k, O);
     const int chunks = dl_ceil_div(BT, tpc);
     char *w = (char *)ws;
-    float *sig = (float *)w; w += prob_sig_bytes(N, k, O);
-    float *xT = (float *)w; w += prob_xT_bytes(B, I);
-    float *cen = (float *)w; w += prob_sig_bytes(N, k, O);
+    float *sig = (float *)saved;  // what the forward of the same x, raw_w and temperature left
+    if (!saved) { sig = (float *)w; w += 2 * prob_sig_bytes(N, k, O) + prob_xT_bytes(B, I); }
+    float *xT = (float *)((char *)sig + prob_sig_bytes(N, k, O)), *cen = (float *)((char *)xT + prob_xT_bytes(B, I));
     float *gmT = (float *)w; w += dl_align256((size_t)BT * NO * k * 64 * sizeof(float));
     float *gpart = (float *)w;
-    if (saved) {  // what the forward of the same x, raw_w and temperature left
-        sig = (float *)saved;
-        xT = (float *)((char *)saved + prob_sig_bytes(N, k, O));
-        cen = (float *)((char *)xT + prob_xT_bytes(B, I));
-    } else {
+    if (!saved)
         prob_launch_to_tiles("prob_to_tiles_x+sig_table", x, xT, B, I, ProbTables{raw_w, nullptr, inv_t, sig, cen, N, L, O}, s);
-    }
     prob_launch_bwd<false>("prob_bwd_t", xT, gy, idx32, cen, gmT, gpart, B, I, N, k, O, tpc, gx != nullptr, s);
     const ProbReduce R = {gpart, sig, inv_t, graw, N, L, O, chunks};
     prob_launch_gather_and_reduce(gmT, inv_ptr, inv_pos, gx, B, I, N, k, O, BT, R, WT, s);
@@ -916,10 +920,7 @@ extern "C" int dl_hybrid_layer_bwd(const float *x, const int32_t *idx32, const i
                            dl_hybrid_bwd_workspace_bytes(B, I, N, k, O), B, I, N, k, O, stream);
 }
 extern "C" size_t dl_hybrid_bwd_saved_workspace_bytes(int B, int I, int N, int k, int O) {
-    if (!hybrid_tiled(B, I, N, k, O)) return 256;
-    const size_t BT = prob_bt(B);
-    const int chunks = dl_ceil_div(prob_bt(B), prob_tiles_per_chunk(B, N, k, O));
-    return dl_align256(BT * N * O * k * 64 * sizeof(float)) + dl_align256((size_t)chunks * N * O * ((size_t)1 << k) * sizeof(float));
+    return hybrid_tiled(B, I, N, k, O) ? prob_gm_bytes(B, N, k, O) : 256;
 }
 extern "C" int dl_hybrid_layer_bwd_saved(const float *x, const void *saved, const int32_t *idx32, const int32_t *inv_ptr,
                                          const int32_t *inv_pos, const float *luts, const float *gy, float *gx, float *gluts,

@@ -599,7 +599,7 @@ class ProbLayerFunction(torch.autograd.Function):
         B, I = x.shape
         gx = torch.empty((B, I), dtype=torch.float32, device=gy.device) if ctx.needs_input_grad[0] else None
         graw = torch.empty_like(raw)
-        ws = _bytes(lib.dl_prob_bwd_workspace_bytes(*ctx.dims), gy.device)
+        ws = _bytes(lib.dl_prob_bwd_saved_workspace_bytes(*ctx.dims), gy.device)
         if T is None:
             nat.check(lib.dl_prob_layer_bwd(nat.ptr(x), nat.ptr(saved), nat.ptr(plan.idx32), nat.ptr(plan.inv_ptr),
                                             nat.ptr(plan.inv_pos),

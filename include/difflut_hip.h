@@ -292,11 +292,12 @@ int dl_hybrid_layer_bwd_saved(const float *x, const void *saved, const int32_t *
  * ------------------------------------------------------------------------ */
 size_t dl_prob_saved_bytes(int B, int I, int N, int k, int O);
 size_t dl_prob_bwd_workspace_bytes(int B, int I, int N, int k, int O);
-/* `saved` (dl_prob_saved_bytes) receives the sigmoid table and the re-tiled input. */
+size_t dl_prob_bwd_saved_workspace_bytes(int B, int I, int N, int k, int O); /* enough for a backward that is given `saved` */
+/* `saved` (dl_prob_saved_bytes) receives the sigmoid table, the re-tiled input and the table less a value per column. */
 int dl_prob_layer_fwd(const float *x, const int32_t *idx32, const float *raw_w, float temperature,
                       float *y, void *saved, size_t saved_bytes,
                       int B, int I, int N, int k, int O, void *stream);
-/* `saved` may be null: then both are rebuilt from x, raw_w and temperature. */
+/* `saved` may be null: then they are rebuilt from x, raw_w and temperature. */
 int dl_prob_layer_bwd(const float *x, const void *saved, const int32_t *idx32,
                       const int32_t *inv_ptr, const int32_t *inv_pos,
                       const float *raw_w, float temperature, const float *gy,

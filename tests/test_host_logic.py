@@ -267,6 +267,21 @@ def test_argument_checks_of_the_later_entry_points_need_no_gpu():
     assert lib.dl_hybrid_bwd_workspace_bytes(*dims) >= 4096 * (16384 + 8192 + 6 * 8192) * 4
 
 
+@pytest.mark.parametrize("dims", [(4096, 16384, 8192, 6, 1), (130, 40, 17, 3, 2), (1, 1, 1, 1, 1)])
+def test_backward_given_what_the_forward_left_asks_for_its_own_arrays_only(dims):
+    """With `saved`, a probabilistic or hybrid backward writes dL/d(mapped inputs) and partial table gradients, nothing else
+    (a [B, N O] array more is 134 MB at 4096 x 8192)."""
+    from difflut_amd import _native as nat
+    lib = nat.lib()
+    B, I, N, k, O = dims
+    tiles = (B + 63) // 64
+    need = tiles * N * O * k * 64 * 4
+    for size in (lib.dl_prob_bwd_saved_workspace_bytes(*dims), lib.dl_hybrid_bwd_saved_workspace_bytes(*dims)):
+        assert need + (N * O * 4 << k) <= size <= need + tiles * (N * O * 4 << k) + 512
+        assert size + 256 <= lib.dl_prob_bwd_workspace_bytes(*dims)
+    assert lib.dl_prob_bwd_saved_workspace_bytes(4096, 16384, 8192, 6, 1) < 4096 * 8192 * 6 * 4 + 40e6
+
+
 @pytest.mark.parametrize("B,N,k", [(147456, 32, 6), (147456, 32, 4), (65536, 1, 6), (65536, 64, 4), (65536, 8, 6)])
 def test_narrow_layers_are_cut_into_chunks_that_fill_the_card(B, N, k):
     """The probabilistic backward of few columns over many rows: what its workspace holds of partial table gradients says into
