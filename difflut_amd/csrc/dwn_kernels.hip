@@ -954,6 +954,7 @@ __global__ __launch_bounds__(256) void dwn_bwd_gx(const float *__restrict__ gyT,
 // around it would keep the compiler from requesting the step's loads together.
 #define DWN_LT 4  // batch tiles per wavefront
 #define DWN_LE 4  // entries per step
+#define DWN_LONG_BLOCKS 900 // see dwn_launch_gx
 template <int K>
 __global__ __launch_bounds__(256) void dwn_bwd_gx_long(const float *__restrict__ gyT, const uint8_t *__restrict__ addrT,
                                                         const float *__restrict__ D, const int *__restrict__ inv_ptr,
@@ -1615,14 +1616,15 @@ static void dwn_launch_gx(const float *gyT, const uint8_t *addrT, const float *D
     // mapping) want fewer inputs per wavefront: more, shorter and evenly filled blocks.  Measured at B = 4096, k = 6:
     // lists of 3 - 16 inputs per wavefront is best (169 vs 221 us); 7.7 - 4 inputs (67 vs 73 us); 15 - 4 (134 vs
     // 179 us); 31 - 4 (368 vs 442 us); 69 with tile-major output - 1 (249 vs 265 vs 375 us).
-    // There four batch tiles per wavefront (dwn_bwd_gx_long) once there are blocks enough. By rows (100
-    // columns, 1152 nodes), one tile / four, us: 147456 rows 608 / 463, 36864 157 / 127, 23040 (2250 blocks) 103 / 88.  The gain
-    // shrinks towards the line; a slower form of the kernel lost below it (18432 rows 81.5 / 83.5, 9216 46 / 50, 4608 27 / 40).
+    // There four batch tiles per wavefront (dwn_bwd_gx_long) once there are blocks enough.  One tile / four, us, k = 6, by
+    // blocks of the latter: lists of 69 (100 columns, 1152 nodes) 14400 608 / 463, 3600 157 / 122, 1800 82 / 70, 1300 63 / 58,
+    // 900 46 / 42, 675 38 / 40, 450 27 / 35; lists of 192 (9 columns) 900 90.8 / 90.9, 700 78 / 80, 450 54 / 73; lists of 276
+    // 900 149 / 141, 460 87 / 104; lists of 92 680 48 / 46, 440 34 / 40.  From 900 on it loses nowhere.
     if (O == 1 && sform && out_tiled && (long long)N * K >= 32LL * I &&
-        (long long)dl_ceil_div(I, 4) * dl_ceil_div(BT, DWN_LT) >= 2048) {
+        (long long)dl_ceil_div(I, 4) * dl_ceil_div(BT, DWN_LT) >= DWN_LONG_BLOCKS) {
         const int grid_l = dl_xcd_grid(dl_ceil_div(I, 4), dl_ceil_div(BT, DWN_LT));
-        DL_TIMED("dwn_bwd_gx", s, (dwn_bwd_gx_long<K><<<grid_l + rb, 256, 0, s>>>(gyT, addrT, D, inv_ptr, inv_pos, gx, I, N, BT,
-                                                                                   grid_l, red)));
+        DL_TIMED("dwn_bwd_gx_long", s, (dwn_bwd_gx_long<K><<<grid_l + rb, 256, 0, s>>>(gyT, addrT, D, inv_ptr, inv_pos, gx, I, N, BT,
+                                                                                        grid_l, red)));
         return;
     }
     if (O == 1 && sform && out_tiled && (long long)N * K >= 32LL * I) {

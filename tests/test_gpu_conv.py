@@ -201,24 +201,37 @@ def test_grouped_connections_cover_every_channel(seed):
     assert y.shape == (2, 16, 6, 6) and torch.isfinite(y).all()
 
 
-def test_conv_gather_of_four_batch_tiles_equals_that_of_one():
-    """29 images of 28 x 28 are 261 batch tiles of patches and 125 columns, 66 x 32 blocks of the gather that takes four tiles
-    per wavefront: the last group has one tile, the last block one column.  15 + 14 images stay with one tile:
-    same terms in the same order, so the same bits."""
+@pytest.mark.parametrize("images,columns,field,channels,k", [(29, 5, 5, 32, 6),   # 261 batch tiles, 125 columns: a last group of one
+                                                             (29, 5, 5, 128, 4),  # as many, lists of 65
+                                                             (30, 5, 5, 32, 6),   # 270 tiles: a last group of two
+                                                             (115, 1, 3, 8, 6)])  # 1215 tiles, 9 columns: three; a block of one column
+def test_conv_gather_of_four_batch_tiles_equals_that_of_one(images, columns, field, channels, k):
+    """The gather that takes four batch tiles per wavefront against the one that takes one, which runs where there are too few
+    tiles for the other: same terms in the same order, so the same bits.  Which of them ran is read from the library's record."""
+    from difflut_amd import _native as nat
     torch.manual_seed(21)
-    layer = _build("dwn", 2, 5, 32, 5, 1, 0, 32).train()
-    assert layer.bank_parameters()[0].shape[0] == 1152
-    x = (torch.rand(29, 5, 28, 28, device=DEV) < 0.5).float()
-    gy = torch.randn(29, 32, 24, 24, device=DEV)
+    layer = _build("dwn", 2, columns, channels, field, 1, 0, 32, n=k).train()
+    side = 28 - field + 1
+    x = (torch.rand(images, columns, 28, 28, device=DEV) < 0.5).float()
+    gy = torch.randn(images, channels, side, side, device=DEV)
 
     def gradient(rows):
         part = x[rows].clone().requires_grad_()
-        layer(part).backward(gy[rows])
-        return part.grad
+        nat.profile_read()
+        nat.profile_enable(True)
+        try:
+            layer(part).backward(gy[rows])
+            names = {name for name, _ in nat.profile_read()}
+        finally:
+            nat.profile_enable(False)
+        return part.grad, "dwn_bwd_gx_long" in names
 
-    whole = gradient(slice(0, 29))
-    assert whole.abs().max() > 0
-    assert torch.equal(whole, torch.cat([gradient(slice(0, 15)), gradient(slice(15, 29))]))
+    whole, long_list = gradient(slice(0, images))
+    assert long_list and whole.abs().max() > 0
+    step = 5  # images: at most 53 tiles, fewer blocks than the line for every width here
+    parts = [gradient(slice(i, min(i + step, images))) for i in range(0, images, step)]
+    assert not any(long_list for _, long_list in parts)
+    assert torch.equal(whole, torch.cat([part for part, _ in parts]))
 
 
 def test_conv_bank_parameters_train_in_place():
