@@ -308,7 +308,7 @@ struct SoftmapArgs {
 // Loads that bypass the registers: lane l's 16 bytes at base + voff land at LDS address lds + 16 l.  The compiler does not
 // count them; the stages below wait for them by number (they complete in order).
 __device__ __forceinline__ void softmap_to_lds(unsigned lds, const char *base, unsigned voff) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base) : "memory", "m0");
 }
 // all of this wavefront's loads but the last N have landed, its LDS reads are done, and every wavefront has got here
 template <int N>
@@ -343,6 +343,8 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
     constexpr int NA = NP * KB * (TR / 64) / 4, NB = NP * KB * (TC / 64) / 4;  // loads per wavefront and stage
     static_assert(NP * KB * (TR / 64) % 4 == 0 && NP * KB * (TC / 64) % 4 == 0, "whole loads per wavefront");
     extern __shared__ __align__(16) char lds[];
+    typedef __attribute__((address_space(3))) char lds_char;
+    const unsigned lds_base = (unsigned)(uintptr_t)(lds_char *)lds;  // what softmap_to_lds counts from
     int inner, outer;
     if (!dl_xcd_map(g.inner_count, g.outer_count, inner, outer)) return;
     const int rt = MODE == 2 ? outer : inner;
@@ -360,7 +362,7 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
     const unsigned b_voff = MODE == 0 ? ((unsigned)(lane / KC) * g.ldb + ((lane % KC) ^ (4 * ((KC == 16 ? lane / 16 : 2 * (wave & 1) + lane / 32) & 3)))) * SM_UNIT
                                       : lane * SM_UNIT;
     auto issue = [&](int st, int buf) __attribute__((always_inline)) {
-        const unsigned base = buf * STAGE;
+        const unsigned base = lds_base + buf * STAGE;
         const int k8 = (s_begin + st) * KB;
 #pragma unroll
         for (int j = 0; j < NA; ++j) {
