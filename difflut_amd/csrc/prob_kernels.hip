@@ -69,7 +69,7 @@ __device__ __forceinline__ void prob_table_element(const ProbTables &q, long lon
     };
     const float v = value(a);
     if (q.sig) q.sig[e] = v;
-    q.cen[e] = v - (q.L > 2 ? 0.5f * (value(0) + value(q.L - 1)) : value(0));  // (k = 1: the one difference itself)
+    q.cen[e] = v - (q.L > 2 ? 0.5f * value(0) + 0.5f * value(q.L - 1) : value(0));  // (k = 1: the one difference itself)
 }
 
 // ceil(C / 64) * tiles blocks of 256 threads, and behind them those that build the tables of `q` (prob_table_blocks): the

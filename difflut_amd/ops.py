@@ -635,7 +635,8 @@ def prob_layer_eval(x, raw, plan, temperature):
 
 # ----------------------------------------------------------------------------- Learnable mapping
 class SoftMapFunction(torch.autograd.Function):
-    """m = x @ softmax(W / tau, dim=-1).T without materialising the softmax."""
+    """m = x @ softmax(W / tau, dim=-1).T.  The softmax numerators are kept as bf16 planes from forward to backward: 6 bytes per
+    entry of W with fp32 operands (precision 0), 2 with bf16."""
 
     @staticmethod
     def forward(ctx, x, W, tau, precision):
