@@ -211,6 +211,8 @@ def test_conv_gather_of_four_batch_tiles_equals_that_of_one(images, columns, fie
     from difflut_amd import _native as nat
     torch.manual_seed(21)
     layer = _build("dwn", 2, columns, channels, field, 1, 0, 32, n=k).train()
+    nodes = layer.bank_parameters()[0].shape[0]
+    assert nodes == channels * k * k and nodes * k >= 32 * columns * field * field  # long lists
     side = 28 - field + 1
     x = (torch.rand(images, columns, 28, 28, device=DEV) < 0.5).float()
     gy = torch.randn(images, channels, side, side, device=DEV)
