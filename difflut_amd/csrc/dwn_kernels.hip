@@ -30,6 +30,7 @@
 #include <mutex>
 #include <type_traits>
 #include "dwn_generic.h"
+#include "dwn_pair.h"
 
 typedef unsigned long long u64;
 
@@ -945,12 +946,20 @@ __global__ __launch_bounds__(256) void dwn_bwd_gx(const float *__restrict__ gyT,
     }
 }
 
+// D-form rows of two entries in one register: lanes 0-31 the even entry's, lanes 32-63 the odd one's
+__device__ __forceinline__ float dwn_walk_diff_packed(float coef, unsigned a, int j, int odd) {
+    const unsigned low = (1u << j) - 1u;
+    const unsigned ap = (a & low) | ((a >> 1) & ~low);  // the address without its bit j
+    return __int_as_float(__builtin_amdgcn_ds_bpermute((int)((ap << 2) | (odd ? 128u : 0u)), __float_as_int(coef)));
+}
+
 // ---------------------------------------------------------------------------------
 // bwd_gx_long: the same sums, tile-major, for inputs with long CSR lists (the patch columns of a convolution, 69 entries each).
 // A wavefront keeps one input and takes DWN_LT batch tiles at once: an entry is decoded and its coefficient row loaded once
 // for all of them, and the address and gradient rows of four entries x four tiles are in flight together.  Bound by those
 // rows, 320 bytes per entry and tile from the L2.  First level of convolutional trees (100 columns, 1152 nodes, 147456
-// rows): 608 -> 463 us a launch, the layer's training step 1107 -> 960.  A lane past the end of the list loads entry 0's rows and adds nothing: a branch
+// rows): 608 -> 463 us a launch with one tile -> four and the S form's two lane reads per entry and tile, 431 with the D form's one
+// (larger batches take most of their tiles through dwn_bwd_pair_gx).  A lane past the end of the list loads entry 0's rows and adds nothing: a branch
 // around it would keep the compiler from requesting the step's loads together.
 #define DWN_LT 4  // batch tiles per wavefront
 #define DWN_LE 4  // entries per step
@@ -961,7 +970,7 @@ __global__ __launch_bounds__(256) void dwn_bwd_gx_long(const float *__restrict__
                                                         const int *__restrict__ inv_pos, float *__restrict__ gx, int I,
                                                         int N, int BT, int gather_blocks, DwnReduce red) {
     if ((int)blockIdx.x >= gather_blocks) return dwn_reduce_block(red, (int)blockIdx.x - gather_blocks);
-    constexpr int L = 1 << K;
+    constexpr int Lh = 1 << (K - 1);
     int slab, group;
     if (!dl_xcd_map((I + 3) / 4, (BT + DWN_LT - 1) / DWN_LT, slab, group)) return;
     const int lane = threadIdx.x & 63;
@@ -998,14 +1007,13 @@ __global__ __launch_bounds__(256) void dwn_bwd_gx_long(const float *__restrict__
                     a[q][u] = addr_t[u][(size_t)rn * 64 + lane];
                     g[q][u] = gy_t[u][(size_t)rn * 64 + lane];
                 }
-                coef[q] = D[(size_t)rn * L + (lane & (L - 1))];
+                coef[q] = D[((size_t)rn * K + rj[q]) * Lh + (lane & (Lh - 1))];
             }
 #pragma unroll
             for (int q = 0; q < DWN_LE; ++q)
 #pragma unroll
                 for (int u = 0; u < DWN_LT; ++u) {
-                    const float term = g[q][u] * (dl_lane_read(coef[q], (int)(a[q][u] | (1u << rj[q]))) -
-                                                  dl_lane_read(coef[q], (int)(a[q][u] & ~(1u << rj[q]))));
+                    const float term = g[q][u] * dwn_walk_diff_packed(coef[q], a[q][u], rj[q], 0);
                     acc[u] = s0 + q < cnt ? acc[u] + term : acc[u];
                 }
         }
@@ -1029,7 +1037,8 @@ __global__ __launch_bounds__(256) void dwn_bwd_gx_long(const float *__restrict__
 // The gather itself is dwn_bwd_gx's (O == 1): the unrolled path for WI inputs of FAN entries each per wavefront, with
 // the entries' coefficient rows kept in registers over all tiles (S form: one row of 64 per entry, WI = 16 or 4; PACK:
 // two D-form rows of 32 per register, WI = 32), the general loop otherwise; same order of additions.
-// gx == null (HIST only): the sums are made for the bins of the layer in front and not stored.
+// gx == null (HIST only): the sums are made for the bins of the layer in front and not stored; store_from: only those of the
+// tiles from there on are, gx begins with that tile.
 // Pacing of the walking gather (ROWS).  Its blocks are independent; left alone they spread over several batch tiles and
 // every tile's rows are fetched into an XCD's L2 more than once (measured at the headline shape, 16 inputs per
 // wavefront: 692 MiB against 320 compulsory, 55 % L2 misses, 160 us).  So every block starts its tile number i no
@@ -1074,12 +1083,6 @@ __device__ __forceinline__ float dwn_walk_diff(float coef, unsigned a, int j) {
     }
     return dl_lane_read(coef, (int)(a | (1u << j))) - dl_lane_read(coef, (int)(a & ~(1u << j)));
 }
-// D-form rows of two entries in one register: lanes 0-31 the even entry's, lanes 32-63 the odd one's
-__device__ __forceinline__ float dwn_walk_diff_packed(float coef, unsigned a, int j, int odd) {
-    const unsigned low = (1u << j) - 1u;
-    const unsigned ap = (a & low) | ((a >> 1) & ~low);  // the address without its bit j
-    return __int_as_float(__builtin_amdgcn_ds_bpermute((int)((ap << 2) | (odd ? 128u : 0u)), __float_as_int(coef)));
-}
 // PACK (with DFORM; with HIST only up to 16 inputs per wavefront): the D-form row of a slot has 2^(K-1) <= 32 values, so the rows of two entries share one
 // register (lanes 0-31 and 32-63) and a wavefront keeps 32 inputs' entries in the registers that 16 inputs' S-form rows
 // take: half as many blocks cover the inputs, and twice as many inputs are resident on an XCD.
@@ -1090,7 +1093,7 @@ __global__ __launch_bounds__(256) void dwn_bwd_gx_walk(const float *__restrict__
                                                         const uint8_t *__restrict__ prev_addrT, float *__restrict__ prev_partial,
                                                         int I, int N, int BT, int slabs, int split, int part,
                                                         int tiles_per_block, int Lp, int gather_blocks, DwnReduce red,
-                                                        int B = 0, int pace = 0, int pace_slot = 0) {
+                                                        int B = 0, int pace = 0, int pace_slot = 0, int store_from = 0) {
     // the fixed-order sum of this layer's own histogram partials rides behind the gather's blocks
     if ((int)blockIdx.x >= gather_blocks) return dwn_reduce_block(red, (int)blockIdx.x - gather_blocks);
     constexpr int IS = 4 * WI;  // inputs per block
@@ -1235,7 +1238,8 @@ __global__ __launch_bounds__(256) void dwn_bwd_gx_walk(const float *__restrict__
                 const int t = cls + ncls * ti;
                 const uint8_t *addr_t = addrT + (size_t)t * N * 64 + lane;
                 const float *gy_t = gyT + (size_t)t * N * 64 + lane;
-                float *gx_t = gx + ((size_t)t * I + i0 + wbeg) * 64 + lane;
+                const bool store = !ROWS && gx && t >= store_from;
+                float *gx_t = gx + ((ptrdiff_t)(t - store_from) * I + i0 + wbeg) * 64 + lane;
                 uint4 haw = {0u, 0u, 0u, 0u};
                 if (HIST) haw = *reinterpret_cast<const uint4 *>(prev_addrT + (size_t)t * I * 64 + hcol);
                 float acc = 0.0f;
@@ -1261,7 +1265,7 @@ __global__ __launch_bounds__(256) void dwn_bwd_gx_walk(const float *__restrict__
                         if (sidx % FAN == FAN - 1) {
                             if (HIST || ROWS) tile[wbeg + sidx / FAN][lane] = acc;
                             // gx as [B/64][I][64], streamed past the L2 (which holds the rows the gather re-reads)
-                            if (!ROWS && gx) __builtin_nontemporal_store(acc, gx_t + (size_t)(sidx / FAN) * 64);
+                            if (store) __builtin_nontemporal_store(acc, gx_t + (size_t)(sidx / FAN) * 64);
                         }
                     }
                 }
@@ -1345,11 +1349,11 @@ __global__ __launch_bounds__(256) void dwn_bwd_gx_walk(const float *__restrict__
                 __builtin_amdgcn_wave_barrier();
                 // gx as [B/64][I][64]: my inputs, 256 B each, streamed past the L2 (which holds the rows the gather
                 // re-reads); gx == null: the sums are only wanted for the bins of the layer in front
-                if (gx) {
+                if (gx && t >= store_from) {
 #pragma unroll
                     for (int r = 0; r < WI; ++r)
                         if (wbeg + r < iend)
-                            __builtin_nontemporal_store(tile[wbeg + r][lane], &gx[((size_t)t * I + i0 + wbeg + r) * 64 + lane]);
+                            __builtin_nontemporal_store(tile[wbeg + r][lane], &gx[((size_t)(t - store_from) * I + i0 + wbeg + r) * 64 + lane]);
                 }
             }
             // the same rows into the bins of the layer in front (rows past the batch carry 0 and add nothing)
@@ -1606,6 +1610,17 @@ extern "C" int dl_dwn_layer_fwd_static(const float *x, const int32_t *idx32, con
     return dwn_forward_fast(x, idx32, luts, y, saved, (u64 *)planes, B, I, N, k, O, s);
 }
 
+static inline bool dwn_long_applies(int BT, int I, int N, int k, int O, int out_tiled) {
+    return O == 1 && out_tiled && (long long)N * k >= 32LL * I &&
+           (long long)dl_ceil_div(I, 4) * dl_ceil_div(BT, DWN_LT) >= DWN_LONG_BLOCKS;
+}
+template <int K>
+static void dwn_launch_gx_long(const float *gyT, const uint8_t *addrT, const float *D, const int *inv_ptr, const int *inv_pos, float *gx,
+                               int BT, int I, int N, const DwnReduce &red, hipStream_t s) {
+    const int grid = dl_xcd_grid(dl_ceil_div(I, 4), dl_ceil_div(BT, DWN_LT));
+    DL_TIMED("dwn_bwd_gx_long", s, (dwn_bwd_gx_long<K><<<grid + dwn_reduce_blocks(red), 256, 0, s>>>(gyT, addrT, D, inv_ptr, inv_pos, gx,
+                                                                                                   I, N, BT, grid, red)));
+}
 template <int K>
 static void dwn_launch_gx(const float *gyT, const uint8_t *addrT, const float *D, const int *inv_ptr, const int *inv_pos,
                           float *gx, int B, int I, int N, int O, bool sform, int out_tiled, const DwnReduce &red,
@@ -1620,13 +1635,7 @@ static void dwn_launch_gx(const float *gyT, const uint8_t *addrT, const float *D
     // blocks of the latter: lists of 69 (100 columns, 1152 nodes) 14400 608 / 463, 3600 157 / 122, 1800 82 / 70, 1300 63 / 58,
     // 900 46 / 42, 675 38 / 40, 450 27 / 35; lists of 192 (9 columns) 900 90.8 / 90.9, 700 78 / 80, 450 54 / 73; lists of 276
     // 900 149 / 141, 460 87 / 104; lists of 92 680 48 / 46, 440 34 / 40.  From 900 on it loses nowhere.
-    if (O == 1 && sform && out_tiled && (long long)N * K >= 32LL * I &&
-        (long long)dl_ceil_div(I, 4) * dl_ceil_div(BT, DWN_LT) >= DWN_LONG_BLOCKS) {
-        const int grid_l = dl_xcd_grid(dl_ceil_div(I, 4), dl_ceil_div(BT, DWN_LT));
-        DL_TIMED("dwn_bwd_gx_long", s, (dwn_bwd_gx_long<K><<<grid_l + rb, 256, 0, s>>>(gyT, addrT, D, inv_ptr, inv_pos, gx, I, N, BT,
-                                                                                        grid_l, red)));
-        return;
-    }
+    if (sform && dwn_long_applies(BT, I, N, K, O, out_tiled)) return dwn_launch_gx_long<K>(gyT, addrT, D, inv_ptr, inv_pos, gx, BT, I, N, red, s);
     if (O == 1 && sform && out_tiled && (long long)N * K >= 32LL * I) {
         const int grid_s = dl_xcd_grid(dl_ceil_div(I, 4), BT);
         DL_TIMED("dwn_bwd_gx", s, (dwn_bwd_gx<K, 1, true, 1><<<grid_s + rb, 256, 0, s>>>(gyT, addrT, D, inv_ptr, inv_pos, gx, B,
@@ -1685,6 +1694,24 @@ struct DwnFusedPrev {
     float *partial;        // [sets][I][2^k_prev] scratch
 };
 __global__ __launch_bounds__(256) void dwn_build_tables(DwnTables tb) { dwn_table_block(tb, blockIdx.x); }
+// The first layer of a chain, whose tile-major input gradient is taken together with its output gradient (dwn_pair.hip)
+struct DwnFirst {
+    const int *idx32, *inv_ptr, *inv_pos;
+    const float *luts, *alpha_n, *beta_n;
+    float beta_abs_max;
+    int I;        // its inputs
+    float *gx;    // [B/64][I][64] out
+    int tiles;    // batch tiles that dwn_bwd_pair_gx takes; the rest through dwn_bwd_gx_long
+    float *D;     // its coefficient tables (D form)
+    int *lists;   // dwn_pair_list_bytes
+    float *gy;    // its output gradient for the rest
+};
+__global__ __launch_bounds__(256) void dwn_pair_setup(DwnTables tb, const int *__restrict__ idx32, const int *__restrict__ inv_ptr1,
+                                                      const int *__restrict__ inv_pos1, int *__restrict__ lists, int N, int K, int I,
+                                                      int table_blocks) {
+    if ((int)blockIdx.x < table_blocks) dwn_efd_table_block(tb, blockIdx.x);
+    else dwn_pair_list_block(idx32, inv_ptr1, inv_pos1, lists, N, K, I, (int)blockIdx.x - table_blocks);
+}
 // one chunk of rows of a backward taken in several (dwn_row_chunks)
 struct DwnRowChunk {
     float *partial_base;  // the partial sets of all chunks
@@ -1727,8 +1754,10 @@ static inline int dwn_fused_wi(int I, int N, int K) {
 // Inputs that are all read six times (equal widths at k = 6) take the packed rows: two D-form rows per register, so a
 // wavefront keeps 16 inputs' 96 entries instead of 4 inputs' 24, and a quarter as many blocks cover the inputs (an
 // 8000-input layer then fits one XCD's resident blocks, and a tile is read through one L2 instead of four).
+// So do inputs that are all read once (the levels of a convolution's trees): one lane read per connection instead of two
+// (147456 rows, 1152 inputs: 262 -> 254 us).
 static inline bool dwn_fused_pack(int I, int N, int K) {
-    return dwn_fused_wi(I, N, K) == DWN_WI_SMALL && (long long)N * K == 6LL * I;
+    return (dwn_fused_wi(I, N, K) == DWN_WI_SMALL && (long long)N * K == 6LL * I) || (long long)N * K == I;
 }
 static inline size_t dwn_fused_partial_bytes(int B, int I, int N, int k, int k_prev) {
     const int wi = dwn_fused_pack(I, N, k) ? DWN_WI : dwn_fused_wi(I, N, k);
@@ -1764,7 +1793,7 @@ static int dwn_backward_fast(const void *saved, const int32_t *inv_ptr, const in
                              int gx_tiled, float *gluts, void *ws, int B, int I, int N, int k, int O, hipStream_t s,
                              const DwnGroupHead *head = nullptr, const float *alpha_n = nullptr,
                              const float *beta_n = nullptr, const DwnFusedPrev *prev = nullptr,
-                             const DwnRowChunk *rc = nullptr) {
+                             const DwnRowChunk *rc = nullptr, const DwnFirst *first = nullptr) {
     const long long NO = (long long)N * O;
     const int L = 1 << k;
     const uint8_t *addrT = (const uint8_t *)saved;
@@ -1809,8 +1838,9 @@ static int dwn_backward_fast(const void *saved, const int32_t *inv_ptr, const in
     const bool gather = gx || prev;  // (prev without gx: the input gradient is summed for the bins in front, not stored)
     const int fused_wi = prev && (gx_tiled || !gx) && O == 1 && sform ? dwn_fused_wi(I, N, k) : 0;
     const bool fused_pack = fused_wi && dwn_fused_pack(I, N, k);
+    const bool long_rows = gx && !prev && !wide && dwn_long_applies(BT, I, N, k, O, gx_tiled);
     DwnTables tb = {gather && (!rc || rc->first) ? luts : nullptr, D, scale, alpha_n, beta_n, alpha, beta, (int)NO, k, O,
-                    sform ? (walk_pack || fused_pack ? 2 : 1) : 0};
+                    sform ? (walk_pack || fused_pack || long_rows ? 2 : 1) : 0};
     if (wide && tb.luts) {
         DL_TIMED("dwn_wide_tables", s, (dwn_wide_tables<<<(unsigned)NO, 256, 0, s>>>(tb)));
         tb.luts = nullptr;
@@ -1858,18 +1888,21 @@ static int dwn_backward_fast(const void *saved, const int32_t *inv_ptr, const in
         const float *src = gy_tiled ? gy : gyT;
         const DwnFusedSplit f = dwn_fused_split(BT, I, prev->k, 4 * (fused_pack ? DWN_WI : fused_wi));
         const int fan = (long long)N * k % I == 0 ? (int)((long long)N * k / I) : 0;  // every input read `fan` times?
+        const int store_from = first ? first->tiles : 0;
+        if (first && first->tiles < BT) gx = first->gy;
         const int gather_blocks = DL_XCDS * f.part * f.groups, grid = gather_blocks + dwn_reduce_blocks(red), Lp = 1 << prev->k;
 #define DWN_GXH(K_, WI_, FAN_)                                                                                                \
     DL_TIMED("dwn_bwd_gx_hist", s, (dwn_bwd_gx_walk<K_, WI_, FAN_><<<grid, 256, 0, s>>>(src, addrT, D, inv_ptr, inv_pos, gx, prev->addrT, \
-                                                                                  prev->partial, I, N, BT, f.slabs, f.split, f.part, f.tpb, Lp, gather_blocks, red)))
+                                                                                  prev->partial, I, N, BT, f.slabs, f.split, f.part, f.tpb, Lp, gather_blocks, red, 0, 0, 0, store_from)))
+#define DWN_GXP(K_, FAN_)                                                                                                     \
+    DL_TIMED("dwn_bwd_gx_hist", s, (dwn_bwd_gx_walk<K_, DWN_WI, FAN_, true, false, true, true><<<grid, 256, 0, s>>>(src, addrT, D, inv_ptr, inv_pos, gx, prev->addrT, \
+                                                                                  prev->partial, I, N, BT, f.slabs, f.split, f.part, f.tpb, Lp, gather_blocks, red, 0, 0, 0, store_from)))
 #define DWN_GXH_K(K_)                                                \
-    if (fused_pack)                                                  \
-        DL_TIMED("dwn_bwd_gx_hist", s, (dwn_bwd_gx_walk<K_, DWN_WI, 6, true, false, true, true><<<grid, 256, 0, s>>>(src, addrT, D, inv_ptr, inv_pos, gx, prev->addrT, \
-                                                                                  prev->partial, I, N, BT, f.slabs, f.split, f.part, f.tpb, Lp, gather_blocks, red))); \
+    if (fused_pack && fan == 1) DWN_GXP(K_, 1);                      \
+    else if (fused_pack) DWN_GXP(K_, 6);                             \
     else if (fused_wi != DWN_WI && fan == 6) DWN_GXH(K_, DWN_WI_SMALL, 6); \
     else if (fused_wi != DWN_WI && fan == 12) DWN_GXH(K_, DWN_WI_SMALL, 12); \
     else if (fused_wi != DWN_WI) DWN_GXH(K_, DWN_WI_SMALL, 0);       \
-    else if (fan == 1) DWN_GXH(K_, DWN_WI, 1);                       \
     else if (fan == 2) DWN_GXH(K_, DWN_WI, 2);                       \
     else if (fan == 3) DWN_GXH(K_, DWN_WI, 3);                       \
     else DWN_GXH(K_, DWN_WI, 0)
@@ -1882,9 +1915,35 @@ static int dwn_backward_fast(const void *saved, const int32_t *inv_ptr, const in
             default: DWN_GXH_K(6); break;
         }
 #undef DWN_GXH_K
+#undef DWN_GXP
 #undef DWN_GXH
         const DwnReduce pred = {prev->partial, prev->gluts, (long long)I * Lp, f.sets, nullptr, Lp, 1};
         DL_TIMED("dwn_reduce_partials", s, (dwn_reduce_partials<<<dwn_reduce_blocks(pred), 256, 0, s>>>(pred)));
+        if (first) {
+            int rcode;
+            const DwnTables ftb = {first->luts, first->D, nullptr, first->alpha_n, first->beta_n, 0.0f, 0.0f, I, prev->k, 1,
+                                   first->beta_abs_max <= 0.5f ? 2 : 0};
+            const int tables = dwn_table_blocks(ftb);
+            DL_TIMED("dwn_pair_setup", s, (dwn_pair_setup<<<tables + dwn_pair_groups(I), 256, 0, s>>>(ftb, first->idx32, inv_ptr, inv_pos, first->lists, I,
+                                                                                                    prev->k, first->I, tables)));
+            rcode = dwn_pair_launch(src, addrT, D, inv_ptr, inv_pos, N, prev->addrT, first->D, first->lists, first->gx, first->I, I, k,
+                                    first->tiles, s);
+            if (rcode || first->tiles == BT) return rcode;
+            const size_t rows = (size_t)first->tiles * 64;
+            const DwnReduce none = {nullptr, nullptr, 0, 0, nullptr, 1, 1};
+            switch (k) {
+#define DWN_REST(K_) dwn_launch_gx_long<K_>(first->gy, prev->addrT + rows * I, first->D, first->inv_ptr, first->inv_pos, first->gx + rows * first->I, \
+                                            BT - first->tiles, first->I, I, none, s); break
+                case 1: DWN_REST(1);
+                case 2: DWN_REST(2);
+                case 3: DWN_REST(3);
+                case 4: DWN_REST(4);
+                case 5: DWN_REST(5);
+                default: DWN_REST(6);
+#undef DWN_REST
+            }
+            return dl_launch_status();
+        }
     } else if (walk_rows) {
         // row-major input gradient of a big layer whose inputs are all read three times: the walking gather, paced
         const float *src = gy_tiled ? gy : gyT;
@@ -2481,4 +2540,48 @@ extern "C" int dl_dwn_layer_bwd_chain_fused(const void *saved, const int32_t *in
     return dwn_backward_fast(saved, inv_ptr, inv_pos, luts, gy, gy_form == 1, 0.0f, beta_abs_max, nullptr, gx, gx_tiled, gluts,
                              ws, B, I, N, k, O, (hipStream_t)stream, gy_form == 2 ? &head : nullptr, alpha_n, beta_n,
                              prev_saved ? &prev : nullptr);
+}
+
+// ---- the same with the first layer's input gradient, where its output gradient is not needed for anything else
+extern "C" int dl_dwn_chain_first_fusable(int B, int I, int N, int k, int O, int k_first, int I_first, float beta_abs_max) {
+    if (k_first != k || dwn_check(B, I_first, I, k, 1)) return 0;
+    return dl_dwn_chain_fusable(B, I, N, k, O, k, beta_abs_max) && dwn_pair_tiles(dwn_bt(B), I_first, I, k, N) > 0;
+}
+extern "C" size_t dl_dwn_bwd_first_workspace_bytes(int B, int I, int N, int k, int O, int I_first) {
+    if (!dwn_fast(N, k, O)) return 256;
+    const int rest = dwn_bt(B) - dwn_pair_tiles(dwn_bt(B), I_first, I, k, N);
+    return dl_dwn_bwd_fused_workspace_bytes(B, I, N, k, O, k) + dwn_table_bytes(I, k, 1) + dwn_pair_list_bytes(I, k) +
+           (size_t)rest * I * 64 * sizeof(float);
+}
+extern "C" int dl_dwn_layer_bwd_chain_first(const void *saved, const int32_t *inv_ptr, const int32_t *inv_pos,
+                                            const float *luts, const float *gy, int gy_form, int groups, float tau,
+                                            const float *alpha_n, const float *beta_n, float beta_abs_max, float *gluts,
+                                            const void *first_saved, float *first_gluts, const int32_t *first_idx32,
+                                            const int32_t *first_inv_ptr, const int32_t *first_inv_pos, const float *first_luts,
+                                            const float *first_alpha_n, const float *first_beta_n, float first_beta_abs_max,
+                                            int I_first, float *first_gx, void *ws, size_t ws_bytes, int B, int I, int N, int k,
+                                            int O, void *stream) {
+    if (!saved || !inv_ptr || !inv_pos || !luts || !gy || !ws || !alpha_n || !beta_n) return DL_ERR_NULL;
+    if (!first_saved || !first_gluts || !first_idx32 || !first_inv_ptr || !first_inv_pos || !first_luts || !first_alpha_n ||
+        !first_beta_n || !first_gx)
+        return DL_ERR_NULL;
+    if (gy_form < 0 || gy_form > 2) return DL_ERR_SHAPE;
+    if (!gluts && gy_form != 1) return DL_ERR_SHAPE;
+    int rc = dwn_check(B, I, N, k, O);
+    if (rc) return rc;
+    if (gy_form == 2 && (groups <= 0 || !(tau > 0.0f))) return DL_ERR_SHAPE;
+    // saved addresses, tile-major gradients and tables are read and written sixteen bytes at a time
+    if (((uintptr_t)saved | (uintptr_t)first_saved | (uintptr_t)first_gx | (uintptr_t)ws) & 15) return DL_ERR_UNSUPPORTED;
+    if (gy_form == 1 && ((uintptr_t)gy & 15)) return DL_ERR_UNSUPPORTED;
+    if (!dl_dwn_chain_first_fusable(B, I, N, k, O, k, I_first, beta_abs_max)) return DL_ERR_UNSUPPORTED;
+    if (ws_bytes < dl_dwn_bwd_first_workspace_bytes(B, I, N, k, O, I_first)) return DL_ERR_WORKSPACE;
+    const DwnFusedPrev prev = {(const uint8_t *)first_saved, first_gluts, k,
+                               (float *)((char *)ws + dl_dwn_bwd_workspace_bytes(B, I, N, k, O))};
+    char *tables = (char *)ws + dl_dwn_bwd_fused_workspace_bytes(B, I, N, k, O, k), *lists = tables + dwn_table_bytes(I, k, 1);
+    const DwnFirst first = {first_idx32, first_inv_ptr, first_inv_pos, first_luts, first_alpha_n, first_beta_n, first_beta_abs_max,
+                            I_first, first_gx, dwn_pair_tiles(dwn_bt(B), I_first, I, k, N), (float *)tables, (int *)lists,
+                            (float *)(lists + dwn_pair_list_bytes(I, k))};
+    const DwnGroupHead head = {groups, gy_form == 2 ? dwn_group_size(N * O, groups) : 1, gy_form == 2 ? 1.0f / tau : 1.0f};
+    return dwn_backward_fast(saved, inv_ptr, inv_pos, luts, gy, gy_form == 1, 0.0f, beta_abs_max, nullptr, nullptr, 1, gluts, ws, B, I,
+                             N, k, O, (hipStream_t)stream, gy_form == 2 ? &head : nullptr, alpha_n, beta_n, &prev, nullptr, &first);
 }

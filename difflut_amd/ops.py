@@ -302,7 +302,13 @@ class DWNStackFunction(torch.autograd.Function):
             B, I, N, k, O = dims = ctx.dims_all[l]
             plan = ctx.plans[l]
             first_wants_input_grad = ctx.needs_input_grad[0] and not ctx.encoded
-            if l > 0:
+            # the second layer's call can give the first layer's input gradient too: its own is then not stored
+            first = (l == 1 and ctx.image is not None and first_wants_input_grad and ctx.dims_all[0][4] == 1
+                     and len(ctx.scalars[0]) == 3 and len(ctx.scalars[1]) == 3
+                     and lib.dl_dwn_chain_first_fusable(*dims, ctx.dims_all[0][3], ctx.dims_all[0][1], float(ctx.scalars[1][2])) == 1)
+            if first:
+                gx, gx_tiled = None, 1
+            elif l > 0:
                 gx = torch.empty(lib.dl_dwn_tiled_bytes(B, I) // 4, dtype=torch.float32, device=device)
                 gx_tiled = 1
             else:
@@ -314,12 +320,12 @@ class DWNStackFunction(torch.autograd.Function):
                     gx = torch.empty(lib.dl_dwn_tiled_bytes(B, I) // 4, dtype=torch.float32, device=device)
                 else:
                     gx = torch.empty((B, I), dtype=torch.float32, device=device)
-            if have_tables[l] and gx is None:  # nothing left to compute for this layer
+            if have_tables[l] and gx is None and not first:  # nothing left to compute for this layer
                 g = None
                 continue
             if not have_tables[l]:
                 grads[l] = torch.empty_like(luts[l])
-            ws = _bytes(lib.dl_dwn_bwd_workspace_bytes(*dims), device)
+            ws = None if first else _bytes(lib.dl_dwn_bwd_workspace_bytes(*dims), device)
             headed = l == n - 1 and ctx.head is not None
             groups, tau = ctx.head if headed else (1, 1.0)
             if len(ctx.scalars[l]) == 3:  # every node's own alpha and beta
@@ -328,11 +334,23 @@ class DWNStackFunction(torch.autograd.Function):
                 # the gather of this layer can fill the table gradient of the layer in front as it goes: that layer's
                 # own pass over its [B, N] output gradient is then left out
                 k_prev = ctx.dims_all[l - 1][3] if l > 0 else 0
-                fuse = (l > 0 and gx_tiled == 1 and ctx.dims_all[l - 1][4] == 1
-                        and lib.dl_dwn_chain_fusable(*dims, k_prev, float(beta_max)) == 1)
+                fuse = first or (l > 0 and gx_tiled == 1 and ctx.dims_all[l - 1][4] == 1
+                                 and lib.dl_dwn_chain_fusable(*dims, k_prev, float(beta_max)) == 1)
                 if fuse:
                     grads[l - 1] = torch.empty_like(luts[l - 1])
                     have_tables[l - 1] = True
+                    if first:
+                        I_first, first_scalars = ctx.dims_all[0][1], ctx.scalars[0]
+                        first_alpha, first_beta = (_per_node(v, I, device) for v in first_scalars[:2])
+                        gy_l, g = g, torch.empty(lib.dl_dwn_tiled_bytes(B, I_first) // 4, dtype=torch.float32, device=device)
+                        ws = _bytes(lib.dl_dwn_bwd_first_workspace_bytes(*dims, I_first), device)
+                        nat.check(lib.dl_dwn_layer_bwd_chain_first(
+                            nat.ptr(saved[l]), nat.ptr(plan.inv_ptr), nat.ptr(plan.inv_pos), nat.ptr(luts[l]), nat.ptr(gy_l),
+                            2 if headed else tiled, int(groups), float(tau), nat.ptr(alpha_n), nat.ptr(beta_n), float(beta_max),
+                            None if have_tables[l] else nat.ptr(grads[l]), nat.ptr(saved[0]), nat.ptr(grads[0]),
+                            nat.ptr(ctx.plans[0].idx32), nat.ptr(ctx.plans[0].inv_ptr), nat.ptr(ctx.plans[0].inv_pos), nat.ptr(luts[0]), nat.ptr(first_alpha), nat.ptr(first_beta),
+                            float(first_scalars[2]), I_first, nat.ptr(g), nat.ptr(ws), ws.numel(), *dims, nat.stream()))
+                        break
                     ws = _bytes(lib.dl_dwn_bwd_fused_workspace_bytes(*dims, k_prev), device)
                     if l == 1 and not first_wants_input_grad:
                         gx = None  # the first layer's table gradient is all that is left: nobody reads this gradient

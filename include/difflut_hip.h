@@ -197,6 +197,23 @@ int dl_dwn_layer_bwd_chain_fused(const void *saved, const int32_t *inv_ptr, cons
                                  const float *beta_n, float beta_abs_max, float *gx, int gx_tiled, float *gluts,
                                  const void *prev_saved, int k_prev, float *prev_gluts, void *ws, size_t ws_bytes,
                                  int B, int I, int N, int k, int O, void *stream);
+/* dl_dwn_layer_bwd_chain_fused for the second layer of a chain, with the input gradient of the FIRST layer (I nodes of k
+ * inputs over I_first inputs, one output each) as well: first_gx [B/64][I_first][64].  The first layer's output gradient is
+ * summed where it is used; only that of a last few batch tiles is stored.  first_idx32 [I, k], first_inv_* (its inverse
+ * mapping), first_luts [I, 2^k], first_alpha_n / first_beta_n [I] are the first layer's, first_beta_abs_max = max
+ * |first_beta_n|.  For shapes where dl_dwn_chain_first_fusable(...) == 1 (few inputs read many times over many rows, every
+ * node of the first layer read once: the trees of a convolution; the same k in both layers) and 16-byte aligned arrays, refused
+ * (DL_ERR_UNSUPPORTED) elsewhere; the values are those of the two calls it replaces.  Workspace
+ * dl_dwn_bwd_first_workspace_bytes. */
+int dl_dwn_chain_first_fusable(int B, int I, int N, int k, int O, int k_first, int I_first, float beta_abs_max);
+size_t dl_dwn_bwd_first_workspace_bytes(int B, int I, int N, int k, int O, int I_first);
+int dl_dwn_layer_bwd_chain_first(const void *saved, const int32_t *inv_ptr, const int32_t *inv_pos, const float *luts,
+                                 const float *gy, int gy_form, int groups, float tau, const float *alpha_n,
+                                 const float *beta_n, float beta_abs_max, float *gluts, const void *first_saved,
+                                 float *first_gluts, const int32_t *first_idx32, const int32_t *first_inv_ptr,
+                                 const int32_t *first_inv_pos, const float *first_luts, const float *first_alpha_n,
+                                 const float *first_beta_n, float first_beta_abs_max, int I_first, float *first_gx, void *ws,
+                                 size_t ws_bytes, int B, int I, int N, int k, int O, void *stream);
 /* The eval forward below with a workspace (dl_dwn_eval_workspace_bytes): the same result for any input, and
  * the bit-plane kernels' speed when every input value is exactly 0 or 1 (checked on the device while packing;
  * no host synchronisation - both kernels are launched and one returns at once). */

@@ -236,6 +236,53 @@ def test_conv_gather_of_four_batch_tiles_equals_that_of_one(images, columns, fie
     assert torch.equal(whole, torch.cat([part for part, _ in parts]))
 
 
+@pytest.mark.parametrize("images,columns,field,channels,k,depth,shuffle", [
+    (113, 1, 4, 16, 6, 2, False),   # 16 inputs, 1104 batch tiles: just enough of both
+    (160, 2, 8, 19, 6, 2, False),   # 128 inputs; 684 nodes: a last step of twelve; 1103 tiles: a last block of three
+    (233, 4, 5, 50, 4, 2, False),   # 2097 tiles: 49 of them through the stored gradient
+    (123, 1, 5, 23, 6, 1, False),   # one level of trees; a wavefront with a single input
+    (113, 1, 4, 19, 3, 2, True),    # nodes that the second layer reads twice or not at all
+    (113, 1, 4, 64, 2, 2, False),
+    (113, 1, 4, 512, 1, 1, False)])
+def test_conv_input_gradient_of_two_levels_at_once(images, columns, field, channels, k, depth, shuffle):
+    """The first level's input gradient from the second level's output gradient against gathering it from the stored output
+    gradient of the first level, which is what smaller batches do: same terms in the same order, so the same bits; the table
+    gradients add their batches in another order.  Which of them ran is read from the library's record."""
+    from difflut_amd import _native as nat
+    torch.manual_seed(23)
+    layer = _build("dwn", depth, columns, channels, field, 1, 0, 32, n=k).train()
+    if shuffle:
+        for tree in layer.trees:
+            table = tree[0]._mapping_indices
+            table.copy_(torch.randint(0, k ** depth, table.shape, device=DEV))
+    side = 28 - field + 1
+    x = (torch.rand(images, columns, 28, 28, device=DEV) < 0.5).float()
+    gy = torch.randn(images, channels, side, side, device=DEV)
+
+    def gradients(rows):
+        part = x[rows].clone().requires_grad_()
+        for p in layer.bank_parameters():
+            p.grad = None
+        nat.profile_read()
+        nat.profile_enable(True)
+        try:
+            layer(part).backward(gy[rows])
+            names = {name for name, _ in nat.profile_read()}
+        finally:
+            nat.profile_enable(False)
+        return part.grad, [p.grad for p in layer.bank_parameters()], "dwn_bwd_pair_gx" in names
+
+    whole, tables, both = gradients(slice(0, images))
+    assert both and whole.abs().max() > 0
+    parts = [gradients(slice(i, min(i + 64, images))) for i in range(0, images, 64)]
+    assert not any(both for _, _, both in parts)
+    assert torch.equal(whole, torch.cat([part for part, _, _ in parts]))
+    for level, grad in enumerate(tables):
+        want = sum(part[level].double() for _, part, _ in parts)
+        # a bin adds at most as many values as there are rows: their rounding, of values up to the largest bin's size
+        torch.testing.assert_close(grad.double(), want, rtol=2e-5, atol=2e-6 * float(want.abs().max()))
+
+
 def test_conv_bank_parameters_train_in_place():
     """An optimizer over bank_parameters() (one tensor per depth level) updates the per-node parameters the
     state dict shows."""
