@@ -7,6 +7,8 @@ with torch's current HIP stream; outputs and workspaces are allocated by the
 caller with torch's caching allocator.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 import torch
@@ -97,7 +99,11 @@ SIGNATURES = {
     "dl_profile_read": (_I, [ctypes.c_char_p, _Z, ctypes.POINTER(_F), _I]),
 }
 
+# the autograd functions over the library (csrc/host_ops.cpp)
+HOST_PATH = os.path.join(_HERE, "lib", "difflut_host.so")
+
 _lib = None
+_host = None
 
 
 def is_built():
@@ -118,6 +124,21 @@ def lib():
             fn.restype, fn.argtypes = res, args
         _lib = handle
     return _lib
+
+
+def host():
+    """Load the native autograd functions once and bind them to the library; raises RuntimeError when not built."""
+    global _host
+    if _host is None:
+        lib()
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError(f"HIP extension not available: {HOST_PATH} is missing. Build it with `python -m difflut_amd.build`.")
+        loader = importlib.machinery.ExtensionFileLoader("difflut_host", HOST_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("difflut_host", loader))
+        loader.exec_module(module)
+        module.load(LIB_PATH)
+        _host = module
+    return _host
 
 
 def check(code):

@@ -140,7 +140,7 @@ class ScalarBank:
     `abs_max()` (the largest magnitude, which selects the form of the EFD coefficient table): read back when the
     bank's version counter changes or after `invalidate()`."""
 
-    _node = None  # as for the ParameterBank
+    _keys = ()  # the nodes' names in their ModuleList
     _PROBES = 16  # nodes checked per call beyond the first and the last when the layer is large
 
     def __init__(self, nodes, name):
@@ -161,11 +161,7 @@ class ScalarBank:
             view._scalar_bank = self
             node._buffers[self.name] = view
             self._views.append(view)
-        self._node = _node_getter(self.nodes)
         self._stale, self._key = False, None
-
-    def __getstate__(self):
-        return {k: v for k, v in self.__dict__.items() if k != "_node"}  # tied() and tie() make it again
 
     def tied(self):
         """Every node's buffer is still the view handed out by tie().  All nodes are checked on small layers; on large
@@ -181,11 +177,17 @@ class ScalarBank:
         else:
             rows = [0, n - 1] + [(self._probe + i) % n for i in range(self._PROBES)]
             self._probe = (self._probe + self._PROBES) % n
-        if self._node is None:
-            self._node = _node_getter(self.nodes)
-        node, name, views = self._node, self.name, self._views
+        name, views, nodes = self.name, self._views, self.nodes
+        if isinstance(nodes, nn.ModuleList):  # as _node_getter does, without a call per node
+            if len(self._keys) != n:
+                self._keys = [str(row) for row in range(n)]
+            nodes, keys = nodes._modules, self._keys
+            for row in rows:
+                if nodes[keys[row]]._buffers[name] is not views[row]:
+                    return False
+            return True
         for row in rows:
-            if node(row)._buffers[name] is not views[row]:
+            if nodes[row]._buffers[name] is not views[row]:
                 return False
         return True
 

@@ -163,7 +163,7 @@ class ConvolutionalLayer(LUTLayerMixin, nn.Module):
         return [bank.tensor() for banks in self._level_banks for bank in banks.values()]
 
     def _level_plans(self, device):
-        tables = [layer._mapping_indices for layer in self._sublayers()]
+        tables = [layer._buffers["_mapping_indices"] for layer in self._sublayers()]
         key = (str(device),) + tuple((t.data_ptr(), t._version) for t in tables)
         if self._plans is None or self._plan_key != key:
             plans = []

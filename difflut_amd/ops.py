@@ -1,6 +1,8 @@
-"""Layer-level operators: torch.autograd.Functions over the C ABI of libdifflut_hip.so.
+"""Layer-level operators: autograd functions over the C ABI of libdifflut_hip.so.
 
-These are the callers of the drop-in boundary.  They keep the conventions of the
+These are the callers of the drop-in boundary.  Those that a training step or an inference request is made of are native
+(csrc/host_ops.cpp; the classes here give them the call conventions of a torch.autograd.Function), the others are
+torch.autograd.Functions over ctypes.  All keep the conventions of the
 reference's autograd wrappers (difflut/layers/random_layer.py:34-100,
 difflut/nodes/dwn_node.py:58-128, difflut/nodes/probabilistic_node.py:39-129,
 difflut/layers/learnable_layer.py:58-123): inputs are made contiguous fp32, outputs
@@ -34,12 +36,6 @@ def _per_node(values, N, device):
     return values.reshape(-1).expand(N).contiguous()
 
 
-def _backward_reads_x(N, k, O):
-    """Whether the DWN backward needs x: not where the forward leaves the address of every node and row (k <= 6 and, within
-    the bounds of the library's dwn_wide, 7 and 8)."""
-    return k > 8 or (k > FAST_K and not (N < 1 << 23 and N * O * (4 << k) < 0x7fffffff))
-
-
 class MappingPlan:
     """Device-side form of an index table idx [N,k] over I inputs.
 
@@ -67,6 +63,7 @@ class MappingPlan:
         self.device = idx.device
         self.source_ptr = idx.data_ptr()
         self.source_version = idx._version
+        self.host = (self.idx32, self.inv_ptr, self.inv_pos, self.I)  # as the native operators take it
 
     def matches(self, idx):
         return (idx.device == self.device and idx.data_ptr() == self.source_ptr
@@ -150,71 +147,32 @@ class UnfoldFunction(torch.autograd.Function):
 
 
 # ----------------------------------------------------------------------------- DWN
-class DWNLayerFunction(torch.autograd.Function):
+class DWNLayerFunction:
     """y[b, n*O+d] = luts[n,d,addr(b,n)] with the extended-finite-difference backward."""
 
     @staticmethod
-    def forward(ctx, x, luts, plan, alpha, beta, beta_abs_max=None):
+    def apply(x, luts, plan, alpha, beta, beta_abs_max=None):
         """alpha, beta: Python floats for the whole layer, or device tensors [N] with every node's own values
         (then beta_abs_max = max |beta|, a host value)."""
         nat.require_device(x, luts)
-        x, luts = _f32(x), _f32(luts)
-        B, I = x.shape
-        N, O, L = luts.shape
-        k = plan.k
-        if (N, 1 << k, I) != (plan.N, L, plan.I):
-            raise RuntimeError(f"shape mismatch: x {tuple(x.shape)}, luts {tuple(luts.shape)}, mapping [{plan.N},{k}] "
-                               f"over {plan.I} inputs")
-        lib = nat.lib()
-        dims = (B, I, N, k, O)
-        y = torch.empty((B, N * O), dtype=torch.float32, device=x.device)
-        saved = _bytes(lib.dl_dwn_saved_bytes(*dims), x.device)
-        ws = _bytes(lib.dl_dwn_fwd_workspace_bytes(*dims), x.device)
-        nat.check(lib.dl_dwn_layer_fwd(nat.ptr(x), nat.ptr(plan.idx32), nat.ptr(luts), nat.ptr(y), nat.ptr(saved),
-                                       nat.ptr(ws), ws.numel(), *dims, nat.stream()))
         if torch.is_tensor(alpha) or torch.is_tensor(beta):
             if any(torch.is_tensor(v) and v.dim() > 1 for v in (alpha, beta)):
                 raise RuntimeError("alpha and beta of a layer are numbers or tensors [N]")
-            alpha, beta = _per_node(alpha, N, x.device), _per_node(beta, N, x.device)
+            alpha, beta = _per_node(alpha, plan.N, x.device), _per_node(beta, plan.N, x.device)
             if beta_abs_max is None:
                 beta_abs_max = float(beta.abs().max())
-            ctx.ab = (alpha, beta, float(beta_abs_max))
-        else:
-            ctx.ab = (float(alpha), float(beta))
-        ctx.save_for_backward(luts, saved, x if _backward_reads_x(N, k, O) else None)
-        ctx.plan, ctx.dims = plan, dims
-        return y
-
-    @staticmethod
-    def backward(ctx, gy):
-        luts, saved, x = ctx.saved_tensors
-        B, I, N, k, O = ctx.dims
-        plan = ctx.plan
-        gy = _f32(gy)
-        lib = nat.lib()
-        gx = torch.empty((B, I), dtype=torch.float32, device=gy.device) if ctx.needs_input_grad[0] else None
-        gl = torch.empty_like(luts)
-        ws = _bytes(lib.dl_dwn_bwd_workspace_bytes(*ctx.dims), gy.device)
-        if len(ctx.ab) == 3:
-            nat.check(lib.dl_dwn_layer_bwd_nodes(nat.ptr(x), nat.ptr(saved), nat.ptr(plan.idx32), nat.ptr(plan.inv_ptr),
-                                                 nat.ptr(plan.inv_pos), nat.ptr(luts), nat.ptr(gy), nat.ptr(ctx.ab[0]),
-                                                 nat.ptr(ctx.ab[1]), ctx.ab[2], nat.ptr(gx), nat.ptr(gl), nat.ptr(ws),
-                                                 ws.numel(), *ctx.dims, nat.stream()))
-        else:
-            nat.check(lib.dl_dwn_layer_bwd(nat.ptr(x), nat.ptr(saved), nat.ptr(plan.idx32), nat.ptr(plan.inv_ptr),
-                                           nat.ptr(plan.inv_pos), nat.ptr(luts), nat.ptr(gy), ctx.ab[0], ctx.ab[1],
-                                           nat.ptr(gx), nat.ptr(gl), nat.ptr(ws), ws.numel(), *ctx.dims, nat.stream()))
-        return gx, gl, None, None, None, None
+            return nat.host().dwn_layer(x, luts, plan.host, alpha, beta, 0.0, beta_abs_max)
+        return nat.host().dwn_layer(x, luts, plan.host, None, None, alpha, beta)
 
 
-class DWNStackFunction(torch.autograd.Function):
+class DWNStackFunction:
     """A chain of RandomLayer + DWN layers in one autograd node.  A following DWN layer only thresholds
     what it is given, so between layers the activations stay bit-planes and the gradients stay
     tile-major: no [B, N] fp32 tensor is written or read except the last layer's output (and the
     first layer's input gradient, if asked for).  Same arithmetic as calling the layers one by one."""
 
     @staticmethod
-    def forward(ctx, x, source, plans, scalars, head, *luts):
+    def apply(x, source, plans, scalars, head, *luts):
         """`scalars`: per layer (alpha, beta) as numbers, or (alpha [N], beta [N], max |beta|) with every node's own.
         `head`: None, or (groups, tau) of a GroupSum that follows the last layer: the function then returns
         the [B, groups] sums and neither the last layer's [B, N] output nor its gradient is ever written.
@@ -226,160 +184,16 @@ class DWNStackFunction(torch.autograd.Function):
                               matrix (rows = output positions), again produced directly as bit-planes; the
                               input gradient is folded back from the tile-major patch gradient.  `flip`
                               (bool [rows, C*KH*KW], optional): patch entries the bit-flip augmentation inverts."""
-        thresholds = source if torch.is_tensor(source) else None
-        geom = tuple(source[:6]) if isinstance(source, tuple) else None
-        flip = source[6] if isinstance(source, tuple) and len(source) > 6 else None
-        nat.require_device(x, thresholds, *luts)
-        x = _f32(x)
-        luts = tuple(_f32(t) for t in luts)
-        lib = nat.lib()
-        ctx.image = None
-        if geom is not None:
-            Bi, C, H, W = x.shape
-            B = int(lib.dl_unfold_rows(Bi, H, W, *geom))
-            if B <= 0:
-                raise RuntimeError(f"receptive field {geom[:2]} with stride {geom[2:4]}, padding {geom[4:]} does not fit "
-                                   f"a {H}x{W} image")
-            width = C * geom[0] * geom[1]
-            planes = _bytes(lib.dl_dwn_planes_bytes(B, width), x.device)
-            flip = _flip_bytes(flip, (B, width))
-            nat.check(lib.dl_unfold_flip(nat.ptr(x), nat.ptr(flip), None, nat.ptr(planes), Bi, C, H, W, *geom, nat.stream()))
-            ctx.image = ((Bi, C, H, W), geom)
-        elif thresholds is None:
-            B, width = x.shape
-            planes = _bytes(lib.dl_dwn_planes_bytes(B, width), x.device)
-            nat.check(lib.dl_dwn_pack_planes(nat.ptr(x), nat.ptr(planes), B, width, nat.stream()))
-        else:
-            B, width = x.shape
-            thr = _f32(thresholds)
-            if thr.dim() != 2 or thr.shape[0] != width:
-                raise RuntimeError(f"thresholds {tuple(thr.shape)} do not match {width} features")
-            nbits = thr.shape[1]
-            planes = _bytes(lib.dl_dwn_planes_bytes(B, width * nbits), x.device)
-            nat.check(lib.dl_thermometer_planes(nat.ptr(x), nat.ptr(thr), nat.ptr(planes), B, width, nbits, nat.stream()))
-            width *= nbits
-        saved, dims_all, y = [], [], None
-        for l, (plan, lut) in enumerate(zip(plans, luts)):
-            N, O, L = lut.shape
-            k = plan.k
-            if k > FAST_K or (N, 1 << k, width) != (plan.N, L, plan.I):
-                raise RuntimeError(f"layer {l}: cannot chain (k={k}, tables {tuple(lut.shape)}, mapping [{plan.N},{k}] over "
-                                   f"{plan.I} inputs, incoming width {width})")
-            dims = (B, width, N, k, O)
-            last = l == len(plans) - 1
-            keep = _bytes(lib.dl_dwn_saved_bytes(*dims), x.device)
-            nxt = None if last else _bytes(lib.dl_dwn_planes_bytes(B, N * O), x.device)
-            if last and head is not None:
-                groups, tau = head
-                y = torch.empty((B, groups), dtype=torch.float32, device=x.device)
-                ws = _bytes(lib.dl_dwn_groups_workspace_bytes(B, N, O, groups), x.device)
-                nat.check(lib.dl_dwn_layer_fwd_planes_groups(nat.ptr(planes), nat.ptr(plan.idx32), nat.ptr(lut), nat.ptr(y),
-                                                             nat.ptr(keep), nat.ptr(ws), ws.numel(), *dims, int(groups),
-                                                             float(tau), nat.stream()))
-            else:
-                y = torch.empty((B, N * O), dtype=torch.float32, device=x.device) if last else None
-                nat.check(lib.dl_dwn_layer_fwd_planes(nat.ptr(planes), nat.ptr(plan.idx32), nat.ptr(lut), nat.ptr(y),
-                                                      nat.ptr(nxt), nat.ptr(keep), *dims, nat.stream()))
-            saved.append(keep)
-            dims_all.append(dims)
-            planes, width = nxt, N * O
-        ctx.save_for_backward(*luts, *saved)
-        ctx.plans, ctx.scalars, ctx.dims_all = plans, scalars, dims_all
-        ctx.encoded = thresholds is not None
-        ctx.head = head
-        return y
-
-    @staticmethod
-    def backward(ctx, gy):
-        n = len(ctx.plans)
-        luts, saved = ctx.saved_tensors[:n], ctx.saved_tensors[n:]
-        lib = nat.lib()
-        g, tiled = _f32(gy), 0
-        device = g.device
-        grads = [None] * n
-        have_tables = [False] * n  # table gradient already produced by the call for the layer behind
-        for l in range(n - 1, -1, -1):
-            B, I, N, k, O = dims = ctx.dims_all[l]
-            plan = ctx.plans[l]
-            first_wants_input_grad = ctx.needs_input_grad[0] and not ctx.encoded
-            # the second layer's call can give the first layer's input gradient too: its own is then not stored
-            first = (l == 1 and ctx.image is not None and first_wants_input_grad and ctx.dims_all[0][4] == 1
-                     and len(ctx.scalars[0]) == 3 and len(ctx.scalars[1]) == 3
-                     and lib.dl_dwn_chain_first_fusable(*dims, ctx.dims_all[0][3], ctx.dims_all[0][1], float(ctx.scalars[1][2])) == 1)
-            if first:
-                gx, gx_tiled = None, 1
-            elif l > 0:
-                gx = torch.empty(lib.dl_dwn_tiled_bytes(B, I) // 4, dtype=torch.float32, device=device)
-                gx_tiled = 1
-            else:
-                want = ctx.needs_input_grad[0] and not ctx.encoded
-                gx_tiled = 1 if ctx.image is not None else 0
-                if not want:
-                    gx = None
-                elif gx_tiled:
-                    gx = torch.empty(lib.dl_dwn_tiled_bytes(B, I) // 4, dtype=torch.float32, device=device)
-                else:
-                    gx = torch.empty((B, I), dtype=torch.float32, device=device)
-            if have_tables[l] and gx is None and not first:  # nothing left to compute for this layer
-                g = None
-                continue
-            if not have_tables[l]:
-                grads[l] = torch.empty_like(luts[l])
-            ws = None if first else _bytes(lib.dl_dwn_bwd_workspace_bytes(*dims), device)
-            headed = l == n - 1 and ctx.head is not None
-            groups, tau = ctx.head if headed else (1, 1.0)
-            if len(ctx.scalars[l]) == 3:  # every node's own alpha and beta
-                alpha_n, beta_n, beta_max = ctx.scalars[l]
-                alpha_n, beta_n = _per_node(alpha_n, N, device), _per_node(beta_n, N, device)
-                # the gather of this layer can fill the table gradient of the layer in front as it goes: that layer's
-                # own pass over its [B, N] output gradient is then left out
-                k_prev = ctx.dims_all[l - 1][3] if l > 0 else 0
-                fuse = first or (l > 0 and gx_tiled == 1 and ctx.dims_all[l - 1][4] == 1
-                                 and lib.dl_dwn_chain_fusable(*dims, k_prev, float(beta_max)) == 1)
-                if fuse:
-                    grads[l - 1] = torch.empty_like(luts[l - 1])
-                    have_tables[l - 1] = True
-                    if first:
-                        I_first, first_scalars = ctx.dims_all[0][1], ctx.scalars[0]
-                        first_alpha, first_beta = (_per_node(v, I, device) for v in first_scalars[:2])
-                        gy_l, g = g, torch.empty(lib.dl_dwn_tiled_bytes(B, I_first) // 4, dtype=torch.float32, device=device)
-                        ws = _bytes(lib.dl_dwn_bwd_first_workspace_bytes(*dims, I_first), device)
-                        nat.check(lib.dl_dwn_layer_bwd_chain_first(
-                            nat.ptr(saved[l]), nat.ptr(plan.inv_ptr), nat.ptr(plan.inv_pos), nat.ptr(luts[l]), nat.ptr(gy_l),
-                            2 if headed else tiled, int(groups), float(tau), nat.ptr(alpha_n), nat.ptr(beta_n), float(beta_max),
-                            None if have_tables[l] else nat.ptr(grads[l]), nat.ptr(saved[0]), nat.ptr(grads[0]),
-                            nat.ptr(ctx.plans[0].idx32), nat.ptr(ctx.plans[0].inv_ptr), nat.ptr(ctx.plans[0].inv_pos), nat.ptr(luts[0]), nat.ptr(first_alpha), nat.ptr(first_beta),
-                            float(first_scalars[2]), I_first, nat.ptr(g), nat.ptr(ws), ws.numel(), *dims, nat.stream()))
-                        break
-                    ws = _bytes(lib.dl_dwn_bwd_fused_workspace_bytes(*dims, k_prev), device)
-                    if l == 1 and not first_wants_input_grad:
-                        gx = None  # the first layer's table gradient is all that is left: nobody reads this gradient
-                nat.check(lib.dl_dwn_layer_bwd_chain_fused(
-                    nat.ptr(saved[l]), nat.ptr(plan.inv_ptr), nat.ptr(plan.inv_pos), nat.ptr(luts[l]), nat.ptr(g),
-                    2 if headed else tiled, int(groups), float(tau), nat.ptr(alpha_n), nat.ptr(beta_n), float(beta_max),
-                    nat.ptr(gx), gx_tiled, None if have_tables[l] else nat.ptr(grads[l]),
-                    nat.ptr(saved[l - 1]) if fuse else None, k_prev, nat.ptr(grads[l - 1]) if fuse else None,
-                    nat.ptr(ws), ws.numel(), *dims, nat.stream()))
-                g, tiled = gx, gx_tiled
-                continue
-            alpha, beta = ctx.scalars[l]
-            if headed:
-                nat.check(lib.dl_dwn_layer_bwd_groups(nat.ptr(saved[l]), nat.ptr(plan.inv_ptr), nat.ptr(plan.inv_pos),
-                                                      nat.ptr(luts[l]), nat.ptr(g), int(groups), float(tau), float(alpha),
-                                                      float(beta), nat.ptr(gx), gx_tiled, nat.ptr(grads[l]), nat.ptr(ws),
-                                                      ws.numel(), *dims, nat.stream()))
-            else:
-                nat.check(lib.dl_dwn_layer_bwd_tiled(nat.ptr(saved[l]), nat.ptr(plan.inv_ptr), nat.ptr(plan.inv_pos),
-                                                     nat.ptr(luts[l]), nat.ptr(g), tiled, float(alpha), float(beta),
-                                                     nat.ptr(gx), gx_tiled, nat.ptr(grads[l]), nat.ptr(ws), ws.numel(), *dims,
-                                                     nat.stream()))
-            g, tiled = gx, gx_tiled
-        if ctx.image is not None and g is not None:
-            shape, geom = ctx.image
-            gimg = torch.empty(shape, dtype=torch.float32, device=device)
-            nat.check(lib.dl_fold(nat.ptr(g), 1, nat.ptr(gimg), *shape, *geom, nat.stream()))
-            g = gimg
-        return (g, None, None, None, None, *grads)
+        nat.require_device(x, source if torch.is_tensor(source) else None, *luts)
+        groups, tau = head if head is not None else (0, 1.0)
+        values = [(alpha, beta[0], 0.0, beta[1]) if beta[1:] else (None, None, alpha, beta[0])
+                  for alpha, *beta in scalars]
+        thresholds, geom, flip = None, (), None
+        if torch.is_tensor(source):
+            thresholds = source
+        elif source is not None:
+            geom, flip = source[:6], source[6] if len(source) > 6 else None
+        return nat.host().dwn_stack(x, luts, [p.host for p in plans], values, thresholds, geom, flip, groups, tau)
 
 
 def dwn_stack_eval(x, thresholds, plans, luts, head=None):
@@ -388,45 +202,8 @@ def dwn_stack_eval(x, thresholds, plans, luts, head=None):
     Activations stay bit-planes between the layers; returns the last layer's 0/1 output [B, N], or with
     `head` = (groups, tau) its GroupSum [B, groups].  Equals calling the layers' eval forward one by one."""
     nat.require_device(x, thresholds, *luts)
-    x = _f32(x)
-    lib = nat.lib()
-    B, width = x.shape
-    if thresholds is None:
-        planes = _bytes(lib.dl_dwn_planes_bytes(B, width), x.device)
-        nat.check(lib.dl_dwn_pack_planes(nat.ptr(x), nat.ptr(planes), B, width, nat.stream()))
-    else:
-        thr = _f32(thresholds)
-        if thr.dim() != 2 or thr.shape[0] != width:
-            raise RuntimeError(f"thresholds {tuple(thr.shape)} do not match {width} features")
-        nbits = thr.shape[1]
-        planes = _bytes(lib.dl_dwn_planes_bytes(B, width * nbits), x.device)
-        nat.check(lib.dl_thermometer_planes(nat.ptr(x), nat.ptr(thr), nat.ptr(planes), B, width, nbits, nat.stream()))
-        width *= nbits
-    y = None
-    for l, (plan, lut) in enumerate(zip(plans, luts)):
-        lut = _f32(lut)
-        N, O, L = lut.shape
-        k = plan.k
-        if k > FAST_K or (N, 1 << k, width) != (plan.N, L, plan.I):
-            raise RuntimeError(f"layer {l}: cannot chain (k={k}, tables {tuple(lut.shape)}, mapping [{plan.N},{k}] over "
-                               f"{plan.I} inputs, incoming width {width})")
-        dims = (B, width, N, k, O)
-        last = l == len(plans) - 1
-        if last and head is not None:
-            groups, tau = head
-            y = torch.empty((B, groups), dtype=torch.float32, device=x.device)
-            ws = _bytes(lib.dl_dwn_groups_workspace_bytes(B, N, O, groups), x.device)
-            nat.check(lib.dl_dwn_layer_eval_planes_groups(nat.ptr(planes), nat.ptr(plan.idx32), nat.ptr(lut), nat.ptr(y),
-                                                          nat.ptr(ws), ws.numel(), *dims, int(groups), float(tau),
-                                                          nat.stream()))
-        else:
-            y = torch.empty((B, N * O), dtype=torch.float32, device=x.device) if last else None
-            nxt = None if last else _bytes(lib.dl_dwn_planes_bytes(B, N * O), x.device)
-            nat.check(lib.dl_dwn_layer_eval_planes(nat.ptr(planes), nat.ptr(plan.idx32), nat.ptr(lut), nat.ptr(y),
-                                                   nat.ptr(nxt), *dims, nat.stream()))
-            planes = nxt
-        width = N * O
-    return y
+    groups, tau = head if head is not None else (0, 1.0)
+    return nat.host().dwn_stack_eval(x, thresholds, luts, [p.host for p in plans], groups, tau)
 
 
 def dwn_layer_eval(x, luts, plan):
@@ -446,130 +223,35 @@ def dwn_layer_eval(x, luts, plan):
 
 
 # ----------------------------------------------------------------------------- DWN-stable and hybrid nodes
-class TableSigmoidFunction(torch.autograd.Function):
+class TableSigmoidFunction:
     """luts = sigmoid(raw_luts), elementwise, for a whole bank of tables at once
     (`_get_luts`, dwn_stable_node.py:289-295, hybrid_node.py:309-315)."""
 
     @staticmethod
-    def forward(ctx, raw):
+    def apply(raw):
         nat.require_device(raw)
-        raw = _f32(raw)
-        luts = torch.empty_like(raw)
-        nat.check(nat.lib().dl_table_sigmoid_fwd(nat.ptr(raw), nat.ptr(luts), raw.numel(), nat.stream()))
-        ctx.save_for_backward(luts)
-        return luts
-
-    @staticmethod
-    def backward(ctx, gl):
-        (luts,) = ctx.saved_tensors
-        gl = _f32(gl)
-        graw = torch.empty_like(luts)
-        nat.check(nat.lib().dl_table_sigmoid_bwd(nat.ptr(gl), nat.ptr(luts), nat.ptr(graw), luts.numel(), nat.stream()))
-        return graw
+        return nat.host().table_sigmoid(raw)
 
 
-def _lookup_dims(x, luts, plan):
-    B, I = x.shape
-    N, O, L = luts.shape
-    k = plan.k
-    if (N, 1 << k, I) != (plan.N, L, plan.I):
-        raise RuntimeError(f"shape mismatch: x {tuple(x.shape)}, luts {tuple(luts.shape)}, mapping [{plan.N},{k}] "
-                           f"over {plan.I} inputs")
-    return B, I, N, k, O
-
-
-def _dwn_lookup(x, luts, plan):
-    """Training forward shared by the DWN-type nodes: (y, saved, dims)."""
-    dims = _lookup_dims(x, luts, plan)
-    B, _, N, _, O = dims
-    lib = nat.lib()
-    y = torch.empty((B, N * O), dtype=torch.float32, device=x.device)
-    saved = _bytes(lib.dl_dwn_saved_bytes(*dims), x.device)
-    ws = _bytes(lib.dl_dwn_fwd_workspace_bytes(*dims), x.device)
-    nat.check(lib.dl_dwn_layer_fwd(nat.ptr(x), nat.ptr(plan.idx32), nat.ptr(luts), nat.ptr(y), nat.ptr(saved),
-                                   nat.ptr(ws), ws.numel(), *dims, nat.stream()))
-    return y, saved, dims
-
-
-class DWNStableLayerFunction(torch.autograd.Function):
+class DWNStableLayerFunction:
     """Thresholded lookup with the gradient-stabilised backward: the EFD sum weighted 1/(h+1) and
     multiplied, like the table gradient, by the node's gradient scale (dwn_stable_node.py:36-206).
     `scale` is a device tensor [N] (one value per node); it gets no gradient, as in the reference."""
 
     @staticmethod
-    def forward(ctx, x, luts, scale, plan):
+    def apply(x, luts, scale, plan):
         nat.require_device(x, luts, scale)
-        x, luts = _f32(x), _f32(luts)
-        scale = _f32(scale.detach()).reshape(-1)
-        if scale.numel() != luts.shape[0]:
-            raise RuntimeError(f"gradient_scale has {scale.numel()} entries for {luts.shape[0]} nodes")
-        y, saved, dims = _dwn_lookup(x, luts, plan)
-        ctx.save_for_backward(luts, saved, scale, x if _backward_reads_x(*dims[2:]) else None)
-        ctx.plan, ctx.dims = plan, dims
-        return y
-
-    @staticmethod
-    def backward(ctx, gy):
-        luts, saved, scale, x = ctx.saved_tensors
-        B, I, N, k, O = ctx.dims
-        plan = ctx.plan
-        gy = _f32(gy)
-        lib = nat.lib()
-        gx = torch.empty((B, I), dtype=torch.float32, device=gy.device) if ctx.needs_input_grad[0] else None
-        gl = torch.empty_like(luts)
-        ws = _bytes(lib.dl_dwn_bwd_workspace_bytes(*ctx.dims), gy.device)
-        nat.check(lib.dl_dwn_stable_layer_bwd(nat.ptr(x), nat.ptr(saved), nat.ptr(plan.idx32), nat.ptr(plan.inv_ptr),
-                                              nat.ptr(plan.inv_pos), nat.ptr(luts), nat.ptr(gy), nat.ptr(scale),
-                                              nat.ptr(gx), nat.ptr(gl), nat.ptr(ws), ws.numel(), *ctx.dims,
-                                              nat.stream()))
-        return gx, gl, None, None
+        return nat.host().dwn_stable_layer(x, luts, scale, plan.host)
 
 
-class HybridLayerFunction(torch.autograd.Function):
+class HybridLayerFunction:
     """Thresholded lookup forward, probabilistic backward on the real-valued inputs (hybrid_node.py:33-204).  Where a
     backward will follow (`keep_tiles`), the forward re-tiles x for it in the pass that thresholds it."""
 
     @staticmethod
-    def forward(ctx, x, luts, plan, keep_tiles=True):
+    def apply(x, luts, plan, keep_tiles=True):
         nat.require_device(x, luts)
-        x, luts = _f32(x), _f32(luts)
-        tiles = None
-        if keep_tiles and plan.k <= FAST_K:
-            dims = _lookup_dims(x, luts, plan)
-            B, _, N, _, O = dims
-            lib = nat.lib()
-            y = torch.empty((B, N * O), dtype=torch.float32, device=x.device)
-            tiles = _bytes(lib.dl_hybrid_saved_bytes(*dims), x.device)
-            ws = _bytes(lib.dl_hybrid_fwd_workspace_bytes(*dims), x.device)
-            nat.check(lib.dl_hybrid_layer_fwd(nat.ptr(x), nat.ptr(plan.idx32), nat.ptr(luts), nat.ptr(y), nat.ptr(tiles),
-                                              tiles.numel(), nat.ptr(ws), ws.numel(), *dims, nat.stream()))
-        else:
-            y, _, dims = _dwn_lookup(x, luts, plan)
-        # the backward reads x itself only where it was not re-tiled
-        ctx.save_for_backward(None if tiles is not None and tiles.numel() > 256 else x, luts, tiles)
-        ctx.plan, ctx.dims = plan, dims
-        return y
-
-    @staticmethod
-    def backward(ctx, gy):
-        x, luts, tiles = ctx.saved_tensors
-        B, I, N, k, O = ctx.dims
-        plan = ctx.plan
-        gy = _f32(gy)
-        lib = nat.lib()
-        gx = torch.empty((B, I), dtype=torch.float32, device=gy.device) if ctx.needs_input_grad[0] else None
-        gl = torch.empty_like(luts)
-        if tiles is None:
-            ws = _bytes(lib.dl_hybrid_bwd_workspace_bytes(*ctx.dims), gy.device)
-            nat.check(lib.dl_hybrid_layer_bwd(nat.ptr(x), nat.ptr(plan.idx32), nat.ptr(plan.inv_ptr), nat.ptr(plan.inv_pos),
-                                              nat.ptr(luts), nat.ptr(gy), nat.ptr(gx), nat.ptr(gl), nat.ptr(ws), ws.numel(),
-                                              *ctx.dims, nat.stream()))
-        else:
-            ws = _bytes(lib.dl_hybrid_bwd_saved_workspace_bytes(*ctx.dims), gy.device)
-            nat.check(lib.dl_hybrid_layer_bwd_saved(nat.ptr(x), nat.ptr(tiles), nat.ptr(plan.idx32), nat.ptr(plan.inv_ptr),
-                                                    nat.ptr(plan.inv_pos), nat.ptr(luts), nat.ptr(gy), nat.ptr(gx),
-                                                    nat.ptr(gl), nat.ptr(ws), ws.numel(), *ctx.dims, nat.stream()))
-        return gx, gl, None, None
+        return nat.host().hybrid_layer(x, luts, plan.host, keep_tiles)
 
 
 # ----------------------------------------------------------------------------- Probabilistic
@@ -580,54 +262,16 @@ def _node_temperatures(temperature, N, device):
     return _per_node(temperature, N, device)
 
 
-class ProbLayerFunction(torch.autograd.Function):
+class ProbLayerFunction:
     """y[b, n*O+d] = sum_a sigmoid(raw[n,a,d]/T) prod_j (x_j a_j + (1-x_j)(1-a_j)); `temperature` is a number for the
     whole layer or a tensor [N] with every node's own value."""
 
     @staticmethod
-    def forward(ctx, x, raw, plan, temperature):
+    def apply(x, raw, plan, temperature):
         nat.require_device(x, raw)
-        x, raw = _f32(x), _f32(raw)
-        B, I = x.shape
-        N, L, O = raw.shape
-        k = plan.k
-        if (N, 1 << k, I) != (plan.N, L, plan.I):
-            raise RuntimeError(f"shape mismatch: x {tuple(x.shape)}, raw_weights {tuple(raw.shape)}, mapping "
-                               f"[{plan.N},{k}] over {plan.I} inputs")
-        y = torch.empty((B, N * O), dtype=torch.float32, device=x.device)
-        dims = (B, I, N, k, O)
-        saved = _bytes(nat.lib().dl_prob_saved_bytes(*dims), x.device)
-        T = _node_temperatures(temperature, N, x.device)
-        if T is None:
-            nat.check(nat.lib().dl_prob_layer_fwd(nat.ptr(x), nat.ptr(plan.idx32), nat.ptr(raw), float(temperature),
-                                                  nat.ptr(y), nat.ptr(saved), saved.numel(), *dims, nat.stream()))
-        else:
-            nat.check(nat.lib().dl_prob_layer_fwd_nodes(nat.ptr(x), nat.ptr(plan.idx32), nat.ptr(raw), nat.ptr(T),
-                                                        nat.ptr(y), nat.ptr(saved), saved.numel(), *dims, nat.stream()))
-        ctx.save_for_backward(x, raw, saved, T)
-        ctx.plan, ctx.T, ctx.dims = plan, None if T is not None else float(temperature), dims
-        return y
-
-    @staticmethod
-    def backward(ctx, gy):
-        x, raw, saved, T = ctx.saved_tensors
-        plan = ctx.plan
-        gy = _f32(gy)
-        lib = nat.lib()
-        B, I = x.shape
-        gx = torch.empty((B, I), dtype=torch.float32, device=gy.device) if ctx.needs_input_grad[0] else None
-        graw = torch.empty_like(raw)
-        ws = _bytes(lib.dl_prob_bwd_saved_workspace_bytes(*ctx.dims), gy.device)
-        if T is None:
-            nat.check(lib.dl_prob_layer_bwd(nat.ptr(x), nat.ptr(saved), nat.ptr(plan.idx32), nat.ptr(plan.inv_ptr),
-                                            nat.ptr(plan.inv_pos),
-                                            nat.ptr(raw), ctx.T, nat.ptr(gy), nat.ptr(gx), nat.ptr(graw), nat.ptr(ws),
-                                            ws.numel(), *ctx.dims, nat.stream()))
-        else:
-            nat.check(lib.dl_prob_layer_bwd_nodes(nat.ptr(x), nat.ptr(saved), nat.ptr(plan.idx32), nat.ptr(plan.inv_ptr),
-                                                  nat.ptr(plan.inv_pos), nat.ptr(raw), nat.ptr(T), nat.ptr(gy), nat.ptr(gx),
-                                                  nat.ptr(graw), nat.ptr(ws), ws.numel(), *ctx.dims, nat.stream()))
-        return gx, graw, None, None
+        if torch.is_tensor(temperature):
+            return nat.host().prob_layer(x, raw, plan.host, temperature, 0.0)
+        return nat.host().prob_layer(x, raw, plan.host, None, temperature)
 
 
 def prob_layer_eval(x, raw, plan, temperature):
@@ -652,42 +296,14 @@ def prob_layer_eval(x, raw, plan, temperature):
 
 
 # ----------------------------------------------------------------------------- Learnable mapping
-class SoftMapFunction(torch.autograd.Function):
+class SoftMapFunction:
     """m = x @ softmax(W / tau, dim=-1).T.  The softmax numerators are kept as bf16 planes from forward to backward: 6 bytes per
     entry of W with fp32 operands (precision 0), 2 with bf16."""
 
     @staticmethod
-    def forward(ctx, x, W, tau, precision):
+    def apply(x, W, tau, precision):
         nat.require_device(x, W)
-        x, W = _f32(x), _f32(W)
-        B, I = x.shape
-        M = W.shape[0]
-        if W.shape[1] != I:
-            raise RuntimeError(f"shape mismatch: x {tuple(x.shape)} vs W {tuple(W.shape)}")
-        lib = nat.lib()
-        m = torch.empty((B, M), dtype=torch.float32, device=x.device)
-        stats = _bytes(lib.dl_soft_map_saved_bytes(B, I, M, precision), x.device)
-        ws = _bytes(lib.dl_soft_map_workspace_bytes(B, I, M, precision), x.device)
-        nat.check(lib.dl_soft_map_fwd(nat.ptr(x), nat.ptr(W), float(tau), nat.ptr(m), nat.ptr(stats), nat.ptr(ws),
-                                      ws.numel(), B, I, M, precision, nat.stream()))
-        ctx.save_for_backward(x, W, m, stats)
-        ctx.tau, ctx.precision = float(tau), precision
-        return m
-
-    @staticmethod
-    def backward(ctx, gm):
-        x, W, m, stats = ctx.saved_tensors
-        gm = _f32(gm)
-        B, I = x.shape
-        M = W.shape[0]
-        lib = nat.lib()
-        gx = torch.empty_like(x)
-        gW = torch.empty_like(W)
-        ws = _bytes(lib.dl_soft_map_workspace_bytes(B, I, M, ctx.precision), x.device)
-        nat.check(lib.dl_soft_map_bwd(nat.ptr(x), nat.ptr(W), ctx.tau, nat.ptr(m), nat.ptr(stats), nat.ptr(gm),
-                                      nat.ptr(gx), nat.ptr(gW), nat.ptr(ws), ws.numel(), B, I, M, ctx.precision,
-                                      nat.stream()))
-        return gx, gW, None, None
+        return nat.host().soft_map(x, W, tau, precision)
 
 
 def row_argmax(W):
@@ -739,31 +355,14 @@ def thermometer_encode(x, thresholds):
     return bits
 
 
-class CrossEntropyFunction(torch.autograd.Function):
+class CrossEntropyFunction:
     """Mean cross-entropy of [B, C] logits against int64 class labels: loss and its gradient from one pass
     (what torch.nn.functional.cross_entropy and its backward compute for the logits GroupSum returns)."""
 
     @staticmethod
-    def forward(ctx, logits, labels):
+    def apply(logits, labels):
         nat.require_device(logits, labels)
-        logits = _f32(logits)
-        if logits.dim() != 2 or labels.shape != (logits.shape[0],):
-            raise RuntimeError(f"expected logits [B, C] and labels [B], got {tuple(logits.shape)} and {tuple(labels.shape)}")
-        labels = labels.to(torch.int64).contiguous()
-        B, C = logits.shape
-        lib = nat.lib()
-        loss = torch.empty((), dtype=torch.float32, device=logits.device)
-        glogits = torch.empty_like(logits)
-        ws = _bytes(lib.dl_cross_entropy_workspace_bytes(B), logits.device)
-        nat.check(lib.dl_cross_entropy(nat.ptr(logits), nat.ptr(labels), nat.ptr(loss), nat.ptr(glogits), nat.ptr(ws),
-                                       ws.numel(), B, C, nat.stream()))
-        ctx.save_for_backward(glogits)
-        return loss
-
-    @staticmethod
-    def backward(ctx, gloss):
-        (glogits,) = ctx.saved_tensors
-        return glogits * gloss, None
+        return nat.host().cross_entropy(logits, labels)
 
 
 class GroupSumFunction(torch.autograd.Function):

@@ -6,7 +6,6 @@ model with ONE kernel launch per step (`dl_adam_step`): the same arithmetic as t
 (bias-corrected first and second moments, optional L2 weight decay, `maximize`).  CPU tensors, other dtypes and sparse
 cases take plain torch operations with the same formula.
 """
-import ctypes
 import math
 
 import torch
@@ -68,12 +67,6 @@ class BankAdam(torch.optim.Optimizer):
         by_device = {}
         for item in batch:
             by_device.setdefault(item[0].device, []).append(item)
-        for device, items in by_device.items():
-            count = len(items)
-            ptrs = [(ctypes.c_void_p * count)(*[t[i].data_ptr() for t in items]) for i in range(4)]
-            numel = (ctypes.c_longlong * count)(*[t[0].numel() for t in items])
-            with torch.cuda.device(device):
-                nat.check(nat.lib().dl_adam_step(ptrs[0], ptrs[1], ptrs[2], ptrs[3], numel, count, float(group["lr"]),
-                                                 float(group["betas"][0]), float(group["betas"][1]), float(group["eps"]),
-                                                 float(group["weight_decay"]), int(step), int(bool(group["maximize"])),
-                                                 nat.stream()))
+        for items in by_device.values():
+            nat.host().adam_step(items, group["lr"], *group["betas"], group["eps"], group["weight_decay"], step,
+                                 bool(group["maximize"]))
