@@ -1,5 +1,5 @@
 // LearnableLayer soft connectivity on gfx950:  m = x * softmax(W / tau)^T  and its adjoint, on the
-// bf16 matrix cores with fp32 accumulation (v_mfma_f32_32x32x16_bf16).
+// 16-bit matrix cores with fp32 accumulation (v_mfma_f32_32x32x16_bf16, ..._f16).
 //
 //   forward   m[b,o]  = rs[o] * sum_i x[b,i] E[o,i]          E = exp((W - max)/tau), rs = 1 / row sum
 //   backward  gx[b,i] = sum_o gs[b,o] E[o,i]                  gs = gm * rs
@@ -17,6 +17,16 @@
 // Where a sum of an operand's size could overflow with that factor, or as the sum before rs, while the result does not, and
 // for infinities and NaN, which planes do not carry, the product is computed with fp32 multiply-adds instead
 // (softmap_plain): the pack pass notes the largest magnitude (softmap_note_large).
+// Pairs.  Large products of precision 0 (SM_PAIR_WORK) take half as many matrix operations: an operand, scaled by a power of two
+// to below 2^15, is hi + 2^-11 lo with hi its rounding to fp16 and lo that of 2^11 times the rest, and a product is hi*hi +
+// 2^-11 (hi*lo + lo*hi), the second part in a sum of its own.  Down to 2^-27 of what the scale is taken from both halves are
+// normal numbers, the pair holds 23 bits or more and the product left out is below 2^-24 of |a*b|; smaller values keep an absolute
+// error of 2^-50 of it.  E is scaled by its row maximum, which is one, x by its largest value; where a value of either that is
+// not zero lies below 2^-27 of that, decided on the device, the products it is in take the planes (launches of either
+// kind that are not to run end at once): with W of N(0, 6) at tau 1, where E spans more, the forward and gx.  gs is scaled row by row and gm column by column, so that no output row answers for
+// another's magnitude, and need no such bound: their smallest values meet an E and an x within theirs.  Error against float64
+// (2-norm) of m / gx / gW, 512 x 3136 x 48000, W of N(0, 1.5), tau 1: 1.1e-7 / 1.7e-7 / 4.3e-7 with pairs, 5.3e-7 / 3.2e-7 /
+// 11.8e-7 with planes: half as many additions, and the sums of groups of stages (below).
 //
 // Layout.  An MFMA lane wants 8 consecutive reduction steps of one row: a "unit" of 16 bytes.  Every operand is stored
 // as [reduction / 8][rows] units, rows padded to whole tiles with zeros, by the pass that has it in registers anyway
@@ -34,6 +44,9 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
+typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
+typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
 typedef short shortx4 __attribute__((ext_vector_type(4)));
 typedef short shortx8 __attribute__((ext_vector_type(8)));
 
@@ -72,6 +85,129 @@ __device__ __forceinline__ uint4 softmap_unit(float *v) {
     return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
+// ---- pairs: eight values, scaled to below 2^15, as a unit of hi = fp16(v) and one of lo = fp16(2^11 (v - hi))
+#define SM_PAIR_EXP 14          // exponent that an operand's largest value is scaled to
+#define SM_PAIR_LO 0x1p11f
+#define SM_PAIR_TURN 8          // stages of a group
+#define SM_PAIR_RANGE 0x1p-27f  // of the largest: above it both halves of a pair are normal numbers
+
+__device__ __forceinline__ void softmap_pair(const float *v, uint4 &hi, uint4 &lo) {
+    unsigned h[4], l[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const floatx2 a = {v[2 * j], v[2 * j + 1]};
+        const halfx2 t = __builtin_convertvector(a, halfx2);
+        const floatx2 r = {(v[2 * j] - (float)t[0]) * SM_PAIR_LO, (v[2 * j + 1] - (float)t[1]) * SM_PAIR_LO};
+        h[j] = __builtin_bit_cast(unsigned, t);
+        l[j] = __builtin_bit_cast(unsigned, __builtin_convertvector(r, halfx2));
+    }
+    hi = make_uint4(h[0], h[1], h[2], h[3]);
+    lo = make_uint4(l[0], l[1], l[2], l[3]);
+}
+// power of two that takes values of up to this magnitude (its bits) below 2^15
+__device__ __forceinline__ int softmap_pair_shift(unsigned largest) { return SM_PAIR_EXP + 127 - (int)(largest >> 23); }
+
+// What the choice between pairs and planes rests on, kept with the statistics: magnitudes of x, as bits, and whether a row of
+// E spans more than the pairs carry.
+struct SoftmapRange {
+    unsigned x_largest, x_smallest, e_wide;  // x_smallest: of the values that are not zero
+};
+__device__ __forceinline__ bool softmap_x_wide(const SoftmapRange *r) {
+    // (an infinity or a NaN among x as well: both sides are positive, and bits of positive floats compare as they do)
+    return !(__uint_as_float(r->x_smallest) >= __uint_as_float(r->x_largest) * SM_PAIR_RANGE);
+}
+__device__ __forceinline__ bool softmap_wide(const SoftmapRange *r) { return r->e_wide != 0 || softmap_x_wide(r); }
+
+__global__ __launch_bounds__(256) void softmap_clear(SoftmapRange *range, unsigned *words, int n) {
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (range && e == 0) { range->x_largest = 0; range->x_smallest = 0x7f7fffffu; range->e_wide = 0; }
+    if (e < n) words[e] = 0;
+}
+
+// The range of x: 512 x 3136 in 11 us.
+__global__ __launch_bounds__(256) void softmap_scan_x(const float *__restrict__ x, long long total, SoftmapRange *range) {
+    unsigned big = 0, small = 0x7f7fffffu;
+    // eight loads in flight; past the end the last value again
+    for (long long e = (long long)blockIdx.x * 2048 + threadIdx.x; e < total; e += (long long)gridDim.x * 2048) {
+        unsigned v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = __float_as_uint(x[e + 256 * q < total ? e + 256 * q : total - 1]) & 0x7fffffffu;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            big = max(big, v[q]);
+            small = min(small, v[q] != 0 ? v[q] : small);
+        }
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        big = max(big, (unsigned)__shfl_xor((int)big, off));
+        small = min(small, (unsigned)__shfl_xor((int)small, off));
+    }
+    __shared__ unsigned part[2][4];
+    if ((threadIdx.x & 63) == 0) { part[0][threadIdx.x >> 6] = big; part[1][threadIdx.x >> 6] = small; }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int q = 1; q < 4; ++q) { big = max(big, part[0][q]); small = min(small, part[1][q]); }
+        // (atomics on one word queue up: most blocks see that they change nothing)
+        if (big > __hip_atomic_load(&range->x_largest, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(&range->x_largest, big);
+        if (small < __hip_atomic_load(&range->x_smallest, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(&range->x_smallest, small);
+    }
+}
+
+// Largest magnitudes, as bits: of every column of gm, of every row of gs = gm * rs, and of gm.  A wavefront has 16 rows of 64
+// columns at a time and goes over SM_SCAN_TILES such tiles of its rows.  512 x 48000 in 40 us, 2.5 TB/s.
+#define SM_SCAN_TILES 4
+__global__ __launch_bounds__(256) void softmap_scan_grad(const float *__restrict__ gm, const float *__restrict__ rs,
+                                                         unsigned *__restrict__ row_max, unsigned *__restrict__ col_max,
+                                                         unsigned *__restrict__ largest, const SoftmapRange *__restrict__ range,
+                                                         int R, int C, int strips) {
+    if (softmap_x_wide(range)) return;  // then nothing of gm goes into pairs
+    const int lane = threadIdx.x & 63, wave = dl_uniform(threadIdx.x >> 6);
+    const int r0 = (int)(blockIdx.x / strips) * 64 + wave * 16, c_first = (int)(blockIdx.x % strips) * (64 * SM_SCAN_TILES) + lane;
+    __shared__ unsigned cols[64 * SM_SCAN_TILES];
+    cols[threadIdx.x] = 0;
+    __syncthreads();
+    unsigned rows[16], big = 0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) rows[i] = 0;
+    // every load in flight at once; past the ends the last row or column again, whose maxima nobody reads there
+    float v[SM_SCAN_TILES][16], f[SM_SCAN_TILES];
+#pragma unroll
+    for (int t = 0; t < SM_SCAN_TILES; ++t) {
+        const int col = min(c_first + t * 64, C - 1);
+        f[t] = rs[col];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[t][i] = gm[(size_t)min(r0 + i, R - 1) * C + col];
+    }
+#pragma unroll
+    for (int t = 0; t < SM_SCAN_TILES; ++t) {
+        unsigned cb = 0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            cb = max(cb, __float_as_uint(v[t][i]) & 0x7fffffffu);
+            rows[i] = max(rows[i], __float_as_uint(v[t][i] * f[t]) & 0x7fffffffu);
+        }
+        atomicMax(&cols[t * 64 + lane], cb);
+        big = max(big, cb);
+    }
+    // the maxima over the lanes, halving the rows a lane has at each of four steps: lane l ends with row l / 4
+#pragma unroll
+    for (int half = 8, off = 32; half > 0; half >>= 1, off >>= 1)
+#pragma unroll
+        for (int i = 0; i < half; ++i) {
+            const bool up = (lane & off) != 0;
+            const unsigned keep = up ? rows[i + half] : rows[i], give = up ? rows[i] : rows[i + half];
+            rows[i] = max(keep, (unsigned)__shfl_xor((int)give, off));
+        }
+    rows[0] = max(rows[0], (unsigned)__shfl_xor((int)rows[0], 2));
+    rows[0] = max(rows[0], (unsigned)__shfl_xor((int)rows[0], 1));
+    if ((lane & 3) == 0 && rows[0] > __hip_atomic_load(row_max + r0 + (lane >> 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(row_max + r0 + (lane >> 2), rows[0]);
+    __syncthreads();
+    if (cols[threadIdx.x] != 0) atomicMax(col_max + (int)(blockIdx.x % strips) * (64 * SM_SCAN_TILES) + threadIdx.x, cols[threadIdx.x]);
+    for (int off = 32; off > 0; off >>= 1) big = max(big, (unsigned)__shfl_xor((int)big, off));
+    if (lane == 0 && big > __hip_atomic_load(largest, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(largest, big);
+}
+
 // Largest magnitude of an operand, as bits (a NaN is larger than all); stays 0 while every value is below SM_LARGE, which is
 // why the word is hardly ever written.  `big`: the bits of this thread's largest.
 __device__ __forceinline__ void softmap_note_large(unsigned *largest, unsigned big) {
@@ -91,11 +227,16 @@ __device__ __forceinline__ float softmap_largest(const unsigned *largest) {
 // between the three steps (NQ values per row and thread), so T * NQ bounds the width; wider rows (NQ = 0) are read
 // three times.  With one plane the sum is that of the rounded values.  Blocks past the last row and columns past I write zeros
 // (the padding the products read).
+// NP = 2: pairs; a block whose rows span more than pairs carry sets e_wide instead, and blocks that find it set, or x too wide,
+// end.  NP = 3 with a range: the launch behind that one, which writes planes where it has come to that.
 template <int NP, int T, int NQ>
-__global__ __launch_bounds__(T) void softmap_rowstats(const float *__restrict__ W, float scale, float *__restrict__ mxs,
+__global__ __launch_bounds__(T, NQ == 8 ? 4 : 1) void softmap_rowstats(const float *__restrict__ W, float scale, float *__restrict__ mxs,
                                                       float *__restrict__ rss, char *__restrict__ E, size_t plane, int M,
-                                                      int I, int Ip, unsigned *__restrict__ largest) {
+                                                      int I, int Ip, unsigned *__restrict__ largest,
+                                                      SoftmapRange *__restrict__ range) {
     constexpr int WV = T / 64;
+    if (NP == 2 && (softmap_x_wide(range) || __hip_atomic_load(&range->e_wide, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) return;
+    if (NP == 3 && range && !softmap_wide(range)) return;
     __shared__ float red[2][8][WV];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int o0 = blockIdx.x * 8;
@@ -135,14 +276,29 @@ __global__ __launch_bounds__(T) void softmap_rowstats(const float *__restrict__ 
         const float e = i < I && o0 + j < M ? softmap_e(w, mx[j], scale) : 0.0f;
         return NP == 1 ? softmap_lo(softmap_pk_bf16(e, 0.0f)) : e;
     };
+    bool bad = false;
+    auto look = [&](const float *e) {  // (zeros are exact in both; a NaN is too wide)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) bad |= !(e[j] >= SM_PAIR_RANGE) && e[j] != 0.0f;
+    };
     auto store = [&](int i, float *e) {
         if (i < Ip) {
+            if (NP == 2) {
+                look(e);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) e[j] *= (float)(1 << SM_PAIR_EXP);
+                uint4 hi, lo;
+                softmap_pair(e, hi, lo);
+                *reinterpret_cast<uint4 *>(out + i) = hi;
+                *reinterpret_cast<uint4 *>(reinterpret_cast<char *>(out + i) + plane) = lo;
+                return;
+            }
             if (NP > 1) {
 #pragma unroll
                 for (int j = 0; j < 8; ++j) e[j] *= SM_SCALE;
             }
 #pragma unroll
-            for (int p = 0; p < NP; ++p)
+            for (int p = 0; p < (NP == 1 ? 1 : 3); ++p)
                 *reinterpret_cast<uint4 *>(reinterpret_cast<char *>(out + i) + p * plane) = softmap_unit(e);
         }
     };
@@ -162,6 +318,7 @@ __global__ __launch_bounds__(T) void softmap_rowstats(const float *__restrict__ 
             store(i, e);
         }
     }
+    if (NP == 2 && __ballot(bad) != 0 && lane == 0) atomicOr(&range->e_wide, 1u);
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         for (int off = 32; off > 0; off >>= 1) sum[j] += __shfl_xor(sum[j], off);
@@ -187,14 +344,19 @@ __global__ __launch_bounds__(T) void softmap_rowstats(const float *__restrict__ 
 // dots[chunk][c] = sum of src * other over the 64 rows of the chunk (unscaled; the reader adds the chunks in order).
 // Block = 64 columns x 64 rows: a thread has sixteen rows of a column, so units along the rows leave straight from registers;
 // those along the columns go through the LDS (row stride 65 words, no conflicts).  `largest` (three planes; nullable): see
-// softmap_note_large; `clear` (nullable): such a word that a later launch fills.  `alternate` (three planes): factor of every
-// second group of SM_GX_STAGE columns in the units along the columns.
+// softmap_note_large; `clear` (nullable): such a word that a later launch fills.  `alternate` (three planes): factor of
+// every second group of SM_GX_STAGE columns in the units along the columns.
+// NP = 2: pairs, or planes where `range` says so: units along the rows are gW's, which takes E from W and asks for x's range only.
+// `row_max` (units along the columns) and `col_max` (units along the rows): the magnitudes that the pairs are scaled by, without
+// them x_largest.
 template <int NP>
 __global__ __launch_bounds__(256) void softmap_pack(const float *__restrict__ src, const float *__restrict__ colscale,
                                                     const float *__restrict__ other, float *__restrict__ dots,
                                                     char *__restrict__ rows8, size_t rows_plane, char *__restrict__ cols8,
                                                     size_t cols_plane, int R, int C, int Rp, int Cp, float alternate, unsigned *__restrict__ largest,
-                                                    unsigned *__restrict__ clear) {
+                                                    unsigned *__restrict__ clear, const SoftmapRange *__restrict__ range,
+                                                    const unsigned *__restrict__ row_max, const unsigned *__restrict__ col_max) {
+    const bool row_pairs = NP == 2 && !softmap_x_wide(range), col_pairs = NP == 2 && !softmap_wide(range);
     // (a grid of one dimension: the second holds 65535 blocks, 4.19 million rows)
     const int cb64 = Cp / 64, bx = blockIdx.x % cb64, by = blockIdx.x / cb64;
     if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0;
@@ -204,7 +366,7 @@ __global__ __launch_bounds__(256) void softmap_pack(const float *__restrict__ sr
     const int col = bx * 64 + c, r0 = by * 64;
     float v[16], dot = 0.0f;
     float f = colscale && col < C ? colscale[col] : 1.0f;
-    if (NP > 1 && (col / SM_GX_STAGE) % 2 != 0) f *= alternate;
+    if (NP > 1 && !col_pairs && (col / SM_GX_STAGE) % 2 != 0) f *= alternate;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
         const int r = r0 + g * 16 + i;
@@ -223,22 +385,39 @@ __global__ __launch_bounds__(256) void softmap_pack(const float *__restrict__ sr
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             big = max(big, __float_as_uint(v[i]) & 0x7fffffffu);
-            v[i] *= SM_SCALE;
+            if (NP == 3) v[i] *= SM_SCALE;
         }
-        if (largest) softmap_note_large(largest, big);
+        if (largest && !row_pairs) softmap_note_large(largest, big);
     }
 #pragma unroll
     for (int i = 0; i < 16; ++i) tile[g * 16 + i][c] = v[i] * f;
     __syncthreads();
     if (other && g == 0) dots[(size_t)by * Cp + col] = ((part[0][c] + part[1][c]) + part[2][c]) + part[3][c];
+    auto put_pairs = [&](float *w, unsigned biggest, char *d, size_t plane) {
+        const int shift = softmap_pair_shift(biggest);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) w[j] = __builtin_amdgcn_ldexpf(w[j], shift);
+        uint4 hi, lo;
+        softmap_pair(w, hi, lo);
+        *reinterpret_cast<uint4 *>(d) = hi;
+        *reinterpret_cast<uint4 *>(d + plane) = lo;
+    };
     if (rows8) {
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int rb = (r0 >> 3) + g * 2 + h;
             if (8 * rb < Rp) {
                 char *d = rows8 + ((size_t)rb * Cp + col) * SM_UNIT;
+                if (row_pairs) {
+                    put_pairs(v + 8 * h, col_max ? col_max[col] : range->x_largest, d, rows_plane);
+                    continue;
+                }
+                if (NP == 2) {
 #pragma unroll
-                for (int p = 0; p < NP; ++p) *reinterpret_cast<uint4 *>(d + p * rows_plane) = softmap_unit(v + 8 * h);
+                    for (int j = 0; j < 8; ++j) v[8 * h + j] *= SM_SCALE;
+                }
+#pragma unroll
+                for (int p = 0; p < (NP == 1 ? 1 : 3); ++p) *reinterpret_cast<uint4 *>(d + p * rows_plane) = softmap_unit(v + 8 * h);
             }
         }
     }
@@ -251,8 +430,16 @@ __global__ __launch_bounds__(256) void softmap_pack(const float *__restrict__ sr
 #pragma unroll
                 for (int j = 0; j < 8; ++j) w[j] = tile[c][cb * 8 + j];
                 char *d = cols8 + ((size_t)(bx * 8 + cb) * Rp + row) * SM_UNIT;
+                if (col_pairs) {
+                    put_pairs(w, row_max ? row_max[row] : range->x_largest, d, cols_plane);
+                    continue;
+                }
+                if (NP == 2) {
 #pragma unroll
-                for (int p = 0; p < NP; ++p) *reinterpret_cast<uint4 *>(d + p * cols_plane) = softmap_unit(w);
+                    for (int j = 0; j < 8; ++j) w[j] *= SM_SCALE;
+                }
+#pragma unroll
+                for (int p = 0; p < (NP == 1 ? 1 : 3); ++p) *reinterpret_cast<uint4 *>(d + p * cols_plane) = softmap_unit(w);
             }
         }
     }
@@ -262,7 +449,9 @@ __global__ __launch_bounds__(256) void softmap_pack(const float *__restrict__ sr
 // result is rounded once however many chunks there are (bound by the reads: no slower).
 template <int VEC>
 __global__ __launch_bounds__(256) void softmap_reduce_chunks(const float *__restrict__ part, float *__restrict__ out,
-                                                              long long total, int chunks) {
+                                                              long long total, int chunks, const SoftmapRange *range, int wide_chunks) {
+    if (range && softmap_wide(range)) chunks = wide_chunks;
+    if (range && chunks == 1) return;  // it is in `out`
     const long long e = ((long long)blockIdx.x * 256 + threadIdx.x) * VEC;
     if (e >= total) return;
     if (VEC == 4) {
@@ -303,6 +492,9 @@ struct SoftmapArgs {
     int lde;
     float scale, inv_tau;
     bool vec_out;             // W and out start on 16-byte boundaries
+    // pairs
+    const SoftmapRange *range;
+    const unsigned *row_max;  // magnitudes that the rows of A are scaled by; forward: none (x_largest)
 };
 
 // Loads that bypass the registers: lane l's 16 bytes at base + voff land at LDS address lds + 16 l.  The compiler does not
@@ -333,16 +525,24 @@ __device__ __forceinline__ void softmap_stage_barrier() {
 // per MFMA a block pulls 24 KB per 32 reduction steps (NP = 1), 48 bytes per clock and CU at the matrix peak where
 // 128 x 128 tiles need 64, all that an L2 channel delivers.  Two blocks share a CU (accumulators 128 registers, 72 KB of LDS
 // each), so one block's MFMAs run under the other's barriers and stores.  Stages are KC deep, NBUF of them in the LDS.
+// Pairs (NP = 2): 128 x 128 tiles, because hi*hi and the rest have accumulators of their own (64 registers each) and the loop has
+// no vector arithmetic but the sign below; three blocks share a CU for gW, whose epilogue is two thirds memory (575 us; 704 with
+// two).  Forward and gx add the sums of SM_PAIR_TURN stages to running ones, signs turned from group to group for the reason
+// given above, and have two blocks per CU.  The same sizes, forward / gx / gW: 503 / 473 / 575 us (planes 703 / 786 / 866).  Bound by power: the matrix cores are busy half of the time at 1.8 GHz.  256 x 128 tiles with one accumulator, the
+// rest's sum scaled and added by every stage: 514 / 560 / 668.  gx in
+// 5, 10 or 15 chunks of the reduction: 445, 486 and 497 with their sum; 10 for the shorter running sums.
 template <int MODE, int NP, int FA>
 __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
+    extern __shared__ __align__(16) char lds[];
+    if (NP > 1 && g.range && dl_uniform(MODE == 2 ? softmap_x_wide(g.range) : softmap_wide(g.range)) != (NP == 3)) return;
     constexpr int TR = 64 * FA, TC = SM_TC;
     constexpr int KC = NP == 1 ? 32 : SM_GX_STAGE, KB = KC / 8;
     constexpr int NBUF = NP == 3 && FA == 4 ? 2 : 3, AHEAD = NBUF - 1;
     constexpr int A_BYTES = NP * TR * KC * 2, STAGE = NP * (TR + TC) * KC * 2;
     constexpr bool BY_STAGE = NP == 3 && MODE == 1;
+    static_assert(NP != 2 || FA == 2, "pairs keep two sums per output");
     constexpr int NA = NP * KB * (TR / 64) / 4, NB = NP * KB * (TC / 64) / 4;  // loads per wavefront and stage
     static_assert(NP * KB * (TR / 64) % 4 == 0 && NP * KB * (TC / 64) % 4 == 0, "whole loads per wavefront");
-    extern __shared__ __align__(16) char lds[];
     typedef __attribute__((address_space(3))) char lds_char;
     const unsigned lds_base = (unsigned)(uintptr_t)(lds_char *)lds;  // what softmap_to_lds counts from
     int inner, outer;
@@ -395,6 +595,22 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
 
+    // pairs: the products with a lower half, times 2^11, and the sums of earlier groups of stages
+    constexpr int FP = NP == 2 ? FA : 1;
+    constexpr bool GROUPS = NP == 2 && MODE != 2;
+    floatx16 low[FP][2], sum[GROUPS ? FP : 1][2];
+    if (NP == 2) {
+#pragma unroll
+        for (int i = 0; i < FP; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    low[i][j][v] = 0.0f;
+                    if (GROUPS) sum[i][j][v] = 0.0f;
+                }
+    }
+
     const int kh = lane >> 5, l32 = lane & 31;
     const unsigned a_rd = (kh * TR + wm + l32) * SM_UNIT;
     unsigned b_rd;
@@ -405,7 +621,7 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
     } else {
         b_rd = A_BYTES + (kh * TC + wn + l32) * SM_UNIT;
     }
-    auto compute = [&](int buf, float sign) __attribute__((always_inline)) {
+    auto compute = [&](int buf, float sign, unsigned turn) __attribute__((always_inline)) {
         const unsigned base = buf * STAGE;
 #pragma unroll
         for (int kk = 0; kk < KC / 16; ++kk) {
@@ -430,7 +646,21 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
             }
             // small products first
             constexpr int PA[6] = {0, 2, 1, 0, 1, 0}, PB[6] = {2, 0, 1, 1, 0, 0};
-            if (BY_STAGE) {
+            if (NP == 2) {
+#pragma unroll
+                for (int i = 0; i < FA; ++i) {
+                    const uintx4 turned = __builtin_bit_cast(uintx4, a[0][i]) ^ (GROUPS ? turn : 0u);
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        const halfx8 ah = __builtin_bit_cast(halfx8, a[0][i]), al = __builtin_bit_cast(halfx8, a[NP - 1][i]);
+                        const halfx8 bh = __builtin_bit_cast(halfx8, b[0][j]), bl = __builtin_bit_cast(halfx8, b[NP - 1][j]);
+                        floatx16 &c = low[i % FP][j];
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(halfx8, turned), bh, acc[i][j], 0, 0, 0);
+                        c = __builtin_amdgcn_mfma_f32_32x32x16_f16(al, bh, c, 0, 0, 0);
+                        c = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah, bl, c, 0, 0, 0);
+                    }
+                }
+            } else if (BY_STAGE) {
 #pragma unroll
                 for (int i = 0; i < FA; ++i) {
                     floatx16 step[2];
@@ -455,7 +685,7 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
                     for (int i = 0; i < FA; ++i)
 #pragma unroll
                         for (int j = 0; j < 2; ++j)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[PA[t]][i], b[PB[t]][j], acc[i][j], 0, 0, 0);
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[PA[t] % NP][i], b[PB[t] % NP][j], acc[i][j], 0, 0, 0);
             }
         }
     };
@@ -464,18 +694,48 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
     for (int s = 0; s < AHEAD; ++s)
         if (s < nst) issue(s, s);
     int buf = 0, nbuf = AHEAD % NBUF;
+    unsigned turn = 0;  // pairs: sign of the group's sums
+    auto add_group = [&]() __attribute__((always_inline)) {
+        const float sign = turn ? -1.0f : 1.0f;
+#pragma unroll
+        for (int i = 0; i < FP; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    sum[GROUPS ? i : 0][j][v] = fmaf(sign, acc[i][j][v], sum[GROUPS ? i : 0][j][v]);
+                    acc[i][j][v] = 0.0f;
+                }
+    };
     for (int s = 0; s < nst; ++s) {
         if (s + AHEAD <= nst) softmap_stage_barrier<(NA + NB) * (AHEAD - 1)>();
         else softmap_stage_barrier<0>();
         if (s + AHEAD < nst) issue(s + AHEAD, nbuf);
-        compute(buf, (s_begin + s) % 2 ? -1.0f : 1.0f);
+        if (GROUPS && s % SM_PAIR_TURN == 0 && s > 0) {
+            add_group();
+            turn ^= 0x80008000u;
+        }
+        compute(buf, (s_begin + s) % 2 ? -1.0f : 1.0f, turn);
         buf = buf + 1 == NBUF ? 0 : buf + 1;
         nbuf = nbuf + 1 == NBUF ? 0 : nbuf + 1;
     }
 
+    if (NP == 2) {
+        if (GROUPS) add_group();
+#pragma unroll
+        for (int i = 0; i < FP; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                    acc[i][j][v] = fmaf(1.0f / SM_PAIR_LO, low[i][j][v], GROUPS ? sum[GROUPS ? i : 0][j][v] : acc[i][j][v]);
+    }
     // accumulator layout of a 32x32 tile: register v of lane l holds row 8*(v/4) + 4*(l/32) + v%4, column l%32:
     // a store instruction writes two whole 128-byte lines
     const int R = g.R, C = g.C;
+    // pairs: shift of the other operand, to be undone with that of the row
+    const int shift = NP != 2 ? 0 : MODE == 0 ? SM_PAIR_EXP + softmap_pair_shift(g.range->x_largest)
+                                  : MODE == 1 ? SM_PAIR_EXP : softmap_pair_shift(g.range->x_largest);
     if (MODE != 2) {
         float *dst = g.out + (size_t)zc * R * C;
 #pragma unroll
@@ -487,7 +747,11 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
 #pragma unroll
                 for (int v = 0; v < 16; ++v) {
                     const int row = r0 + wm + i * 32 + 8 * (v >> 2) + 4 * kh + (v & 3);
-                    if (row < R && col < C) dst[(size_t)row * C + col] = acc[i][j][v] * f;
+                    if (row < R && col < C) {
+                        float o = acc[i][j][v] * f;
+                        if (NP == 2) o = __builtin_amdgcn_ldexpf(o, -(shift + (MODE == 1 ? softmap_pair_shift(g.row_max[row]) : 0)));
+                        dst[(size_t)row * C + col] = o;
+                    }
                 }
         }
     } else {
@@ -500,12 +764,13 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
             rr[tid] = t;
             rr[TR + tid] = g.mx[r0 + tid];
             rr[2 * TR + tid] = g.rs[r0 + tid] * g.inv_tau;
+            if (NP == 2) rr[3 * TR + tid] = __int_as_float(-(shift + softmap_pair_shift(g.row_max[r0 + tid])));
         }
         __syncthreads();
         // 32 rows x 64 columns at a time go through the wavefront's own corner of the LDS, so that a lane owns four consecutive
         // columns of a row: 16-byte stores in runs of 256 bytes
         constexpr int TS = 68;  // floats per staged row: 64 + 4 keeps 16-byte alignment
-        float *stg = rr + 3 * TR + wave * (32 * TS);
+        float *stg = rr + 4 * TR + wave * (32 * TS);
         const int rrow = lane >> 4, c4 = (lane & 15) * 4, col4 = c0 + wn + c4;
         const bool vec = C % 4 == 0 && g.vec_out;
 #pragma unroll
@@ -526,8 +791,13 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
                 for (int q = 0; q < 4; ++q) {
                     const float4 rv = *reinterpret_cast<const float4 *>(rr + lr0 + 8 * q + 4 * kh);
                     constexpr float f = NP == 3 ? SM_UNSCALE : 1.0f;
-                    float o[4] = {acc[i][j][4 * q] * f - rv.x, acc[i][j][4 * q + 1] * f - rv.y,
-                                  acc[i][j][4 * q + 2] * f - rv.z, acc[i][j][4 * q + 3] * f - rv.w};
+                    float o[4] = {acc[i][j][4 * q] * f, acc[i][j][4 * q + 1] * f, acc[i][j][4 * q + 2] * f, acc[i][j][4 * q + 3] * f};
+                    if (NP == 2) {
+                        const int4 sv = *reinterpret_cast<const int4 *>(rr + 3 * TR + lr0 + 8 * q + 4 * kh);
+                        o[0] = __builtin_amdgcn_ldexpf(o[0], sv.x); o[1] = __builtin_amdgcn_ldexpf(o[1], sv.y);
+                        o[2] = __builtin_amdgcn_ldexpf(o[2], sv.z); o[3] = __builtin_amdgcn_ldexpf(o[3], sv.w);
+                    }
+                    o[0] -= rv.x; o[1] -= rv.y; o[2] -= rv.z; o[3] -= rv.w;
                     if (NP == 1) {
                         const float4 fv = *reinterpret_cast<const float4 *>(rr + 2 * TR + lr0 + 8 * q + 4 * kh);
                         o[0] *= softmap_lo(e[j][q].x) * fv.x; o[1] *= softmap_hi(e[j][q].x) * fv.y;
@@ -545,7 +815,7 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
                 const size_t at = (size_t)row * C + col4;
                 if (vec) {
                     if (row < R && col4 < C) {
-                        if (NP == 3) {
+                        if (NP != 1) {
                             const float4 w = *reinterpret_cast<const float4 *>(g.W + at);
                             const float mx = rr[TR + lr0 + lr], f = rr[2 * TR + lr0 + lr];
                             o.x *= softmap_e(w.x, mx, g.scale) * f; o.y *= softmap_e(w.y, mx, g.scale) * f;
@@ -558,7 +828,7 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
 #pragma unroll
                     for (int n = 0; n < 4; ++n)
                         if (row < R && col4 + n < C)
-                            g.out[at + n] = NP == 3 ? os[n] * (softmap_e(g.W[at + n], rr[TR + lr0 + lr], g.scale) * rr[2 * TR + lr0 + lr]) : os[n];
+                            g.out[at + n] = NP != 1 ? os[n] * (softmap_e(g.W[at + n], rr[TR + lr0 + lr], g.scale) * rr[2 * TR + lr0 + lr]) : os[n];
                 }
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -745,22 +1015,29 @@ struct SoftmapShape {
     int fwd_stages, fwd_chunk, fwd_chunks;            // reduction over I
     int gx_stages, gx_chunk, gx_chunks;               // reduction over M
     size_t e_plane, x_plane, g_plane;                 // bytes of a plane of E, of x, of gs
+    bool pairs;                                       // precision 0: pairs where the values allow them
+    int pair_row_tiles, pair_fwd_chunk, pair_fwd_chunks, pair_gx_chunk, pair_gx_chunks;
 };
 
 // A product whose tiles do not fill the card's 512 resident blocks (two per CU) cuts its reduction into chunks, whose
 // partial results are added in order by a second launch.  gx at 512 x 3136 x 48000 (50 tiles): 10 chunks, one round of 500
 // blocks.  A chunk keeps at least 8 stages, below which a block is mostly its own start and end.
-static void softmap_chunks(int stages, long long tiles, int *chunk, int *chunks) {
-    long long n = 512 / tiles;
+static void softmap_chunks(int stages, long long tiles, long long blocks, int *chunk, int *chunks) {
+    long long n = blocks / tiles;
     if (n > stages / 8) n = stages / 8;
     if (n < 1) n = 1;
     *chunk = dl_ceil_div(stages, n);
     *chunks = dl_ceil_div(stages, *chunk);
 }
+// Pairs cost a pass over x and one over gm and seven launches of about 5 us a step, four of which end at once.  Measured, forward +
+// backward, planes against pairs: 512 x 512 x 24000 (6.3e9) 332 -> 322 us, 64 x 3136 x 30000 (6.0e9) 716 -> 594, 300 x 1500 x 20000
+// (9.0e9) 578 -> 468, 512 x 3136 x 48000 2659 -> 2562 where E spans too much; below, planes.
+#define SM_PAIR_WORK 6e9
 static SoftmapShape softmap_shape(int B, int I, int M, int precision) {
     SoftmapShape h;
     h.B = B; h.I = I; h.M = M;
     h.np = precision == 1 ? 1 : 3;
+    h.pairs = h.np == 3 && (double)B * I * M >= SM_PAIR_WORK;
     h.fa = B > 128 ? 4 : 2;
     h.depth = h.np == 1 ? 32 : 16;
     h.Bp = softmap_round(B, 64 * h.fa);
@@ -771,8 +1048,11 @@ static SoftmapShape softmap_shape(int B, int I, int M, int precision) {
     h.gx_col_tiles = h.Ip / SM_TC;
     h.fwd_stages = dl_ceil_div(I, h.depth);
     h.gx_stages = dl_ceil_div(M, h.depth);
-    softmap_chunks(h.fwd_stages, (long long)h.row_tiles * h.fwd_col_tiles, &h.fwd_chunk, &h.fwd_chunks);
-    softmap_chunks(h.gx_stages, (long long)h.row_tiles * h.gx_col_tiles, &h.gx_chunk, &h.gx_chunks);
+    softmap_chunks(h.fwd_stages, (long long)h.row_tiles * h.fwd_col_tiles, 512, &h.fwd_chunk, &h.fwd_chunks);
+    softmap_chunks(h.gx_stages, (long long)h.row_tiles * h.gx_col_tiles, 512, &h.gx_chunk, &h.gx_chunks);
+    h.pair_row_tiles = h.Bp / 128;
+    softmap_chunks(h.fwd_stages, (long long)h.pair_row_tiles * h.fwd_col_tiles, 512, &h.pair_fwd_chunk, &h.pair_fwd_chunks);
+    softmap_chunks(h.gx_stages, (long long)h.pair_row_tiles * h.gx_col_tiles, 1024, &h.pair_gx_chunk, &h.pair_gx_chunks);
     h.e_plane = dl_align256((size_t)(h.Mp / 8) * h.Ip * SM_UNIT);
     h.x_plane = dl_align256((size_t)(h.Ip / 8) * h.Bp * SM_UNIT);
     h.g_plane = dl_align256((size_t)(h.Mp / 8) * h.Bp * SM_UNIT);
@@ -780,7 +1060,7 @@ static SoftmapShape softmap_shape(int B, int I, int M, int precision) {
 }
 
 // `stats`, kept for the backward: max [Mp], 1/sum [Mp], x in units along the inputs (the forward's operand), E, and with
-// fp32 operands the largest magnitude of x
+// fp32 operands the range (its first word the largest magnitude of x)
 static inline size_t softmap_vec_bytes(const SoftmapShape &h) { return dl_align256((size_t)h.Mp * sizeof(float)); }
 extern "C" size_t dl_soft_map_saved_bytes(int B, int I, int M, int precision) {
     if (B <= 0 || I <= 0 || M <= 0) return 256;
@@ -789,9 +1069,12 @@ extern "C" size_t dl_soft_map_saved_bytes(int B, int I, int M, int precision) {
 }
 
 // workspace: partial products of the forward or of gx, partial r, x and gm in units along the batch, gs along the rows of W, the
-// largest magnitude of gm
+// largest magnitude of gm, those of the rows of gs and the columns of gm
 static inline size_t softmap_part_bytes(const SoftmapShape &h) {
-    const size_t fwd = h.fwd_chunks > 1 ? (size_t)h.fwd_chunks * h.B * h.M : 0, gx = h.gx_chunks > 1 ? (size_t)h.gx_chunks * h.B * h.I : 0;
+    int nf = h.fwd_chunks, ng = h.gx_chunks;
+    if (h.pairs && h.pair_fwd_chunks > nf) nf = h.pair_fwd_chunks;
+    if (h.pairs && h.pair_gx_chunks > ng) ng = h.pair_gx_chunks;
+    const size_t fwd = nf > 1 ? (size_t)nf * h.B * h.M : 0, gx = ng > 1 ? (size_t)ng * h.B * h.I : 0;
     return dl_align256((fwd > gx ? fwd : gx) * sizeof(float));
 }
 static inline size_t softmap_dots_bytes(const SoftmapShape &h) {
@@ -800,15 +1083,16 @@ static inline size_t softmap_dots_bytes(const SoftmapShape &h) {
 extern "C" size_t dl_soft_map_workspace_bytes(int B, int I, int M, int precision) {
     if (B <= 0 || I <= 0 || M <= 0) return 256;
     const SoftmapShape h = softmap_shape(B, I, M, precision);
-    return 256 + softmap_part_bytes(h) + softmap_dots_bytes(h) + h.np * (h.x_plane + 2 * h.g_plane);
+    return 256 + softmap_part_bytes(h) + softmap_dots_bytes(h) + h.np * (h.x_plane + 2 * h.g_plane) +
+           (h.pairs ? dl_align256((size_t)(h.Bp + h.Mp) * sizeof(unsigned)) : 0);
 }
 
 template <int NP>
 static void softmap_stats_launch(const SoftmapShape &h, const float *W, float scale, float *mx, float *rs, char *E,
-                                 unsigned *largest, hipStream_t s) {
+                                 unsigned *largest, SoftmapRange *range, hipStream_t s) {
     const int grid = h.Mp / 8;
 #define SM_STATS(T, NQ) \
-    DL_TIMED("softmap_rowstats", s, (softmap_rowstats<NP, T, NQ><<<grid, T, 0, s>>>(W, scale, mx, rs, E, h.e_plane, h.M, h.I, h.Ip, largest)))
+    DL_TIMED("softmap_rowstats", s, (softmap_rowstats<NP, T, NQ><<<grid, T, 0, s>>>(W, scale, mx, rs, E, h.e_plane, h.M, h.I, h.Ip, largest, range)))
     if (h.Ip <= 256 * 4) SM_STATS(256, 4);
     else if (h.Ip <= 256 * 8) SM_STATS(256, 8);
     else if (h.Ip <= 512 * 8) SM_STATS(512, 8);
@@ -818,20 +1102,23 @@ static void softmap_stats_launch(const SoftmapShape &h, const float *W, float sc
 }
 static void softmap_pack_launch(int np, const float *src, const float *colscale, const float *other, float *dots, char *rows8,
                                 size_t rows_plane, char *cols8, size_t cols_plane, int R, int C, int Rp, int Cp, float alternate,
-                                unsigned *largest, unsigned *clear, hipStream_t s) {
+                                unsigned *largest, unsigned *clear, const SoftmapRange *range, const unsigned *row_max,
+                                const unsigned *col_max, hipStream_t s) {
     const int grid = Cp / 64 * dl_ceil_div(Rp, 64);
-    if (np == 1)
-        DL_TIMED("softmap_pack", s, (softmap_pack<1><<<grid, 256, 0, s>>>(src, colscale, other, dots, rows8, rows_plane, cols8, cols_plane, R, C, Rp, Cp, alternate, largest, clear)));
-    else
-        DL_TIMED("softmap_pack", s, (softmap_pack<3><<<grid, 256, 0, s>>>(src, colscale, other, dots, rows8, rows_plane, cols8, cols_plane, R, C, Rp, Cp, alternate, largest, clear)));
+#define SM_PACK(NP) \
+    DL_TIMED("softmap_pack", s, (softmap_pack<NP><<<grid, 256, 0, s>>>(src, colscale, other, dots, rows8, rows_plane, cols8, cols_plane, R, C, Rp, Cp, alternate, largest, clear, range, row_max, col_max)))
+    if (np == 1) SM_PACK(1);
+    else if (range) SM_PACK(2);
+    else SM_PACK(3);
+#undef SM_PACK
 }
-static void softmap_reduce(const float *part, float *out, long long total, int chunks, hipStream_t s) {
+static void softmap_reduce(const float *part, float *out, long long total, int chunks, const SoftmapRange *range, int wide_chunks, hipStream_t s) {
     if (total % 4 == 0 && ((uintptr_t)out & 15) == 0)
         DL_TIMED("softmap_reduce_chunks", s,
-                 (softmap_reduce_chunks<4><<<dl_ceil_div(total / 4, 256), 256, 0, s>>>(part, out, total, chunks)));
+                 (softmap_reduce_chunks<4><<<dl_ceil_div(total / 4, 256), 256, 0, s>>>(part, out, total, chunks, range, wide_chunks)));
     else
         DL_TIMED("softmap_reduce_chunks", s,
-                 (softmap_reduce_chunks<1><<<dl_ceil_div(total, 256), 256, 0, s>>>(part, out, total, chunks)));
+                 (softmap_reduce_chunks<1><<<dl_ceil_div(total, 256), 256, 0, s>>>(part, out, total, chunks, range, wide_chunks)));
 }
 template <int MODE>
 static void softmap_product(const char *name, const SoftmapShape &h, int fa, const SoftmapArgs &g, hipStream_t s) {
@@ -856,24 +1143,47 @@ extern "C" int dl_soft_map_fwd(const float *x, const float *W, float tau, float 
     if (precision == 1 && ws_bytes < dl_soft_map_workspace_bytes(B, I, M, precision)) return DL_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
     SoftmapShape h = softmap_shape(B, I, M, precision);
-    if (!ws || ws_bytes < dl_soft_map_workspace_bytes(B, I, M, precision)) { h.fwd_chunk = h.fwd_stages; h.fwd_chunks = 1; }
+    if (!ws || ws_bytes < dl_soft_map_workspace_bytes(B, I, M, precision)) {
+        h.fwd_chunk = h.pair_fwd_chunk = h.fwd_stages;
+        h.fwd_chunks = h.pair_fwd_chunks = 1;
+    }
     char *p = (char *)stats;
     float *mx = (float *)p, *rs = (float *)(p + softmap_vec_bytes(h));
     char *x8 = p + 2 * softmap_vec_bytes(h), *E = x8 + h.np * h.x_plane;
     unsigned *x_largest = h.np > 1 ? (unsigned *)(E + h.np * h.e_plane) : nullptr;
-    if (h.np == 1) softmap_stats_launch<1>(h, W, SM_LOG2E / tau, mx, rs, E, x_largest, s);
-    else softmap_stats_launch<3>(h, W, SM_LOG2E / tau, mx, rs, E, x_largest, s);
-    softmap_pack_launch(h.np, x, nullptr, nullptr, nullptr, nullptr, 0, x8, h.x_plane, B, I, h.Bp, h.Ip, 1.0f, x_largest, nullptr, s);
+    SoftmapRange *range = h.pairs ? (SoftmapRange *)x_largest : nullptr;
+    const float scale = SM_LOG2E / tau;
+    if (h.np == 1) softmap_stats_launch<1>(h, W, scale, mx, rs, E, nullptr, nullptr, s);
+    else if (!h.pairs) softmap_stats_launch<3>(h, W, scale, mx, rs, E, x_largest, nullptr, s);
+    else {
+        DL_TIMED("softmap_clear", s, (softmap_clear<<<1, 256, 0, s>>>(range, nullptr, 0)));
+        const int grid = dl_ceil_div((long long)B * I, 256 * 8);
+        DL_TIMED("softmap_scan", s, (softmap_scan_x<<<grid < 256 ? grid : 256, 256, 0, s>>>(x, (long long)B * I, range)));
+        softmap_stats_launch<2>(h, W, scale, mx, rs, E, nullptr, range, s);
+        softmap_stats_launch<3>(h, W, scale, mx, rs, E, nullptr, range, s);
+    }
+    softmap_pack_launch(h.np, x, nullptr, nullptr, nullptr, nullptr, 0, x8, h.x_plane, B, I, h.Bp, h.Ip, 1.0f, h.pairs ? nullptr : x_largest,
+                        nullptr, range, nullptr, nullptr, s);
     SoftmapArgs g{};
     g.A = x8; g.a_plane = h.x_plane; g.lda = h.Bp;
     g.Bm = E; g.b_plane = h.e_plane; g.ldb = h.Ip;
-    g.out = h.fwd_chunks > 1 ? (float *)ws : m;
     g.R = B; g.C = M;
-    g.stages = h.fwd_stages; g.chunk_stages = h.fwd_chunk;
-    g.inner_count = h.row_tiles; g.outer_count = h.fwd_col_tiles * h.fwd_chunks; g.col_tiles = h.fwd_col_tiles;
-    g.rs = rs;
+    g.stages = h.fwd_stages;
+    g.col_tiles = h.fwd_col_tiles;
+    g.rs = rs; g.range = range;
+    auto product = [&](int row_tiles, int chunk, int chunks) {
+        g.out = chunks > 1 ? (float *)ws : m;
+        g.chunk_stages = chunk;
+        g.inner_count = row_tiles; g.outer_count = h.fwd_col_tiles * chunks;
+    };
+    if (h.pairs) {
+        product(h.pair_row_tiles, h.pair_fwd_chunk, h.pair_fwd_chunks);
+        DL_TIMED("softmap_fwd", s, (softmap_launch<0, 2, 2>(g, s)));
+    }
+    product(h.row_tiles, h.fwd_chunk, h.fwd_chunks);
     softmap_product<0>("softmap_fwd", h, h.fa, g, s);
-    if (h.fwd_chunks > 1) softmap_reduce((const float *)ws, m, (long long)B * M, h.fwd_chunks, s);
+    if (h.pairs ? h.pair_fwd_chunks > 1 || h.fwd_chunks > 1 : h.fwd_chunks > 1)
+        softmap_reduce((const float *)ws, m, (long long)B * M, h.pairs ? h.pair_fwd_chunks : h.fwd_chunks, range, h.fwd_chunks, s);
     if (h.np > 1) {
         SoftmapPlain q{};
         q.x = x; q.W = W; q.mx = mx; q.rs = rs; q.m = m; q.x_largest = x_largest;
@@ -905,17 +1215,37 @@ extern "C" int dl_soft_map_bwd(const float *x, const float *W, float tau, const 
     char *gb = w; w += h.np * h.g_plane;     // gm [Bp/8][Mp]
     char *go = w; w += h.np * h.g_plane;     // gs [Mp/8][Bp]
     unsigned *gm_largest = h.np > 1 ? (unsigned *)w : nullptr;
-    softmap_pack_launch(h.np, x, nullptr, nullptr, nullptr, xb, h.x_plane, nullptr, 0, B, I, h.Bp, h.Ip, 1.0f, nullptr, gm_largest, s);
-    softmap_pack_launch(h.np, gm, rs, m, dots, gb, h.g_plane, go, h.g_plane, B, M, h.Bp, h.Mp, -1.0f, gm_largest, nullptr, s);
+    const SoftmapRange *range = h.pairs ? (const SoftmapRange *)x_largest : nullptr;
+    unsigned *row_max = h.pairs ? (unsigned *)(w + 256) : nullptr, *col_max = h.pairs ? row_max + h.Bp : nullptr;
+    if (h.pairs) {
+        const int words = 64 + h.Bp + h.Mp, strips = dl_ceil_div(M, 64 * SM_SCAN_TILES);
+        DL_TIMED("softmap_clear", s, (softmap_clear<<<dl_ceil_div(words, 256), 256, 0, s>>>(nullptr, gm_largest, words)));
+        DL_TIMED("softmap_scan", s, (softmap_scan_grad<<<(unsigned)strips * dl_ceil_div(B, 64), 256, 0, s>>>(gm, rs, row_max, col_max, gm_largest, range, B, M, strips)));
+    }
+    softmap_pack_launch(h.np, x, nullptr, nullptr, nullptr, xb, h.x_plane, nullptr, 0, B, I, h.Bp, h.Ip, 1.0f, nullptr,
+                        h.pairs ? nullptr : gm_largest, range, nullptr, nullptr, s);
+    softmap_pack_launch(h.np, gm, rs, m, dots, gb, h.g_plane, go, h.g_plane, B, M, h.Bp, h.Mp, -1.0f, gm_largest, nullptr,
+                        range, row_max, col_max, s);
     SoftmapArgs g{};
     g.A = go; g.a_plane = h.g_plane; g.lda = h.Bp;
     g.Bm = E; g.b_plane = h.e_plane; g.ldb = h.Ip;
-    g.out = h.gx_chunks > 1 ? part : gx;
     g.R = B; g.C = I;
-    g.stages = h.gx_stages; g.chunk_stages = h.gx_chunk;
-    g.inner_count = h.row_tiles; g.outer_count = h.gx_col_tiles * h.gx_chunks; g.col_tiles = h.gx_col_tiles;
+    g.stages = h.gx_stages;
+    g.col_tiles = h.gx_col_tiles;
+    g.range = range; g.row_max = row_max;
+    auto product = [&](int row_tiles, int chunk, int chunks) {
+        g.out = chunks > 1 ? part : gx;
+        g.chunk_stages = chunk;
+        g.inner_count = row_tiles; g.outer_count = h.gx_col_tiles * chunks;
+    };
+    if (h.pairs) {
+        product(h.pair_row_tiles, h.pair_gx_chunk, h.pair_gx_chunks);
+        DL_TIMED("softmap_gx", s, (softmap_launch<1, 2, 2>(g, s)));
+    }
+    product(h.row_tiles, h.gx_chunk, h.gx_chunks);
     softmap_product<1>("softmap_gx", h, h.fa, g, s);
-    if (h.gx_chunks > 1) softmap_reduce(part, gx, (long long)B * I, h.gx_chunks, s);
+    if (h.pairs ? h.pair_gx_chunks > 1 || h.gx_chunks > 1 : h.gx_chunks > 1)
+        softmap_reduce(part, gx, (long long)B * I, h.pairs ? h.pair_gx_chunks : h.gx_chunks, range, h.gx_chunks, s);
     // gW: tiles of 256 rows of W where they fill the card, else of 128
     const int fa = (long long)(h.Mp / 256) * h.gx_col_tiles >= 512 ? 4 : 2;
     SoftmapArgs q{};
@@ -924,10 +1254,16 @@ extern "C" int dl_soft_map_bwd(const float *x, const float *W, float tau, const 
     q.out = gW;
     q.R = M; q.C = I;
     q.stages = dl_ceil_div(B, h.depth); q.chunk_stages = q.stages;
-    q.inner_count = h.gx_col_tiles; q.outer_count = dl_ceil_div(M, 64 * fa); q.col_tiles = h.gx_col_tiles;
+    q.inner_count = h.gx_col_tiles; q.col_tiles = h.gx_col_tiles;
     q.rs = rs; q.dots = dots; q.parts = dl_ceil_div(B, 64); q.dot_ld = h.Mp;
     q.mx = mx; q.W = W; q.E = E; q.lde = h.Ip; q.scale = SM_LOG2E / tau; q.inv_tau = 1.0f / tau;
+    q.range = range; q.row_max = col_max;
     q.vec_out = (((uintptr_t)W | (uintptr_t)gW) & 15) == 0;
+    if (h.pairs) {
+        q.outer_count = dl_ceil_div(M, 128);
+        DL_TIMED("softmap_gw", s, (softmap_launch<2, 2, 2>(q, s)));
+    }
+    q.outer_count = dl_ceil_div(M, 64 * fa);
     softmap_product<2>("softmap_gw", h, fa, q, s);
     if (h.np > 1) {
         SoftmapPlain u{};

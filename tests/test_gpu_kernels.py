@@ -893,6 +893,57 @@ def test_soft_mapping_fp32_range(shape, side, case):
         assert float(rel.max()) <= 1e-5
 
 
+@pytest.mark.parametrize("case", ["ordinary", "two_orders", "wide_e", "wide_x", "scaled_gradients", "tiny", "huge", "infinite_x", "nan_gm"])
+@pytest.mark.parametrize("shape", [(100, 1030, 60100), (257, 515, 50001)])  # 128- and 256-row tiles, ragged on every side
+def test_soft_mapping_fp32_pairs(shape, case):
+    """Products large enough for pairs of fp16 halves, and what sends them back to three planes or to fp32 sums.  A pair holds 23
+    of 24 bits, so every output stays within 1e-5 (in the 2-norm, as test_soft_mapping_tile_edges derives it) of the sum of its
+    terms' magnitudes; gx row by row, however far apart the rows' magnitudes are."""
+    ops = _ops()
+    B, I, M = shape
+    g = torch.Generator("cuda").manual_seed(B + len(case))
+    x = torch.rand(B, I, device="cuda", generator=g) + 0.01
+    W = torch.randn(M, I, device="cuda", generator=g)
+    gm = torch.randn(B, M, device="cuda", generator=g)
+    if case == "two_orders":
+        x[:, ::2] *= 0.01
+        x[x < 0.002] = 0.0
+    elif case == "wide_e":  # in the last of the rows: everything else has been written as pairs by then
+        W[M - 1, 5] = 40.0
+    elif case == "wide_x":
+        x[B - 1] *= 1e-20
+    elif case == "scaled_gradients":
+        gm[::3] *= 1e-25
+        gm[1::3] *= 1e10
+        gm[:, ::7] *= 1e-6
+        gm[5] = 0.0
+    elif case == "tiny":
+        x *= 1e-33
+        gm *= 1e-5
+    elif case == "huge":
+        x *= 1e25
+    elif case == "infinite_x":
+        x[3, 7] = float("inf")
+    elif case == "nan_gm":
+        gm[4, 9] = float("nan")
+    xt, Wt = x.clone().requires_grad_(), W.clone().requires_grad_()
+    m = ops.SoftMapFunction.apply(xt, Wt, 1.0, 0)
+    m.backward(gm)
+    xd, gd = x.double(), gm.double()
+    S = torch.softmax(W.double(), dim=-1)
+    md = xd @ S.t()
+    G, r = gd.t() @ xd, (gd * md).sum(0)
+    for name, got, want, size in (("m", m.detach(), md, xd.abs() @ S.t()), ("gx", xt.grad, gd @ S, gd.abs() @ S),
+                                  ("gW", Wt.grad, S * (G - r[:, None]), S * (G.abs() + (gd * md).abs().sum(0)[:, None]))):
+        got = got.double()
+        assert torch.equal(torch.isnan(got), torch.isnan(want)), name
+        assert torch.equal(torch.isinf(got), torch.isinf(want)), name
+        finite = torch.isfinite(want) & torch.isfinite(size)
+        diff, size = (got - want).where(finite, 0.0), size.where(finite, 0.0)
+        rows = (diff.norm(dim=1) <= 1e-5 * size.norm(dim=1) + 1e-43 * got.shape[1] ** 0.5)
+        assert rows.all(), (name, float((diff.norm(dim=1) / size.norm(dim=1)).nan_to_num().max()))
+
+
 @pytest.mark.parametrize("precision", [0, 1])
 def test_soft_mapping_of_more_rows_than_a_grid_dimension(precision):
     """4.19 million rows are 65536 blocks of 64 rows; limits as in test_soft_mapping_tile_edges."""
