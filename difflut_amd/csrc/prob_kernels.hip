@@ -284,6 +284,15 @@ __device__ __forceinline__ void prob_fold_gradient(const float (&v0)[1 << KH], c
     }
 }
 
+// The gradient of the mapped inputs is written once and read once.  Where it is too large for the 256 MB behind the L2s to hold it
+// beside x and gx, it is written and read, and gx written, past that cache's keeping (STREAM), which leaves it to what is read
+// again.  Forward and backward, us, as ordinary accesses / so: hybrid 1024 x 8192 -> 6000 (147 MB) 136 / 133, 2048 x 8192 -> 4096 (201 MB)
+// 196 / 176, 2048 x 8192 -> 8192 (403 MB) 335 / 310, 4096 x 16384 -> 8192 (805 MB) 686 / 659; probabilistic 4096 x 16384 -> 8192, k = 4
+// (537 MB) 567 / 534.  Smaller ones lose what the gather would have found there: 512 x 6000 -> 8000 (98 MB) 94 / 96.  (A compile-time
+// choice: the two stores of a branch become one without the hint.)
+static inline bool prob_gm_stream(int B, int N, int k, int O) { return (double)B * N * O * k * sizeof(float) >= 128e6; }
+#define PROB_NT 2  // cache policy of a buffer load: read once
+
 // one wavefront per (column, chunk of batch tiles); W wavefronts, i.e. sixteen columns (or four), per block.
 // HYB (hybrid node): the table is used as given and the input gradient carries the factor
 // q / (q + 1e-8), q = x_j (1 - x_j), of that node's backward.
@@ -300,7 +309,7 @@ __device__ __forceinline__ void prob_fold_gradient(const float (&v0)[1 << KH], c
 // batch tile is fetched one value per thread a tile ahead and turned through the LDS (two buffers, one barrier per tile).
 // W = 4 (at most 12 columns): blocks of four columns, so that at most three wavefronts of a block have none, and four
 // blocks on a CU.  65536 rows x 8 columns, k = 6: 84 us in blocks of sixteen and at most 16 chunks, 14.5 in blocks of four.
-template <int K, bool HYB, int W = 16>
+template <int K, bool HYB, int W, bool STREAM>
 __global__ __launch_bounds__(64 * W) void prob_bwd_t(const float *__restrict__ xT, const float *__restrict__ gy,
                                                    const int *__restrict__ idx32, const float *__restrict__ cen,
                                                    float *__restrict__ gmT, float *__restrict__ gpart, int I, int N,
@@ -375,7 +384,11 @@ __global__ __launch_bounds__(64 * W) void prob_bwd_t(const float *__restrict__ x
             }
             if (live) {
 #pragma unroll
-                for (int j = 0; j < K; ++j) gmT[(((size_t)t * NO + c) * K + j) * 64 + lane] = g * dx[j];
+                for (int j = 0; j < K; ++j) {
+                    float *at = &gmT[(((size_t)t * NO + c) * K + j) * 64 + lane];
+                    if constexpr (STREAM) __builtin_nontemporal_store(g * dx[j], at);
+                    else *at = g * dx[j];
+                }
             }
         }
 #pragma unroll
@@ -454,7 +467,7 @@ __device__ __forceinline__ void prob_reduce_element(const ProbReduce &R, long lo
 // FAST (one output per node): the CSR entries of a wavefront's 16 inputs are held one per lane
 // (row offset, local input) and replayed eight at a time with buffer loads whose offset travels
 // in an SGPR, the next eight requested before the current ones are summed.
-template <bool FAST>
+template <bool FAST, bool STREAM>
 __global__ __launch_bounds__(256) void prob_gather_t(const float *__restrict__ gmT, const int *__restrict__ inv_ptr,
                                                       const int *__restrict__ inv_pos, float *__restrict__ gx, int B,
                                                       int I, int N, int K, int O, int BT, int gather_blocks, ProbReduce R) {
@@ -496,7 +509,7 @@ __global__ __launch_bounds__(256) void prob_gather_t(const float *__restrict__ g
                 for (int q = 0; q < PROB_EG; ++q) {
                     const int r = __builtin_amdgcn_readlane(rec, s0 + q);
                     G.r[q] = r;
-                    G.g[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, lane4, r & ~255, 0));
+                    G.g[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, lane4, r & ~255, STREAM ? PROB_NT : 0));
                 }
             };
             auto sum_up = [&](const Group &G, int s0) {
@@ -555,7 +568,10 @@ __global__ __launch_bounds__(256) void prob_gather_t(const float *__restrict__ g
             const int r = e / (PROB_IS / 4), i4 = (e % (PROB_IS / 4)) * 4;
             const int b = t * 64 + r;
             const prob_f4 v = {tile[i4][r], tile[i4 + 1][r], tile[i4 + 2][r], tile[i4 + 3][r]};
-            if (b < B) *reinterpret_cast<prob_f4 *>(&gx[(size_t)b * I + i0 + i4]) = v;
+            if (b >= B) continue;
+            prob_f4 *at = reinterpret_cast<prob_f4 *>(&gx[(size_t)b * I + i0 + i4]);
+            if constexpr (STREAM) __builtin_nontemporal_store(v, at);
+            else *at = v;
         }
     } else {
         for (int e = threadIdx.x; e < 64 * PROB_IS; e += 256) {
@@ -576,12 +592,13 @@ static void prob_launch_gather_and_reduce(const float *gmT, const int *inv_ptr, 
         return;
     }
     const int gblocks = dl_xcd_grid(dl_ceil_div(I, PROB_IS), BT);
-    if (O == 1)
-        DL_TIMED("prob_gather_t+reduce", s, (prob_gather_t<true><<<gblocks + rblocks, 256, 0, s>>>(gmT, inv_ptr, inv_pos, gx, B, I,
-                                                                                               N, k, O, BT, gblocks, R)));
-    else
-        DL_TIMED("prob_gather_t+reduce", s, (prob_gather_t<false><<<gblocks + rblocks, 256, 0, s>>>(gmT, inv_ptr, inv_pos, gx, B, I,
-                                                                                                N, k, O, BT, gblocks, R)));
+#define GATHER(FAST, STREAM)                                                                                                  \
+    DL_TIMED("prob_gather_t+reduce", s, (prob_gather_t<FAST, STREAM><<<gblocks + rblocks, 256, 0, s>>>(gmT, inv_ptr, inv_pos, gx, B, I, \
+                                                                                                       N, k, O, BT, gblocks, R)))
+    if (O != 1) GATHER(false, false);
+    else if (prob_gm_stream(B, N, k, O)) GATHER(true, true);
+    else GATHER(true, false);
+#undef GATHER
 }
 
 // ---------------------------------------------------------------------------------
@@ -782,10 +799,13 @@ static void prob_launch_bwd(const char *name, const float *xT, const float *gy, 
     const dim3 grid(dl_ceil_div(NO, W), dl_ceil_div(BT, tpc));
 #define CALL(KK)                                                                                                                  \
     do {                                                                                                                          \
-        if (W == 4) DL_TIMED(name, s, (prob_bwd_t<KK, HYB, 4><<<grid, 256, 0, s>>>(xT, gy, idx32, table, gmT, gpart, I, N, O, BT, \
+        if (W == 4) DL_TIMED(name, s, (prob_bwd_t<KK, HYB, 4, false><<<grid, 256, 0, s>>>(xT, gy, idx32, table, gmT, gpart, I, N, \
+                                                                                          O, BT, tpc, want_gm, B)));              \
+        else if (O == 1 && prob_gm_stream(B, N, k, O))                                                                            \
+            DL_TIMED(name, s, (prob_bwd_t<KK, HYB, 16, true><<<grid, 1024, 0, s>>>(xT, gy, idx32, table, gmT, gpart, I, N, O, BT, \
                                                                                    tpc, want_gm, B)));                            \
-        else DL_TIMED(name, s, (prob_bwd_t<KK, HYB><<<grid, 1024, 0, s>>>(xT, gy, idx32, table, gmT, gpart, I, N, O, BT, tpc,     \
-                                                                          want_gm, B)));                                          \
+        else DL_TIMED(name, s, (prob_bwd_t<KK, HYB, 16, false><<<grid, 1024, 0, s>>>(xT, gy, idx32, table, gmT, gpart, I, N, O,   \
+                                                                                     BT, tpc, want_gm, B)));                      \
     } while (0)
     PROB_DISPATCH(k, CALL)
 #undef CALL

@@ -434,3 +434,31 @@ def test_nodes_against_reference_vectors(golden_next, name, kind, tag):
     node.eval()
     with torch.no_grad():
         assert np.array_equal(node(dev(g[f"{kind}_{tag}_eval_x"])).cpu().numpy(), g[f"{kind}_{tag}_eval_y"])
+
+
+@pytest.mark.parametrize("name", ["probabilistic", "hybrid"])
+@pytest.mark.parametrize("inputs", [700, 701])  # 16-byte stores of gx, and single ones
+def test_backward_past_the_cache_equals_its_halves(name, inputs):
+    """1003 rows x 5400 nodes of six inputs are 130 MB of mapped gradients, which are written and read past the cache; their halves
+    are not.  The same sums in the same order: gx bit for bit; the tables' gradients are sums over rows in another order (fp32,
+    sqrt(1003) roundings of 2^-24, with cancellation below 1e-5 of the 2-norm)."""
+    from difflut_amd import REGISTRY
+    from difflut_amd.nodes.node_config import NodeConfig
+
+    layer = REGISTRY.get_layer("random")(inputs, 5400, REGISTRY.get_node(name), NodeConfig(input_dim=6, output_dim=1), seed=4)
+    layer = layer.to("cuda").train()
+    table = layer.bank_parameters()[0]
+    g = torch.Generator("cuda").manual_seed(inputs)
+    x = torch.rand(1003, inputs, device="cuda", generator=g)
+    gy = torch.randn(1003, 5400, device="cuda", generator=g)
+
+    def backward(rows):
+        xr = x[rows].contiguous().requires_grad_()
+        table.grad = None
+        layer(xr).backward(gy[rows].contiguous())
+        return xr.grad, table.grad.double()
+
+    whole, table_whole = backward(slice(0, 1003))
+    (a, ta), (b, tb) = backward(slice(0, 512)), backward(slice(512, 1003))
+    assert torch.equal(whole, torch.cat([a, b]))
+    assert float((table_whole - ta - tb).norm()) <= 1e-5 * float(table_whole.norm())
