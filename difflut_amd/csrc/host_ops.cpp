@@ -440,15 +440,21 @@ struct DwnStack : torch::autograd::Function<DwnStack> {
             // the second layer's call can give the first layer's input gradient too: its own is then not stored
             const bool first = l == 1 && st->patches && wants_input_grad && st->dims[0].O == 1 && nodes && st->per_node[0][0].defined() &&
                                L.dl_dwn_chain_first_fusable(DIMS(d), st->dims[0].k, st->dims[0].I, beta_max) == 1;
+            // the gather of this layer can fill the table gradient of the layer in front as it goes: that layer's own
+            // pass over its [B, N] output gradient is then left out
+            const int k_prev = l > 0 ? st->dims[l - 1].k : 0;
+            const bool fuse = first || (nodes && l > 0 && st->dims[l - 1].O == 1 && L.dl_dwn_chain_fusable(DIMS(d), k_prev, beta_max) == 1);
+            // the first layer's table gradient is then all that is left: nobody reads this input gradient
+            const bool unread = fuse && l == 1 && !wants_input_grad;
             Tensor gx;
             int gx_tiled = 1;
             if (l > 0) {
-                if (!first) gx = tiled_array(d.B, d.I);
+                if (!first && !unread) gx = tiled_array(d.B, d.I);
             } else {
                 gx_tiled = st->patches;
                 if (wants_input_grad) gx = gx_tiled ? tiled_array(d.B, d.I) : floats({d.B, d.I}, like);
             }
-            if (have_tables[l] && !gx.defined() && !first) {  // nothing left to compute for this layer
+            if (have_tables[l] && !gx.defined() && !first && !unread) {  // nothing left to compute for this layer
                 g = Tensor();
                 continue;
             }
@@ -459,10 +465,6 @@ struct DwnStack : torch::autograd::Function<DwnStack> {
             const float tau = headed ? (float)st->tau : 1.0f;
             if (nodes) {  // every node's own alpha and beta
                 const Tensor alpha_n = per_node(st->per_node[l][0], d.N, like), beta_n = per_node(st->per_node[l][1], d.N, like);
-                // the gather of this layer can fill the table gradient of the layer in front as it goes: that layer's own
-                // pass over its [B, N] output gradient is then left out
-                const int k_prev = l > 0 ? st->dims[l - 1].k : 0;
-                const bool fuse = first || (l > 0 && st->dims[l - 1].O == 1 && L.dl_dwn_chain_fusable(DIMS(d), k_prev, beta_max) == 1);
                 if (fuse) {
                     grads[l - 1] = at::empty_like(luts[l - 1]);
                     have_tables[l - 1] = true;
@@ -480,7 +482,6 @@ struct DwnStack : torch::autograd::Function<DwnStack> {
                     g = gfirst;
                     break;
                 }
-                if (fuse && l == 1 && !wants_input_grad) gx = Tensor();  // the first layer's table gradient is all that is left
                 const Tensor ws = bytes(fuse ? L.dl_dwn_bwd_fused_workspace_bytes(DIMS(d), k_prev) : L.dl_dwn_bwd_workspace_bytes(DIMS(d)), like);
                 check(L.dl_dwn_layer_bwd_chain_fused(
                     raw(saved[l]), ints(p.inv_ptr), ints(p.inv_pos), in(luts[l]), in(g), headed ? 2 : tiled, groups, tau, in(alpha_n),
