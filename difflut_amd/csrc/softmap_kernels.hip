@@ -19,14 +19,17 @@
 // (softmap_plain): the pack pass notes the largest magnitude (softmap_note_large).
 // Pairs.  Large products of precision 0 (SM_PAIR_WORK) take half as many matrix operations: an operand, scaled by a power of two
 // to below 2^15, is hi + 2^-11 lo with hi its rounding to fp16 and lo that of 2^11 times the rest, and a product is hi*hi +
-// 2^-11 (hi*lo + lo*hi), the second part in a sum of its own.  Down to 2^-27 of what the scale is taken from both halves are
-// normal numbers, the pair holds 23 bits or more and the product left out is below 2^-24 of |a*b|; smaller values keep an absolute
-// error of 2^-50 of it.  E is scaled by its row maximum, which is one, x by its largest value; where a value of either that is
-// not zero lies below 2^-27 of that, decided on the device, the products it is in take the planes (launches of either
-// kind that are not to run end at once): with W of N(0, 6) at tau 1, where E spans more, the forward and gx.  gs is scaled row by row and gm column by column, so that no output row answers for
-// another's magnitude, and need no such bound: their smallest values meet an E and an x within theirs.  Error against float64
-// (2-norm) of m / gx / gW, 512 x 3136 x 48000, W of N(0, 1.5), tau 1: 1.1e-7 / 1.7e-7 / 4.3e-7 with pairs, 5.3e-7 / 3.2e-7 /
-// 11.8e-7 with planes: half as many additions, and the sums of groups of stages (below).
+// 2^-11 (hi*lo + lo*hi), the second part in a sum of its own.  From 2^-13 on - 2^-27 of the largest - a pair is within 2^-23 of
+// its value (23 of 24 bits); below, within 2^-36 of itself, whatever is left of the value.  The product left out, lo*lo, is below 2^-22
+// of |a*b| (|lo| <= 2^-11 of the value), 2^-25 on average.  So no value may lie below: a sum can be made of small ones alone, where
+// zeros of the other operand take out the large ones.
+//   E is scaled by its row maximum, which is one, x by its largest value; where a value of either that is not zero lies below
+//   2^-27 of that, decided on the device, the products it is in take the planes (launches of either kind that are not to run
+//   end at once): with W of N(0, 6) at tau 1, where E spans more, the forward and gx.
+//   gs is scaled row by row and gm column by column, so that no output row answers for another's magnitude.  Ordinary gradients
+//   have a few values below 2^-27 of those (one in a few million of N(0, 1)): the pack pass leaves up to SM_TINY_MOST of them
+//   out and softmap_plain adds their terms; where there are more, the product takes the planes, gx with E's made from its pairs
+//   (SoftmapArgs::tiny).
 //
 // Layout.  An MFMA lane wants 8 consecutive reduction steps of one row: a "unit" of 16 bytes.  Every operand is stored
 // as [reduction / 8][rows] units, rows padded to whole tiles with zeros, by the pass that has it in registers anyway
@@ -89,7 +92,11 @@ __device__ __forceinline__ uint4 softmap_unit(float *v) {
 #define SM_PAIR_EXP 14          // exponent that an operand's largest value is scaled to
 #define SM_PAIR_LO 0x1p11f
 #define SM_PAIR_TURN 8          // stages of a group
-#define SM_PAIR_RANGE 0x1p-27f  // of the largest: above it both halves of a pair are normal numbers
+#define SM_PAIR_RANGE 0x1p-27f  // of the largest: from there on a pair holds 23 bits of a value
+#define SM_PAIR_LEAST 0x1p-13f  // the same of a scaled one
+// Values below that are summed one by one, at most.  The backward at 512 x 3136 x 48000, us: none 1345, 400 of them scattered 1432,
+// all in one column 1562, 600 (planes) 1918; without pairs 1922.
+#define SM_TINY_MOST 512
 
 __device__ __forceinline__ void softmap_pair(const float *v, uint4 &hi, uint4 &lo) {
     unsigned h[4], l[4];
@@ -348,15 +355,27 @@ __global__ __launch_bounds__(T, NQ == 8 ? 4 : 1) void softmap_rowstats(const flo
 // every second group of SM_GX_STAGE columns in the units along the columns.
 // NP = 2: pairs, or planes where `range` says so: units along the rows are gW's, which takes E from W and asks for x's range only.
 // `row_max` (units along the columns) and `col_max` (units along the rows): the magnitudes that the pairs are scaled by, without
-// them x_largest.
+// them x_largest.  `tiny`: how many values the pairs along the columns ([0]) and along the rows ([1]) leave out.  With `tiny_at`
+// this launch finds them and lists the first SM_TINY_MOST of each as (row of the product's result, step of its reduction); else
+// they are counted already, and where there are more than that the units along the rows are planes, with `again` those along the
+// columns too, and nothing else is written.
 template <int NP>
 __global__ __launch_bounds__(256) void softmap_pack(const float *__restrict__ src, const float *__restrict__ colscale,
                                                     const float *__restrict__ other, float *__restrict__ dots,
                                                     char *__restrict__ rows8, size_t rows_plane, char *__restrict__ cols8,
                                                     size_t cols_plane, int R, int C, int Rp, int Cp, float alternate, unsigned *__restrict__ largest,
                                                     unsigned *__restrict__ clear, const SoftmapRange *__restrict__ range,
-                                                    const unsigned *__restrict__ row_max, const unsigned *__restrict__ col_max) {
-    const bool row_pairs = NP == 2 && !softmap_x_wide(range), col_pairs = NP == 2 && !softmap_wide(range);
+                                                    const unsigned *__restrict__ row_max, const unsigned *__restrict__ col_max,
+                                                    unsigned *__restrict__ tiny, int2 *__restrict__ tiny_at, bool again) {
+    bool row_pairs = NP == 2 && !softmap_x_wide(range), col_pairs = NP == 2 && !softmap_wide(range);
+    if (NP == 2 && tiny && !tiny_at) {
+        const bool rows_many = row_pairs && tiny[1] > SM_TINY_MOST, cols_many = col_pairs && tiny[0] > SM_TINY_MOST;
+        if (again && !rows_many) rows8 = nullptr;
+        if (again && !cols_many) cols8 = nullptr;
+        if (!rows8 && !cols8) return;
+        row_pairs = row_pairs && !rows_many;
+        col_pairs = col_pairs && !cols_many;
+    }
     // (a grid of one dimension: the second holds 65535 blocks, 4.19 million rows)
     const int cb64 = Cp / 64, bx = blockIdx.x % cb64, by = blockIdx.x / cb64;
     if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0;
@@ -393,10 +412,23 @@ __global__ __launch_bounds__(256) void softmap_pack(const float *__restrict__ sr
     for (int i = 0; i < 16; ++i) tile[g * 16 + i][c] = v[i] * f;
     __syncthreads();
     if (other && g == 0) dots[(size_t)by * Cp + col] = ((part[0][c] + part[1][c]) + part[2][c]) + part[3][c];
-    auto put_pairs = [&](float *w, unsigned biggest, char *d, size_t plane) {
+    // eight steps of the reduction, from `step` on, of row `row` of the result
+    auto put_pairs = [&](float *w, unsigned biggest, char *d, size_t plane, int which, int row, int step) {
         const int shift = softmap_pair_shift(biggest);
+        unsigned left_out = 0;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) w[j] = __builtin_amdgcn_ldexpf(w[j], shift);
+        for (int j = 0; j < 8; ++j) {
+            const float scaled = __builtin_amdgcn_ldexpf(w[j], shift);
+            const bool out = w[j] != 0.0f && fabsf(scaled) < SM_PAIR_LEAST;
+            left_out |= out ? 1u << j : 0u;
+            w[j] = out ? 0.0f : scaled;
+        }
+        if (tiny_at && left_out != 0 && __hip_atomic_load(tiny + which, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <= SM_TINY_MOST) {
+            // (past the limit nobody looks at the list, and the number no longer matters)
+            unsigned at = atomicAdd(tiny + which, (unsigned)__popc(left_out));
+            for (; left_out != 0 && at < SM_TINY_MOST; ++at, left_out &= left_out - 1)
+                tiny_at[which * SM_TINY_MOST + at] = make_int2(row, step + __ffs(left_out) - 1);
+        }
         uint4 hi, lo;
         softmap_pair(w, hi, lo);
         *reinterpret_cast<uint4 *>(d) = hi;
@@ -409,7 +441,7 @@ __global__ __launch_bounds__(256) void softmap_pack(const float *__restrict__ sr
             if (8 * rb < Rp) {
                 char *d = rows8 + ((size_t)rb * Cp + col) * SM_UNIT;
                 if (row_pairs) {
-                    put_pairs(v + 8 * h, col_max ? col_max[col] : range->x_largest, d, rows_plane);
+                    put_pairs(v + 8 * h, col_max ? col_max[col] : range->x_largest, d, rows_plane, 1, col, rb * 8);
                     continue;
                 }
                 if (NP == 2) {
@@ -431,7 +463,7 @@ __global__ __launch_bounds__(256) void softmap_pack(const float *__restrict__ sr
                 for (int j = 0; j < 8; ++j) w[j] = tile[c][cb * 8 + j];
                 char *d = cols8 + ((size_t)(bx * 8 + cb) * Rp + row) * SM_UNIT;
                 if (col_pairs) {
-                    put_pairs(w, row_max ? row_max[row] : range->x_largest, d, cols_plane);
+                    put_pairs(w, row_max ? row_max[row] : range->x_largest, d, cols_plane, 0, row, (bx * 8 + cb) * 8);
                     continue;
                 }
                 if (NP == 2) {
@@ -449,8 +481,9 @@ __global__ __launch_bounds__(256) void softmap_pack(const float *__restrict__ sr
 // result is rounded once however many chunks there are (bound by the reads: no slower).
 template <int VEC>
 __global__ __launch_bounds__(256) void softmap_reduce_chunks(const float *__restrict__ part, float *__restrict__ out,
-                                                              long long total, int chunks, const SoftmapRange *range, int wide_chunks) {
-    if (range && softmap_wide(range)) chunks = wide_chunks;
+                                                              long long total, int chunks, const SoftmapRange *range, const unsigned *tiny,
+                                                              int wide_chunks) {
+    if (range && (softmap_wide(range) || (tiny && *tiny > SM_TINY_MOST))) chunks = wide_chunks;
     if (range && chunks == 1) return;  // it is in `out`
     const long long e = ((long long)blockIdx.x * 256 + threadIdx.x) * VEC;
     if (e >= total) return;
@@ -495,6 +528,7 @@ struct SoftmapArgs {
     // pairs
     const SoftmapRange *range;
     const unsigned *row_max;  // magnitudes that the rows of A are scaled by; forward: none (x_largest)
+    const unsigned *tiny;     // gx, gW: how many values the pairs of A leave out
 };
 
 // Loads that bypass the registers: lane l's 16 bytes at base + voff land at LDS address lds + 16 l.  The compiler does not
@@ -531,18 +565,26 @@ __device__ __forceinline__ void softmap_stage_barrier() {
 // given above, and have two blocks per CU.  The same sizes, forward / gx / gW: 503 / 473 / 575 us (planes 703 / 786 / 866).  Bound by power: the matrix cores are busy half of the time at 1.8 GHz.  256 x 128 tiles with one accumulator, the
 // rest's sum scaled and added by every stage: 514 / 560 / 668.  gx in
 // 5, 10 or 15 chunks of the reduction: 445, 486 and 497 with their sum; 10 for the shorter running sums.
-template <int MODE, int NP, int FA>
+// NPB = 2 with NP = 3 (gx): gs in planes, E in pairs, whose planes - times 2^10, which makes their scale the planes' - are made on
+// the way out of the LDS; for gradients that span too much where E does not.
+template <int MODE, int NP, int FA, int NPB>
 __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
     extern __shared__ __align__(16) char lds[];
-    if (NP > 1 && g.range && dl_uniform(MODE == 2 ? softmap_x_wide(g.range) : softmap_wide(g.range)) != (NP == 3)) return;
+    constexpr bool FROM_PAIRS = NP == 3 && NPB == 2;
+    static_assert(NPB == NP || (FROM_PAIRS && MODE == 1), "only gx mixes planes and pairs");
+    if (NP > 1 && g.range) {
+        const bool wide = dl_uniform(MODE == 2 ? softmap_x_wide(g.range) : softmap_wide(g.range));
+        const bool many = MODE != 0 && dl_uniform((int)(*g.tiny > SM_TINY_MOST));
+        if (NP == 2 ? wide || many : FROM_PAIRS ? wide || !many : MODE == 1 ? !wide : !wide && !many) return;
+    }
     constexpr int TR = 64 * FA, TC = SM_TC;
     constexpr int KC = NP == 1 ? 32 : SM_GX_STAGE, KB = KC / 8;
     constexpr int NBUF = NP == 3 && FA == 4 ? 2 : 3, AHEAD = NBUF - 1;
-    constexpr int A_BYTES = NP * TR * KC * 2, STAGE = NP * (TR + TC) * KC * 2;
+    constexpr int A_BYTES = NP * TR * KC * 2, STAGE = (NP * TR + NPB * TC) * KC * 2;
     constexpr bool BY_STAGE = NP == 3 && MODE == 1;
     static_assert(NP != 2 || FA == 2, "pairs keep two sums per output");
-    constexpr int NA = NP * KB * (TR / 64) / 4, NB = NP * KB * (TC / 64) / 4;  // loads per wavefront and stage
-    static_assert(NP * KB * (TR / 64) % 4 == 0 && NP * KB * (TC / 64) % 4 == 0, "whole loads per wavefront");
+    constexpr int NA = NP * KB * (TR / 64) / 4, NB = NPB * KB * (TC / 64) / 4;  // loads per wavefront and stage
+    static_assert(NP * KB * (TR / 64) % 4 == 0 && NPB * KB * (TC / 64) % 4 == 0, "whole loads per wavefront");
     typedef __attribute__((address_space(3))) char lds_char;
     const unsigned lds_base = (unsigned)(uintptr_t)(lds_char *)lds;  // what softmap_to_lds counts from
     int inner, outer;
@@ -629,7 +671,7 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
 #pragma unroll
             for (int p = 0; p < NP; ++p) {
 #pragma unroll
-                for (int j = 0; j < 2; ++j) {
+                for (int j = 0; p < NPB && j < 2; ++j) {
                     if (MODE == 0) {
                         typedef __attribute__((address_space(3))) shortx4 lds_shortx4;
                         const unsigned at = base + b_rd + (p * (TC / 8) * KC + j * 4 * KC + kk * 16) * SM_UNIT;
@@ -643,6 +685,17 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
 #pragma unroll
                 for (int i = 0; i < FA; ++i)
                     a[p][i] = *reinterpret_cast<const bf16x8 *>(lds + base + a_rd + ((p * KB + kk * 2) * TR + i * 32) * SM_UNIT);
+            }
+            if (FROM_PAIRS) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const halfx8 h = __builtin_bit_cast(halfx8, b[0][j]), l = __builtin_bit_cast(halfx8, b[1][j]);
+                    float e[8];
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) e[q] = fmaf((float)l[q], SM_SCALE / SM_PAIR_LO / (1 << SM_PAIR_EXP), (float)h[q] * (SM_SCALE / (1 << SM_PAIR_EXP)));
+#pragma unroll
+                    for (int p = 0; p < NP; ++p) b[p][j] = __builtin_bit_cast(bf16x8, softmap_unit(e));
+                }
             }
             // small products first
             constexpr int PA[6] = {0, 2, 1, 0, 1, 0}, PB[6] = {2, 0, 1, 1, 0, 0};
@@ -837,14 +890,14 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
     }
 }
 
-template <int MODE, int NP, int FA>
+template <int MODE, int NP, int FA, int NPB = NP>
 static void softmap_launch(const SoftmapArgs &g, hipStream_t s) {
     constexpr int KC = NP == 1 ? 32 : 16, NBUF = NP == 3 && FA == 4 ? 2 : 3;
-    constexpr int lds_bytes = NBUF * NP * (64 * FA + SM_TC) * KC * 2;
+    constexpr int lds_bytes = NBUF * (NP * 64 * FA + NPB * SM_TC) * KC * 2;
     if (lds_bytes > 65536)
-        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&softmap_mfma<MODE, NP, FA>),
+        (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&softmap_mfma<MODE, NP, FA, NPB>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
-    softmap_mfma<MODE, NP, FA><<<dl_xcd_grid(g.inner_count, g.outer_count), 256, lds_bytes, s>>>(g);
+    softmap_mfma<MODE, NP, FA, NPB><<<dl_xcd_grid(g.inner_count, g.outer_count), 256, lds_bytes, s>>>(g);
 }
 
 // ---------------------------------------------------------------------------------
@@ -860,6 +913,9 @@ struct SoftmapPlain {
     const unsigned *x_largest, *gm_largest;
     int B, I, M, parts, dot_ld;
     float scale, inv_tau;
+    const SoftmapRange *range;  // pairs: what decided between them and planes
+    const unsigned *tiny;       // and the values of gs ([0]) and gm ([1]) that they leave out
+    const int2 *tiny_at;
 };
 #define SM_PT 128  // edge of a tile
 #define SM_PLD 132 // its row in the LDS
@@ -975,6 +1031,39 @@ __device__ void softmap_plain_tile(const SoftmapPlain &p, float (&As)[16][SM_PLD
             }
         }
 }
+// The terms of the values that the pairs leave out, added to gx (MODE 1) or gW (MODE 2): a block has a row of the result and
+// 256 of its columns, and takes the row's values in order, so that the sums are the same every time.
+template <int MODE>
+__device__ void softmap_tiny_terms(const SoftmapPlain &p, const int2 *__restrict__ found, int count, int2 *list) {
+    __syncthreads();  // (`list`, of twice SM_TINY_MOST, may hold the other result's)
+    int2 *as_found = list + SM_TINY_MOST;
+    for (int e = threadIdx.x; e < count; e += 256) as_found[e] = found[e];
+    __syncthreads();
+    for (int e = threadIdx.x; e < count; e += 256) {
+        const int2 mine = as_found[e];
+        int rank = 0;
+        for (int q = 0; q < count; ++q) {
+            const int2 v = as_found[q];
+            rank += v.x < mine.x || (v.x == mine.x && v.y < mine.y) ? 1 : 0;
+        }
+        list[rank] = mine;
+    }
+    __syncthreads();
+    const int strips = (p.I + 255) / 256;
+    for (int it = blockIdx.x; it < count * strips; it += gridDim.x) {
+        const int first = it / strips, i = it % strips * 256 + (int)threadIdx.x, row = list[first].x;
+        if ((first > 0 && list[first - 1].x == row) || i >= p.I) continue;
+        float sum = 0.0f;
+        for (int e = first; e < count && list[e].x == row; ++e) {
+            const int k = list[e].y;
+            if (MODE == 1) sum = fmaf(p.gm[(size_t)row * p.M + k] * p.rs[k], softmap_e(p.W[(size_t)k * p.I + i], p.mx[k], p.scale), sum);
+            else sum = fmaf(p.gm[(size_t)k * p.M + row], p.x[(size_t)k * p.I + i], sum);
+        }
+        const size_t at = (size_t)row * p.I + i;
+        if (MODE == 1) p.gx[at] += sum;
+        else p.gW[at] = fmaf(sum, softmap_e(p.W[at], p.mx[row], p.scale) * (p.rs[row] * p.inv_tau), p.gW[at]);
+    }
+}
 template <bool BWD>
 __global__ __launch_bounds__(256, 2) void softmap_plain(SoftmapPlain p) {
     __shared__ float As[16][SM_PLD], Bs[16][SM_PLD];
@@ -987,12 +1076,22 @@ __global__ __launch_bounds__(256, 2) void softmap_plain(SoftmapPlain p) {
             softmap_plain_tile<0>(p, As, Bs, (int)(t % bt) * SM_PT, (int)(t / bt) * SM_PT);
         return;
     }
-    if (!(gm * (float)p.M < SM_BOUND))
+    __shared__ int2 list[BWD ? 2 * SM_TINY_MOST : 1];
+    // (values are left out where the pairs ran: not by planes, which they gave way to beyond SM_TINY_MOST)
+    const int rows_tiny = p.range && !softmap_wide(p.range) && p.tiny[0] <= SM_TINY_MOST ? (int)p.tiny[0] : 0;
+    const int cols_tiny = p.range && !softmap_x_wide(p.range) && p.tiny[1] <= SM_TINY_MOST ? (int)p.tiny[1] : 0;
+    if (!(gm * (float)p.M < SM_BOUND)) {
         for (long long t = blockIdx.x; t < (long long)bt * it; t += gridDim.x)
             softmap_plain_tile<1>(p, As, Bs, (int)(t / it) * SM_PT, (int)(t % it) * SM_PT);
-    if (!(gm * (float)p.B * x < SM_BOUND))
+    } else if (rows_tiny > 0) {
+        softmap_tiny_terms<1>(p, p.tiny_at, rows_tiny, list);
+    }
+    if (!(gm * (float)p.B * x < SM_BOUND)) {
         for (long long t = blockIdx.x; t < (long long)mt * it; t += gridDim.x)
             softmap_plain_tile<2>(p, As, Bs, (int)(t / it) * SM_PT, (int)(t % it) * SM_PT);
+    } else if (cols_tiny > 0) {
+        softmap_tiny_terms<2>(p, p.tiny_at + SM_TINY_MOST, cols_tiny, list);
+    }
 }
 #define SM_PLAIN_BLOCKS 512  // two per CU
 
@@ -1029,7 +1128,7 @@ static void softmap_chunks(int stages, long long tiles, long long blocks, int *c
     *chunk = dl_ceil_div(stages, n);
     *chunks = dl_ceil_div(stages, *chunk);
 }
-// Pairs cost a pass over x and one over gm and seven launches of about 5 us a step, four of which end at once.  Measured, forward +
+// Pairs cost a pass over x and one over gm and ten launches of about 5 us a step, six of which end at once.  Measured, forward +
 // backward, planes against pairs: 512 x 512 x 24000 (6.3e9) 332 -> 322 us, 64 x 3136 x 30000 (6.0e9) 716 -> 594, 300 x 1500 x 20000
 // (9.0e9) 578 -> 468, 512 x 3136 x 48000 2659 -> 2562 where E spans too much; below, planes.
 #define SM_PAIR_WORK 6e9
@@ -1069,7 +1168,8 @@ extern "C" size_t dl_soft_map_saved_bytes(int B, int I, int M, int precision) {
 }
 
 // workspace: partial products of the forward or of gx, partial r, x and gm in units along the batch, gs along the rows of W, the
-// largest magnitude of gm, those of the rows of gs and the columns of gm
+// largest magnitude of gm (and how many values of gs and gm the pairs leave out), those of the rows of gs and the columns of gm,
+// where the values left out are
 static inline size_t softmap_part_bytes(const SoftmapShape &h) {
     int nf = h.fwd_chunks, ng = h.gx_chunks;
     if (h.pairs && h.pair_fwd_chunks > nf) nf = h.pair_fwd_chunks;
@@ -1084,7 +1184,7 @@ extern "C" size_t dl_soft_map_workspace_bytes(int B, int I, int M, int precision
     if (B <= 0 || I <= 0 || M <= 0) return 256;
     const SoftmapShape h = softmap_shape(B, I, M, precision);
     return 256 + softmap_part_bytes(h) + softmap_dots_bytes(h) + h.np * (h.x_plane + 2 * h.g_plane) +
-           (h.pairs ? dl_align256((size_t)(h.Bp + h.Mp) * sizeof(unsigned)) : 0);
+           (h.pairs ? dl_align256((size_t)(h.Bp + h.Mp) * sizeof(unsigned)) + 2 * SM_TINY_MOST * sizeof(int2) : 0);
 }
 
 template <int NP>
@@ -1103,22 +1203,23 @@ static void softmap_stats_launch(const SoftmapShape &h, const float *W, float sc
 static void softmap_pack_launch(int np, const float *src, const float *colscale, const float *other, float *dots, char *rows8,
                                 size_t rows_plane, char *cols8, size_t cols_plane, int R, int C, int Rp, int Cp, float alternate,
                                 unsigned *largest, unsigned *clear, const SoftmapRange *range, const unsigned *row_max,
-                                const unsigned *col_max, hipStream_t s) {
+                                const unsigned *col_max, unsigned *tiny, int2 *tiny_at, bool again, hipStream_t s) {
     const int grid = Cp / 64 * dl_ceil_div(Rp, 64);
 #define SM_PACK(NP) \
-    DL_TIMED("softmap_pack", s, (softmap_pack<NP><<<grid, 256, 0, s>>>(src, colscale, other, dots, rows8, rows_plane, cols8, cols_plane, R, C, Rp, Cp, alternate, largest, clear, range, row_max, col_max)))
+    DL_TIMED("softmap_pack", s, (softmap_pack<NP><<<grid, 256, 0, s>>>(src, colscale, other, dots, rows8, rows_plane, cols8, cols_plane, R, C, Rp, Cp, alternate, largest, clear, range, row_max, col_max, tiny, tiny_at, again)))
     if (np == 1) SM_PACK(1);
     else if (range) SM_PACK(2);
     else SM_PACK(3);
 #undef SM_PACK
 }
-static void softmap_reduce(const float *part, float *out, long long total, int chunks, const SoftmapRange *range, int wide_chunks, hipStream_t s) {
+static void softmap_reduce(const float *part, float *out, long long total, int chunks, const SoftmapRange *range, const unsigned *tiny,
+                           int wide_chunks, hipStream_t s) {
     if (total % 4 == 0 && ((uintptr_t)out & 15) == 0)
         DL_TIMED("softmap_reduce_chunks", s,
-                 (softmap_reduce_chunks<4><<<dl_ceil_div(total / 4, 256), 256, 0, s>>>(part, out, total, chunks, range, wide_chunks)));
+                 (softmap_reduce_chunks<4><<<dl_ceil_div(total / 4, 256), 256, 0, s>>>(part, out, total, chunks, range, tiny, wide_chunks)));
     else
         DL_TIMED("softmap_reduce_chunks", s,
-                 (softmap_reduce_chunks<1><<<dl_ceil_div(total, 256), 256, 0, s>>>(part, out, total, chunks, range, wide_chunks)));
+                 (softmap_reduce_chunks<1><<<dl_ceil_div(total, 256), 256, 0, s>>>(part, out, total, chunks, range, tiny, wide_chunks)));
 }
 template <int MODE>
 static void softmap_product(const char *name, const SoftmapShape &h, int fa, const SoftmapArgs &g, hipStream_t s) {
@@ -1163,7 +1264,7 @@ extern "C" int dl_soft_map_fwd(const float *x, const float *W, float tau, float 
         softmap_stats_launch<3>(h, W, scale, mx, rs, E, nullptr, range, s);
     }
     softmap_pack_launch(h.np, x, nullptr, nullptr, nullptr, nullptr, 0, x8, h.x_plane, B, I, h.Bp, h.Ip, 1.0f, h.pairs ? nullptr : x_largest,
-                        nullptr, range, nullptr, nullptr, s);
+                        nullptr, range, nullptr, nullptr, nullptr, nullptr, false, s);
     SoftmapArgs g{};
     g.A = x8; g.a_plane = h.x_plane; g.lda = h.Bp;
     g.Bm = E; g.b_plane = h.e_plane; g.ldb = h.Ip;
@@ -1183,7 +1284,7 @@ extern "C" int dl_soft_map_fwd(const float *x, const float *W, float tau, float 
     product(h.row_tiles, h.fwd_chunk, h.fwd_chunks);
     softmap_product<0>("softmap_fwd", h, h.fa, g, s);
     if (h.pairs ? h.pair_fwd_chunks > 1 || h.fwd_chunks > 1 : h.fwd_chunks > 1)
-        softmap_reduce((const float *)ws, m, (long long)B * M, h.pairs ? h.pair_fwd_chunks : h.fwd_chunks, range, h.fwd_chunks, s);
+        softmap_reduce((const float *)ws, m, (long long)B * M, h.pairs ? h.pair_fwd_chunks : h.fwd_chunks, range, nullptr, h.fwd_chunks, s);
     if (h.np > 1) {
         SoftmapPlain q{};
         q.x = x; q.W = W; q.mx = mx; q.rs = rs; q.m = m; q.x_largest = x_largest;
@@ -1222,17 +1323,27 @@ extern "C" int dl_soft_map_bwd(const float *x, const float *W, float tau, const 
         DL_TIMED("softmap_clear", s, (softmap_clear<<<dl_ceil_div(words, 256), 256, 0, s>>>(nullptr, gm_largest, words)));
         DL_TIMED("softmap_scan", s, (softmap_scan_grad<<<(unsigned)strips * dl_ceil_div(B, 64), 256, 0, s>>>(gm, rs, row_max, col_max, gm_largest, range, B, M, strips)));
     }
-    softmap_pack_launch(h.np, x, nullptr, nullptr, nullptr, xb, h.x_plane, nullptr, 0, B, I, h.Bp, h.Ip, 1.0f, nullptr,
-                        h.pairs ? nullptr : gm_largest, range, nullptr, nullptr, s);
+    unsigned *tiny = h.pairs ? gm_largest + 2 : nullptr;
+    int2 *tiny_at = h.pairs ? (int2 *)(w + 256 + dl_align256((size_t)(h.Bp + h.Mp) * sizeof(unsigned))) : nullptr;
+    auto pack_x = [&]() {
+        softmap_pack_launch(h.np, x, nullptr, nullptr, nullptr, xb, h.x_plane, nullptr, 0, B, I, h.Bp, h.Ip, 1.0f, nullptr,
+                            h.pairs ? nullptr : gm_largest, range, nullptr, nullptr, tiny, nullptr, false, s);
+    };
+    if (!h.pairs) pack_x();  // which clears gm_largest for the next
     softmap_pack_launch(h.np, gm, rs, m, dots, gb, h.g_plane, go, h.g_plane, B, M, h.Bp, h.Mp, -1.0f, gm_largest, nullptr,
-                        range, row_max, col_max, s);
+                        range, row_max, col_max, tiny, tiny_at, false, s);
+    if (h.pairs) {
+        softmap_pack_launch(h.np, gm, rs, nullptr, nullptr, gb, h.g_plane, go, h.g_plane, B, M, h.Bp, h.Mp, -1.0f, nullptr, nullptr,
+                            range, row_max, col_max, tiny, nullptr, true, s);
+        pack_x();
+    }
     SoftmapArgs g{};
     g.A = go; g.a_plane = h.g_plane; g.lda = h.Bp;
     g.Bm = E; g.b_plane = h.e_plane; g.ldb = h.Ip;
     g.R = B; g.C = I;
     g.stages = h.gx_stages;
     g.col_tiles = h.gx_col_tiles;
-    g.range = range; g.row_max = row_max;
+    g.range = range; g.row_max = row_max; g.tiny = tiny;
     auto product = [&](int row_tiles, int chunk, int chunks) {
         g.out = chunks > 1 ? part : gx;
         g.chunk_stages = chunk;
@@ -1244,8 +1355,12 @@ extern "C" int dl_soft_map_bwd(const float *x, const float *W, float tau, const 
     }
     product(h.row_tiles, h.gx_chunk, h.gx_chunks);
     softmap_product<1>("softmap_gx", h, h.fa, g, s);
+    if (h.pairs) {
+        if (h.fa == 4) DL_TIMED("softmap_gx", s, (softmap_launch<1, 3, 4, 2>(g, s)));
+        else DL_TIMED("softmap_gx", s, (softmap_launch<1, 3, 2, 2>(g, s)));
+    }
     if (h.pairs ? h.pair_gx_chunks > 1 || h.gx_chunks > 1 : h.gx_chunks > 1)
-        softmap_reduce(part, gx, (long long)B * I, h.pairs ? h.pair_gx_chunks : h.gx_chunks, range, h.gx_chunks, s);
+        softmap_reduce(part, gx, (long long)B * I, h.pairs ? h.pair_gx_chunks : h.gx_chunks, range, tiny, h.gx_chunks, s);
     // gW: tiles of 256 rows of W where they fill the card, else of 128
     const int fa = (long long)(h.Mp / 256) * h.gx_col_tiles >= 512 ? 4 : 2;
     SoftmapArgs q{};
@@ -1257,7 +1372,7 @@ extern "C" int dl_soft_map_bwd(const float *x, const float *W, float tau, const 
     q.inner_count = h.gx_col_tiles; q.col_tiles = h.gx_col_tiles;
     q.rs = rs; q.dots = dots; q.parts = dl_ceil_div(B, 64); q.dot_ld = h.Mp;
     q.mx = mx; q.W = W; q.E = E; q.lde = h.Ip; q.scale = SM_LOG2E / tau; q.inv_tau = 1.0f / tau;
-    q.range = range; q.row_max = col_max;
+    q.range = range; q.row_max = col_max; q.tiny = h.pairs ? tiny + 1 : nullptr;
     q.vec_out = (((uintptr_t)W | (uintptr_t)gW) & 15) == 0;
     if (h.pairs) {
         q.outer_count = dl_ceil_div(M, 128);
@@ -1269,6 +1384,7 @@ extern "C" int dl_soft_map_bwd(const float *x, const float *W, float tau, const 
         SoftmapPlain u{};
         u.x = x; u.W = W; u.gm = gm; u.mx = mx; u.rs = rs; u.dots = dots; u.gx = gx; u.gW = gW;
         u.x_largest = x_largest; u.gm_largest = gm_largest;
+        u.range = range; u.tiny = tiny; u.tiny_at = tiny_at;
         u.B = B; u.I = I; u.M = M; u.parts = q.parts; u.dot_ld = q.dot_ld; u.scale = q.scale; u.inv_tau = q.inv_tau;
         const int grid = softmap_plain_grid((long long)(M > B ? dl_ceil_div(M, SM_PT) : dl_ceil_div(B, SM_PT)) * dl_ceil_div(I, SM_PT));
         DL_TIMED("softmap_plain", s, (softmap_plain<true><<<grid, 256, 0, s>>>(u)));

@@ -944,6 +944,75 @@ def test_soft_mapping_fp32_pairs(shape, case):
         assert rows.all(), (name, float((diff.norm(dim=1) / size.norm(dim=1)).nan_to_num().max()))
 
 
+@pytest.mark.parametrize("case", ["blank_sample", "blank_sample_512", "blank_sample_513", "masked_weights", "masked_weights_few",
+                                  "any_magnitude", "few_of_any_magnitude", "wide_e_any_magnitude", "wide_x_any_magnitude"])
+@pytest.mark.parametrize("shape", [(257, 515, 50001), (100, 1030, 60100)])
+def test_soft_mapping_fp32_pairs_gradients_of_any_span(shape, case):
+    """Gradients whose smallest values lie below what a pair holds beside the largest, where only they make a result: exact zeros
+    in x or in the softmax take the large ones out of it.  Every element of m, gx and gW against float64, relative to the sum of
+    its own terms' magnitudes: a product is good to 2^-22, a sum of n fp32 terms, in whatever order, on average to sqrt(n) 2^-24,
+    60100 terms 1.5e-5 if they rounded one by one; they go in groups of 16 and more, so a quarter of it."""
+    ops = _ops()
+    B, I, M = shape
+    g = torch.Generator("cuda").manual_seed(B + len(case))
+    x = torch.rand(B, I, device="cuda", generator=g) + 0.01
+    W = torch.randn(M, I, device="cuda", generator=g)
+    gm = torch.randn(B, M, device="cuda", generator=g)
+    small = torch.randn(B, M, device="cuda", generator=g) * 2.0 ** -45
+    if case == "blank_sample":  # the largest gradients belong to a sample without input
+        x[0] = 0.0
+        gm[1:] = small[1:]
+    elif case.startswith("blank_sample_"):  # in a few columns: as many values as are summed one by one, and one more
+        x[0] = 0.0
+        gm = torch.where(gm < 0, gm - 0.01, gm + 0.01)  # no small values but those
+        gm[0] = gm[0].abs() + 1.0
+        first = int(case.rsplit("_", 1)[1])
+        cols = torch.arange(1, 1 + first // (B - 1), device="cuda")
+        gm[1:, cols] = small[1:, cols].abs() + 2.0 ** -46
+        rest = first % (B - 1)
+        gm[1 : 1 + rest, M - 1] = 2.0 ** -46
+        gm[1 + rest :, M - 1] = 0.0
+    elif case.startswith("masked_weights"):  # no row of W with large gradients reads the first inputs
+        few = case.endswith("few")
+        rows = torch.tensor([3, 700, M - 2] if few else [7], device="cuda")
+        if few:
+            W[:, :9] = -float("inf")
+            W[rows, :9] = 0.0
+            gm[:, rows] = small[:, rows]
+        else:
+            W[rows, : I // 2] = -float("inf")
+            gm = small
+            gm[:, rows] = 1.0
+    else:
+        powers = torch.rand(B, M, device="cuda", generator=g) * 100.0 - 90.0
+        spread = gm * torch.exp2(powers)
+        if case == "few_of_any_magnitude":
+            gm[5, 100:150], gm[90, 41:300] = spread[5, 100:150], spread[90, 41:300]
+        else:
+            gm = spread
+        x[:, ::3] = 0.0
+        W[:, 1::4] = -float("inf")
+        W[::2, 2::4] = -float("inf")
+        if case.startswith("wide_e"):
+            W[M - 1, 0] = 25.0
+        elif case.startswith("wide_x"):
+            x[B - 1] *= 1e-12
+    xt, Wt = x.clone().requires_grad_(), W.clone().requires_grad_()
+    m = ops.SoftMapFunction.apply(xt, Wt, 1.0, 0)
+    again = torch.autograd.grad(m, (xt, Wt), gm, retain_graph=True)
+    m.backward(gm)
+    assert torch.equal(xt.grad, again[0]) and torch.equal(Wt.grad, again[1])
+    xd, gd = x.double(), gm.double()
+    S = torch.softmax(W.double(), dim=-1)
+    md = xd @ S.t()
+    G, r = gd.t() @ xd, (gd * md).sum(0)
+    for name, got, want, size in (("m", m.detach(), md, md), ("gx", xt.grad, gd @ S, gd.abs() @ S),
+                                  ("gW", Wt.grad, S * (G - r[:, None]), S * (gd.abs().t() @ xd + (gd * md).abs().sum(0)[:, None]))):
+        error = (got.double() - want).abs()
+        worst = float((error / (size + 1e-37)).max())
+        assert worst <= 4e-6, (name, worst)
+
+
 @pytest.mark.parametrize("precision", [0, 1])
 def test_soft_mapping_of_more_rows_than_a_grid_dimension(precision):
     """4.19 million rows are 65536 blocks of 64 rows; limits as in test_soft_mapping_tile_edges."""
