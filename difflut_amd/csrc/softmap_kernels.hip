@@ -242,10 +242,16 @@ __global__ __launch_bounds__(T, NQ == 8 ? 4 : 1) void softmap_rowstats(const flo
                                                       int I, int Ip, unsigned *__restrict__ largest,
                                                       SoftmapRange *__restrict__ range) {
     constexpr int WV = T / 64;
-    if (NP == 2 && (softmap_x_wide(range) || __hip_atomic_load(&range->e_wide, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)) return;
+    if (NP == 2 && softmap_x_wide(range)) return;
     if (NP == 3 && range && !softmap_wide(range)) return;
     __shared__ float red[2][8][WV];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    if (NP == 2) {  // read once for the block: another may set it meanwhile, and the barriers below are for all wavefronts or none
+        __shared__ unsigned found_wide;
+        if (tid == 0) found_wide = __hip_atomic_load(&range->e_wide, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (found_wide != 0) return;
+    }
     const int o0 = blockIdx.x * 8;
     uint4 *out = reinterpret_cast<uint4 *>(E + (size_t)blockIdx.x * Ip * SM_UNIT);
     float v[NQ > 0 ? NQ : 1][8];
