@@ -298,6 +298,7 @@ struct SoftMap : torch::autograd::Function<SoftMap> {
         require_device(x_);
         require_device(W_);
         const Tensor x = f32(x_), W = f32(W_);
+        TORCH_CHECK_VALUE(x.dim() == 2, "expected x [B, I], got ", x.sizes());
         const int B = (int)x.size(0), I = (int)x.size(1), M = (int)W.size(0), prec = (int)precision;
         TORCH_CHECK(W.size(1) == I, "shape mismatch: x ", x.sizes(), " vs W ", W.sizes());
         const Tensor m = floats({B, M}, x), stats = bytes(L.dl_soft_map_saved_bytes(B, I, M, prec), x),

@@ -153,3 +153,9 @@ def test_the_current_stream_and_tensors_on_the_cpu(name):
     assert torch.equal(out, y) and all(torch.equal(a, b) for a, b in zip(side_grads, grads))
     with pytest.raises(RuntimeError, match="ROCm devices only"):
         call(*[t.cpu() for t in inputs])
+
+
+@pytest.mark.parametrize("shape", [(8,), (4, 8, 2), (4, 8, 1), ()])
+def test_soft_map_refuses_inputs_that_are_no_matrix(shape):
+    with pytest.raises((ValueError, IndexError, RuntimeError)):
+        _ops().SoftMapFunction.apply(torch.rand(shape, device=DEV), torch.rand(6, 8, device=DEV), 1.0, 0)
