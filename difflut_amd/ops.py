@@ -186,8 +186,11 @@ class DWNStackFunction:
                               (bool [rows, C*KH*KW], optional): patch entries the bit-flip augmentation inverts."""
         nat.require_device(x, source if torch.is_tensor(source) else None, *luts)
         groups, tau = head if head is not None else (0, 1.0)
-        values = [(alpha, beta[0], 0.0, beta[1]) if beta[1:] else (None, None, alpha, beta[0])
-                  for alpha, *beta in scalars]
+        def node_values(v, plan):  # a number stands for every node's value
+            return v if torch.is_tensor(v) else _per_node(v, plan.N, x.device)
+
+        values = [(node_values(alpha, p), node_values(beta[0], p), 0.0, beta[1]) if beta[1:] else (None, None, alpha, beta[0])
+                  for p, (alpha, *beta) in zip(plans, scalars)]
         thresholds, geom, flip = None, (), None
         if torch.is_tensor(source):
             thresholds = source

@@ -159,3 +159,21 @@ def test_the_current_stream_and_tensors_on_the_cpu(name):
 def test_soft_map_refuses_inputs_that_are_no_matrix(shape):
     with pytest.raises((ValueError, IndexError, RuntimeError)):
         _ops().SoftMapFunction.apply(torch.rand(shape, device=DEV), torch.rand(6, 8, device=DEV), 1.0, 0)
+
+
+@pytest.mark.parametrize("alpha,beta", [(0.3, "tensor"), ("tensor", 0.25), (0.3, 0.25), ([0.3], "tensor")])
+def test_stack_takes_a_number_beside_per_node_values(alpha, beta):
+    ops = _ops()
+    _, (x, luts, luts2) = _calls()["stack"]
+    plan = ops.MappingPlan(torch.arange(65 * 4, device=DEV, dtype=torch.int32).reshape(65, 4) % 40, 40)
+    plan2 = ops.MappingPlan(torch.arange(64 * 4, device=DEV, dtype=torch.int32).reshape(64, 4) % 65, 65)
+
+    def scalars(n, as_given):
+        return tuple(torch.full((n,), fill, device=DEV) if v == "tensor" or not as_given else v for v, fill in ((alpha, 0.3), (beta, 0.25)))
+
+    def run(as_given):
+        both = [scalars(n, as_given) + (0.25,) for n in (65, 64)]
+        return _run(lambda a, s, t: ops.DWNStackFunction.apply(a, None, [plan, plan2], both, None, s, t), [x, luts, luts2])
+
+    (y, grads), (want, want_grads) = run(True), run(False)
+    assert torch.equal(y, want) and all(torch.equal(a, b) for a, b in zip(grads, want_grads))
