@@ -107,14 +107,15 @@ _host = None
 
 
 def is_built():
-    return os.path.exists(LIB_PATH)
+    """Whether both libraries are there: the kernels, and the autograd functions that training and chained inference go through."""
+    return os.path.exists(LIB_PATH) and os.path.exists(HOST_PATH)
 
 
 def lib():
     """Load the shared library once; raises RuntimeError when it has not been built."""
     global _lib
     if _lib is None:
-        if not is_built():
+        if not os.path.exists(LIB_PATH):
             raise RuntimeError(
                 f"HIP extension not available: {LIB_PATH} is missing. Build it with "
                 "`python -m difflut_amd.build` (needs hipcc); device tensors have no other path.")

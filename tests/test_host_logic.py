@@ -35,6 +35,24 @@ def test_library_exports_every_declared_symbol():
     assert nat.lib().dl_dwn_fwd_workspace_bytes(4096, 16384, 8192, 6, 1) == 64 * 16384 * 8
 
 
+@pytest.mark.parametrize("missing", ["LIB_PATH", "HOST_PATH"])
+def test_not_built_without_either_library(monkeypatch, tmp_path, missing):
+    """Layers and nodes offer their kernels by is_built(): a tree with one library of two does not have them."""
+    from difflut_amd import _native as nat
+
+    for name in ("LIB_PATH", "HOST_PATH"):
+        path = tmp_path / os.path.basename(getattr(nat, name))
+        path.write_bytes(b"")
+        monkeypatch.setattr(nat, name, str(path))
+    assert nat.is_built()
+    os.remove(getattr(nat, missing))
+    assert not nat.is_built()
+    monkeypatch.setattr(nat, "_host", None)
+    monkeypatch.setattr(nat, "_lib", None if missing == "LIB_PATH" else object())
+    with pytest.raises(RuntimeError, match=os.path.basename(getattr(nat, missing))):
+        nat.host()
+
+
 def test_registry_names_and_errors():
     from difflut_amd import REGISTRY
     from difflut_amd.layers import LearnableLayer, RandomLayer
