@@ -1462,6 +1462,7 @@ static inline bool dwn_wide(int N, int k, int O) {
 }
 static inline bool dwn_lanes(int N, int k, int O) { return dwn_fast(N, k, O) || dwn_wide(N, k, O); }
 
+extern "C" int dl_dwn_bwd_reads_x(int N, int k, int O) { return dwn_lanes(N, k, O) ? 0 : 1; }
 extern "C" size_t dl_dwn_saved_bytes(int B, int I, int N, int k, int O) {
     (void)I;
     if (!dwn_lanes(N, k, O)) return 256;  // nothing is kept; a token allocation keeps callers simple

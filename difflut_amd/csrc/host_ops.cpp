@@ -21,19 +21,19 @@ namespace {
 
 // ------------------------------------------------------------------ the library
 #define DL_FUNCTIONS(X)                                                                                                  \
-    X(dl_error_string) X(dl_dwn_saved_bytes) X(dl_dwn_fwd_workspace_bytes) X(dl_dwn_bwd_workspace_bytes) X(dl_dwn_layer_fwd) \
-    X(dl_dwn_layer_bwd) X(dl_dwn_layer_bwd_nodes) X(dl_dwn_stable_layer_bwd) X(dl_table_sigmoid_fwd) X(dl_table_sigmoid_bwd) \
-    X(dl_hybrid_saved_bytes) X(dl_hybrid_fwd_workspace_bytes) X(dl_hybrid_bwd_workspace_bytes)                               \
-    X(dl_hybrid_bwd_saved_workspace_bytes) X(dl_hybrid_layer_fwd) X(dl_hybrid_layer_bwd) X(dl_hybrid_layer_bwd_saved)         \
-    X(dl_prob_saved_bytes) X(dl_prob_bwd_saved_workspace_bytes) X(dl_prob_layer_fwd) X(dl_prob_layer_fwd_nodes)               \
-    X(dl_prob_layer_bwd) X(dl_prob_layer_bwd_nodes) X(dl_soft_map_saved_bytes) X(dl_soft_map_workspace_bytes)                 \
-    X(dl_soft_map_fwd) X(dl_soft_map_bwd) X(dl_unfold_rows) X(dl_unfold_flip) X(dl_fold) X(dl_dwn_planes_bytes)               \
-    X(dl_dwn_tiled_bytes) X(dl_dwn_pack_planes) X(dl_thermometer_planes) X(dl_dwn_groups_workspace_bytes)                     \
-    X(dl_dwn_layer_fwd_planes) X(dl_dwn_layer_fwd_planes_groups) X(dl_dwn_layer_eval_planes)                                  \
-    X(dl_dwn_layer_eval_planes_groups) X(dl_dwn_layer_bwd_groups) X(dl_dwn_layer_bwd_tiled) X(dl_dwn_chain_fusable)           \
-    X(dl_dwn_bwd_fused_workspace_bytes) X(dl_dwn_layer_bwd_chain_fused) X(dl_dwn_chain_first_fusable)                         \
-    X(dl_dwn_bwd_first_workspace_bytes) X(dl_dwn_layer_bwd_chain_first) X(dl_cross_entropy_workspace_bytes)                   \
-    X(dl_cross_entropy) X(dl_adam_step)
+    X(dl_error_string) X(dl_dwn_saved_bytes) X(dl_dwn_fwd_workspace_bytes) X(dl_dwn_bwd_workspace_bytes)                 \
+    X(dl_dwn_bwd_reads_x) X(dl_dwn_layer_fwd) X(dl_dwn_layer_bwd) X(dl_dwn_layer_bwd_nodes) X(dl_dwn_stable_layer_bwd)   \
+    X(dl_table_sigmoid_fwd) X(dl_table_sigmoid_bwd) X(dl_hybrid_saved_bytes) X(dl_hybrid_fwd_workspace_bytes)            \
+    X(dl_hybrid_bwd_workspace_bytes) X(dl_hybrid_bwd_saved_workspace_bytes) X(dl_hybrid_layer_fwd)                       \
+    X(dl_hybrid_layer_bwd) X(dl_hybrid_layer_bwd_saved) X(dl_prob_saved_bytes) X(dl_prob_bwd_saved_workspace_bytes)      \
+    X(dl_prob_layer_fwd) X(dl_prob_layer_fwd_nodes) X(dl_prob_layer_bwd) X(dl_prob_layer_bwd_nodes)                      \
+    X(dl_soft_map_saved_bytes) X(dl_soft_map_workspace_bytes) X(dl_soft_map_fwd) X(dl_soft_map_bwd) X(dl_unfold_rows)    \
+    X(dl_unfold_flip) X(dl_fold) X(dl_dwn_planes_bytes) X(dl_dwn_tiled_bytes) X(dl_dwn_pack_planes)                      \
+    X(dl_thermometer_planes) X(dl_dwn_groups_workspace_bytes) X(dl_dwn_layer_fwd_planes)                                 \
+    X(dl_dwn_layer_fwd_planes_groups) X(dl_dwn_layer_eval_planes) X(dl_dwn_layer_eval_planes_groups)                     \
+    X(dl_dwn_layer_bwd_groups) X(dl_dwn_layer_bwd_tiled) X(dl_dwn_chain_fusable) X(dl_dwn_bwd_fused_workspace_bytes)     \
+    X(dl_dwn_layer_bwd_chain_fused) X(dl_dwn_chain_first_fusable) X(dl_dwn_bwd_first_workspace_bytes)                    \
+    X(dl_dwn_layer_bwd_chain_first) X(dl_cross_entropy_workspace_bytes) X(dl_cross_entropy) X(dl_adam_step)
 struct Library {
 #define X(name) decltype(&::name) name = nullptr;
     DL_FUNCTIONS(X)
@@ -110,11 +110,8 @@ Dims lookup_dims(const Tensor &x, const Tensor &luts, const Plan &p) {
                 ", luts ", luts.sizes(), ", mapping [", p.N, ",", p.k, "] over ", p.I, " inputs");
     return {(int)x.size(0), (int)x.size(1), (int)luts.size(0), p.k, (int)luts.size(1)};
 }
-// whether the DWN backward needs x: not where the forward leaves the address of every node and row (k <= 6 and, within the
-// bounds of the library's dwn_wide, 7 and 8)
-bool backward_reads_x(const Dims &d) {
-    return d.k > 8 || (d.k > 6 && !(d.N < (1 << 23) && (int64_t)d.N * d.O * ((int64_t)4 << d.k) < 0x7fffffffLL));
-}
+// whether the DWN backward needs x: not where the forward leaves the address of every node and row
+bool backward_reads_x(const Dims &d) { return L.dl_dwn_bwd_reads_x(d.N, d.k, d.O) != 0; }
 std::pair<Tensor, Tensor> dwn_lookup(const Tensor &x, const Tensor &luts, const Plan &p, const Dims &d) {
     Tensor y = floats({d.B, (int64_t)d.N * d.O}, x), saved = bytes(L.dl_dwn_saved_bytes(DIMS(d)), x),
            ws = bytes(L.dl_dwn_fwd_workspace_bytes(DIMS(d)), x);

@@ -90,6 +90,8 @@ int dl_gather_bwd(const float *gm, const int32_t *inv_ptr, const int32_t *inv_po
 size_t dl_dwn_saved_bytes(int B, int I, int N, int k, int O);
 size_t dl_dwn_fwd_workspace_bytes(int B, int I, int N, int k, int O);
 size_t dl_dwn_bwd_workspace_bytes(int B, int I, int N, int k, int O);
+/* 1 where the layer's backward reads x although it is given `saved` and its workspace, 0 where x may be null. */
+int dl_dwn_bwd_reads_x(int N, int k, int O);
 int dl_dwn_layer_fwd(const float *x, const int32_t *idx32, const float *luts, float *y,
                      void *saved, void *ws, size_t ws_bytes,
                      int B, int I, int N, int k, int O, void *stream);
@@ -115,8 +117,9 @@ int dl_dwn_layer_fwd_static(const float *x, const int32_t *idx32, const float *l
  *   gluts[n,d,e] = sum_b [addr(b,n) = e] gy[b,n,d]
  * gx may be null (input does not need a gradient); gx and gluts are overwritten.
  * k <= DL_MAX_FAST_K: x is not read and may be null.  k = 7, 8: with `saved` as the forward wrote it (every forward given a
- * `saved` does) and dl_dwn_bwd_workspace_bytes of workspace the same kernels run and x is not read; without either, and for
- * k > 8, x is read and `saved` is not.  Then the workspace is optional (ws may be null): with it, |beta| <= 1/2 and
+ * `saved` does) and dl_dwn_bwd_workspace_bytes of workspace the same kernels run and x is not read; without either, for
+ * k > 8, and for layers of 2^23 nodes or of 2 GiB of tables and more (dl_dwn_bwd_reads_x), x is read and `saved` is not.
+ * Then the workspace is optional (ws may be null): with it, |beta| <= 1/2 and
  * k <= 12 the input gradient is taken from tables smoothed once per call (two loads per row and connection); without, from
  * the 2^k-term sum of the formula per row and connection.  The table gradient of that path is summed with atomics. */
 int dl_dwn_layer_bwd(const float *x, const void *saved, const int32_t *idx32,

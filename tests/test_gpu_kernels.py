@@ -421,6 +421,27 @@ def test_dwn_forward_keeps_addresses_instead_of_x(k, stable):
     assert torch.isfinite(leaf.grad).all() and leaf.grad.abs().max() > 0
 
 
+def test_dwn_layer_of_more_nodes_than_the_lane_kernels_number():
+    """2^23 nodes: the general kernels, whose backward reads x.  Sums of 2048 fp32 terms of either sign."""
+    ops = _ops()
+    B, I, N = 2, 4096, 1 << 23
+    g = torch.Generator("cuda").manual_seed(8)
+    idx = torch.randint(0, I, (N, 1), device="cuda", generator=g, dtype=torch.int32)
+    x = torch.rand(B, I, device="cuda", generator=g).requires_grad_()
+    luts = (torch.rand(N, 1, 2, device="cuda", generator=g) * 2 - 1).requires_grad_()
+    gy = torch.randn(B, N, device="cuda", generator=g)
+    y = ops.DWNLayerFunction.apply(x, luts, ops.MappingPlan(idx, I), 0.3, 0.25)
+    y.backward(gy)
+    col = idx[:, 0].long()
+    addr = (x.detach()[:, col] >= 0.5).long()
+    table = luts.detach()[:, 0]
+    assert torch.equal(y, torch.gather(table.expand(B, N, 2), 2, addr[..., None])[..., 0])
+    assert torch.equal(luts.grad[:, 0], sum(torch.nn.functional.one_hot(addr[b], 2) * gy[b][:, None] for b in range(B)))
+    terms = 0.3 * gy.double() * (table[:, 1] - table[:, 0]).double()
+    want, size = (torch.zeros(B, I, dtype=torch.float64, device="cuda").index_add_(1, col, t) for t in (terms, terms.abs()))
+    assert float(((x.grad.double() - want).abs() / size).max()) <= 64 * 2.0 ** -24
+
+
 def test_dwn_no_input_grad_and_unused_inputs():
     ops = _ops()
     B, I, N, k, O = 40, 50, 3, 2, 1  # 44 of the 50 inputs feed no node: their gradient must be 0

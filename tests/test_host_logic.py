@@ -35,6 +35,16 @@ def test_library_exports_every_declared_symbol():
     assert nat.lib().dl_dwn_fwd_workspace_bytes(4096, 16384, 8192, 6, 1) == 64 * 16384 * 8
 
 
+@pytest.mark.parametrize("k", [1, 6, 7, 8, 9, 12])
+def test_dwn_backward_reads_x_where_nothing_was_kept(k):
+    """The forward keeps every node's addresses, or a token allocation and then the backward has to have x."""
+    from difflut_amd import _native as nat
+
+    for N, O in ((1, 1), (5000, 2), ((1 << 23) - 1, 1), (1 << 23, 1), ((1 << 29 - k) - 1, 1), (1 << 29 - k, 1), (1 << 27 - k, 4)):
+        kept = nat.lib().dl_dwn_saved_bytes(1024, 64, N, k, O) == N * 1024
+        assert nat.lib().dl_dwn_bwd_reads_x(N, k, O) == (0 if kept else 1), (N, O)
+
+
 @pytest.mark.parametrize("missing", ["LIB_PATH", "HOST_PATH"])
 def test_not_built_without_either_library(monkeypatch, tmp_path, missing):
     """Layers and nodes offer their kernels by is_built(): a tree with one library of two does not have them."""
