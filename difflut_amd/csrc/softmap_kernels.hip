@@ -30,6 +30,9 @@
 //   have a few values below 2^-27 of those (one in a few million of N(0, 1)): the pack pass leaves up to SM_TINY_MOST of them
 //   out and softmap_plain adds their terms; where there are more, the product takes the planes, gx with E's made from its pairs
 //   (SoftmapArgs::tiny).
+// Error against float64 (2-norm) of m / gx / gW, 512 x 3136 x 48000, W of N(0, 1.5), tau 1: 1.1e-7 / 1.7e-7 / 4.3e-7 with pairs,
+// 5.3e-7 / 3.2e-7 / 11.8e-7 with planes, whose operands are exact but whose sums have twice as many additions and no groups of
+// stages (below); short sums: SM_PAIR_CHUNK.
 //
 // Layout.  An MFMA lane wants 8 consecutive reduction steps of one row: a "unit" of 16 bytes.  Every operand is stored
 // as [reduction / 8][rows] units, rows padded to whole tiles with zeros, by the pass that has it in registers anyway
@@ -1135,9 +1138,16 @@ static void softmap_chunks(int stages, long long tiles, long long blocks, int *c
     *chunks = dl_ceil_div(stages, *chunk);
 }
 // Pairs cost a pass over x and one over gm and ten launches of about 5 us a step, six of which end at once.  Measured, forward +
-// backward, planes against pairs: 512 x 512 x 24000 (6.3e9) 332 -> 322 us, 64 x 3136 x 30000 (6.0e9) 716 -> 594, 300 x 1500 x 20000
+// backward, planes against pairs: 512 x 512 x 24000 (6.3e9) 332 -> 322 us (planes all the same, see below), 64 x 3136 x 30000 (6.0e9) 716 -> 594, 300 x 1500 x 20000
 // (9.0e9) 578 -> 468, 512 x 3136 x 48000 2659 -> 2562 where E spans too much; below, planes.
 #define SM_PAIR_WORK 6e9
+// gx in chunks of the reduction shorter than this many stages takes the planes, and with it the whole call, which has one form of
+// E: a pair's 23 bits are seen there, where longer sums round more than that.  Error of gx against float64 (2-norm, units of 1e-7),
+// planes / pairs, by the planes' stages per chunk, W of N(0, 1.5), gm of N(0, 1): 24 (512 x 512 x 24000) 1.28 / 1.42, 25 (512 x 3136 x 4000)
+// 1.23 / 1.38, 32 1.29 / 1.36, 36 1.38 / 1.41, 39 1.37 / 1.35, 41 1.41 / 1.39, 47 1.49 / 1.40, 57 1.57 / 1.41, 104 2.03 / 1.50, 300
+// (512 x 3136 x 48000) 3.18 / 1.73; the same with W of N(0, 0.1) and with gm a product of two N(0, 1).  m and gW are closer with pairs at
+// all of these, by 0.2 to 0.7.
+#define SM_PAIR_CHUNK 40
 static SoftmapShape softmap_shape(int B, int I, int M, int precision) {
     SoftmapShape h;
     h.B = B; h.I = I; h.M = M;
@@ -1155,6 +1165,7 @@ static SoftmapShape softmap_shape(int B, int I, int M, int precision) {
     h.gx_stages = dl_ceil_div(M, h.depth);
     softmap_chunks(h.fwd_stages, (long long)h.row_tiles * h.fwd_col_tiles, 512, &h.fwd_chunk, &h.fwd_chunks);
     softmap_chunks(h.gx_stages, (long long)h.row_tiles * h.gx_col_tiles, 512, &h.gx_chunk, &h.gx_chunks);
+    h.pairs = h.pairs && h.gx_chunk >= SM_PAIR_CHUNK;
     h.pair_row_tiles = h.Bp / 128;
     softmap_chunks(h.fwd_stages, (long long)h.pair_row_tiles * h.fwd_col_tiles, 512, &h.pair_fwd_chunk, &h.pair_fwd_chunks);
     softmap_chunks(h.gx_stages, (long long)h.pair_row_tiles * h.gx_col_tiles, 1024, &h.pair_gx_chunk, &h.pair_gx_chunks);
