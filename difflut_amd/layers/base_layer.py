@@ -21,6 +21,7 @@ The per-node scalar buffers the fused kernels need (`alpha`, `beta`, `temperatur
 gives nodes different values lands in the array the kernels are handed on every call: every fused path (single
 layers, chained stacks, convolutional levels) uses each node's own values, as the reference's node loop does.
 """
+import functools
 import warnings
 from abc import ABC, abstractmethod
 
@@ -71,13 +72,20 @@ class BankedParameter(nn.Parameter):
         return (nn.Parameter, (self.data.clone(), self.requires_grad))
 
 
+@functools.lru_cache(maxsize=16)
+def _node_names(count):
+    """The names of `count` modules in a ModuleList, one tuple for the banks of a layer.  Making it takes 0.6 ms for 8192 nodes, so
+    banks ask for it when they are tied and not on a layer's first call."""
+    return tuple(map(str, range(count)))
+
+
 def _node_getter(nodes):
     """row -> node without ModuleList.__getitem__, whose index arithmetic costs more than the checks below (they run on
     every call of a layer).  Looks the node up anew each time, in the list's present dict (deleting an entry gives it a
     new one), so a replaced node is seen."""
     if not isinstance(nodes, nn.ModuleList):
         return nodes.__getitem__
-    keys = [str(row) for row in range(len(nodes))]
+    keys = _node_names(len(nodes))
     return lambda row: nodes._modules[keys[row]]
 
 
@@ -161,6 +169,7 @@ class ScalarBank:
             view._scalar_bank = self
             node._buffers[self.name] = view
             self._views.append(view)
+        self._keys = _node_names(len(self._views))
         self._stale, self._key = False, None
 
     def tied(self):
@@ -179,8 +188,8 @@ class ScalarBank:
             self._probe = (self._probe + self._PROBES) % n
         name, views, nodes = self.name, self._views, self.nodes
         if isinstance(nodes, nn.ModuleList):  # as _node_getter does, without a call per node
-            if len(self._keys) != n:
-                self._keys = [str(row) for row in range(n)]
+            if len(self._keys) != n:  # of a bank that was saved without them
+                self._keys = _node_names(n)
             nodes, keys = nodes._modules, self._keys
             for row in rows:
                 if nodes[keys[row]]._buffers[name] is not views[row]:

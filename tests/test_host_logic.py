@@ -63,6 +63,29 @@ def test_not_built_without_either_library(monkeypatch, tmp_path, missing):
         nat.host()
 
 
+@pytest.mark.parametrize("origin", ["built", "copied", "pickled", "converted"])
+def test_first_call_does_not_name_the_nodes(origin):
+    """What the per-call checks look nodes up by is there before the first call, which would else make it for every node
+    (8192 nodes: a first training pass of 1.9 ms instead of 1.2)."""
+    import copy
+    import pickle
+
+    from difflut_amd.layers import RandomLayer
+    from difflut_amd.nodes import DWNNode, NodeConfig
+
+    layer = RandomLayer(40, 130, DWNNode, NodeConfig(input_dim=3, output_dim=1), seed=1)
+    if origin == "copied":
+        layer = copy.deepcopy(layer)
+    elif origin == "pickled":
+        layer = pickle.loads(pickle.dumps(layer))
+    elif origin == "converted":
+        layer = layer.double().float()
+    for bank in layer._scalars.values():
+        keys = bank._keys
+        assert list(keys) == list(layer.nodes._modules)
+        assert bank.tied() and bank._keys is keys
+
+
 def test_registry_names_and_errors():
     from difflut_amd import REGISTRY
     from difflut_amd.layers import LearnableLayer, RandomLayer
