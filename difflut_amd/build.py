@@ -32,9 +32,11 @@ def host_command():
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
     torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
     includes = cpp_extension.include_paths() + [sysconfig.get_paths()["include"], os.path.join(rocm, "include")]
-    return (["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-w", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+    return (["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-Wextra",
+             "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
              "-D_GLIBCXX_USE_CXX11_ABI=" + str(int(torch._C._GLIBCXX_USE_CXX11_ABI)), "-DTORCH_API_INCLUDE_EXTENSION_H"]
-            + ["-I" + d for d in includes] + [os.path.join(CSRC, "host_ops.cpp"), "-o", HOST_PATH, "-L" + torch_lib]
+            + [flag for d in includes for flag in ("-isystem", d)]  # (warnings of this source only, not of the headers)
+            + [os.path.join(CSRC, "host_ops.cpp"), "-o", HOST_PATH, "-L" + torch_lib]
             + ["-l" + lib for lib in ("c10", "c10_hip", "torch_cpu", "torch_hip", "torch", "torch_python", "dl")]
             + ["-Wl,-rpath," + torch_lib])
 
@@ -64,6 +66,8 @@ def build(verbose=False, jobs=None):
         res = subprocess.run(cmd, capture_output=True, text=True)
         if res.returncode != 0:
             raise RuntimeError("g++ failed on host_ops.cpp:\n" + res.stdout + res.stderr)
+        if res.stderr:
+            print(res.stderr)
         if verbose:
             print(" ".join(cmd))
 
