@@ -63,7 +63,11 @@ class MappingPlan:
         self.device = idx.device
         self.source_ptr = idx.data_ptr()
         self.source_version = idx._version
-        self.host = (self.idx32, self.inv_ptr, self.inv_pos, self.I)  # as the native operators take it
+
+    @property
+    def host(self):
+        """As the native operators take it."""
+        return self.idx32, self.inv_ptr, self.inv_pos, self.I
 
     def matches(self, idx):
         return (idx.device == self.device and idx.data_ptr() == self.source_ptr

@@ -63,6 +63,20 @@ def test_not_built_without_either_library(monkeypatch, tmp_path, missing):
         nat.host()
 
 
+def test_plan_saved_before_the_native_operators():
+    """A layer saved whole takes its mapping plan along; plans of earlier files hold the four tables' attributes only."""
+    import pickle
+
+    from difflut_amd import ops
+
+    plan = ops.MappingPlan(torch.randint(0, 9, (5, 3)), 9)
+    for name in set(vars(plan)) - {"N", "k", "I", "idx32", "inv_ptr", "inv_pos", "device", "source_ptr", "source_version"}:
+        delattr(plan, name)
+    plan = pickle.loads(pickle.dumps(plan))
+    idx, inv_ptr, inv_pos, width = plan.host
+    assert idx is plan.idx32 and inv_ptr is plan.inv_ptr and inv_pos is plan.inv_pos and width == 9
+
+
 @pytest.mark.parametrize("origin", ["built", "copied", "pickled", "converted"])
 def test_first_call_does_not_name_the_nodes(origin):
     """What the per-call checks look nodes up by is there before the first call, which would else make it for every node
