@@ -204,6 +204,7 @@ static void dwn_pair_launch_k(const float *gy1, const uint8_t *addr1, const floa
 #define DWN_PAIR(WI_)                                                                                                  \
     DL_TIMED("dwn_bwd_pair_gx", s, (dwn_bwd_pair_gx<K, WI_><<<blocks, 512, 0, s>>>(gy1, addr1, D1, inv_ptr1, inv_pos1, N1, addr0, \
                                                                                     D0, lists, gx, I, N0, BT, per)))
+    // registers for the sums of a wavefront's inputs: up to 40 inputs, up to 104 (5 x 5 patches of four channels), 128
     if (per <= 5) DWN_PAIR(5);
     else if (per <= 13) DWN_PAIR(13);
     else DWN_PAIR(16);
@@ -214,6 +215,11 @@ static void dwn_pair_launch_k(const float *gy1, const uint8_t *addr1, const floa
 // at once and take 249 us together, 199 where there are only half as many of them, so a last round that is too empty is left
 // to the gather from a stored output gradient, which goes by the tile.  Kernels of this path with setup against that one's,
 // us, 100 columns, 1152 nodes: 769 tiles 280 / 269, 1026 344 / 350, 1530 387 / 501, 2052 (of which 4 in a second round) 445 / 654.
+// The whole training step with this path and without, us, by inputs x nodes of the first level (k = 6; 512: k = 4), at about
+// 1110, 1300, 2040 and 2300 tiles: 16 x 576 322 / 334, 326 / 368, 389 / 494, 479 / 534; 16 x 512 289 / 291, 298 / 318, 357 / 435,
+// 421 / 461; 36 x 576 326 / 320, 335 / 353, 430 / 497, 458 / 538; 75 x 576 347 / 340, 354 / 371, 435 / 534, 487 / 572; 100 x 1152
+// 535 / 544, 557 / 602, 675 / 849, 780 / 946; 128 x 1152 561 / 567, 588 / 625, 696 / 871, 799 / 964: at the least it loses 2 % at
+// worst, from 1300 on it wins everywhere.
 // Fewer than 16 inputs leave wavefronts without one; lists shorter than 32 take the gather that fills the table gradient in
 // front, which reads a node's rows seldom enough.
 int dwn_pair_tiles(int BT, int I, int N0, int k, int N1) {

@@ -27,7 +27,7 @@
 //   2^-27 of that, decided on the device, the products it is in take the planes (launches of either kind that are not to run
 //   end at once): with W of N(0, 6) at tau 1, where E spans more, the forward and gx.
 //   gs is scaled row by row and gm column by column, so that no output row answers for another's magnitude.  Ordinary gradients
-//   have a few values below 2^-27 of those (one in a few million of N(0, 1)): the pack pass leaves up to SM_TINY_MOST of them
+//   have a few values below 2^-27 of those (58 of the 24.6 million of a learnable layer's step): the pack pass leaves up to SM_TINY_MOST of them
 //   out and softmap_plain adds their terms; where there are more, the product takes the planes, gx with E's made from its pairs
 //   (SoftmapArgs::tiny).
 // Error against float64 (2-norm) of m / gx / gW, 512 x 3136 x 48000, W of N(0, 1.5), tau 1: 1.1e-7 / 1.7e-7 / 4.3e-7 with pairs,
@@ -575,7 +575,8 @@ __device__ __forceinline__ void softmap_stage_barrier() {
 // rest's sum scaled and added by every stage: 514 / 560 / 668.  gx in
 // 5, 10 or 15 chunks of the reduction: 445, 486 and 497 with their sum; 10 for the shorter running sums.
 // NPB = 2 with NP = 3 (gx): gs in planes, E in pairs, whose planes - times 2^10, which makes their scale the planes' - are made on
-// the way out of the LDS; for gradients that span too much where E does not.
+// the way out of the LDS; for gradients that span too much where E does not.  The backward at 512 x 3136 x 48000 with such
+// gradients 1651 us, 1782 with E in planes throughout.
 template <int MODE, int NP, int FA, int NPB>
 __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
     extern __shared__ __align__(16) char lds[];

@@ -4,7 +4,7 @@ Training: every node input is a softmax-weighted mix of all layer inputs,
 m = x @ softmax(W / tau, -1).T; evaluation: the argmax input is selected.  Constructor,
 `mapping.W` [output_size*n, input_size] (xavier-uniform), tau schedule and
 `get_mapping_matrix` follow difflut/layers/learnable_layer.py:173-486.  The contraction, its
-backward (the softmax numerators kept as bf16 planes) and the hard selection run in libdifflut_hip.so.
+backward (the softmax numerators kept as 16-bit planes) and the hard selection run in libdifflut_hip.so.
 """
 import warnings
 

@@ -304,8 +304,8 @@ def prob_layer_eval(x, raw, plan, temperature):
 
 # ----------------------------------------------------------------------------- Learnable mapping
 class SoftMapFunction:
-    """m = x @ softmax(W / tau, dim=-1).T.  The softmax numerators are kept as bf16 planes from forward to backward: 6 bytes per
-    entry of W with fp32 operands (precision 0), 2 with bf16."""
+    """m = x @ softmax(W / tau, dim=-1).T.  The softmax numerators are kept as 16-bit planes from forward to backward: 6 bytes per
+    entry of W with fp32 operands (precision 0: three bf16 planes, or two fp16 halves in the same room), 2 with bf16."""
 
     @staticmethod
     def apply(x, W, tau, precision):

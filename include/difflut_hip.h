@@ -350,19 +350,21 @@ int dl_prob_layer_eval_ws_nodes(const float *x, const int32_t *idx32, const floa
  * learnable_mapping_cuda.soft_forward (learnable_mapping_cuda_kernel.cu:99-223),
  * and learnable_mapping_cuda.forward/.backward for argmax selection
  * (learnable_mapping_cuda_kernel.cu:22-81,236-257; learnable_layer.py:216-236).
- *   x [B,I], W [M,I], m [B,M];   S = softmax(W / tau) along I, kept as its numerators' bf16 planes in `stats`.
- * precision: 0 = fp32 operands (reference numerics; each the exact sum of three bf16 planes on the matrix cores, fp32
- *                matrix instructions where a value is too large or not finite),
+ *   x [B,I], W [M,I], m [B,M];   S = softmax(W / tau) along I, kept as its numerators' 16-bit planes in `stats`.
+ * precision: 0 = fp32 operands (reference numerics; on the matrix cores each the exact sum of three bf16 planes, or, in
+ *                products of B*I*M >= 6e9 with a long reduction, two fp16 halves that hold 23 of its 24 bits, where their sums
+ *                round more than that and the values' range allows it; fp32 matrix instructions where a value is too large
+ *                or not finite),
  *            1 = bf16 operands, fp32 accumulation (tolerance documented with the tests).
  * stats (dl_soft_map_saved_bytes bytes) is written by the forward and read by the backward.
  *   gx = gm * S,   gW = S * (G - r) / tau with G = gm^T x and r[o] = sum_b gm[b,o] m[b,o].
  * ------------------------------------------------------------------------ */
 /* size of `stats`: what the forward keeps for the backward (row maximum, 1/sum, the packed x and the softmax
- * numerators as bf16 planes: M*I*2 bytes with precision 1, M*I*6 with precision 0 (903 MB at 48000 x 3136), rounded up
- * to whole tiles) */
+ * numerators as 16-bit planes: M*I*2 bytes with precision 1, M*I*6 with precision 0 (903 MB at 48000 x 3136; a third of it
+ * stays unused where the device takes the two halves), rounded up to whole tiles) */
 size_t dl_soft_map_saved_bytes(int B, int I, int M, int precision);
 /* scratch of either direction (one size for both): partial products of small shapes, the backward's partial r and
- * packed x and gm.  With precision 0 the forward runs without it (ws = NULL), then without splitting the reduction. */
+ * packed x and gm, where gradients that the two halves leave out lie.  With precision 0 the forward runs without it (ws = NULL), then without splitting the reduction. */
 size_t dl_soft_map_workspace_bytes(int B, int I, int M, int precision);
 int dl_soft_map_fwd(const float *x, const float *W, float tau, float *m, float *stats,
                     void *ws, size_t ws_bytes, int B, int I, int M, int precision, void *stream);
