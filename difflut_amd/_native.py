@@ -72,6 +72,10 @@ SIGNATURES = {
     "dl_prob_layer_bwd": (_I, [_P, _P, _P, _P, _P, _P, _F, _P, _P, _P, _P, _Z, _I, _I, _I, _I, _I, _P]),
     "dl_prob_layer_fwd_nodes": (_I, [_P, _P, _P, _P, _P, _P, _Z, _I, _I, _I, _I, _I, _P]),
     "dl_prob_layer_bwd_nodes": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _Z, _I, _I, _I, _I, _I, _P]),
+    "dl_prob_ordered_saved_bytes": (_Z, [_I] * 2),
+    "dl_prob_ordered_bwd_workspace_bytes": (_Z, [_I] * 3),
+    "dl_prob_ordered_fwd": (_I, [_P, _P, _F, _P, _P, _P, _Z, _I, _I, _I, _P]),
+    "dl_prob_ordered_bwd": (_I, [_P, _P, _F, _P, _P, _P, _P, _P, _Z, _I, _I, _I, _P]),
     "dl_prob_layer_eval_ws_nodes": (_I, [_P, _P, _P, _P, _P, _P, _Z, _I, _I, _I, _I, _I, _P]),
     "dl_prob_eval_workspace_bytes": (_Z, [_I] * 5),
     "dl_prob_layer_eval_ws": (_I, [_P, _P, _P, _F, _P, _P, _Z, _I, _I, _I, _I, _I, _P]),

@@ -284,6 +284,36 @@ __device__ __forceinline__ void prob_fold_gradient(const float (&v0)[1 << KH], c
     }
 }
 
+// Sum the 64 per-row partials of every table entry with L - 1 + (6 - K) exchanges instead of 6 L:
+// round r pairs the entries (2i, 2i+1); the half of the wavefront with lane bit (5 - r) set keeps
+// the odd one and hands over the even one, so after K rounds a lane holds one entry,
+// a = sum_r ((lane >> (5 - r)) & 1) << r, summed over the lanes that differ in the top K bits.
+template <int K>
+__device__ __forceinline__ float prob_sum_lanes(float (&acc)[1 << K], int lane) {
+#pragma unroll
+    for (int r = 0; r < K; ++r) {
+        const int width = 32 >> r;
+        const bool upper = (lane & width) != 0;
+#pragma unroll
+        for (int i = 0; i < ((1 << K) >> (r + 1)); ++i) {
+            const float keep = upper ? acc[2 * i + 1] : acc[2 * i];
+            const float send = upper ? acc[2 * i] : acc[2 * i + 1];
+            acc[i] = keep + __shfl_xor(send, width);
+        }
+    }
+    float mine = acc[0];
+#pragma unroll
+    for (int width = 32 >> K; width > 0; width >>= 1) mine += __shfl_xor(mine, width);
+    return mine;
+}
+template <int K>
+__device__ __forceinline__ int prob_sum_entry(int lane) {
+    int a = 0;
+#pragma unroll
+    for (int r = 0; r < K; ++r) a |= ((lane >> (5 - r)) & 1) << r;
+    return a;
+}
+
 // The gradient of the mapped inputs is written once and read once.  Where it is too large for the 256 MB behind the L2s to hold it
 // beside x and gx, it is written and read, and gx written, past that cache's keeping (STREAM), which leaves it to what is read
 // again.  Forward and backward, us, as ordinary accesses / so: hybrid 1024 x 8192 -> 6000 (147 MB) 136 / 133, 2048 x 8192 -> 4096 (201 MB)
@@ -398,28 +428,245 @@ __global__ __launch_bounds__(64 * W) void prob_bwd_t(const float *__restrict__ x
             for (int hi = 0; hi < LU; ++hi) acc[lo | (hi << KL)] = fmaf(gu, w[hi], acc[lo | (hi << KL)]);
         }
     }
-    // Sum the 64 per-row partials of every table entry with L - 1 + (6 - K) exchanges instead of 6 L:
-    // round r pairs the entries (2i, 2i+1); the half of the wavefront with lane bit (5 - r) set keeps
-    // the odd one and hands over the even one, so after K rounds a lane holds one entry,
-    // a = sum_r ((lane >> (5 - r)) & 1) << r, summed over the lanes that differ in the top K bits.
+    const float mine = prob_sum_lanes<K>(acc, lane);
+    if (live && (lane & ((64 >> K) - 1)) == 0) gpart[((size_t)chunk * NO + c) * L + prob_sum_entry<K>(lane)] = mine;
+}
+
+// ---------------------------------------------------------------------------------
+// Nodes that read their inputs in order: node n has columns n K .. n K + K - 1 of x [B][N K], one output (what a learned mapping
+// hands its nodes).  Sixteen nodes are then 16 K consecutive values of a row, so x and the gradient of x are read and written
+// as they lie: no re-tiling of x, no tiled gradient, no gather.  A block is sixteen wavefronts, one per node, and walks the
+// batch tiles of a chunk: the 64 x 16 K piece of a tile comes a tile ahead through registers into the LDS (odd stride: a lane's row
+// lies on a bank of its own), a wavefront has its K columns and its table in registers, results leave through the LDS, one barrier
+// per tile.  The backward writes the gradient over the inputs that it has read, so three pieces take turns: one being
+// filled, one in use, one being stored.  Arithmetic and its order are those of prob_fwd_t and prob_bwd_t.
+// Bound by HBM forward (x and y once), by vector arithmetic backward.
+// 512 x 48000 -> 8000 nodes of six inputs: forward 30 us, backward 62, 3.8 and 3.4 TB/s; re-tiled, two and two launches, 63 and 93.
+// The learnable layer's step 1022 -> 951 us with bf16 operands, 2027 -> 1957 with fp32.
+#define PROB_ON 16  // nodes per block
+// W: values per access, as many as the width of x and the alignment allow.  Accesses go through a buffer descriptor of the
+// tile's rows that the batch has (rows past it lie past its end: zeros, nothing stored), with one byte offset per access for all
+// tiles, of x and of its gradient.
+template <int W>
+struct ProbWide;
+template <>
+struct ProbWide<4> { typedef unsigned type __attribute__((ext_vector_type(4))); };
+template <>
+struct ProbWide<2> { typedef unsigned type __attribute__((ext_vector_type(2))); };
+template <int K, int W>
+struct ProbPiece {  // my share of the 64 x 16 K piece of a batch tile
+    static constexpr int S = PROB_ON * K + 1, PER_ROW = PROB_ON * K / W, COUNT = 64 * PER_ROW;
+    static constexpr int PASSES = (COUNT + 64 * PROB_ON - 1) / (64 * PROB_ON);
+    static constexpr unsigned NOWHERE = 0x80000000u;  // past the end of every descriptor: 64 rows of less than 2^23 values
+    unsigned off[PASSES];
+    float v[PASSES][W];
+    static __device__ __forceinline__ int element(int p) { return p * 64 * PROB_ON + (int)threadIdx.x; }
+    __device__ __forceinline__ void place(int M, int cols) {
 #pragma unroll
-    for (int r = 0; r < K; ++r) {
-        const int width = 32 >> r;
-        const bool upper = (lane & width) != 0;
-#pragma unroll
-        for (int i = 0; i < (L >> (r + 1)); ++i) {
-            const float keep = upper ? acc[2 * i + 1] : acc[2 * i];
-            const float send = upper ? acc[2 * i] : acc[2 * i + 1];
-            acc[i] = keep + __shfl_xor(send, width);
+        for (int p = 0; p < PASSES; ++p) {
+            const int row = element(p) / PER_ROW, col = element(p) % PER_ROW * W;
+            off[p] = element(p) < COUNT && col < cols ? (unsigned)(row * M + col) * 4u : NOWHERE;
         }
     }
-    float mine = acc[0];
+    // at: column c0 of the tile's first row
+    static __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile(const float *at, int M, int c0, int rows) {
+        return __builtin_amdgcn_make_buffer_rsrc((void *)at, 0, (unsigned)(min(rows, 64) * M - c0) * 4u, PROB_RSRC);
+    }
+    __device__ __forceinline__ void request(__amdgpu_buffer_rsrc_t r) {
 #pragma unroll
-    for (int width = 32 >> K; width > 0; width >>= 1) mine += __shfl_xor(mine, width);
-    int a = 0;
+        for (int p = 0; p < PASSES; ++p) {
+            if constexpr (W == 4) {
+                const typename ProbWide<4>::type q = __builtin_amdgcn_raw_buffer_load_b128(r, off[p], 0, 0);
 #pragma unroll
-    for (int r = 0; r < K; ++r) a |= ((lane >> (5 - r)) & 1) << r;
-    if (live && (lane & ((64 >> K) - 1)) == 0) gpart[((size_t)chunk * NO + c) * L + a] = mine;
+                for (int w = 0; w < 4; ++w) v[p][w] = __uint_as_float(q[w]);
+            } else if constexpr (W == 2) {
+                const typename ProbWide<2>::type q = __builtin_amdgcn_raw_buffer_load_b64(r, off[p], 0, 0);
+                v[p][0] = __uint_as_float(q[0]); v[p][1] = __uint_as_float(q[1]);
+            } else {
+                v[p][0] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off[p], 0, 0));
+            }
+        }
+    }
+    __device__ __forceinline__ void put(float (*piece)[S]) const {
+#pragma unroll
+        for (int p = 0; p < PASSES; ++p)
+            if (COUNT % (64 * PROB_ON) == 0 || element(p) < COUNT) {
+#pragma unroll
+                for (int w = 0; w < W; ++w) piece[element(p) / PER_ROW][element(p) % PER_ROW * W + w] = v[p][w];
+            }
+    }
+    __device__ __forceinline__ void store(float (*piece)[S], __amdgpu_buffer_rsrc_t r) const {
+#pragma unroll
+        for (int p = 0; p < PASSES; ++p) {
+            if (COUNT % (64 * PROB_ON) != 0 && element(p) >= COUNT) continue;
+            const float *from = &piece[element(p) / PER_ROW][element(p) % PER_ROW * W];
+            if constexpr (W == 4) {
+                const typename ProbWide<4>::type q = {__float_as_uint(from[0]), __float_as_uint(from[1]), __float_as_uint(from[2]), __float_as_uint(from[3])};
+                __builtin_amdgcn_raw_buffer_store_b128(q, r, off[p], 0, 0);
+            } else if constexpr (W == 2) {
+                const typename ProbWide<2>::type q = {__float_as_uint(from[0]), __float_as_uint(from[1])};
+                __builtin_amdgcn_raw_buffer_store_b64(q, r, off[p], 0, 0);
+            } else {
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(*from), r, off[p], 0, 0);
+            }
+        }
+    }
+};
+// a value of every lane below L as wave-uniform ones
+template <int L>
+__device__ __forceinline__ void prob_spread(float mine, float (&all)[L]) {
+#pragma unroll
+    for (int a = 0; a < L; ++a) all[a] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mine), a));
+}
+
+template <int K, int W>
+__global__ __launch_bounds__(64 * PROB_ON, 8) void prob_ordered_fwd(const float *__restrict__ x, const float *__restrict__ raw,
+                                                                  ProbTemp T, float *__restrict__ sig, float *__restrict__ y, int B,
+                                                                  int N, int BT, int tiles_per_chunk) {
+    constexpr int L = 1 << K;
+    typedef ProbPiece<K, W> Piece;
+    __shared__ float xt[2][64][Piece::S], yt[2][64][PROB_ON + 1];
+    const int lane = threadIdx.x & 63, wave = dl_uniform(threadIdx.x >> 6);
+    const int n0 = blockIdx.x * PROB_ON, n = n0 + wave, M = N * K, cols = min(PROB_ON * K, M - n0 * K);
+    const bool live = n < N;
+    float tab[L];
+    {
+        float s = 0.0f;
+        if (live && lane < L) {
+            s = dl_sigmoid(raw[(size_t)n * L + lane] * prob_inv_t_of(T, n));
+            if (blockIdx.y == 0) sig[(size_t)n * L + lane] = s;
+        }
+        prob_spread<L>(s, tab);
+    }
+    const int t0 = blockIdx.y * tiles_per_chunk, t1 = min(BT, t0 + tiles_per_chunk);
+    Piece next;
+    next.place(M, cols);
+    auto request = [&](int t) { next.request(Piece::tile(x + (size_t)t * 64 * M + n0 * K, M, n0 * K, B - t * 64)); };
+    const int yr = threadIdx.x / PROB_ON, yc = threadIdx.x % PROB_ON;
+    auto store = [&](int t, int buf) {
+        if (t * 64 + yr < B && n0 + yc < N) y[(size_t)(t * 64 + yr) * N + n0 + yc] = yt[buf][yr][yc];
+    };
+    request(t0);
+    int buf = 0;
+    for (int t = t0; t < t1; ++t, buf ^= 1) {
+        next.put(xt[buf]);
+        __syncthreads();  // (the other piece and the other yt are written again only after the next one)
+        if (t + 1 < t1) request(t + 1);
+        if (t > t0) store(t - 1, buf ^ 1);
+        float xs[K];
+#pragma unroll
+        for (int j = 0; j < K; ++j) xs[j] = xt[buf][lane][wave * K + j];
+        float v[L / 2 > 0 ? L / 2 : 1];
+        {
+            const float om = 1.0f - xs[0];
+#pragma unroll
+            for (int a = 0; a < L / 2; ++a) v[a] = fmaf(tab[2 * a + 1], xs[0], tab[2 * a] * om);
+        }
+#pragma unroll
+        for (int j = 1; j < K; ++j) {
+#pragma unroll
+            for (int a = 0; a < (L >> (j + 1)); ++a) v[a] = v[2 * a] + xs[j] * (v[2 * a + 1] - v[2 * a]);
+        }
+        yt[buf][lane][wave] = v[0];
+    }
+    __syncthreads();
+    store(t1 - 1, buf ^ 1);
+}
+
+// gpart: as prob_bwd_t leaves it, or null where the block has the whole batch: it then writes graw itself
+template <int K, int W>
+__global__ __launch_bounds__(64 * PROB_ON) void prob_ordered_bwd(const float *__restrict__ x, const float *__restrict__ gy,
+                                                                  const float *__restrict__ sig, ProbTemp T, float *__restrict__ gx,
+                                                                  float *__restrict__ gpart, float *__restrict__ graw, int B, int N,
+                                                                  int BT, int tiles_per_chunk) {
+    constexpr int L = 1 << K;
+    constexpr int KL = K / 2, KU = K - KL, LL = 1 << KL, LU = 1 << KU;
+    typedef ProbPiece<K, W> Piece;
+    __shared__ float xt[3][64][Piece::S], gturn[2][PROB_ON][65];
+    const int lane = threadIdx.x & 63, wave = dl_uniform(threadIdx.x >> 6);
+    const int n0 = blockIdx.x * PROB_ON, n = n0 + wave, M = N * K, cols = min(PROB_ON * K, M - n0 * K);
+    const bool live = n < N;
+    float tab[L];  // the table less a value of its own (prob_table_element)
+    {
+        const float s = live && lane < L ? sig[(size_t)n * L + lane] : 0.0f;
+        const float first = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s), 0)),
+                    last = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s), L - 1));
+        prob_spread<L>(s - (L > 2 ? 0.5f * first + 0.5f * last : first), tab);
+    }
+    float acc[L];
+#pragma unroll
+    for (int a = 0; a < L; ++a) acc[a] = 0.0f;
+    const int t0 = blockIdx.y * tiles_per_chunk, t1 = min(BT, t0 + tiles_per_chunk);
+    Piece next;
+    next.place(M, cols);
+    float ng = 0.0f;
+    const int trow = threadIdx.x / PROB_ON, tcol = threadIdx.x % PROB_ON;
+    auto request = [&](int t) {
+        next.request(Piece::tile(x + (size_t)t * 64 * M + n0 * K, M, n0 * K, B - t * 64));
+        const int b = t * 64 + trow;
+        ng = (b < B && n0 + tcol < N) ? gy[(size_t)b * N + n0 + tcol] : 0.0f;
+    };
+    auto store = [&](int t, int piece) { next.store(xt[piece], Piece::tile(gx + (size_t)t * 64 * M + n0 * K, M, n0 * K, B - t * 64)); };
+    request(t0);
+    int piece = 0, before = 2;
+    for (int t = t0; t < t1; ++t) {
+        const int buf = (t - t0) & 1;
+        next.put(xt[piece]);
+        gturn[buf][tcol][trow] = ng;
+        __syncthreads();  // this piece is filled, the one before holds its gradient, the third has been stored
+        if (t + 1 < t1) request(t + 1);
+        if (gx && t > t0) store(t - 1, before);
+        float xs[K], om[K];
+#pragma unroll
+        for (int j = 0; j < K; ++j) { xs[j] = xt[piece][lane][wave * K + j]; om[j] = 1.0f - xs[j]; }
+        const float g = gturn[buf][wave][lane];
+        float u[LL], w[LU], dx[K];
+        prob_products<KL>(xs, om, u);
+        prob_products<KU>(xs + KL, om + KL, w);
+        if (gx) {
+            if constexpr (KL > 0) {
+                float V[LL];
+#pragma unroll
+                for (int lo = 0; lo < LL; ++lo) {
+                    V[lo] = tab[lo] * w[0];
+#pragma unroll
+                    for (int hi = 1; hi < LU; ++hi) V[lo] = fmaf(tab[lo | (hi << KL)], w[hi], V[lo]);
+                }
+                prob_fold_gradient<KL>(V, xs, om, dx);
+            }
+            float Z[LU];
+#pragma unroll
+            for (int hi = 0; hi < LU; ++hi) {
+                Z[hi] = tab[hi << KL] * u[0];
+#pragma unroll
+                for (int lo = 1; lo < LL; ++lo) Z[hi] = fmaf(tab[lo | (hi << KL)], u[lo], Z[hi]);
+            }
+            prob_fold_gradient<KU>(Z, xs + KL, om + KL, dx + KL);
+#pragma unroll
+            for (int j = 0; j < K; ++j) xt[piece][lane][wave * K + j] = g * dx[j];
+        }
+#pragma unroll
+        for (int lo = 0; lo < LL; ++lo) {
+            const float gu = g * u[lo];
+#pragma unroll
+            for (int hi = 0; hi < LU; ++hi) acc[lo | (hi << KL)] = fmaf(gu, w[hi], acc[lo | (hi << KL)]);
+        }
+        before = piece;
+        piece = piece == 2 ? 0 : piece + 1;
+    }
+    if (gx) {
+        __syncthreads();
+        store(t1 - 1, before);
+    }
+    const float mine = prob_sum_lanes<K>(acc, lane);
+    const int a = prob_sum_entry<K>(lane);
+    if (!live || (lane & ((64 >> K) - 1)) != 0) return;
+    if (gpart) {
+        gpart[((size_t)blockIdx.y * N + n) * L + a] = mine;
+    } else {
+        const float s = sig[(size_t)n * L + a];
+        graw[(size_t)n * L + a] = mine * s * (1.0f - s) * prob_inv_t_of(T, n);
+    }
 }
 
 // graw[n,a,d] = sigmoid'(w/T)/T * sum over chunks of gpart[chunk][c][a];
@@ -706,10 +953,9 @@ static inline int prob_block_columns(long long NO) { return NO <= 12 ? 4 : 16; }
 // keep it (k = 5: 31.7 against 34.7 in more).  Few columns over many rows, with at most 16 chunks / as here, kernel and
 // gather with the sum, us: 147456 rows x 32 columns, k = 6 243 + 42 / 52 + 46, k = 4 144 + 27 / 37 + 29; 65536 rows x 1 column, k = 6
 // 67 + 7 / 11 + 11, x 64 columns, k = 4 57 + 17 / 26 + 17.
-static inline int prob_tiles_per_chunk(int B, int N, int k, int O) {
-    const int BT = prob_bt(B), own = k >= 6 ? 6 : (k == 5 ? 4 : 2);
-    const int W = prob_block_columns((long long)N * O), resident = 256 * 16 / W;
-    const long long blocks = dl_ceil_div((long long)N * O, W);
+static inline int prob_tiles_per_chunk_of(int BT, long long columns, int W, int own) {
+    const int resident = 256 * 16 / W;
+    const long long blocks = dl_ceil_div(columns, W);
     int best = BT;
     double best_cost = 0.0;
     auto consider = [&](long long c) {
@@ -723,6 +969,10 @@ static inline int prob_tiles_per_chunk(int B, int N, int k, int O) {
     for (int c = 20; c <= BT; c += c / 4) consider(c);
     for (int rounds = 1; rounds <= 4; ++rounds) consider(rounds * resident / blocks);  // no CU idle in the last round
     return best;
+}
+static inline int prob_bwd_own_tiles(int k) { return k >= 6 ? 6 : (k == 5 ? 4 : 2); }
+static inline int prob_tiles_per_chunk(int B, int N, int k, int O) {
+    return prob_tiles_per_chunk_of(prob_bt(B), (long long)N * O, prob_block_columns((long long)N * O), prob_bwd_own_tiles(k));
 }
 static inline size_t prob_sig_bytes(int N, int k, int O) { return dl_align256((size_t)N * O * ((size_t)1 << k) * sizeof(float)); }
 static inline size_t prob_xT_bytes(int B, int I) { return dl_align256((size_t)prob_bt(B) * I * 64 * sizeof(float)); }
@@ -860,6 +1110,84 @@ extern "C" int dl_prob_layer_bwd_nodes(const float *x, const void *saved, const 
     if (!temperature_n) return DL_ERR_NULL;
     return prob_backward(x, saved, idx32, inv_ptr, inv_pos, raw_w, prob_temp(1.0f, temperature_n), gy, gx, graw, ws, ws_bytes,
                          B, I, N, k, O, stream);
+}
+
+// Nodes that read their inputs in order (prob_ordered_*).
+static inline int prob_ordered_check(int B, int N, int k) {
+    const int rc = prob_check(B, 1, N, k, 1);
+    if (rc) return rc;
+    return k <= DL_MAX_FAST_K && (long long)N * k < (1 << 23) ? DL_OK : DL_ERR_UNSUPPORTED;
+}
+static inline int prob_ordered_bwd_tiles(int B, int N, int k) {
+    return prob_tiles_per_chunk_of(prob_bt(B), N, PROB_ON, prob_bwd_own_tiles(k));
+}
+// values per access: the rows of x and gx have to start on multiples of that (and a block's columns to end there)
+static inline int prob_ordered_wide(const float *x, const float *gx, int N, int k) {
+    const uintptr_t at = (uintptr_t)x | (uintptr_t)gx;
+    const long long M = (long long)N * k;
+    return M % 4 == 0 && at % 16 == 0 ? 4 : M % 2 == 0 && at % 8 == 0 ? 2 : 1;
+}
+extern "C" size_t dl_prob_ordered_saved_bytes(int N, int k) {
+    return N <= 0 || k <= 0 || k > DL_MAX_FAST_K ? 256 : prob_sig_bytes(N, k, 1);
+}
+extern "C" size_t dl_prob_ordered_bwd_workspace_bytes(int B, int N, int k) {
+    if (B <= 0 || prob_ordered_check(B, N, k) != DL_OK) return 256;
+    const int chunks = dl_ceil_div(prob_bt(B), prob_ordered_bwd_tiles(B, N, k));
+    return chunks > 1 ? chunks * prob_sig_bytes(N, k, 1) : 256;
+}
+extern "C" int dl_prob_ordered_fwd(const float *x, const float *raw_w, float temperature, const float *temperature_n, float *y,
+                                   void *saved, size_t saved_bytes, int B, int N, int k, void *stream) {
+    if (!x || !raw_w || !y || !saved) return DL_ERR_NULL;
+    const int rc = prob_ordered_check(B, N, k);
+    if (rc) return rc;
+    if (saved_bytes < dl_prob_ordered_saved_bytes(N, k)) return DL_ERR_WORKSPACE;
+    hipStream_t s = (hipStream_t)stream;
+    const ProbTemp T = prob_temp(temperature, temperature_n);
+    const int BT = prob_bt(B), tpc = prob_tiles_per_chunk_of(BT, N, PROB_ON, 1);
+    const dim3 grid(dl_ceil_div(N, PROB_ON), dl_ceil_div(BT, tpc));
+    const int wide = prob_ordered_wide(x, nullptr, N, k);
+#define CALL(KK)                                                                                                                \
+    do {                                                                                                                        \
+        if (wide == 4) DL_TIMED("prob_ordered_fwd", s, (prob_ordered_fwd<KK, 4><<<grid, 64 * PROB_ON, 0, s>>>(                  \
+            x, raw_w, T, (float *)saved, y, B, N, BT, tpc)));                                                                   \
+        else if (wide == 2) DL_TIMED("prob_ordered_fwd", s, (prob_ordered_fwd<KK, 2><<<grid, 64 * PROB_ON, 0, s>>>(             \
+            x, raw_w, T, (float *)saved, y, B, N, BT, tpc)));                                                                   \
+        else DL_TIMED("prob_ordered_fwd", s, (prob_ordered_fwd<KK, 1><<<grid, 64 * PROB_ON, 0, s>>>(                            \
+            x, raw_w, T, (float *)saved, y, B, N, BT, tpc)));                                                                   \
+    } while (0)
+    PROB_DISPATCH(k, CALL)
+#undef CALL
+    return dl_launch_status();
+}
+extern "C" int dl_prob_ordered_bwd(const float *x, const void *saved, float temperature, const float *temperature_n, const float *gy,
+                                   float *gx, float *graw, void *ws, size_t ws_bytes, int B, int N, int k, void *stream) {
+    if (!x || !saved || !gy || !graw || !ws) return DL_ERR_NULL;
+    const int rc = prob_ordered_check(B, N, k);
+    if (rc) return rc;
+    if (ws_bytes < dl_prob_ordered_bwd_workspace_bytes(B, N, k)) return DL_ERR_WORKSPACE;
+    hipStream_t s = (hipStream_t)stream;
+    const ProbTemp T = prob_temp(temperature, temperature_n);
+    const int BT = prob_bt(B), tpc = prob_ordered_bwd_tiles(B, N, k), chunks = dl_ceil_div(BT, tpc), L = 1 << k;
+    const dim3 grid(dl_ceil_div(N, PROB_ON), chunks);
+    const float *sig = (const float *)saved;
+    float *gpart = chunks > 1 ? (float *)ws : nullptr;
+    const int wide = prob_ordered_wide(x, gx, N, k);
+#define CALL(KK)                                                                                                                \
+    do {                                                                                                                        \
+        if (wide == 4) DL_TIMED("prob_ordered_bwd", s, (prob_ordered_bwd<KK, 4><<<grid, 64 * PROB_ON, 0, s>>>(                  \
+            x, gy, sig, T, gx, gpart, graw, B, N, BT, tpc)));                                                                   \
+        else if (wide == 2) DL_TIMED("prob_ordered_bwd", s, (prob_ordered_bwd<KK, 2><<<grid, 64 * PROB_ON, 0, s>>>(             \
+            x, gy, sig, T, gx, gpart, graw, B, N, BT, tpc)));                                                                   \
+        else DL_TIMED("prob_ordered_bwd", s, (prob_ordered_bwd<KK, 1><<<grid, 64 * PROB_ON, 0, s>>>(                            \
+            x, gy, sig, T, gx, gpart, graw, B, N, BT, tpc)));                                                                   \
+    } while (0)
+    PROB_DISPATCH(k, CALL)
+#undef CALL
+    if (chunks > 1) {
+        const ProbReduce R = {gpart, sig, T, graw, N, L, 1, chunks};
+        DL_TIMED("prob_reduce_weights", s, (prob_reduce_weights<<<dl_ceil_div((long long)N * L, 256), 256, 0, s>>>(R)));
+    }
+    return dl_launch_status();
 }
 
 // Hybrid nodes: the forward is the DWN lookup; the backward is the probabilistic one on the table as given.

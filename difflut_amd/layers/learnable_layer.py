@@ -97,8 +97,7 @@ class LearnableLayer(BaseLUTLayer):
     def _identity_node_plan(self, device):
         """Nodes read the mapped tensor [batch, N*n] in order: node i takes columns i*n .. i*n+n-1."""
         if self._node_plan is None or self._node_plan.device != device:
-            table = torch.arange(self.output_size * self.n, dtype=torch.int32, device=device)
-            self._node_plan = ops.MappingPlan(table.view(self.output_size, self.n), self.output_size * self.n)
+            self._node_plan = ops.MappingPlan.in_order(self.output_size, self.n, device)
         return self._node_plan
 
     def get_mapping(self, x):

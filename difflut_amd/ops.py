@@ -45,6 +45,8 @@ class MappingPlan:
     Built once per table with torch ops (sort + bincount); the kernels only read it.
     """
 
+    ordered = False  # position p reads input p: known of a plan made by in_order()
+
     def __init__(self, idx, input_size):
         if idx.dim() != 2:
             raise ValueError(f"mapping indices must be 2D (nodes, inputs per node), got {tuple(idx.shape)}")
@@ -72,6 +74,17 @@ class MappingPlan:
     def matches(self, idx):
         return (idx.device == self.device and idx.data_ptr() == self.source_ptr
                 and idx._version == self.source_version and tuple(idx.shape) == (self.N, self.k))
+
+    @classmethod
+    def in_order(cls, N, k, device):
+        """The plan of N nodes that take the N*k inputs in order: every one of its tables counts up."""
+        plan = cls.__new__(cls)
+        plan.N, plan.k, plan.I, plan.device, plan.ordered = N, k, N * k, device, True
+        counting = torch.arange(N * k + 1, dtype=torch.int32, device=device)
+        plan.inv_ptr, plan.inv_pos = counting, counting[:-1]
+        plan.idx32 = plan.inv_pos.view(N, k)
+        plan.source_ptr, plan.source_version = plan.idx32.data_ptr(), plan.idx32._version
+        return plan
 
     @staticmethod
     def identity(k, device):
@@ -277,8 +290,8 @@ class ProbLayerFunction:
     def apply(x, raw, plan, temperature):
         nat.require_device(x, raw)
         if torch.is_tensor(temperature):
-            return nat.host().prob_layer(x, raw, plan.host, temperature, 0.0)
-        return nat.host().prob_layer(x, raw, plan.host, None, temperature)
+            return nat.host().prob_layer(x, raw, plan.host, plan.ordered, temperature, 0.0)
+        return nat.host().prob_layer(x, raw, plan.host, plan.ordered, None, temperature)
 
 
 def prob_layer_eval(x, raw, plan, temperature):

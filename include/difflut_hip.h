@@ -331,6 +331,16 @@ int dl_prob_layer_bwd_nodes(const float *x, const void *saved, const int32_t *id
                             const int32_t *inv_pos, const float *raw_w, const float *temperature_n, const float *gy,
                             float *gx, float *graw, void *ws, size_t ws_bytes, int B, int I, int N, int k, int O,
                             void *stream);
+/* The same for nodes of one output that read their inputs in order, x [B, N*k] with node n on columns n*k .. n*k+k-1 (what
+ * LearnableLayer's mapping hands its nodes, difflut/layers/learnable_layer.py:418-445): x, y and the gradients are read and
+ * written as they lie.  `saved` (dl_prob_ordered_saved_bytes) receives the sigmoid table.  temperature_n (nullable): every
+ * node's own.  gx [B, N*k] (nullable) and graw are overwritten.  k <= DL_MAX_FAST_K, N*k < 2^23. */
+size_t dl_prob_ordered_saved_bytes(int N, int k);
+size_t dl_prob_ordered_bwd_workspace_bytes(int B, int N, int k);
+int dl_prob_ordered_fwd(const float *x, const float *raw_w, float temperature, const float *temperature_n, float *y,
+                        void *saved, size_t saved_bytes, int B, int N, int k, void *stream);
+int dl_prob_ordered_bwd(const float *x, const void *saved, float temperature, const float *temperature_n, const float *gy,
+                        float *gx, float *graw, void *ws, size_t ws_bytes, int B, int N, int k, void *stream);
 /* Eval forward (probabilistic_node.py:302-328): y = (sigmoid(raw_w[n,addr,d]/T) >= 0.5). */
 int dl_prob_layer_eval(const float *x, const int32_t *idx32, const float *raw_w, float temperature,
                        float *y, int B, int I, int N, int k, int O, void *stream);

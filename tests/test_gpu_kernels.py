@@ -705,6 +705,42 @@ def test_prob_backward_of_few_columns(B, N, O, hybrid, k):
     np.testing.assert_allclose(wt.grad.cpu().numpy(), gw, rtol=1e-5, atol=2e-5)
 
 
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("B,N,offset", [(64, 16, 0),     # one block, one batch tile
+                                        (1, 13, 0),      # one row, a block that is not full
+                                        (65, 17, 0), (65, 18, 2), (200, 20, 1),  # a row and columns past that; x off 16 and off 8 bytes
+                                        (129, 4112, 0),  # one chunk of tiles: no partial sums
+                                        (1500, 33, 0)])  # several chunks
+def test_prob_nodes_in_order(B, N, offset, k):
+    """Nodes that take their inputs in order: the same sums in the same order as through an index table that says so, which the
+    oracle checks in the tests above, so the tolerance is that of a differently contracted multiply-add: a few units of the last place."""
+    ops = _ops()
+    g = torch.Generator("cuda").manual_seed(B + N + k)
+    M = N * k
+    x = torch.rand(B * M + offset, device="cuda", generator=g)[offset:].view(B, M)
+    x[:, 0] = (x[:, 0] > 0.5).float()
+    raw = torch.randn(N, 1 << k, 1, device="cuda", generator=g)
+    gy = torch.randn(B, N, device="cuda", generator=g)
+    T = torch.rand(N, device="cuda", generator=g) + 0.5
+    general = ops.MappingPlan(torch.arange(M, device="cuda", dtype=torch.int32).view(N, k), M)
+    ordered = ops.MappingPlan.in_order(N, k, x.device)
+    for name in ("idx32", "inv_ptr", "inv_pos"):
+        assert torch.equal(getattr(general, name), getattr(ordered, name)) and getattr(general, name).dtype == getattr(ordered, name).dtype
+    assert ordered.ordered and not general.ordered and general.I == ordered.I
+    for temperature in (T, 0.7):
+        got = []
+        for plan in (general, ordered):
+            xt, wt = x.detach().requires_grad_(), raw.clone().requires_grad_()
+            y = ops.ProbLayerFunction.apply(xt, wt, plan, temperature)
+            y.backward(gy)
+            w2 = raw.clone().requires_grad_()  # the tables alone
+            ops.ProbLayerFunction.apply(x, w2, plan, temperature).backward(gy)
+            assert torch.equal(w2.grad, wt.grad)
+            got.append((y.detach(), xt.grad, wt.grad))
+        for a, b, floor in zip(*got, (5e-7, 2e-6, 2e-6 * B ** 0.5)):
+            torch.testing.assert_close(a, b, rtol=1e-6, atol=floor)
+
+
 @pytest.mark.parametrize("tag", ["k4o2", "k6o1"])
 def test_prob_node_against_reference_vectors(golden, tag):
     from difflut_amd.nodes.probabilistic_node import probabilistic_forward
