@@ -1483,14 +1483,11 @@ static void dwn_launch_lookup(const u64 *planes, const int *idx32, const float *
     const int BT = dwn_bt(B);
     const int grid = dl_xcd_grid(dl_ceil_div((long long)N * O, DWN_TC), BT);
     if (eval) {  // addrT is not written
-#define DWN_EVAL(O1_, CHAIN_, GSUM_)                                                                                     \
-    DL_TIMED("dwn_lookup_eval", s, (dwn_lookup_fwd<K, O1_, CHAIN_, GSUM_, true><<<grid, 64 * DWN_FW, 0, s>>>(            \
-                                       planes, idx32, luts, y, addrT, planes_out, B, I, N, O, BT, gsize > 0 ? gsize : 1, \
-                                       slots > 0 ? slots : 1, run_if_set)))
-        if (gsize > 0 && O == 1) DWN_EVAL(true, false, true);
-        else if (gsize > 0) DWN_EVAL(false, false, true);
-        else if (O == 1) DWN_EVAL(true, true, false);
-        else DWN_EVAL(false, true, false);
+#define DWN_EVAL(O1_)                                                                                        \
+    DL_TIMED("dwn_lookup_eval", s, (dwn_lookup_fwd<K, O1_, true, false, true><<<grid, 64 * DWN_FW, 0, s>>>( \
+                                       planes, idx32, luts, y, addrT, planes_out, B, I, N, O, BT, 1, 1, run_if_set)))
+        if (O == 1) DWN_EVAL(true);
+        else DWN_EVAL(false);
 #undef DWN_EVAL
         return;
     }
@@ -2104,6 +2101,72 @@ extern "C" int dl_table_sigmoid_bwd(const float *gluts, const float *luts, float
 // SAVE: the training forward of a chained hidden layer - the same planes out, plus the address of every
 // (node, row) for the backward ([tile][node][64] bytes): the k plane words are turned into 16 words of four
 // address bytes each (a nibble of rows times 0x204081 puts its four bits at the bottom of four bytes).
+// 64 x 64 bits over the lanes of a wavefront turned: bit b of lane l becomes bit l of lane b
+__device__ __forceinline__ u64 dwn_turn_bits(u64 v, int lane) {
+    unsigned lo = (unsigned)v, hi = (unsigned)(v >> 32);
+    {  // the halves: lane l < 32 keeps its low word and takes lane l + 32's, which keeps the high ones
+        const bool up = (lane & 32) != 0;
+        const unsigned got = (unsigned)__shfl_xor((int)(up ? lo : hi), 32);
+        if (up) lo = got;
+        else hi = got;
+    }
+    const auto step = [&](auto by, unsigned low) __attribute__((always_inline)) {
+        constexpr int S = decltype(by)::value;
+        const bool up = (lane & S) != 0;
+        const unsigned olo = (unsigned)__builtin_amdgcn_ds_swizzle((int)lo, (S << 10) | 0x1f),  // lane ^ S of the same 32
+                       ohi = (unsigned)__builtin_amdgcn_ds_swizzle((int)hi, (S << 10) | 0x1f);
+        lo = up ? (lo & ~low) | ((olo >> S) & low) : (lo & low) | ((olo << S) & ~low);
+        hi = up ? (hi & ~low) | ((ohi >> S) & low) : (hi & low) | ((ohi << S) & ~low);
+    };
+    step(std::integral_constant<int, 16>{}, 0x0000ffffu);
+    step(std::integral_constant<int, 8>{}, 0x00ff00ffu);
+    step(std::integral_constant<int, 4>{}, 0x0f0f0f0fu);
+    step(std::integral_constant<int, 2>{}, 0x33333333u);
+    step(std::integral_constant<int, 1>{}, 0x55555555u);
+    return ((u64)hi << 32) | lo;
+}
+// truth tables of the wavefront's 64 columns from c0 on: row u of the tables is read with lane = entry, its bits are turned
+template <int K>
+__device__ __forceinline__ void dwn_truth_bits(const float *__restrict__ luts, int c0, int NO, int lane, unsigned &t_lo, unsigned &t_hi) {
+    constexpr int L = 1 << K;
+    t_lo = t_hi = 0u;
+    float tv[64];  // all 64 rows asked for at once: one trip to memory, not one per handful of rows
+#pragma unroll
+    for (int u = 0; u < 64; ++u) tv[u] = lane < L ? luts[(size_t)min(c0 + u, NO - 1) * L + lane] : 0.0f;
+#pragma unroll
+    for (int u = 0; u < 32; ++u) {
+        t_lo |= tv[u] >= 0.5f ? 1u << u : 0u;
+        t_hi |= tv[32 + u] >= 0.5f ? 1u << u : 0u;
+    }
+    const u64 turned = dwn_turn_bits(((u64)t_hi << 32) | t_lo, lane);
+    t_lo = (unsigned)turned;
+    t_hi = (unsigned)(turned >> 32);
+}
+template <int K>
+__device__ __forceinline__ u64 dwn_sliced(unsigned t_lo, unsigned t_hi, const u64 (&w)[K]) {
+    constexpr int L = 1 << K;
+    unsigned vlo[L / 2 > 0 ? L / 2 : 1], vhi[L / 2 > 0 ? L / 2 : 1];
+    const unsigned x0lo = (unsigned)w[0], x0hi = (unsigned)(w[0] >> 32);
+#pragma unroll
+    for (int i = 0; i < L / 2; ++i) {  // level of input 0: the leaves are table bits, spread to 0 / ~0
+        const unsigned src0 = (2 * i < 32) ? t_lo : t_hi, src1 = (2 * i + 1 < 32) ? t_lo : t_hi;
+        const unsigned m0 = (unsigned)__builtin_amdgcn_sbfe((int)src0, (2 * i) & 31, 1);
+        const unsigned m1 = (unsigned)__builtin_amdgcn_sbfe((int)src1, (2 * i + 1) & 31, 1);
+        const unsigned d = m0 ^ m1;
+        vlo[i] = m0 ^ (d & x0lo);
+        vhi[i] = m0 ^ (d & x0hi);
+    }
+#pragma unroll
+    for (int j = 1; j < K; ++j) {
+        const unsigned xlo = (unsigned)w[j], xhi = (unsigned)(w[j] >> 32);
+#pragma unroll
+        for (int i = 0; i < (L >> (j + 1)); ++i) {
+            vlo[i] = vlo[2 * i] ^ ((vlo[2 * i] ^ vlo[2 * i + 1]) & xlo);
+            vhi[i] = vhi[2 * i] ^ ((vhi[2 * i] ^ vhi[2 * i + 1]) & xhi);
+        }
+    }
+    return ((u64)vhi[0] << 32) | vlo[0];
+}
 template <int K, bool SAVE = false>
 __global__ __launch_bounds__(256) void dwn_eval_bitsliced(const u64 *__restrict__ planes, const int *__restrict__ idx32,
                                                            const float *__restrict__ luts, u64 *__restrict__ planes_out,
@@ -2118,18 +2181,8 @@ __global__ __launch_bounds__(256) void dwn_eval_bitsliced(const u64 *__restrict_
     const int wc0 = (blockIdx.x * 4 + wave) * 64;  // my wavefront's first column
     if (wc0 >= NO) return;
     const int c = min(wc0 + lane, NO - 1);
-    // truth tables of the wavefront's 64 columns: row u of the tables is read with lane = entry and voted on
-    unsigned t_lo = 0u, t_hi = 0u;
-    {
-        float tv[64];  // all 64 rows asked for at once: one trip to memory, not one per handful of rows
-#pragma unroll
-        for (int u = 0; u < 64; ++u) tv[u] = lane < L ? luts[(size_t)min(wc0 + u, NO - 1) * L + lane] : 0.0f;
-#pragma unroll
-        for (int u = 0; u < 64; ++u) {
-            const u64 bits = __ballot(tv[u] >= 0.5f);
-            if (lane == u) { t_lo = (unsigned)bits; t_hi = (unsigned)(bits >> 32); }
-        }
-    }
+    unsigned t_lo, t_hi;
+    dwn_truth_bits<K>(luts, wc0, NO, lane, t_lo, t_hi);
     int off[K];  // word offsets of my inputs inside a tile's planes
 #pragma unroll
     for (int j = 0; j < K; ++j) off[j] = idx32[(size_t)(c / O) * K + j];
@@ -2143,29 +2196,10 @@ __global__ __launch_bounds__(256) void dwn_eval_bitsliced(const u64 *__restrict_
     if (t_begin < t_end) fetch(t_begin, w);
     for (int t = t_begin; t < t_end; ++t) {
         if (t + 1 < t_end) fetch(t + 1, wn);
-        unsigned vlo[L / 2 > 0 ? L / 2 : 1], vhi[L / 2 > 0 ? L / 2 : 1];
-        const unsigned x0lo = (unsigned)w[0], x0hi = (unsigned)(w[0] >> 32);
-#pragma unroll
-        for (int i = 0; i < L / 2; ++i) {  // level of input 0: the leaves are table bits, spread to 0 / ~0
-            const unsigned src0 = (2 * i < 32) ? t_lo : t_hi, src1 = (2 * i + 1 < 32) ? t_lo : t_hi;
-            const unsigned m0 = (unsigned)__builtin_amdgcn_sbfe((int)src0, (2 * i) & 31, 1);
-            const unsigned m1 = (unsigned)__builtin_amdgcn_sbfe((int)src1, (2 * i + 1) & 31, 1);
-            const unsigned d = m0 ^ m1;
-            vlo[i] = m0 ^ (d & x0lo);
-            vhi[i] = m0 ^ (d & x0hi);
-        }
-#pragma unroll
-        for (int j = 1; j < K; ++j) {
-            const unsigned xlo = (unsigned)w[j], xhi = (unsigned)(w[j] >> 32);
-#pragma unroll
-            for (int i = 0; i < (L >> (j + 1)); ++i) {
-                vlo[i] = vlo[2 * i] ^ ((vlo[2 * i] ^ vlo[2 * i + 1]) & xlo);
-                vhi[i] = vhi[2 * i] ^ ((vhi[2 * i] ^ vhi[2 * i + 1]) & xhi);
-            }
-        }
+        const u64 bits = dwn_sliced<K>(t_lo, t_hi, w);
         const int rows = min(64, B - t * 64);  // rows past B stay 0, like the planes packed from x
         const u64 valid = rows == 64 ? ~0ull : ((1ull << rows) - 1ull);
-        if (wc0 + lane < NO) planes_out[(size_t)t * NO + wc0 + lane] = (((u64)vhi[0] << 32) | vlo[0]) & valid;
+        if (wc0 + lane < NO) planes_out[(size_t)t * NO + wc0 + lane] = bits & valid;
         if (SAVE && wc0 + lane < NO && c % O == 0) {
             u4v *dst = reinterpret_cast<u4v *>(addrT + ((size_t)t * N + c / O) * 64);
             // word q = the address bytes of rows 4q .. 4q + 3.  Bit j of those four bytes: nibble q of plane j times
@@ -2237,6 +2271,189 @@ static void dwn_launch_eval_bitsliced(const u64 *planes, const int *idx32, const
     else
         DL_TIMED("dwn_eval_bitsliced", s, (dwn_eval_bitsliced<K><<<dim3(col_blocks, dl_ceil_div(BT, tpb)), 256, 0, s>>>(
                                               planes, idx32, luts, planes_out, B, I, N, O, BT, tpb)));
+}
+
+// ---------------------------------------------------------------------------------
+// The last layer of an inference chain under a GroupSum head, bit-sliced: logits straight from the planes.  A wavefront evaluates
+// 64 columns of a group on a batch tile as dwn_eval_bitsliced does - lane = column, bit = row -, turns the 64 x 64 bits in six
+// exchanges between lanes, so that a lane has its ROW's outputs, and counts them; the counts of a group's columns add up in a
+// register per tile.  A block has one group and DWN_GROUP_TILES tiles, its wavefronts share the group's columns.  Before: the lookup
+// of the training forward with 0/1 outputs and partial sums that a second launch added.
+// Bound by the chain tables, indices, plane words.  5001 rows, 4000-2000-1000 nodes of six inputs in 10 groups: the model 42.4 -> 36.3 us.
+// Eight wavefronts to a block rather than four: 64 rows of 8000 nodes 30 -> 21 us.
+#define DWN_GROUP_TILES 4
+#define DWN_GROUP_WAVES 8
+template <int K>
+__global__ __launch_bounds__(64 * DWN_GROUP_WAVES) void dwn_eval_groups(const u64 *__restrict__ planes, const int *__restrict__ idx32,
+                                                        const float *__restrict__ luts, float *__restrict__ logits, int B, int I,
+                                                        int NO, int O, int BT, int groups, int gsize, float inv_tau) {
+    __shared__ int part[DWN_GROUP_WAVES][DWN_GROUP_TILES][64];
+    const int lane = threadIdx.x & 63, wave = dl_uniform(threadIdx.x >> 6), waves = blockDim.x >> 6;
+    const int g = blockIdx.x, t0 = blockIdx.y * DWN_GROUP_TILES;
+    const int c_lo = g * gsize, c_hi = min(NO, c_lo + gsize);
+    int count[DWN_GROUP_TILES];
+#pragma unroll
+    for (int q = 0; q < DWN_GROUP_TILES; ++q) count[q] = 0;
+    for (int c0 = c_lo + wave * 64; c0 < c_hi; c0 += waves * 64) {
+        unsigned t_lo, t_hi;
+        dwn_truth_bits<K>(luts, c0, NO, lane, t_lo, t_hi);
+        const int c = min(c0 + lane, c_hi - 1);
+        int off[K];
+#pragma unroll
+        for (int j = 0; j < K; ++j) off[j] = idx32[(size_t)(c / O) * K + j];
+        u64 w[DWN_GROUP_TILES][K];
+#pragma unroll
+        for (int q = 0; q < DWN_GROUP_TILES; ++q)
+#pragma unroll
+            for (int j = 0; j < K; ++j) w[q][j] = planes[(size_t)min(t0 + q, BT - 1) * I + off[j]];
+#pragma unroll
+        for (int q = 0; q < DWN_GROUP_TILES; ++q) {
+            const u64 bits = dwn_sliced<K>(t_lo, t_hi, w[q]);
+            count[q] += __popcll(dwn_turn_bits(c0 + lane < c_hi ? bits : 0ull, lane));
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < DWN_GROUP_TILES; ++q) part[wave][q][lane] = count[q];
+    __syncthreads();
+    for (int e = threadIdx.x; e < DWN_GROUP_TILES * 64; e += blockDim.x) {
+        int sum = 0;
+        for (int v = 0; v < waves; ++v) sum += part[v][e >> 6][e & 63];
+        const int b = t0 * 64 + e;
+        if (b < B) logits[(size_t)b * groups + g] = (float)sum * inv_tau;
+    }
+}
+template <int K>
+static void dwn_launch_eval_groups(const u64 *planes, const int *idx32, const float *luts, float *logits, int B, int I, int N, int O,
+                                   int groups, int gsize, float tau, hipStream_t s) {
+    const int BT = dwn_bt(B), pieces = dl_ceil_div(gsize, 64), waves = pieces < DWN_GROUP_WAVES ? pieces : DWN_GROUP_WAVES;
+    DL_TIMED("dwn_eval_groups", s, (dwn_eval_groups<K><<<dim3(groups, dl_ceil_div(BT, DWN_GROUP_TILES)), 64 * waves, 0, s>>>(
+                                       planes, idx32, luts, logits, B, I, N * O, O, BT, groups, gsize, 1.0f / tau)));
+}
+
+// ---------------------------------------------------------------------------------
+// A layer of an inference chain on few rows, one launch: what it reads may be the raw features behind a thermometer encoder
+// (DWN_FROM_CODE), 0/1 values (DWN_FROM_X) or planes, what it leaves planes or, under a GroupSum head, the logits.  A thread is a
+// column and has R rows: it reads the indices, then its rows' inputs (and thresholds), then a table entry per row - three trips to
+// memory, which with the launch itself is all the time such a call takes.  No planes of the input, no partial sums, no second and
+// third launch.  A block is a group, or as many columns.  R = 1: fewer than eight rows of a whole model (HEAD); else eight rows, a byte of
+// every plane word.  What a load of one value per lane at random places costs is the texture addresser's 64 cycles, so the rows of x
+// are staged in the LDS where they fit (STAGE).
+#define DWN_FROM_PLANES 0
+#define DWN_FROM_CODE 1
+#define DWN_FROM_X 2
+struct DwnRows {
+    const float *x, *thr;
+    const uint8_t *planes;
+    const int *idx32;
+    const float *luts;
+    uint8_t *planes_out;
+    float *logits;
+    int B, I, NO, O, nbits, groups, gsize;
+    float inv_tau;
+};
+template <int K, int IN, bool HEAD, int R, bool STAGE>
+__global__ __launch_bounds__(1024) void dwn_eval_rows(DwnRows a) {
+    constexpr int L = 1 << K;
+    static_assert(R == 8 || (R == 1 && HEAD), "a plane's byte has one writer");
+    __shared__ int part[16][R];
+    const int tid = threadIdx.x, b0 = blockIdx.y * R, rows = min(R, a.B - b0);
+    const int c_lo = HEAD ? blockIdx.x * a.gsize : blockIdx.x * blockDim.x;
+    const int c_hi = min(a.NO, c_lo + (HEAD ? a.gsize : (int)blockDim.x));
+    const int width = IN == DWN_FROM_CODE ? a.I / a.nbits : a.I;
+    extern __shared__ float staged[];  // [row][width]
+    if constexpr (STAGE) {
+        const float *from = a.x + (size_t)b0 * width;
+        for (int e = tid; e < rows * width; e += blockDim.x) staged[e] = from[e];
+        __syncthreads();
+    }
+    int count[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) count[r] = 0;
+    for (int c0 = c_lo; c0 < c_hi; c0 += blockDim.x) {
+        const bool live = c0 + tid < c_hi;
+        const int c = min(c0 + tid, c_hi - 1);
+        int idx[K];
+#pragma unroll
+        for (int j = 0; j < K; ++j) idx[j] = a.idx32[(size_t)(c / a.O) * K + j];
+        unsigned addr[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) addr[r] = 0;
+        if constexpr (IN == DWN_FROM_PLANES) {
+#pragma unroll
+            for (int j = 0; j < K; ++j) {
+                const unsigned byte = a.planes[((size_t)(b0 >> 6) * a.I + idx[j]) * 8 + ((b0 & 63) >> 3)] >> (b0 & 7);
+#pragma unroll
+                for (int r = 0; r < R; ++r) addr[r] |= ((byte >> r) & 1u) << j;
+            }
+        } else {
+            float limit[K];
+            int col[K];
+#pragma unroll
+            for (int j = 0; j < K; ++j) {
+                col[j] = IN == DWN_FROM_CODE ? (int)((unsigned)idx[j] / (unsigned)a.nbits) : idx[j];
+                limit[j] = IN == DWN_FROM_CODE ? a.thr[idx[j]] : 0.5f;
+            }
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int first = min(r, rows - 1) * width;
+                const float *row = a.x + (size_t)b0 * width + first;
+#pragma unroll
+                for (int j = 0; j < K; ++j) {
+                    const float v = STAGE ? staged[first + col[j]] : row[col[j]];
+                    addr[r] |= ((IN == DWN_FROM_CODE ? v > limit[j] : v >= limit[j]) ? 1u : 0u) << j;
+                }
+            }
+        }
+        bool bit[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) bit[r] = a.luts[(size_t)c * L + addr[r]] >= 0.5f;
+        if constexpr (HEAD) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) count[r] += __popcll(__ballot(live && bit[r]));
+        } else if (live) {
+            unsigned byte = 0;
+#pragma unroll
+            for (int r = 0; r < R; ++r) byte |= r < rows && bit[r] ? 1u << r : 0u;
+            uint8_t *word = a.planes_out + ((size_t)(b0 >> 6) * a.NO + c) * 8;
+            word[(b0 & 63) >> 3] = (uint8_t)byte;
+            if (blockIdx.y == gridDim.y - 1)  // the rows of the last tile that the batch does not have
+                for (int q = ((b0 & 63) >> 3) + 1; q < 8; ++q) word[q] = 0;
+        }
+    }
+    if constexpr (HEAD) {
+        if ((tid & 63) == 0) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) part[tid >> 6][r] = count[r];
+        }
+        __syncthreads();
+        if (tid < rows) {
+            int sum = 0;
+            for (int w = 0; w < (int)blockDim.x >> 6; ++w) sum += part[w][tid];
+            a.logits[(size_t)(b0 + tid) * a.groups + blockIdx.x] = (float)sum * a.inv_tau;
+        }
+    }
+}
+template <int K>
+static void dwn_launch_eval_rows(const DwnRows &a, hipStream_t s) {
+    const bool head = a.logits != nullptr;
+    const int per_block = head ? a.gsize : a.NO, most = head ? 1024 : 256;
+    const int threads = per_block >= most ? most : (per_block + 63) / 64 * 64;
+    const int R = head && a.B < 8 ? 1 : 8;
+    const dim3 grid(head ? a.groups : dl_ceil_div(a.NO, threads), dl_ceil_div(a.B, R));
+    const size_t lds = a.planes ? 0 : (size_t)R * (a.thr ? a.I / a.nbits : a.I) * sizeof(float);
+    const bool stage = lds > 0 && lds <= 64 * 1024;
+#define DWN_ROWS(IN, STAGE)                                                                                                             \
+    do {                                                                                                                                \
+        if (!head) DL_TIMED("dwn_eval_rows", s, (dwn_eval_rows<K, IN, false, 8, STAGE><<<grid, threads, STAGE ? lds : 0, s>>>(a)));      \
+        else if (R == 8) DL_TIMED("dwn_eval_rows", s, (dwn_eval_rows<K, IN, true, 8, STAGE><<<grid, threads, STAGE ? lds : 0, s>>>(a))); \
+        else DL_TIMED("dwn_eval_rows", s, (dwn_eval_rows<K, IN, true, 1, STAGE><<<grid, threads, STAGE ? lds : 0, s>>>(a)));             \
+    } while (0)
+    if (a.planes) DWN_ROWS(DWN_FROM_PLANES, false);
+    else if (a.thr && stage) DWN_ROWS(DWN_FROM_CODE, true);
+    else if (a.thr) DWN_ROWS(DWN_FROM_CODE, false);
+    else if (stage) DWN_ROWS(DWN_FROM_X, true);
+    else DWN_ROWS(DWN_FROM_X, false);
+#undef DWN_ROWS
 }
 
 // ---------------------------------------------------------------------------------
@@ -2427,19 +2644,40 @@ extern "C" int dl_dwn_layer_eval_planes_groups(const void *planes_in, const int3
     if (ws_bytes < dl_dwn_groups_workspace_bytes(B, N, O, groups)) return DL_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
     const u64 *planes = (const u64 *)planes_in;
-    float *partial = (float *)ws;
-    uint8_t *none = (uint8_t *)const_cast<float *>(luts);
     switch (k) {
-        case 1: dwn_launch_lookup<1>(planes, idx32, luts, partial, none, nullptr, B, I, N, O, s, gsize, slots, true); break;
-        case 2: dwn_launch_lookup<2>(planes, idx32, luts, partial, none, nullptr, B, I, N, O, s, gsize, slots, true); break;
-        case 3: dwn_launch_lookup<3>(planes, idx32, luts, partial, none, nullptr, B, I, N, O, s, gsize, slots, true); break;
-        case 4: dwn_launch_lookup<4>(planes, idx32, luts, partial, none, nullptr, B, I, N, O, s, gsize, slots, true); break;
-        case 5: dwn_launch_lookup<5>(planes, idx32, luts, partial, none, nullptr, B, I, N, O, s, gsize, slots, true); break;
-        default: dwn_launch_lookup<6>(planes, idx32, luts, partial, none, nullptr, B, I, N, O, s, gsize, slots, true); break;
+        case 1: dwn_launch_eval_groups<1>(planes, idx32, luts, logits, B, I, N, O, groups, gsize, tau, s); break;
+        case 2: dwn_launch_eval_groups<2>(planes, idx32, luts, logits, B, I, N, O, groups, gsize, tau, s); break;
+        case 3: dwn_launch_eval_groups<3>(planes, idx32, luts, logits, B, I, N, O, groups, gsize, tau, s); break;
+        case 4: dwn_launch_eval_groups<4>(planes, idx32, luts, logits, B, I, N, O, groups, gsize, tau, s); break;
+        case 5: dwn_launch_eval_groups<5>(planes, idx32, luts, logits, B, I, N, O, groups, gsize, tau, s); break;
+        default: dwn_launch_eval_groups<6>(planes, idx32, luts, logits, B, I, N, O, groups, gsize, tau, s); break;
     }
-    DL_TIMED("dwn_group_finish", s,
-             (dwn_group_finish<<<dl_ceil_div((long long)B * groups, 256), 256, 0, s>>>(partial, logits, B, dwn_bt(B) * 64, F,
-                                                                                     groups, gsize, slots, 1.0f / tau)));
+    return dl_launch_status();
+}
+
+// One launch for a layer on few rows: see dwn_eval_rows.
+extern "C" int dl_dwn_layer_eval_rows(const float *x, const float *thr, int nbits, const void *planes_in, const int32_t *idx32,
+                                      const float *luts, void *planes_out, float *logits, int B, int I, int N, int k, int O,
+                                      int groups, float tau, void *stream) {
+    if (!idx32 || !luts || !x == !planes_in || !planes_out == !logits || (thr && !x)) return DL_ERR_NULL;
+    int rc = dwn_check(B, I, N, k, O);
+    if (rc) return rc;
+    if (thr && (nbits <= 0 || I % nbits != 0)) return DL_ERR_SHAPE;
+    if (logits && (groups <= 0 || !(tau > 0.0f))) return DL_ERR_SHAPE;
+    if (!dwn_fast(N, k, O) || B > 65535) return DL_ERR_UNSUPPORTED;
+    const int F = N * O;
+    if (logits && dwn_group_slots(dwn_group_size(F, groups)) > DWN_GS_SLOTS) return DL_ERR_UNSUPPORTED;  // as with a workspace
+    const DwnRows a = {x, thr, (const uint8_t *)planes_in, idx32, luts, (uint8_t *)planes_out, logits, B, I, F, O, nbits,
+                       groups, logits ? dwn_group_size(F, groups) : 1, logits ? 1.0f / tau : 0.0f};
+    hipStream_t s = (hipStream_t)stream;
+    switch (k) {
+        case 1: dwn_launch_eval_rows<1>(a, s); break;
+        case 2: dwn_launch_eval_rows<2>(a, s); break;
+        case 3: dwn_launch_eval_rows<3>(a, s); break;
+        case 4: dwn_launch_eval_rows<4>(a, s); break;
+        case 5: dwn_launch_eval_rows<5>(a, s); break;
+        default: dwn_launch_eval_rows<6>(a, s); break;
+    }
     return dl_launch_status();
 }
 

@@ -31,7 +31,7 @@ namespace {
     X(dl_soft_map_saved_bytes) X(dl_soft_map_workspace_bytes) X(dl_soft_map_fwd) X(dl_soft_map_bwd) X(dl_unfold_rows)    \
     X(dl_unfold_flip) X(dl_fold) X(dl_dwn_planes_bytes) X(dl_dwn_tiled_bytes) X(dl_dwn_pack_planes)                      \
     X(dl_thermometer_planes) X(dl_dwn_groups_workspace_bytes) X(dl_dwn_layer_fwd_planes)                                 \
-    X(dl_dwn_layer_fwd_planes_groups) X(dl_dwn_layer_eval_planes) X(dl_dwn_layer_eval_planes_groups)                     \
+    X(dl_dwn_layer_fwd_planes_groups) X(dl_dwn_layer_eval_planes) X(dl_dwn_layer_eval_planes_groups) X(dl_dwn_layer_eval_rows) \
     X(dl_dwn_layer_bwd_groups) X(dl_dwn_layer_bwd_tiled) X(dl_dwn_chain_fusable) X(dl_dwn_bwd_fused_workspace_bytes)     \
     X(dl_dwn_layer_bwd_chain_fused) X(dl_dwn_chain_first_fusable) X(dl_dwn_bwd_first_workspace_bytes)                    \
     X(dl_dwn_layer_bwd_chain_first) X(dl_cross_entropy_workspace_bytes) X(dl_cross_entropy) X(dl_adam_step)
@@ -344,6 +344,12 @@ struct Stack : torch::CustomClassHolder {
     std::vector<int64_t> image;
     std::vector<Dims> dims;
 };
+Tensor code_thresholds(const Tensor &thresholds, int features) {
+    require_device(thresholds);
+    const Tensor thr = f32(thresholds);
+    TORCH_CHECK(thr.dim() == 2 && thr.size(0) == features, "thresholds ", thr.sizes(), " do not match ", features, " features");
+    return thr;
+}
 // bit-planes of the first layer's input: x itself, its thermometer code or its patch matrix; sets rows and width
 Tensor first_planes(const Tensor &x, const Tensor &thresholds, const Tensor &flip_, Stack &st, int &B, int &width) {
     if (st.patches) {
@@ -375,9 +381,7 @@ Tensor first_planes(const Tensor &x, const Tensor &thresholds, const Tensor &fli
         check(L.dl_dwn_pack_planes(in(x), raw(planes), B, width, stream()));
         return planes;
     }
-    require_device(thresholds);
-    const Tensor thr = f32(thresholds);
-    TORCH_CHECK(thr.dim() == 2 && thr.size(0) == width, "thresholds ", thr.sizes(), " do not match ", width, " features");
+    const Tensor thr = code_thresholds(thresholds, width);
     const int nbits = (int)thr.size(1);
     const Tensor planes = bytes(L.dl_dwn_planes_bytes(B, width * nbits), x);
     check(L.dl_thermometer_planes(in(x), in(thr), raw(planes), B, width, nbits, stream()));
@@ -619,32 +623,56 @@ Tensor dwn_stack(const Tensor &x, const std::vector<Tensor> &luts, const std::ve
     const Tensor thr = tensor_of(thresholds), mask = tensor_of(flip);
     return DwnStack::apply(x, at::TensorList(luts), &thr, &mask, st);
 }
+// Up to so many rows, and rows times columns of all layers, a chain goes a launch per layer (dl_dwn_layer_eval_rows).  On the device,
+// us, planes / rows (nodes of six inputs, ten groups): 2000 nodes B = 1 11.3 / 3.1, 768 14.6 / 11.4, 2048 15.7 / 33; 7920 nodes B = 8 20.4 /
+// 6.4, 384 22.5 / 15.6, 768 22.6 / 30.7; 4000-2000 B = 512 19.2 / 17.6, 768 19.6 / 22.7; 8000-4000 B = 256 24.2 / 19.5, 384 24.4 / 24.5.  And two
+// launches and two allocations less on the host.
+constexpr int64_t ROWS_MOST = 768, ROWS_MOST_WORK = 3 << 20;
 Tensor dwn_stack_eval(const Tensor &x_, const Maybe &thresholds, const std::vector<Tensor> &luts_, const std::vector<PlanArgs> &plans,
                       int64_t groups, double tau) {
     at::NoGradGuard no_grad;
     require_device(x_);
     const Tensor x = f32(x_);
     auto st = stack_of(plans, luts_.size(), groups, tau);
-    int B = 0, width = 0;
-    Tensor planes = first_planes(x, tensor_of(thresholds), Tensor(), *st, B, width), y;
-    for (size_t l = 0; l < luts_.size(); ++l) {
+    const size_t n = luts_.size();
+    int B = 0, width = 0, nbits = 1;
+    Tensor planes, thr, y;
+    // few rows: a launch per layer, the first reads x as it comes
+    int64_t columns = 0;
+    for (const Tensor &t : luts_) columns += t.dim() == 3 ? t.size(0) * t.size(1) : 0;
+    const bool rows = x.dim() == 2 && x.size(0) <= ROWS_MOST && x.size(0) * columns <= ROWS_MOST_WORK && (n > 1 || groups);
+    if (rows) {
+        B = (int)x.size(0), width = (int)x.size(1);
+        if (thresholds) {
+            thr = code_thresholds(*thresholds, width);
+            nbits = (int)thr.size(1);
+            width *= nbits;
+        }
+    } else {
+        planes = first_planes(x, tensor_of(thresholds), Tensor(), *st, B, width);
+    }
+    for (size_t l = 0; l < n; ++l) {
         require_device(luts_[l]);
         const Tensor lut = f32(luts_[l]);
         const Plan &p = st->plans[l];
         const Dims d = chain_dims(l, p, lut, B, width);
-        const bool last = l + 1 == luts_.size();
-        if (last && groups) {
-            y = floats({B, groups}, x);
+        const bool last = l + 1 == n, head = last && groups;
+        Tensor next;
+        if (head) y = floats({B, groups}, x);
+        else if (last) y = floats({B, (int64_t)d.N * d.O}, x);
+        else next = bytes(L.dl_dwn_planes_bytes(B, d.N * d.O), x);
+        if (rows && (head || !last)) {
+            const bool first = !planes.defined();
+            check(L.dl_dwn_layer_eval_rows(first ? in(x) : nullptr, first ? in(thr) : nullptr, nbits, raw(planes), ints(p.idx), in(lut),
+                                           raw(next), head ? out(y) : nullptr, DIMS(d), (int)groups, (float)tau, stream()));
+        } else if (head) {
             const Tensor ws = bytes(L.dl_dwn_groups_workspace_bytes(B, d.N, d.O, (int)groups), x);
             check(L.dl_dwn_layer_eval_planes_groups(raw(planes), ints(p.idx), in(lut), out(y), raw(ws), ws.numel(), DIMS(d), (int)groups,
                                                     (float)tau, stream()));
         } else {
-            Tensor next;
-            if (last) y = floats({B, (int64_t)d.N * d.O}, x);
-            else next = bytes(L.dl_dwn_planes_bytes(B, d.N * d.O), x);
             check(L.dl_dwn_layer_eval_planes(raw(planes), ints(p.idx), in(lut), out(y), raw(next), DIMS(d), stream()));
-            planes = next;
         }
+        planes = next;
         width = d.N * d.O;
     }
     return y;

@@ -591,6 +591,52 @@ def test_gather_through_the_lds(shape):
     assert np.array_equal(xt.grad.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("B", [1, 7, 8, 9, 63, 64, 65, 200])
+@pytest.mark.parametrize("source", ["code", "x", "planes"])
+@pytest.mark.parametrize("width,N,k,O,groups", [(40, 192, 6, 1, 3),    # groups of one wavefront
+                                                (33, 65, 1, 1, 1),     # a group one column longer
+                                                (96, 330, 4, 2, 9),    # groups of 74 columns, the last of 68, two outputs
+                                                (2100, 1300, 5, 1, 1)])  # more than a block's threads; rows too wide for the LDS
+def test_eval_of_few_rows(B, source, width, N, k, O, groups):
+    """One launch per layer against the bit-plane kernels: the same bits, as planes and as group sums; and the group sums from
+    planes against the sums of the layer's output.  Sums of zeros and ones: exact."""
+    from difflut_amd import _native as nat
+
+    lib = nat.lib()
+    g = torch.Generator("cuda").manual_seed(B + width)
+    nbits = 3 if source == "code" else 1
+    I, F = width * nbits, N * O
+    idx = torch.randint(0, I, (N, k), device=DEV, generator=g, dtype=torch.int32)
+    luts = torch.randn(N, O, 1 << k, device=DEV, generator=g)
+    luts[0] = 0.5
+    x = torch.rand(B, width, device=DEV, generator=g)
+    thr = torch.rand(width, nbits, device=DEV, generator=g)
+    x[0, 0] = thr[0, 0]  # not greater
+    if source != "code":
+        x = (x < 0.5).float()
+    planes = torch.empty(lib.dl_dwn_planes_bytes(B, I), dtype=torch.uint8, device=DEV)
+    if source == "code":
+        nat.check(lib.dl_thermometer_planes(x.data_ptr(), thr.data_ptr(), planes.data_ptr(), B, width, nbits, nat.stream()))
+    else:
+        nat.check(lib.dl_dwn_pack_planes(x.data_ptr(), planes.data_ptr(), B, I, nat.stream()))
+    dims = (B, I, N, k, O)
+    y = torch.empty(B, F, device=DEV)
+    used = (B + 63) // 64 * F * 8
+    want, got = (torch.full((max(used, 256),), 7, dtype=torch.uint8, device=DEV) for _ in range(2))
+    nat.check(lib.dl_dwn_layer_eval_planes(planes.data_ptr(), idx.data_ptr(), luts.data_ptr(), y.data_ptr(), want.data_ptr(), *dims, nat.stream()))
+    given = (None, None, 1, planes.data_ptr()) if source == "planes" else (x.data_ptr(), thr.data_ptr() if source == "code" else None, nbits, None)
+    nat.check(lib.dl_dwn_layer_eval_rows(*given, idx.data_ptr(), luts.data_ptr(), got.data_ptr(), None, *dims, 0, 1.0, nat.stream()))
+    assert torch.equal(want[:used], got[:used])
+    gs = -(-F // groups)
+    sums = torch.stack([y[:, q * gs:(q + 1) * gs].sum(1) for q in range(groups)], 1) * (1.0 / 0.5)
+    logits = torch.full((2, B, groups), -1.0, device=DEV)
+    nat.check(lib.dl_dwn_layer_eval_rows(*given, idx.data_ptr(), luts.data_ptr(), None, logits[0].data_ptr(), *dims, groups, 0.5, nat.stream()))
+    ws = torch.empty(lib.dl_dwn_groups_workspace_bytes(B, N, O, groups), dtype=torch.uint8, device=DEV)
+    nat.check(lib.dl_dwn_layer_eval_planes_groups(planes.data_ptr(), idx.data_ptr(), luts.data_ptr(), logits[1].data_ptr(), ws.data_ptr(),
+                                                  ws.numel(), *dims, groups, 0.5, nat.stream()))
+    assert torch.equal(logits[0], sums) and torch.equal(logits[1], sums)
+
+
 # ------------------------------------------------------------------------------ probabilistic
 PROB_SHAPES = [(32, 40, 24, 4, 2), (64, 128, 300, 4, 1), (17, 30, 9, 6, 1), (20, 9, 5, 1, 1), (10, 50, 7, 2, 3),
                (6, 40, 5, 7, 2), (200, 300, 260, 4, 1), (130, 70, 33, 5, 2), (65, 1000, 515, 3, 1),
