@@ -31,6 +31,7 @@
 #include <type_traits>
 #include "dwn_generic.h"
 #include "dwn_pair.h"
+#include "dwn_rows.h"
 
 typedef unsigned long long u64;
 
@@ -1520,10 +1521,22 @@ static void dwn_launch_lookup_wide(const u64 *planes, const int *idx32, const fl
     else DL_TIMED("dwn_lookup_fwd", s, (dwn_lookup_fwd<K, false><<<grid, 64 * DWN_FW, 0, s>>>(planes, idx32, luts, y, addrT, nullptr, B, I, N, O, BT)));
 }
 
+// Few rows of x: one launch (dwn_rows.hip) instead of two, and no planes.  Pack and lookup / one launch, us on the device: 512 inputs, 128
+// columns, any B up to 4096 9 / 4; 2532 x 746 B = 64 10.0 / 6.0, 1024 11.3 / 7.6, 4096 21 / 21; 4096 x 4096 B = 64 9.9 / 7.6, 384 13.5 / 10.3, 768
+// 17.5 / 21.5; 8192 x 2000 B = 384 12.0 / 10.1, 1024 18.3 / 19.1; 8000 x 8000 B = 160 15.4 / 14.2, 256 15.0 / 16.5.  Wider inputs take
+// longer to turn than to pack: 16384 x 2000 B = 64 11.3 / 11.6, 256 11.7 / 15.7.
+static inline bool dwn_few_rows(int B, int I, int N, int k, int O) {
+    return k <= DL_MAX_FAST_K && I <= 8192 && (double)B * (I + (double)N * O) <= 3.5e6;
+}
 // forward of the k <= 8 path: x -> bit-planes (scratch) -> y and the saved addresses
 static int dwn_forward_fast(const float *x, const int32_t *idx32, const float *luts, float *y, void *saved, u64 *planes,
                             int B, int I, int N, int k, int O, hipStream_t s) {
     const int BT = dwn_bt(B);
+    if (dwn_few_rows(B, I, N, k, O)) {  // neither planes nor a second launch
+        const DwnRows a = {x, nullptr, nullptr, idx32, luts, y, nullptr, nullptr, (uint8_t *)saved, B, I, N, O, 1, 1, 1, 0.0f};
+        dwn_launch_rows(k, a, s);
+        return dl_launch_status();
+    }
     if (I % 4 == 0 && ((uintptr_t)x & 15) == 0)
         DL_TIMED("dwn_pack_planes", s, (dwn_pack_planes<4><<<dim3(dl_ceil_div(I, 1024), dwn_pack_grid_y(BT)), 256, 0, s>>>(x, planes, B, I)));
     else
@@ -2331,132 +2344,6 @@ static void dwn_launch_eval_groups(const u64 *planes, const int *idx32, const fl
 }
 
 // ---------------------------------------------------------------------------------
-// A layer of an inference chain on few rows, one launch: what it reads may be the raw features behind a thermometer encoder
-// (DWN_FROM_CODE), 0/1 values (DWN_FROM_X) or planes, what it leaves planes or, under a GroupSum head, the logits.  A thread is a
-// column and has R rows: it reads the indices, then its rows' inputs (and thresholds), then a table entry per row - three trips to
-// memory, which with the launch itself is all the time such a call takes.  No planes of the input, no partial sums, no second and
-// third launch.  A block is a group, or as many columns.  R = 1: fewer than eight rows of a whole model (HEAD); else eight rows, a byte of
-// every plane word.  What a load of one value per lane at random places costs is the texture addresser's 64 cycles, so the rows of x
-// are staged in the LDS where they fit (STAGE).
-#define DWN_FROM_PLANES 0
-#define DWN_FROM_CODE 1
-#define DWN_FROM_X 2
-struct DwnRows {
-    const float *x, *thr;
-    const uint8_t *planes;
-    const int *idx32;
-    const float *luts;
-    uint8_t *planes_out;
-    float *logits;
-    int B, I, NO, O, nbits, groups, gsize;
-    float inv_tau;
-};
-template <int K, int IN, bool HEAD, int R, bool STAGE>
-__global__ __launch_bounds__(1024) void dwn_eval_rows(DwnRows a) {
-    constexpr int L = 1 << K;
-    static_assert(R == 8 || (R == 1 && HEAD), "a plane's byte has one writer");
-    __shared__ int part[16][R];
-    const int tid = threadIdx.x, b0 = blockIdx.y * R, rows = min(R, a.B - b0);
-    const int c_lo = HEAD ? blockIdx.x * a.gsize : blockIdx.x * blockDim.x;
-    const int c_hi = min(a.NO, c_lo + (HEAD ? a.gsize : (int)blockDim.x));
-    const int width = IN == DWN_FROM_CODE ? a.I / a.nbits : a.I;
-    extern __shared__ float staged[];  // [row][width]
-    if constexpr (STAGE) {
-        const float *from = a.x + (size_t)b0 * width;
-        for (int e = tid; e < rows * width; e += blockDim.x) staged[e] = from[e];
-        __syncthreads();
-    }
-    int count[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) count[r] = 0;
-    for (int c0 = c_lo; c0 < c_hi; c0 += blockDim.x) {
-        const bool live = c0 + tid < c_hi;
-        const int c = min(c0 + tid, c_hi - 1);
-        int idx[K];
-#pragma unroll
-        for (int j = 0; j < K; ++j) idx[j] = a.idx32[(size_t)(c / a.O) * K + j];
-        unsigned addr[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) addr[r] = 0;
-        if constexpr (IN == DWN_FROM_PLANES) {
-#pragma unroll
-            for (int j = 0; j < K; ++j) {
-                const unsigned byte = a.planes[((size_t)(b0 >> 6) * a.I + idx[j]) * 8 + ((b0 & 63) >> 3)] >> (b0 & 7);
-#pragma unroll
-                for (int r = 0; r < R; ++r) addr[r] |= ((byte >> r) & 1u) << j;
-            }
-        } else {
-            float limit[K];
-            int col[K];
-#pragma unroll
-            for (int j = 0; j < K; ++j) {
-                col[j] = IN == DWN_FROM_CODE ? (int)((unsigned)idx[j] / (unsigned)a.nbits) : idx[j];
-                limit[j] = IN == DWN_FROM_CODE ? a.thr[idx[j]] : 0.5f;
-            }
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const int first = min(r, rows - 1) * width;
-                const float *row = a.x + (size_t)b0 * width + first;
-#pragma unroll
-                for (int j = 0; j < K; ++j) {
-                    const float v = STAGE ? staged[first + col[j]] : row[col[j]];
-                    addr[r] |= ((IN == DWN_FROM_CODE ? v > limit[j] : v >= limit[j]) ? 1u : 0u) << j;
-                }
-            }
-        }
-        bool bit[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) bit[r] = a.luts[(size_t)c * L + addr[r]] >= 0.5f;
-        if constexpr (HEAD) {
-#pragma unroll
-            for (int r = 0; r < R; ++r) count[r] += __popcll(__ballot(live && bit[r]));
-        } else if (live) {
-            unsigned byte = 0;
-#pragma unroll
-            for (int r = 0; r < R; ++r) byte |= r < rows && bit[r] ? 1u << r : 0u;
-            uint8_t *word = a.planes_out + ((size_t)(b0 >> 6) * a.NO + c) * 8;
-            word[(b0 & 63) >> 3] = (uint8_t)byte;
-            if (blockIdx.y == gridDim.y - 1)  // the rows of the last tile that the batch does not have
-                for (int q = ((b0 & 63) >> 3) + 1; q < 8; ++q) word[q] = 0;
-        }
-    }
-    if constexpr (HEAD) {
-        if ((tid & 63) == 0) {
-#pragma unroll
-            for (int r = 0; r < R; ++r) part[tid >> 6][r] = count[r];
-        }
-        __syncthreads();
-        if (tid < rows) {
-            int sum = 0;
-            for (int w = 0; w < (int)blockDim.x >> 6; ++w) sum += part[w][tid];
-            a.logits[(size_t)(b0 + tid) * a.groups + blockIdx.x] = (float)sum * a.inv_tau;
-        }
-    }
-}
-template <int K>
-static void dwn_launch_eval_rows(const DwnRows &a, hipStream_t s) {
-    const bool head = a.logits != nullptr;
-    const int per_block = head ? a.gsize : a.NO, most = head ? 1024 : 256;
-    const int threads = per_block >= most ? most : (per_block + 63) / 64 * 64;
-    const int R = head && a.B < 8 ? 1 : 8;
-    const dim3 grid(head ? a.groups : dl_ceil_div(a.NO, threads), dl_ceil_div(a.B, R));
-    const size_t lds = a.planes ? 0 : (size_t)R * (a.thr ? a.I / a.nbits : a.I) * sizeof(float);
-    const bool stage = lds > 0 && lds <= 64 * 1024;
-#define DWN_ROWS(IN, STAGE)                                                                                                             \
-    do {                                                                                                                                \
-        if (!head) DL_TIMED("dwn_eval_rows", s, (dwn_eval_rows<K, IN, false, 8, STAGE><<<grid, threads, STAGE ? lds : 0, s>>>(a)));      \
-        else if (R == 8) DL_TIMED("dwn_eval_rows", s, (dwn_eval_rows<K, IN, true, 8, STAGE><<<grid, threads, STAGE ? lds : 0, s>>>(a))); \
-        else DL_TIMED("dwn_eval_rows", s, (dwn_eval_rows<K, IN, true, 1, STAGE><<<grid, threads, STAGE ? lds : 0, s>>>(a)));             \
-    } while (0)
-    if (a.planes) DWN_ROWS(DWN_FROM_PLANES, false);
-    else if (a.thr && stage) DWN_ROWS(DWN_FROM_CODE, true);
-    else if (a.thr) DWN_ROWS(DWN_FROM_CODE, false);
-    else if (stage) DWN_ROWS(DWN_FROM_X, true);
-    else DWN_ROWS(DWN_FROM_X, false);
-#undef DWN_ROWS
-}
-
-// ---------------------------------------------------------------------------------
 // Chained layers: activations between two DWN layers never take their [B, N] fp32 form.
 extern "C" size_t dl_dwn_planes_bytes(int B, int C) { return (B > 0 && C > 0) ? dwn_planes_bytes(B, C) : 256; }
 extern "C" size_t dl_dwn_tiled_bytes(int B, int C) {
@@ -2655,29 +2542,21 @@ extern "C" int dl_dwn_layer_eval_planes_groups(const void *planes_in, const int3
     return dl_launch_status();
 }
 
-// One launch for a layer on few rows: see dwn_eval_rows.
-extern "C" int dl_dwn_layer_eval_rows(const float *x, const float *thr, int nbits, const void *planes_in, const int32_t *idx32,
-                                      const float *luts, void *planes_out, float *logits, int B, int I, int N, int k, int O,
-                                      int groups, float tau, void *stream) {
+// One launch for a layer on few rows (dwn_rows.hip).
+extern "C" int dl_dwn_layer_rows(const float *x, const float *thr, int nbits, const void *planes_in, const int32_t *idx32,
+                                 const float *luts, void *planes_out, float *logits, void *saved, int B, int I, int N, int k, int O,
+                                 int groups, float tau, void *stream) {
     if (!idx32 || !luts || !x == !planes_in || !planes_out == !logits || (thr && !x)) return DL_ERR_NULL;
     int rc = dwn_check(B, I, N, k, O);
     if (rc) return rc;
     if (thr && (nbits <= 0 || I % nbits != 0)) return DL_ERR_SHAPE;
     if (logits && (groups <= 0 || !(tau > 0.0f))) return DL_ERR_SHAPE;
-    if (!dwn_fast(N, k, O) || B > 65535) return DL_ERR_UNSUPPORTED;
+    if (!dwn_fast(N, k, O) || B > 65535 || (x && I > DL_DWN_ROWS_INPUTS)) return DL_ERR_UNSUPPORTED;
     const int F = N * O;
     if (logits && dwn_group_slots(dwn_group_size(F, groups)) > DWN_GS_SLOTS) return DL_ERR_UNSUPPORTED;  // as with a workspace
-    const DwnRows a = {x, thr, (const uint8_t *)planes_in, idx32, luts, (uint8_t *)planes_out, logits, B, I, F, O, nbits,
-                       groups, logits ? dwn_group_size(F, groups) : 1, logits ? 1.0f / tau : 0.0f};
-    hipStream_t s = (hipStream_t)stream;
-    switch (k) {
-        case 1: dwn_launch_eval_rows<1>(a, s); break;
-        case 2: dwn_launch_eval_rows<2>(a, s); break;
-        case 3: dwn_launch_eval_rows<3>(a, s); break;
-        case 4: dwn_launch_eval_rows<4>(a, s); break;
-        case 5: dwn_launch_eval_rows<5>(a, s); break;
-        default: dwn_launch_eval_rows<6>(a, s); break;
-    }
+    const DwnRows a = {x, thr, (const uint8_t *)planes_in, idx32, luts, nullptr, (uint8_t *)planes_out, logits, (uint8_t *)saved,
+                       B, I, N, O, nbits, groups, logits ? dwn_group_size(F, groups) : 1, logits ? 1.0f / tau : 0.0f};
+    dwn_launch_rows(k, a, (hipStream_t)stream);
     return dl_launch_status();
 }
 

@@ -31,7 +31,7 @@ namespace {
     X(dl_soft_map_saved_bytes) X(dl_soft_map_workspace_bytes) X(dl_soft_map_fwd) X(dl_soft_map_bwd) X(dl_unfold_rows)    \
     X(dl_unfold_flip) X(dl_fold) X(dl_dwn_planes_bytes) X(dl_dwn_tiled_bytes) X(dl_dwn_pack_planes)                      \
     X(dl_thermometer_planes) X(dl_dwn_groups_workspace_bytes) X(dl_dwn_layer_fwd_planes)                                 \
-    X(dl_dwn_layer_fwd_planes_groups) X(dl_dwn_layer_eval_planes) X(dl_dwn_layer_eval_planes_groups) X(dl_dwn_layer_eval_rows) \
+    X(dl_dwn_layer_fwd_planes_groups) X(dl_dwn_layer_eval_planes) X(dl_dwn_layer_eval_planes_groups) X(dl_dwn_layer_rows) \
     X(dl_dwn_layer_bwd_groups) X(dl_dwn_layer_bwd_tiled) X(dl_dwn_chain_fusable) X(dl_dwn_bwd_fused_workspace_bytes)     \
     X(dl_dwn_layer_bwd_chain_fused) X(dl_dwn_chain_first_fusable) X(dl_dwn_bwd_first_workspace_bytes)                    \
     X(dl_dwn_layer_bwd_chain_first) X(dl_cross_entropy_workspace_bytes) X(dl_cross_entropy) X(dl_adam_step)
@@ -388,6 +388,28 @@ Tensor first_planes(const Tensor &x, const Tensor &thresholds, const Tensor &fli
     width *= nbits;
     return planes;
 }
+// Up to so many rows, and rows times columns of all layers, a chain goes a launch per layer (dl_dwn_layer_rows), which saves the
+// first layer's planes and the last one's partial sums.  On the device, us, planes / rows (nodes of six inputs): inference, 2000 nodes B = 1
+// 11.4 / 3.5, 768 14.5 / 12.1, 2048 15.7 / 27; 7920 nodes B = 64 21.4 / 6.7, 384 22.5 / 13.3; 4000-2000 B = 512 19.2 / 14.6, 1024 20.0 / 23.3;
+// 8000-4000 B = 256 24.1 / 15.8, 512 24.7 / 25.6; training forward of one layer, 2000 nodes B = 256 12.9 / 8.0, 768 13.6 / 13.3, 1024
+// 13.5 / 15.7; 8000 nodes B = 64 15.5 / 7.6, 384 15.8 / 15.5, 512 15.9 / 21.1.
+constexpr int64_t ROWS_MOST = 768, ROWS_MOST_WORK = 3 << 20;
+bool few_rows(const Tensor &x, const Tensor &thresholds, at::ArrayRef<Tensor> luts, int64_t groups) {
+    if (x.dim() != 2 || x.size(0) > ROWS_MOST || (luts.size() == 1 && !groups)) return false;
+    int64_t columns = 0;
+    for (const Tensor &t : luts) columns += t.dim() == 3 ? t.size(0) * t.size(1) : 0;
+    const int64_t inputs = x.size(1) * (thresholds.defined() && thresholds.dim() == 2 ? thresholds.size(1) : 1);
+    return x.size(0) * columns <= ROWS_MOST_WORK && inputs <= DL_DWN_ROWS_INPUTS;
+}
+// where the first layer reads x itself: its rows and width, and the thresholds of its code (undefined: none)
+Tensor as_it_comes(const Tensor &x, const Tensor &thresholds, int &B, int &width, int &nbits) {
+    B = (int)x.size(0), width = (int)x.size(1);
+    if (!thresholds.defined()) return thresholds;
+    const Tensor thr = code_thresholds(thresholds, width);
+    nbits = (int)thr.size(1);
+    width *= nbits;
+    return thr;
+}
 Dims chain_dims(size_t l, const Plan &p, const Tensor &lut, int B, int width) {
     TORCH_CHECK(lut.dim() == 3 && p.k <= DL_MAX_FAST_K && lut.size(0) == p.N && lut.size(2) == (int64_t)1 << p.k && width == p.I,
                 "layer ", l, ": cannot chain (k=", p.k, ", tables ", lut.sizes(), ", mapping [", p.N, ",", p.k, "] over ", p.I,
@@ -406,9 +428,12 @@ struct DwnStack : torch::autograd::Function<DwnStack> {
             require_device(t);
             luts.push_back(f32(t));
         }
-        int B = 0, width = 0;
+        int B = 0, width = 0, nbits = 1;
         st->encoded = thresholds->defined();
-        Tensor planes = first_planes(x, *thresholds, *flip, *st, B, width), y;
+        Tensor planes, thr, y;
+        const bool rows = !st->patches && few_rows(x, *thresholds, luts, st->groups);
+        if (rows) thr = as_it_comes(x, *thresholds, B, width, nbits);
+        else planes = first_planes(x, *thresholds, *flip, *st, B, width);
         variable_list save(luts.begin(), luts.end());
         for (size_t l = 0; l < luts.size(); ++l) {
             const Plan &p = st->plans[l];
@@ -416,7 +441,14 @@ struct DwnStack : torch::autograd::Function<DwnStack> {
             const bool last = l + 1 == luts.size();
             const Tensor kept = bytes(L.dl_dwn_saved_bytes(DIMS(d)), x);
             Tensor next;
-            if (last && st->groups) {
+            if (rows && (st->groups || !last)) {
+                const bool first = !planes.defined();
+                if (last) y = floats({B, st->groups}, x);
+                else next = bytes(L.dl_dwn_planes_bytes(B, d.N * d.O), x);
+                check(L.dl_dwn_layer_rows(first ? in(x) : nullptr, first ? in(thr) : nullptr, nbits, raw(planes), ints(p.idx),
+                                          in(luts[l]), raw(next), last ? out(y) : nullptr, raw(kept), DIMS(d), (int)st->groups,
+                                          (float)st->tau, stream()));
+            } else if (last && st->groups) {
                 y = floats({B, st->groups}, x);
                 const Tensor ws = bytes(L.dl_dwn_groups_workspace_bytes(B, d.N, d.O, (int)st->groups), x);
                 check(L.dl_dwn_layer_fwd_planes_groups(raw(planes), ints(p.idx), in(luts[l]), out(y), raw(kept), raw(ws), ws.numel(),
@@ -623,11 +655,6 @@ Tensor dwn_stack(const Tensor &x, const std::vector<Tensor> &luts, const std::ve
     const Tensor thr = tensor_of(thresholds), mask = tensor_of(flip);
     return DwnStack::apply(x, at::TensorList(luts), &thr, &mask, st);
 }
-// Up to so many rows, and rows times columns of all layers, a chain goes a launch per layer (dl_dwn_layer_eval_rows).  On the device,
-// us, planes / rows (nodes of six inputs, ten groups): 2000 nodes B = 1 11.3 / 3.1, 768 14.6 / 11.4, 2048 15.7 / 33; 7920 nodes B = 8 20.4 /
-// 6.4, 384 22.5 / 15.6, 768 22.6 / 30.7; 4000-2000 B = 512 19.2 / 17.6, 768 19.6 / 22.7; 8000-4000 B = 256 24.2 / 19.5, 384 24.4 / 24.5.  And two
-// launches and two allocations less on the host.
-constexpr int64_t ROWS_MOST = 768, ROWS_MOST_WORK = 3 << 20;
 Tensor dwn_stack_eval(const Tensor &x_, const Maybe &thresholds, const std::vector<Tensor> &luts_, const std::vector<PlanArgs> &plans,
                       int64_t groups, double tau) {
     at::NoGradGuard no_grad;
@@ -637,20 +664,9 @@ Tensor dwn_stack_eval(const Tensor &x_, const Maybe &thresholds, const std::vect
     const size_t n = luts_.size();
     int B = 0, width = 0, nbits = 1;
     Tensor planes, thr, y;
-    // few rows: a launch per layer, the first reads x as it comes
-    int64_t columns = 0;
-    for (const Tensor &t : luts_) columns += t.dim() == 3 ? t.size(0) * t.size(1) : 0;
-    const bool rows = x.dim() == 2 && x.size(0) <= ROWS_MOST && x.size(0) * columns <= ROWS_MOST_WORK && (n > 1 || groups);
-    if (rows) {
-        B = (int)x.size(0), width = (int)x.size(1);
-        if (thresholds) {
-            thr = code_thresholds(*thresholds, width);
-            nbits = (int)thr.size(1);
-            width *= nbits;
-        }
-    } else {
-        planes = first_planes(x, tensor_of(thresholds), Tensor(), *st, B, width);
-    }
+    const bool rows = few_rows(x, tensor_of(thresholds), luts_, groups);
+    if (rows) thr = as_it_comes(x, tensor_of(thresholds), B, width, nbits);
+    else planes = first_planes(x, tensor_of(thresholds), Tensor(), *st, B, width);
     for (size_t l = 0; l < n; ++l) {
         require_device(luts_[l]);
         const Tensor lut = f32(luts_[l]);
@@ -663,8 +679,8 @@ Tensor dwn_stack_eval(const Tensor &x_, const Maybe &thresholds, const std::vect
         else next = bytes(L.dl_dwn_planes_bytes(B, d.N * d.O), x);
         if (rows && (head || !last)) {
             const bool first = !planes.defined();
-            check(L.dl_dwn_layer_eval_rows(first ? in(x) : nullptr, first ? in(thr) : nullptr, nbits, raw(planes), ints(p.idx), in(lut),
-                                           raw(next), head ? out(y) : nullptr, DIMS(d), (int)groups, (float)tau, stream()));
+            check(L.dl_dwn_layer_rows(first ? in(x) : nullptr, first ? in(thr) : nullptr, nbits, raw(planes), ints(p.idx), in(lut),
+                                           raw(next), head ? out(y) : nullptr, nullptr, DIMS(d), (int)groups, (float)tau, stream()));
         } else if (head) {
             const Tensor ws = bytes(L.dl_dwn_groups_workspace_bytes(B, d.N, d.O, (int)groups), x);
             check(L.dl_dwn_layer_eval_planes_groups(raw(planes), ints(p.idx), in(lut), out(y), raw(ws), ws.numel(), DIMS(d), (int)groups,

@@ -236,12 +236,14 @@ int dl_dwn_layer_eval_planes(const void *planes_in, const int32_t *idx32, const 
 int dl_dwn_layer_eval_planes_groups(const void *planes_in, const int32_t *idx32, const float *luts, float *logits,
                                     void *ws, size_t ws_bytes, int B, int I, int N, int k, int O,
                                     int groups, float tau, void *stream);
-/* The same on few rows (B <= 65535; meant for a few hundred), one launch that reads its input as it comes: planes_in, or x - the raw
- * features [B, I/nbits] of a thermometer code with thresholds thr [I/nbits, nbits], or with thr null the 0/1 values [B, I].
- * Exactly one of x and planes_in, and of planes_out and logits [B, groups], is given. */
-int dl_dwn_layer_eval_rows(const float *x, const float *thr, int nbits, const void *planes_in, const int32_t *idx32,
-                           const float *luts, void *planes_out, float *logits, int B, int I, int N, int k, int O,
-                           int groups, float tau, void *stream);
+/* A layer of a chain on few rows (B <= 65535; meant for a few hundred), one launch that reads its input as it comes: planes_in, or
+ * x - the raw features [B, I/nbits] of a thermometer code with thresholds thr [I/nbits, nbits], or with thr null the values
+ * [B, I] themselves (I <= DL_DWN_ROWS_INPUTS: a byte of LDS each).  Exactly one of x and planes_in, and of planes_out and logits [B, groups], is given.  saved
+ * (dl_dwn_saved_bytes): training, as dl_dwn_layer_fwd_planes[_groups]; null: inference, as dl_dwn_layer_eval_planes[_groups]. */
+#define DL_DWN_ROWS_INPUTS 64512
+int dl_dwn_layer_rows(const float *x, const float *thr, int nbits, const void *planes_in, const int32_t *idx32,
+                      const float *luts, void *planes_out, float *logits, void *saved, int B, int I, int N, int k, int O,
+                      int groups, float tau, void *stream);
 /* Eval forward (DWNNode.forward_eval, dwn_node.py:457-483): addr = floor(sum_j x_j 2^j)
  * with no thresholding of x (clamped to the table), y = (luts[n,d,addr] >= 0.5) as 0/1. */
 int dl_dwn_layer_eval(const float *x, const int32_t *idx32, const float *luts, float *y,

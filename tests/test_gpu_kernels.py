@@ -596,7 +596,7 @@ def test_gather_through_the_lds(shape):
 @pytest.mark.parametrize("width,N,k,O,groups", [(40, 192, 6, 1, 3),    # groups of one wavefront
                                                 (33, 65, 1, 1, 1),     # a group one column longer
                                                 (96, 330, 4, 2, 9),    # groups of 74 columns, the last of 68, two outputs
-                                                (2100, 1300, 5, 1, 1)])  # more than a block's threads; rows too wide for the LDS
+                                                (2100, 1300, 5, 1, 1)])  # more columns than a block's threads
 def test_eval_of_few_rows(B, source, width, N, k, O, groups):
     """One launch per layer against the bit-plane kernels: the same bits, as planes and as group sums; and the group sums from
     planes against the sums of the layer's output.  Sums of zeros and ones: exact."""
@@ -625,16 +625,54 @@ def test_eval_of_few_rows(B, source, width, N, k, O, groups):
     want, got = (torch.full((max(used, 256),), 7, dtype=torch.uint8, device=DEV) for _ in range(2))
     nat.check(lib.dl_dwn_layer_eval_planes(planes.data_ptr(), idx.data_ptr(), luts.data_ptr(), y.data_ptr(), want.data_ptr(), *dims, nat.stream()))
     given = (None, None, 1, planes.data_ptr()) if source == "planes" else (x.data_ptr(), thr.data_ptr() if source == "code" else None, nbits, None)
-    nat.check(lib.dl_dwn_layer_eval_rows(*given, idx.data_ptr(), luts.data_ptr(), got.data_ptr(), None, *dims, 0, 1.0, nat.stream()))
+    nat.check(lib.dl_dwn_layer_rows(*given, idx.data_ptr(), luts.data_ptr(), got.data_ptr(), None, None, *dims, 0, 1.0, nat.stream()))
     assert torch.equal(want[:used], got[:used])
     gs = -(-F // groups)
     sums = torch.stack([y[:, q * gs:(q + 1) * gs].sum(1) for q in range(groups)], 1) * (1.0 / 0.5)
     logits = torch.full((2, B, groups), -1.0, device=DEV)
-    nat.check(lib.dl_dwn_layer_eval_rows(*given, idx.data_ptr(), luts.data_ptr(), None, logits[0].data_ptr(), *dims, groups, 0.5, nat.stream()))
+    nat.check(lib.dl_dwn_layer_rows(*given, idx.data_ptr(), luts.data_ptr(), None, logits[0].data_ptr(), None, *dims, groups, 0.5, nat.stream()))
     ws = torch.empty(lib.dl_dwn_groups_workspace_bytes(B, N, O, groups), dtype=torch.uint8, device=DEV)
     nat.check(lib.dl_dwn_layer_eval_planes_groups(planes.data_ptr(), idx.data_ptr(), luts.data_ptr(), logits[1].data_ptr(), ws.data_ptr(),
                                                   ws.numel(), *dims, groups, 0.5, nat.stream()))
     assert torch.equal(logits[0], sums) and torch.equal(logits[1], sums)
+    # the training forward: planes and addresses the same (rows that the batch does not have are zeros); sums of up to 1300 values
+    # of size 1 in another order
+    saved = torch.full((2, lib.dl_dwn_saved_bytes(*dims)), 7, dtype=torch.uint8, device=DEV)
+    nat.check(lib.dl_dwn_layer_fwd_planes(planes.data_ptr(), idx.data_ptr(), luts.data_ptr(), None, want.data_ptr(), saved[0].data_ptr(), *dims, nat.stream()))
+    nat.check(lib.dl_dwn_layer_rows(*given, idx.data_ptr(), luts.data_ptr(), got.data_ptr(), None, saved[1].data_ptr(), *dims, 0, 1.0, nat.stream()))
+    held = (B + 63) // 64 * N * 64
+    assert torch.equal(want[:used], got[:used]) and torch.equal(saved[0][:held], saved[1][:held])
+    nat.check(lib.dl_dwn_layer_fwd_planes_groups(planes.data_ptr(), idx.data_ptr(), luts.data_ptr(), logits[0].data_ptr(), saved[0].data_ptr(),
+                                                 ws.data_ptr(), ws.numel(), *dims, groups, 0.5, nat.stream()))
+    saved[1] = 7
+    nat.check(lib.dl_dwn_layer_rows(*given, idx.data_ptr(), luts.data_ptr(), None, logits[1].data_ptr(), saved[1].data_ptr(), *dims, groups, 0.5, nat.stream()))
+    assert torch.equal(saved[0][:held], saved[1][:held])
+    torch.testing.assert_close(logits[0], logits[1], rtol=1e-5, atol=1e-4)
+
+
+@pytest.mark.parametrize("B", [1, 8, 65, 130])
+@pytest.mark.parametrize("I,N,k,O", [(64, 64, 6, 1), (100, 33, 3, 2), (8192, 1100, 4, 1), (8193, 40, 5, 1)])  # the last: planes
+def test_layer_forward_of_few_rows(B, I, N, k, O):
+    """A single layer on few rows, one launch: output and addresses those of the bit-plane kernels."""
+    from difflut_amd import _native as nat
+
+    lib = nat.lib()
+    g = torch.Generator("cuda").manual_seed(B + I)
+    idx = torch.randint(0, I, (N, k), device=DEV, generator=g, dtype=torch.int32)
+    luts = torch.randn(N, O, 1 << k, device=DEV, generator=g)
+    x = torch.rand(B, I, device=DEV, generator=g)
+    x[0, :4] = torch.tensor([0.5, float("nan"), float("inf"), -0.0], device=DEV)
+    dims = (B, I, N, k, O)
+    planes = torch.empty(lib.dl_dwn_planes_bytes(B, I), dtype=torch.uint8, device=DEV)
+    y = torch.full((2, B, N * O), -7.0, device=DEV)
+    saved = torch.full((2, lib.dl_dwn_saved_bytes(*dims)), 7, dtype=torch.uint8, device=DEV)
+    nat.check(lib.dl_dwn_pack_planes(x.data_ptr(), planes.data_ptr(), B, I, nat.stream()))
+    nat.check(lib.dl_dwn_layer_fwd_planes(planes.data_ptr(), idx.data_ptr(), luts.data_ptr(), y[0].data_ptr(), None, saved[0].data_ptr(), *dims, nat.stream()))
+    ws = torch.empty(lib.dl_dwn_fwd_workspace_bytes(*dims), dtype=torch.uint8, device=DEV)
+    nat.check(lib.dl_dwn_layer_fwd(x.data_ptr(), idx.data_ptr(), luts.data_ptr(), y[1].data_ptr(), saved[1].data_ptr(), ws.data_ptr(), ws.numel(),
+                                   *dims, nat.stream()))
+    held = (B + 63) // 64 * N * 64
+    assert torch.equal(y[0], y[1]) and torch.equal(saved[0][:held], saved[1][:held])
 
 
 # ------------------------------------------------------------------------------ probabilistic
