@@ -1280,6 +1280,27 @@ def test_cross_entropy_against_torch(shape):
         np.testing.assert_allclose(l2.item(), ref.item(), rtol=1e-6)
 
 
+@pytest.mark.parametrize("B,C", [(64, 2), (65, 3), (1024, 10), (1025, 10), (70000, 2)])
+def test_cross_entropy_blocks(B, C):
+    """One block up to 1024 rows, sums of blocks beyond; the last has more blocks than the kernel that adds them has threads.  A
+    row's gradient is (p - 1) / B or p / B, p within 2e-7 (an exponential, a sum of C, a reciprocal); the loss a sum of B values of
+    size up to 20 by halves: rtol 2e-6."""
+    from difflut_amd.utils import cross_entropy
+
+    g = torch.Generator("cuda").manual_seed(B + C)
+    z = torch.randn(B, C, device=DEV, generator=g) * 5
+    y = torch.randint(0, C, (B,), device=DEV, generator=g)
+    zt = z.clone().requires_grad_()
+    loss = cross_entropy(zt, y)
+    loss.backward()
+    zr = z.double().requires_grad_()
+    want = torch.nn.functional.cross_entropy(zr, y)
+    want.backward()
+    torch.testing.assert_close(loss.double(), want.detach(), rtol=2e-6, atol=0.0)
+    torch.testing.assert_close(zt.grad.double(), zr.grad, rtol=1e-5, atol=2e-7 / B)
+
+
+
 # ------------------------------------------------------------------------------ error paths
 def test_argument_errors_are_reported_not_launched():
     from difflut_amd import _native as nat
