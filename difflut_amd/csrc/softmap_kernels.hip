@@ -558,18 +558,18 @@ __device__ __forceinline__ void softmap_stage_barrier() {
 // signs as well; on the fp32 matrix cores 0.62e-6.  It costs 675 -> 725 us there.
 //
 // One product kernel, three operand modes.  At 512 x 3136 x 48000 (1.54e11 flop a product; before: 128 x 128 tiles staged
-// through registers) forward / gx / gW take 182 / 160 / 298 us with bf16 operands (before 236 / 453 / 365) and 660 / 725 /
-// 840 us with three planes (before, on the fp32 matrix cores, 1318 / 1494 / 1347): 0.85-0.96 and 1.27-1.40 PFLOP/s of bf16
+// through registers) forward / gx / gW take 161 / 151 / 264 us with bf16 operands (before 236 / 453 / 365) and 660 / 725 /
+// 840 us with three planes (before, on the fp32 matrix cores, 1318 / 1494 / 1347): 1.0 and 1.27-1.40 PFLOP/s of bf16
 // products, the latter what the matrix cores hold under power; gW adds 602 MB of stores and 301 (602) MB of reads.
 // MODE 0: forward   rows=b cols=o red=i   A = x    B = E (turned)   out = C rs[o]
 // MODE 1: gx        rows=b cols=i red=o   A = gs   B = E
 // MODE 2: gW        rows=o cols=i red=b   A = gm   B = x            out = rs E (C - r) / tau
 // Block = 256 threads = 2 x 2 wavefronts, tile 64 FA x 128, a wavefront FA x 2 MFMA tiles of 32 x 32.  FA = 4 (256 rows):
 // per MFMA a block pulls 24 KB per 32 reduction steps (NP = 1), 48 bytes per clock and CU at the matrix peak where
-// 128 x 128 tiles need 64, all that an L2 channel delivers.  Two blocks share a CU (accumulators 128 registers, 72 KB of LDS
+// 128 x 128 tiles need 64, all that an L2 channel delivers.  Two or three blocks share a CU (accumulators 128 registers, 72 or 48 KB of LDS
 // each), so one block's MFMAs run under the other's barriers and stores.  Stages are KC deep, NBUF of them in the LDS.
 // Pairs (NP = 2): 128 x 128 tiles, because hi*hi and the rest have accumulators of their own (64 registers each) and the loop has
-// no vector arithmetic but the sign below; three blocks share a CU for gW, whose epilogue is two thirds memory (575 us; 704 with
+// no vector arithmetic but the sign below; three blocks share a CU for gW, whose epilogue is two thirds memory (575 us before its reads were asked for ahead, 540 so; 704 with
 // two).  Forward and gx add the sums of SM_PAIR_TURN stages to running ones, signs turned from group to group for the reason
 // given above, and have two blocks per CU.  The same sizes, forward / gx / gW: 503 / 473 / 575 us (planes 703 / 786 / 866).  Bound by power: the matrix cores are busy half of the time at 1.8 GHz.  256 x 128 tiles with one accumulator, the
 // rest's sum scaled and added by every stage: 514 / 560 / 668.  gx in
@@ -577,8 +577,15 @@ __device__ __forceinline__ void softmap_stage_barrier() {
 // NPB = 2 with NP = 3 (gx): gs in planes, E in pairs, whose planes - times 2^10, which makes their scale the planes' - are made on
 // the way out of the LDS; for gradients that span too much where E does not.  The backward at 512 x 3136 x 48000 with such
 // gradients 1651 us, 1782 with E in planes throughout.
+// Stages in the LDS, and blocks per CU that the registers have to allow.  bf16 operands in 256 x 128 tiles: the forward and gx with two
+// stages and three blocks (161 / 149 us; three stages and two blocks 178 / 154), gW, whose epilogue is most of its time, with three
+// stages and two blocks (261; two and three 288).
+static constexpr int softmap_stages(int mode, int np, int fa) { return fa == 4 && (np == 3 || (np == 1 && mode != 2)) ? 2 : 3; }
+static constexpr int softmap_blocks(int mode, int np, int fa) {
+    return (mode == 2 && np == 2) || (mode != 2 && np == 1 && fa == 4) ? 3 : 2;
+}
 template <int MODE, int NP, int FA, int NPB>
-__global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
+__global__ __launch_bounds__(256, softmap_blocks(MODE, NP, FA)) void softmap_mfma(SoftmapArgs g) {
     extern __shared__ __align__(16) char lds[];
     constexpr bool FROM_PAIRS = NP == 3 && NPB == 2;
     static_assert(NPB == NP || (FROM_PAIRS && MODE == 1), "only gx mixes planes and pairs");
@@ -589,7 +596,7 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
     }
     constexpr int TR = 64 * FA, TC = SM_TC;
     constexpr int KC = NP == 1 ? 32 : SM_GX_STAGE, KB = KC / 8;
-    constexpr int NBUF = NP == 3 && FA == 4 ? 2 : 3, AHEAD = NBUF - 1;
+    constexpr int NBUF = softmap_stages(MODE, NP, FA), AHEAD = NBUF - 1;
     constexpr int A_BYTES = NP * TR * KC * 2, STAGE = (NP * TR + NPB * TC) * KC * 2;
     constexpr bool BY_STAGE = NP == 3 && MODE == 1;
     static_assert(NP != 2 || FA == 2, "pairs keep two sums per output");
@@ -756,6 +763,47 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
 #pragma unroll
     for (int s = 0; s < AHEAD; ++s)
         if (s < nst) issue(s, s);
+    // gW, of the tile's rows, for the epilogue and behind the stages in the LDS: r (its parts added in order), for E rebuilt from W the
+    // maximum, rs / tau, and the pairs' shift.  Read while the first stages come, eight parts at a time: one after the other, and at the
+    // end of the block, they were eight trips to memory that nothing ran beside.
+    float *rr = reinterpret_cast<float *>(lds + NBUF * STAGE);
+    if (MODE == 2 && tid < TR) {
+        float t = 0.0f;
+        for (int q = 0; q < g.parts; q += 8) {
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = g.dots[(size_t)min(q + u, g.parts - 1) * g.dot_ld + r0 + tid];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) t = q + u < g.parts ? t + v[u] : t;
+        }
+        rr[tid] = t;
+        rr[TR + tid] = g.mx[r0 + tid];
+        rr[2 * TR + tid] = g.rs[r0 + tid] * g.inv_tau;
+        if (NP == 2) rr[3 * TR + tid] = __int_as_float(-(softmap_pair_shift(g.range->x_largest) + softmap_pair_shift(g.row_max[r0 + tid])));
+    }
+    // what the epilogue reads of E or W for 32 rows of the wavefront's tile is asked for before the rows ahead of them are stored, E's first
+    // rows before the last stage: with the parts above, gW 316 -> 264 us (bf16 operands), 575 -> 540 (pairs)
+    const int rrow = lane >> 4, c4 = (lane & 15) * 4, col4 = c0 + wn + c4;
+    const bool vec = g.C % 4 == 0 && g.vec_out;
+    uint2 e[2][NP == 1 ? 8 : 1];
+    floatx4 w4[NP != 1 ? 8 : 1];
+    auto ask = [&](int i, int at) __attribute__((always_inline)) {
+        const int row0 = r0 + wm + i * 32;
+        if (NP == 1) {  // E as units of 8 rows: half a unit is this lane's four rows of a column
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    e[at][NP == 1 ? j * 4 + q : 0] = *reinterpret_cast<const uint2 *>(
+                        g.E + ((size_t)((row0 >> 3) + q) * g.lde + c0 + wn + j * 32 + l32) * SM_UNIT + kh * 8);
+        } else if (vec) {
+#pragma unroll
+            for (int it = 0; it < 8; ++it) {
+                const int row = row0 + it * 4 + rrow;
+                if (row < g.R && col4 < g.C) w4[NP != 1 ? it : 0] = *reinterpret_cast<const floatx4 *>(g.W + (size_t)row * g.C + col4);
+            }
+        }
+    };
     int buf = 0, nbuf = AHEAD % NBUF;
     unsigned turn = 0;  // pairs: sign of the group's sums
     auto add_group = [&]() __attribute__((always_inline)) {
@@ -774,6 +822,7 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
         if (s + AHEAD <= nst) softmap_stage_barrier<(NA + NB) * (AHEAD - 1)>();
         else softmap_stage_barrier<0>();
         if (s + AHEAD < nst) issue(s + AHEAD, nbuf);
+        if (MODE == 2 && NP == 1 && s + 1 == nst) ask(0, 0);
         if (GROUPS && s % SM_PAIR_TURN == 0 && s > 0) {
             add_group();
             turn ^= 0x80008000u;
@@ -818,36 +867,16 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
                 }
         }
     } else {
-        // of the tile's rows: r (its parts added in order), for E rebuilt from W the maximum, and rs / tau
-        float *rr = reinterpret_cast<float *>(lds);
-        softmap_stage_barrier<0>();
-        if (tid < TR) {
-            float t = 0.0f;
-            for (int q = 0; q < g.parts; ++q) t += g.dots[(size_t)q * g.dot_ld + r0 + tid];
-            rr[tid] = t;
-            rr[TR + tid] = g.mx[r0 + tid];
-            rr[2 * TR + tid] = g.rs[r0 + tid] * g.inv_tau;
-            if (NP == 2) rr[3 * TR + tid] = __int_as_float(-(shift + softmap_pair_shift(g.row_max[r0 + tid])));
-        }
-        __syncthreads();
+        softmap_stage_barrier<63>();  // (the stages' reads are done; what the epilogue has asked for may be on its way)
         // 32 rows x 64 columns at a time go through the wavefront's own corner of the LDS, so that a lane owns four consecutive
         // columns of a row: 16-byte stores in runs of 256 bytes
         constexpr int TS = 68;  // floats per staged row: 64 + 4 keeps 16-byte alignment
-        float *stg = rr + 4 * TR + wave * (32 * TS);
-        const int rrow = lane >> 4, c4 = (lane & 15) * 4, col4 = c0 + wn + c4;
-        const bool vec = C % 4 == 0 && g.vec_out;
+        float *stg = reinterpret_cast<float *>(lds) + wave * (32 * TS);
 #pragma unroll
         for (int i = 0; i < FA; ++i) {
             const int lr0 = wm + i * 32, row0 = r0 + lr0;
-            uint2 e[2][4];
-            if (NP == 1) {  // E as units of 8 rows: half a unit is this lane's four rows of a column
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        e[j][q] = *reinterpret_cast<const uint2 *>(
-                            g.E + ((size_t)((row0 >> 3) + q) * g.lde + c0 + wn + j * 32 + l32) * SM_UNIT + kh * 8);
-            }
+            if (NP != 1) ask(i, 0);  // (not earlier: the registers are the sums')
+            else if (i + 1 < FA) ask(i + 1, (i + 1) & 1);
 #pragma unroll
             for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -863,8 +892,9 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
                     o[0] -= rv.x; o[1] -= rv.y; o[2] -= rv.z; o[3] -= rv.w;
                     if (NP == 1) {
                         const float4 fv = *reinterpret_cast<const float4 *>(rr + 2 * TR + lr0 + 8 * q + 4 * kh);
-                        o[0] *= softmap_lo(e[j][q].x) * fv.x; o[1] *= softmap_hi(e[j][q].x) * fv.y;
-                        o[2] *= softmap_lo(e[j][q].y) * fv.z; o[3] *= softmap_hi(e[j][q].y) * fv.w;
+                        const uint2 eq = e[i & 1][NP == 1 ? j * 4 + q : 0];
+                        o[0] *= softmap_lo(eq.x) * fv.x; o[1] *= softmap_hi(eq.x) * fv.y;
+                        o[2] *= softmap_lo(eq.y) * fv.z; o[3] *= softmap_hi(eq.y) * fv.w;
                     }
 #pragma unroll
                     for (int n = 0; n < 4; ++n) stg[(8 * q + 4 * kh + n) * TS + j * 32 + l32] = o[n];
@@ -879,7 +909,7 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
                 if (vec) {
                     if (row < R && col4 < C) {
                         if (NP != 1) {
-                            const float4 w = *reinterpret_cast<const float4 *>(g.W + at);
+                            const floatx4 w = w4[NP != 1 ? it : 0];
                             const float mx = rr[TR + lr0 + lr], f = rr[2 * TR + lr0 + lr];
                             o.x *= softmap_e(w.x, mx, g.scale) * f; o.y *= softmap_e(w.y, mx, g.scale) * f;
                             o.z *= softmap_e(w.z, mx, g.scale) * f; o.w *= softmap_e(w.w, mx, g.scale) * f;
@@ -902,8 +932,8 @@ __global__ __launch_bounds__(256, 2) void softmap_mfma(SoftmapArgs g) {
 
 template <int MODE, int NP, int FA, int NPB = NP>
 static void softmap_launch(const SoftmapArgs &g, hipStream_t s) {
-    constexpr int KC = NP == 1 ? 32 : 16, NBUF = NP == 3 && FA == 4 ? 2 : 3;
-    constexpr int lds_bytes = NBUF * (NP * 64 * FA + NPB * SM_TC) * KC * 2;
+    constexpr int KC = NP == 1 ? 32 : 16, NBUF = softmap_stages(MODE, NP, FA);
+    constexpr int lds_bytes = NBUF * (NP * 64 * FA + NPB * SM_TC) * KC * 2 + (MODE == 2 ? 4 * 64 * FA * 4 : 0);
     if (lds_bytes > 65536)
         (void)hipFuncSetAttribute(reinterpret_cast<const void *>(&softmap_mfma<MODE, NP, FA, NPB>),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
