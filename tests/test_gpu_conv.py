@@ -99,6 +99,22 @@ def test_unfold_rows_planes_and_fold(case):
     assert torch.equal(gx, xt.grad)  # same terms in the same order
 
 
+@pytest.mark.parametrize("case", [
+    ((3, 2, 30, 60), (3, 3, 1, 1, 0, 2)),    # a padded row of 64 bits
+    ((1, 1, 70, 64), (1, 1, 1, 1, 0, 0)),    # lines of 64 positions
+    ((2, 1, 8, 66), (3, 3, 1, 1, 0, 0)),     # rows too long for bits
+    ((2, 3, 9, 63), (2, 5, 1, 1, 1, 0)),     # lines that cross tiles everywhere
+    ((300, 1, 3, 3), (3, 3, 1, 1, 1, 1)),    # several images to a tile
+    ((40, 1, 5, 5), (5, 5, 1, 1, 2, 2)),
+    ((2, 200, 16, 16), (3, 3, 1, 1, 1, 1)),  # an image of 800 words: fewer tiles to a block
+    ((1, 300, 32, 32), (1, 1, 1, 1, 0, 0)),  # of 4800: not by bits
+    ((2, 4, 20, 20), (4, 4, 1, 1, 0, 0)),    # patches of a width without a fold of its own
+])
+def test_unfold_by_bits_and_fold_by_lines(case):
+    """The edges of the stride-1 forms."""
+    test_unfold_rows_planes_and_fold(case)
+
+
 def test_unfold_rejects_bad_geometry():
     from difflut_amd import ops
     with pytest.raises(RuntimeError):
