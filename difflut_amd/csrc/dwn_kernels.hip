@@ -35,14 +35,6 @@
 
 typedef unsigned long long u64;
 
-// addr <- 2*addr + (bit `lane` of mask): the 64-bit scalar is used directly as a per-lane carry-in.
-__device__ __forceinline__ unsigned dwn_shift_in(unsigned addr, u64 mask) {
-    unsigned out;
-    u64 carry_out;
-    asm("v_addc_co_u32_e64 %0, %1, %2, %2, %3" : "=v"(out), "=s"(carry_out) : "v"(addr), "s"(mask));
-    return out;
-}
-
 // entry `a` of a table kept 64 entries to a register, one per lane
 template <int NR>
 __device__ __forceinline__ float dwn_table_read(const float (&entry)[NR], unsigned a) {
@@ -122,12 +114,14 @@ __global__ void dwn_set_flag(int *flag, int value) {
 
 // ---------------------------------------------------------------------------------
 // lookup_fwd: one block per (128-column tile, 64-row batch tile), 512 threads = 8 wavefronts,
-// lane = batch row, column = node*O + output.  A wavefront owns 16 consecutive columns.  Their
-// k*16 input indices are fetched once (one per lane) and handed out with readlane; the bit-plane
-// word of (tile, input) is wave-uniform, so it comes through a scalar load and is used directly
-// as a lane mask: one add-with-carry per input shifts the lane's bit into its address
-// (addr <- 2*addr + bit), one bpermute per column reads the table entry.  Columns are taken four
-// at a time so that the 4*k scalar loads of a group are in flight together.
+// lane = batch row, column = node*O + output.  A wavefront owns 16 consecutive columns.  The k*16 plane words of
+// their inputs are fetched one per lane and laid out in the LDS by halves, rows 0-31 and 32-63, so that a lane reads the
+// half with its row four words at a time (two addresses per instruction, no conflicts) and takes its bit out of each:
+// two vector instructions per input; one bpermute per column reads the table entry.  Columns are taken four
+// at a time.
+// Before, a plane word came through a scalar load whose offset a readlane had made: the scalar unit, one for four SIMDs, was
+// 70 % busy with 27 instructions per column.  4096 rows, 16384 -> 8192 nodes of six inputs: 53 -> 43 us (178 MB, 4.1 TB/s), under a
+// hybrid layer 66 -> 49.
 #define DWN_TC 128
 #define DWN_FW 8                      // wavefronts per block
 #define DWN_WC (DWN_TC / DWN_FW)      // columns per wavefront
@@ -141,22 +135,24 @@ __global__ void dwn_set_flag(int *flag, int value) {
 // EVAL: the inference form (DWNNode.forward_eval on inputs that are exactly 0 or 1, where its address
 // floor(sum x_j 2^j) is the thresholded one): the output is (table entry >= 0.5) as 0/1, nothing is saved
 // for a backward.
-template <int K, bool O1, bool CHAIN = false, bool GSUM = false, bool EVAL = false>
-__global__ __launch_bounds__(64 * DWN_FW) void dwn_lookup_fwd(const u64 *__restrict__ planes, const int *__restrict__ idx32,
+template <int K, bool O1, bool CHAIN = false, bool GSUM = false, bool EVAL = false, int FW = DWN_FW>
+__global__ __launch_bounds__(64 * FW) void dwn_lookup_fwd(const u64 *__restrict__ planes, const int *__restrict__ idx32,
                                                                const float *__restrict__ luts, float *__restrict__ y,
                                                                uint8_t *__restrict__ addrT, u64 *__restrict__ planes_out,
                                                                int B, int I, int N, int O, int BT, int gsize = 1,
                                                                int slots = 1, const int *__restrict__ run_if_set = nullptr) {
     if (EVAL && run_if_set && *run_if_set == 0) return;  // the inputs were not all 0/1: the generic kernel answers
-    __shared__ float tile[DWN_TC][65];  // [column][row]
-    __shared__ u64 plane_tile[CHAIN ? DWN_TC : 1];  // thresholded outputs of the tile's columns, one bit per row
-    __shared__ float gpart[GSUM ? DWN_FW : 1][GSUM ? DWN_GS_SLOTS : 1][64];  // [wavefront][slot][row]
+    constexpr int TC = FW * DWN_WC;
+    __shared__ float tile[TC][65];  // [column][row]
+    __shared__ __align__(16) unsigned words[FW][2][DWN_WC * K];  // [wavefront][rows 0-31, 32-63][slot]
+    __shared__ u64 plane_tile[CHAIN ? TC : 1];  // thresholded outputs of the tile's columns, one bit per row
+    __shared__ float gpart[GSUM ? FW : 1][GSUM ? DWN_GS_SLOTS : 1][64];  // [wavefront][slot][row]
     constexpr int L = 1 << K;
     constexpr int NIDX = (DWN_WC * K + 63) / 64;  // index registers per lane
     const int NO = N * O;
     int ctile, t;
-    if (!dl_xcd_map((NO + DWN_TC - 1) / DWN_TC, BT, ctile, t)) return;
-    const int c0 = ctile * DWN_TC;
+    if (!dl_xcd_map((NO + TC - 1) / TC, BT, ctile, t)) return;
+    const int c0 = ctile * TC;
     const int lane = threadIdx.x & 63;
     const int wave = dl_uniform(threadIdx.x >> 6);
     const u64 *pl = planes + (size_t)t * I;
@@ -165,16 +161,30 @@ __global__ __launch_bounds__(64 * DWN_FW) void dwn_lookup_fwd(const u64 *__restr
         __builtin_amdgcn_make_buffer_rsrc((void *)(addrT + (size_t)t * N * 64), 0, N * 64, 0x00020000);
     const int lane4s = (lane & (L - 1)) * 4;
     constexpr int NR = L > 64 ? L / 64 : 1;  // registers of a table
-    const int cend = min(DWN_TC, NO - c0);
+    const int cend = min(TC, NO - c0);
     const int wbeg = wave * DWN_WC;
     // slot s = (column within my 16) * K + j  ->  lane s % 64 of register s / 64
-    int myidx[NIDX];
+    {
+        u64 word[NIDX];
 #pragma unroll
-    for (int v = 0; v < NIDX; ++v) {
-        const int s = v * 64 + lane;
-        const int c = min(c0 + wbeg + min(s / K, DWN_WC - 1), NO - 1);
-        myidx[v] = idx32[(O1 ? c : c / O) * K + s % K] * 8;  // byte offset of the input's plane word
+        for (int v = 0; v < NIDX; ++v) {
+            const int s = v * 64 + lane;
+            const int c = min(c0 + wbeg + min(s / K, DWN_WC - 1), NO - 1);
+            word[v] = pl[idx32[(O1 ? c : c / O) * K + s % K]];
+        }
+#pragma unroll
+        for (int v = 0; v < NIDX; ++v) {
+            const int s = v * 64 + lane;
+            if ((v + 1) * 64 <= DWN_WC * K || s < DWN_WC * K) {
+                words[wave][0][s] = (unsigned)word[v];
+                words[wave][1][s] = (unsigned)(word[v] >> 32);
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
     }
+    const unsigned *mine = words[wave][lane >> 5];  // the words' half that holds my row
+    const int my_bit = lane & 31;
     // FULL: all 128 columns of the tile exist (every tile but possibly the last): no clamps, no per-column checks,
     // so the column offsets fold into the instructions
     u64 my_plane = 0;  // CHAIN: lane l keeps the thresholded bits of my wavefront's column l
@@ -182,7 +192,7 @@ __global__ __launch_bounds__(64 * DWN_FW) void dwn_lookup_fwd(const u64 *__restr
         constexpr bool FULL = decltype(full_tag)::value;
 #pragma unroll
         for (int g = 0; g < DWN_WC; g += DWN_CG) {
-            u64 w[DWN_CG][K];
+            unsigned w[DWN_CG * K];
             float entry[DWN_CG][NR];
 #pragma unroll
             for (int q = 0; q < DWN_CG; ++q) {
@@ -191,23 +201,20 @@ __global__ __launch_bounds__(64 * DWN_FW) void dwn_lookup_fwd(const u64 *__restr
 #pragma unroll
                 for (int r = 0; r < NR; ++r)
                     entry[q][r] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs_luts, lane4s & 255, c * (L * 4) + r * 256, 0));
+            }
+            typedef unsigned u4v __attribute__((ext_vector_type(4)));
 #pragma unroll
-                for (int j = 0; j < K; ++j) {
-                    constexpr int dummy = 0;
-                    (void)dummy;
-                    const int s = (g + q) * K + j;  // compile-time after unrolling
-                    // wave-uniform unsigned byte offset: a scalar load with the offset in an SGPR,
-                    // no scalar address arithmetic
-                    const unsigned src = (unsigned)__builtin_amdgcn_readlane(myidx[s / 64], s % 64);
-                    w[q][j] = *reinterpret_cast<const u64 *>(reinterpret_cast<const char *>(pl) + src);
-                }
+            for (int v = 0; v < DWN_CG * K / 4; ++v) {
+                const u4v q4 = *reinterpret_cast<const u4v *>(mine + g * K + 4 * v);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) w[4 * v + e] = q4[e];
             }
 #pragma unroll
             for (int q = 0; q < DWN_CG; ++q) {
                 const int cc = wbeg + g + q;
                 unsigned addr = 0;
 #pragma unroll
-                for (int j = K - 1; j >= 0; --j) addr = dwn_shift_in(addr, w[q][j]);
+                for (int j = 0; j < K; ++j) addr |= __builtin_amdgcn_ubfe(w[q * K + j], my_bit, 1) << j;
                 const float v = dwn_table_read<NR>(entry[q], addr);
                 if (FULL || cc < cend) {
                     tile[cc][lane] = EVAL ? (v >= 0.5f ? 1.0f : 0.0f) : v;
@@ -223,7 +230,7 @@ __global__ __launch_bounds__(64 * DWN_FW) void dwn_lookup_fwd(const u64 *__restr
             }
         }
     };
-    if (CHAIN && c0 + DWN_TC <= NO) {  // (the variant that writes y gains nothing from a second copy of the loop)
+    if (CHAIN && c0 + TC <= NO) {  // (the variant that writes y gains nothing from a second copy of the loop)
         columns(std::true_type{});
     } else if (wbeg < cend) {
         columns(std::false_type{});
@@ -241,7 +248,7 @@ __global__ __launch_bounds__(64 * DWN_FW) void dwn_lookup_fwd(const u64 *__restr
         float acc[DWN_GS_SLOTS];
 #pragma unroll
         for (int sl = 0; sl < DWN_GS_SLOTS; ++sl) acc[sl] = 0.0f;
-        for (int cc = wave; cc < cend; cc += DWN_FW) {
+        for (int cc = wave; cc < cend; cc += FW) {
             const int sl = (cc >= b1 ? 1 : 0) + (cc >= b1 + gsize ? 1 : 0) + (cc >= b1 + 2 * gsize ? 1 : 0);  // wave-uniform
             const float v = tile[cc][lane];
 #pragma unroll
@@ -254,26 +261,26 @@ __global__ __launch_bounds__(64 * DWN_FW) void dwn_lookup_fwd(const u64 *__restr
             const int sl = threadIdx.x >> 6;
             float sum = 0.0f;
 #pragma unroll
-            for (int w = 0; w < DWN_FW; ++w) sum += gpart[w][sl][lane];
+            for (int w = 0; w < FW; ++w) sum += gpart[w][sl][lane];
             y[((size_t)ctile * slots + sl) * ((size_t)BT * 64) + t * 64 + lane] = sum;  // y = the partial sums here
         }
         return;
     }
     if (CHAIN && !y) return;
-    if (cend == DWN_TC && t * 64 + 64 <= B && (NO & 3) == 0 && (((uintptr_t)y) & 15) == 0) {
+    if (cend == TC && t * 64 + 64 <= B && (NO & 3) == 0 && (((uintptr_t)y) & 15) == 0) {
         // whole tile: 16-byte stores, a wavefront covers two 512-byte row pieces per instruction
         typedef float f4v __attribute__((ext_vector_type(4)));
 #pragma unroll
-        for (int pass = 0; pass < 64 * DWN_TC / 4 / (64 * DWN_FW); ++pass) {
-            const int e = pass * 64 * DWN_FW + threadIdx.x;
-            const int r = e / (DWN_TC / 4), c4 = (e % (DWN_TC / 4)) * 4;
+        for (int pass = 0; pass < 64 * TC / 4 / (64 * FW); ++pass) {
+            const int e = pass * 64 * FW + threadIdx.x;
+            const int r = e / (TC / 4), c4 = (e % (TC / 4)) * 4;
             const f4v v = {tile[c4][r], tile[c4 + 1][r], tile[c4 + 2][r], tile[c4 + 3][r]};
             __builtin_nontemporal_store(v, reinterpret_cast<f4v *>(&y[(size_t)(t * 64 + r) * NO + c0 + c4]));
         }
         return;
     }
-    for (int e = threadIdx.x; e < 64 * DWN_TC; e += 64 * DWN_FW) {
-        const int r = e / DWN_TC, cc = e % DWN_TC;
+    for (int e = threadIdx.x; e < 64 * TC; e += 64 * FW) {
+        const int r = e / TC, cc = e % TC;
         const int b = t * 64 + r;
         if (b < B && cc < cend) __builtin_nontemporal_store(tile[cc][r], &y[(size_t)b * NO + c0 + cc]);
     }
@@ -599,7 +606,7 @@ __global__ __launch_bounds__(256) void dwn_bwd_transpose_hist(const float *__res
     for (int e = threadIdx.x; e < DWN_HC * ld; e += 256) hist[e] = 0.0f;
     const int t_begin = blockIdx.y * tiles_per_chunk;
     const int t_end = min(BT, t_begin + tiles_per_chunk);
-    const bool vec4 = (NO % 4 == 0) && cend == DWN_HC;
+    const bool vec4 = NO % 4 == 0 && ((uintptr_t)gy & 15) == 0;  // (a piece of four columns is there or not)
     const int q = threadIdx.x & 15, rr = threadIdx.x >> 4;  // 16 threads x 16 B cover one 64-column row piece
     const int N = NO / O;
     const int wc0 = wave * (DWN_HC / 4);  // my wavefront's first column
@@ -613,6 +620,7 @@ __global__ __launch_bounds__(256) void dwn_bwd_transpose_hist(const float *__res
             if (b < B) {
                 const float *src = gy + (size_t)b * NO + c0 + q * 4;
                 if (vec4) {
+                    if (q * 4 >= cend) continue;
                     typedef float f4v __attribute__((ext_vector_type(4)));
                     const f4v g4 = __builtin_nontemporal_load(reinterpret_cast<const f4v *>(src));  // gy is read once
                     pre[p] = make_float4(g4.x, g4.y, g4.z, g4.w);
@@ -1506,6 +1514,14 @@ static void dwn_launch_lookup(const u64 *planes, const int *idx32, const float *
              (dwn_lookup_fwd<K, O1_, CHAIN_><<<grid, 64 * DWN_FW, 0, s>>>(planes, idx32, luts, y, addrT, planes_out, B, I, \
                                                                          N, O, BT)))
     const bool chain = planes_out != nullptr || y == nullptr;
+    // up to 64 columns, blocks of as many wavefronts as they take: in one of eight the others wait
+    // (147456 rows x 32 columns 23 -> 12 us)
+#define DWN_NARROW(FW_)                                                                                                   \
+    DL_TIMED("dwn_lookup_fwd", s,                                                                                         \
+             (dwn_lookup_fwd<K, true, false, false, false, FW_><<<grid, 64 * FW_, 0, s>>>(planes, idx32, luts, y, addrT, nullptr, B, I, N, O, BT)))
+    if (O == 1 && !chain && N <= 32) { DWN_NARROW(2); return; }
+    if (O == 1 && !chain && N <= 64) { DWN_NARROW(4); return; }
+#undef DWN_NARROW
     if (O == 1 && !chain) DWN_LOOKUP(true, false);
     else if (O == 1) DWN_LOOKUP(true, true);
     else if (!chain) DWN_LOOKUP(false, false);
