@@ -148,6 +148,11 @@ def host():
     return _host
 
 
+def host_if_loaded():
+    """The native functions where something has loaded them already, else None."""
+    return _host
+
+
 def check(code):
     if code != 0:
         raise RuntimeError(f"libdifflut_hip: {lib().dl_error_string(code).decode()} (code {code})")

@@ -28,6 +28,7 @@ from abc import ABC, abstractmethod
 import torch
 import torch.nn as nn
 
+from .. import _native, ops
 from ..nodes.node_config import NodeConfig
 from ..utils.warnings import warn_default_value
 from .layer_config import LayerConfig, validate_layer_options
@@ -181,15 +182,18 @@ class ScalarBank:
         n = len(self.nodes)
         if n != len(self._views):
             return False
-        if n <= 4 * self._PROBES:
-            rows = range(n)
-        else:
-            rows = [0, n - 1] + [(self._probe + i) % n for i in range(self._PROBES)]
-            self._probe = (self._probe + self._PROBES) % n
+        start, count = self._probe, n
+        if n > 4 * self._PROBES:
+            count = self._PROBES
+            self._probe = (start + count) % n
         name, views, nodes = self.name, self._views, self.nodes
-        if isinstance(nodes, nn.ModuleList):  # as _node_getter does, without a call per node
-            if len(self._keys) != n:  # of a bank that was saved without them
-                self._keys = _node_names(n)
+        chain = isinstance(nodes, nn.ModuleList)
+        if chain and len(self._keys) != n:  # of a bank that was saved without them
+            self._keys = _node_names(n)
+        if chain and _native.host_if_loaded() is not None:  # (a layer on the CPU needs no library)
+            return _native.host_if_loaded().views_hold(nodes._modules, self._keys, name, views, start, count)
+        rows = [0, n - 1] + [(start + i) % n for i in range(count)]
+        if chain:  # as _node_getter does, without a call per node
             nodes, keys = nodes._modules, self._keys
             for row in rows:
                 if nodes[keys[row]]._buffers[name] is not views[row]:
@@ -289,8 +293,7 @@ class LUTLayerMixin(nn.Module):
             return grad
         dims = None if self.grad_stabilization == "layerwise" else 1
         if grad.is_cuda and grad.dim() == 2 and grad.dtype == torch.float32:
-            from .. import ops  # one or two library launches instead of seven torch kernels
-
+            # one or two library launches instead of seven torch kernels
             return ops.grad_stabilize(grad, dims == 1, self.grad_target_std, self.grad_subtract_mean, self.grad_epsilon)
         g = grad.clone()
         if self.grad_subtract_mean:
@@ -404,22 +407,16 @@ class BaseLUTLayer(ABC, LUTLayerMixin, nn.Module):
     def _run_nodes(self, x, plan):
         """All nodes on x [batch, width] through `plan` (index table over width) -> [batch, N*O]."""
         if self._fused == "dwn":
-            from .. import ops
-
             luts = self._banks["luts"].tensor()
             if self.training:
                 return ops.dwn_layer(x, luts, plan, *self.efd_scalars())
             return ops.dwn_layer_eval(x, luts.detach(), plan)
         if self._fused == "probabilistic":
-            from .. import ops
-
             raw = self._banks["raw_weights"].tensor()
             if self.training:
                 return ops.prob_layer(x, raw, plan, self.temperatures())
             return ops.prob_layer_eval(x, raw.detach(), plan, self.temperatures())
         if self._fused in ("dwn_stable", "hybrid"):
-            from .. import ops
-
             raw = self._banks["raw_luts"].tensor()
             if not self.training:
                 with torch.no_grad():

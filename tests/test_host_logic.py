@@ -428,6 +428,33 @@ def test_banks_notice_a_deleted_and_an_appended_node():
     assert float(layer.efd_scalars()[0][11]) == 0.125
 
 
+@pytest.mark.parametrize("native", [False, True])
+@pytest.mark.parametrize("count", [1, 12, 64, 65, 200])  # all nodes are looked at up to 64
+def test_scalar_banks_look_at_every_node_in_time(count, native, monkeypatch):
+    """A buffer swapped behind the module's back is noticed: at once among up to 64 nodes and at either end, otherwise when the window
+    has come round.  The same from the native check and the one in Python."""
+    from difflut_amd import _native as nat
+    from difflut_amd.layers import RandomLayer
+    from difflut_amd.nodes import DWNNode, NodeConfig
+
+    if native:
+        nat.host()
+    else:
+        monkeypatch.setattr(nat, "_host", None)
+    layer = RandomLayer(40, count, DWNNode, NodeConfig(input_dim=3, output_dim=1), seed=1)
+    bank = layer._scalars["alpha"]
+    windows = 1 if count <= 64 else -(-count // 16)
+    for row in sorted({0, count // 2, count - 1, min(17, count - 1)}):
+        assert all(bank.tied() for _ in range(2 * windows))
+        buffers = layer.nodes[row]._buffers
+        buffers["alpha"] = buffers["alpha"].clone()
+        seen = [not bank.tied() for _ in range(windows)]
+        assert any(seen) and (seen[0] or row not in (0, count - 1))
+        bank.tie()
+    del layer.nodes[count - 1]
+    assert not bank.tied()
+
+
 @pytest.mark.parametrize("how", ["copy", "deepcopy", "pickle"])
 def test_a_copied_bank_answers_by_itself(how):
     """A bank that is copied without its layer (in a user's own object, or while a layer is being put together again) can be
