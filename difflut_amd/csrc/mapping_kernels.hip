@@ -255,31 +255,43 @@ __global__ __launch_bounds__(256) void thermometer_kernel(const float *__restric
 // Thermometer bits as bit-planes for a following DWN layer: word (t, f*nbits + j) holds, in bit r,
 // (x[64t + r][f] > thr[f][j]).  Block = (64 features, batch tile t): the x tile is read row-wise
 // (coalesced) into LDS; then every thread builds whole output words, one (feature, threshold) pair at a
-// time, by walking the 64 rows of its feature in LDS (lanes of one feature read the same word: a
-// broadcast; different features sit in different banks).  Consecutive threads hold consecutive words, so
-// the stores are contiguous.  Rows past B read as "not greater".
+// time, from the 64 rows of its feature in LDS, four at a time (lanes of one feature read the same words: a
+// broadcast).  Consecutive threads hold consecutive words, so the stores are contiguous.  Rows past B read as "not
+// greater".  Bound by the chain of a block, load, turn, compare: the tile's loads go out together, with clamped addresses (a
+// condition around each let them out one at a time: 5001 x 784, four thresholds 10 -> 7.5 us).
 __global__ __launch_bounds__(256) void thermometer_planes_kernel(const float *__restrict__ x, const float *__restrict__ thr,
                                                                   unsigned long long *__restrict__ planes, int B, int F,
                                                                   int nbits) {
-    __shared__ float tile[64][65];  // [feature][row]
-    const int t = blockIdx.y, f0 = blockIdx.x * 64;
-    for (int e = threadIdx.x; e < 4096; e += 256) {
-        const int r = e >> 6, c = e & 63;
-        const int b = t * 64 + r;
-        tile[c][r] = (b < B && f0 + c < F) ? x[(size_t)b * F + f0 + c] : -INFINITY;
-    }
-    __syncthreads();
+    __shared__ __align__(16) float tile[64][68];  // [feature][row]; rows of a feature are read four at a time
+    const int t = blockIdx.y, f0 = blockIdx.x * 64, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const float *col = x + min(f0 + lane, F - 1);
+    float v[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) v[q] = col[(size_t)min(t * 64 + wave * 16 + q, B - 1) * F];  // all on their way, whatever is past the ends
     const int words = min(64, F - f0) * nbits;
     const float *th = thr + (size_t)f0 * nbits;
+    float limit = th[min((int)threadIdx.x, words - 1)];
+#pragma unroll
+    for (int q = 0; q < 16; q += 4) {
+        float4 four;
+        four.x = t * 64 + wave * 16 + q < B ? v[q] : -INFINITY;
+        four.y = t * 64 + wave * 16 + q + 1 < B ? v[q + 1] : -INFINITY;
+        four.z = t * 64 + wave * 16 + q + 2 < B ? v[q + 2] : -INFINITY;
+        four.w = t * 64 + wave * 16 + q + 3 < B ? v[q + 3] : -INFINITY;
+        *reinterpret_cast<float4 *>(&tile[lane][wave * 16 + q]) = four;
+    }
+    __syncthreads();
     unsigned long long *out = planes + ((size_t)t * F + f0) * nbits;
     for (int w = threadIdx.x; w < words; w += 256) {
-        const float *row = tile[w / nbits];
-        const float limit = th[w];
+        const float4 *row = reinterpret_cast<const float4 *>(tile[w / nbits]);
+        const float mine = limit;
+        limit = th[min(w + 256, words - 1)];
         unsigned lo = 0u, hi = 0u;
 #pragma unroll
-        for (int r = 0; r < 32; ++r) {
-            lo |= (row[r] > limit ? 1u : 0u) << r;  // strict compare, as the encoder
-            hi |= (row[r + 32] > limit ? 1u : 0u) << r;
+        for (int r = 0; r < 8; ++r) {
+            const float4 a = row[r], b = row[r + 8];  // strict compare, as the encoder
+            lo |= (a.x > mine ? 1u : 0u) << (4 * r) | (a.y > mine ? 2u : 0u) << (4 * r) | (a.z > mine ? 4u : 0u) << (4 * r) | (a.w > mine ? 8u : 0u) << (4 * r);
+            hi |= (b.x > mine ? 1u : 0u) << (4 * r) | (b.y > mine ? 2u : 0u) << (4 * r) | (b.z > mine ? 4u : 0u) << (4 * r) | (b.w > mine ? 8u : 0u) << (4 * r);
         }
         out[w] = ((unsigned long long)hi << 32) | lo;
     }
