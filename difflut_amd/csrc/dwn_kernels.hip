@@ -457,55 +457,83 @@ __device__ __forceinline__ void dwn_table_block(const DwnTables &tb, int block) 
     else dwn_efd_table_block(tb, block);
 }
 
-// The D form of tables with 128 or 256 entries, one block per table, the table in LDS as doubles.  EFD with |beta| <= 1/2:
-// smoothed along every input once; the difference across bit j is then (1 - beta) times the D-form value.  Other betas:
-// smoothed along all inputs but j, for every j.  Stabilised node: the 2^(k-1)-term sums.
-__global__ __launch_bounds__(256) void dwn_wide_tables(DwnTables tb) {
-    __shared__ double tab[256], tmp[256];
-    __shared__ double rec[16];
-    const int c = blockIdx.x, K = tb.K, L = 1 << K, Lh = L >> 1, a = threadIdx.x;
+// The D form of tables with 128 or 256 entries.  EFD: a wavefront per table, 2 or 4 doubles of it per lane, exchanged between lanes for
+// the lower six inputs and between registers for the others, no LDS and no barrier, so that these blocks ride in the histogram's
+// launch too.  |beta| <= 1/2: smoothed along every input once; the difference across bit j is then (1 - beta) times the D-form
+// value.  Other betas: smoothed along all inputs but j, for every j.  (A launch of its own with a block per table, the table in the
+// LDS and two barriers per input: 9.5 us for 2048 tables of 256, where these add 7.5 to the histogram's
+// 20.5, whose bins leave room for one block per CU; layer of 1024 rows, 4096 -> 2048 nodes of eight inputs 74 -> 72.6.)
+template <int NR>
+__device__ __forceinline__ void dwn_wide_smooth(double (&v)[NR], double beta, int skip) {
+#pragma unroll
+    for (int m = 0; m < 6; ++m) {
+        if (m == skip) continue;
+#pragma unroll
+        for (int r = 0; r < NR; ++r) v[r] += beta * __shfl_xor(v[r], 1 << m);
+    }
+#pragma unroll
+    for (int m = 1; m < NR; m <<= 1) {
+        if ((m == 1 ? 6 : 7) == skip) continue;
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            if (r & m) continue;
+            const double lo = v[r], hi = v[r | m];
+            v[r] = lo + beta * hi;
+            v[r | m] = hi + beta * lo;
+        }
+    }
+}
+template <int NR>
+__device__ __forceinline__ void dwn_wide_efd_table(const DwnTables &tb, int c) {
+    constexpr int K = NR == 2 ? 7 : 8, L = 64 * NR, Lh = L / 2;
+    const int lane = threadIdx.x & 63;
     const double alpha = tb.alpha_n ? (double)tb.alpha_n[c / tb.O] : (double)tb.alpha;
     const double beta = tb.beta_n ? (double)tb.beta_n[c / tb.O] : (double)tb.beta;
+    float *__restrict__ D = tb.D + (size_t)c * K * Lh;
+    double v[NR];
+#pragma unroll
+    for (int r = 0; r < NR; ++r) v[r] = (double)tb.luts[(size_t)c * L + 64 * r + lane];
+    const bool compact = beta >= -0.5 && beta <= 0.5;  // (the wavefront's)
+    const double factor = compact ? alpha / (1.0 - beta) : alpha;
+    if (compact) dwn_wide_smooth<NR>(v, beta, -1);
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+        double u[NR];
+#pragma unroll
+        for (int r = 0; r < NR; ++r) u[r] = v[r];
+        if (!compact) dwn_wide_smooth<NR>(u, beta, j);
+#pragma unroll
+        for (int r = 0; r < NR; ++r) {
+            const int a = 64 * r + lane;
+            const double upper = j < 6 ? __shfl_xor(u[r], 1 << (j < 6 ? j : 0)) : u[(r | (j == 6 ? 1 : 2)) % NR];
+            if (!((a >> j) & 1)) D[j * Lh + ((a & ((1 << j) - 1)) | ((a >> (j + 1)) << j))] = (float)(factor * (upper - u[r]));
+        }
+    }
+}
+__device__ __forceinline__ void dwn_wide_efd_block(const DwnTables &tb, int block) {
+    const int c = block * 4 + dl_uniform(threadIdx.x >> 6);
+    if (c >= tb.NO) return;
+    if (tb.K == 7) dwn_wide_efd_table<2>(tb, c);
+    else dwn_wide_efd_table<4>(tb, c);
+}
+// Stabilised node: the 2^(k-1)-term sums, one block per table, the table in the LDS as doubles.
+__global__ __launch_bounds__(256) void dwn_wide_tables(DwnTables tb) {
+    __shared__ double tab[256];
+    __shared__ double rec[16];
+    const int c = blockIdx.x, K = tb.K, L = 1 << K, Lh = L >> 1, a = threadIdx.x;
     float *__restrict__ D = tb.D + (size_t)c * K * Lh;
     if (a < L) tab[a] = (double)tb.luts[(size_t)c * L + a];
     if (a < 16) rec[a] = 1.0 / (double)(a + 1);
     __syncthreads();
-    auto smooth = [&](double *t, int skip) {  // t <- t smoothed along every input but `skip`; called by the whole block
-        for (int m = 0; m < K; ++m) {
-            if (m == skip) continue;
-            double lo = 0.0, hi = 0.0;
-            const bool mine = a < L && !((a >> m) & 1);
-            if (mine) { lo = t[a]; hi = t[a | (1 << m)]; }
-            __syncthreads();
-            if (mine) { t[a] = lo + beta * hi; t[a | (1 << m)] = hi + beta * lo; }
-            __syncthreads();
+    const double sc = (double)tb.scale[c / tb.O];
+    for (int o = a; o < K * Lh; o += 256) {
+        const int j = o / Lh, ap = o - j * Lh, low = (1 << j) - 1;
+        double acc = 0.0;
+        for (int kp = 0; kp < Lh; ++kp) {
+            const int at = (kp & low) | ((kp & ~low) << 1);
+            acc += (tab[at | (1 << j)] - tab[at]) * rec[__popc(ap ^ kp)];
         }
-    };
-    auto squeeze = [](int v, int j) { return (v & ((1 << j) - 1)) | ((v >> (j + 1)) << j); };
-    if (tb.scale) {
-        const double sc = (double)tb.scale[c / tb.O];
-        for (int o = a; o < K * Lh; o += 256) {
-            const int j = o / Lh, ap = o - j * Lh, low = (1 << j) - 1;
-            double acc = 0.0;
-            for (int kp = 0; kp < Lh; ++kp) {
-                const int at = (kp & low) | ((kp & ~low) << 1);
-                acc += (tab[at | (1 << j)] - tab[at]) * rec[__popc(ap ^ kp)];
-            }
-            D[o] = (float)(sc * acc);
-        }
-    } else if (beta >= -0.5 && beta <= 0.5) {
-        smooth(tab, -1);
-        if (a < L)
-            for (int j = 0; j < K; ++j)
-                if (!((a >> j) & 1)) D[j * Lh + squeeze(a, j)] = (float)(alpha / (1.0 - beta) * (tab[a | (1 << j)] - tab[a]));
-    } else {
-        for (int j = 0; j < K; ++j) {
-            if (a < L) tmp[a] = tab[a];
-            __syncthreads();
-            smooth(tmp, j);
-            if (a < L && !((a >> j) & 1)) D[j * Lh + squeeze(a, j)] = (float)(alpha * (tmp[a | (1 << j)] - tmp[a]));
-            __syncthreads();
-        }
+        D[o] = (float)(sc * acc);
     }
 }
 
@@ -598,7 +626,10 @@ __global__ __launch_bounds__(256) void dwn_bwd_transpose_hist(const float *__res
     float *const hist = WIDE ? hist_d : hist_s;
     const int ld = WIDE ? L + 1 : 65;
     __shared__ __align__(16) uint8_t atile[DWN_HC][64 + 4];  // [column][row] addresses
-    if ((int)blockIdx.y >= chunks) return dwn_table_block(tb, ((int)blockIdx.y - chunks) * gridDim.x + blockIdx.x);
+    if ((int)blockIdx.y >= chunks) {
+        const int block = ((int)blockIdx.y - chunks) * gridDim.x + blockIdx.x;
+        return WIDE ? dwn_wide_efd_block(tb, block) : dwn_table_block(tb, block);
+    }
     const int c0 = blockIdx.x * DWN_HC;
     const int lane = threadIdx.x & 63;
     const int wave = dl_uniform(threadIdx.x >> 6);
@@ -1868,7 +1899,7 @@ static int dwn_backward_fast(const void *saved, const int32_t *inv_ptr, const in
     const bool long_rows = gx && !prev && !wide && dwn_long_applies(BT, I, N, k, O, gx_tiled);
     DwnTables tb = {gather && (!rc || rc->first) ? luts : nullptr, D, scale, alpha_n, beta_n, alpha, beta, (int)NO, k, O,
                     sform ? (walk_pack || fused_pack || long_rows ? 2 : 1) : 0};
-    if (wide && tb.luts) {
+    if (wide && tb.luts && scale) {
         DL_TIMED("dwn_wide_tables", s, (dwn_wide_tables<<<(unsigned)NO, 256, 0, s>>>(tb)));
         tb.luts = nullptr;
     }

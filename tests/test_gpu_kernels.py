@@ -675,6 +675,29 @@ def test_layer_forward_of_few_rows(B, I, N, k, O):
     assert torch.equal(y[0], y[1]) and torch.equal(saved[0][:held], saved[1][:held])
 
 
+@pytest.mark.parametrize("k", [7, 8])
+@pytest.mark.parametrize("beta", [1 / 3, -0.5, 0.8])  # the compact form of the tables, its edge, the other one
+@pytest.mark.parametrize("B,N,O", [(65, 5, 1), (130, 67, 2)])
+def test_wide_coefficient_tables(B, N, O, beta, k):
+    """Tables of 128 and 256 entries are built by a wavefront each, beside the histogram.  Floors as for the other gradients: a
+    connection's term is a difference of two fp32 roundings of sums of up to 2^(k-1) products of size 1."""
+    ops = _ops()
+    I = 50
+    rng = np.random.default_rng(B + k)
+    x = rng.uniform(0, 1, (B, I)).astype(np.float32)
+    idx = orc.random_mapping(I, N, k, seed=4).numpy().astype(np.int64)
+    luts = rng.uniform(-1, 1, (N, O, 1 << k)).astype(np.float32)
+    gy = rng.standard_normal((B, N, O)).astype(np.float32)
+    xt, lt = dev(x).requires_grad_(), dev(luts).requires_grad_()
+    alpha = 0.4 * 0.75 ** (k - 1)
+    y = ops.DWNLayerFunction.apply(xt, lt, ops.MappingPlan(dev(idx, torch.int32), I), alpha, beta)
+    y.backward(dev(gy.reshape(B, -1)))
+    gx, gl = orc.dwn_layer_backward(x, idx, luts, gy, np.float32(alpha), np.float32(beta))
+    scale = float(np.abs(gx).max())
+    np.testing.assert_allclose(xt.grad.cpu().numpy(), gx, rtol=1e-5, atol=1e-6 * scale)
+    np.testing.assert_allclose(lt.grad.cpu().numpy(), gl, rtol=1e-5, atol=1e-5)
+
+
 # ------------------------------------------------------------------------------ probabilistic
 PROB_SHAPES = [(32, 40, 24, 4, 2), (64, 128, 300, 4, 1), (17, 30, 9, 6, 1), (20, 9, 5, 1, 1), (10, 50, 7, 2, 3),
                (6, 40, 5, 7, 2), (200, 300, 260, 4, 1), (130, 70, 33, 5, 2), (65, 1000, 515, 3, 1),
