@@ -66,6 +66,8 @@ SIGNATURES = {
     "dl_hybrid_bwd_saved_workspace_bytes": (_Z, [_I] * 5),
     "dl_hybrid_layer_fwd": (_I, [_P, _P, _P, _P, _P, _Z, _P, _Z, _I, _I, _I, _I, _I, _P]),
     "dl_hybrid_layer_bwd_saved": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _Z, _I, _I, _I, _I, _I, _P]),
+    "dl_hybrid_raw_fwd": (_I, [_P, _P, _P, _P, _P, _P, _Z, _P, _Z, _I, _I, _I, _I, _I, _P]),
+    "dl_hybrid_raw_bwd": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _Z, _I, _I, _I, _I, _I, _P]),
     "dl_prob_saved_bytes": (_Z, [_I] * 5),
     "dl_prob_bwd_workspace_bytes": (_Z, [_I] * 5),
     "dl_prob_bwd_saved_workspace_bytes": (_Z, [_I] * 5),

@@ -25,7 +25,7 @@ namespace {
     X(dl_dwn_bwd_reads_x) X(dl_dwn_layer_fwd) X(dl_dwn_layer_bwd) X(dl_dwn_layer_bwd_nodes) X(dl_dwn_stable_layer_bwd)   \
     X(dl_table_sigmoid_fwd) X(dl_table_sigmoid_bwd) X(dl_hybrid_saved_bytes) X(dl_hybrid_fwd_workspace_bytes)            \
     X(dl_hybrid_bwd_workspace_bytes) X(dl_hybrid_bwd_saved_workspace_bytes) X(dl_hybrid_layer_fwd)                       \
-    X(dl_hybrid_layer_bwd) X(dl_hybrid_layer_bwd_saved) X(dl_prob_saved_bytes) X(dl_prob_bwd_saved_workspace_bytes)      \
+    X(dl_hybrid_layer_bwd) X(dl_hybrid_layer_bwd_saved) X(dl_hybrid_raw_fwd) X(dl_hybrid_raw_bwd) X(dl_prob_saved_bytes) X(dl_prob_bwd_saved_workspace_bytes)      \
     X(dl_prob_layer_fwd) X(dl_prob_layer_fwd_nodes) X(dl_prob_layer_bwd) X(dl_prob_layer_bwd_nodes)                      \
     X(dl_prob_ordered_saved_bytes) X(dl_prob_ordered_bwd_workspace_bytes) X(dl_prob_ordered_fwd) X(dl_prob_ordered_bwd)  \
     X(dl_soft_map_saved_bytes) X(dl_soft_map_workspace_bytes) X(dl_soft_map_fwd) X(dl_soft_map_bwd) X(dl_unfold_rows)    \
@@ -243,6 +243,35 @@ struct HybridLayer : torch::autograd::Function<HybridLayer> {
                                               out(gx), out(gl), raw(ws), ws.numel(), DIMS(d), stream()));
         }
         return {gx, gl, Tensor(), Tensor()};
+    }
+};
+
+// The same on the tables' raw values, whose sigmoid and its gradient are part of the launches: for a layer small enough that what it
+// costs is launches and autograd nodes, two of six and one of two.
+struct HybridRaw : torch::autograd::Function<HybridRaw> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &x_, const Tensor &raw_, const Kept *given) {
+        const Tensor x = f32(x_), w = f32(raw_), luts = at::empty_like(w);
+        auto k = c10::make_intrusive<Kept>(*given);
+        const Dims d = k->dims = lookup_dims(x, w, k->plan);
+        const Tensor y = floats({d.B, (int64_t)d.N * d.O}, x), tiles = bytes(L.dl_hybrid_saved_bytes(DIMS(d)), x),
+                     ws = bytes(L.dl_hybrid_fwd_workspace_bytes(DIMS(d)), x);
+        check(L.dl_hybrid_raw_fwd(in(x), ints(k->plan.idx), in(w), out(luts), out(y), raw(tiles), tiles.numel(), raw(ws), ws.numel(), DIMS(d),
+                                  stream()));
+        ctx->save_for_backward({luts, tiles});
+        keep(ctx, std::move(k));
+        return y;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        const auto s = ctx->get_saved_variables();
+        const auto k = kept_of<Kept>(ctx);
+        const Dims &d = k->dims;
+        const Plan &p = k->plan;
+        const Tensor gy = f32(grads[0]);
+        const Tensor gx = ctx->needs_input_grad(0) ? floats({d.B, d.I}, gy) : Tensor();
+        const Tensor graw = at::empty_like(s[0]), ws = bytes(L.dl_hybrid_bwd_saved_workspace_bytes(DIMS(d)), gy);
+        check(L.dl_hybrid_raw_bwd(raw(s[1]), ints(p.idx), ints(p.inv_ptr), ints(p.inv_pos), in(s[0]), in(gy), out(gx), out(graw), raw(ws),
+                                  ws.numel(), DIMS(d), stream()));
+        return {gx, graw, Tensor()};
     }
 };
 
@@ -624,6 +653,16 @@ Tensor hybrid_layer(const Tensor &x, const Tensor &luts, const PlanArgs &plan, b
     k.plan = plan_of(plan);
     return HybridLayer::apply(x, luts, (const Kept *)&k, keep_tiles);
 }
+Tensor hybrid_raw_layer(const Tensor &x, const Tensor &w, const PlanArgs &plan, bool keep_tiles) {
+    require_device(x);
+    require_device(w);
+    Kept k;
+    k.plan = plan_of(plan);
+    if (keep_tiles && x.dim() == 2 && w.dim() == 3 && k.plan.k <= DL_MAX_FAST_K &&
+        L.dl_hybrid_saved_bytes((int)x.size(0), k.plan.I, k.plan.N, k.plan.k, (int)w.size(1)) > 256)
+        return HybridRaw::apply(x, w, (const Kept *)&k);
+    return HybridLayer::apply(x, TableSigmoid::apply(w), (const Kept *)&k, keep_tiles);
+}
 Tensor prob_layer(const Tensor &x, const Tensor &w, const PlanArgs &plan, bool ordered, const Maybe &T_n, double T) {
     Kept k;
     k.plan = plan_of(plan);
@@ -728,6 +767,7 @@ PYBIND11_MODULE(difflut_host, m) {
     m.def("dwn_layer", &dwn_layer, free_gil);
     m.def("dwn_stable_layer", &dwn_stable_layer, free_gil);
     m.def("hybrid_layer", &hybrid_layer, free_gil);
+    m.def("hybrid_raw_layer", &hybrid_raw_layer, free_gil);
     m.def("table_sigmoid", [](const Tensor &t) { return TableSigmoid::apply(t); }, free_gil);
     m.def("prob_layer", &prob_layer, free_gil);
     m.def("soft_map", [](const Tensor &x, const Tensor &W, double tau, int64_t precision) { return SoftMap::apply(x, W, tau, precision); },

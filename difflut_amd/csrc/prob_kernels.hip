@@ -57,6 +57,7 @@ struct ProbTables {
     ProbTemp T;
     float *sig, *cen;
     int N, L, O;
+    bool flat = false;        // hybrid: raw in the table's own layout
 };
 __device__ __forceinline__ void prob_table_element(const ProbTables &q, long long e) {
     if (e >= (long long)q.N * q.L * q.O) return;
@@ -65,7 +66,7 @@ __device__ __forceinline__ void prob_table_element(const ProbTables &q, long lon
     const int n = (int)(c / q.O), d = (int)(c % q.O);
     const float inv = q.luts ? 1.0f : prob_inv_t_of(q.T, n);
     auto value = [&](int at) -> float {
-        return q.luts ? q.luts[c * q.L + at] : dl_sigmoid(q.raw[((size_t)n * q.L + at) * q.O + d] * inv);
+        return q.luts ? q.luts[c * q.L + at] : dl_sigmoid(q.raw[q.flat ? (size_t)c * q.L + at : ((size_t)n * q.L + at) * q.O + d] * inv);
     };
     const float v = value(a);
     if (q.sig) q.sig[e] = v;
@@ -676,6 +677,7 @@ struct ProbReduce {  // the table-gradient reduction, also carried as extra bloc
     ProbTemp T;
     float *graw;
     int N, L, O, chunks;
+    bool flat = false;  // hybrid: the gradient of what the table is the sigmoid of, in the table's own layout
 };
 __device__ __forceinline__ void prob_reduce_element(const ProbReduce &R, long long e);
 __global__ __launch_bounds__(256) void prob_reduce_weights(ProbReduce R) {
@@ -701,10 +703,14 @@ __device__ __forceinline__ void prob_reduce_element(const ProbReduce &R, long lo
         graw[e] = acc;
         return;
     }
+    const float s = sig[e];
+    if (R.flat) {
+        graw[e] = acc * s * (1.0f - s);
+        return;
+    }
     const int a = (int)(e % L);
     const long long c = e / L;
     const int n = (int)(c / O), d = (int)(c % O);
-    const float s = sig[e];
     graw[((size_t)n * L + a) * O + d] = acc * s * (1.0f - s) * prob_inv_t_of(R.T, n);
 }
 
@@ -1216,9 +1222,9 @@ extern "C" size_t dl_hybrid_fwd_workspace_bytes(int B, int I, int N, int k, int 
     const size_t planes = dl_align256(dl_dwn_planes_bytes(B, I)), own = dl_align256(dl_dwn_fwd_workspace_bytes(B, I, N, k, O));
     return dl_align256(dl_dwn_saved_bytes(B, I, N, k, O)) + (planes > own ? planes : own);
 }
-extern "C" int dl_hybrid_layer_fwd(const float *x, const int32_t *idx32, const float *luts, float *y, void *saved,
-                                   size_t saved_bytes, void *ws, size_t ws_bytes, int B, int I, int N, int k, int O,
-                                   void *stream) {
+// raw (nullable): the tables are its sigmoid and written to `luts`, by the blocks that build the backward's
+static int hybrid_forward(const float *x, const int32_t *idx32, const float *raw, float *luts, float *y, void *saved,
+                          size_t saved_bytes, void *ws, size_t ws_bytes, int B, int I, int N, int k, int O, void *stream) {
     if (!x || !idx32 || !luts || !y || !saved || !ws) return DL_ERR_NULL;
     if (B <= 0 || I <= 0 || N <= 0 || k <= 0 || O <= 0) return DL_ERR_SHAPE;
     if (saved_bytes < dl_hybrid_saved_bytes(B, I, N, k, O) || ws_bytes < dl_hybrid_fwd_workspace_bytes(B, I, N, k, O))
@@ -1226,18 +1232,30 @@ extern "C" int dl_hybrid_layer_fwd(const float *x, const int32_t *idx32, const f
     hipStream_t s = (hipStream_t)stream;
     const size_t addr_bytes = dl_align256(dl_dwn_saved_bytes(B, I, N, k, O));
     char *rest = (char *)ws + addr_bytes;
+    if (raw && !hybrid_tiled(B, I, N, k, O)) return DL_ERR_UNSUPPORTED;
     if (hybrid_tiled(B, I, N, k, O)) {
-        const ProbTables q{nullptr, luts, ProbTemp{1.0f, nullptr}, nullptr, (float *)((char *)saved + prob_xT_bytes(B, I)), N, 1 << k, O};
+        const ProbTables q{raw, raw ? nullptr : luts, ProbTemp{1.0f, nullptr}, raw ? luts : nullptr, (float *)((char *)saved + prob_xT_bytes(B, I)),
+                           N, 1 << k, O, true};
         prob_launch_to_tiles<true>("hybrid_tiles+planes", x, (float *)saved, B, I, q, s, (unsigned long long *)rest);
         const int rc = dl_dwn_layer_fwd_planes(rest, idx32, luts, y, nullptr, ws, B, I, N, k, O, stream);
         if (rc != DL_ERR_UNSUPPORTED) return rc;
     }
     return dl_dwn_layer_fwd(x, idx32, luts, y, ws, rest, ws_bytes - addr_bytes, B, I, N, k, O, stream);
 }
+extern "C" int dl_hybrid_layer_fwd(const float *x, const int32_t *idx32, const float *luts, float *y, void *saved,
+                                   size_t saved_bytes, void *ws, size_t ws_bytes, int B, int I, int N, int k, int O,
+                                   void *stream) {
+    return hybrid_forward(x, idx32, nullptr, const_cast<float *>(luts), y, saved, saved_bytes, ws, ws_bytes, B, I, N, k, O, stream);
+}
+extern "C" int dl_hybrid_raw_fwd(const float *x, const int32_t *idx32, const float *raw_luts, float *luts, float *y, void *saved,
+                                 size_t saved_bytes, void *ws, size_t ws_bytes, int B, int I, int N, int k, int O, void *stream) {
+    if (!raw_luts) return DL_ERR_NULL;
+    return hybrid_forward(x, idx32, raw_luts, luts, y, saved, saved_bytes, ws, ws_bytes, B, I, N, k, O, stream);
+}
 
 static int hybrid_backward(const float *x, const void *saved, const int32_t *idx32, const int32_t *inv_ptr,
                            const int32_t *inv_pos, const float *luts, const float *gy, float *gx, float *gluts, void *ws,
-                           size_t ws_bytes, size_t ws_needed, int B, int I, int N, int k, int O, void *stream) {
+                           size_t ws_bytes, size_t ws_needed, int B, int I, int N, int k, int O, void *stream, bool to_raw = false) {
     if (!idx32 || !luts || !gy || !gluts) return DL_ERR_NULL;
     if (!x && !(saved && hybrid_tiled(B, I, N, k, O))) return DL_ERR_NULL;
     if (gx && (!inv_ptr || !inv_pos)) return DL_ERR_NULL;
@@ -1269,7 +1287,7 @@ static int hybrid_backward(const float *x, const void *saved, const int32_t *idx
     float *gmT = (float *)w; w += dl_align256((size_t)BT * NO * k * 64 * sizeof(float));
     float *gpart = (float *)w;
     prob_launch_bwd<true>("hybrid_bwd_t", xT, gy, idx32, cen, gmT, gpart, B, I, N, k, O, tpc, gx != nullptr, s);
-    const ProbReduce R = {gpart, nullptr, ProbTemp{1.0f, nullptr}, gluts, N, L, O, chunks};
+    const ProbReduce R = {gpart, to_raw ? luts : nullptr, ProbTemp{1.0f, nullptr}, gluts, N, L, O, chunks, true};
     prob_launch_gather_and_reduce(gmT, inv_ptr, inv_pos, gx, B, I, N, k, O, BT, R, WT, s);
     return dl_launch_status();
 }
@@ -1289,6 +1307,16 @@ extern "C" int dl_hybrid_layer_bwd_saved(const float *x, const void *saved, cons
     if (!saved) return DL_ERR_NULL;
     return hybrid_backward(x, saved, idx32, inv_ptr, inv_pos, luts, gy, gx, gluts, ws, ws_bytes,
                            dl_hybrid_bwd_saved_workspace_bytes(B, I, N, k, O), B, I, N, k, O, stream);
+}
+
+// of a forward that made the tables: gluts is the gradient of what they are the sigmoid of
+extern "C" int dl_hybrid_raw_bwd(const void *saved, const int32_t *idx32, const int32_t *inv_ptr, const int32_t *inv_pos, const float *luts,
+                                 const float *gy, float *gx, float *graw, void *ws, size_t ws_bytes, int B, int I, int N, int k, int O,
+                                 void *stream) {
+    if (!saved) return DL_ERR_NULL;
+    if (B > 0 && I > 0 && N > 0 && k > 0 && O > 0 && !hybrid_tiled(B, I, N, k, O)) return DL_ERR_UNSUPPORTED;
+    return hybrid_backward(nullptr, saved, idx32, inv_ptr, inv_pos, luts, gy, gx, graw, ws, ws_bytes,
+                           dl_hybrid_bwd_saved_workspace_bytes(B, I, N, k, O), B, I, N, k, O, stream, true);
 }
 
 // Eval forward with a workspace: the binarised sigmoid table of every node is the table of a DWN layer, so the

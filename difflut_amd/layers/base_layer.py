@@ -421,10 +421,9 @@ class BaseLUTLayer(ABC, LUTLayerMixin, nn.Module):
             if not self.training:
                 with torch.no_grad():
                     return ops.dwn_layer_eval(x, ops.table_sigmoid(raw), plan)
-            luts = ops.table_sigmoid(raw)
             if self._fused == "hybrid":
-                return ops.hybrid_layer(x, luts, plan)
-            return ops.dwn_stable_layer(x, luts, self._banks["gradient_scale"].tensor().detach(), plan)
+                return ops.hybrid_raw_layer(x, raw, plan)
+            return ops.dwn_stable_layer(x, ops.table_sigmoid(raw), self._banks["gradient_scale"].tensor().detach(), plan)
         return None
 
     def _loop_nodes(self, mapped):

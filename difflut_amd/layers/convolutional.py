@@ -218,7 +218,7 @@ class ConvolutionalLayer(LUTLayerMixin, nn.Module):
                 with torch.no_grad():
                     h = ops.dwn_layer_eval(h, ops.table_sigmoid(bank["raw_luts"]), plan)
             elif kind == "hybrid":
-                h = ops.hybrid_layer(h, ops.table_sigmoid(bank["raw_luts"]), plan)
+                h = ops.hybrid_raw_layer(h, bank["raw_luts"], plan)
             else:
                 h = ops.dwn_stable_layer(h, ops.table_sigmoid(bank["raw_luts"]),
                                                      bank["gradient_scale"].detach(), plan)

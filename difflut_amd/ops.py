@@ -429,6 +429,14 @@ def hybrid_layer(x, luts, plan):
     return HybridLayerFunction.apply(x, luts, plan, keep)
 
 
+def hybrid_raw_layer(x, raw, plan):
+    """hybrid_layer(x, table_sigmoid(raw), plan), as one operator."""
+    if not x.is_cuda:
+        return cpu_ops.hybrid_layer(x, table_sigmoid(raw), plan)
+    keep = torch.is_grad_enabled() and (x.requires_grad or raw.requires_grad)
+    return nat.host().hybrid_raw_layer(x, raw, plan.host, keep)
+
+
 def table_sigmoid(raw):
     return TableSigmoidFunction.apply(raw) if raw.is_cuda else torch.sigmoid(raw.float())
 

@@ -304,6 +304,14 @@ int dl_hybrid_layer_fwd(const float *x, const int32_t *idx32, const float *luts,
 int dl_hybrid_layer_bwd_saved(const float *x, const void *saved, const int32_t *idx32, const int32_t *inv_ptr,
                               const int32_t *inv_pos, const float *luts, const float *gy, float *gx, float *gluts,
                               void *ws, size_t ws_bytes, int B, int I, int N, int k, int O, void *stream);
+/* The same pair with the sigmoid of the tables in it (hybrid_node.py:309-315): raw_luts [N,O,L] in, luts = sigmoid(raw_luts)
+ * written by the forward for the backward, whose graw is the gradient of raw_luts.  Where dl_hybrid_saved_bytes reports 256 they
+ * are refused (DL_ERR_UNSUPPORTED). */
+int dl_hybrid_raw_fwd(const float *x, const int32_t *idx32, const float *raw_luts, float *luts, float *y, void *saved,
+                      size_t saved_bytes, void *ws, size_t ws_bytes, int B, int I, int N, int k, int O, void *stream);
+int dl_hybrid_raw_bwd(const void *saved, const int32_t *idx32, const int32_t *inv_ptr, const int32_t *inv_pos,
+                      const float *luts, const float *gy, float *gx, float *graw, void *ws, size_t ws_bytes,
+                      int B, int I, int N, int k, int O, void *stream);
 
 /* ------------------------------------------------------------------------
  * RandomLayer + Probabilistic nodes, whole layer in one call.

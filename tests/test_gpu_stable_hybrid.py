@@ -177,6 +177,31 @@ def test_hybrid_layer_forward_backward(shape):
     np.testing.assert_allclose(rt.grad.cpu().numpy(), graw, rtol=1e-5, atol=2e-6)
 
 
+@pytest.mark.parametrize("shape", SHAPES + [(1500, 40, 50, 5, 2), (64, 30, 16, 6, 1)])
+@pytest.mark.parametrize("grads", ["both", "tables", "none"])
+def test_hybrid_with_the_sigmoid_inside(shape, grads):
+    """One operator on the raw tables against the two: the same bits, also where only the tables want a gradient, where nothing does
+    and where the kernels with an atomic sum take over (k > 6: equal up to the order of those)."""
+    B, I, N, k, O = shape
+    ops = _ops()
+    x, idx, raw, gy, _ = make_case(sum(shape) + 2, *shape, interior=True)
+    plan = ops.MappingPlan(dev(idx, torch.int32), I)
+    got = []
+    for inside in (False, True):
+        xt = dev(x).requires_grad_(grads == "both")
+        rt = dev(raw).requires_grad_(grads != "none")
+        y = ops.hybrid_raw_layer(xt, rt, plan) if inside else ops.hybrid_layer(xt, ops.table_sigmoid(rt), plan)
+        assert y.requires_grad == (grads != "none")
+        if grads != "none":
+            y.backward(dev(gy.reshape(B, N * O)))
+        got.append((y.detach(), xt.grad, rt.grad))
+    for a, b in zip(*got):
+        if a is None or k <= 6:
+            assert (a is None and b is None) or torch.equal(a, b)
+        else:
+            torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-5)
+
+
 @pytest.mark.parametrize("shape", [(66, 20, 30, 4, 1), (12, 30, 8, 7, 1)])
 def test_hybrid_binary_inputs_get_zero_gradient(shape):
     """x_j (1 - x_j) = 0 at a binary input, so the reference's factor (a_j - x_j) / (x_j (1 - x_j) + 1e-8)
