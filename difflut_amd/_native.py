@@ -57,6 +57,7 @@ SIGNATURES = {
     "dl_dwn_layer_bwd_chain_first": (_I, [_P, _P, _P, _P, _P, _I, _I, _F, _P, _P, _F, _P, _P, _P, _P, _P, _P, _P, _P, _P, _F, _I, _P,
                                           _P, _Z, _I, _I, _I, _I, _I, _P]),
     "dl_dwn_stable_layer_bwd": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _Z, _I, _I, _I, _I, _I, _P]),
+    "dl_dwn_stable_raw_bwd": (_I, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _Z, _I, _I, _I, _I, _I, _P]),
     "dl_table_sigmoid_fwd": (_I, [_P, _P, ctypes.c_longlong, _P]),
     "dl_table_sigmoid_bwd": (_I, [_P, _P, _P, ctypes.c_longlong, _P]),
     "dl_hybrid_bwd_workspace_bytes": (_Z, [_I] * 5),

@@ -23,6 +23,7 @@ namespace {
 #define DL_FUNCTIONS(X)                                                                                                  \
     X(dl_error_string) X(dl_dwn_saved_bytes) X(dl_dwn_fwd_workspace_bytes) X(dl_dwn_bwd_workspace_bytes)                 \
     X(dl_dwn_bwd_reads_x) X(dl_dwn_layer_fwd) X(dl_dwn_layer_bwd) X(dl_dwn_layer_bwd_nodes) X(dl_dwn_stable_layer_bwd)   \
+    X(dl_dwn_stable_raw_bwd)                                                                                             \
     X(dl_table_sigmoid_fwd) X(dl_table_sigmoid_bwd) X(dl_hybrid_saved_bytes) X(dl_hybrid_fwd_workspace_bytes)            \
     X(dl_hybrid_bwd_workspace_bytes) X(dl_hybrid_bwd_saved_workspace_bytes) X(dl_hybrid_layer_fwd)                       \
     X(dl_hybrid_layer_bwd) X(dl_hybrid_layer_bwd_saved) X(dl_hybrid_raw_fwd) X(dl_hybrid_raw_bwd) X(dl_prob_saved_bytes) X(dl_prob_bwd_saved_workspace_bytes)      \
@@ -199,6 +200,34 @@ struct DwnStableLayer : torch::autograd::Function<DwnStableLayer> {
         check(L.dl_dwn_stable_layer_bwd(in(s[3]), raw(s[1]), ints(p.idx), ints(p.inv_ptr), ints(p.inv_pos), in(s[0]), in(gy), in(s[2]),
                                         out(gx), out(gl), raw(ws), ws.numel(), DIMS(d), stream()));
         return {gx, gl, Tensor(), Tensor()};
+    }
+};
+
+// The same on the tables' raw values: one node, and the sigmoid's adjoint where the table gradient is written.
+struct DwnStableRaw : torch::autograd::Function<DwnStableRaw> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &x_, const Tensor &raw_, const Tensor &scale_, const Kept *given) {
+        require_device(scale_);
+        const Tensor x = f32(x_), w = f32(raw_), scale = f32(scale_.detach()).reshape({-1}), luts = at::empty_like(w);
+        TORCH_CHECK(scale.numel() == w.size(0), "gradient_scale has ", scale.numel(), " entries for ", w.size(0), " nodes");
+        auto k = c10::make_intrusive<Kept>(*given);
+        k->dims = lookup_dims(x, w, k->plan);
+        check(L.dl_table_sigmoid_fwd(in(w), out(luts), w.numel(), stream()));
+        auto [y, saved] = dwn_lookup(x, luts, k->plan, k->dims);
+        ctx->save_for_backward({luts, saved, scale});
+        keep(ctx, std::move(k));
+        return y;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        const auto s = ctx->get_saved_variables();
+        const auto k = kept_of<Kept>(ctx);
+        const Dims &d = k->dims;
+        const Plan &p = k->plan;
+        const Tensor gy = f32(grads[0]);
+        const Tensor gx = ctx->needs_input_grad(0) ? floats({d.B, d.I}, gy) : Tensor();
+        const Tensor graw = at::empty_like(s[0]), ws = bytes(L.dl_dwn_bwd_workspace_bytes(DIMS(d)), gy);
+        check(L.dl_dwn_stable_raw_bwd(raw(s[1]), ints(p.idx), ints(p.inv_ptr), ints(p.inv_pos), in(s[0]), in(gy), in(s[2]), out(gx), out(graw),
+                                      raw(ws), ws.numel(), DIMS(d), stream()));
+        return {gx, graw, Tensor(), Tensor()};
     }
 };
 
@@ -653,6 +682,14 @@ Tensor hybrid_layer(const Tensor &x, const Tensor &luts, const PlanArgs &plan, b
     k.plan = plan_of(plan);
     return HybridLayer::apply(x, luts, (const Kept *)&k, keep_tiles);
 }
+Tensor dwn_stable_raw_layer(const Tensor &x, const Tensor &w, const Tensor &scale, const PlanArgs &plan) {
+    require_device(x);
+    require_device(w);
+    Kept k;
+    k.plan = plan_of(plan);
+    if (w.dim() == 3 && L.dl_dwn_bwd_reads_x(k.plan.N, k.plan.k, (int)w.size(1)) == 0) return DwnStableRaw::apply(x, w, scale, (const Kept *)&k);
+    return DwnStableLayer::apply(x, TableSigmoid::apply(w), scale, (const Kept *)&k);
+}
 Tensor hybrid_raw_layer(const Tensor &x, const Tensor &w, const PlanArgs &plan, bool keep_tiles) {
     require_device(x);
     require_device(w);
@@ -767,6 +804,7 @@ PYBIND11_MODULE(difflut_host, m) {
     m.def("dwn_layer", &dwn_layer, free_gil);
     m.def("dwn_stable_layer", &dwn_stable_layer, free_gil);
     m.def("hybrid_layer", &hybrid_layer, free_gil);
+    m.def("dwn_stable_raw_layer", &dwn_stable_raw_layer, free_gil);
     m.def("hybrid_raw_layer", &hybrid_raw_layer, free_gil);
     m.def("table_sigmoid", [](const Tensor &t) { return TableSigmoid::apply(t); }, free_gil);
     m.def("prob_layer", &prob_layer, free_gil);

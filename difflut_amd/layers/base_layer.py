@@ -423,7 +423,7 @@ class BaseLUTLayer(ABC, LUTLayerMixin, nn.Module):
                     return ops.dwn_layer_eval(x, ops.table_sigmoid(raw), plan)
             if self._fused == "hybrid":
                 return ops.hybrid_raw_layer(x, raw, plan)
-            return ops.dwn_stable_layer(x, ops.table_sigmoid(raw), self._banks["gradient_scale"].tensor().detach(), plan)
+            return ops.dwn_stable_raw_layer(x, raw, self._banks["gradient_scale"].tensor().detach(), plan)
         return None
 
     def _loop_nodes(self, mapped):

@@ -220,8 +220,7 @@ class ConvolutionalLayer(LUTLayerMixin, nn.Module):
             elif kind == "hybrid":
                 h = ops.hybrid_raw_layer(h, bank["raw_luts"], plan)
             else:
-                h = ops.dwn_stable_layer(h, ops.table_sigmoid(bank["raw_luts"]),
-                                                     bank["gradient_scale"].detach(), plan)
+                h = ops.dwn_stable_raw_layer(h, bank["raw_luts"], bank["gradient_scale"].detach(), plan)
         return h
 
     def _loop_trees(self, patches):

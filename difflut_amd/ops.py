@@ -429,6 +429,13 @@ def hybrid_layer(x, luts, plan):
     return HybridLayerFunction.apply(x, luts, plan, keep)
 
 
+def dwn_stable_raw_layer(x, raw, scale, plan):
+    """dwn_stable_layer(x, table_sigmoid(raw), scale, plan), as one operator."""
+    if not x.is_cuda:
+        return cpu_ops.dwn_stable_layer(x, table_sigmoid(raw), scale, plan)
+    return nat.host().dwn_stable_raw_layer(x, raw, scale, plan.host)
+
+
 def hybrid_raw_layer(x, raw, plan):
     """hybrid_layer(x, table_sigmoid(raw), plan), as one operator."""
     if not x.is_cuda:

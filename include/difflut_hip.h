@@ -272,6 +272,11 @@ int dl_dwn_stable_layer_bwd(const float *x, const void *saved, const int32_t *id
                             const float *luts, const float *gy, const float *gradient_scale,
                             float *gx, float *gluts, void *ws, size_t ws_bytes,
                             int B, int I, int N, int k, int O, void *stream);
+/* The same with the adjoint of the table sigmoid in it: luts = sigmoid(raw_luts), graw the gradient of raw_luts.  Refused
+ * (DL_ERR_UNSUPPORTED) where dl_dwn_bwd_reads_x is 1. */
+int dl_dwn_stable_raw_bwd(const void *saved, const int32_t *idx32, const int32_t *inv_ptr, const int32_t *inv_pos,
+                          const float *luts, const float *gy, const float *gradient_scale, float *gx, float *graw,
+                          void *ws, size_t ws_bytes, int B, int I, int N, int k, int O, void *stream);
 
 /* ------------------------------------------------------------------------
  * RandomLayer + hybrid nodes (node type "hybrid"): thresholded lookup forward (dl_table_sigmoid_fwd,

@@ -202,6 +202,31 @@ def test_hybrid_with_the_sigmoid_inside(shape, grads):
             torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("shape", SHAPES + [(64, 30, 16, 6, 1),     # one chunk of batch tiles: the histogram writes the gradient
+                                            (1500, 40, 50, 5, 2),   # several: their sum does
+                                            (4200, 20, 3, 4, 1),    # more than 64, summed by lanes
+                                            (70, 30, 9, 9, 1)])     # tables too long for either
+@pytest.mark.parametrize("grads", ["both", "tables"])
+def test_stable_with_the_sigmoid_inside(shape, grads):
+    """One operator on the raw tables against the two: the same bits (k > 8, atomic sums: up to their order)."""
+    B, I, N, k, O = shape
+    ops = _ops()
+    x, idx, raw, gy, _ = make_case(sum(shape) + 3, *shape)
+    plan = ops.MappingPlan(dev(idx, torch.int32), I)
+    scale = torch.linspace(0.5, 2.0, N, device=DEV)
+    got = []
+    for inside in (False, True):
+        xt, rt = dev(x).requires_grad_(grads == "both"), dev(raw).requires_grad_()
+        y = ops.dwn_stable_raw_layer(xt, rt, scale, plan) if inside else ops.dwn_stable_layer(xt, ops.table_sigmoid(rt), scale, plan)
+        y.backward(dev(gy.reshape(B, N * O)))
+        got.append((y.detach(), xt.grad, rt.grad))
+    for a, b in zip(*got):
+        if a is None or k <= 8:
+            assert (a is None and b is None) or torch.equal(a, b)
+        else:
+            torch.testing.assert_close(a, b, rtol=1e-5, atol=1e-5)
+
+
 @pytest.mark.parametrize("shape", [(66, 20, 30, 4, 1), (12, 30, 8, 7, 1)])
 def test_hybrid_binary_inputs_get_zero_gradient(shape):
     """x_j (1 - x_j) = 0 at a binary input, so the reference's factor (a_j - x_j) / (x_j (1 - x_j) + 1e-8)
