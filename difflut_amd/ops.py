@@ -171,12 +171,12 @@ class DWNLayerFunction:
     def apply(x, luts, plan, alpha, beta, beta_abs_max=None):
         """alpha, beta: Python floats for the whole layer, or device tensors [N] with every node's own values
         (then beta_abs_max = max |beta|, a host value)."""
+        nat.require_device(x, luts)
         if isinstance(alpha, torch.Tensor) or isinstance(beta, torch.Tensor):
             if any(isinstance(v, torch.Tensor) and v.dim() > 1 for v in (alpha, beta)):
                 raise RuntimeError("alpha and beta of a layer are numbers or tensors [N]")
             # (what a layer's bank hands over goes on as it is: the native side looks at it as _per_node would)
             if beta_abs_max is None or not (isinstance(alpha, torch.Tensor) and isinstance(beta, torch.Tensor)):
-                nat.require_device(x, luts)
                 alpha, beta = _per_node(alpha, plan.N, x.device), _per_node(beta, plan.N, x.device)
                 beta_abs_max = float(beta.abs().max()) if beta_abs_max is None else beta_abs_max
             return nat.host().dwn_layer(x, luts, plan.host, alpha, beta, 0.0, beta_abs_max)
@@ -289,6 +289,7 @@ class ProbLayerFunction:
 
     @staticmethod
     def apply(x, raw, plan, temperature):
+        nat.require_device(x, raw)
         if isinstance(temperature, torch.Tensor):
             return nat.host().prob_layer(x, raw, plan.host, plan.ordered, temperature, 0.0)
         return nat.host().prob_layer(x, raw, plan.host, plan.ordered, None, temperature)
