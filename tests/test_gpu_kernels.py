@@ -1417,3 +1417,27 @@ def test_grad_stabilize_against_the_reference_formula(per_row, subtract_mean):
     np.testing.assert_allclose(out.cpu().numpy(), want.cpu().numpy(), rtol=1e-5, atol=1e-6)
     again = _ops().grad_stabilize(g, per_row, 0.7, subtract_mean, 1e-8)
     assert torch.equal(out, again)  # fixed order of additions
+
+
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 5, 6])
+@pytest.mark.parametrize("B,N,O", [(63, 64, 1), (200, 301, 1), (129, 70, 3)])  # ragged rows, ragged wavefronts, stores by a node each
+def test_address_bytes_of_hidden_layers(k, B, N, O):
+    """The address of every node and row that a hidden layer of a chain keeps for its backward, against the inputs' bits."""
+    from difflut_amd import _native as nat
+
+    lib = nat.lib()
+    g = torch.Generator("cuda").manual_seed(B + k)
+    I = 90
+    idx = torch.randint(0, I, (N, k), device=DEV, generator=g, dtype=torch.int32)
+    luts = torch.randn(N, O, 1 << k, device=DEV, generator=g)
+    x = (torch.rand(B, I, device=DEV, generator=g) < 0.5).float()
+    tiles = (B + 63) // 64
+    planes, out = (torch.empty(lib.dl_dwn_planes_bytes(B, c), dtype=torch.uint8, device=DEV) for c in (I, N * O))
+    saved = torch.full((lib.dl_dwn_saved_bytes(B, I, N, k, O),), 77, dtype=torch.uint8, device=DEV)
+    nat.check(lib.dl_dwn_pack_planes(x.data_ptr(), planes.data_ptr(), B, I, nat.stream()))
+    nat.check(lib.dl_dwn_layer_fwd_planes(planes.data_ptr(), idx.data_ptr(), luts.data_ptr(), None, out.data_ptr(), saved.data_ptr(),
+                                          B, I, N, k, O, nat.stream()))
+    bits = torch.zeros(tiles * 64, I, dtype=torch.int64, device=DEV)
+    bits[:B] = x.long()
+    want = (bits[:, idx.long()] << torch.arange(k, device=DEV)).sum(-1).view(tiles, 64, N).transpose(1, 2)
+    assert torch.equal(saved[:tiles * N * 64].view(tiles, N, 64).long(), want)
