@@ -1583,8 +1583,9 @@ static void dwn_launch_lookup_wide(const u64 *planes, const int *idx32, const fl
 // columns, any B up to 4096 9 / 4; 2532 x 746 B = 64 10.0 / 6.0, 1024 11.3 / 7.6, 4096 21 / 21; 4096 x 4096 B = 64 9.9 / 7.6, 384 13.5 / 10.3, 768
 // 17.5 / 21.5; 8192 x 2000 B = 384 12.0 / 10.1, 1024 18.3 / 19.1; 8000 x 8000 B = 160 15.4 / 14.2, 256 15.0 / 16.5.  Wider inputs take
 // longer to turn than to pack: 16384 x 2000 B = 64 11.3 / 11.6, 256 11.7 / 15.7.
+// (65535: eights of rows are a grid dimension that a layer of a few columns would outgrow.)
 static inline bool dwn_few_rows(int B, int I, int N, int k, int O) {
-    return k <= DL_MAX_FAST_K && I <= 8192 && (double)B * (I + (double)N * O) <= 3.5e6;
+    return k <= DL_MAX_FAST_K && I <= 8192 && B <= 65535 && (double)B * (I + (double)N * O) <= 3.5e6;
 }
 // forward of the k <= 8 path: x -> bit-planes (scratch) -> y and the saved addresses
 static int dwn_forward_fast(const float *x, const int32_t *idx32, const float *luts, float *y, void *saved, u64 *planes,
@@ -2386,7 +2387,7 @@ __global__ __launch_bounds__(64 * DWN_GROUP_WAVES) void dwn_eval_groups(const u6
                                                         int NO, int O, int BT, int groups, int gsize, float inv_tau) {
     __shared__ int part[DWN_GROUP_WAVES][DWN_GROUP_TILES][64];
     const int lane = threadIdx.x & 63, wave = dl_uniform(threadIdx.x >> 6), waves = blockDim.x >> 6;
-    const int g = blockIdx.x, t0 = blockIdx.y * DWN_GROUP_TILES;
+    const int g = blockIdx.x % groups, t0 = (int)(blockIdx.x / groups) * DWN_GROUP_TILES;  // (tiles can outgrow the second dimension)
     const int c_lo = g * gsize, c_hi = min(NO, c_lo + gsize);
     int count[DWN_GROUP_TILES];
 #pragma unroll
@@ -2423,7 +2424,7 @@ template <int K>
 static void dwn_launch_eval_groups(const u64 *planes, const int *idx32, const float *luts, float *logits, int B, int I, int N, int O,
                                    int groups, int gsize, float tau, hipStream_t s) {
     const int BT = dwn_bt(B), pieces = dl_ceil_div(gsize, 64), waves = pieces < DWN_GROUP_WAVES ? pieces : DWN_GROUP_WAVES;
-    DL_TIMED("dwn_eval_groups", s, (dwn_eval_groups<K><<<dim3(groups, dl_ceil_div(BT, DWN_GROUP_TILES)), 64 * waves, 0, s>>>(
+    DL_TIMED("dwn_eval_groups", s, (dwn_eval_groups<K><<<(unsigned)groups * dl_ceil_div(BT, DWN_GROUP_TILES), 64 * waves, 0, s>>>(
                                        planes, idx32, luts, logits, B, I, N * O, O, BT, groups, gsize, 1.0f / tau)));
 }
 

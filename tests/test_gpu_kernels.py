@@ -1441,3 +1441,19 @@ def test_address_bytes_of_hidden_layers(k, B, N, O):
     bits[:B] = x.long()
     want = (bits[:, idx.long()] << torch.arange(k, device=DEV)).sum(-1).view(tiles, 64, N).transpose(1, 2)
     assert torch.equal(saved[:tiles * N * 64].view(tiles, N, 64).long(), want)
+
+
+def test_forward_of_a_narrow_layer_on_very_many_rows():
+    """A few columns on more rows than eight grid rows each could cover: y and the addresses against the bits."""
+    ops = _ops()
+    B, I, N, k = 8 * 65536 + 3, 3, 2, 2
+    g = torch.Generator("cuda").manual_seed(3)
+    x = (torch.rand(B, I, device=DEV, generator=g) < 0.5).float()
+    idx = torch.tensor([[0, 2], [1, 0]], dtype=torch.int32, device=DEV)
+    luts = torch.randn(N, 1, 1 << k, device=DEV, generator=g).requires_grad_()
+    y = ops.dwn_layer(x, luts, ops.MappingPlan(idx, I), 0.1, 0.1)
+    at = (x.long()[:, idx.long()] << torch.arange(k, device=DEV)).sum(-1)  # [B, N]
+    assert torch.equal(y, luts.detach()[:, 0].gather(1, at.t()).t())
+    y.backward(torch.ones_like(y))
+    # ones, added in single precision by quads of rows: whole numbers below 2^24, so exact
+    assert torch.equal(luts.grad[:, 0], torch.stack([torch.bincount(at[:, n], minlength=1 << k) for n in range(N)]).float())
