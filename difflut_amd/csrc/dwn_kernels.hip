@@ -648,7 +648,7 @@ __global__ __launch_bounds__(256) void dwn_bwd_transpose_hist(const float *__res
     for (int e = threadIdx.x; e < DWN_HC * ld; e += 256) hist[e] = 0.0f;
     const int t_begin = blockIdx.y * tiles_per_chunk;
     const int t_end = min(BT, t_begin + tiles_per_chunk);
-    const bool vec4 = NO % 4 == 0 && ((uintptr_t)gy & 15) == 0;  // (a piece of four columns is there or not)
+    const bool vec4 = NO % 4 == 0 && cend == DWN_HC && ((uintptr_t)gy & 15) == 0;
     const int q = threadIdx.x & 15, rr = threadIdx.x >> 4;  // 16 threads x 16 B cover one 64-column row piece
     const int N = NO / O;
     const int wc0 = wave * (DWN_HC / 4);  // my wavefront's first column
@@ -662,7 +662,6 @@ __global__ __launch_bounds__(256) void dwn_bwd_transpose_hist(const float *__res
             if (b < B) {
                 const float *src = gy + (size_t)b * NO + c0 + q * 4;
                 if (vec4) {
-                    if (q * 4 >= cend) continue;
                     typedef float f4v __attribute__((ext_vector_type(4)));
                     const f4v g4 = __builtin_nontemporal_load(reinterpret_cast<const f4v *>(src));  // gy is read once
                     pre[p] = make_float4(g4.x, g4.y, g4.z, g4.w);
