@@ -1533,11 +1533,14 @@ static void dwn_launch_lookup(const u64 *planes, const int *idx32, const float *
     const int BT = dwn_bt(B);
     const int grid = dl_xcd_grid(dl_ceil_div((long long)N * O, DWN_TC), BT);
     if (eval) {  // addrT is not written
-#define DWN_EVAL(O1_)                                                                                        \
-    DL_TIMED("dwn_lookup_eval", s, (dwn_lookup_fwd<K, O1_, true, false, true><<<grid, 64 * DWN_FW, 0, s>>>( \
-                                       planes, idx32, luts, y, addrT, planes_out, B, I, N, O, BT, 1, 1, run_if_set)))
-        if (O == 1) DWN_EVAL(true);
-        else DWN_EVAL(false);
+#define DWN_EVAL(O1_, CHAIN_, GSUM_)                                                                                     \
+    DL_TIMED("dwn_lookup_eval", s, (dwn_lookup_fwd<K, O1_, CHAIN_, GSUM_, true><<<grid, 64 * DWN_FW, 0, s>>>(            \
+                                       planes, idx32, luts, y, addrT, planes_out, B, I, N, O, BT, gsize > 0 ? gsize : 1, \
+                                       slots > 0 ? slots : 1, run_if_set)))
+        if (gsize > 0 && O == 1) DWN_EVAL(true, false, true);
+        else if (gsize > 0) DWN_EVAL(false, false, true);
+        else if (O == 1) DWN_EVAL(true, true, false);
+        else DWN_EVAL(false, true, false);
 #undef DWN_EVAL
         return;
     }
@@ -2419,6 +2422,17 @@ __global__ __launch_bounds__(64 * DWN_GROUP_WAVES) void dwn_eval_groups(const u6
         if (b < B) logits[(size_t)b * groups + g] = (float)sum * inv_tau;
     }
 }
+// Groups of up to 256 columns are half a pass of a block, which has a CU to itself (156 registers); a full pass is about 7 us.  Wider
+// groups take their passes one after the other, and with few groups or rows on few CUs, where the lookup - a block per 128 columns and
+// 64 rows, then a launch that adds - spreads over the chip: it stays where its time, 8 us and 0.075 per 1000 columns and tile, is less.
+// The head alone, us, lookup / bit-sliced: 8000 columns in 2 groups B = 1024 26 / 63, 5000 58 / 63, 8192 83 / 61; in 10 groups
+// B = 300 12 / 19, 1024 18 / 19, 2500 31 / 19; 4000 columns in one group B = 1024 20 / 63, 8192 53 / 63, 30000 146 / 62; 2000 in 2 groups
+// B = 2500 15 / 19, 5000 21 / 18; 4000 in 10 B = 300 9.9 / 10.9, 1000 in 10 B = 300 8.9 / 8.3, 8192 18 / 12.
+static inline bool dwn_groups_sliced(int B, int F, int groups, int gsize) {
+    const int passes = dl_ceil_div(gsize, 64 * DWN_GROUP_WAVES), BT = dwn_bt(B);
+    const long long rounds = ((long long)groups * dl_ceil_div(BT, DWN_GROUP_TILES) + 255) / 256;
+    return gsize <= 256 || 96 * passes * rounds < (long long)F * BT / 1000 + 46;
+}
 template <int K>
 static void dwn_launch_eval_groups(const u64 *planes, const int *idx32, const float *luts, float *logits, int B, int I, int N, int O,
                                    int groups, int gsize, float tau, hipStream_t s) {
@@ -2615,14 +2629,24 @@ extern "C" int dl_dwn_layer_eval_planes_groups(const void *planes_in, const int3
     if (ws_bytes < dl_dwn_groups_workspace_bytes(B, N, O, groups)) return DL_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
     const u64 *planes = (const u64 *)planes_in;
+    const bool sliced = dwn_groups_sliced(B, F, groups, gsize);
+    const auto head = [&](auto inputs) {
+        constexpr int K = decltype(inputs)::value;
+        if (sliced) dwn_launch_eval_groups<K>(planes, idx32, luts, logits, B, I, N, O, groups, gsize, tau, s);
+        else dwn_launch_lookup<K>(planes, idx32, luts, (float *)ws, (uint8_t *)const_cast<float *>(luts), nullptr, B, I, N, O, s, gsize, slots, true);
+    };
     switch (k) {
-        case 1: dwn_launch_eval_groups<1>(planes, idx32, luts, logits, B, I, N, O, groups, gsize, tau, s); break;
-        case 2: dwn_launch_eval_groups<2>(planes, idx32, luts, logits, B, I, N, O, groups, gsize, tau, s); break;
-        case 3: dwn_launch_eval_groups<3>(planes, idx32, luts, logits, B, I, N, O, groups, gsize, tau, s); break;
-        case 4: dwn_launch_eval_groups<4>(planes, idx32, luts, logits, B, I, N, O, groups, gsize, tau, s); break;
-        case 5: dwn_launch_eval_groups<5>(planes, idx32, luts, logits, B, I, N, O, groups, gsize, tau, s); break;
-        default: dwn_launch_eval_groups<6>(planes, idx32, luts, logits, B, I, N, O, groups, gsize, tau, s); break;
+        case 1: head(std::integral_constant<int, 1>{}); break;
+        case 2: head(std::integral_constant<int, 2>{}); break;
+        case 3: head(std::integral_constant<int, 3>{}); break;
+        case 4: head(std::integral_constant<int, 4>{}); break;
+        case 5: head(std::integral_constant<int, 5>{}); break;
+        default: head(std::integral_constant<int, 6>{}); break;
     }
+    if (!sliced)
+        DL_TIMED("dwn_group_finish", s,
+                 (dwn_group_finish<<<dl_ceil_div((long long)B * groups, 256), 256, 0, s>>>((const float *)ws, logits, B, dwn_bt(B) * 64, F,
+                                                                                         groups, gsize, slots, 1.0f / tau)));
     return dl_launch_status();
 }
 

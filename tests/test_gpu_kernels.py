@@ -650,6 +650,48 @@ def test_eval_of_few_rows(B, source, width, N, k, O, groups):
     torch.testing.assert_close(logits[0], logits[1], rtol=1e-5, atol=1e-4)
 
 
+def _kernels_of(call):
+    """The library kernels that `call` launches, from the library's record."""
+    from difflut_amd import _native as nat
+
+    nat.profile_read()
+    nat.profile_enable(True)
+    try:
+        call()
+        return [name for name, _ in nat.profile_read()]
+    finally:
+        nat.profile_enable(False)
+
+
+@pytest.mark.parametrize("B,N,k,O,groups,kernel", [
+    (300, 2560, 6, 1, 10, "dwn_eval_groups"),    # 256 columns a group
+    (100, 2570, 6, 1, 10, "dwn_lookup_eval"),    # 257: a pass of more wavefronts
+    (4000, 2570, 4, 1, 10, "dwn_eval_groups"),
+    (1100, 4000, 3, 1, 1, "dwn_lookup_eval"),    # eight passes of one block per tile
+    (9000, 2000, 2, 2, 2, "dwn_eval_groups"),    # four passes, many tiles
+    (1024, 1500, 5, 2, 2, "dwn_lookup_eval")])
+def test_eval_heads_of_wide_groups(B, N, k, O, groups, kernel):
+    """Bit-sliced, or by the lookup where a wide group would keep few blocks busy for many passes: whole numbers, exact."""
+    from difflut_amd import _native as nat
+
+    lib = nat.lib()
+    g = torch.Generator("cuda").manual_seed(B + N)
+    I, F = 500, N * O
+    idx = torch.randint(0, I, (N, k), device=DEV, generator=g, dtype=torch.int32)
+    luts = torch.randn(N, O, 1 << k, device=DEV, generator=g)
+    x = (torch.rand(B, I, device=DEV, generator=g) < 0.5).float()
+    planes = torch.empty(lib.dl_dwn_planes_bytes(B, I), dtype=torch.uint8, device=DEV)
+    nat.check(lib.dl_dwn_pack_planes(x.data_ptr(), planes.data_ptr(), B, I, nat.stream()))
+    y = torch.empty(B, F, device=DEV)
+    nat.check(lib.dl_dwn_layer_eval_planes(planes.data_ptr(), idx.data_ptr(), luts.data_ptr(), y.data_ptr(), None, B, I, N, k, O, nat.stream()))
+    logits = torch.full((B, groups), -1.0, device=DEV)
+    ws = torch.empty(lib.dl_dwn_groups_workspace_bytes(B, N, O, groups), dtype=torch.uint8, device=DEV)
+    ran = _kernels_of(lambda: nat.check(lib.dl_dwn_layer_eval_planes_groups(
+        planes.data_ptr(), idx.data_ptr(), luts.data_ptr(), logits.data_ptr(), ws.data_ptr(), ws.numel(), B, I, N, k, O, groups, 0.5, nat.stream())))
+    assert ran == ([kernel] if kernel == "dwn_eval_groups" else [kernel, "dwn_group_finish"])
+    assert torch.equal(logits, y.view(B, groups, F // groups).sum(2) * 2.0)
+
+
 @pytest.mark.parametrize("B", [1, 8, 65, 130])
 @pytest.mark.parametrize("I,N,k,O", [(64, 64, 6, 1), (100, 33, 3, 2), (8192, 1100, 4, 1), (8193, 40, 5, 1)])  # the last: planes
 def test_layer_forward_of_few_rows(B, I, N, k, O):
