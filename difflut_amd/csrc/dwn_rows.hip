@@ -17,6 +17,15 @@ __global__ __launch_bounds__(1024) void dwn_rows(DwnRows a, int span) {
     __shared__ float part[16][R];
     const int tid = threadIdx.x, b0 = blockIdx.y * R, rows = min(R, a.B - b0);
     const int NO = a.N * a.O, width = a.thr ? a.I / a.nbits : a.I;
+    const int c_lo = blockIdx.x * span, c_hi = min(NO, c_lo + span);
+    if (R == 8 && rows <= 0) {  // eight rows of the last tile that the batch does not have: zeros
+        for (int c = c_lo + tid; c < c_hi; c += blockDim.x) {
+            if (a.planes_out) a.planes_out[((size_t)(b0 >> 6) * NO + c) * 8 + ((b0 & 63) >> 3)] = 0;
+            if (a.saved && c % a.O == 0)
+                *reinterpret_cast<uint2 *>(a.saved + ((size_t)(b0 >> 6) * a.N + c / a.O) * 64 + (b0 & 63)) = make_uint2(0, 0);
+        }
+        return;
+    }
     if constexpr (!PLANES && R == 8) {
         const float *from = a.x + (size_t)b0 * width;
         for (int f = tid; f < width; f += blockDim.x) {
@@ -43,7 +52,6 @@ __global__ __launch_bounds__(1024) void dwn_rows(DwnRows a, int span) {
     float sum[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) sum[r] = 0.0f;
-    const int c_lo = blockIdx.x * span, c_hi = min(NO, c_lo + span);
     for (int c0 = c_lo; c0 < c_hi; c0 += blockDim.x) {
         const bool live = c0 + tid < c_hi;
         const int c = min(c0 + tid, c_hi - 1), n = c / a.O;
@@ -86,21 +94,14 @@ __global__ __launch_bounds__(1024) void dwn_rows(DwnRows a, int span) {
                 if (r < rows) a.y[(size_t)(b0 + r) * NO + c] = v[r];
         }
         if constexpr (R == 8) {
-            const bool last = blockIdx.y == gridDim.y - 1;  // the rows of its tile that the batch does not have are zeros
             const int at = b0 & 63;
-            if (a.planes_out) {
-                uint8_t *word = a.planes_out + ((size_t)(b0 >> 6) * NO + c) * 8;
-                word[at >> 3] = (uint8_t)ones;
-                for (int q = (at >> 3) + 1; last && q < 8; ++q) word[q] = 0;
-            }
+            if (a.planes_out) a.planes_out[((size_t)(b0 >> 6) * NO + c) * 8 + (at >> 3)] = (uint8_t)ones;
             if (a.saved && c == n * a.O) {
                 unsigned lo = 0, hi = 0;
 #pragma unroll
                 for (int r = 0; r < 8; ++r)
                     if (r < rows) (r < 4 ? lo : hi) |= addr[r] << (8 * (r & 3));
-                uint2 *bytes = reinterpret_cast<uint2 *>(a.saved + ((size_t)(b0 >> 6) * a.N + n) * 64 + at);
-                bytes[0] = make_uint2(lo, hi);
-                for (int q = (at >> 3) + 1; last && q < 8; ++q) *++bytes = make_uint2(0, 0);
+                *reinterpret_cast<uint2 *>(a.saved + ((size_t)(b0 >> 6) * a.N + n) * 64 + at) = make_uint2(lo, hi);
             }
         }
     }
@@ -124,7 +125,7 @@ __global__ __launch_bounds__(1024) void dwn_rows(DwnRows a, int span) {
 template <int K>
 static void dwn_rows_of(const DwnRows &a, hipStream_t s) {
     const int NO = a.N * a.O, width = a.thr ? a.I / a.nbits : a.I;
-    const int R = a.logits && !a.saved && a.B < 8 ? 1 : 8, by = dl_ceil_div(a.B, R);
+    const int R = a.logits && !a.saved && a.B < 8 ? 1 : 8, by = a.planes_out || a.saved ? (a.B + 63) / 64 * 8 : dl_ceil_div(a.B, R);
     // a thread per column, more where the input has more values to turn than that; blocks of 1024 share the columns as far as two
     // blocks per CU (of one group each: the groups)
     const int columns = a.logits ? a.gsize : NO;
