@@ -274,19 +274,9 @@ extern "C" int dl_fold(const float *gpatches, int tiled, float *gx, int B, int C
     if (rc) return rc;
     hipStream_t s = (hipStream_t)stream;
     const long long total = (long long)B * C * H * W;
-    if (tiled && SH == 1 && SW == 1 && total <= 0x7fffffffLL - 256 && (long long)B * g.OH * g.OW <= 0x7fffffffLL && KW <= 7) {
-#define CONV_FOLD(KW_) \
-    case KW_: DL_TIMED("conv_fold", s, (conv_fold_lines<KW_><<<dl_ceil_div(total, 256), 256, 0, s>>>(gpatches, gx, g, C * KH * KW_))); break
-        switch (KW) {
-            CONV_FOLD(1);
-            CONV_FOLD(2);
-            CONV_FOLD(3);
-            CONV_FOLD(4);
-            CONV_FOLD(5);
-            CONV_FOLD(6);
-            CONV_FOLD(7);
-        }
-#undef CONV_FOLD
+    if (tiled && SH == 1 && SW == 1 && total <= 0x7fffffffLL - 256 && (long long)B * g.OH * g.OW <= 0x7fffffffLL && (KW == 3 || KW == 5)) {
+        if (KW == 3) DL_TIMED("conv_fold", s, (conv_fold_lines<3><<<dl_ceil_div(total, 256), 256, 0, s>>>(gpatches, gx, g, C * KH * KW)));
+        else DL_TIMED("conv_fold", s, (conv_fold_lines<5><<<dl_ceil_div(total, 256), 256, 0, s>>>(gpatches, gx, g, C * KH * KW)));
         return dl_launch_status();
     }
     DL_TIMED("conv_fold", s, (conv_fold<<<dl_ceil_div(total, 256), 256, 0, s>>>(gpatches, gx, g, C * KH * KW, tiled)));
