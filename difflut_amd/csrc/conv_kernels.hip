@@ -142,27 +142,11 @@ __global__ __launch_bounds__(64 * CONV_BIT_WAVES) void conv_unfold_bits(const fl
         planes[((size_t)(r0 >> 6) + t) * cols + c] = word;  // (past the last row there are no lines)
     }
 }
-// Whether the words come sooner that way.  A block stages its images, 3.4 us per 128 words, before it makes a word, and then takes a turn of
-// 1024 words line by line; the votes take 0.18 us a word of a wavefront and nothing in front.  So few words, patches of one or two
-// columns, many channels and short lines (a word of 64 positions is many of them) are better voted on.  The terms are fitted to 267 sizes (1-64 channels,
-// 7-60 pixels, fields of 1-7, 1-256 images, both kernels): with the margin, none of those with lines of eight positions is slower by bits where the rule takes it.
-// us, votes / bits: 256 images of 4 x 28 x 28, field 5 30 / 12, field 1 7.7 / 9.7; 16 images of 3 x 16 x 16, field 3 5.2 / 6.9; 16 of 64 x 28 x 28, field
-// 2 18 / 41, field 5 90 / 65; 64 of 64 x 7 x 7, field 4 55 / 79.
-static inline bool conv_bits_pay(const ConvGeom &g, long long rows, int cols, int words, int tiles) {
-    const long long P = (long long)g.OH * g.OW, images = tiles * 64 / P + 2;
-    const double blocks = dl_ceil_div(rows, 64LL * tiles), rounds = dl_ceil_div((long long)blocks, 512);
-    const double trips = dl_ceil_div((images < g.B ? images : g.B) * words, 128);
-    const double turns = dl_ceil_div((long long)tiles * cols, 64 * CONV_BIT_WAVES) * (64.0 / g.OW + 1.0);
-    const double bits = 3.1 + (3.4 * rounds + 0.0002 * blocks) * trips + (0.016 * rounds + 0.0023 * blocks) * turns;
-    const double votes = 4.2 + cols * (0.045 + 0.00006 * dl_ceil_div(rows, 64));
-    return g.OW >= 8 && bits < 0.85 * votes;
-}
 // tiles per block, 0: not by bits
-static int conv_bit_tiles(const ConvGeom &g, long long rows, int cols, int words) {
+static int conv_bit_tiles(const ConvGeom &g, int words) {
     if (g.SH != 1 || g.SW != 1 || g.W + 2 * g.PW > 64) return 0;
     for (int tiles = 8; tiles > 0; tiles /= 2)
-        if (((long long)tiles * 64 / ((long long)g.OH * g.OW) + 2) * words <= CONV_BIT_WORDS)
-            return conv_bits_pay(g, rows, cols, words, tiles) ? tiles : 0;
+        if (((long long)tiles * 64 / ((long long)g.OH * g.OW) + 2) * words <= CONV_BIT_WORDS) return tiles;
     return 0;
 }
 
@@ -197,9 +181,8 @@ __global__ __launch_bounds__(256) void conv_fold(const float *__restrict__ gp, f
 }
 
 // The tile-major form at stride 1, patches KW wide: the positions of a line lie together, so the KW values of a line are asked for at
-// once; 32-bit arithmetic.  Bound by the reads of the gradient, each value once.  256 images of 4 x 28 x 28, fields of 1 to 7, us, a thread
-// that walks the patch / so: 7.2 / 5.2, 11 / 6.1, 18 / 8.0, 25 / 10, 34 / 13, 44 / 17, 56 / 20; wider ones, whose values would take more
-// registers than a thread that is alone with them should, keep the walk.
+// once; 32-bit arithmetic.  Bound by the reads of the gradient, each value once.  256 images of 4 x 28 x 28, 5 x 5 patches (59 MB):
+// 39 -> 15 us.
 template <int KW>
 __global__ __launch_bounds__(256) void conv_fold_lines(const float *__restrict__ gp, float *__restrict__ gx, ConvGeom g, int cols) {
     const int e = blockIdx.x * 256 + threadIdx.x;
@@ -256,10 +239,10 @@ extern "C" int dl_unfold_flip(const float *x, const uint8_t *flip, float *patche
     const long long rows = (long long)B * g.OH * g.OW;
     const int cols = C * KH * KW, grid = dl_ceil_div(rows, 64);
     if (patches) DL_TIMED("conv_unfold_rows", s, (conv_unfold_rows<<<grid, 256, 0, s>>>(x, patches, g, rows, cols, flip)));
-    const int words = dl_ceil_div((long long)C * H * W, 64), tiles = planes && !flip ? conv_bit_tiles(g, rows, cols, words) : 0;
+    const int words = dl_ceil_div((long long)C * H * W, 64), tiles = planes && !flip ? conv_bit_tiles(g, words) : 0;
     if (tiles) {
         const size_t lds = ((size_t)tiles * 64 / ((size_t)g.OH * g.OW) + 2) * words * sizeof(unsigned long long);
-        DL_TIMED("conv_unfold_bits", s, (conv_unfold_bits<<<dl_ceil_div(rows, 64LL * tiles), 64 * CONV_BIT_WAVES, lds, s>>>(
+        DL_TIMED("conv_unfold_planes", s, (conv_unfold_bits<<<dl_ceil_div(rows, 64LL * tiles), 64 * CONV_BIT_WAVES, lds, s>>>(
                                               x, (unsigned long long *)planes, g, rows, cols, tiles, words)));
     } else if (planes)
         DL_TIMED("conv_unfold_planes", s,
@@ -275,19 +258,9 @@ extern "C" int dl_fold(const float *gpatches, int tiled, float *gx, int B, int C
     if (rc) return rc;
     hipStream_t s = (hipStream_t)stream;
     const long long total = (long long)B * C * H * W;
-    if (tiled && SH == 1 && SW == 1 && total <= 0x7fffffffLL - 256 && (long long)B * g.OH * g.OW <= 0x7fffffffLL && KW <= 7) {
-#define CONV_FOLD(KW_) \
-    case KW_: DL_TIMED("conv_fold", s, (conv_fold_lines<KW_><<<dl_ceil_div(total, 256), 256, 0, s>>>(gpatches, gx, g, C * KH * KW_))); break
-        switch (KW) {
-            CONV_FOLD(1);
-            CONV_FOLD(2);
-            CONV_FOLD(3);
-            CONV_FOLD(4);
-            CONV_FOLD(5);
-            CONV_FOLD(6);
-            CONV_FOLD(7);
-        }
-#undef CONV_FOLD
+    if (tiled && SH == 1 && SW == 1 && total <= 0x7fffffffLL - 256 && (long long)B * g.OH * g.OW <= 0x7fffffffLL && (KW == 3 || KW == 5)) {
+        if (KW == 3) DL_TIMED("conv_fold", s, (conv_fold_lines<3><<<dl_ceil_div(total, 256), 256, 0, s>>>(gpatches, gx, g, C * KH * KW)));
+        else DL_TIMED("conv_fold", s, (conv_fold_lines<5><<<dl_ceil_div(total, 256), 256, 0, s>>>(gpatches, gx, g, C * KH * KW)));
         return dl_launch_status();
     }
     DL_TIMED("conv_fold", s, (conv_fold<<<dl_ceil_div(total, 256), 256, 0, s>>>(gpatches, gx, g, C * KH * KW, tiled)));

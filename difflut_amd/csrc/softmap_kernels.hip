@@ -875,10 +875,10 @@ __global__ __launch_bounds__(256, softmap_blocks(MODE, NP, FA)) void softmap_mfm
 #pragma unroll
         for (int i = 0; i < FA; ++i) {
             const int lr0 = wm + i * 32, row0 = r0 + lr0;
-            if (NP == 1 && i + 1 < FA) ask(i + 1, (i + 1) & 1);
+            if (NP != 1) ask(i, 0);  // (not earlier: the registers are the sums')
+            else if (i + 1 < FA) ask(i + 1, (i + 1) & 1);
 #pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                if (NP != 1 && j == 1) ask(i, 0);  // (not earlier: the registers are the sums')
+            for (int j = 0; j < 2; ++j)
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const float4 rv = *reinterpret_cast<const float4 *>(rr + lr0 + 8 * q + 4 * kh);
@@ -899,7 +899,6 @@ __global__ __launch_bounds__(256, softmap_blocks(MODE, NP, FA)) void softmap_mfm
 #pragma unroll
                     for (int n = 0; n < 4; ++n) stg[(8 * q + 4 * kh + n) * TS + j * 32 + l32] = o[n];
                 }
-            }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             __builtin_amdgcn_wave_barrier();
 #pragma unroll
