@@ -2653,6 +2653,10 @@ extern "C" int dl_dwn_layer_eval_planes_groups(const void *planes_in, const int3
     return dl_launch_status();
 }
 
+extern "C" int dl_dwn_rows_pay(int B, int width, int nbits, int N, int k, int O, int groups, int training) {
+    if (B <= 0 || width < 0 || nbits <= 0 || N <= 0 || O <= 0 || groups < 0 || !dwn_fast(N, k, O)) return 0;
+    return dwn_rows_pay(B, width, nbits, N * O, groups, training != 0);
+}
 // One launch for a layer on few rows (dwn_rows.hip).
 extern "C" int dl_dwn_layer_rows(const float *x, const float *thr, int nbits, const void *planes_in, const int32_t *idx32,
                                  const float *luts, void *planes_out, float *logits, void *saved, int B, int I, int N, int k, int O,

@@ -16,3 +16,5 @@ struct DwnRows {
 };
 // k <= DL_MAX_FAST_K
 void dwn_launch_rows(int k, const DwnRows &a, hipStream_t s);
+// 1 where dwn_launch_rows is the better launch for a layer of a chain: width features or values of x with nbits columns each, 0 planes in
+int dwn_rows_pay(int B, int width, int nbits, int NO, int groups, bool training);

@@ -122,25 +122,60 @@ __global__ __launch_bounds__(1024) void dwn_rows(DwnRows a, int span) {
     }
 }
 
-template <int K>
-static void dwn_rows_of(const DwnRows &a, hipStream_t s) {
-    const int NO = a.N * a.O, width = a.thr ? a.I / a.nbits : a.I;
-    const int R = a.logits && !a.saved && a.B < 8 ? 1 : 8, by = a.planes_out || a.saved ? (a.B + 63) / 64 * 8 : dl_ceil_div(a.B, R);
+struct DwnRowsGrid {
+    int R, by, bx, threads, span, blocks;  // rows and columns of a block; blocks that have rows
+};
+// width: features or values that a block turns, 0 with planes; groups: of a head, else 0
+static DwnRowsGrid dwn_rows_grid(int B, int width, int NO, int groups, bool planes_out, bool saved) {
+    DwnRowsGrid q;
+    q.R = groups && !saved && B < 8 ? 1 : 8;
+    const int rows_by = dl_ceil_div(B, q.R);
+    q.by = planes_out || saved ? (B + 63) / 64 * 8 : rows_by;
     // a thread per column, more where the input has more values to turn than that; blocks of 1024 share the columns as far as two
     // blocks per CU (of one group each: the groups)
-    const int columns = a.logits ? a.gsize : NO;
-    int threads = a.planes || R == 1 || columns > width ? columns : width;
-    if (a.logits && threads > 512 && (long long)a.groups * by > 256) threads = columns > 512 ? columns : 512;
-    threads = threads >= 1024 ? 1024 : (threads + 63) / 64 * 64;
-    int bx = a.groups, span = a.gsize;
-    if (!a.logits) {
+    const int columns = groups ? (NO + groups - 1) / groups : NO;
+    int threads = width == 0 || q.R == 1 || columns > width ? columns : width;
+    if (groups && threads > 512 && (long long)groups * q.by > 256) threads = columns > 512 ? columns : 512;
+    threads = q.threads = threads >= 1024 ? 1024 : (threads + 63) / 64 * 64;
+    int bx = groups, span = columns;
+    if (!groups) {
         bx = dl_ceil_div(NO, threads);
-        if (bx > 1 && (long long)bx * by > 512) bx = by >= 512 ? 1 : dl_ceil_div(512, by) < bx ? dl_ceil_div(512, by) : bx;
+        if (bx > 1 && (long long)bx * q.by > 512) bx = q.by >= 512 ? 1 : dl_ceil_div(512, q.by) < bx ? dl_ceil_div(512, q.by) : bx;
         span = dl_ceil_div(dl_ceil_div(NO, bx), threads) * threads;
         bx = dl_ceil_div(NO, span);
     }
+    q.bx = bx, q.span = span, q.blocks = bx * rows_by;
+    return q;
+}
+// Where it is the better launch of a chain.  us on the device, planes (code or pack, layer, sums of a head) / rows, nodes of six inputs,
+// 3136 inputs are 784 features with four thresholds; drawn from 4560 measurements for each of k = 6 and 3 (64-60000 features or
+// values, 300-8000 columns, heads of 1, 2 and 10 groups or none, 1-768 rows, inference and training).
+// - Fewer than eight rows asked for logits read x at its places: 1000 columns in 10 groups 11.6 / 4.1.  A block has a group: two
+//   passes of 1024 columns (8000 in one group 21 / 30).
+// - Planes in: only under a head, groups of up to 1024 columns (training 512), a million values: 1000 columns in 10 groups B = 64 8.7 / 4.5,
+//   768 9.2 / 6.2, 4000 in 2 groups B = 64 10 / 13.  A hidden layer is bit-sliced in 4.5-5 us and takes 7.6-13 here.
+// - x in: every block turns the whole input of its eight rows.  Up to 8192 inputs, and 1.5 million for all blocks: in 10 groups, B = 768,
+//   1000 columns of 3136 inputs 13.9 / 13.0, of 8000 values 21 / 38, of 60000 53 / 201.  Under a head also two passes and 1.6 million
+//   outputs: 3136 inputs, 4000 columns in 10 groups B = 64 13.8 / 8.1, 300 14.2 / 10.6, 768 16 / 17.  Without, 256 blocks: 4000 columns B = 64
+//   10.6 / 8.2, 300 10.9 / 8.8, 768 11.4 / 15.2.
+int dwn_rows_pay(int B, int width, int nbits, int NO, int groups, bool training) {
+    if (B > 768 || (long long)width * nbits > DL_DWN_ROWS_INPUTS) return 0;
+    const DwnRowsGrid q = dwn_rows_grid(B, width, NO, groups, !groups, training);
+    const int passes = dl_ceil_div(q.span, q.threads);
+    if (q.R == 1) return passes <= 2;
+    const double work = (double)B * NO;
+    if (width == 0) return groups && q.span <= (training ? 512 : 1024) && work <= 1e6;
+    if (width * nbits > 8192 || (double)q.blocks * width * nbits > 1.5e6) return 0;
+    return groups ? passes <= 2 && work <= 1.6e6 : q.blocks <= 256;
+}
+
+template <int K>
+static void dwn_rows_of(const DwnRows &a, hipStream_t s) {
+    const DwnRowsGrid q = dwn_rows_grid(a.B, a.planes ? 0 : a.thr ? a.I / a.nbits : a.I, a.N * a.O, a.logits ? a.groups : 0,
+                                        a.planes_out != nullptr, a.saved != nullptr);
+    const int R = q.R, threads = q.threads, span = q.span;
     const size_t lds = a.planes || R == 1 ? 0 : (size_t)a.I;
-    const dim3 grid(bx, by);
+    const dim3 grid(q.bx, q.by);
     if (a.planes && R == 8) DL_TIMED("dwn_rows", s, (dwn_rows<K, true, 8><<<grid, threads, 0, s>>>(a, span)));
     else if (a.planes) DL_TIMED("dwn_rows", s, (dwn_rows<K, true, 1><<<grid, threads, 0, s>>>(a, span)));
     else if (R == 8) DL_TIMED("dwn_rows", s, (dwn_rows<K, false, 8><<<grid, threads, lds, s>>>(a, span)));

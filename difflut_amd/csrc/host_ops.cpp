@@ -8,6 +8,7 @@
 // The conventions are those of the operators' Python side (difflut_amd/ops.py): inputs made contiguous fp32, outputs new
 // tensors, everything on torch's current stream, errors as RuntimeError, no synchronisation.
 #include <c10/hip/HIPStream.h>
+#include <climits>
 #include <dlfcn.h>
 #include <torch/extension.h>
 
@@ -32,7 +33,7 @@ namespace {
     X(dl_soft_map_saved_bytes) X(dl_soft_map_workspace_bytes) X(dl_soft_map_fwd) X(dl_soft_map_bwd) X(dl_unfold_rows)    \
     X(dl_unfold_flip) X(dl_fold) X(dl_dwn_planes_bytes) X(dl_dwn_tiled_bytes) X(dl_dwn_pack_planes)                      \
     X(dl_thermometer_planes) X(dl_dwn_groups_workspace_bytes) X(dl_dwn_layer_fwd_planes)                                 \
-    X(dl_dwn_layer_fwd_planes_groups) X(dl_dwn_layer_eval_planes) X(dl_dwn_layer_eval_planes_groups) X(dl_dwn_layer_rows) \
+    X(dl_dwn_layer_fwd_planes_groups) X(dl_dwn_layer_eval_planes) X(dl_dwn_layer_eval_planes_groups) X(dl_dwn_layer_rows) X(dl_dwn_rows_pay) \
     X(dl_dwn_layer_bwd_groups) X(dl_dwn_layer_bwd_tiled) X(dl_dwn_chain_fusable) X(dl_dwn_bwd_fused_workspace_bytes)     \
     X(dl_dwn_layer_bwd_chain_fused) X(dl_dwn_chain_first_fusable) X(dl_dwn_bwd_first_workspace_bytes)                    \
     X(dl_dwn_layer_bwd_chain_first) X(dl_cross_entropy_workspace_bytes) X(dl_cross_entropy) X(dl_adam_step)
@@ -446,18 +447,13 @@ Tensor first_planes(const Tensor &x, const Tensor &thresholds, const Tensor &fli
     width *= nbits;
     return planes;
 }
-// Up to so many rows, and rows times columns of all layers, a chain goes a launch per layer (dl_dwn_layer_rows), which saves the
-// first layer's planes and the last one's partial sums.  On the device, us, planes / rows (nodes of six inputs): inference, 2000 nodes B = 1
-// 11.4 / 3.5, 768 14.5 / 12.1, 2048 15.7 / 27; 7920 nodes B = 64 21.4 / 6.7, 384 22.5 / 13.3; 4000-2000 B = 512 19.2 / 14.6, 1024 20.0 / 23.3;
-// 8000-4000 B = 256 24.1 / 15.8, 512 24.7 / 25.6; training forward of one layer, 2000 nodes B = 256 12.9 / 8.0, 768 13.6 / 13.3, 1024
-// 13.5 / 15.7; 8000 nodes B = 64 15.5 / 7.6, 384 15.8 / 15.5, 512 15.9 / 21.1.
-constexpr int64_t ROWS_MOST = 768, ROWS_MOST_WORK = 3 << 20;
-bool few_rows(const Tensor &x, const Tensor &thresholds, at::ArrayRef<Tensor> luts, int64_t groups) {
-    if (x.dim() != 2 || x.size(0) > ROWS_MOST || (luts.size() == 1 && !groups)) return false;
-    int64_t columns = 0;
-    for (const Tensor &t : luts) columns += t.dim() == 3 ? t.size(0) * t.size(1) : 0;
-    const int64_t inputs = x.size(1) * (thresholds.defined() && thresholds.dim() == 2 ? thresholds.size(1) : 1);
-    return x.size(0) * columns <= ROWS_MOST_WORK && inputs <= DL_DWN_ROWS_INPUTS;
+// Whether a chain's first layer reads x itself, in one launch without planes (dl_dwn_layer_rows)
+bool first_by_rows(const Tensor &x, const Tensor &thresholds, at::ArrayRef<Tensor> luts, const Plan &p, int64_t groups, bool training) {
+    const Tensor &t = luts[0];
+    if (x.dim() != 2 || t.dim() != 3 || (thresholds.defined() && thresholds.dim() != 2) || (luts.size() == 1 && !groups)) return false;
+    const int64_t bits = thresholds.defined() ? thresholds.size(1) : 1;
+    if (x.size(0) > INT_MAX || x.size(1) > INT_MAX || bits > INT_MAX || x.size(1) == 0) return false;
+    return L.dl_dwn_rows_pay((int)x.size(0), (int)x.size(1), (int)bits, p.N, p.k, (int)t.size(1), luts.size() == 1 ? (int)groups : 0, training) == 1;
 }
 // where the first layer reads x itself: its rows and width, and the thresholds of its code (undefined: none)
 Tensor as_it_comes(const Tensor &x, const Tensor &thresholds, int &B, int &width, int &nbits) {
@@ -489,8 +485,7 @@ struct DwnStack : torch::autograd::Function<DwnStack> {
         int B = 0, width = 0, nbits = 1;
         st->encoded = thresholds->defined();
         Tensor planes, thr, y;
-        const bool rows = !st->patches && few_rows(x, *thresholds, luts, st->groups);
-        if (rows) thr = as_it_comes(x, *thresholds, B, width, nbits);
+        if (!st->patches && first_by_rows(x, *thresholds, luts, st->plans[0], st->groups, true)) thr = as_it_comes(x, *thresholds, B, width, nbits);
         else planes = first_planes(x, *thresholds, *flip, *st, B, width);
         variable_list save(luts.begin(), luts.end());
         for (size_t l = 0; l < luts.size(); ++l) {
@@ -499,8 +494,8 @@ struct DwnStack : torch::autograd::Function<DwnStack> {
             const bool last = l + 1 == luts.size();
             const Tensor kept = bytes(L.dl_dwn_saved_bytes(DIMS(d)), x);
             Tensor next;
-            if (rows && (st->groups || !last)) {
-                const bool first = !planes.defined();
+            const bool first = !planes.defined();  // reads x itself
+            if (first || (last && st->groups && L.dl_dwn_rows_pay(B, 0, 1, d.N, d.k, d.O, (int)st->groups, 1) == 1)) {
                 if (last) y = floats({B, st->groups}, x);
                 else next = bytes(L.dl_dwn_planes_bytes(B, d.N * d.O), x);
                 check(L.dl_dwn_layer_rows(first ? in(x) : nullptr, first ? in(thr) : nullptr, nbits, raw(planes), ints(p.idx),
@@ -740,8 +735,7 @@ Tensor dwn_stack_eval(const Tensor &x_, const Maybe &thresholds, const std::vect
     const size_t n = luts_.size();
     int B = 0, width = 0, nbits = 1;
     Tensor planes, thr, y;
-    const bool rows = few_rows(x, tensor_of(thresholds), luts_, groups);
-    if (rows) thr = as_it_comes(x, tensor_of(thresholds), B, width, nbits);
+    if (first_by_rows(x, tensor_of(thresholds), luts_, st->plans[0], groups, false)) thr = as_it_comes(x, tensor_of(thresholds), B, width, nbits);
     else planes = first_planes(x, tensor_of(thresholds), Tensor(), *st, B, width);
     for (size_t l = 0; l < n; ++l) {
         require_device(luts_[l]);
@@ -753,8 +747,8 @@ Tensor dwn_stack_eval(const Tensor &x_, const Maybe &thresholds, const std::vect
         if (head) y = floats({B, groups}, x);
         else if (last) y = floats({B, (int64_t)d.N * d.O}, x);
         else next = bytes(L.dl_dwn_planes_bytes(B, d.N * d.O), x);
-        if (rows && (head || !last)) {
-            const bool first = !planes.defined();
+        const bool first = !planes.defined();  // reads x itself
+        if (first || (head && L.dl_dwn_rows_pay(B, 0, 1, d.N, d.k, d.O, (int)groups, 0) == 1)) {
             check(L.dl_dwn_layer_rows(first ? in(x) : nullptr, first ? in(thr) : nullptr, nbits, raw(planes), ints(p.idx), in(lut),
                                            raw(next), head ? out(y) : nullptr, nullptr, DIMS(d), (int)groups, (float)tau, stream()));
         } else if (head) {

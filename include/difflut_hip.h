@@ -241,6 +241,9 @@ int dl_dwn_layer_eval_planes_groups(const void *planes_in, const int32_t *idx32,
  * [B, I] themselves (I <= DL_DWN_ROWS_INPUTS: a byte of LDS each).  Exactly one of x and planes_in, and of planes_out and logits [B, groups], is given.  saved
  * (dl_dwn_saved_bytes): training, as dl_dwn_layer_fwd_planes[_groups]; null: inference, as dl_dwn_layer_eval_planes[_groups]. */
 #define DL_DWN_ROWS_INPUTS 64512
+/* 1 where that launch is the better one: x [B, width] with nbits thresholds (1: values), or planes (width 0), under a head of `groups` (0:
+ * planes out), inference or training. */
+int dl_dwn_rows_pay(int B, int width, int nbits, int N, int k, int O, int groups, int training);
 int dl_dwn_layer_rows(const float *x, const float *thr, int nbits, const void *planes_in, const int32_t *idx32,
                       const float *luts, void *planes_out, float *logits, void *saved, int B, int I, int N, int k, int O,
                       int groups, float tau, void *stream);

@@ -692,6 +692,50 @@ def test_eval_heads_of_wide_groups(B, N, k, O, groups, kernel):
     assert torch.equal(logits, y.view(B, groups, F // groups).sum(2) * 2.0)
 
 
+@pytest.mark.parametrize("train", [False, True])
+@pytest.mark.parametrize("B,features,bits,widths,groups,first,launches", [
+    (100, 784, 4, (2000,), 10, "dwn_rows", 1),
+    (768, 6000, 1, (1000,), 10, "dwn_pack_planes", 1),       # every group's blocks would turn the whole input
+    (64, 5000, 2, (1000,), 10, "thermometer_planes", 1),     # 10 000 inputs
+    (64, 300, 1, (4000,), 1, "dwn_pack_planes", 0),          # four passes of a block
+    (200, 784, 4, (3000, 2000, 1000), 10, "dwn_rows", 2),    # not the hidden layer
+    (200, 784, 4, (3000, 2000), 0, "dwn_rows", 1),
+    (520, 3000, 1, (4000, 3000), 2, "dwn_pack_planes", 0)])  # 260 blocks
+def test_few_rows_of_a_chain_layer_by_layer(B, features, bits, widths, groups, first, launches, train):
+    """A launch per layer (dwn_rows) where that is the better one, layer by layer, and the results of the plane kernels: exact in
+    inference; in training a group's sum has up to 4000 values of size 1, added in another order."""
+    from difflut_amd import _native as nat
+    from difflut_amd import ops
+
+    g = torch.Generator("cuda").manual_seed(B + features)
+    x = torch.rand(B, features, device=DEV, generator=g)
+    thr = torch.rand(features, bits, device=DEV, generator=g).sort(1)[0].contiguous() if bits > 1 else None
+    plans, luts, width = [], [], features * bits
+    for n in widths:
+        plans.append(ops.MappingPlan(torch.randint(0, width, (n, 6), device=DEV, generator=g), width))
+        luts.append(torch.rand(n, 1, 64, device=DEV, generator=g) * 2 - 1)
+        width = n
+    got, hosts = [], [p.host for p in plans]
+    if train:
+        scalars = [(None, None, 0.1, 1 / 3)] * len(luts)
+        ran = _kernels_of(lambda: got.append(nat.host().dwn_stack(x, luts, hosts, scalars, thr, [], None, groups, 1.0)))
+    else:
+        ran = _kernels_of(lambda: got.append(nat.host().dwn_stack_eval(x, thr, luts, hosts, groups, 1.0)))
+    assert ran[0] == first and ran.count("dwn_rows") == launches
+    bits_in = (x[:, :, None] > thr[None] if thr is not None else x >= 0.5).view(B, -1)
+    for l, (plan, table) in enumerate(zip(plans, luts)):
+        addr = (bits_in[:, plan.idx32.long()].long() << torch.arange(6, device=DEV)).sum(2)
+        y = torch.gather(table[:, 0].expand(B, -1, -1), 2, addr[:, :, None])[:, :, 0]
+        bits_in = y >= 0.5
+    out = y if train else bits_in.float()
+    if groups:
+        out = out.double().view(B, groups, -1).sum(2).float()
+    if train and groups:
+        torch.testing.assert_close(got[0], out, rtol=1e-5, atol=1e-3)
+    else:
+        assert torch.equal(got[0], out)
+
+
 @pytest.mark.parametrize("B", [1, 8, 65, 130])
 @pytest.mark.parametrize("I,N,k,O", [(64, 64, 6, 1), (100, 33, 3, 2), (8192, 1100, 4, 1), (8193, 40, 5, 1)])  # the last: planes
 def test_layer_forward_of_few_rows(B, I, N, k, O):

@@ -551,3 +551,22 @@ def test_size_limits_and_argument_errors_are_reported_before_any_launch():
     assert lib.dl_dwn_layer_fwd_static(p, p, p, p, p, 4097, 16384, 8, 6, 1, None) == -6
     for code in (NULL, SHAPE, UNSUPPORTED, WORKSPACE, -5, -6):
         assert len(lib.dl_error_string(code)) > 10
+
+
+def test_where_a_chain_takes_a_layer_on_few_rows():
+    """dl_dwn_rows_pay: bounds on rows, inputs, blocks that each turn the whole input, and passes over wide groups."""
+    from difflut_amd import _native as nat
+    pay = nat.lib().dl_dwn_rows_pay
+    # B, width, nbits, N, k, O, groups, training
+    assert pay(1, 784, 4, 2000, 6, 1, 10, 0) == 1 and pay(256, 784, 4, 2000, 6, 1, 10, 1) == 1
+    assert pay(768, 784, 4, 2000, 6, 1, 10, 0) == 0 and pay(769, 8, 1, 100, 6, 1, 1, 0) == 0   # rows
+    assert pay(768, 60000, 1, 1000, 6, 1, 10, 0) == 0 and pay(16, 16000, 4, 1000, 6, 1, 10, 0) == 0  # inputs
+    assert pay(64, 8192, 1, 1000, 6, 1, 10, 1) == 1 and pay(64, 8193, 1, 1000, 6, 1, 10, 1) == 0
+    assert pay(400, 8000, 1, 1000, 6, 1, 10, 0) == 0                                               # blocks x inputs
+    assert pay(64, 784, 4, 4000, 6, 1, 1, 1) == 0 and pay(64, 784, 4, 4000, 6, 1, 2, 1) == 1      # passes
+    assert pay(3, 64512, 1, 2048, 6, 1, 1, 0) == 1 and pay(3, 64513, 1, 2048, 6, 1, 1, 0) == 0
+    assert pay(64, 0, 1, 4000, 6, 1, 0, 0) == 0                                                    # a hidden layer is bit-sliced
+    assert pay(64, 0, 1, 1024, 6, 1, 1, 0) == 1 and pay(64, 0, 1, 1024, 6, 1, 1, 1) == 0
+    for bad in ((0, 8, 1, 8, 2, 1, 1, 0), (4, -1, 1, 8, 2, 1, 1, 0), (4, 8, 0, 8, 2, 1, 1, 0), (4, 8, 1, 0, 2, 1, 1, 0), (4, 8, 1, 8, 7, 1, 1, 0)):
+        assert pay(*bad) == 0
+    assert pay(4, 2 ** 31 - 1, 2 ** 31 - 1, 8, 2, 1, 1, 0) == 0
