@@ -338,8 +338,15 @@ __global__ __launch_bounds__(256) void group_sum_bwd_kernel(const float *__restr
 // training configurations): one thread per row computes the row's loss (logsumexp - logit[label]) and the
 // gradient of the MEAN loss, (softmax - onehot) / B; a block adds its rows' losses, and where there are several blocks a single
 // one adds their sums, both in a fixed order.  Bound by the launches: 8192 rows of 10 logits 16 -> 9 us with sums of blocks in the
-// place of every row's loss; up to 1024 rows are one block and one launch, 256 rows 7.6 -> 5 us.
+// place of every row's loss.
+// One block and one launch, which writes the mean itself, where it is the only one anyhow (256 rows) and, up to 1024 rows, where its
+// logits stay in the L1 of its CU: 5120 of them, and no multiple of eight classes, whose rows fall on few of its sets.  One block
+// / blocks of 256 and their sum, us: 256 rows of 10 classes 6.6 / 7.8, of 100 54.9 / 55.9; 512 of 10 7.3 / 8.2, of 8 8.6 / 7.6, of 16 16.5 / 12.4, of
+// 100 100 / 57; 1024 of 5 5.5 / 6.6, of 10 11.3 / 8.8, of 100 212 / 58, of 1000 2422 / 609.
 #define CE_ONE 1024
+static inline bool cross_entropy_one(int B, int C) {
+    return B <= 256 || (B <= CE_ONE && C % 8 != 0 && (long long)B * C <= 5120);
+}
 template <int T>
 __device__ __forceinline__ float cross_entropy_sum(float mine) {  // of the block's threads, to thread 0
     __shared__ float part[T / 64];
@@ -499,7 +506,7 @@ extern "C" int dl_cross_entropy(const float *logits, const long long *labels, fl
     if (B <= 0 || C <= 0) return DL_ERR_SHAPE;
     if (ws_bytes < dl_cross_entropy_workspace_bytes(B)) return DL_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
-    if (B <= CE_ONE) {
+    if (cross_entropy_one(B, C)) {
         DL_TIMED("cross_entropy_rows", s,
                  (cross_entropy_rows<CE_ONE><<<1, (B + 63) / 64 * 64, 0, s>>>(logits, labels, (float *)ws, loss, glogits, B, C)));
         return dl_launch_status();

@@ -1389,6 +1389,26 @@ def test_cross_entropy_against_torch(shape):
         np.testing.assert_allclose(l2.item(), ref.item(), rtol=1e-6)
 
 
+@pytest.mark.parametrize("B,C,blocks", [(256, 100, 1), (257, 19, 1), (512, 10, 1), (1024, 5, 1),
+                                        (257, 20, 2), (512, 8, 2), (1024, 10, 4), (1024, 100, 4), (1000, 64, 4)])
+def test_cross_entropy_of_many_classes(B, C, blocks):
+    """One block only where its rows' logits stay in the L1 of a CU, and the same loss and gradient on either side of the line.  A row's
+    loss is within 2e-6 of its size, its gradient within 2e-7 / B of an exponential, a sum of C and a reciprocal."""
+    from difflut_amd import ops
+
+    g = torch.Generator("cuda").manual_seed(B + C)
+    z = torch.randn(B, C, device=DEV, generator=g)
+    labels = torch.randint(0, C, (B,), device=DEV, generator=g)
+    zt = z.clone().requires_grad_()
+    ran = _kernels_of(lambda: ops.CrossEntropyFunction.apply(zt, labels).backward())
+    assert ran.count("cross_entropy_rows") == 1 and ran.count("cross_entropy_mean") == (blocks > 1)
+    zr = z.double().cpu().requires_grad_()
+    want = torch.nn.functional.cross_entropy(zr, labels.cpu())
+    want.backward()
+    torch.testing.assert_close(ops.CrossEntropyFunction.apply(z, labels).double().cpu(), want.detach(), rtol=2e-6, atol=0)
+    torch.testing.assert_close(zt.grad.double().cpu(), zr.grad, rtol=1e-5, atol=1e-6 / B)
+
+
 @pytest.mark.parametrize("B,C", [(64, 2), (65, 3), (1024, 10), (1025, 10), (70000, 2)])
 def test_cross_entropy_blocks(B, C):
     """One block up to 1024 rows, sums of blocks beyond; the last has more blocks than the kernel that adds them has threads.  A
