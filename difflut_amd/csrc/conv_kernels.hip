@@ -142,11 +142,27 @@ __global__ __launch_bounds__(64 * CONV_BIT_WAVES) void conv_unfold_bits(const fl
         planes[((size_t)(r0 >> 6) + t) * cols + c] = word;  // (past the last row there are no lines)
     }
 }
+// Whether the words come sooner that way.  A block stages its images, 3.4 us per 128 words, before it makes a word, and then takes a turn of
+// 1024 words line by line; the votes take 0.18 us a word of a wavefront and nothing in front.  So few words, patches of one or two
+// columns, many channels and short lines (a word of 64 positions is many of them) are better voted on.  The terms are fitted to 267 sizes (1-64 channels,
+// 7-60 pixels, fields of 1-7, 1-256 images, both kernels): with the margin, none of those with lines of eight positions is slower by bits where the rule takes it.
+// us, votes / bits: 256 images of 4 x 28 x 28, field 5 30 / 12, field 1 7.7 / 9.7; 16 images of 3 x 16 x 16, field 3 5.2 / 6.9; 16 of 64 x 28 x 28, field
+// 2 18 / 41, field 5 90 / 65; 64 of 64 x 7 x 7, field 4 55 / 79.
+static inline bool conv_bits_pay(const ConvGeom &g, long long rows, int cols, int words, int tiles) {
+    const long long P = (long long)g.OH * g.OW, images = tiles * 64 / P + 2;
+    const double blocks = dl_ceil_div(rows, 64LL * tiles), rounds = dl_ceil_div((long long)blocks, 512);
+    const double trips = dl_ceil_div((images < g.B ? images : g.B) * words, 128);
+    const double turns = dl_ceil_div((long long)tiles * cols, 64 * CONV_BIT_WAVES) * (64.0 / g.OW + 1.0);
+    const double bits = 3.1 + (3.4 * rounds + 0.0002 * blocks) * trips + (0.016 * rounds + 0.0023 * blocks) * turns;
+    const double votes = 4.2 + cols * (0.045 + 0.00006 * dl_ceil_div(rows, 64));
+    return g.OW >= 8 && bits < 0.85 * votes;
+}
 // tiles per block, 0: not by bits
-static int conv_bit_tiles(const ConvGeom &g, int words) {
+static int conv_bit_tiles(const ConvGeom &g, long long rows, int cols, int words) {
     if (g.SH != 1 || g.SW != 1 || g.W + 2 * g.PW > 64) return 0;
     for (int tiles = 8; tiles > 0; tiles /= 2)
-        if (((long long)tiles * 64 / ((long long)g.OH * g.OW) + 2) * words <= CONV_BIT_WORDS) return tiles;
+        if (((long long)tiles * 64 / ((long long)g.OH * g.OW) + 2) * words <= CONV_BIT_WORDS)
+            return conv_bits_pay(g, rows, cols, words, tiles) ? tiles : 0;
     return 0;
 }
 
@@ -239,10 +255,10 @@ extern "C" int dl_unfold_flip(const float *x, const uint8_t *flip, float *patche
     const long long rows = (long long)B * g.OH * g.OW;
     const int cols = C * KH * KW, grid = dl_ceil_div(rows, 64);
     if (patches) DL_TIMED("conv_unfold_rows", s, (conv_unfold_rows<<<grid, 256, 0, s>>>(x, patches, g, rows, cols, flip)));
-    const int words = dl_ceil_div((long long)C * H * W, 64), tiles = planes && !flip ? conv_bit_tiles(g, words) : 0;
+    const int words = dl_ceil_div((long long)C * H * W, 64), tiles = planes && !flip ? conv_bit_tiles(g, rows, cols, words) : 0;
     if (tiles) {
         const size_t lds = ((size_t)tiles * 64 / ((size_t)g.OH * g.OW) + 2) * words * sizeof(unsigned long long);
-        DL_TIMED("conv_unfold_planes", s, (conv_unfold_bits<<<dl_ceil_div(rows, 64LL * tiles), 64 * CONV_BIT_WAVES, lds, s>>>(
+        DL_TIMED("conv_unfold_bits", s, (conv_unfold_bits<<<dl_ceil_div(rows, 64LL * tiles), 64 * CONV_BIT_WAVES, lds, s>>>(
                                               x, (unsigned long long *)planes, g, rows, cols, tiles, words)));
     } else if (planes)
         DL_TIMED("conv_unfold_planes", s,

@@ -115,6 +115,46 @@ def test_unfold_by_bits_and_fold_by_lines(case):
     test_unfold_rows_planes_and_fold(case)
 
 
+def _kernels_of(call):
+    """The library kernels that `call` launches, from the library's record."""
+    from difflut_amd import _native as nat
+    nat.profile_read()
+    nat.profile_enable(True)
+    try:
+        nat.check(call())
+        return {name for name, _ in nat.profile_read()}
+    finally:
+        nat.profile_enable(False)
+
+
+@pytest.mark.parametrize("case,by_bits", [
+    (((40, 4, 20, 60), (5, 5, 1, 1, 2, 2)), True),     # a padded row of 64 bits
+    (((90, 6, 12, 63), (3, 5, 1, 1, 1, 0)), True),     # lines that cross tiles everywhere
+    (((200, 8, 8, 12), (5, 5, 1, 1, 2, 0)), True),     # several images to a block, lines of eight positions
+    (((23, 30, 10, 9), (5, 5, 1, 1, 1, 2)), True),     # a last tile of 56 rows
+    (((6, 160, 24, 24), (5, 5, 1, 1, 0, 0)), True),    # an image of 1440 words: four tiles to a block
+    (((1, 40, 30, 30), (5, 5, 1, 1, 0, 0)), True),
+    (((256, 4, 28, 28), (1, 1, 1, 1, 0, 0)), False),   # few words to make
+    (((16, 1, 28, 28), (5, 5, 1, 1, 0, 0)), False),
+    (((64, 64, 7, 7), (4, 4, 1, 1, 0, 0)), False),     # short lines
+    (((16, 64, 28, 28), (2, 2, 1, 1, 0, 0)), False)])  # much to stage
+def test_unfold_by_bits_where_it_pays(case, by_bits):
+    """Plane words from the image's bits or by votes: the same as the patch matrix gives, and which of them ran."""
+    from difflut_amd import _native as nat
+    lib = nat.lib()
+    shape, geom = case
+    x = torch.rand(shape, device=DEV, generator=torch.Generator(DEV).manual_seed(sum(shape)))
+    rows, cols = lib.dl_unfold_rows(shape[0], shape[2], shape[3], *geom), shape[1] * geom[0] * geom[1]
+    patches = torch.empty(rows, cols, device=DEV)
+    want, got = (torch.full((lib.dl_dwn_planes_bytes(rows, cols),), 7, dtype=torch.uint8, device=DEV) for _ in range(2))
+    nat.check(lib.dl_unfold(x.data_ptr(), patches.data_ptr(), None, *shape, *geom, nat.stream()))
+    nat.check(lib.dl_dwn_pack_planes(patches.data_ptr(), want.data_ptr(), rows, cols, nat.stream()))
+    ran = _kernels_of(lambda: lib.dl_unfold(x.data_ptr(), None, got.data_ptr(), *shape, *geom, nat.stream()))
+    assert ran == {"conv_unfold_bits" if by_bits else "conv_unfold_planes"}
+    used = (rows + 63) // 64 * cols * 8
+    assert torch.equal(want[:used], got[:used])
+
+
 def test_unfold_rejects_bad_geometry():
     from difflut_amd import ops
     with pytest.raises(RuntimeError):
