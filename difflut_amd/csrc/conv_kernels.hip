@@ -197,8 +197,9 @@ __global__ __launch_bounds__(256) void conv_fold(const float *__restrict__ gp, f
 }
 
 // The tile-major form at stride 1, patches KW wide: the positions of a line lie together, so the KW values of a line are asked for at
-// once; 32-bit arithmetic.  Bound by the reads of the gradient, each value once.  256 images of 4 x 28 x 28, 5 x 5 patches (59 MB):
-// 39 -> 15 us.
+// once; 32-bit arithmetic.  Bound by the reads of the gradient, each value once.  256 images of 4 x 28 x 28, fields of 1 to 7, us, a thread
+// that walks the patch / so: 7.2 / 5.2, 11 / 6.1, 18 / 8.0, 25 / 10, 34 / 13, 44 / 17, 56 / 20; wider ones, whose values would take more
+// registers than a thread that is alone with them should, keep the walk.
 template <int KW>
 __global__ __launch_bounds__(256) void conv_fold_lines(const float *__restrict__ gp, float *__restrict__ gx, ConvGeom g, int cols) {
     const int e = blockIdx.x * 256 + threadIdx.x;
@@ -274,9 +275,19 @@ extern "C" int dl_fold(const float *gpatches, int tiled, float *gx, int B, int C
     if (rc) return rc;
     hipStream_t s = (hipStream_t)stream;
     const long long total = (long long)B * C * H * W;
-    if (tiled && SH == 1 && SW == 1 && total <= 0x7fffffffLL - 256 && (long long)B * g.OH * g.OW <= 0x7fffffffLL && (KW == 3 || KW == 5)) {
-        if (KW == 3) DL_TIMED("conv_fold", s, (conv_fold_lines<3><<<dl_ceil_div(total, 256), 256, 0, s>>>(gpatches, gx, g, C * KH * KW)));
-        else DL_TIMED("conv_fold", s, (conv_fold_lines<5><<<dl_ceil_div(total, 256), 256, 0, s>>>(gpatches, gx, g, C * KH * KW)));
+    if (tiled && SH == 1 && SW == 1 && total <= 0x7fffffffLL - 256 && (long long)B * g.OH * g.OW <= 0x7fffffffLL && KW <= 7) {
+#define CONV_FOLD(KW_) \
+    case KW_: DL_TIMED("conv_fold", s, (conv_fold_lines<KW_><<<dl_ceil_div(total, 256), 256, 0, s>>>(gpatches, gx, g, C * KH * KW_))); break
+        switch (KW) {
+            CONV_FOLD(1);
+            CONV_FOLD(2);
+            CONV_FOLD(3);
+            CONV_FOLD(4);
+            CONV_FOLD(5);
+            CONV_FOLD(6);
+            CONV_FOLD(7);
+        }
+#undef CONV_FOLD
         return dl_launch_status();
     }
     DL_TIMED("conv_fold", s, (conv_fold<<<dl_ceil_div(total, 256), 256, 0, s>>>(gpatches, gx, g, C * KH * KW, tiled)));

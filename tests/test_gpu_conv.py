@@ -155,6 +155,22 @@ def test_unfold_by_bits_where_it_pays(case, by_bits):
     assert torch.equal(want[:used], got[:used])
 
 
+@pytest.mark.parametrize("width", range(1, 9))
+def test_fold_of_every_width(width):
+    """Tile-major patch gradients, by lines up to a width of seven: the sums of the row-major form, in its order."""
+    from difflut_amd import _native as nat
+    lib = nat.lib()
+    shape, geom = (3, 2, 9, 13), (2, width, 1, 1, 1, width // 2)
+    rows, cols = lib.dl_unfold_rows(shape[0], shape[2], shape[3], *geom), shape[1] * geom[0] * geom[1]
+    g = torch.zeros((rows + 63) // 64 * 64, cols, device=DEV)
+    g[:rows] = torch.randn(rows, cols, device=DEV, generator=torch.Generator(DEV).manual_seed(width))
+    tiled = g.view(-1, 64, cols).transpose(1, 2).contiguous()
+    want, got = (torch.full(shape, 7.0, device=DEV) for _ in range(2))
+    nat.check(lib.dl_fold(g.data_ptr(), 0, want.data_ptr(), *shape, *geom, nat.stream()))
+    nat.check(lib.dl_fold(tiled.data_ptr(), 1, got.data_ptr(), *shape, *geom, nat.stream()))
+    assert torch.equal(want, got)
+
+
 def test_unfold_rejects_bad_geometry():
     from difflut_amd import ops
     with pytest.raises(RuntimeError):
