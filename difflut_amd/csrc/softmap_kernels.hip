@@ -569,9 +569,9 @@ __device__ __forceinline__ void softmap_stage_barrier() {
 // 128 x 128 tiles need 64, all that an L2 channel delivers.  Two or three blocks share a CU (accumulators 128 registers, 72 or 48 KB of LDS
 // each), so one block's MFMAs run under the other's barriers and stores.  Stages are KC deep, NBUF of them in the LDS.
 // Pairs (NP = 2): 128 x 128 tiles, because hi*hi and the rest have accumulators of their own (64 registers each) and the loop has
-// no vector arithmetic but the sign below; three blocks share a CU for gW, whose epilogue is two thirds memory (575 us before its reads were asked for ahead, 540 so; 704 with
+// no vector arithmetic but the sign below; three blocks share a CU for gW, whose epilogue is two thirds memory (575 us before its reads were asked for ahead, 510 so; 704 with
 // two).  Forward and gx add the sums of SM_PAIR_TURN stages to running ones, signs turned from group to group for the reason
-// given above, and have two blocks per CU.  The same sizes, forward / gx / gW: 503 / 473 / 575 us (planes 703 / 786 / 866).  Bound by power: the matrix cores are busy half of the time at 1.8 GHz.  256 x 128 tiles with one accumulator, the
+// given above, and have two blocks per CU.  The same sizes, forward / gx / gW: 475 / 448 / 510 us (planes 703 / 786 / 866).  Bound by power: the matrix cores are busy half of the time at 1.8 GHz.  256 x 128 tiles with one accumulator, the
 // rest's sum scaled and added by every stage: 514 / 560 / 668.  gx in
 // 5, 10 or 15 chunks of the reduction: 445, 486 and 497 with their sum; 10 for the shorter running sums.
 // NPB = 2 with NP = 3 (gx): gs in planes, E in pairs, whose planes - times 2^10, which makes their scale the planes' - are made on
@@ -782,7 +782,7 @@ __global__ __launch_bounds__(256, softmap_blocks(MODE, NP, FA)) void softmap_mfm
         if (NP == 2) rr[3 * TR + tid] = __int_as_float(-(softmap_pair_shift(g.range->x_largest) + softmap_pair_shift(g.row_max[r0 + tid])));
     }
     // what the epilogue reads of E or W for 32 rows of the wavefront's tile is asked for before the rows ahead of them are stored, E's first
-    // rows before the last stage: with the parts above, gW 316 -> 264 us (bf16 operands), 575 -> 540 (pairs)
+    // rows before the last stage: with the parts above, gW 316 -> 264 us (bf16 operands), 575 -> 510 (pairs)
     const int rrow = lane >> 4, c4 = (lane & 15) * 4, col4 = c0 + wn + c4;
     const bool vec = g.C % 4 == 0 && g.vec_out;
     uint2 e[2][NP == 1 ? 8 : 1];
@@ -875,10 +875,10 @@ __global__ __launch_bounds__(256, softmap_blocks(MODE, NP, FA)) void softmap_mfm
 #pragma unroll
         for (int i = 0; i < FA; ++i) {
             const int lr0 = wm + i * 32, row0 = r0 + lr0;
-            if (NP != 1) ask(i, 0);  // (not earlier: the registers are the sums')
-            else if (i + 1 < FA) ask(i + 1, (i + 1) & 1);
+            if (NP == 1 && i + 1 < FA) ask(i + 1, (i + 1) & 1);
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
+            for (int j = 0; j < 2; ++j) {
+                if (NP != 1 && j == 1) ask(i, 0);  // (not earlier: the registers are the sums', and in front of j = 0 eight spill: 535 us)
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const float4 rv = *reinterpret_cast<const float4 *>(rr + lr0 + 8 * q + 4 * kh);
@@ -899,6 +899,7 @@ __global__ __launch_bounds__(256, softmap_blocks(MODE, NP, FA)) void softmap_mfm
 #pragma unroll
                     for (int n = 0; n < 4; ++n) stg[(8 * q + 4 * kh + n) * TS + j * 32 + l32] = o[n];
                 }
+            }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             __builtin_amdgcn_wave_barrier();
 #pragma unroll
