@@ -46,6 +46,7 @@ SIGNATURES = {
     "dl_dwn_rows_pay": (_I, [_I] * 8),
     "dl_dwn_layer_rows": (_I, [_P, _P, _I, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _F, _P]),
     "dl_dwn_groups_workspace_bytes": (_Z, [_I] * 4),
+    "dl_dwn_eval_groups_workspace_bytes": (_Z, [_I] * 4),
     "dl_dwn_layer_fwd_planes_groups": (_I, [_P, _P, _P, _P, _P, _P, _Z, _I, _I, _I, _I, _I, _I, _F, _P]),
     "dl_dwn_layer_bwd_groups": (_I, [_P, _P, _P, _P, _P, _I, _F, _F, _F, _P, _I, _P, _P, _Z, _I, _I, _I, _I, _I, _P]),
     "dl_dwn_layer_bwd_chain_nodes": (_I, [_P, _P, _P, _P, _P, _I, _I, _F, _P, _P, _F, _P, _I, _P, _P, _Z, _I, _I, _I, _I, _I, _P]),

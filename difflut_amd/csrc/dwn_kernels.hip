@@ -2619,20 +2619,27 @@ extern "C" int dl_dwn_layer_eval_ws(const float *x, const int32_t *idx32, const 
     return dwn_generic_eval(x, idx32, luts, y, B, I, N, k, O, flag, s);
 }
 
+// what a head needs that goes through the lookup; the bit-sliced one needs nothing
+extern "C" size_t dl_dwn_eval_groups_workspace_bytes(int B, int N, int O, int groups) {
+    if (B <= 0 || N <= 0 || O <= 0 || groups <= 0 || (long long)N * O > 0x7fffffffLL) return 256;
+    const int F = N * O;
+    return dwn_groups_sliced(B, F, groups, dwn_group_size(F, groups)) ? 0 : dl_dwn_groups_workspace_bytes(B, N, O, groups);
+}
 extern "C" int dl_dwn_layer_eval_planes_groups(const void *planes_in, const int32_t *idx32, const float *luts,
                                                float *logits, void *ws, size_t ws_bytes, int B, int I, int N, int k, int O,
                                                int groups, float tau, void *stream) {
-    if (!planes_in || !idx32 || !luts || !logits || !ws) return DL_ERR_NULL;
+    if (!planes_in || !idx32 || !luts || !logits) return DL_ERR_NULL;
     int rc = dwn_check(B, I, N, k, O);
     if (rc) return rc;
     if (groups <= 0 || !(tau > 0.0f)) return DL_ERR_SHAPE;
     if (!dwn_fast(N, k, O)) return DL_ERR_UNSUPPORTED;
     const int F = N * O, gsize = dwn_group_size(F, groups), slots = dwn_group_slots(gsize);
     if (slots > DWN_GS_SLOTS) return DL_ERR_UNSUPPORTED;
-    if (ws_bytes < dl_dwn_groups_workspace_bytes(B, N, O, groups)) return DL_ERR_WORKSPACE;
+    const bool sliced = dwn_groups_sliced(B, F, groups, gsize);
+    if (!sliced && !ws) return DL_ERR_NULL;
+    if (ws_bytes < dl_dwn_eval_groups_workspace_bytes(B, N, O, groups)) return DL_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
     const u64 *planes = (const u64 *)planes_in;
-    const bool sliced = dwn_groups_sliced(B, F, groups, gsize);
     const auto head = [&](auto inputs) {
         constexpr int K = decltype(inputs)::value;
         if (sliced) dwn_launch_eval_groups<K>(planes, idx32, luts, logits, B, I, N, O, groups, gsize, tau, s);

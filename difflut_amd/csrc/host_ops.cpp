@@ -32,7 +32,7 @@ namespace {
     X(dl_prob_ordered_saved_bytes) X(dl_prob_ordered_bwd_workspace_bytes) X(dl_prob_ordered_fwd) X(dl_prob_ordered_bwd)  \
     X(dl_soft_map_saved_bytes) X(dl_soft_map_workspace_bytes) X(dl_soft_map_fwd) X(dl_soft_map_bwd) X(dl_unfold_rows)    \
     X(dl_unfold_flip) X(dl_fold) X(dl_dwn_planes_bytes) X(dl_dwn_tiled_bytes) X(dl_dwn_pack_planes)                      \
-    X(dl_thermometer_planes) X(dl_dwn_groups_workspace_bytes) X(dl_dwn_layer_fwd_planes)                                 \
+    X(dl_thermometer_planes) X(dl_dwn_groups_workspace_bytes) X(dl_dwn_eval_groups_workspace_bytes) X(dl_dwn_layer_fwd_planes)                                 \
     X(dl_dwn_layer_fwd_planes_groups) X(dl_dwn_layer_eval_planes) X(dl_dwn_layer_eval_planes_groups) X(dl_dwn_layer_rows) X(dl_dwn_rows_pay) \
     X(dl_dwn_layer_bwd_groups) X(dl_dwn_layer_bwd_tiled) X(dl_dwn_chain_fusable) X(dl_dwn_bwd_fused_workspace_bytes)     \
     X(dl_dwn_layer_bwd_chain_fused) X(dl_dwn_chain_first_fusable) X(dl_dwn_bwd_first_workspace_bytes)                    \
@@ -752,8 +752,9 @@ Tensor dwn_stack_eval(const Tensor &x_, const Maybe &thresholds, const std::vect
             check(L.dl_dwn_layer_rows(first ? in(x) : nullptr, first ? in(thr) : nullptr, nbits, raw(planes), ints(p.idx), in(lut),
                                            raw(next), head ? out(y) : nullptr, nullptr, DIMS(d), (int)groups, (float)tau, stream()));
         } else if (head) {
-            const Tensor ws = bytes(L.dl_dwn_groups_workspace_bytes(B, d.N, d.O, (int)groups), x);
-            check(L.dl_dwn_layer_eval_planes_groups(raw(planes), ints(p.idx), in(lut), out(y), raw(ws), ws.numel(), DIMS(d), (int)groups,
+            const size_t need = L.dl_dwn_eval_groups_workspace_bytes(B, d.N, d.O, (int)groups);
+            const Tensor ws = need ? bytes(need, x) : Tensor();
+            check(L.dl_dwn_layer_eval_planes_groups(raw(planes), ints(p.idx), in(lut), out(y), raw(ws), need, DIMS(d), (int)groups,
                                                     (float)tau, stream()));
         } else {
             check(L.dl_dwn_layer_eval_planes(raw(planes), ints(p.idx), in(lut), out(y), raw(next), DIMS(d), stream()));

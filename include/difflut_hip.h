@@ -229,10 +229,11 @@ int dl_dwn_layer_eval_ws(const float *x, const int32_t *idx32, const float *luts
  * dl_thermometer_planes / a preceding call write them; y (nullable) = (table entry >= 0.5) as 0/1 fp32
  * [B, N*O]; planes_out (nullable) = the same bits as planes for the next layer.  The *_groups form
  * returns GroupSum of that output instead (utils/modules.py:116-163; workspace
- * dl_dwn_groups_workspace_bytes, groups >= 64 columns wide).  No counterpart in the reference, which
+ * dl_dwn_eval_groups_workspace_bytes, null where that is 0; groups >= 64 columns wide).  No counterpart in the reference, which
  * runs its layers on [B, N] fp32 tensors in eval mode too.  k <= DL_MAX_FAST_K. */
 int dl_dwn_layer_eval_planes(const void *planes_in, const int32_t *idx32, const float *luts, float *y,
                              void *planes_out, int B, int I, int N, int k, int O, void *stream);
+size_t dl_dwn_eval_groups_workspace_bytes(int B, int N, int O, int groups);
 int dl_dwn_layer_eval_planes_groups(const void *planes_in, const int32_t *idx32, const float *luts, float *logits,
                                     void *ws, size_t ws_bytes, int B, int I, int N, int k, int O,
                                     int groups, float tau, void *stream);

@@ -685,9 +685,11 @@ def test_eval_heads_of_wide_groups(B, N, k, O, groups, kernel):
     y = torch.empty(B, F, device=DEV)
     nat.check(lib.dl_dwn_layer_eval_planes(planes.data_ptr(), idx.data_ptr(), luts.data_ptr(), y.data_ptr(), None, B, I, N, k, O, nat.stream()))
     logits = torch.full((B, groups), -1.0, device=DEV)
-    ws = torch.empty(lib.dl_dwn_groups_workspace_bytes(B, N, O, groups), dtype=torch.uint8, device=DEV)
+    need = lib.dl_dwn_eval_groups_workspace_bytes(B, N, O, groups)
+    assert (need == 0) == (kernel == "dwn_eval_groups")  # which writes the logits itself
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV) if need else None
     ran = _kernels_of(lambda: nat.check(lib.dl_dwn_layer_eval_planes_groups(
-        planes.data_ptr(), idx.data_ptr(), luts.data_ptr(), logits.data_ptr(), ws.data_ptr(), ws.numel(), B, I, N, k, O, groups, 0.5, nat.stream())))
+        planes.data_ptr(), idx.data_ptr(), luts.data_ptr(), logits.data_ptr(), nat.ptr(ws), need, B, I, N, k, O, groups, 0.5, nat.stream())))
     assert ran == ([kernel] if kernel == "dwn_eval_groups" else [kernel, "dwn_group_finish"])
     assert torch.equal(logits, y.view(B, groups, F // groups).sum(2) * 2.0)
 

@@ -570,3 +570,19 @@ def test_where_a_chain_takes_a_layer_on_few_rows():
     for bad in ((0, 8, 1, 8, 2, 1, 1, 0), (4, -1, 1, 8, 2, 1, 1, 0), (4, 8, 0, 8, 2, 1, 1, 0), (4, 8, 1, 0, 2, 1, 1, 0), (4, 8, 1, 8, 7, 1, 1, 0)):
         assert pay(*bad) == 0
     assert pay(4, 2 ** 31 - 1, 2 ** 31 - 1, 8, 2, 1, 1, 0) == 0
+
+
+def test_eval_head_workspace():
+    """A bit-sliced head needs none; the lookup's partial sums are refused what is missing or short."""
+    from difflut_amd import _native as nat
+    lib = nat.lib()
+    buf = ctypes.create_string_buffer(64)
+    p = ctypes.addressof(buf)
+    assert lib.dl_dwn_eval_groups_workspace_bytes(5001, 1000, 1, 10) == 0
+    need = lib.dl_dwn_eval_groups_workspace_bytes(1024, 4000, 1, 1)
+    assert need == lib.dl_dwn_groups_workspace_bytes(1024, 4000, 1, 1) > 0
+    args = (1024, 64, 4000, 6, 1, 1, 1.0, None)
+    assert lib.dl_dwn_layer_eval_planes_groups(p, p, p, p, None, need, *args) == -1
+    assert lib.dl_dwn_layer_eval_planes_groups(p, p, p, p, p, need - 1, *args) == -4
+    assert lib.dl_dwn_layer_eval_planes_groups(p, p, p, p, p, 0, 5001, 64, 400, 6, 1, 10, 1.0, None) == -3  # groups of 40 columns
+    assert lib.dl_dwn_eval_groups_workspace_bytes(0, 1000, 1, 10) == 256
