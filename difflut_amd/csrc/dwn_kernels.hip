@@ -470,9 +470,9 @@ __device__ __forceinline__ void dwn_table_block(const DwnTables &tb, int block) 
 // The D form of tables with 128 or 256 entries.  EFD: a wavefront per table, 2 or 4 doubles of it per lane, exchanged between lanes for
 // the lower six inputs and between registers for the others, no LDS and no barrier, so that these blocks ride in the histogram's
 // launch too.  |beta| <= 1/2: smoothed along every input once; the difference across bit j is then (1 - beta) times the D-form
-// value.  Other betas: smoothed along all inputs but j, for every j.  (A launch of its own with a block per table, the table in the
-// LDS and two barriers per input: 9.5 us for 2048 tables of 256, where these add 7.5 to the histogram's
-// 20.5, whose bins leave room for one block per CU; layer of 1024 rows, 4096 -> 2048 nodes of eight inputs 74 -> 72.6.)
+// value.  Other betas: smoothed along all inputs but j, for every j.  A launch of its own with a block per table, the table in the
+// LDS and two barriers per input, took 10 us for 2048 tables of 256 beside a histogram of 21; together they take 27.  Layer on the device,
+// forward and backward, us: 1024 rows, 4096 -> 2048 nodes of eight inputs 72.7 -> 70.6, of seven 58.1 -> 54.4; 256 rows, 512 -> 300 of eight 43 -> 39.
 template <int NR>
 __device__ __forceinline__ void dwn_wide_smooth(double (&v)[NR], double beta, int skip) {
 #pragma unroll
@@ -1559,7 +1559,7 @@ static void dwn_launch_lookup(const u64 *planes, const int *idx32, const float *
                                                                          N, O, BT)))
     const bool chain = planes_out != nullptr || y == nullptr;
     // up to 64 columns, blocks of as many wavefronts as they take: in one of eight the others wait
-    // (147456 rows x 32 columns 23 -> 12 us)
+    // (147456 rows x 32 columns 19 -> 10 us)
 #define DWN_NARROW(FW_)                                                                                                   \
     DL_TIMED("dwn_lookup_fwd", s,                                                                                         \
              (dwn_lookup_fwd<K, true, false, false, false, FW_><<<grid, 64 * FW_, 0, s>>>(planes, idx32, luts, y, addrT, nullptr, B, I, N, O, BT)))

@@ -571,7 +571,9 @@ __device__ __forceinline__ void softmap_stage_barrier() {
 // Pairs (NP = 2): 128 x 128 tiles, because hi*hi and the rest have accumulators of their own (64 registers each) and the loop has
 // no vector arithmetic but the sign below; three blocks share a CU for gW, whose epilogue is two thirds memory (575 us before its reads were asked for ahead, 510 so; 704 with
 // two).  Forward and gx add the sums of SM_PAIR_TURN stages to running ones, signs turned from group to group for the reason
-// given above, and have two blocks per CU.  The same sizes, forward / gx / gW: 475 / 448 / 510 us (planes 703 / 786 / 866).  Bound by power: the matrix cores are busy half of the time at 1.8 GHz.  256 x 128 tiles with one accumulator, the
+// given above, and have two blocks per CU.  The same sizes, forward / gx / gW: 475 / 448 / 510 us (planes 703 / 786 / 866).  Bound by the fills of the stages: a CU pulls 21-24 bytes
+// a clock, 48-82 lines in flight of 300-470 clocks each, and the matrix cores are busy 49 / 56 / 46 % of a clock that is 1.8 GHz (with bf16 operands
+// 2.15).  256 x 128 tiles with one accumulator, the
 // rest's sum scaled and added by every stage: 514 / 560 / 668.  gx in
 // 5, 10 or 15 chunks of the reduction: 445, 486 and 497 with their sum; 10 for the shorter running sums.
 // NPB = 2 with NP = 3 (gx): gs in planes, E in pairs, whose planes - times 2^10, which makes their scale the planes' - are made on

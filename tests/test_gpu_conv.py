@@ -108,10 +108,10 @@ def test_unfold_rows_planes_and_fold(case):
     ((40, 1, 5, 5), (5, 5, 1, 1, 2, 2)),
     ((2, 200, 16, 16), (3, 3, 1, 1, 1, 1)),  # an image of 800 words: fewer tiles to a block
     ((1, 300, 32, 32), (1, 1, 1, 1, 0, 0)),  # of 4800: not by bits
-    ((2, 4, 20, 20), (4, 4, 1, 1, 0, 0)),    # patches of a width without a fold of its own
+    ((2, 4, 20, 20), (4, 4, 1, 1, 0, 0)),
 ])
 def test_unfold_by_bits_and_fold_by_lines(case):
-    """The edges of the stride-1 forms."""
+    """The edges of the stride-1 forms; the planes are voted on at most of these sizes (by bits: test_unfold_by_bits_where_it_pays)."""
     test_unfold_rows_planes_and_fold(case)
 
 

@@ -1413,7 +1413,7 @@ def test_cross_entropy_of_many_classes(B, C, blocks):
 
 @pytest.mark.parametrize("B,C", [(64, 2), (65, 3), (1024, 10), (1025, 10), (70000, 2)])
 def test_cross_entropy_blocks(B, C):
-    """One block up to 1024 rows, sums of blocks beyond; the last has more blocks than the kernel that adds them has threads.  A
+    """One block, or sums of blocks; the last has more blocks than the kernel that adds them has threads.  A
     row's gradient is (p - 1) / B or p / B, p within 2e-7 (an exponential, a sum of C, a reciprocal); the loss a sum of B values of
     size up to 20 by halves: rtol 2e-6."""
     from difflut_amd.utils import cross_entropy
