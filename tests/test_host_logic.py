@@ -586,3 +586,45 @@ def test_eval_head_workspace():
     assert lib.dl_dwn_layer_eval_planes_groups(p, p, p, p, p, need - 1, *args) == -4
     assert lib.dl_dwn_layer_eval_planes_groups(p, p, p, p, p, 0, 5001, 64, 400, 6, 1, 10, 1.0, None) == -3  # groups of 40 columns
     assert lib.dl_dwn_eval_groups_workspace_bytes(0, 1000, 1, 10) == 256
+
+
+def _kernel_resources():
+    """{symbol: its metadata} of every kernel in the built library, from the notes of the code objects."""
+    import struct
+
+    from difflut_amd import _native as nat
+    msgpack = pytest.importorskip("msgpack")
+    nat.lib()
+    with open(nat.LIB_PATH, "rb") as f:
+        data = f.read()
+    kernels, magic = {}, b"__CLANG_OFFLOAD_BUNDLE__"
+    at = data.find(magic)
+    while at >= 0:
+        head, = struct.unpack_from("<Q", data, at + 24)
+        entry = at + 32
+        for _ in range(head):
+            offset, size, length = struct.unpack_from("<QQQ", data, entry)
+            target = data[entry + 24:entry + 24 + length]
+            entry += 24 + length
+            if b"gfx950" not in target or not size:
+                continue
+            elf = data[at + offset:at + offset + size]
+            table, step, count = struct.unpack_from("<Q", elf, 40)[0], *struct.unpack_from("<HH", elf, 58)
+            for s in range(count):
+                kind, = struct.unpack_from("<I", elf, table + s * step + 4)
+                if kind != 7:  # SHT_NOTE
+                    continue
+                start, _ = struct.unpack_from("<QQ", elf, table + s * step + 24)
+                name, desc, _ = struct.unpack_from("<III", elf, start)
+                note = start + 12 + (name + 3) // 4 * 4
+                for kernel in msgpack.unpackb(elf[note:note + desc], strict_map_key=False)["amdhsa.kernels"]:
+                    kernels[kernel[".name"]] = kernel
+        at = data.find(magic, at + 1)
+    assert kernels
+    return kernels
+
+
+def test_product_kernels_do_not_spill():
+    """gW's epilogue fits the registers that three blocks per CU leave."""
+    spilled = {n: k[".vgpr_spill_count"] for n, k in _kernel_resources().items() if "softmap" in n}
+    assert spilled and not any(spilled.values()), spilled
