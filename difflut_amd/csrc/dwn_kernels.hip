@@ -144,11 +144,15 @@ __global__ __launch_bounds__(64 * FW) void dwn_lookup_fwd(const u64 *__restrict_
     if (EVAL && run_if_set && *run_if_set == 0) return;  // the inputs were not all 0/1: the generic kernel answers
     constexpr int TC = FW * DWN_WC;
     __shared__ float tile[TC][65];  // [column][row]
-    __shared__ __align__(16) unsigned words[FW][2][DWN_WC * K];  // [wavefront][rows 0-31, 32-63][slot]
+    // the columns' plane words; of eight inputs half of the columns' at a time, since with all of them a CU holds three blocks instead
+    // of four (4096 rows, 6000 -> 8000 nodes, packing and lookup 118.5 -> 117 us; 4000 rows, 700 -> 5000 61.6 -> 58.7; 2000 rows,
+    // 3000 -> 2000 nodes with two outputs 31.2 -> 28.6)
+    constexpr int PC = K == 8 ? DWN_WC / 2 : DWN_WC, PARTS = DWN_WC / PC;
+    __shared__ __align__(16) unsigned words[FW][2][PC * K];  // [wavefront][rows 0-31, 32-63][slot]
     __shared__ u64 plane_tile[CHAIN ? TC : 1];  // thresholded outputs of the tile's columns, one bit per row
     __shared__ float gpart[GSUM ? FW : 1][GSUM ? DWN_GS_SLOTS : 1][64];  // [wavefront][slot][row]
     constexpr int L = 1 << K;
-    constexpr int NIDX = (DWN_WC * K + 63) / 64;  // index registers per lane
+    constexpr int NIDX = (PC * K + 63) / 64;  // words of a part per lane
     const int NO = N * O;
     int ctile, t;
     if (!dl_xcd_map((NO + TC - 1) / TC, BT, ctile, t)) return;
@@ -163,26 +167,29 @@ __global__ __launch_bounds__(64 * FW) void dwn_lookup_fwd(const u64 *__restrict_
     constexpr int NR = L > 64 ? L / 64 : 1;  // registers of a table
     const int cend = min(TC, NO - c0);
     const int wbeg = wave * DWN_WC;
-    // slot s = (column within my 16) * K + j  ->  lane s % 64 of register s / 64
-    {
-        u64 word[NIDX];
+    // slot s = (column within the part) * K + j  ->  lane s % 64 of register s / 64
+    u64 word[PARTS][NIDX];
+#pragma unroll
+    for (int p = 0; p < PARTS; ++p)
 #pragma unroll
         for (int v = 0; v < NIDX; ++v) {
             const int s = v * 64 + lane;
-            const int c = min(c0 + wbeg + min(s / K, DWN_WC - 1), NO - 1);
-            word[v] = pl[idx32[(O1 ? c : c / O) * K + s % K]];
+            const int c = min(c0 + wbeg + p * PC + min(s / K, PC - 1), NO - 1);
+            word[p][v] = pl[idx32[(O1 ? c : c / O) * K + s % K]];
         }
+    auto lay_out = [&](const u64 (&w)[NIDX]) __attribute__((always_inline)) {
 #pragma unroll
         for (int v = 0; v < NIDX; ++v) {
             const int s = v * 64 + lane;
-            if ((v + 1) * 64 <= DWN_WC * K || s < DWN_WC * K) {
-                words[wave][0][s] = (unsigned)word[v];
-                words[wave][1][s] = (unsigned)(word[v] >> 32);
+            if ((v + 1) * 64 <= PC * K || s < PC * K) {
+                words[wave][0][s] = (unsigned)w[v];
+                words[wave][1][s] = (unsigned)(w[v] >> 32);
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
-    }
+    };
+    lay_out(word[0]);
     const unsigned *mine = words[wave][lane >> 5];  // the words' half that holds my row
     const int my_bit = lane & 31;
     // FULL: all 128 columns of the tile exist (every tile but possibly the last): no clamps, no per-column checks,
@@ -194,6 +201,11 @@ __global__ __launch_bounds__(64 * FW) void dwn_lookup_fwd(const u64 *__restrict_
         for (int g = 0; g < DWN_WC; g += DWN_CG) {
             unsigned w[DWN_CG * K];
             float entry[DWN_CG][NR];
+            if (PARTS > 1 && g == PC) {  // the first half's words have been read
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                lay_out(word[PARTS - 1]);
+            }
 #pragma unroll
             for (int q = 0; q < DWN_CG; ++q) {
                 const int c = FULL ? c0 + wbeg + g + q : min(c0 + wbeg + g + q, NO - 1);
@@ -205,7 +217,7 @@ __global__ __launch_bounds__(64 * FW) void dwn_lookup_fwd(const u64 *__restrict_
             typedef unsigned u4v __attribute__((ext_vector_type(4)));
 #pragma unroll
             for (int v = 0; v < DWN_CG * K / 4; ++v) {
-                const u4v q4 = *reinterpret_cast<const u4v *>(mine + g * K + 4 * v);
+                const u4v q4 = *reinterpret_cast<const u4v *>(mine + g % PC * K + 4 * v);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) w[4 * v + e] = q4[e];
             }

@@ -628,3 +628,10 @@ def test_product_kernels_do_not_spill():
     """gW's epilogue fits the registers that three blocks per CU leave."""
     spilled = {n: k[".vgpr_spill_count"] for n, k in _kernel_resources().items() if "softmap" in n}
     assert spilled and not any(spilled.values()), spilled
+
+
+def test_lookup_blocks_that_a_cu_holds():
+    """Four (160 KB of LDS), whatever the number of inputs."""
+    lds = {n: k[".group_segment_fixed_size"] for n, k in _kernel_resources().items()
+           if "dwn_lookup_fwd" in n and "ELb0ELb0ELb0ELi8E" in n}
+    assert len(lds) == 16 and all(4 * size <= 160 << 10 for size in lds.values()), lds
