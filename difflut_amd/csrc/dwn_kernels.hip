@@ -2672,9 +2672,27 @@ extern "C" int dl_dwn_layer_eval_planes_groups(const void *planes_in, const int3
     return dl_launch_status();
 }
 
+// What few rows take under a head without dl_dwn_layer_rows, us on the device: the code or the packing (width > 0), then the training
+// lookup, the eval lookup or the bit-sliced head, and the sums of a lookup's head.  Fitted with dwn_rows_us to the same sizes, 8 % rms.
+static double dwn_planes_us(int B, int width, int nbits, int NO, int k, int groups, bool training) {
+    struct Terms { double launch, code, code_read, code_width, code_bits, columns, tables, group; };
+    constexpr Terms TRAINING = {6.97, 2.4, 0.19, 0.18, 0.028, 1.16, 1.91, 1.31}, LOOKUP = {6.54, 2.3, 0.23, 0.12, 0.032, 1.09, 2.15, 1.27},
+                    SLICED = {6.68, 2.35, 0.26, 0.02, 0.053, 0.0, 6.86, 0.55};
+    const int gsize = dwn_group_size(NO, groups), BT = dwn_bt(B);
+    const Terms t = training ? TRAINING : dwn_groups_sliced(B, NO, groups, gsize) ? SLICED : LOOKUP;
+    const double inputs = 1e-4 * width * nbits, columns = 1e-4 * NO;
+    return t.launch + (width ? t.code + BT * t.code_read * inputs + t.code_width * inputs + t.code_bits * nbits : 0.0) +
+           t.columns * columns * BT + t.tables * columns * (1 << k) / 64 + t.group * 1e-3 * gsize;
+}
+// Under a head one launch where it is the sooner one by 5 %.  Of the 16478 sizes it takes 1 % that are slower so by more than 5 % and leaves 2 %
+// that would be faster; on the average it is 1 % above the better of the two.  us, planes / rows, k = 6 if not stated, width x in to columns in groups: 3136 in (784
+// features) to 1000 in 10, B = 1 11.6 / 4.1, 768 13.9 / 13.0; 110 to 5841 in 3, k = 4, B = 325 16.4 / 8.4; 83 to 4778 in 2, k = 4, B = 2 12.4 / 5.3; 8000 values
+// to 1000 in 10, B = 768 21 / 38, 60000 53 / 201; planes in, 7830 in 10, k = 4, B = 75 11.3 / 7.5; 4000 in 2, B = 64 10 / 13.
 extern "C" int dl_dwn_rows_pay(int B, int width, int nbits, int N, int k, int O, int groups, int training) {
-    if (B <= 0 || width < 0 || nbits <= 0 || N <= 0 || O <= 0 || groups < 0 || !dwn_fast(N, k, O)) return 0;
-    return dwn_rows_pay(B, width, nbits, N * O, groups, training != 0);
+    if (B <= 0 || B > 768 || width < 0 || nbits <= 0 || (long long)width * nbits > DL_DWN_ROWS_INPUTS || groups < 0 || N <= 0 || O <= 0 || !dwn_fast(N, k, O)) return 0;
+    const int NO = N * O;
+    if (!groups) return dwn_rows_planes_pay(B, width, nbits, NO, training != 0);
+    return dwn_rows_us(B, width, nbits, NO, k, groups, training != 0) < 0.95 * dwn_planes_us(B, width, nbits, NO, k, groups, training != 0);
 }
 // One launch for a layer on few rows (dwn_rows.hip).
 extern "C" int dl_dwn_layer_rows(const float *x, const float *thr, int nbits, const void *planes_in, const int32_t *idx32,

@@ -16,5 +16,7 @@ struct DwnRows {
 };
 // k <= DL_MAX_FAST_K
 void dwn_launch_rows(int k, const DwnRows &a, hipStream_t s);
-// 1 where dwn_launch_rows is the better launch for a layer of a chain: width features or values of x with nbits columns each, 0 planes in
-int dwn_rows_pay(int B, int width, int nbits, int NO, int groups, bool training);
+// us of that launch under a head, and whether it is the better one for a layer that writes planes: width features or values of x with
+// nbits columns each, 0 planes in; up to DL_DWN_ROWS_INPUTS inputs
+double dwn_rows_us(int B, int width, int nbits, int NO, int k, int groups, bool training);
+bool dwn_rows_planes_pay(int B, int width, int nbits, int NO, bool training);

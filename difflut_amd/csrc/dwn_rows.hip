@@ -147,26 +147,31 @@ static DwnRowsGrid dwn_rows_grid(int B, int width, int NO, int groups, bool plan
     q.bx = bx, q.span = span, q.blocks = bx * rows_by;
     return q;
 }
-// Where it is the better launch of a chain.  us on the device, planes (code or pack, layer, sums of a head) / rows, nodes of six inputs,
-// 3136 inputs are 784 features with four thresholds; drawn from 4560 measurements for each of k = 6 and 3 (64-60000 features or
-// values, 300-8000 columns, heads of 1, 2 and 10 groups or none, 1-768 rows, inference and training).
-// - Fewer than eight rows asked for logits read x at its places: 1000 columns in 10 groups 11.6 / 4.1.  A block has a group: two
-//   passes of 1024 columns (8000 in one group 21 / 30).
-// - Planes in: only under a head, groups of up to 1024 columns (training 512), a million values: 1000 columns in 10 groups B = 64 8.7 / 4.5,
-//   768 9.2 / 6.2, 4000 in 2 groups B = 64 10 / 13.  A hidden layer is bit-sliced in 4.5-5 us and takes 7.6-13 here.
-// - x in: every block turns the whole input of its eight rows.  Up to 8192 inputs, and 1.5 million for all blocks: in 10 groups, B = 768,
-//   1000 columns of 3136 inputs 13.9 / 13.0, of 8000 values 21 / 38, of 60000 53 / 201.  Under a head also two passes and 1.6 million
-//   outputs: 3136 inputs, 4000 columns in 10 groups B = 64 13.8 / 8.1, 300 14.2 / 10.6, 768 16 / 17.  Without, 256 blocks: 4000 columns B = 64
-//   10.6 / 8.2, 300 10.9 / 8.8, 768 11.4 / 15.2.
-int dwn_rows_pay(int B, int width, int nbits, int NO, int groups, bool training) {
-    if (B > 768 || (long long)width * nbits > DL_DWN_ROWS_INPUTS) return 0;
-    const DwnRowsGrid q = dwn_rows_grid(B, width, NO, groups, !groups, training);
-    const int passes = dl_ceil_div(q.span, q.threads);
-    if (q.R == 1) return passes <= 2;
-    const double work = (double)B * NO;
-    if (width == 0) return groups && q.span <= (training ? 512 : 1024) && work <= 1e6;
-    if (width * nbits > 8192 || (double)q.blocks * width * nbits > 1.5e6) return 0;
-    return groups ? passes <= 2 && work <= 1.6e6 : q.blocks <= 256;
+// What the launch takes on the device as a layer under a head, us; the same arguments, width features or values of nbits columns each.  Terms:
+// a launch and its blocks' threads; the turn of a block's eight rows (width 0: none) and its passes over the columns, as often as blocks
+// follow one another on a CU; what all blocks read of x; outputs, and table entries, which of large tables come from further away.  Fitted to 16478 sizes (k = 2-6,
+// 1-768 rows, 8-64512 inputs, 200-8000 columns in 1-20 groups, both modes), 7-9 % rms.
+double dwn_rows_us(int B, int width, int nbits, int NO, int k, int groups, bool training) {
+    const DwnRowsGrid q = dwn_rows_grid(B, width, NO, groups, false, training);
+    const double passes = dl_ceil_div(q.span, q.threads), table = (1 << k) / 64.0, outputs = (double)B * NO * 1e-6, wide = q.threads / 1024.0;
+    if (q.R == 1) return 1.9 + wide + passes * (0.35 + 0.18 * k + (width ? 0.3 : 0.0)) + 9.6 * outputs;
+    const int in_lds = width ? (160 << 10) / (width * nbits + 512) : 32, per_cu = 2048 / q.threads < in_lds ? 2048 / q.threads : in_lds;
+    double rounds = q.blocks / (256.0 * (per_cu > 0 ? per_cu : 1));
+    if (rounds < 1.0) rounds = 1.0;
+    const double fill = q.blocks / 256.0 * wide, turned = rounds * passes, entries = 1e-4 * NO * table;
+    if (!width)
+        return 0.59 + 2.98 * wide + turned * (2.54 + 0.35 * table + (training ? 0.32 : 0.0)) + 1.04 * outputs * table + 2.34 * fill + 0.85 * entries;
+    return 1.54 + 2.38 * wide + rounds * dl_ceil_div(width, q.threads) * (0.34 + 0.1 * nbits) + turned * (1.62 + 0.09 * table + (training ? 0.43 : 0.0)) +
+           0.64e-6 * q.blocks * width * nbits + outputs * (0.67 + 0.42 * table) + 1.22 * fill + 0.59 * entries;
+}
+// Whether it is the better launch for a layer that writes planes.  A first one: every block turns the whole input of its eight rows, so
+// up to 8192 inputs, 1.5 million for all blocks and 256 blocks.  us on the device, code or packing and the layer / rows, nodes of six
+// inputs, 3136 inputs: 4000 columns B = 64 10.6 / 8.2, 300 10.9 / 8.8, 768 11.4 / 15.2.  Of 6662 measured sizes it takes 1 % that are slower so and
+// leaves 2 % that would be faster, by more than 5 %.  With planes in a hidden layer is bit-sliced in 4.5-5 us and would take 7.6-13.
+bool dwn_rows_planes_pay(int B, int width, int nbits, int NO, bool training) {
+    if (!width) return false;
+    const int blocks = dwn_rows_grid(B, width, NO, 0, true, training).blocks;
+    return width * nbits <= 8192 && (double)blocks * width * nbits <= 1.5e6 && blocks <= 256;
 }
 
 template <int K>

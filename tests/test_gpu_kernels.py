@@ -698,8 +698,10 @@ def test_eval_heads_of_wide_groups(B, N, k, O, groups, kernel):
 @pytest.mark.parametrize("B,features,bits,widths,groups,first,launches", [
     (100, 784, 4, (2000,), 10, "dwn_rows", 1),
     (768, 6000, 1, (1000,), 10, "dwn_pack_planes", 1),       # every group's blocks would turn the whole input
-    (64, 5000, 2, (1000,), 10, "thermometer_planes", 1),     # 10 000 inputs
-    (64, 300, 1, (4000,), 1, "dwn_pack_planes", 0),          # four passes of a block
+    (64, 6000, 8, (1000,), 10, "thermometer_planes", 1),     # 48 000 inputs
+    (64, 300, 1, (4000,), 1, "dwn_rows", 1),                 # four passes of a block
+    (5, 83, 3, (4779,), 3, "dwn_rows", 1),                   # two, in inference a row at a time
+    (768, 3000, 1, (8000,), 10, "dwn_pack_planes", 0),       # 960 blocks that read 23 million values, 6 million outputs
     (200, 784, 4, (3000, 2000, 1000), 10, "dwn_rows", 2),    # not the hidden layer
     (200, 784, 4, (3000, 2000), 0, "dwn_rows", 1),
     (520, 3000, 1, (4000, 3000), 2, "dwn_pack_planes", 0)])  # 260 blocks

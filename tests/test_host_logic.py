@@ -553,20 +553,31 @@ def test_size_limits_and_argument_errors_are_reported_before_any_launch():
         assert len(lib.dl_error_string(code)) > 10
 
 
+# B, width, nbits, N, k, O, groups, training; us on the device through planes / in one launch
+@pytest.mark.parametrize("call,planes,rows", [
+    ((1, 784, 4, 2000, 6, 1, 10, 0), 11.4, 3.5), ((256, 784, 4, 2000, 6, 1, 10, 1), 12.9, 8.0),
+    ((325, 55, 2, 5841, 4, 1, 3, 0), 16.4, 8.4), ((2, 83, 1, 4778, 4, 1, 2, 0), 12.4, 5.3),          # two and three passes
+    ((1, 109, 1, 5504, 6, 1, 1, 0), 16.6, 10.3), ((426, 669, 4, 3900, 6, 1, 3, 0), 14.0, 9.4),
+    ((456, 9, 4, 4580, 2, 1, 20, 1), 12.1, 8.6), ((161, 1550, 8, 442, 5, 1, 2, 1), 11.7, 8.8),       # 12400 inputs of few columns
+    ((75, 0, 1, 7830, 4, 1, 10, 1), 11.3, 7.5), ((97, 0, 1, 1734, 6, 1, 3, 1), 9.1, 6.9),            # planes in
+    ((768, 8000, 1, 1000, 6, 1, 10, 0), 21, 38), ((768, 60000, 1, 1000, 6, 1, 10, 0), 53, 201),      # blocks x inputs
+    ((64, 0, 1, 4000, 6, 1, 2, 0), 10, 13), ((17, 0, 1, 4481, 6, 1, 1, 0), 13.5, 24.2),              # passes, planes in
+])
+def test_where_a_chain_takes_a_head_on_few_rows(call, planes, rows):
+    """dl_dwn_rows_pay takes the launch that was measured to be the sooner one."""
+    from difflut_amd import _native as nat
+    assert nat.lib().dl_dwn_rows_pay(*call) == int(rows < planes)
+
+
 def test_where_a_chain_takes_a_layer_on_few_rows():
-    """dl_dwn_rows_pay: bounds on rows, inputs, blocks that each turn the whole input, and passes over wide groups."""
+    """dl_dwn_rows_pay: bounds on rows and inputs, and on the blocks of a first layer, which each turn the whole input."""
     from difflut_amd import _native as nat
     pay = nat.lib().dl_dwn_rows_pay
-    # B, width, nbits, N, k, O, groups, training
-    assert pay(1, 784, 4, 2000, 6, 1, 10, 0) == 1 and pay(256, 784, 4, 2000, 6, 1, 10, 1) == 1
-    assert pay(768, 784, 4, 2000, 6, 1, 10, 0) == 0 and pay(769, 8, 1, 100, 6, 1, 1, 0) == 0   # rows
-    assert pay(768, 60000, 1, 1000, 6, 1, 10, 0) == 0 and pay(16, 16000, 4, 1000, 6, 1, 10, 0) == 0  # inputs
-    assert pay(64, 8192, 1, 1000, 6, 1, 10, 1) == 1 and pay(64, 8193, 1, 1000, 6, 1, 10, 1) == 0
-    assert pay(400, 8000, 1, 1000, 6, 1, 10, 0) == 0                                               # blocks x inputs
-    assert pay(64, 784, 4, 4000, 6, 1, 1, 1) == 0 and pay(64, 784, 4, 4000, 6, 1, 2, 1) == 1      # passes
-    assert pay(3, 64512, 1, 2048, 6, 1, 1, 0) == 1 and pay(3, 64513, 1, 2048, 6, 1, 1, 0) == 0
+    assert pay(769, 8, 1, 100, 6, 1, 1, 0) == 0 and pay(1, 8, 1, 100, 6, 1, 1, 0) == 1                # rows
+    assert pay(3, 64512, 1, 2048, 6, 1, 1, 0) == 1 and pay(3, 64513, 1, 2048, 6, 1, 1, 0) == 0        # inputs: a byte of LDS each
+    assert pay(64, 8192, 1, 1000, 6, 1, 0, 1) == 1 and pay(64, 8193, 1, 1000, 6, 1, 0, 1) == 0
+    assert pay(300, 784, 4, 4000, 6, 1, 0, 0) == 1 and pay(768, 784, 4, 4000, 6, 1, 0, 0) == 0
     assert pay(64, 0, 1, 4000, 6, 1, 0, 0) == 0                                                    # a hidden layer is bit-sliced
-    assert pay(64, 0, 1, 1024, 6, 1, 1, 0) == 1 and pay(64, 0, 1, 1024, 6, 1, 1, 1) == 0
     for bad in ((0, 8, 1, 8, 2, 1, 1, 0), (4, -1, 1, 8, 2, 1, 1, 0), (4, 8, 0, 8, 2, 1, 1, 0), (4, 8, 1, 0, 2, 1, 1, 0), (4, 8, 1, 8, 7, 1, 1, 0)):
         assert pay(*bad) == 0
     assert pay(4, 2 ** 31 - 1, 2 ** 31 - 1, 8, 2, 1, 1, 0) == 0
