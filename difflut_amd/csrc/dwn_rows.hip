@@ -167,9 +167,11 @@ double dwn_rows_us(int B, int width, int nbits, int NO, int k, int groups, bool 
 // Whether it is the better launch for a layer that writes planes.  A first one: every block turns the whole input of its eight rows, so
 // up to 8192 inputs, 1.5 million for all blocks and 256 blocks.  us on the device, code or packing and the layer / rows, nodes of six
 // inputs, 3136 inputs: 4000 columns B = 64 10.6 / 8.2, 300 10.9 / 8.8, 768 11.4 / 15.2.  Of 6662 measured sizes it takes 1 % that are slower so and
-// leaves 2 % that would be faster, by more than 5 %.  With planes in a hidden layer is bit-sliced in 4.5-5 us and would take 7.6-13.
+// leaves 2 % that would be faster, by more than 5 %.  With planes in, hidden layers of one block's few columns: up to 384, in training 512.  Any B up to
+// 768, k = 2-6, bit-sliced or looked up / rows: 64-150 columns 4.1 / 3.1 and 4.8 / 3.2, 320-384 4.1 / 3.75 and 4.8 / 3.9, 384-448 4.2 / 4.0, 448-512 4.1 / 4.2
+// and 4.8 / 4.3, 600-1200 4.2 / 5.4 and 4.9 / 5.7.
 bool dwn_rows_planes_pay(int B, int width, int nbits, int NO, bool training) {
-    if (!width) return false;
+    if (!width) return NO <= (training ? 512 : 384);
     const int blocks = dwn_rows_grid(B, width, NO, 0, true, training).blocks;
     return width * nbits <= 8192 && (double)blocks * width * nbits <= 1.5e6 && blocks <= 256;
 }

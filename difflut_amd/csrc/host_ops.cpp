@@ -495,7 +495,7 @@ struct DwnStack : torch::autograd::Function<DwnStack> {
             const Tensor kept = bytes(L.dl_dwn_saved_bytes(DIMS(d)), x);
             Tensor next;
             const bool first = !planes.defined();  // reads x itself
-            if (first || (last && st->groups && L.dl_dwn_rows_pay(B, 0, 1, d.N, d.k, d.O, (int)st->groups, 1) == 1)) {
+            if (first || ((!last || st->groups) && L.dl_dwn_rows_pay(B, 0, 1, d.N, d.k, d.O, last ? (int)st->groups : 0, 1) == 1)) {
                 if (last) y = floats({B, st->groups}, x);
                 else next = bytes(L.dl_dwn_planes_bytes(B, d.N * d.O), x);
                 check(L.dl_dwn_layer_rows(first ? in(x) : nullptr, first ? in(thr) : nullptr, nbits, raw(planes), ints(p.idx),
@@ -748,7 +748,7 @@ Tensor dwn_stack_eval(const Tensor &x_, const Maybe &thresholds, const std::vect
         else if (last) y = floats({B, (int64_t)d.N * d.O}, x);
         else next = bytes(L.dl_dwn_planes_bytes(B, d.N * d.O), x);
         const bool first = !planes.defined();  // reads x itself
-        if (first || (head && L.dl_dwn_rows_pay(B, 0, 1, d.N, d.k, d.O, (int)groups, 0) == 1)) {
+        if (first || ((head || !last) && L.dl_dwn_rows_pay(B, 0, 1, d.N, d.k, d.O, head ? (int)groups : 0, 0) == 1)) {
             check(L.dl_dwn_layer_rows(first ? in(x) : nullptr, first ? in(thr) : nullptr, nbits, raw(planes), ints(p.idx), in(lut),
                                            raw(next), head ? out(y) : nullptr, nullptr, DIMS(d), (int)groups, (float)tau, stream()));
         } else if (head) {

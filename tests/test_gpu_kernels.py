@@ -703,6 +703,8 @@ def test_eval_heads_of_wide_groups(B, N, k, O, groups, kernel):
     (5, 83, 3, (4779,), 3, "dwn_rows", 1),                   # two, in inference a row at a time
     (768, 3000, 1, (8000,), 10, "dwn_pack_planes", 0),       # 960 blocks that read 23 million values, 6 million outputs
     (200, 784, 4, (3000, 2000, 1000), 10, "dwn_rows", 2),    # not the hidden layer
+    (200, 784, 4, (3000, 380, 1000), 10, "dwn_rows", 3),
+    (77, 6000, 8, (300, 200, 100), 0, "thermometer_planes", 2),
     (200, 784, 4, (3000, 2000), 0, "dwn_rows", 1),
     (520, 3000, 1, (4000, 3000), 2, "dwn_pack_planes", 0)])  # 260 blocks
 def test_few_rows_of_a_chain_layer_by_layer(B, features, bits, widths, groups, first, launches, train):

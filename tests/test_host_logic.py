@@ -577,7 +577,9 @@ def test_where_a_chain_takes_a_layer_on_few_rows():
     assert pay(3, 64512, 1, 2048, 6, 1, 1, 0) == 1 and pay(3, 64513, 1, 2048, 6, 1, 1, 0) == 0        # inputs: a byte of LDS each
     assert pay(64, 8192, 1, 1000, 6, 1, 0, 1) == 1 and pay(64, 8193, 1, 1000, 6, 1, 0, 1) == 0
     assert pay(300, 784, 4, 4000, 6, 1, 0, 0) == 1 and pay(768, 784, 4, 4000, 6, 1, 0, 0) == 0
-    assert pay(64, 0, 1, 4000, 6, 1, 0, 0) == 0                                                    # a hidden layer is bit-sliced
+    for training, most in ((0, 384), (1, 512)):                                                    # wider hidden layers are bit-sliced
+        assert pay(768, 0, 1, most, 6, 1, 0, training) == 1 and pay(1, 0, 1, most + 1, 6, 1, 0, training) == 0
+        assert pay(64, 0, 1, most // 2, 6, 2, 0, training) == 1 and pay(64, 0, 1, most // 2 + 1, 6, 2, 0, training) == 0
     for bad in ((0, 8, 1, 8, 2, 1, 1, 0), (4, -1, 1, 8, 2, 1, 1, 0), (4, 8, 0, 8, 2, 1, 1, 0), (4, 8, 1, 0, 2, 1, 1, 0), (4, 8, 1, 8, 7, 1, 1, 0)):
         assert pay(*bad) == 0
     assert pay(4, 2 ** 31 - 1, 2 ** 31 - 1, 8, 2, 1, 1, 0) == 0
