@@ -142,20 +142,21 @@ __global__ __launch_bounds__(64 * CONV_BIT_WAVES) void conv_unfold_bits(const fl
         planes[((size_t)(r0 >> 6) + t) * cols + c] = word;  // (past the last row there are no lines)
     }
 }
-// Whether the words come sooner that way.  A block stages its images, 3.4 us per 128 words, before it makes a word, and then takes a turn of
-// 1024 words line by line; the votes take 0.18 us a word of a wavefront and nothing in front.  So few words, patches of one or two
-// columns, many channels and short lines (a word of 64 positions is many of them) are better voted on.  The terms are fitted to 267 sizes (1-64 channels,
-// 7-60 pixels, fields of 1-7, 1-256 images, both kernels): with the margin, none of those with lines of eight positions is slower by bits where the rule takes it.
+// Whether the words come sooner that way.  A block stages its images, 2.4 us per 128 words, before it makes a word, and then takes a turn of
+// 1024 words line by line; the votes take 0.19 us a word of a wavefront and nothing in front.  So few words, patches of one or two
+// columns and many channels on many blocks are better voted on, and few rows of many columns, where the votes have few wavefronts, are not.
+// The terms are fitted to 2269 sizes (1-64 channels, 5-60 pixels, fields of 1-7, 1-256 images, both kernels; 11 and 9 % rms): 2 % of them are slower by bits
+// by more than 5 % where the rule takes them (1.24 times at most), 3 % would be faster where it does not, and on the average it is 1 % above the better one.
 // us, votes / bits: 256 images of 4 x 28 x 28, field 5 30 / 12, field 1 7.7 / 9.7; 16 images of 3 x 16 x 16, field 3 5.2 / 6.9; 16 of 64 x 28 x 28, field
-// 2 18 / 41, field 5 90 / 65; 64 of 64 x 7 x 7, field 4 55 / 79.
+// 2 18 / 41, field 5 90 / 65; 64 of 64 x 7 x 7, field 4 55 / 79; one of 32 x 8 x 8, field 7 81 / 7.6; 5 of 64 x 8 x 8, field 5 83 / 21.
 static inline bool conv_bits_pay(const ConvGeom &g, long long rows, int cols, int words, int tiles) {
-    const long long P = (long long)g.OH * g.OW, images = tiles * 64 / P + 2;
-    const double blocks = dl_ceil_div(rows, 64LL * tiles), rounds = dl_ceil_div((long long)blocks, 512);
-    const double trips = dl_ceil_div((images < g.B ? images : g.B) * words, 128);
-    const double turns = dl_ceil_div((long long)tiles * cols, 64 * CONV_BIT_WAVES) * (64.0 / g.OW + 1.0);
-    const double bits = 3.1 + (3.4 * rounds + 0.0002 * blocks) * trips + (0.016 * rounds + 0.0023 * blocks) * turns;
-    const double votes = 4.2 + cols * (0.045 + 0.00006 * dl_ceil_div(rows, 64));
-    return g.OW >= 8 && bits < 0.85 * votes;
+    const int P = g.OH * g.OW, BT = dl_ceil_div(rows, 64), held = tiles < BT ? tiles : BT, span = 64 * held;
+    const int images = (span - 1) / P + 1 + (P % span != 0 && span % P != 0), blocks = dl_ceil_div(rows, 64LL * tiles);
+    const double rounds = blocks > 512 ? blocks / 512.0 : 1.0, trips = dl_ceil_div((long long)(images < g.B ? images : g.B) * words, 128);
+    const double turns = dl_ceil_div((long long)held * cols, 64 * CONV_BIT_WAVES), lines = turns * (64.0 / g.OW + (64 % g.OW != 0));
+    const double bits = 2.0 + rounds * (2.44 * trips + 1.7 * turns + 0.068 * lines) + blocks * (0.0042 * trips + 0.00048 * lines);
+    const double votes = 3.35 + cols * (0.048 + 0.000038 * BT + 0.000062 * (BT > 2048 ? BT - 2048 : 0)) + 0.00077 * BT;
+    return bits < 0.95 * votes;
 }
 // tiles per block, 0: not by bits
 static int conv_bit_tiles(const ConvGeom &g, long long rows, int cols, int words) {

@@ -134,6 +134,9 @@ def _kernels_of(call):
     (((23, 30, 10, 9), (5, 5, 1, 1, 1, 2)), True),     # a last tile of 56 rows
     (((6, 160, 24, 24), (5, 5, 1, 1, 0, 0)), True),    # an image of 1440 words: four tiles to a block
     (((1, 40, 30, 30), (5, 5, 1, 1, 0, 0)), True),
+    (((1, 32, 8, 8), (7, 7, 1, 1, 0, 0)), True),       # lines of two positions, a block's only tile of four rows
+    (((5, 64, 8, 8), (5, 5, 1, 1, 0, 0)), True),       # of four
+    (((3, 32, 5, 5), (5, 5, 1, 1, 2, 2)), True),       # of five, padded
     (((256, 4, 28, 28), (1, 1, 1, 1, 0, 0)), False),   # few words to make
     (((16, 1, 28, 28), (5, 5, 1, 1, 0, 0)), False),
     (((64, 64, 7, 7), (4, 4, 1, 1, 0, 0)), False),     # short lines
